@@ -1049,11 +1049,8 @@ int unpack_launch(jl_ctx* c, int type, const PlaneRef& pl, int nrows, int k, voi
     a.dst = (uint8_t*)dst; a.qs = pl.qs; a.d = pl.d; a.sc = pl.sc;
     a.nrows = nrows; a.k = k; a.row0 = pl.row; a.stride = pl.stride;
     void* params[] = {&a};
-    if (type == JL_TYPE_Q8_0 || type == JL_TYPE_MXFP4)
-        return launch(c, type == JL_TYPE_Q8_0 ? "jl_unpack_q8_0" : "jl_unpack_mxfp4", (unsigned)((nrows + 255) / 256),
-                      (unsigned)(k / 32), 256, 0, st, params);
-    return launch(c, type == JL_TYPE_Q6_K ? "jl_unpack_q6k" : "jl_unpack_q4k", (unsigned)((nrows + 255) / 256),
-                  (unsigned)(k / 256), 256, 0, st, params);
+    const char* name = type == JL_TYPE_Q4_K ? "jl_unpack_q4k" : type == JL_TYPE_Q6_K ? "jl_unpack_q6k" : type == JL_TYPE_Q8_0 ? "jl_unpack_q8_0" : "jl_unpack_mxfp4";
+    return launch(c, name, (unsigned)((nrows + 63) / 64), (unsigned)((k + 255) / 256), 256, 0, st, params);
 }
 
 int packed_matmul_launch(jl_ctx* c, float* out, int type, const PlaneRef& pl, const float* x, int nrows,

@@ -120,11 +120,13 @@ extern "C" __global__ __launch_bounds__(1024) void jl_matvec_segments(MatVecMult
 // ---------------------------------------------------------- packed planes
 // grid = (ceil(nrows/256), k/256 or k/32 for Q8_0), block = 256
 extern "C" __global__ __launch_bounds__(256) void jl_pack_weights(PackArgs p) { pack_weights_body(p); }
-extern "C" __global__ __launch_bounds__(256) void jl_unpack_q4k(UnpackArgs p) { unpack_q4k_body(p); }
-extern "C" __global__ __launch_bounds__(256) void jl_unpack_q6k(UnpackArgs p) { unpack_q6k_body(p); }
-// grid = (ceil(nrows/256), k/32)
-extern "C" __global__ __launch_bounds__(256) void jl_unpack_q8_0(UnpackArgs p) { unpack_q8_0_body(p); }
-extern "C" __global__ __launch_bounds__(256) void jl_unpack_mxfp4(UnpackArgs p) { unpack_mxfp4_body(p); }
+// grid = (ceil(nrows/64), ceil(k/256)), block = 256
+#define JL_UNPACK_KERNEL(T, TYPE)                                                              \
+    extern "C" __global__ __launch_bounds__(256) void jl_unpack_##T(UnpackArgs p) {            \
+        __shared__ __attribute__((aligned(16))) uint8_t lds[JL_UNPACK_LDS];                    \
+        unpack_body<TYPE>(p, lds);                                                             \
+    }
+JL_UNPACK_KERNEL(q4k, JL_Q4_K) JL_UNPACK_KERNEL(q6k, JL_Q6_K) JL_UNPACK_KERNEL(q8_0, JL_Q8_0) JL_UNPACK_KERNEL(mxfp4, JL_MXFP4)
 // jl_matvec_packed_<type>_w<rows per wavefront>: grid = ceil(nrows/RW), block = 64..1024
 // XPRE = chunks whose activation loads go out ahead of the weights (register budget).
 // jl_matvec_packed_<type>_w<RW> quantizes f32 x itself; jl_matvec_packed_q8_<type>_w<RW>

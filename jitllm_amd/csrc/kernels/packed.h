@@ -149,119 +149,140 @@ __device__ __forceinline__ void pack_weights_body(const PackArgs& p) {
     else pack_q8_0(p, r, u);
 }
 
-// The inverse for Q4_K: planes (row range row0.. of a buffer of `stride` rows) back
-// to GGUF row-major super-blocks, bit for bit.  The 12 scale bytes are the sixteen
-// 6-bit values in ggml's arrangement (format/quant/dequant.go:360-365).
-__device__ __forceinline__ void unpack_q4k_body(const UnpackArgs& p) {
-    const int rl = blockIdx.x * 256 + threadIdx.x, sb = blockIdx.y;
-    if (rl >= p.nrows) return;
-    const size_t n = (size_t)p.stride, r = (size_t)p.row0 + rl;
-    const int nsb = p.k / 256;
-    u32* blk = (u32*)(p.dst + ((size_t)rl * nsb + sb) * 144);
-    blk[0] = p.d[(size_t)sb * n + r];
-    u32 ws[3];
+// The inverse: planes (row range row0.. of a buffer of `stride` rows) back to GGUF row-major blocks, bit for
+// bit.  A plane word's neighbours belong to 64 other rows and a row's bytes to consecutive words, so the
+// workgroup turns a tile of 64 rows x 256 of K round in LDS: words come in along the rows (256 bytes a
+// wavefront), the tile's rows go out 16 bytes a lane.  (One thread a (row, unit) that stored its own block's
+// words scattered every store over 64 rows: Q8_0 12428 x 4096 166 us for 108 MB; this form is bound by the
+// two streams.)  grid = (ceil(nrows / 64), ceil(k / 256)), block = 256, static LDS = JL_UNPACK_LDS.
+__device__ __forceinline__ void st4_a2(uint8_t* p, u32 v) { ((u32_a2*)p)->v = v; }
+struct __attribute__((packed, aligned(1))) u32_a1 { u32 v; };
+struct __attribute__((packed, aligned(1))) u32x4_st1 { u32x4 v; };
+#define JL_UNPACK_LDS (64 * 276)
+
+// One (row, sub-unit) of the tile into the row's image.  q: which quarter of the 256 elements.
+__device__ __forceinline__ void unpack_q4k_quarter(const UnpackArgs& p, int sb, int q, size_t r, uint8_t* img) {
+    const size_t n = (size_t)p.stride;
+    u32* blk = (u32*)img;
+    if (q == 0) {
+        blk[0] = p.d[(size_t)sb * n + r];
+        u32 ws[3];
 #pragma unroll
-    for (int w = 0; w < 3; w++) ws[w] = p.sc[((size_t)sb * 3 + w) * n + r];
-    const uint64_t lo = ws[0] | ((uint64_t)ws[1] << 32), hi = ws[1] | ((uint64_t)ws[2] << 32);
-    u32 sc[8], m[8];
+        for (int w = 0; w < 3; w++) ws[w] = p.sc[((size_t)sb * 3 + w) * n + r];
+        const uint64_t lo = ws[0] | ((uint64_t)ws[1] << 32), hi = ws[1] | ((uint64_t)ws[2] << 32);
+        u32 sc[8], m[8];
 #pragma unroll
-    for (int s = 0; s < 8; s++) {
-        const int bit = 12 * s;
-        const u32 f = bit < 32 ? (u32)(lo >> bit) : (u32)(hi >> (bit - 32));
-        sc[s] = f & 63;
-        m[s] = (f >> 6) & 63;
+        for (int s = 0; s < 8; s++) {
+            const int bit = 12 * s;
+            const u32 f = bit < 32 ? (u32)(lo >> bit) : (u32)(hi >> (bit - 32));
+            sc[s] = f & 63;
+            m[s] = (f >> 6) & 63;
+        }
+        u32 s0 = 0, s1 = 0, s2 = 0;
+        // the sixteen 6-bit values in ggml's arrangement (format/quant/dequant.go:360-365)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            s0 |= (sc[j] | ((sc[j + 4] >> 4) << 6)) << (8 * j);
+            s1 |= (m[j] | ((m[j + 4] >> 4) << 6)) << (8 * j);
+            s2 |= ((sc[j + 4] & 0xF) | ((m[j + 4] & 0xF) << 4)) << (8 * j);
+        }
+        blk[1] = s0; blk[2] = s1; blk[3] = s2;
     }
-    u32 s0 = 0, s1 = 0, s2 = 0;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        s0 |= (sc[j] | ((sc[j + 4] >> 4) << 6)) << (8 * j);
-        s1 |= (m[j] | ((m[j + 4] >> 4) << 6)) << (8 * j);
-        s2 |= ((sc[j + 4] & 0xF) | ((m[j + 4] & 0xF) << 4)) << (8 * j);
-    }
-    blk[1] = s0; blk[2] = s1; blk[3] = s2;
     const u32 M = 0x0F0F0F0Fu;
 #pragma unroll
-    for (int g = 0; g < 4; g++)
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-            const u32 e = p.qs[((size_t)(sb * 8 + 2 * g) * 4 + w) * n + r];
-            const u32 o = p.qs[((size_t)(sb * 8 + 2 * g + 1) * 4 + w) * n + r];
-            blk[4 + g * 8 + w] = (e & M) | ((o & M) << 4);
-            blk[4 + g * 8 + 4 + w] = ((e >> 4) & M) | (o & ~M);
-        }
+    for (int w = 0; w < 4; w++) {
+        const u32 e = p.qs[((size_t)(sb * 8 + 2 * q) * 4 + w) * n + r];
+        const u32 o = p.qs[((size_t)(sb * 8 + 2 * q + 1) * 4 + w) * n + r];
+        blk[4 + q * 8 + w] = (e & M) | ((o & M) << 4);
+        blk[4 + q * 8 + 4 + w] = ((e >> 4) & M) | (o & ~M);
+    }
 }
 
-// The inverse for Q6_K (pack_q6k above): one thread per (row, super-block).  Per (half, run)
-// the four sub-blocks 8*half + 2*grp + run share sixteen ql bytes pairwise (grp and grp + 2:
-// low and high nibbles) and sixteen qh bytes all four (two bits each); a plane word holds the
-// nibbles of elements j and j + 8 (w0) or 4 + j and 12 + j (w1) in byte j, the bit-pair word
-// the top bits of elements j, 4 + j, 8 + j, 12 + j.  Blocks are 210 bytes: 2-byte aligned stores.
-__device__ __forceinline__ void st4_a2(uint8_t* p, u32 v) { ((u32_a2*)p)->v = v; }
-
-__device__ __forceinline__ void unpack_q6k_body(const UnpackArgs& p) {
-    const int rl = blockIdx.x * 256 + threadIdx.x, sb = blockIdx.y;
-    if (rl >= p.nrows) return;
-    const size_t n = (size_t)p.stride, r = (size_t)p.row0 + rl;
-    const int nsb = p.k / 256;
-    uint8_t* blk = p.dst + ((size_t)rl * nsb + sb) * 210;
-    *(uint16_t*)(blk + 208) = (uint16_t)p.d[(size_t)sb * n + r];
-#pragma unroll
-    for (int j = 0; j < 4; j++)   // int8 scales are stored + 128
-        st4_a2(blk + 192 + 4 * j, p.sc[((size_t)sb * 4 + j) * n + r] ^ 0x80808080u);
+// Q6_K: quarter q = (half, run).  The four sub-blocks 8*half + 2*grp + run share sixteen ql bytes pairwise
+// (grp and grp + 2: low and high nibbles) and sixteen qh bytes all four (two bits each); a plane word holds
+// the nibbles of elements j and j + 8 (w0) or 4 + j and 12 + j (w1) in byte j, the bit-pair word the top
+// bits of elements j, 4 + j, 8 + j, 12 + j.
+__device__ __forceinline__ void unpack_q6k_quarter(const UnpackArgs& p, int sb, int q, size_t r, uint8_t* img) {
+    const size_t n = (size_t)p.stride;
+    const int half = q >> 1, run = q & 1;
+    st4_a2(img + 192 + 4 * q, p.sc[((size_t)sb * 4 + q) * n + r] ^ 0x80808080u);   // int8 scales are stored + 128
+    if (q == 0) *(uint16_t*)(img + 208) = (uint16_t)p.d[(size_t)sb * n + r];
     const u32 M = 0x0F0F0F0Fu, T = 0x03030303u;
+    u32 N[4][4], H[4];   // [grp][four elements] nibbles in bytes; bit-pair words
 #pragma unroll
-    for (int half = 0; half < 2; half++)
+    for (int g = 0; g < 4; g++) {
+        const size_t base = ((size_t)(sb * 16 + half * 8 + 2 * g + run) * 3) * n + r;
+        const u32 w0 = p.qs[base], w1 = p.qs[base + n];
+        H[g] = p.qs[base + 2 * n];
+        N[g][0] = w0 & M; N[g][2] = (w0 >> 4) & M;
+        N[g][1] = w1 & M; N[g][3] = (w1 >> 4) & M;
+    }
 #pragma unroll
-        for (int run = 0; run < 2; run++) {
-            u32 N[4][4], H[4];   // [grp][four elements] nibbles in bytes; bit-pair words
+    for (int i = 0; i < 4; i++) {
+        st4_a2(img + half * 64 + run * 16 + 4 * i, N[0][i] | (N[2][i] << 4));
+        st4_a2(img + half * 64 + 32 + run * 16 + 4 * i, N[1][i] | (N[3][i] << 4));
+        u32 h = 0;
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const size_t base = ((size_t)(sb * 16 + half * 8 + 2 * g + run) * 3) * n + r;
-                const u32 w0 = p.qs[base], w1 = p.qs[base + n];
-                H[g] = p.qs[base + 2 * n];
-                N[g][0] = w0 & M; N[g][2] = (w0 >> 4) & M;
-                N[g][1] = w1 & M; N[g][3] = (w1 >> 4) & M;
-            }
+        for (int g = 0; g < 4; g++) h |= ((H[g] >> (2 * i)) & T) << (2 * g);
+        st4_a2(img + 128 + half * 32 + run * 16 + 4 * i, h);
+    }
+}
+
+// Q8_0 (two rows share a word of the D plane) and MXFP4: blocks 2q and 2q + 1 of the eight.
+__device__ __forceinline__ void unpack_q8_0_quarter(const UnpackArgs& p, int u, int q, size_t r, uint8_t* img) {
+    const size_t n = (size_t)p.stride;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                st4_a2(blk + half * 64 + run * 16 + 4 * i, N[0][i] | (N[2][i] << 4));
-                st4_a2(blk + half * 64 + 32 + run * 16 + 4 * i, N[1][i] | (N[3][i] << 4));
-                u32 q = 0;
+    for (int i = 0; i < 2; i++) {
+        const int b = u * 8 + 2 * q + i;
+        if (b >= p.k / 32) return;
+        uint8_t* blk = img + (2 * q + i) * 34;
+        const u32 dd = p.d[(size_t)b * ((n + 1) / 2) + (r >> 1)];
+        *(uint16_t*)blk = (uint16_t)(r & 1 ? dd >> 16 : dd);
 #pragma unroll
-                for (int g = 0; g < 4; g++) q |= ((H[g] >> (2 * i)) & T) << (2 * g);
-                st4_a2(blk + 128 + half * 32 + run * 16 + 4 * i, q);
-            }
+        for (int w = 0; w < 8; w++) st4_a2(blk + 2 + 4 * w, p.qs[((size_t)b * 8 + w) * n + r]);
+    }
+}
+__device__ __forceinline__ void unpack_mxfp4_quarter(const UnpackArgs& p, int u, int q, size_t r, uint8_t* img) {
+    const size_t n = (size_t)p.stride;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int b = u * 8 + 2 * q + i;
+        if (b >= p.k / 32) return;
+        uint8_t* blk = img + (2 * q + i) * 17;
+        const u32 dd = p.d[(size_t)b * ((n + 3) / 4) + (r >> 2)];
+        blk[0] = (uint8_t)(((dd >> (8 * (r & 3))) & 0xFF) + 1);
+#pragma unroll
+        for (int w = 0; w < 4; w++) ((u32_a1*)(blk + 1 + 4 * w))->v = p.qs[((size_t)b * 4 + w) * n + r];
+    }
+}
+
+template <int TYPE>
+__device__ __forceinline__ void unpack_body(const UnpackArgs& p, uint8_t* lds) {
+    constexpr int UB = TYPE == JL_Q4_K ? 144 : TYPE == JL_Q6_K ? 210 : TYPE == JL_Q8_0 ? 272 : 136;   // bytes of 256 elements
+    constexpr int RS = (UB + 3) / 4 * 4 + 4;                          // an odd number of words: rows spread over the banks
+    const int rt = blockIdx.x * 64, u = blockIdx.y, lane = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const int rl = min(rt + lane, p.nrows - 1);
+    uint8_t* img = lds + lane * RS;
+    const size_t r = (size_t)p.row0 + rl;
+    if constexpr (TYPE == JL_Q4_K) unpack_q4k_quarter(p, u, q, r, img);
+    else if constexpr (TYPE == JL_Q6_K) unpack_q6k_quarter(p, u, q, r, img);
+    else if constexpr (TYPE == JL_Q8_0) unpack_q8_0_quarter(p, u, q, r, img);
+    else unpack_mxfp4_quarter(p, u, q, r, img);
+    __syncthreads();
+    const int row_bytes = TYPE == JL_Q4_K || TYPE == JL_Q6_K ? p.k / 256 * UB : p.k / 32 * (UB / 8);
+    const int nb = min(UB, row_bytes - u * UB);                       // (the last unit of a K that is no multiple of 256)
+    const int np = (nb + 15) / 16, live = min(64, p.nrows - rt);
+    for (int i = threadIdx.x; i < live * np; i += 256) {
+        const int rr = i / np, at = 16 * (i % np);
+        const uint8_t* s = lds + rr * RS + at;
+        uint8_t* o = p.dst + (size_t)(rt + rr) * row_bytes + (size_t)u * UB + at;
+        if (at + 16 <= nb) {
+            const u32* w = (const u32*)s;
+            ((u32x4_st1*)o)->v = u32x4{w[0], w[1], w[2], w[3]};
+        } else {
+            for (int j = 0; j < nb - at; j++) o[j] = s[j];
         }
-}
-
-// The inverse for Q8_0 (pack_q8_0 above): one thread per (row, block); two rows share a word
-// of the D plane.
-__device__ __forceinline__ void unpack_q8_0_body(const UnpackArgs& p) {
-    const int rl = blockIdx.x * 256 + threadIdx.x, b = blockIdx.y;
-    if (rl >= p.nrows) return;
-    const size_t n = (size_t)p.stride, r = (size_t)p.row0 + rl;
-    const int nb = p.k / 32;
-    uint8_t* blk = p.dst + ((size_t)rl * nb + b) * 34;
-    const u32 dd = p.d[(size_t)b * ((n + 1) / 2) + (r >> 1)];
-    *(uint16_t*)blk = (uint16_t)(r & 1 ? dd >> 16 : dd);
-#pragma unroll
-    for (int w = 0; w < 8; w++) st4_a2(blk + 2 + 4 * w, p.qs[((size_t)b * 8 + w) * n + r]);
-}
-
-// The inverse for MXFP4 (pack_mxfp4 above): one thread per (row, block).
-struct __attribute__((packed, aligned(1))) u32x4_st1 { u32x4 v; };
-__device__ __forceinline__ void unpack_mxfp4_body(const UnpackArgs& p) {
-    const int rl = blockIdx.x * 256 + threadIdx.x, b = blockIdx.y;
-    if (rl >= p.nrows) return;
-    const size_t n = (size_t)p.stride, r = (size_t)p.row0 + rl;
-    const int nb = p.k / 32;
-    uint8_t* blk = p.dst + ((size_t)rl * nb + b) * 17;
-    const u32 dd = p.d[(size_t)b * ((n + 3) / 4) + (r >> 2)];
-    blk[0] = (uint8_t)(((dd >> (8 * (r & 3))) & 0xFF) + 1);
-    u32x4 q;
-#pragma unroll
-    for (int w = 0; w < 4; w++) q[w] = p.qs[((size_t)b * 4 + w) * n + r];
-    ((u32x4_st1*)(blk + 1))->v = q;
+    }
 }
 
 // ---------------------------------------------------------------- matvec
