@@ -94,8 +94,10 @@ int jl_synchronize(jl_ctx *ctx);
  * "matvec.act_split" (1: a group's gated activation is formed and quantized once, by a launch of
  * its own, instead of by every workgroup), "gemm.min_tok"
  * (fewest tokens sent to the matrix-core GEMM), "gemm.form" (1: 128 x 64 tiles, 2: 256 x 128
- * tiles, 3: two-pass, 4 / 5: the few-token forms, 6: 128 x 64 tiles over the whole of K on two
- * groups of wavefronts, 9: token by token), "gemm.rows" (64 or 128),
+ * tiles, 3: two-pass, 4: up to 64 tokens on the int8 matrix cores, 5: 32 rows x 64 tokens a
+ * workgroup, 6: 128 x 64 tiles over the whole of K on two groups of wavefronts, 9: token by
+ * token), "gemm.few" (form 4: 1 for any number of tokens, 2 never), "few.nt" / "few.rt" /
+ * "few.waves" (its token tiles, row tiles and wavefronts a workgroup), "gemm.rows" (64 or 128),
  * "gemm.split" (K slices), "gemm.prep" (4: the four-wavefront activation prep), "gemm.planes"
  * (2: restore rows from planes before the GEMM), "packed.rw" (rows per wavefront of the
  * packed-plane matvec: 16, 32, 64), "packed.block" (its threads per workgroup), "moe.shares"

@@ -42,6 +42,8 @@ struct Tuning {
     int gemm_split = 0;
     int gemm_prep = 0;
     int gemm_planes = 0;
+    int gemm_few = 0;           // the int8 few-token form: 1 wherever it fits, 2 never
+    int few_nt = 0, few_rt = 0, few_waves = 0;
     int moe_form = 0;
     int moe_g16 = 0;
     int gemm_fold = 0, gemm_fold_waves = 0;
@@ -576,12 +578,11 @@ constexpr int kGemmWideTok = 256;
 constexpr unsigned kGemmK2LdsBytes = 2u * (2u * 64u * 136u * 2u + 2u * 64u * 24u * 2u + 2u * 64u * 2u * 4u + 2u * 128u * 4u);
 constexpr unsigned kGemmWideLdsBytes = 2u * 128u * 136u * 2u + 2u * 128u * 24u * 2u + 2u * 128u * 2u * 4u + 2u * kGemmWideTok * 4u;   // JL_GEMM_WIDE_LDS_BYTES
 
-// Few tokens, or a grid of at most a round and a half of 32-row workgroups: the forms that
-// take a lane's operand words straight from GGUF rows (no plane form of them exists).
+// A grid of at most a round and a half of 32-row workgroups: the form that takes a lane's operand
+// words straight from GGUF rows (no plane form of it exists).
 bool gemm_q4k_few_applies(const jl_ctx* c, int nrows, int k, int ntok) {
     const int form = c->tune.gemm_form;
     if ((size_t)nrows * (size_t)(k / 256) * 144 >= ((size_t)1 << 32)) return false;
-    if ((form == 0 || form == 4) && ntok <= 64) return true;
     const long few32_groups = (long)((nrows + 31) / 32) * ((ntok + 63) / 64);
     return ((form == 0 && 2 * few32_groups <= 3L * c->num_cu) || (form == 5 && ntok <= 1024)) && ntok > 64;
 }
@@ -592,32 +593,8 @@ int gemm_q4k_launch(jl_ctx* c, float* out, const void* w, const float* x, int nr
                     hipStream_t st, const PlaneRef* pl = nullptr) {
     int form = c->tune.gemm_form;
     if (pl && form == 3) form = 0;
-    if (!pl && (form == 0 || form == 4) && ntok <= 64 && (size_t)nrows * (size_t)(k / 256) * 144 < ((size_t)1 << 32)) {
-        // few tokens: 16-row workgroups that split K over their wavefronts, one launch after
-        // the activation prep (kernels/gemm_q4k.h, "few tokens")
-        const int tok_pad = (ntok + 31) / 32 * 32, nsb = k / 256, nt = (ntok + 15) / 16;
-        int rc = gemm_ws_ensure(c, gemm_ws_need(tok_pad, k));
-        if (rc != JL_OK) return rc;
-        uint16_t* bq = (uint16_t*)c->gemm_ws;
-        float* da = (float*)((char*)c->gemm_ws + (size_t)nsb * 2 * (tok_pad / 32) * kGemmAStageBytes);
-        GemmPrepArgs pa;
-        pa.x = x; pa.bq = bq; pa.da = da; pa.ntok = ntok; pa.tok_pad = tok_pad; pa.k = k;
-        void* pp[] = {&pa};
-        rc = launch(c, "jl_gemm_prep_q4k_w16", (unsigned)nsb, (unsigned)(tok_pad / 32), 1024, 0, st, pp);
-        if (rc != JL_OK) return rc;
-        GemmArgs ga;
-        ga.out = out; ga.w = (const uint8_t*)w; ga.bq = bq; ga.da = da;
-        ga.nrows = nrows; ga.k = k; ga.ntok = ntok; ga.tok_pad = tok_pad; ga.row_bytes = nsb * 144;
-        ga.out_stride = nrows; ga.sb_per = 0;
-        void* gp[] = {&ga};
-        char name[32];
-        snprintf(name, sizeof name, "jl_gemm_q4k_few_t%d", nt);
-        return launch(c, name, (unsigned)((nrows + 15) / 16), 1, 512, 0, st, gp);
-    }
-    const long few32_groups = (long)((nrows + 31) / 32) * ((ntok + 63) / 64);
-    if (!pl && ((form == 0 && 2 * few32_groups <= 3L * c->num_cu) || (form == 5 && ntok <= 1024)) && ntok > 64 &&
-        (size_t)nrows * (size_t)(k / 256) * 144 < ((size_t)1 << 32)) {
-        // some more tokens, few enough rows: the same scheme on 32-row x 64-token workgroups,
+    if (!pl && gemm_q4k_few_applies(c, nrows, k, ntok)) {
+        // some more than few tokens, few enough rows: 32-row x 64-token workgroups that split K,
         // one to a CU, while the grid is at most a round and a half (4096 rows: up to 192
         // tokens; measured against the tiled forms, 128 tokens x 4096 rows 24.6 -> 16.5 us;
         // at 14336 rows the tiled forms win)
@@ -871,6 +848,98 @@ int gemm_w32_launch(jl_ctx* c, float* out, int type, const void* w, const float*
     return launch(c, kernel, (unsigned)(tok_pad / kGemmTile), (unsigned)((nrows + 63) / 64), 256, lds, st, gp);
 }
 
+// Few tokens, or few columns an expert, on the int8 matrix cores (kernels/few_i8.h): up to two
+// matrices (banks) of one type and shape over the same columns.
+struct FewCall {
+    int type = 0, nrows = 0, k = 0, ncols = 0, nmat = 1, n_expert = 1;
+    const void* w[2] = {nullptr, nullptr};        // GGUF rows
+    const PlaneRef* pl[2] = {nullptr, nullptr};   // or planes
+    size_t sheet_bytes = 0, sheet_words = 0;
+    int row_step = 0;
+    const float *x = nullptr, *x2 = nullptr;
+    const uint32_t *src = nullptr, *start = nullptr;
+    float *out[2] = {nullptr, nullptr}, *resid = nullptr;
+};
+
+// K in chunks of 128 (Q8_0 may end inside one); GGUF row offsets and plane words within 32 bits
+bool few_fits(const jl_ctx* c, int type, bool planes, int nrows, int k, int ncols, int stride) {
+    const TypeInfo* ti = type_info(type);
+    if (!ti || c->tune.gemm_few == 2 || k % ti->block_elems || ncols > 65535 * 4 || (k + 255) / 256 > 65535) return false;
+    if (planes) return (size_t)stride * 4 * 8 < ((size_t)1 << 32);
+    if (type == JL_TYPE_Q8_0 && k % 64) return false;   // (rows on 4-byte boundaries)
+    return (size_t)nrows * (size_t)(k / ti->block_elems) * ti->block_bytes < ((size_t)1 << 32);
+}
+
+int few_launch(jl_ctx* c, const FewCall& f, hipStream_t st) {
+    const bool planes = f.pl[0] != nullptr;
+    const TypeInfo* ti = type_info(f.type);
+    const int nch = (f.k + 255) / 256 * 2;
+    const int nslots = f.start ? f.ncols / 16 + f.n_expert + 1 : (f.ncols + 15) / 16;
+    const size_t q_bytes = (size_t)nch * nslots * 2048, s_bytes = (size_t)nch * nslots * 256;
+    void** ws = f.start ? &c->moe_q_ws : &c->gemm_ws;
+    int rc = grow(c, ws, f.start ? &c->moe_q_ws_bytes : &c->gemm_ws_bytes, q_bytes + 2 * s_bytes);
+    if (rc != JL_OK) return rc;
+    FewI8PrepArgs pa;
+    pa.x = f.x; pa.x2 = f.x2; pa.src = f.src; pa.start = f.start;
+    pa.bq = (uint32_t*)*ws; pa.da = (float*)((char*)*ws + q_bytes);
+    pa.ds = f.type == JL_TYPE_Q4_K ? (float*)((char*)*ws + q_bytes + s_bytes) : nullptr;
+    pa.k = f.k; pa.per = c->act_window / 32; pa.ncols = f.ncols; pa.n_expert = f.n_expert; pa.nslots = nslots;
+    pa.nch = nch;
+    pa.order = f.type == JL_TYPE_Q8_0 || !planes ? 0 : f.type == JL_TYPE_Q4_K ? 1 : 2;
+    const bool w256 = f.type != JL_TYPE_Q8_0 && c->act_window == 256;
+    pa.isum = w256;
+    void* pp[] = {&pa};
+    rc = launch(c, "jl_few_prep", (unsigned)((f.k + 255) / 256), (unsigned)((f.ncols + 3) / 4), 256, 0, st, pp);
+    if (rc != JL_OK) return rc;
+    FewI8Args a;
+    memset(&a, 0, sizeof a);
+    for (int m = 0; m < f.nmat; m++) {
+        a.out[m] = f.out[m];
+        a.w[m] = (const uint8_t*)f.w[m];
+        if (planes) { a.pqs[m] = f.pl[m]->qs; a.pd[m] = f.pl[m]->d; a.psc[m] = f.pl[m]->sc; }
+    }
+    a.resid = f.resid; a.bq = pa.bq; a.da = pa.da; a.ds = pa.ds; a.start = f.start;
+    a.sheet_bytes = f.sheet_bytes; a.sheet_words = f.sheet_words; a.row_step = f.row_step;
+    if (planes) { a.prow0 = f.pl[0]->row; a.pstride = f.pl[0]->stride; }
+    a.nrows = f.nrows; a.k = f.k; a.row_bytes = (f.k / ti->block_elems) * ti->block_bytes;
+    a.ncols = f.ncols; a.nslots = nslots; a.nch = nch;
+    // Token tiles a workgroup: what the (average) group fills.  Row tiles: more rows a workgroup share the
+    // activations' loads, and over planes widen the weights' (measured at 14336 x 4096 / 4096 x 4096, us, row
+    // tiles 1 / 2 / 4: Q8_0 planes 16 tokens 28.8 20.6 18.7 / 11.6 11.3 14.7; Q4_K planes 20.1 15.4 14.4 /
+    // 8.4 9.4 12.6; Q4_K rows 18.2 16.4 - / 8.5 10.2 -; Q8_0 rows 64 tokens 39.3 35.0 - / 13.5 18.0 -): as
+    // many as leave most CUs a workgroup.
+    const long avg = ((long)f.ncols + f.n_expert - 1) / f.n_expert;
+    const int nt = c->tune.few_nt ? c->tune.few_nt : avg <= 16 ? 1 : avg <= 32 ? 2 : 4;
+    const long sheets = (long)f.n_expert * f.nmat, cus = c->num_cu;
+    int rt = 1;
+    if (planes ? (f.nrows + 31) / 32 * sheets >= cus : nt != 2 && (f.type == JL_TYPE_Q4_K || nt == 4) && (f.nrows + 31) / 32 * sheets >= cus)
+        rt = 2;
+    if (planes && nt <= 2 && (nt == 2 || f.type != JL_TYPE_Q6_K) && (f.nrows + 63) / 64 * sheets * 10 >= cus * 7) rt = 4;
+    if (c->tune.few_rt) rt = c->tune.few_rt;
+    if (f.nrows < rt) rt = 1;
+    int nw = c->tune.few_waves ? c->tune.few_waves : 8;
+    if (nw > nch / 2) nw = nch / 2;
+    while (nw > 1 && (size_t)nw * JL_FEW_WAVE_BYTES(f.type, planes, rt) > c->lds_limit) nw--;
+    a.nwaves = nw;
+    const unsigned lds = (unsigned)std::max(nw * JL_FEW_WAVE_BYTES(f.type, planes, rt), JL_FEW_RED_BYTES(nw, nt, rt));
+    if (lds > c->lds_limit) return JL_DECLINED;
+    char name[48];
+    snprintf(name, sizeof name, "jl_few_%s%s_%s_t%dr%d", ti->tag, w256 ? "w" : "",
+             planes ? "planes" : "rows", nt, rt);
+    void* ap[] = {&a};
+    return launch(c, name, (unsigned)((f.nrows + 16 * rt - 1) / (16 * rt)), (unsigned)f.n_expert, (unsigned)(64 * nw), lds, st, ap,
+                  (unsigned)f.nmat);
+}
+
+// Where the int8 few-token form serves a plain matmul.
+bool few_applies(const jl_ctx* c, int type, bool planes, int nrows, int k, int ntok, int stride) {
+    if (!few_fits(c, type, planes, nrows, k, ntok, stride)) return false;
+    if (c->tune.gemm_few == 1 || (c->tune.gemm_form == 4 && ntok <= 64)) return true;
+    if (c->tune.gemm_form != 0 || ntok > 64) return false;
+    // (two tokens: two matvecs are as fast for the k-quants, not for Q8_0: 21 against 22 us, 9.6 against 10.6)
+    return ntok >= (type == JL_TYPE_Q8_0 ? 2 : c->gemm_min_tok);
+}
+
 // out [ntok][nrows] = x [ntok][k] W^T on device operands: the matrix-core GEMM where it
 // applies, else one fused matvec launch per token (same values, token by token).
 int matmul_launch(jl_ctx* c, float* out, int type, const void* w, const float* x, int nrows, int k,
@@ -880,6 +949,12 @@ int matmul_launch(jl_ctx* c, float* out, int type, const void* w, const float* x
     if (rc != JL_OK) return rc;
     if (!out || !w || !x || ntok <= 0) return fail(c, JL_ERR_ARG, "matmul: bad operand");
     if (!aligned16(x) || (k % 4) != 0) return JL_DECLINED;
+    if (few_applies(c, type, false, nrows, k, ntok, 0) && ((uintptr_t)w & (type == JL_TYPE_Q4_K ? 15 : 3)) == 0) {
+        FewCall f;
+        f.type = type; f.nrows = nrows; f.k = k; f.ncols = ntok; f.w[0] = w; f.x = x; f.out[0] = out;
+        rc = few_launch(c, f, st);
+        if (rc != JL_DECLINED) return rc;
+    }
     const bool gemm = type == JL_TYPE_Q4_K && c->act_window == 256 && ntok >= c->gemm_min_tok &&
                       aligned16(w) && ntok <= 65535 * 4 && kGemmLdsBytes <= c->lds_limit;
     if (gemm) return gemm_q4k_launch(c, out, w, x, nrows, k, ntok, st);
@@ -1060,6 +1135,12 @@ int packed_matmul_launch(jl_ctx* c, float* out, int type, const PlaneRef& pl, co
     if (rc != JL_OK) return rc;
     if (!out || !x || ntok <= 0) return fail(c, JL_ERR_ARG, "packed matmul: bad operand");
     if (!aligned16(x) || (k % 4) != 0) return JL_DECLINED;
+    if (few_applies(c, type, true, nrows, k, ntok, pl.stride)) {
+        FewCall f;
+        f.type = type; f.nrows = nrows; f.k = k; f.ncols = ntok; f.pl[0] = &pl; f.x = x; f.out[0] = out;
+        rc = few_launch(c, f, st);
+        if (rc != JL_DECLINED) return rc;
+    }
     // the matrix-core forms read GGUF rows: the planes are turned back into rows in a workspace
     const bool gemm = type == JL_TYPE_Q4_K && c->act_window == 256 && ntok >= c->gemm_min_tok &&
                       ntok <= 65535 * 4 && kGemmLdsBytes <= c->lds_limit && k / 256 <= 65535;
@@ -1436,8 +1517,13 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     if (e != hipSuccess)
         return bail(JL_ERR_HIP, "hipModuleLoad(" + path + "): " + H->GetErrorString(e));
 
-    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_multi_q4k_res", "jl_matvec_multi_q4k_x4_res", "jl_matvec_multi_q4k_q_res", "jl_matvec_multi_q8_0_res", "jl_matvec_multi_q8_0_x4_res", "jl_matvec_multi_q8_0_q_res", "jl_matvec_multi_q6k_res", "jl_matvec_multi_q6k_x4_res", "jl_matvec_multi_q6k_q_res", "jl_matvec_multi_q8_0p_res", "jl_matvec_multi_q8_0p_x4_res", "jl_matvec_multi_q8_0p_q_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q6k_r64", "jl_gemm_prep_w32", "jl_gemm_q8_0_w32", "jl_gemm_q6k_w32", "jl_gemm_q4k_w32", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few_t1", "jl_gemm_q4k_few_t2", "jl_gemm_q4k_few_t3", "jl_gemm_q4k_few_t4", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_group", "jl_moe_group2", "jl_moe_group2_wide", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_prep_q6k", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_g16q6_c1", "jl_moe_g16q6_c2", "jl_moe_g16q6_c3", "jl_moe_g16q6_f1", "jl_moe_g16q6_f2", "jl_moe_g16q6_f3", "jl_moe_g16q6_g1", "jl_moe_g16q6_g2", "jl_moe_g16q6_g3", "jl_moe_g16q6_d1", "jl_moe_g16q6_d2", "jl_moe_g16q6_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_moe_gemm_q6k_r64", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_fill_u32", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
+    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_multi_q4k_res", "jl_matvec_multi_q4k_x4_res", "jl_matvec_multi_q4k_q_res", "jl_matvec_multi_q8_0_res", "jl_matvec_multi_q8_0_x4_res", "jl_matvec_multi_q8_0_q_res", "jl_matvec_multi_q6k_res", "jl_matvec_multi_q6k_x4_res", "jl_matvec_multi_q6k_q_res", "jl_matvec_multi_q8_0p_res", "jl_matvec_multi_q8_0p_x4_res", "jl_matvec_multi_q8_0p_q_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q6k_r64", "jl_gemm_prep_w32", "jl_gemm_q8_0_w32", "jl_gemm_q6k_w32", "jl_gemm_q4k_w32", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_group", "jl_moe_group2", "jl_moe_group2_wide", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_prep_q6k", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_g16q6_c1", "jl_moe_g16q6_c2", "jl_moe_g16q6_c3", "jl_moe_g16q6_f1", "jl_moe_g16q6_f2", "jl_moe_g16q6_f3", "jl_moe_g16q6_g1", "jl_moe_g16q6_g2", "jl_moe_g16q6_g3", "jl_moe_g16q6_d1", "jl_moe_g16q6_d2", "jl_moe_g16q6_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_moe_gemm_q6k_r64", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_fill_u32", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
                                       "jl_pack_weights", "jl_unpack_q4k", "jl_unpack_q6k", "jl_unpack_q8_0"};
+    names.push_back("jl_few_prep");
+    for (const char* tag : {"q4k", "q4kw", "q8_0", "q6k", "q6kw"})
+        for (const char* layout : {"rows", "planes"})
+            for (const char* size : {"t1r1", "t1r2", "t2r1", "t4r1", "t4r2", "t1r4", "t2r2", "t2r4"})
+                if (layout[0] == 'p' || (strcmp(size, "t1r4") && strcmp(size, "t2r2") && strcmp(size, "t2r4"))) names.push_back(std::string("jl_few_") + tag + "_" + layout + "_" + size);
     for (const char* tag : {"q4k", "q8_0", "q6k"})
         for (int rw : {16, 32, 64})
             for (const char* form : {"", "q8_"})
@@ -1568,6 +1654,10 @@ int jl_set_tuning(jl_ctx* c, const char* key, int value) {
     else if (!strcmp(key, "gemm.split")) c->tune.gemm_split = value;
     else if (!strcmp(key, "gemm.prep")) c->tune.gemm_prep = value;
     else if (!strcmp(key, "gemm.planes")) c->tune.gemm_planes = value;
+    else if (!strcmp(key, "gemm.few")) c->tune.gemm_few = value;
+    else if (!strcmp(key, "few.nt")) c->tune.few_nt = value;
+    else if (!strcmp(key, "few.rt")) c->tune.few_rt = value;
+    else if (!strcmp(key, "few.waves")) c->tune.few_waves = value;
     else if (!strcmp(key, "gemm.min_tok")) c->gemm_min_tok = value > 0 ? value : 3;
     else return fail(c, JL_ERR_ARG, "unknown tuning key %s", key);
     return JL_OK;

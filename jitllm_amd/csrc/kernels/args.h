@@ -78,6 +78,42 @@ struct GemmArgs {
     int prow0 = 0, pstride = 0, psb0 = 0;
 };
 
+// Few tokens on the int8 matrix cores (kernels/few_i8.h).  The prep's layout, by chunk (128 of K) and slot
+// (16 columns): bq [chunk][slot][2 pairs of blocks][64 lanes][4 words] int8, da and ds [chunk][slot][16
+// columns][4 blocks] (the columns' scales, and scale * sum of the block's values; ds only where the
+// weights have minimums).
+struct FewI8PrepArgs {
+    const float* x;
+    const float* x2;        // null: plain activation, else silu(x) * x2
+    const uint32_t* src;    // null: column c reads row c
+    const uint32_t* start;  // null: one group, column c in slot c / 16
+    uint32_t* bq;
+    float* da;
+    float* ds;              // may be null
+    int k, per, ncols, n_expert, nslots, nch, order;
+    int isum;               // ds: the block sums themselves, as integers
+};
+#define JL_FEW_SC_BYTES 896   // a row tile's scales, and the header words on their way to them
+// a wavefront's LDS: scales, and over GGUF rows a staged super-block (ggml types 8, 12, 14)
+#define JL_FEW_WAVE_BYTES(type, planes, rt) \
+    ((rt) * (JL_FEW_SC_BYTES + ((planes) ? 0 : 16 * ((type) == 8 ? 272 : (type) == 12 ? 144 : 224))))
+#define JL_FEW_RED_BYTES(nw, nt, rt) ((nw) * 16 * (nt) * (16 * (rt) + 4) * 4)
+struct FewI8Args {
+    float* out[2];          // [column][nrows]; may be null when resid is set
+    const uint8_t* w[2];    // GGUF: sheets of sheet_bytes
+    const uint32_t* pqs[2];
+    const uint32_t* pd[2];
+    const uint32_t* psc[2];
+    float* resid;           // null, or resid[column][nrows] += the result
+    const uint32_t* bq;
+    const float* da;
+    const float* ds;
+    const uint32_t* start;  // null: one expert of ncols columns
+    size_t sheet_bytes, sheet_words;
+    int nrows, k, row_bytes, ncols, nslots, nch, nwaves;
+    int prow0, row_step, pstride;
+};
+
 // Mixture block on the matrix cores (Q4_K, activation window 256).  An expert's columns are
 // cut into groups of 32; group g of expert e has the workspace slot start[e]/32 + e + g
 // (distinct for distinct groups, below ncols/32 + n_expert + 1 = nslots).  The prep kernel

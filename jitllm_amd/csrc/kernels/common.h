@@ -20,6 +20,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // Loads of 2-byte-aligned block fields.  The amdhsa target runs with unaligned
 // global access enabled, so these lower to single wide loads.
 struct __attribute__((packed, aligned(2))) u32x4_a2 { u32x4 v; };
+struct __attribute__((packed, aligned(4))) u32x4_a4 { u32x4 v; };
 struct __attribute__((packed, aligned(2))) u32x2_a2 { u32x2 v; };
 struct __attribute__((packed, aligned(2))) u32_a2 { u32 v; };
 

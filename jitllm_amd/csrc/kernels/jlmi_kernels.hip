@@ -4,6 +4,7 @@
 // Entry points are extern "C" so the host can look them up by name.
 #include "common.h"
 #include "dequant.h"
+#include "few_i8.h"
 #include "gemm_q4k.h"
 #include "gemm_q4k_k2.h"
 #include "gemm_q4k_fold.h"
@@ -117,6 +118,25 @@ extern "C" __global__ __launch_bounds__(1024) void jl_matvec_segments(MatVecMult
     }
 }
 
+// -------------------------------------------------- few tokens, int8 matrix cores
+extern "C" __global__ __launch_bounds__(256) void jl_few_prep(FewI8PrepArgs p) { few_i8_prep_body(p); }
+// jl_few_<type>_<rows | planes>_t<token tiles>r<row tiles>: grid = (row tiles, experts, matrices)
+#define JL_FEW_KERNEL(T, TYPE, P, PL, NT, RT, W256)                                                             \
+    extern "C" __global__ __launch_bounds__(512) void jl_few_##T##_##P##_t##NT##r##RT(FewI8Args p) {            \
+        few_i8_body<TYPE, PL, NT, RT, W256>(p, jl_smem);                                                        \
+    }
+#define JL_FEW_SIZES(T, TYPE, P, PL, W256)                                                                      \
+    JL_FEW_KERNEL(T, TYPE, P, PL, 1, 1, W256) JL_FEW_KERNEL(T, TYPE, P, PL, 1, 2, W256)                         \
+    JL_FEW_KERNEL(T, TYPE, P, PL, 2, 1, W256) JL_FEW_KERNEL(T, TYPE, P, PL, 4, 1, W256)                         \
+    JL_FEW_KERNEL(T, TYPE, P, PL, 4, 2, W256)
+#define JL_FEW_WIDE(T, TYPE, W256)                                                                              \
+    JL_FEW_KERNEL(T, TYPE, planes, true, 1, 4, W256) JL_FEW_KERNEL(T, TYPE, planes, true, 2, 2, W256)           \
+    JL_FEW_KERNEL(T, TYPE, planes, true, 2, 4, W256)
+#define JL_FEW_FORMS(T, TYPE, W256)                                                                             \
+    JL_FEW_SIZES(T, TYPE, rows, false, W256) JL_FEW_SIZES(T, TYPE, planes, true, W256) JL_FEW_WIDE(T, TYPE, W256)
+JL_FEW_FORMS(q8_0, JL_Q8_0, false) JL_FEW_FORMS(q4k, JL_Q4_K, false) JL_FEW_FORMS(q6k, JL_Q6_K, false)
+JL_FEW_FORMS(q4kw, JL_Q4_K, true) JL_FEW_FORMS(q6kw, JL_Q6_K, true)   // (the k-quant window)
+
 // ---------------------------------------------------------- packed planes
 // grid = (ceil(nrows/256), k/256 or k/32 for Q8_0), block = 256
 extern "C" __global__ __launch_bounds__(256) void jl_pack_weights(PackArgs p) { pack_weights_body(p); }
@@ -158,13 +178,6 @@ JL_PACKED_MULTI_KERNEL(q6k, JL_Q6_K, 64, 4) JL_PACKED_MULTI_KERNEL(q6k, JL_Q6_K,
 
 // ------------------------------------------------------------ prefill GEMM
 // grid = (k/256, tok_pad/4), block = 256: one wavefront per (token, super-block)
-// few tokens: grid = ceil(nrows / 16), block = 512; _t<NT>: up to 16 NT tokens
-#define JL_GEMM_FEW_KERNEL(NT)                                                                     \
-    extern "C" __global__ __launch_bounds__(512) void jl_gemm_q4k_few_t##NT(GemmArgs p) {          \
-        __shared__ __attribute__((aligned(16))) float part[8 * NT * 256];                          \
-        gemm_q4k_few_body<NT>(p, part);                                                            \
-    }
-JL_GEMM_FEW_KERNEL(1) JL_GEMM_FEW_KERNEL(2) JL_GEMM_FEW_KERNEL(3) JL_GEMM_FEW_KERNEL(4)
 // some more tokens: grid = (ceil(nrows / 32), ceil(ntok / 64)), block = 512
 extern "C" __global__ __launch_bounds__(512) void jl_gemm_q4k_few32(GemmArgs p) {
     __shared__ __attribute__((aligned(16))) float part[8 * 2 * 1024];

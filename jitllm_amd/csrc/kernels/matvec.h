@@ -22,7 +22,6 @@
 #include "common.h"
 #include "quantize.h"
 
-struct __attribute__((packed, aligned(4))) u32x4_a4 { u32x4 v; };   // a 16-byte load on a 4-byte boundary
 
 // Activation staging area in LDS: int8 a[k], then f32 da[k/32], then f32 s16[k/16].
 struct ActLds {

@@ -1,0 +1,72 @@
+"""The int8 few-token matmul (up to 64 tokens) and the planes-to-rows kernels at the sizes where they can go
+wrong: one token and every edge of a token tile, rows that end inside a row tile, K of one super-block, K that
+ends inside a unit of 256 (Q8_0), more super-blocks than wavefronts, a row range of a larger plane set.  Bar:
+NMSE <= 1e-10 against the f64 evaluation of the same int8 activations."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import nmse
+from jitllm_amd import quant, synth
+from jitllm_amd.device import Packed
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 16, 256), (3, 37, 1280), (16, 100, 2816), (17, 130, 1024), (33, 48, 512), (64, 200, 2304), (5, 33, 160),
+          (20, 50, 320), (7, 64, 832)]
+# (token tiles, row tiles): the built-in choice and every compiled pair
+TILES = [(0, 0), (1, 1), (1, 2), (2, 1), (4, 1), (4, 2), (1, 4), (2, 2), (2, 4)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("window", [32, 256])
+@pytest.mark.parametrize("t", [quant.Q8_0, quant.Q4_K, quant.Q6_K], ids=["q8_0", "q4_k", "q6_k"])
+def test_few_tokens_rows_and_planes(dev, devbuf, t, window, shape):
+    ntok, nrows, k = shape
+    if k % quant.block_elems(t):
+        pytest.skip("K is not a whole number of this type's blocks")
+    dev.SetActWindow(window)
+    w = synth.random_weights(t, nrows, k, seed=ntok)
+    x = np.stack([synth.activations(k, seed=100 + i) * np.float32(1 + i % 7) for i in range(ntok)])
+    x[ntok // 2, :32] = 0
+    want = oracle.matmul_q8act_f64(t, w, x, nrows, k, ntok, window)
+    wd, xd = devbuf(w), devbuf(x)
+    planes = [devbuf(np.zeros(max(n, 4), np.uint32)) for n in quant.packed_words(t, nrows, k)]
+    assert dev.pack_weights_dev(t, wd.ptr, nrows, k, *[p.ptr for p in planes])
+    r0, part = 3, nrows - 7
+    try:
+        for nt, rt in TILES:
+            dev.set_tuning(gemm__few=1, few__nt=nt, few__rt=rt)
+            calls = [(True, 0, nrows), (True, r0, part)]
+            if nt < 4 and rt < 4 and (nt, rt) != (2, 2) or nt == 4:
+                calls.append((False, 0, nrows))
+            for packed, lo, n in calls:
+                out = devbuf(np.full(ntok * n + 8, 3e30, np.float32))
+                if packed:
+                    assert dev.matmul_packed_dev(out.ptr, t, Packed(*[p.ptr for p in planes], lo, nrows), xd.ptr, n, k, ntok)
+                else:
+                    assert dev.matmul_dev(out.ptr, t, wd.ptr, xd.ptr, n, k, ntok)
+                dev.synchronize()
+                got = out.get()
+                assert np.all(got[ntok * n:] == np.float32(3e30)), "wrote past the output"
+                e = nmse(got[:ntok * n].reshape(ntok, n), want[:, lo:lo + n])
+                assert e <= 1e-10, (nt, rt, packed, lo, e)
+    finally:
+        dev.set_tuning(gemm__few=0, few__nt=0, few__rt=0)
+        dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("t,nrows,k", [(quant.Q8_0, 65, 32), (quant.Q8_0, 130, 544), (quant.Q4_K, 63, 256), (quant.Q6_K, 129, 768),
+                                       (quant.MXFP4, 67, 96), (quant.MXFP4, 200, 800)])
+def test_planes_to_rows_round_trip(dev, devbuf, t, nrows, k):
+    src = synth.random_weights(t, nrows, k, seed=k)
+    wd = devbuf(src)
+    planes = [devbuf(np.zeros(max(n, 4), np.uint32)) for n in quant.packed_words(t, nrows, k)]
+    assert dev.pack_weights_dev(t, wd.ptr, nrows, k, *[p.ptr for p in planes])
+    rb = quant.row_bytes(t, k)
+    for lo, n in ((0, nrows), (1, nrows - 2), (nrows - 1, 1)):
+        dst = devbuf(np.full(n * rb + 32, 0xEE, np.uint8))
+        assert dev.unpack_weights_dev(t, Packed(*[p.ptr for p in planes], lo, nrows), n, k, dst.ptr)
+        dev.synchronize()
+        got = dst.get()
+        assert np.array_equal(got[:n * rb], src[lo * rb:(lo + n) * rb]) and np.all(got[n * rb:] == 0xEE)
