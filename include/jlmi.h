@@ -124,7 +124,8 @@ int jl_set_tuning(jl_ctx *ctx, const char *key, int value);
 
 /* Kernels this context has launched so far: how callers and tests check that a grouped
  * call was one launch, the point of the reference's grouped forms
- * (engine/nn/packedgroup.go:13-20). */
+ * (engine/nn/packedgroup.go:13-20).  The staging of a host-pointer call's operands and results is
+ * not counted. */
 unsigned long long jl_launch_count(const jl_ctx *ctx);
 
 /* Measurement only; no counterpart in the reference.  What a single launch costs on this

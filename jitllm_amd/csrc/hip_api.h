@@ -27,6 +27,8 @@ struct HipApi {
                                      unsigned, unsigned, hipStream_t, void**, void**) = nullptr;
     hipError_t (*Malloc)(void**, size_t) = nullptr;
     hipError_t (*Free)(void*) = nullptr;
+    hipError_t (*HostMalloc)(void**, size_t, unsigned) = nullptr;
+    hipError_t (*HostFree)(void*) = nullptr;
     hipError_t (*Memcpy)(void*, const void*, size_t, hipMemcpyKind) = nullptr;
     hipError_t (*MemcpyAsync)(void*, const void*, size_t, hipMemcpyKind, hipStream_t) = nullptr;
     hipError_t (*GetLastError)() = nullptr;
@@ -73,6 +75,8 @@ inline const HipApi* hip_api(std::string* why) {
             JL_SYM(ModuleLaunchKernel, "hipModuleLaunchKernel");
             JL_SYM(Malloc, "hipMalloc");
             JL_SYM(Free, "hipFree");
+            JL_SYM(HostMalloc, "hipHostMalloc");
+            JL_SYM(HostFree, "hipHostFree");
             JL_SYM(Memcpy, "hipMemcpy");
             JL_SYM(MemcpyAsync, "hipMemcpyAsync");
             JL_SYM(GetLastError, "hipGetLastError");

@@ -143,6 +143,12 @@ struct jl_ctx {
     void* stage_x = nullptr;    // device
     void* stage_out = nullptr;  // device
     size_t stage_x_bytes = 0, stage_out_bytes = 0;
+    // pinned host memory the small operands and results of a host-pointer call go through, and the word
+    // that is raised to the call's number when its results are in
+    void* pin = nullptr;
+    size_t pin_bytes = 0;
+    volatile uint32_t* pin_flag = nullptr;
+    uint32_t pin_number = 0;
 };
 
 namespace {
@@ -255,13 +261,14 @@ bool q8_pair_form(const jl_ctx* c, int type, const void* w, int k) {
            act_lds_bytes(k) + (size_t)k + 16 <= c->lds_limit;
 }
 
+// counted: whether jl_launch_count counts it (a host-pointer call's copies are not).
 int launch(jl_ctx* c, const char* name, unsigned gx, unsigned gy, unsigned block, unsigned lds,
-           hipStream_t st, void** params, unsigned gz = 1) {
+           hipStream_t st, void** params, unsigned gz = 1, bool counted = true) {
     auto it = c->fn.find(name);
     if (it == c->fn.end()) return fail(c, JL_ERR_ARG, "kernel %s is not in the code object", name);
     if (call_dry_run(c)) return JL_OK;
     HIP_TRY(c, H->ModuleLaunchKernel(it->second, gx, gy, gz, block, 1, 1, lds, st, params, nullptr));
-    c->launches++;
+    if (counted) c->launches++;
     return JL_OK;
 }
 
@@ -1517,7 +1524,7 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     if (e != hipSuccess)
         return bail(JL_ERR_HIP, "hipModuleLoad(" + path + "): " + H->GetErrorString(e));
 
-    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_multi_q4k_res", "jl_matvec_multi_q4k_x4_res", "jl_matvec_multi_q4k_q_res", "jl_matvec_multi_q8_0_res", "jl_matvec_multi_q8_0_x4_res", "jl_matvec_multi_q8_0_q_res", "jl_matvec_multi_q6k_res", "jl_matvec_multi_q6k_x4_res", "jl_matvec_multi_q6k_q_res", "jl_matvec_multi_q8_0p_res", "jl_matvec_multi_q8_0p_x4_res", "jl_matvec_multi_q8_0p_q_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q6k_r64", "jl_gemm_prep_w32", "jl_gemm_q8_0_w32", "jl_gemm_q6k_w32", "jl_gemm_q4k_w32", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_group", "jl_moe_group2", "jl_moe_group2_wide", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_prep_q6k", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_g16q6_c1", "jl_moe_g16q6_c2", "jl_moe_g16q6_c3", "jl_moe_g16q6_f1", "jl_moe_g16q6_f2", "jl_moe_g16q6_f3", "jl_moe_g16q6_g1", "jl_moe_g16q6_g2", "jl_moe_g16q6_g3", "jl_moe_g16q6_d1", "jl_moe_g16q6_d2", "jl_moe_g16q6_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_moe_gemm_q6k_r64", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_fill_u32", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
+    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_multi_q4k_res", "jl_matvec_multi_q4k_x4_res", "jl_matvec_multi_q4k_q_res", "jl_matvec_multi_q8_0_res", "jl_matvec_multi_q8_0_x4_res", "jl_matvec_multi_q8_0_q_res", "jl_matvec_multi_q6k_res", "jl_matvec_multi_q6k_x4_res", "jl_matvec_multi_q6k_q_res", "jl_matvec_multi_q8_0p_res", "jl_matvec_multi_q8_0p_x4_res", "jl_matvec_multi_q8_0p_q_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q6k_r64", "jl_gemm_prep_w32", "jl_gemm_q8_0_w32", "jl_gemm_q6k_w32", "jl_gemm_q4k_w32", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_group", "jl_moe_group2", "jl_moe_group2_wide", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_prep_q6k", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_g16q6_c1", "jl_moe_g16q6_c2", "jl_moe_g16q6_c3", "jl_moe_g16q6_f1", "jl_moe_g16q6_f2", "jl_moe_g16q6_f3", "jl_moe_g16q6_g1", "jl_moe_g16q6_g2", "jl_moe_g16q6_g3", "jl_moe_g16q6_d1", "jl_moe_g16q6_d2", "jl_moe_g16q6_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_moe_gemm_q6k_r64", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_fill_u32", "jl_host_in", "jl_host_done", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
                                       "jl_pack_weights", "jl_unpack_q4k", "jl_unpack_q6k", "jl_unpack_q8_0"};
     names.push_back("jl_few_prep");
     for (const char* tag : {"q4k", "q4kw", "q8_0", "q6k", "q6kw"})
@@ -1596,6 +1603,8 @@ void jl_ctx_destroy(jl_ctx* c) {
         if (kv.second.mem) (void)H->Free(kv.second.mem);
     if (c->one_group) (void)H->Free(c->one_group);
     if (c->mx_ws) (void)H->Free(c->mx_ws);
+    if (c->pin) (void)H->HostFree(c->pin);
+    if (c->pin_flag) (void)H->HostFree((void*)c->pin_flag);
     if (c->stage_x) (void)H->Free(c->stage_x);
     if (c->stage_out) (void)H->Free(c->stage_out);
     if (c->module) (void)H->ModuleUnload(c->module);
@@ -2546,42 +2555,6 @@ int jl_matmul_mxfp4_packed_bf16_dev(jl_ctx* c, float* out, const uint32_t* qs, c
 
 /* ------------------------------------------------------- host-pointer seam */
 
-int jl_matvec(jl_ctx* c, float* out, int type, const void* w, size_t wbytes, const float* x,
-              int nrows, int k) {
-    return jl_matmul(c, out, type, w, wbytes, x, nrows, k, 1);
-}
-
-int jl_matmul(jl_ctx* c, float* out, int type, const void* w, size_t wbytes, const float* x,
-              int nrows, int k, int ntok) {
-    if (!c) return JL_ERR_ARG;
-    CtxLock lock(c);
-    drain_forget(c);
-    if (c->no_device) return fail(c, JL_ERR_HIP, "this context is bound to no device");
-    const TypeInfo* ti = nullptr;
-    int rc = matvec_check(c, type, nrows, k, &ti);
-    if (rc != JL_OK) return rc;
-    if (!out || !w || !x || ntok <= 0) return fail(c, JL_ERR_ARG, "matmul: bad operand");
-    size_t need = (size_t)nrows * (size_t)(k / ti->block_elems) * ti->block_bytes;
-    if (wbytes < need)
-        return fail(c, JL_ERR_ARG, "matmul: weight has %zu bytes, %dx%d needs %zu", wbytes, nrows, k, need);
-    HIP_TRY(c, H->SetDevice(c->device));
-    void* wd = nullptr;
-    rc = resident_weight(c, w, need, &wd);
-    if (rc != JL_OK) return rc;
-    size_t xb = (size_t)ntok * k * 4, ob = (size_t)ntok * nrows * 4;
-    if ((rc = ensure_stage(c, &c->stage_x, &c->stage_x_bytes, xb)) != JL_OK) return rc;
-    if ((rc = ensure_stage(c, &c->stage_out, &c->stage_out_bytes, ob)) != JL_OK) return rc;
-    HIP_TRY(c, H->MemcpyAsync(c->stage_x, x, xb, hipMemcpyHostToDevice, c->stream));
-    rc = matmul_launch(c, (float*)c->stage_out, type, wd, (const float*)c->stage_x, nrows, k, ntok, c->stream);
-    if (rc != JL_OK) {
-        (void)H->StreamSynchronize(c->stream);
-        return rc;
-    }
-    HIP_TRY(c, H->MemcpyAsync(out, c->stage_out, ob, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, H->StreamSynchronize(c->stream));
-    return JL_OK;
-}
-
 namespace {
 // The three planes of a matrix in host memory as ONE device allocation keyed on the QS pointer
 // (uploaded on first use, jl_forget over the QS pointer releases it).  Called with c->mu held.
@@ -2614,13 +2587,156 @@ int resident_planes(jl_ctx* c, int type, const PlaneRef& host, int k, PlaneRef* 
     return JL_OK;
 }
 
-// Host floats -> the staging buffer at a float offset (the buffer is already large enough).
+// ---- a host-pointer call's operands and results.  Up to kPinMost bytes each way they go through pinned host
+// memory that kernels read and write in stream order, and the calling thread watches the word jl_host_done
+// raises behind them: no copy and no wait through the runtime, whose cost is latency (Q6_K 4096 x 4096 matvec
+// of 4.9 us on the device: 31 us a call with copies).  More than that, and whenever pinned memory is not to be
+// had, is copied.  Called with c->mu held, in this order: host_io_begin, stage_in for every operand,
+// host_io_go, the launches (which write the results to host_results()), host_out for every result, host_io_end.
+constexpr size_t kPinMost = (size_t)1 << 20;
+struct HostIo {
+    bool pinned = false;
+    size_t in_bytes = 0, out_bytes = 0;
+    struct Out { float* dst; size_t off, n; };
+    std::vector<Out> outs;
+};
+thread_local HostIo g_io;
+
+// Pinned memory of `need` bytes; *ok stays false where there is none to be had.
+int host_pin(jl_ctx* c, size_t need, bool* ok) {
+    if (!c->pin_flag) {
+        void* f = nullptr;
+        if (H->HostMalloc(&f, 256, hipHostMallocCoherent) != hipSuccess) { (void)H->GetLastError(); return JL_OK; }
+        memset(f, 0, 256);
+        c->pin_flag = (volatile uint32_t*)f;
+    }
+    if (c->pin_bytes < need) {   // (nothing of an earlier call is in flight: each ends when its results are in)
+        if (c->pin) {
+            HIP_TRY(c, H->StreamSynchronize(c->stream));
+            (void)H->HostFree(c->pin);
+        }
+        c->pin = nullptr;
+        c->pin_bytes = 0;
+        size_t want = (size_t)64 << 10;
+        while (want < need) want <<= 1;
+        if (H->HostMalloc(&c->pin, want, hipHostMallocCoherent) != hipSuccess) {
+            (void)H->GetLastError();
+            c->pin = nullptr;
+            return JL_OK;
+        }
+        c->pin_bytes = want;
+    }
+    *ok = true;
+    return JL_OK;
+}
+
+// Device staging for in_floats of operands (c->stage_x), a place for out_floats of results: pinned memory for
+// both, or device staging (c->stage_out).
+int host_io_begin(jl_ctx* c, size_t in_floats, size_t out_floats) {
+    HostIo& io = g_io;
+    io.outs.clear();
+    io.in_bytes = (in_floats * 4 + 255) & ~(size_t)255;
+    io.out_bytes = (out_floats * 4 + 255) & ~(size_t)255;
+    io.pinned = false;
+    int rc = ensure_stage(c, &c->stage_x, &c->stage_x_bytes, io.in_bytes);
+    if (rc != JL_OK) return rc;
+    if (io.in_bytes <= kPinMost && io.out_bytes <= kPinMost && (rc = host_pin(c, io.in_bytes + io.out_bytes, &io.pinned)) != JL_OK) return rc;
+    return io.pinned ? JL_OK : ensure_stage(c, &c->stage_out, &c->stage_out_bytes, io.out_bytes);
+}
+
+float* host_results(jl_ctx* c) { return g_io.pinned ? (float*)((char*)c->pin + g_io.in_bytes) : (float*)c->stage_out; }
+// Host floats -> the staging buffer at a float offset.
 int stage_in(jl_ctx* c, size_t off, const float* src, size_t n) {
+    if (g_io.pinned) {
+        memcpy((float*)c->pin + off, src, n * 4);
+        return JL_OK;
+    }
     HIP_TRY(c, H->MemcpyAsync((float*)c->stage_x + off, src, n * 4, hipMemcpyHostToDevice, c->stream));
     return JL_OK;
 }
+
+// The operands, where the launches find them.  read_once: every launch reads an operand's words once (the
+// activation prep of a matmul), so they can stay where the caller's were put; a decode matvec reads its
+// activation in every workgroup.
+int host_io_go(jl_ctx* c, const float** operands, bool read_once = false) {
+    *operands = g_io.pinned && read_once ? (const float*)c->pin : (const float*)c->stage_x;
+    if (!g_io.pinned || read_once) return JL_OK;
+    const void* src = c->pin;
+    void* dst = c->stage_x;
+    uint32_t n = (uint32_t)(g_io.in_bytes / 16);
+    void* pp[] = {&src, &dst, &n};
+    return launch(c, "jl_host_in", std::min(64u, (n + 255) / 256), 1, 256, 0, c->stream, pp, 1, false);
+}
+
+// A result that is updated in place in device memory (16-byte aligned, n rounded up to four floats readable).
+int host_result_copy(jl_ctx* c, size_t off, const float* src, size_t n) {
+    void* dst = host_results(c) + off;
+    uint32_t n4 = (uint32_t)((n + 3) / 4);
+    void* pp[] = {(void*)&src, &dst, &n4};
+    return launch(c, "jl_host_in", std::min(64u, (n4 + 255) / 256), 1, 256, 0, c->stream, pp, 1, false);
+}
+// A result: n floats at a float offset of host_results().
+void host_out(size_t off, float* dst, size_t n) { g_io.outs.push_back({dst, off, n}); }
+
+// Waits for the call's results and hands them over.  On an error of the call's (rc): waits for the stream.
+int host_io_end(jl_ctx* c, int rc) {
+    HostIo& io = g_io;
+    if (rc == JL_OK && io.pinned) {
+        uint32_t number = ++c->pin_number;
+        uint32_t* flag = (uint32_t*)c->pin_flag;
+        void* pp[] = {&flag, &number};
+        rc = launch(c, "jl_host_done", 1, 1, 64, 0, c->stream, pp, 1, false);
+        if (rc == JL_OK) {
+            // watch the word for a few milliseconds, then leave the wait (and any error) to the runtime
+            bool seen = false;
+            for (int i = 0; i < 200000 && !(seen = __atomic_load_n(flag, __ATOMIC_ACQUIRE) == number); i++) __builtin_ia32_pause();
+            if (!seen) HIP_TRY(c, H->StreamSynchronize(c->stream));
+            const float* r = host_results(c);
+            for (const HostIo::Out& o : io.outs) memcpy(o.dst, r + o.off, o.n * 4);
+            return JL_OK;
+        }
+    }
+    if (rc == JL_OK)
+        for (const HostIo::Out& o : io.outs)
+            HIP_TRY(c, H->MemcpyAsync(o.dst, (const float*)c->stage_out + o.off, o.n * 4, hipMemcpyDeviceToHost, c->stream));
+    hipError_t e = H->StreamSynchronize(c->stream);
+    if (rc == JL_OK && e != hipSuccess) return fail(c, JL_ERR_HIP, "stream: %s", H->GetErrorString(e));
+    return rc;
+}
 size_t up64(size_t n) { return (n + 63) & ~(size_t)63; }   // floats: keeps every staged vector 256-byte aligned
 }  // namespace
+
+int jl_matvec(jl_ctx* c, float* out, int type, const void* w, size_t wbytes, const float* x,
+              int nrows, int k) {
+    return jl_matmul(c, out, type, w, wbytes, x, nrows, k, 1);
+}
+
+int jl_matmul(jl_ctx* c, float* out, int type, const void* w, size_t wbytes, const float* x,
+              int nrows, int k, int ntok) {
+    if (!c) return JL_ERR_ARG;
+    CtxLock lock(c);
+    drain_forget(c);
+    if (c->no_device) return fail(c, JL_ERR_HIP, "this context is bound to no device");
+    const TypeInfo* ti = nullptr;
+    int rc = matvec_check(c, type, nrows, k, &ti);
+    if (rc != JL_OK) return rc;
+    if (!out || !w || !x || ntok <= 0) return fail(c, JL_ERR_ARG, "matmul: bad operand");
+    size_t need = (size_t)nrows * (size_t)(k / ti->block_elems) * ti->block_bytes;
+    if (wbytes < need)
+        return fail(c, JL_ERR_ARG, "matmul: weight has %zu bytes, %dx%d needs %zu", wbytes, nrows, k, need);
+    HIP_TRY(c, H->SetDevice(c->device));
+    void* wd = nullptr;
+    rc = resident_weight(c, w, need, &wd);
+    if (rc != JL_OK) return rc;
+    const size_t nx = (size_t)ntok * k, no = (size_t)ntok * nrows;
+    if ((rc = host_io_begin(c, nx, no)) != JL_OK) return rc;
+    rc = stage_in(c, 0, x, nx);
+    const float* xd = nullptr;
+    if (rc == JL_OK) rc = host_io_go(c, &xd, few_applies(c, type, false, nrows, k, ntok, 0));
+    if (rc == JL_OK) rc = matmul_launch(c, host_results(c), type, wd, xd, nrows, k, ntok, c->stream);
+    host_out(0, out, no);
+    return host_io_end(c, rc);
+}
 
 int jl_matvec_packed(jl_ctx* c, float* out, int type, const uint32_t* qs, const uint32_t* d,
                      const uint32_t* sc, int row, int stride, const float* x, int nrows, int k) {
@@ -2654,31 +2770,24 @@ int jl_matvec_packed_multi(jl_ctx* c, float* const* outs, int type, const uint32
         if (rc != JL_OK) return rc;
     }
     const size_t nx = xstride ? (size_t)(m - 1) * xstride + (size_t)k : (size_t)k, o_up = up64(nx);
-    int rc = ensure_stage(c, &c->stage_x, &c->stage_x_bytes, (o_up + (up ? nx : 0)) * 4);
-    if (rc != JL_OK) return rc;
     const size_t orow = up64((size_t)nrows);
-    if ((rc = ensure_stage(c, &c->stage_out, &c->stage_out_bytes, (size_t)m * orow * 4)) != JL_OK) return rc;
-    if ((rc = stage_in(c, 0, x, nx)) != JL_OK) return rc;
-    if (up && (rc = stage_in(c, o_up, up, nx)) != JL_OK) return rc;
-    const float* xd = (const float*)c->stage_x;
+    int rc = host_io_begin(c, o_up + (up ? nx : 0), (size_t)m * orow);
+    if (rc != JL_OK) return rc;
+    rc = stage_in(c, 0, x, nx);
+    if (rc == JL_OK && up) rc = stage_in(c, o_up, up, nx);
+    const float* xd = nullptr;
+    if (rc == JL_OK) rc = host_io_go(c, &xd);
     const float* ud = up ? xd + o_up : nullptr;
-    for (int j0 = 0; j0 < m; j0 += JL_MAX_MULTI) {   // sixteen matrices a launch
+    for (int j0 = 0; j0 < m && rc == JL_OK; j0 += JL_MAX_MULTI) {   // sixteen matrices a launch
         const int n = std::min(m - j0, (int)JL_MAX_MULTI);
         float* od[JL_MAX_MULTI];
-        for (int j = 0; j < n; j++) od[j] = (float*)c->stage_out + (size_t)(j0 + j) * orow;
+        for (int j = 0; j < n; j++) od[j] = host_results(c) + (size_t)(j0 + j) * orow;
         rc = packed_matvec_multi_launch(c, type, n, od, &pls[(size_t)j0], xd + (size_t)j0 * xstride, xstride,
                                         ud ? ud + (size_t)j0 * xstride : nullptr, nullptr, 0.f, nullptr, nullptr, 0.f,
                                         nullptr, nrows, k, c->stream);
-        if (rc != JL_OK) {
-            (void)H->StreamSynchronize(c->stream);
-            return rc;
-        }
     }
-    for (int j = 0; j < m; j++)
-        HIP_TRY(c, H->MemcpyAsync(outs[j], (float*)c->stage_out + (size_t)j * orow, (size_t)nrows * 4,
-                                  hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, H->StreamSynchronize(c->stream));
-    return JL_OK;
+    for (int j = 0; j < m; j++) host_out((size_t)j * orow, outs[j], (size_t)nrows);
+    return host_io_end(c, rc);
 }
 
 int jl_moe_grouped(jl_ctx* c, float* resid, int type, const void* gate_bank, const void* up_bank,
@@ -2706,21 +2815,20 @@ int jl_moe_grouped(jl_ctx* c, float* resid, int type, const void* gate_bank, con
     // staged as floats: x, resid, wt, then the selections (32-bit words as well)
     const size_t nx = (size_t)rows * n_embd, o_res = up64(nx), o_wt = o_res + up64(nx),
                  o_sel = o_wt + up64((size_t)rows * k_used), total = o_sel + up64((size_t)rows * sel_stride);
-    if ((rc = ensure_stage(c, &c->stage_x, &c->stage_x_bytes, total * 4)) != JL_OK) return rc;
-    if ((rc = stage_in(c, 0, x, nx)) != JL_OK) return rc;
-    if ((rc = stage_in(c, o_res, resid, nx)) != JL_OK) return rc;
-    if ((rc = stage_in(c, o_wt, wt, (size_t)rows * k_used)) != JL_OK) return rc;
-    if ((rc = stage_in(c, o_sel, (const float*)sel, (size_t)rows * sel_stride)) != JL_OK) return rc;
+    if ((rc = host_io_begin(c, total, nx)) != JL_OK) return rc;
+    rc = stage_in(c, 0, x, nx);
+    if (rc == JL_OK) rc = stage_in(c, o_res, resid, nx);
+    if (rc == JL_OK) rc = stage_in(c, o_wt, wt, (size_t)rows * k_used);
+    if (rc == JL_OK) rc = stage_in(c, o_sel, (const float*)sel, (size_t)rows * sel_stride);
+    const float* xd = nullptr;
+    if (rc == JL_OK) rc = host_io_go(c, &xd);
     float* base = (float*)c->stage_x;
-    rc = moe_ffn(c, base + o_res, type, type, gd, ud, dd, nullptr, nullptr, nullptr, base, (const uint32_t*)(base + o_sel),
+    if (rc == JL_OK)
+        rc = moe_ffn(c, base + o_res, type, type, gd, ud, dd, nullptr, nullptr, nullptr, base, (const uint32_t*)(base + o_sel),
                  sel_stride, base + o_wt, rows, k_used, n_expert, n_ffn, n_embd, c->stream);
-    if (rc != JL_OK) {
-        (void)H->StreamSynchronize(c->stream);
-        return rc;
-    }
-    HIP_TRY(c, H->MemcpyAsync(resid, base + o_res, nx * 4, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, H->StreamSynchronize(c->stream));
-    return JL_OK;
+    if (rc == JL_OK) rc = host_result_copy(c, 0, base + o_res, nx);
+    host_out(0, resid, nx);
+    return host_io_end(c, rc);
 }
 
 int jl_matvec_packed_group(jl_ctx* c, int n, float* const* outs, const int* types, const uint32_t* const* qs,
@@ -2752,38 +2860,34 @@ int jl_matvec_packed_group(jl_ctx* c, int n, float* const* outs, const int* type
     }
     // staged: x, the gate's partner, the residual (matrix 0's rows)
     const size_t o_up = up64((size_t)k), o_res = o_up + (act_up ? up64((size_t)k) : 0);
-    int rc = ensure_stage(c, &c->stage_x, &c->stage_x_bytes, (o_res + (resid ? up64((size_t)rows[0]) : 0)) * 4);
-    if (rc != JL_OK) return rc;
     size_t o_out[JL_MAX_GROUP], total = 0;
     for (int i = 0; i < n; i++) { o_out[i] = total; total += up64((size_t)rows[i]); }
-    if ((rc = ensure_stage(c, &c->stage_out, &c->stage_out_bytes, total * 4)) != JL_OK) return rc;
-    if ((rc = stage_in(c, 0, x, (size_t)k)) != JL_OK) return rc;
-    if (act_up && (rc = stage_in(c, o_up, act_up, (size_t)k)) != JL_OK) return rc;
-    if (resid && (rc = stage_in(c, o_res, resid, (size_t)rows[0])) != JL_OK) return rc;
-    const float* xd = (const float*)c->stage_x;
+    const size_t o_rd = total;   // the updated residual comes behind the outputs
+    if (resid) total += up64((size_t)rows[0]);
+    int rc = host_io_begin(c, o_res + (resid ? up64((size_t)rows[0]) : 0), total);
+    if (rc != JL_OK) return rc;
+    rc = stage_in(c, 0, x, (size_t)k);
+    if (rc == JL_OK && act_up) rc = stage_in(c, o_up, act_up, (size_t)k);
+    if (rc == JL_OK && resid) rc = stage_in(c, o_res, resid, (size_t)rows[0]);
+    const float* xd = nullptr;
+    if (rc == JL_OK) rc = host_io_go(c, &xd);
     const float* ud = act_up ? xd + o_up : nullptr;
     float* rd = resid ? (float*)c->stage_x + o_res : nullptr;
     // matrices of one type and row count that follow one another share a launch (a block's gate
     // and up); the residual rides on matrix 0 (MVGroup.Resid, packedgroup.go:32-36)
-    for (int i = 0; i < n;) {
+    for (int i = 0; i < n && rc == JL_OK;) {
         int e = i + 1;
         while (e < n && types[e] == types[i] && rows[e] == rows[i] && pls[e].stride == pls[i].stride) e++;
         float* od[JL_MAX_GROUP];
-        for (int j = i; j < e; j++) od[j - i] = (float*)c->stage_out + o_out[j];
+        for (int j = i; j < e; j++) od[j - i] = host_results(c) + o_out[j];
         rc = packed_matvec_multi_launch(c, types[i], e - i, od, &pls[i], xd, 0, ud, i == 0 ? rd : nullptr, alpha, nullptr,
                                         nullptr, 0.f, nullptr, rows[i], k, c->stream);
-        if (rc != JL_OK) {
-            (void)H->StreamSynchronize(c->stream);
-            return rc;
-        }
         i = e;
     }
-    for (int i = 0; i < n; i++)
-        HIP_TRY(c, H->MemcpyAsync(outs[i], (float*)c->stage_out + o_out[i], (size_t)rows[i] * 4, hipMemcpyDeviceToHost,
-                                  c->stream));
-    if (resid) HIP_TRY(c, H->MemcpyAsync(resid, rd, (size_t)rows[0] * 4, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, H->StreamSynchronize(c->stream));
-    return JL_OK;
+    if (rc == JL_OK && resid) rc = host_result_copy(c, o_rd, rd, (size_t)rows[0]);
+    if (resid) host_out(o_rd, resid, (size_t)rows[0]);
+    for (int i = 0; i < n; i++) host_out(o_out[i], outs[i], (size_t)rows[i]);
+    return host_io_end(c, rc);
 }
 
 int jl_matmul_packed(jl_ctx* c, float* out, int type, const uint32_t* qs, const uint32_t* d,
@@ -2800,21 +2904,17 @@ int jl_matmul_packed(jl_ctx* c, float* out, int type, const uint32_t* qs, const 
     HIP_TRY(c, H->SetDevice(c->device));
     PlaneRef pl;
     if ((rc = resident_planes(c, type, host, k, &pl)) != JL_OK) return rc;
-    size_t xb = (size_t)ntok * k * 4, ob = (size_t)ntok * nrows * 4;
-    if ((rc = ensure_stage(c, &c->stage_x, &c->stage_x_bytes, xb)) != JL_OK) return rc;
-    if ((rc = ensure_stage(c, &c->stage_out, &c->stage_out_bytes, ob)) != JL_OK) return rc;
-    HIP_TRY(c, H->MemcpyAsync(c->stage_x, x, xb, hipMemcpyHostToDevice, c->stream));
-    rc = ntok == 1 ? packed_matvec_launch(c, (float*)c->stage_out, type, pl, (const float*)c->stage_x, nullptr,
+    const size_t nx = (size_t)ntok * k, no = (size_t)ntok * nrows;
+    if ((rc = host_io_begin(c, nx, no)) != JL_OK) return rc;
+    rc = stage_in(c, 0, x, nx);
+    const float* xd = nullptr;
+    if (rc == JL_OK) rc = host_io_go(c, &xd, few_applies(c, type, true, nrows, k, ntok, pl.stride));
+    if (rc == JL_OK) rc = ntok == 1 ? packed_matvec_launch(c, host_results(c), type, pl, xd, nullptr,
                                           nullptr, nullptr, nrows, k, c->stream)
-                   : packed_matmul_launch(c, (float*)c->stage_out, type, pl, (const float*)c->stage_x, nrows, k,
+                   : packed_matmul_launch(c, host_results(c), type, pl, xd, nrows, k,
                                           ntok, c->stream);
-    if (rc != JL_OK) {
-        (void)H->StreamSynchronize(c->stream);
-        return rc;
-    }
-    HIP_TRY(c, H->MemcpyAsync(out, c->stage_out, ob, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, H->StreamSynchronize(c->stream));
-    return JL_OK;
+    host_out(0, out, no);
+    return host_io_end(c, rc);
 }
 
 int jl_forget(jl_ctx* c, const void* p, size_t n) {

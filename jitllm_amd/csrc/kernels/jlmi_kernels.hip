@@ -452,6 +452,20 @@ extern "C" __global__ __launch_bounds__(256) void jl_fill_u32(u32* __restrict__ 
     if (i < n) dst[i] = value;
 }
 
+// ------------------------------------------------- host-pointer calls: operands and results
+// A host-pointer call's activations and results are tens of kilobytes: what a copy through the runtime costs
+// (two pageable copies and a stream wait: 31 us round a 5 us matvec) is latency, not bytes.  jl_host_in copies
+// the operands from pinned host memory, 16 bytes a lane, in stream order with the matrix work; results are
+// stored to pinned host memory by the kernels that make them, and jl_host_done behind them raises the call's
+// number there, which the calling thread watches.  (A kernel that copied the results out and raised the number
+// itself took 4.7 us for 16 KB; this one takes an empty launch.)
+extern "C" __global__ __launch_bounds__(256) void jl_host_in(const u32x4* __restrict__ src, u32x4* __restrict__ dst, u32 n) {
+    for (u32 i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) dst[i] = src[i];
+}
+extern "C" __global__ __launch_bounds__(64) void jl_host_done(u32* flag, u32 number) {
+    if (threadIdx.x == 0) __hip_atomic_store(flag, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ------------------------------------------------------------------ probes
 // What one launch costs on this machine before any arithmetic: jl_probe_read streams nvec
 // 16-byte vectors with every thread keeping eight loads in flight and folds them into a word
