@@ -1524,7 +1524,7 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     if (e != hipSuccess)
         return bail(JL_ERR_HIP, "hipModuleLoad(" + path + "): " + H->GetErrorString(e));
 
-    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_multi_q4k_res", "jl_matvec_multi_q4k_x4_res", "jl_matvec_multi_q4k_q_res", "jl_matvec_multi_q8_0_res", "jl_matvec_multi_q8_0_x4_res", "jl_matvec_multi_q8_0_q_res", "jl_matvec_multi_q6k_res", "jl_matvec_multi_q6k_x4_res", "jl_matvec_multi_q6k_q_res", "jl_matvec_multi_q8_0p_res", "jl_matvec_multi_q8_0p_x4_res", "jl_matvec_multi_q8_0p_q_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q6k_r64", "jl_gemm_prep_w32", "jl_gemm_q8_0_w32", "jl_gemm_q6k_w32", "jl_gemm_q4k_w32", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_group", "jl_moe_group2", "jl_moe_group2_wide", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_prep_q6k", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_g16q6_c1", "jl_moe_g16q6_c2", "jl_moe_g16q6_c3", "jl_moe_g16q6_f1", "jl_moe_g16q6_f2", "jl_moe_g16q6_f3", "jl_moe_g16q6_g1", "jl_moe_g16q6_g2", "jl_moe_g16q6_g3", "jl_moe_g16q6_d1", "jl_moe_g16q6_d2", "jl_moe_g16q6_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_moe_gemm_q6k_r64", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_fill_u32", "jl_host_in", "jl_host_done", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
+    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_multi_q4k_res", "jl_matvec_multi_q4k_x4_res", "jl_matvec_multi_q4k_q_res", "jl_matvec_multi_q8_0_res", "jl_matvec_multi_q8_0_x4_res", "jl_matvec_multi_q8_0_q_res", "jl_matvec_multi_q6k_res", "jl_matvec_multi_q6k_x4_res", "jl_matvec_multi_q6k_q_res", "jl_matvec_multi_q8_0p_res", "jl_matvec_multi_q8_0p_x4_res", "jl_matvec_multi_q8_0p_q_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q6k_r64", "jl_gemm_prep_w32", "jl_gemm_q8_0_w32", "jl_gemm_q6k_w32", "jl_gemm_q4k_w32", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_group", "jl_moe_group2", "jl_moe_group2_wide", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_prep_q6k", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_g16q6_c1", "jl_moe_g16q6_c2", "jl_moe_g16q6_c3", "jl_moe_g16q6_f1", "jl_moe_g16q6_f2", "jl_moe_g16q6_f3", "jl_moe_g16q6_g1", "jl_moe_g16q6_g2", "jl_moe_g16q6_g3", "jl_moe_g16q6_d1", "jl_moe_g16q6_d2", "jl_moe_g16q6_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_moe_gemm_q6k_r64", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_silu_mul", "jl_add_rows", "jl_host_in", "jl_host_done", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
                                       "jl_pack_weights", "jl_unpack_q4k", "jl_unpack_q6k", "jl_unpack_q8_0"};
     names.push_back("jl_few_prep");
     for (const char* tag : {"q4k", "q4kw", "q8_0", "q6k", "q6kw"})
@@ -2094,6 +2094,55 @@ int moe_ws(jl_ctx* c, int rows, int k_used, int n_expert, int n_ffn, int n_embd,
     return JL_OK;
 }
 
+// "moe.form" asks for one of the mixture's own kernels
+bool moe_dense_wanted(const jl_ctx* c) { return c->tune.moe_form == 0; }
+
+// A dense gated feed-forward block for n rows: y = W_down (silu(W_gate x) * W_up x), resid[r] += wt[r] * y[r]
+// (wt null: 1).  g, u: n n_ffn floats each, y: n n_embd.  Up to 64 rows two few-token matmuls -- gate and up in one
+// launch, the gated activation formed by down's activation prep, the residual added where the result is made
+// when its weight is one -- and above that three prefill GEMMs: nothing is routed, so nothing of the mixture's
+// grouping, work lists and column gathers is needed.  (As a mixture of one expert: Q4_K 3584 / 13056 over
+// planes, 34 rows 194 us, Q4_K 1536 / 3328, 17 rows 88 us.)  JL_DECLINED when a matmul has no such form.
+int dense_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate, const void* up, const void* down,
+              const PlaneRef* pg, const PlaneRef* pu, const PlaneRef* pd, const float* x, const float* wt, int n, int n_ffn,
+              int n_embd, float* g, float* u, float* y, hipStream_t st) {
+    const bool planes = pg != nullptr;
+    auto few = [&](int t, const void* w, const PlaneRef* p, int nrows, int k) {
+        return n <= 64 && few_fits(c, t, planes, nrows, k, n, planes ? p->stride : 0) && (planes || ((uintptr_t)w & (t == JL_TYPE_Q4_K ? 15 : 3)) == 0);
+    };
+    int rc;
+    if (n > 65535 || n_embd % 4 || n_ffn % 4) return JL_DECLINED;
+    if (few(type, gate, pg, n_ffn, n_embd) && few(type, up, pu, n_ffn, n_embd) && (!planes || (pg->row == pu->row && pg->stride == pu->stride))) {
+        FewCall f;
+        f.type = type; f.nrows = n_ffn; f.k = n_embd; f.ncols = n; f.nmat = 2; f.x = x;
+        f.w[0] = gate; f.w[1] = up; f.pl[0] = pg; f.pl[1] = pu; f.out[0] = g; f.out[1] = u;
+        rc = few_launch(c, f, st);
+    } else {
+        rc = planes ? packed_matmul_launch(c, g, type, *pg, x, n_ffn, n_embd, n, st) : matmul_launch(c, g, type, gate, x, n_ffn, n_embd, n, st);
+        if (rc == JL_OK)
+            rc = planes ? packed_matmul_launch(c, u, type, *pu, x, n_ffn, n_embd, n, st) : matmul_launch(c, u, type, up, x, n_ffn, n_embd, n, st);
+    }
+    if (rc != JL_OK) return rc;
+    if (few(down_type, down, pd, n_embd, n_ffn)) {
+        FewCall f;
+        f.type = down_type; f.nrows = n_embd; f.k = n_ffn; f.ncols = n; f.x = g; f.x2 = u;
+        f.w[0] = down; f.pl[0] = pd;
+        if (wt) f.out[0] = y; else f.resid = resid;
+        rc = few_launch(c, f, st);
+        if (rc != JL_OK || !wt) return rc;
+    } else {
+        size_t nh = (size_t)n * n_ffn;
+        void* ap[] = {&g, &u, &nh};
+        rc = launch(c, "jl_silu_mul", (unsigned)((nh / 4 + 255) / 256), 1, 256, 0, st, ap);
+        if (rc == JL_OK)
+            rc = planes ? packed_matmul_launch(c, y, down_type, *pd, g, n_embd, n_ffn, n, st)
+                        : matmul_launch(c, y, down_type, down, g, n_embd, n_ffn, n, st);
+        if (rc != JL_OK) return rc;
+    }
+    void* rp[] = {&resid, &y, (void*)&wt, &n_embd};
+    return launch(c, "jl_add_rows", (unsigned)((n_embd / 4 + 255) / 256), (unsigned)n, 256, 0, st, rp);
+}
+
 int moe_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate_bank, const void* up_bank,
             const void* down_bank, const jl_packed_bank* pg, const jl_packed_bank* pu, const jl_packed_bank* pd,
             const float* x, const uint32_t* sel, int sel_stride, const float* wt, int rows, int k_used, int n_expert,
@@ -2110,6 +2159,17 @@ int moe_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate_b
     if (rc != JL_OK) return rc;
     uint32_t *start = w.start, *perm = w.perm, *pos = w.pos;
     float *g = w.g, *u = w.u, *y = w.y;
+    // one expert: every row is its column, nothing to group
+    if (n_expert == 1 && k_used == 1 && (!pg || (!pg->sheet_bytes && !pu->sheet_bytes && !pd->sheet_bytes)) && moe_dense_wanted(c)) {
+        PlaneRef a{}, b{}, d{};
+        if (pg) {
+            a = PlaneRef{pg->qs, pg->d, pg->sc, 0, pg->stride}; b = PlaneRef{pu->qs, pu->d, pu->sc, 0, pu->stride};
+            d = PlaneRef{pd->qs, pd->d, pd->sc, 0, pd->stride};
+        }
+        rc = dense_ffn(c, resid, type, down_type, gate_bank, up_bank, down_bank, pg ? &a : nullptr, pg ? &b : nullptr, pg ? &d : nullptr,
+                       x, wt, rows, n_ffn, n_embd, g, u, y, st);
+        if (rc != JL_DECLINED) return rc;
+    }
     rc = jl_moe_group_dev(c, sel, sel_stride, rows, k_used, n_expert, start, perm, pos, st);
     if (rc != JL_OK) return rc;
     // gate and up: columns read the routed rows of x
@@ -2332,24 +2392,14 @@ int jl_layer_ffn_dev(jl_ctx* c, int li, const float* h, float* resid, int n, voi
         return moe_block(c, resid, P.type, P.down_type, L.gate, L.up, L.down, P.packed ? &bg : nullptr, P.packed ? &bu : nullptr,
                          P.packed ? &bd : nullptr, JL_TYPE_F32, L.router, h, n, P.k_used, P.n_expert, F, E, nullptr, nullptr, st);
     }
-    // dense.  More than one row without a norm in front: the grouped kernels, the block as a
-    // mixture of one expert that every row selects with weight 1.
-    if (n > 1 && !L.norm_w && F % 256 == 0 && E % 256 == 0 && (!P.packed || P.type == P.down_type)) {
-        const size_t o_wt = up256((size_t)n * 2 * 4);
-        int rc = grow(c, &c->layer_ws, &c->layer_ws_bytes, o_wt + up256((size_t)n * 4));
+    // dense, more than one row without a norm in front: as matmuls
+    if (n > 1 && !L.norm_w && moe_dense_wanted(c)) {
+        MoeWs w;
+        int rc = moe_ws(c, n, 1, 1, F, E, &w);
         if (rc != JL_OK) return rc;
-        uint32_t* sel = (uint32_t*)c->layer_ws;
-        float* wt = (float*)((char*)c->layer_ws + o_wt);
-        size_t n_sel = (size_t)n * 2, n_wt = (size_t)n;
-        uint32_t zero = 0, one = 0x3F800000u;
-        void* p0[] = {&sel, &n_sel, &zero};
-        rc = launch(c, "jl_fill_u32", (unsigned)((n_sel + 255) / 256), 1, 256, 0, st, p0);
-        if (rc != JL_OK) return rc;
-        void* p1[] = {&wt, &n_wt, &one};
-        rc = launch(c, "jl_fill_u32", (unsigned)((n_wt + 255) / 256), 1, 256, 0, st, p1);
-        if (rc != JL_OK) return rc;
-        rc = moe_ffn(c, resid, P.type, P.down_type, L.gate, L.up, L.down, P.packed ? &bg : nullptr, P.packed ? &bu : nullptr,
-                     P.packed ? &bd : nullptr, h, sel, 2, wt, n, 1, 1, F, E, st);
+        const PlaneRef a = {L.gp[0], L.gp[1], L.gp[2], 0, F}, b = {L.upl[0], L.upl[1], L.upl[2], 0, F}, d = {L.dp[0], L.dp[1], L.dp[2], 0, E};
+        rc = dense_ffn(c, resid, P.type, P.down_type, L.gate, L.up, L.down, P.packed ? &a : nullptr, P.packed ? &b : nullptr,
+                       P.packed ? &d : nullptr, h, nullptr, n, F, E, w.g, w.u, w.y, st);
         if (rc != JL_DECLINED) return rc;
     }
     // one row at a time: gate and up in one launch (the norm riding in front), down over

@@ -447,9 +447,24 @@ extern "C" __global__ __launch_bounds__(256) void jl_q4k_fold_range(FoldRangeArg
     if (!(d * 945.f + dmin * 63.f <= 65504.f)) atomicOr(a.flag, 1u);
 }
 
-extern "C" __global__ __launch_bounds__(256) void jl_fill_u32(u32* __restrict__ dst, size_t n, u32 value) {
+// A dense feed-forward block's pieces between its prefill GEMMs: g = silu(g) * u, n a multiple of four;
+// resid[r] += wt[r] * y[r] (wt null: 1), grid = (ceil(n_embd / 4 / 256), rows).
+extern "C" __global__ __launch_bounds__(256) void jl_silu_mul(float* __restrict__ g, const float* __restrict__ u, size_t n) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) dst[i] = value;
+    if (i * 4 >= n) return;
+    const f32x4 a = ((const f32x4*)g)[i], b = ((const f32x4*)u)[i];
+    ((f32x4*)g)[i] = f32x4{silu_f32(a.x) * b.x, silu_f32(a.y) * b.y, silu_f32(a.z) * b.z, silu_f32(a.w) * b.w};
+}
+extern "C" __global__ __launch_bounds__(256) void jl_add_rows(float* __restrict__ resid, const float* __restrict__ y,
+                                                              const float* __restrict__ wt, int n_embd) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i * 4 >= n_embd) return;
+    const size_t o = (size_t)blockIdx.y * n_embd / 4 + i;
+    const float w = wt ? wt[blockIdx.y] : 1.0f;
+    const f32x4 v = ((const f32x4*)y)[o];
+    f32x4 r = ((f32x4*)resid)[o];
+    r.x += w * v.x; r.y += w * v.y; r.z += w * v.z; r.w += w * v.w;
+    ((f32x4*)resid)[o] = r;
 }
 
 // ------------------------------------------------- host-pointer calls: operands and results
