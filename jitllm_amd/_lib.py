@@ -6,6 +6,13 @@ loading raises, and so does every operator built on it.
 import ctypes as C
 import os
 
+from . import quant
+try:
+    from . import _calls
+except ImportError as e:
+    raise ImportError("jitllm_amd/_calls.so is missing: build it with `make -C jitllm_amd/csrc` "
+                      "(or __graft_entry__.build()); there is no fallback path") from e
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libjlmi.so")
 CODE_OBJECT_PATH = os.path.join(_HERE, "jlmi_gfx950.hsaco")
@@ -144,5 +151,6 @@ def load():
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.restype, fn.argtypes = res, args
+        _calls.bind({n: C.cast(getattr(lib, n), C.c_void_p).value for n in SIGNATURES}, quant.BLOCK, PackedBank)
         _lib = lib
     return _lib

@@ -57,6 +57,65 @@ struct Tuning {
     int mx_split = 0;
 };
 
+// The code object's kernels by name.  Looked up on every launch, so without a string to allocate or a tree to
+// walk: open addressing over the names' hashes.
+struct KernelTable {
+    struct Slot { uint64_t hash = 0; std::string name; hipFunction_t fn = nullptr; };
+    std::vector<Slot> slots;
+    size_t used = 0;
+    static uint64_t hash_of(const char* s) {
+        uint64_t h = 1469598103934665603ull;   // FNV-1a
+        for (; *s; s++) h = (h ^ (uint8_t)*s) * 1099511628211ull;
+        return h ? h : 1;
+    }
+    hipFunction_t find(const char* name) const {
+        if (slots.empty()) return nullptr;
+        const uint64_t h = hash_of(name);
+        for (size_t i = h & (slots.size() - 1); slots[i].hash; i = (i + 1) & (slots.size() - 1))
+            if (slots[i].hash == h && slots[i].name == name) return slots[i].fn;
+        return nullptr;
+    }
+    void add(const std::string& name, hipFunction_t fn) {
+        if (2 * (used + 1) > slots.size()) {
+            std::vector<Slot> old(slots.empty() ? 64 : 2 * slots.size());
+            old.swap(slots);
+            used = 0;
+            for (const Slot& o : old)
+                if (o.hash) add(o.name, o.fn);
+        }
+        const uint64_t h = hash_of(name.c_str());
+        size_t i = h & (slots.size() - 1);
+        while (slots[i].hash && slots[i].name != name) i = (i + 1) & (slots.size() - 1);
+        if (!slots[i].hash) used++;
+        slots[i] = Slot{h, name, fn};
+    }
+};
+
+// A kernel's name put together from its parts.
+struct Name {
+    char s[64];
+    unsigned n = 0;
+    Name() { s[0] = 0; }
+    Name& operator<<(const char* p) {
+        while (*p && n < sizeof s - 1) s[n++] = *p++;
+        s[n] = 0;
+        return *this;
+    }
+    Name& operator<<(char ch) {
+        const char t[2] = {ch, 0};
+        return *this << t;
+    }
+    Name& operator<<(int v) {
+        char t[12];
+        int i = 11;
+        t[i] = 0;
+        do t[--i] = (char)('0' + v % 10);
+        while ((v /= 10) && i > 0);
+        return *this << (t + i);
+    }
+    operator const char*() const { return s; }
+};
+
 struct Resident {
     void* dev = nullptr;
     size_t bytes = 0;
@@ -82,7 +141,7 @@ struct jl_ctx {
     int act_window = 32;
     hipStream_t stream = nullptr;
     hipModule_t module = nullptr;
-    std::map<std::string, hipFunction_t> fn;
+    KernelTable fn;
     std::string err;
     std::mutex mu;  // serialises the host-pointer seam (one staging area per context)
     std::atomic<std::thread::id> mu_owner{};   // the thread inside mu (jl_forget must not try it again)
@@ -264,10 +323,10 @@ bool q8_pair_form(const jl_ctx* c, int type, const void* w, int k) {
 // counted: whether jl_launch_count counts it (a host-pointer call's copies are not).
 int launch(jl_ctx* c, const char* name, unsigned gx, unsigned gy, unsigned block, unsigned lds,
            hipStream_t st, void** params, unsigned gz = 1, bool counted = true) {
-    auto it = c->fn.find(name);
-    if (it == c->fn.end()) return fail(c, JL_ERR_ARG, "kernel %s is not in the code object", name);
+    const hipFunction_t f = c->fn.find(name);
+    if (!f) return fail(c, JL_ERR_ARG, "kernel %s is not in the code object", name);
     if (call_dry_run(c)) return JL_OK;
-    HIP_TRY(c, H->ModuleLaunchKernel(it->second, gx, gy, gz, block, 1, 1, lds, st, params, nullptr));
+    HIP_TRY(c, H->ModuleLaunchKernel(f, gx, gy, gz, block, 1, 1, lds, st, params, nullptr));
     if (counted) c->launches++;
     return JL_OK;
 }
@@ -363,9 +422,8 @@ int matvec_launch(jl_ctx* c, float* out, int type, const void* w, const float* x
     a.ngroups = (int)grid;
     a.resid = resid; a.alpha = alpha; a.resid_gate = resid ? resid_gate : nullptr;
     const int xpre = c->tune.xpre == 1 || c->tune.xpre == 4 ? c->tune.xpre : (k / 4 > 2 * block ? 4 : 1);   // three groups a thread and more
-    char name[64];
-    snprintf(name, sizeof name, "jl_matvec_%s_r%d%s%s", pair ? "q8_0p" : ti->tag, rpw, !x ? "_pq" : xpre == 4 ? "_x4" : "",
-             resid ? "_res" : "");
+    Name name;
+    name << "jl_matvec_" << (pair ? "q8_0p" : ti->tag) << "_r" << rpw << (!x ? "_pq" : xpre == 4 ? "_x4" : "") << (resid ? "_res" : "");
     void* params[] = {&a};
     unsigned lds = (unsigned)(act_lds_bytes(k) + (pair ? (size_t)k + 16 : 0));
     return launch(c, name, (unsigned)grid, 1, (unsigned)block, lds, st, params);
@@ -415,7 +473,7 @@ int matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, const vo
     if (gx < 1) gx = 1;
     a.nwaves = nwaves; a.ngroups = (int)gx;
     const int xpre = c->tune.xpre == 1 || c->tune.xpre == 4 ? c->tune.xpre : (k / 4 > 2 * nwaves * 64 ? 4 : 1);
-    char name[64];
+    Name name;
     bool pair = !types;
     for (int i = 0; i < m && pair; i++) pair = q8_pair_form(c, type, ws[i], k);
     // "matvec.act_split" = 1: a gated activation shared by the group's matrices is formed and
@@ -457,14 +515,13 @@ int matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, const vo
         rc = launch(c, "jl_quantize_act", (unsigned)((k / 4 + 255) / 256), 1, 256, 0, st, qp);
         if (rc != JL_OK) return rc;
         a.x = nullptr; a.x2 = nullptr; a.q = q; a.as = as; a.s16 = s16;
-        snprintf(name, sizeof name, "jl_matvec_multi_%s_q%s", pair ? "q8_0p" : ti->tag, resid ? "_res" : "");
+        name << "jl_matvec_multi_" << (pair ? "q8_0p" : ti->tag) << "_q" << (resid ? "_res" : "");
         void* params[] = {&a};
         unsigned lds = (unsigned)(act_lds_bytes(k) + (pair ? (size_t)k + 16 : 0));
         return launch(c, name, (unsigned)gx, (unsigned)m, nwaves * 64, lds, st, params);
     }
-    if (types) snprintf(name, sizeof name, "jl_matvec_segments");
-    else snprintf(name, sizeof name, "jl_matvec_multi_%s%s%s", pair ? "q8_0p" : ti->tag, xpre == 4 ? "_x4" : "",
-                  resid ? "_res" : "");
+    if (types) name << "jl_matvec_segments";
+    else name << "jl_matvec_multi_" << (pair ? "q8_0p" : ti->tag) << (xpre == 4 ? "_x4" : "") << (resid ? "_res" : "");
     void* params[] = {&a};
     // (+ 16 to round the staging area up, + JL_NORM_LDS_BYTES for the RMSNorm's partial sums)
     unsigned lds = (unsigned)(act_lds_bytes(k) + (pair ? (size_t)k + 16 : 0) + 16 + 160);
@@ -930,9 +987,8 @@ int few_launch(jl_ctx* c, const FewCall& f, hipStream_t st) {
     a.nwaves = nw;
     const unsigned lds = (unsigned)std::max(nw * JL_FEW_WAVE_BYTES(f.type, planes, rt), JL_FEW_RED_BYTES(nw, nt, rt));
     if (lds > c->lds_limit) return JL_DECLINED;
-    char name[48];
-    snprintf(name, sizeof name, "jl_few_%s%s_%s_t%dr%d", ti->tag, w256 ? "w" : "",
-             planes ? "planes" : "rows", nt, rt);
+    Name name;
+    name << "jl_few_" << ti->tag << (w256 ? "w_" : "_") << (planes ? "planes" : "rows") << "_t" << nt << "r" << rt;
     void* ap[] = {&a};
     return launch(c, name, (unsigned)((f.nrows + 16 * rt - 1) / (16 * rt)), (unsigned)f.n_expert, (unsigned)(64 * nw), lds, st, ap,
                   (unsigned)f.nmat);
@@ -1059,8 +1115,8 @@ int packed_matvec_launch(jl_ctx* c, float* out, int type, const PlaneRef& pl, co
     a.nrows = nrows; a.k = k; a.row0 = pl.row; a.stride = pl.stride; a.per = c->act_window / 32;
     a.nwaves = nw; a.ngroups = (nrows + rw - 1) / rw;
     a.x2 = nullptr; a.resid = nullptr; a.alpha = 0.f; a.norm_out = nullptr; a.norm_eps = 0.f;
-    char name[64];
-    snprintf(name, sizeof name, "jl_matvec_packed_%s%s_w%d", x ? "" : "q8_", ti->tag, rw);
+    Name name;
+    name << "jl_matvec_packed_" << (x ? "" : "q8_") << ti->tag << "_w" << rw;
     void* params[] = {&a};
     return launch(c, name, (unsigned)((nrows + rw - 1) / rw), 1, (unsigned)(nw * 64),
                   (unsigned)(nw * (384 + 65 * 4)), st, params);  // JL_PK_LDS_BYTES
@@ -1107,8 +1163,8 @@ int packed_matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, c
     a.norm_w = norm_w; a.norm_eps = norm_eps; a.norm_out = norm_w ? norm_out : nullptr;
     a.nrows = nrows; a.k = k; a.stride = pls[0].stride; a.per = c->act_window / 32;
     a.nwaves = nw; a.ngroups = (nrows + rw - 1) / rw;
-    char name[64];
-    snprintf(name, sizeof name, "jl_matvec_packed_multi_%s%s_w%d", up ? "act_" : norm_w ? "norm_" : "", ti->tag, rw);
+    Name name;
+    name << "jl_matvec_packed_multi_" << (up ? "act_" : norm_w ? "norm_" : "") << ti->tag << "_w" << rw;
     void* params[] = {&a};
     return launch(c, name, (unsigned)a.ngroups, (unsigned)m, (unsigned)(nw * 64), (unsigned)(nw * (384 + 65 * 4)), st,
                   params);   // JL_PK_LDS_BYTES
@@ -1310,8 +1366,8 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
             // of them in flight measured 5 % slower)
             int ch = planes ? 1 : (nsb <= 3 ? nsb : 2);
             if (c->tune.moe_chunk >= 1 && c->tune.moe_chunk <= 3) ch = std::min(c->tune.moe_chunk, nsb);
-            char name[32];
-            snprintf(name, sizeof name, "jl_moe_g16%s_%c%d", planes ? "p" : q6k ? "q6" : "", fused ? (x2 ? 'g' : 'f') : two ? 'd' : 'c', ch);
+            Name name;
+            name << "jl_moe_g16" << (planes ? "p_" : q6k ? "q6_" : "_") << (fused ? (x2 ? 'g' : 'f') : two ? 'd' : 'c') << ch;
             void* gp[] = {&ga};
             return launch(c, name, (unsigned)grid, 1, (unsigned)(64 * nwaves), (unsigned)(two ? 2 * frag16 + 16 : lds16), st, gp);
         }
@@ -1461,8 +1517,8 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     if (shares < 1) shares = 1;
     if (shares > 65535) shares = 65535;
     a.nwaves = nwaves; a.shares = shares;
-    char name[64];
-    snprintf(name, sizeof name, "jl_moe_matvec_%s_l%d", ti->tag, lpr);
+    Name name;
+    name << "jl_moe_matvec_" << ti->tag << "_l" << lpr;
     void* params[] = {&a};
     return launch(c, name, (unsigned)shares, (unsigned)n_expert, nwaves * 64, (unsigned)lds, st, params, (unsigned)nmat);
 }
@@ -1561,7 +1617,7 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
         e = H->ModuleGetFunction(&f, c->module, n.c_str());
         if (e != hipSuccess)
             return bail(JL_ERR_HIP, "hipModuleGetFunction(" + n + "): " + H->GetErrorString(e));
-        c->fn[n] = f;
+        c->fn.add(n, f);
     }
     {
         uint32_t tab[2 * 17];
@@ -2454,8 +2510,8 @@ int jl_matmul_mxfp4_bf16_dev(jl_ctx* c, float* out, const void* w, const uint16_
     if (ntok == 1 && k <= 3 * 2048 && c->tune.mx_rows != 1) {
         // one token: the activation stays in registers while a wavefront walks its rows
         const int nbi = (k / 32 + 63) / 64;
-        char name[32];
-        snprintf(name, sizeof name, "jl_mxfp4_matvec1_b%d", nbi);
+        Name name;
+        name << "jl_mxfp4_matvec1_b" << nbi;
         // (a wavefront a workgroup: four wavefronts a workgroup of four rows each were 180 workgroups for
         // 2880 rows and left 76 CUs without one: 4.65 -> 4.18 us)
         return launch(c, name, (unsigned)((nrows + JL_MX1_RPW - 1) / JL_MX1_RPW), 1, 64, 0, st, params);
@@ -2474,8 +2530,8 @@ int jl_matmul_mxfp4_bf16_dev(jl_ctx* c, float* out, const void* w, const uint16_
         rc = launch(c, "jl_mxfp4_prep_few", (unsigned)groups, (unsigned)nt, 256, 0, st, pp);
         if (rc != JL_OK) return rc;
         a.x = (const uint16_t*)c->gemm_ws; a.tok_pad = 16 * nt;
-        char name[32];
-        snprintf(name, sizeof name, "jl_mxfp4_few_t%d", nt);
+        Name name;
+        name << "jl_mxfp4_few_t" << nt;
         return launch(c, name, (unsigned)((nrows + 15) / 16), 1, 512, 0, st, params);
     }
     const unsigned lds = 2u * 128u * 264u * 2u;   // two weight stages [128][264] bf16
@@ -2569,8 +2625,8 @@ int jl_matmul_mxfp4_packed_bf16_dev(jl_ctx* c, float* out, const uint32_t* qs, c
         int rl = c->tune.mx_planes == 64 || c->tune.mx_planes == 32 || c->tune.mx_planes == 16 ? c->tune.mx_planes : 0;
         // (measured: 2880 rows 5.4 us at 16 against 6.8 at 64; 5760 rows 6.3 at 32 against 7.1 and 8.6)
         if (!rl) rl = (nrows + 63) / 64 * 10 >= c->num_cu * 7 ? 64 : ((nrows + 31) / 32 * 10 >= c->num_cu * 7 ? 32 : 16);
-        char name[40];
-        snprintf(name, sizeof name, "jl_mxfp4_matvec_planes_r%d", rl);
+        Name name;
+        name << "jl_mxfp4_matvec_planes_r" << rl;
         void* params[] = {&a};
         return launch(c, name, (unsigned)((nrows + rl - 1) / rl), 1, (unsigned)(64 * a.nwaves),
                       (unsigned)(a.nwaves * 8 * 64 * 4), st, params);

@@ -11,7 +11,7 @@ import ctypes as C
 
 import numpy as np
 
-from . import _lib, quant
+from . import _calls, _lib, quant
 
 
 class DeviceError(RuntimeError):
@@ -47,7 +47,10 @@ class MVGroup:
         self.ActUp, self.Act, self.Resid, self.Alpha = ActUp, Act, Resid, Alpha
 
 
-class Device:
+class Device(_calls.Calls):
+    """The calls a program makes once a matrix (MatVec, MatMul and their packed forms, matvec_dev, matvec_group_dev,
+    matmul_dev, layer_ffn_dev, moe_block_dev, ...) are methods of the C base type (csrc/pycalls.cpp)."""
+
     def __init__(self, device=0, act_window=32, code_object=None):
         self._l = _lib.load()
         self._ctx = C.c_void_p()
@@ -58,6 +61,7 @@ class Device:
             msg = self._l.jl_last_error(None).decode()
             self._ctx = None
             raise DeviceError(f"jl_ctx_create failed ({rc}): {msg}")
+        self._attach(self._ctx.value)
 
     def launch_count(self):
         """Kernels launched so far by this device."""
@@ -65,6 +69,7 @@ class Device:
 
     def close(self):
         if getattr(self, "_ctx", None):
+            self._attach(None)
             self._l.jl_ctx_destroy(self._ctx)
             self._ctx = None
 
@@ -123,11 +128,6 @@ class Device:
                               host(router))
         return self._served(self._l.jl_prep_layer(self._ctx, int(li), C.byref(plan)), "jl_prep_layer")
 
-    def layer_ffn_dev(self, li, h, resid, n, stream=None):
-        """Run prepared block li's feed-forward for n rows: resid [n][n_embd] += ffn(h [n][n_embd])."""
-        return self._served(self._l.jl_layer_ffn_dev(self._ctx, int(li), _ptr(h), _ptr(resid), int(n), stream),
-                            "jl_layer_ffn_dev")
-
     def ReleaseLayers(self, lo, hi):
         """nn.LayerDevice.ReleaseLayers (/root/reference/engine/nn/device.go:1160-1176)."""
         self._served(self._l.jl_release_layers(self._ctx, int(lo), int(hi)), "jl_release_layers")
@@ -170,24 +170,6 @@ class Device:
         self._served(self._l.jl_synchronize(self._ctx), "jl_synchronize")
 
     # -- host-pointer seam ---------------------------------------------------
-    def MatVec(self, out, t, w, x, nrows, k):
-        """nn.Device.MatVec: out[0:nrows] = W x over raw GGUF bytes; False = declined."""
-        if t not in quant.BLOCK:
-            return False
-        assert out.dtype == np.float32 and x.dtype == np.float32 and w.dtype == np.uint8
-        assert out.size >= nrows and x.size >= k
-        return self._served(self._l.jl_matvec(self._ctx, _ptr(out), t, _ptr(w), w.nbytes, _ptr(x),
-                                              nrows, k), "jl_matvec")
-
-    def MatMul(self, out, t, w, x, nrows, k, ntok):
-        """JIT.MatMul (/root/reference/engine/nn/matmul.go:27): x [ntok][k] -> out [ntok][nrows]."""
-        if t not in quant.BLOCK:
-            return False
-        assert out.dtype == np.float32 and x.dtype == np.float32 and w.dtype == np.uint8
-        assert out.size >= ntok * nrows and x.size >= ntok * k
-        return self._served(self._l.jl_matmul(self._ctx, _ptr(out), t, _ptr(w), w.nbytes, _ptr(x),
-                                              nrows, k, ntok), "jl_matmul")
-
     def Forget(self, w):
         """nn.CopyForgetter.Forget: drop the device copy keyed on this host buffer."""
         self._served(self._l.jl_forget(self._ctx, _ptr(w), w.nbytes), "jl_forget")
@@ -198,20 +180,6 @@ class Device:
         nq, nd, nsc = C.c_size_t(), C.c_size_t(), C.c_size_t()
         rc = self._l.jl_packed_words(t, nrows, k, C.byref(nq), C.byref(nd), C.byref(nsc))
         return (nq.value, nd.value, nsc.value) if rc == _lib.OK else None
-
-    def MatVecPacked(self, out, t, p, x, nrows, k):
-        """JIT.MatVecPacked (/root/reference/engine/nn/packed.go:24); p = Packed(qs, d, sc, row, stride)."""
-        assert out.dtype == np.float32 and x.dtype == np.float32
-        return self._served(self._l.jl_matvec_packed(self._ctx, _ptr(out), t, _ptr(p.qs), _ptr(p.d),
-                                                     _opt(p.sc), p.row, p.stride, _ptr(x), nrows, k),
-                            "jl_matvec_packed")
-
-    def MatMulPacked(self, out, t, p, x, nrows, k, ntok):
-        """JIT.MatMulPacked (/root/reference/engine/nn/packedmm.go:23)."""
-        assert out.dtype == np.float32 and x.dtype == np.float32
-        return self._served(self._l.jl_matmul_packed(self._ctx, _ptr(out), t, _ptr(p.qs), _ptr(p.d),
-                                                     _opt(p.sc), p.row, p.stride, _ptr(x), nrows, k, ntok),
-                            "jl_matmul_packed")
 
     def _packed_multi(self, outs, t, ps, x, xstride, up, act, nrows, k, what):
         m = len(ps)
@@ -284,21 +252,11 @@ class Device:
                                                           p.row, p.stride, nrows, k, _ptr(dst), stream),
                             "jl_unpack_weights_dev")
 
-    def matvec_packed_dev(self, out, t, p, x, nrows, k, stream=None):
-        return self._served(self._l.jl_matvec_packed_dev(self._ctx, _ptr(out), t, _ptr(p.qs), _ptr(p.d),
-                                                         _opt(p.sc), p.row, p.stride, _ptr(x), nrows, k,
-                                                         stream), "jl_matvec_packed_dev")
-
     def matvec_packed_q8_dev(self, out, t, p, q, a_s, sum16, nrows, k, stream=None):
         return self._served(self._l.jl_matvec_packed_q8_dev(self._ctx, _ptr(out), t, _ptr(p.qs), _ptr(p.d),
                                                             _opt(p.sc), p.row, p.stride, _ptr(q), _ptr(a_s),
                                                             _ptr(sum16), nrows, k, stream),
                             "jl_matvec_packed_q8_dev")
-
-    def matmul_packed_dev(self, out, t, p, x, nrows, k, ntok, stream=None):
-        return self._served(self._l.jl_matmul_packed_dev(self._ctx, _ptr(out), t, _ptr(p.qs), _ptr(p.d),
-                                                         _opt(p.sc), p.row, p.stride, _ptr(x), nrows, k,
-                                                         ntok, stream), "jl_matmul_packed_dev")
 
     def quantize_act_dev(self, x, ntok, k, q, a_s, sum16, stream=None):
         return self._served(self._l.jl_quantize_act_dev(self._ctx, _ptr(x), ntok, k, _ptr(q),
@@ -309,27 +267,10 @@ class Device:
         return self._served(self._l.jl_dequant_dev(self._ctx, t, _ptr(src), _ptr(dst), n, stream),
                             "jl_dequant_dev")
 
-    def matvec_dev(self, out, t, w, x, nrows, k, stream=None):
-        return self._served(self._l.jl_matvec_dev(self._ctx, _ptr(out), t, _ptr(w), _ptr(x),
-                                                  nrows, k, stream), "jl_matvec_dev")
-
     def matvec_q8_dev(self, out, t, w, q, a_s, sum16, nrows, k, stream=None):
         return self._served(self._l.jl_matvec_q8_dev(self._ctx, _ptr(out), t, _ptr(w), _ptr(q),
                                                      _ptr(a_s), _ptr(sum16), nrows, k, stream),
                             "jl_matvec_q8_dev")
-
-    def matvec_group_dev(self, outs, types, ws, rows, x, k, act_up=None, resid=None, alpha=0.0, stream=None,
-                         norm_w=None, norm_eps=0.0, norm_out=None, resid_gate=None):
-        """JIT.MatVecPackedGroup: up to four matvecs reading one activation, optional
-        RMSNorm(x) * norm_w first, optional silu(x) * act_up and resid += alpha * out[0]
-        (alpha * sigmoid(*resid_gate) when a device logit gates the add), in one launch."""
-        g = _lib.MVGroup()
-        g.n = len(outs)
-        for i in range(g.n):
-            g.out[i], g.type[i], g.w[i], g.rows[i] = _ptr(outs[i]), types[i], _ptr(ws[i]), rows[i]
-        g.x, g.k, g.act_up, g.resid, g.alpha = _ptr(x), k, _opt(act_up), _opt(resid), alpha
-        g.norm_w, g.norm_eps, g.norm_out, g.resid_gate = _opt(norm_w), norm_eps, _opt(norm_out), _opt(resid_gate)
-        return self._served(self._l.jl_matvec_group_dev(self._ctx, C.byref(g), stream), "jl_matvec_group_dev")
 
     def matvec_gather_dev(self, outs, t, ws, x, xstride, up, nrows, k, stream=None):
         """JIT.MatVecPackedGather[Act] (xstride > 0) / MatVecPackedMulti (xstride 0, up None)."""
@@ -364,11 +305,6 @@ class Device:
     def packed_multi_call(self, args, stream=None):
         return self._served(self._l.jl_matvec_packed_multi_dev(self._ctx, *args, stream),
                             "jl_matvec_packed_multi_dev")
-
-    def matmul_dev(self, out, t, w, x, nrows, k, ntok, stream=None):
-        """x [ntok][k] -> out [ntok][nrows] on device operands (JIT.MatMulPacked semantics)."""
-        return self._served(self._l.jl_matmul_dev(self._ctx, _ptr(out), t, _ptr(w), _ptr(x),
-                                                  nrows, k, ntok, stream), "jl_matmul_dev")
 
     def matmul_static_dev(self, out, t, w, x, nrows, k, ntok, stream=None):
         """jl_matmul_dev on the library's static device workspace: allocates nothing."""
@@ -435,28 +371,3 @@ class Device:
                                                          sel_stride, _ptr(wt), rows, k_used, n_expert, n_ffn, n_embd,
                                                          stream),
                             "jl_moe_ffn_types_dev")
-
-    def moe_block_dev(self, resid, t, gate, up, down, router, x, rows, k_used, n_expert, n_ffn, n_embd, sel=None,
-                      wt=None, stream=None, down_type=None, router_type=0):
-        """The whole mixture block, router included: resid [rows][n_embd] += mixture output.  gate / up /
-        down: banks of GGUF sheets (device addresses), or three packed_bank(...) structures."""
-        if isinstance(gate, _lib.PackedBank):
-            return self._served(self._l.jl_moe_block_packed_dev(
-                self._ctx, _ptr(resid), t, C.byref(gate), C.byref(up), C.byref(down), router_type, _ptr(router), _ptr(x),
-                rows, k_used, n_expert, n_ffn, n_embd, _opt(sel), _opt(wt), stream), "jl_moe_block_packed_dev")
-        return self._served(self._l.jl_moe_block_dev(
-            self._ctx, _ptr(resid), t, t if down_type is None else down_type, _ptr(gate), _ptr(up), _ptr(down),
-            router_type, _ptr(router), _ptr(x), rows, k_used, n_expert, n_ffn, n_embd, _opt(sel), _opt(wt), stream),
-            "jl_moe_block_dev")
-
-    def matmul_mxfp4_bf16_dev(self, out, w, x, nrows, k, ntok, stream=None):
-        """MXFP4 weights x bf16 activations (bits as uint16) -> f32 out [ntok][nrows]."""
-        return self._served(self._l.jl_matmul_mxfp4_bf16_dev(self._ctx, _ptr(out), _ptr(w), _ptr(x),
-                                                             nrows, k, ntok, stream),
-                            "jl_matmul_mxfp4_bf16_dev")
-
-    def matmul_mxfp4_packed_bf16_dev(self, out, p, x, nrows, k, ntok, stream=None):
-        """The same over packed MXFP4 planes; p = Packed(qs, d, None, row, stride)."""
-        return self._served(self._l.jl_matmul_mxfp4_packed_bf16_dev(self._ctx, _ptr(out), _ptr(p.qs), _ptr(p.d),
-                                                                    p.row, p.stride, _ptr(x), nrows, k, ntok,
-                                                                    stream), "jl_matmul_mxfp4_packed_bf16_dev")
