@@ -307,6 +307,14 @@ int matvec_max_block(int type, int rpw, bool q8_pair = false) {
     return 0;
 }
 
+// Float4 groups of the activation that a thread of a matvec loads ahead of its weights: all of them up to two,
+// else four ("matvec.xpre" = 1, 2 or 4 asks for one).  A group that is loaded when its turn comes waits out a
+// trip to memory behind the weights (Q4_K 4096 x 8192 6.0 us with one ahead, 5.5 with all).
+int x_groups(const jl_ctx* c, int k, int threads) {
+    if (c->tune.xpre == 1 || c->tune.xpre == 2 || c->tune.xpre == 4) return c->tune.xpre;
+    return k / 4 > 2 * threads ? 4 : k / 4 > threads ? 2 : 1;
+}
+
 hipStream_t pick_stream(jl_ctx* c, void* s) { return s ? (hipStream_t)s : c->stream; }
 
 // LDS of the decode matvec: int8 activations, a scale per 32, a sum per 16
@@ -387,23 +395,27 @@ int matvec_launch(jl_ctx* c, float* out, int type, const void* w, const float* x
     if (type == JL_TYPE_Q4_K && !aligned16(w)) return JL_DECLINED;
     if (((uintptr_t)w & 1) != 0) return JL_DECLINED;
 
-    // Shape choice, from sweeps on MI355X: one row per wavefront; a matrix with at
-    // most sixteen rows per CU runs one 16-wavefront workgroup per CU (the CU
-    // quantizes x once), larger ones a persistent grid of two 12-wavefront
-    // workgroups per CU that stride over the row groups.
+    // Shape choice, from sweeps on MI355X: one row per wavefront.  At most sixteen rows a CU: one workgroup a CU of as
+    // many wavefronts as it has rows, eight at least (the workgroup quantizes x; Q4_K 1500 x 13312 on eight 6.9 us, on
+    // sixteen 7.8; 3000 x 11008 on twelve 6.2 and 6.6).  Taller ones: a persistent grid over the row groups with
+    // sixteen wavefronts a CU for the k-quants, whose registers leave room for no more (a second round of workgroups
+    // quantizes x again: Q6_K 10822 x 768 7.0 us -> 5.6, 14336 x 4096 10.2 -> 8.6), as two workgroups of eight, which
+    // cover each other's barriers (9988 x 5120 Q6_K 9.4 against 10.3 as one; 6000 x 4096 Q4_K 4.5 and 4.5);
+    // Q8_0: two workgroups of twelve, or, up to two rounds of them, one of sixteen wavefronts (14336 x 4096 10.2
+    // against 10.6, 8192 x 4096 7.3 against 6.8).
     int rpw = c->tune.rpw, block = c->tune.block;
     if (rpw <= 0 || resid || !x) rpw = 1;   // (the kernels with the residual add or a quantized activation: one row a wavefront)
     if (rpw != 1 && rpw != 2 && rpw != 4) return fail(c, JL_ERR_ARG, "matvec: rpw=%d", rpw);
-    const bool small = nrows <= 16 * c->num_cu;
-    // (Q4_K 14336 x 4096: one 16-wavefront workgroup a CU 8.1 us, two of twelve 8.6)
-    const bool one_per_cu = small || type == JL_TYPE_Q6_K || type == JL_TYPE_Q4_K;
-    if (block <= 0) block = one_per_cu ? 1024 : 768;
-    if (block % 64 != 0 || block > 1024) return fail(c, JL_ERR_ARG, "matvec: block=%d", block);
     const bool pair = q8_pair_form(c, type, w, k);
+    const bool small = nrows <= 16 * c->num_cu;
+    const bool one_per_cu = small || (type == JL_TYPE_Q8_0 && pair && nrows <= 32 * c->num_cu && k >= 4096);
+    if (block <= 0)
+        block = small ? 64 * std::max(8, (nrows + c->num_cu - 1) / c->num_cu) : one_per_cu ? 1024 : type == JL_TYPE_Q8_0 ? 768 : 512;
+    if (block % 64 != 0 || block > 1024) return fail(c, JL_ERR_ARG, "matvec: block=%d", block);
     if (block > matvec_max_block(type, rpw, pair)) block = matvec_max_block(type, rpw, pair);
     const int rows_per_block = (block / 64) * rpw;
     long groups = ((long)nrows + rows_per_block - 1) / rows_per_block;
-    long grid = c->tune.grid > 0 ? c->tune.grid : (long)c->num_cu * (type == JL_TYPE_Q4_K && !small ? 1 : 2);
+    long grid = c->tune.grid > 0 ? c->tune.grid : (long)c->num_cu * (one_per_cu && rpw == 1 ? 1 : 2);
     if (grid > groups) grid = groups;
     if (grid < 1) grid = 1;
 
@@ -421,9 +433,9 @@ int matvec_launch(jl_ctx* c, float* out, int type, const void* w, const float* x
     a.nwaves = block / 64;
     a.ngroups = (int)grid;
     a.resid = resid; a.alpha = alpha; a.resid_gate = resid ? resid_gate : nullptr;
-    const int xpre = c->tune.xpre == 1 || c->tune.xpre == 4 ? c->tune.xpre : (k / 4 > 2 * block ? 4 : 1);   // three groups a thread and more
+    const int xpre = x_groups(c, k, block);
     Name name;
-    name << "jl_matvec_" << (pair ? "q8_0p" : ti->tag) << "_r" << rpw << (!x ? "_pq" : xpre == 4 ? "_x4" : "") << (resid ? "_res" : "");
+    name << "jl_matvec_" << (pair ? "q8_0p" : ti->tag) << "_r" << rpw << (!x ? "_pq" : xpre == 4 ? "_x4" : xpre == 2 ? "_x2" : "") << (resid ? "_res" : "");
     void* params[] = {&a};
     unsigned lds = (unsigned)(act_lds_bytes(k) + (pair ? (size_t)k + 16 : 0));
     return launch(c, name, (unsigned)grid, 1, (unsigned)block, lds, st, params);
@@ -462,20 +474,27 @@ int matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, const vo
     }
     a.x = x; a.x2 = x2; a.resid = resid; a.alpha = alpha; a.resid_gate = resid ? resid_gate : nullptr;
     a.xstride = xstride;
-    a.norm_w = norm_w; a.norm_eps = norm_eps; a.norm_out = norm_out;
+    a.norm_w = norm_w; a.norm_eps = norm_eps; a.norm_out = norm_out; a.inv_k = 1.0 / k;
     a.k = k; a.row_bytes = (k / ti->block_elems) * ti->block_bytes; a.per = c->act_window / 32;
-    // sixteen wavefronts a workgroup, one row each; about two workgroups per CU over all
-    // the matrices, never more row groups than the tallest matrix has
-    const int nwaves = 16;
-    long groups = ((long)max_rows + nwaves - 1) / nwaves;
-    long gx = (2L * c->num_cu + m - 1) / m;
-    if (gx > groups) gx = groups;
-    if (gx < 1) gx = 1;
-    a.nwaves = nwaves; a.ngroups = (int)gx;
-    const int xpre = c->tune.xpre == 1 || c->tune.xpre == 4 ? c->tune.xpre : (k / 4 > 2 * nwaves * 64 ? 4 : 1);
-    Name name;
     bool pair = !types;
     for (int i = 0; i < m && pair; i++) pair = q8_pair_form(c, type, ws[i], k);
+    // Sixteen wavefronts a workgroup, one row each.  As many workgroups as are resident at once over all the
+    // matrices -- one a CU, two for the paired Q8_0 form, whose registers allow them -- because one more round of
+    // workgroups stages (norms, gates) the activation once more (us, with 512 workgroups for every type -> now:
+    // gate + up with a norm in front Q4_K 2048 / 7168 7.9 -> 6.7, 4096 / 14336 13.0 -> 12.3, Q6_K 1536 / 4608 9.6 -> 7.1;
+    // q + k + v of a 4096 k-quant block 8.2 -> 6.1); never more row groups than a matrix has.
+    const int nwaves = 16;
+    const long slots = c->tune.grid > 0 ? c->tune.grid : (pair ? 2L : 1L) * c->num_cu;
+    long lo = 1, gx = ((long)max_rows + nwaves - 1) / nwaves;
+    while (lo < gx) {   // the largest gx whose workgroups with work are at most `slots`
+        const long mid = (lo + gx + 1) / 2;
+        long n = 0;
+        for (int i = 0; i < m; i++) n += std::min(mid, ((long)rows[i] + nwaves - 1) / nwaves);
+        if (n <= slots) lo = mid; else gx = mid - 1;
+    }
+    a.nwaves = nwaves; a.ngroups = (int)gx;
+    const int xpre = x_groups(c, k, nwaves * 64);
+    Name name;
     // "matvec.act_split" = 1: a gated activation shared by the group's matrices is formed and
     // quantized once, by the quantizer kernel, and the matvec stages the int8 copy (the same
     // values, bit for bit).  Not the default: the extra launch costs what it saves (Q6_K
@@ -521,7 +540,8 @@ int matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, const vo
         return launch(c, name, (unsigned)gx, (unsigned)m, nwaves * 64, lds, st, params);
     }
     if (types) name << "jl_matvec_segments";
-    else name << "jl_matvec_multi_" << (pair ? "q8_0p" : ti->tag) << (xpre == 4 ? "_x4" : "") << (resid ? "_res" : "");
+    else name << "jl_matvec_multi_" << (pair ? "q8_0p" : ti->tag);
+    name << (norm_w ? x2 ? "_na" : "_n" : x2 ? "_a" : "") << (types || xpre == 1 ? "" : xpre == 4 ? "_x4" : "_x2") << (resid ? "_res" : "");
     void* params[] = {&a};
     // (+ 16 to round the staging area up, + JL_NORM_LDS_BYTES for the RMSNorm's partial sums)
     unsigned lds = (unsigned)(act_lds_bytes(k) + (pair ? (size_t)k + 16 : 0) + 16 + 160);
@@ -1114,7 +1134,7 @@ int packed_matvec_launch(jl_ctx* c, float* out, int type, const PlaneRef& pl, co
     a.x = x; a.q = q; a.as = as; a.s16 = s16;
     a.nrows = nrows; a.k = k; a.row0 = pl.row; a.stride = pl.stride; a.per = c->act_window / 32;
     a.nwaves = nw; a.ngroups = (nrows + rw - 1) / rw;
-    a.x2 = nullptr; a.resid = nullptr; a.alpha = 0.f; a.norm_out = nullptr; a.norm_eps = 0.f;
+    a.x2 = nullptr; a.resid = nullptr; a.alpha = 0.f; a.norm_out = nullptr; a.norm_eps = 0.f; a.inv_k = 0.0;
     Name name;
     name << "jl_matvec_packed_" << (x ? "" : "q8_") << ti->tag << "_w" << rw;
     void* params[] = {&a};
@@ -1148,9 +1168,10 @@ int packed_matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, c
     }
     if (rw != 16 && rw != 32 && rw != 64) return fail(c, JL_ERR_ARG, "packed multi: rw=%d", rw);
     const int nchunks = (k + 255) / 256;
-    // sixteen-row runs: eight wavefronts a workgroup, two workgroups a CU (measured against sixteen,
-    // us: Q4_K 4096 x 4096 4.87 against 5.06, Q6_K 4096 x 14336 14.46 against 14.69)
-    int nw = c->tune.packed_block > 0 ? c->tune.packed_block / 64 : rw == 16 ? 8 : 16;
+    // eight wavefronts a workgroup, two and more workgroups a CU, unless there is not one a CU to be had: sixteen then
+    // (gated block of 4096 / 14336 over planes, us: gate + up on eight, down on sixteen 26.6 where sixteen and eight
+    // took 29.1; 2816 / 7936 down on sixteen 14.2 against 14.9)
+    int nw = c->tune.packed_block > 0 ? c->tune.packed_block / 64 : (long)m * ((nrows + rw - 1) / rw) <= c->num_cu ? 16 : 8;
     if (nw > nchunks) nw = nchunks;
     if (nw < 1 || nw > 16) return fail(c, JL_ERR_ARG, "packed multi: block=%d", nw * 64);
     PackedMultiArgs a;
@@ -1160,14 +1181,14 @@ int packed_matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, c
     }
     a.x = x; a.x2 = up; a.xstride = xstride; a.resid = resid; a.alpha = alpha;
     a.resid_gate = resid ? resid_gate : nullptr;
-    a.norm_w = norm_w; a.norm_eps = norm_eps; a.norm_out = norm_w ? norm_out : nullptr;
+    a.norm_w = norm_w; a.norm_eps = norm_eps; a.norm_out = norm_w ? norm_out : nullptr; a.inv_k = 1.0 / k;
     a.nrows = nrows; a.k = k; a.stride = pls[0].stride; a.per = c->act_window / 32;
     a.nwaves = nw; a.ngroups = (nrows + rw - 1) / rw;
     Name name;
     name << "jl_matvec_packed_multi_" << (up ? "act_" : norm_w ? "norm_" : "") << ti->tag << "_w" << rw;
     void* params[] = {&a};
-    return launch(c, name, (unsigned)a.ngroups, (unsigned)m, (unsigned)(nw * 64), (unsigned)(nw * (384 + 65 * 4)), st,
-                  params);   // JL_PK_LDS_BYTES
+    return launch(c, name, (unsigned)a.ngroups, (unsigned)m, (unsigned)(nw * 64),
+                  (unsigned)(nw * (384 + 65 * 4) + (norm_w ? 16 + 160 : 0)), st, params);   // JL_PK_LDS_BYTES + JL_NORM_LDS_BYTES
 }
 
 // MXFP4 planes (QS and D only): rows row .. row+nrows of a buffer of `stride` rows.
@@ -1580,7 +1601,7 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     if (e != hipSuccess)
         return bail(JL_ERR_HIP, "hipModuleLoad(" + path + "): " + H->GetErrorString(e));
 
-    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_multi_q4k_res", "jl_matvec_multi_q4k_x4_res", "jl_matvec_multi_q4k_q_res", "jl_matvec_multi_q8_0_res", "jl_matvec_multi_q8_0_x4_res", "jl_matvec_multi_q8_0_q_res", "jl_matvec_multi_q6k_res", "jl_matvec_multi_q6k_x4_res", "jl_matvec_multi_q6k_q_res", "jl_matvec_multi_q8_0p_res", "jl_matvec_multi_q8_0p_x4_res", "jl_matvec_multi_q8_0p_q_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q6k_r64", "jl_gemm_prep_w32", "jl_gemm_q8_0_w32", "jl_gemm_q6k_w32", "jl_gemm_q4k_w32", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_group", "jl_moe_group2", "jl_moe_group2_wide", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_prep_q6k", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_g16q6_c1", "jl_moe_g16q6_c2", "jl_moe_g16q6_c3", "jl_moe_g16q6_f1", "jl_moe_g16q6_f2", "jl_moe_g16q6_f3", "jl_moe_g16q6_g1", "jl_moe_g16q6_g2", "jl_moe_g16q6_g3", "jl_moe_g16q6_d1", "jl_moe_g16q6_d2", "jl_moe_g16q6_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_moe_gemm_q6k_r64", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_silu_mul", "jl_add_rows", "jl_host_in", "jl_host_done", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
+    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q6k_r64", "jl_gemm_prep_w32", "jl_gemm_q8_0_w32", "jl_gemm_q6k_w32", "jl_gemm_q4k_w32", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_group", "jl_moe_group2", "jl_moe_group2_wide", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_prep_q6k", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_g16q6_c1", "jl_moe_g16q6_c2", "jl_moe_g16q6_c3", "jl_moe_g16q6_f1", "jl_moe_g16q6_f2", "jl_moe_g16q6_f3", "jl_moe_g16q6_g1", "jl_moe_g16q6_g2", "jl_moe_g16q6_g3", "jl_moe_g16q6_d1", "jl_moe_g16q6_d2", "jl_moe_g16q6_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_moe_gemm_q6k_r64", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_silu_mul", "jl_add_rows", "jl_host_in", "jl_host_done", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
                                       "jl_pack_weights", "jl_unpack_q4k", "jl_unpack_q6k", "jl_unpack_q8_0"};
     names.push_back("jl_few_prep");
     for (const char* tag : {"q4k", "q4kw", "q8_0", "q6k", "q6kw"})
@@ -1599,15 +1620,21 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
             char nm[64];
             snprintf(nm, sizeof nm, "jl_matvec_%s_r%d", type_info(t)->tag, rpw);
             names.push_back(nm);
+            names.push_back(std::string(nm) + "_x2");
             names.push_back(std::string(nm) + "_x4");
         }
-    for (int rpw : {1, 2, 4}) names.push_back("jl_matvec_q8_0p_r" + std::to_string(rpw) + "_x4");
+    for (int rpw : {1, 2, 4})
+        for (const char* xp : {"_x2", "_x4"}) names.push_back("jl_matvec_q8_0p_r" + std::to_string(rpw) + xp);
+    for (const char* tag : {"q4k", "q8_0", "q6k", "q8_0p"}) names.push_back(std::string("jl_matvec_") + tag + "_r1_x2_res");
     for (const char* tag : {"q4k", "q8_0", "q6k", "q8_0p"}) {
-        names.push_back(std::string("jl_matvec_multi_") + tag);
-        names.push_back(std::string("jl_matvec_multi_") + tag + "_x4");
-        names.push_back(std::string("jl_matvec_multi_") + tag + "_q");
+        for (const char* res : {"", "_res"}) {
+            for (const char* pre : {"", "_n", "_a", "_na"})
+                for (const char* xp : {"", "_x2", "_x4"}) names.push_back(std::string("jl_matvec_multi_") + tag + pre + xp + res);
+            names.push_back(std::string("jl_matvec_multi_") + tag + "_q" + res);
+        }
     }
-    names.push_back("jl_matvec_segments");
+    for (const char* pre : {"", "_n", "_a", "_na"})
+        for (const char* res : {"", "_res"}) names.push_back(std::string("jl_matvec_segments") + pre + res);
     for (const char* tag : {"q4k", "q8_0", "q6k"})
         for (int rw : {16, 32, 64})
             for (const char* form : {"", "act_", "norm_"})

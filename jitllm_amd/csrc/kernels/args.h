@@ -47,6 +47,7 @@ struct MatVecMultiArgs {
     const float* norm_w; // null: none; else the activation is RMSNorm(x) * norm_w first
     float* norm_out;     // optional: the normed activation, written once
     float norm_eps;
+    double inv_k;        // 1 / k
 };
 
 // Activation preparation for the Q4_K prefill GEMM: quantize x and lay it out
@@ -427,6 +428,7 @@ struct PackedMatVecArgs {
     float alpha;
     float* norm_out;      // norm kernels only: null, or where the normed activation goes
     float norm_eps;
+    double inv_k;        // 1 / k
 };
 
 // Several packed matvecs of one type and shape in one launch, grid = (row groups,
@@ -448,4 +450,5 @@ struct PackedMultiArgs {
     const float* norm_w;  // norm kernels only: RMSNorm weights [k]; every x_j is normed ahead of its quantizer
     float* norm_out;      // null, or where matrix 0's normed activation goes
     float norm_eps;
+    double inv_k;        // 1 / k
 };

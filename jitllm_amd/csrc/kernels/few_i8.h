@@ -53,7 +53,11 @@ __device__ __forceinline__ void jl_few_order(int order, int w, int& g, int& h) {
 // One wavefront per (column, 256 elements): quantize, lay out.  K past the end is zero (values and
 // scales) up to a multiple of 128; columns that fill no group's last slot keep what was there (their
 // results are not stored).  grid = (ceil(k / 256), ceil(ncols / 4)), block = 256.
-__device__ __forceinline__ void few_i8_prep_body(const FewI8PrepArgs& p) {
+__device__ __forceinline__ void few_i8_prep_body(const FewI8PrepArgs& args) {
+    FewI8PrepArgs p = args;
+    JL_NOW(p.x, p.x2, p.src, p.start, p.bq, p.da, p.ds, p.k, p.per, p.ncols, p.n_expert, p.nslots, p.nch, p.order, p.isum);
+    p.x = as_global(p.x); p.x2 = as_global(p.x2); p.src = as_global(p.src); p.start = as_global(p.start);
+    p.bq = as_global(p.bq); p.da = as_global(p.da); p.ds = as_global(p.ds);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const u32 c = blockIdx.y * 4 + wave;
     if (c >= (u32)p.ncols) return;   // whole wavefronts, no barrier below
@@ -524,21 +528,45 @@ __device__ __forceinline__ void few_planes_half(int c, const FewPlaneW<TYPE>* W,
 
 // grid = (ceil(nrows / (16 RT)), experts, matrices), block = 64 * p.nwaves, dynamic LDS: JL_FEW_LDS_BYTES.
 template <int TYPE, bool PL, int NT, int RT, bool W256>
-__device__ __forceinline__ void few_i8_body(const FewI8Args& p, uint8_t* smem) {
+__device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem) {
+    const int e = blockIdx.y;
+    FewI8Args p;   // the matrix's arguments, asked for at once
+    {
+        const int mat = blockIdx.z;
+        p.out[0] = args.out[mat];
+        p.w[0] = PL ? nullptr : args.w[mat];
+        p.pqs[0] = PL ? args.pqs[mat] : nullptr; p.pd[0] = PL ? args.pd[mat] : nullptr; p.psc[0] = PL && TYPE != JL_Q8_0 ? args.psc[mat] : nullptr;
+        p.resid = args.resid; p.bq = args.bq; p.da = args.da; p.ds = TYPE == JL_Q4_K ? args.ds : nullptr; p.start = args.start;
+        p.sheet_bytes = PL ? 0 : args.sheet_bytes; p.sheet_words = PL ? args.sheet_words : 0;
+        p.row_step = PL ? args.row_step : 0; p.prow0 = PL ? args.prow0 : 0; p.pstride = PL ? args.pstride : 0;
+        p.nrows = args.nrows; p.k = args.k; p.row_bytes = PL ? 0 : args.row_bytes; p.ncols = args.ncols; p.nslots = args.nslots;
+        p.nch = args.nch; p.nwaves = args.nwaves;
+        if constexpr (PL) {
+            JL_NOW(p.out[0], p.pqs[0], p.pd[0], p.psc[0], p.resid, p.bq, p.da, p.ds, p.start, p.sheet_words, p.row_step, p.prow0, p.pstride,
+                   p.nrows, p.k, p.ncols, p.nslots, p.nch, p.nwaves);
+            p.pqs[0] = as_global(p.pqs[0]); p.pd[0] = as_global(p.pd[0]); p.psc[0] = as_global(p.psc[0]);
+        } else {
+            JL_NOW(p.out[0], p.w[0], p.resid, p.bq, p.da, p.ds, p.start, p.sheet_bytes, p.nrows, p.k, p.row_bytes, p.ncols, p.nslots, p.nch,
+                   p.nwaves);
+            p.w[0] = as_global(p.w[0]);
+        }
+        p.out[0] = as_global(p.out[0]); p.resid = as_global(p.resid); p.bq = as_global(p.bq); p.da = as_global(p.da); p.ds = as_global(p.ds);
+        p.start = as_global(p.start);
+    }
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nw = p.nwaves;
-    const int r16 = lane & 15, g = lane >> 4, e = blockIdx.y, mat = blockIdx.z;
+    const int r16 = lane & 15, g = lane >> 4;
     u32 col0 = 0, ncol = (u32)p.ncols;
     if (p.start) {
-        col0 = p.start[e];
-        ncol = p.start[e + 1] - col0;
+        col0 = (u32)__builtin_amdgcn_readfirstlane((i32)p.start[e]);
+        ncol = (u32)__builtin_amdgcn_readfirstlane((i32)p.start[e + 1]) - col0;
         if (ncol == 0) return;
     }
     const int r0 = blockIdx.x * 16 * RT;
     FewMat m;
-    m.w = PL ? nullptr : p.w[mat] + (size_t)e * p.sheet_bytes;
-    m.qs = PL ? p.pqs[mat] + (size_t)e * p.sheet_words : nullptr;
-    m.dp = PL ? p.pd[mat] + (size_t)e * p.sheet_words : nullptr;
-    m.sp = PL && TYPE != JL_Q8_0 ? p.psc[mat] + (size_t)e * p.sheet_words : nullptr;
+    m.w = PL ? nullptr : p.w[0] + (size_t)e * p.sheet_bytes;
+    m.qs = PL ? p.pqs[0] + (size_t)e * p.sheet_words : nullptr;
+    m.dp = PL ? p.pd[0] + (size_t)e * p.sheet_words : nullptr;
+    m.sp = PL && TYPE != JL_Q8_0 ? p.psc[0] + (size_t)e * p.sheet_words : nullptr;
     u32 va = 16u * lane, vd = 16u * r16;
     float* sc = (float*)(smem + wave * JL_FEW_WAVE_BYTES(TYPE, PL, RT));
     uint8_t* st = (uint8_t*)sc + JL_FEW_SC_BYTES * RT;   // GGUF rows: the staged super-block
@@ -716,7 +744,7 @@ __device__ __forceinline__ void few_i8_body(const FewI8Args& p, uint8_t* smem) {
             for (int q = 0; q < nw; q++) v += red[(q * 16 * NT + tok) * RS + rr];
             if ((u32)tok < left && r0 + rr < p.nrows) {
                 const size_t o = (size_t)(col0 + t0 * 16 + tok) * p.nrows + r0 + rr;
-                if (p.out[mat]) p.out[mat][o] = v;
+                if (p.out[0]) p.out[0][o] = v;
                 if (p.resid) p.resid[o] += v;
             }
         }

@@ -56,11 +56,14 @@ extern "C" __global__ __launch_bounds__(256) void jl_dequant(
 // ---------------------------------------------------------------- matvec
 // jl_matvec_<type>_r<rows per wavefront>; the workgroup is 64..1024 threads.
 // MAXT is the largest workgroup the variant's register use allows.
-// _x4: the same for an activation longer than one float4 group a thread, whose first four
+// _x2, _x4: the same for an activation of two, of more float4 groups a thread, whose first two (four)
 // groups a thread loads together ahead of its weights.
 #define JL_MATVEC_KERNEL(T, TYPE, RPW, MAXT)                                                 \
     extern "C" __global__ __launch_bounds__(MAXT) void jl_matvec_##T##_r##RPW(MatVecArgs p) { \
         matvec_body<TYPE, RPW, 1>(p, jl_smem);                                               \
+    }                                                                                        \
+    extern "C" __global__ __launch_bounds__(MAXT) void jl_matvec_##T##_r##RPW##_x2(MatVecArgs p) { \
+        matvec_body<TYPE, RPW, 2>(p, jl_smem);                                               \
     }                                                                                        \
     extern "C" __global__ __launch_bounds__(MAXT) void jl_matvec_##T##_r##RPW##_x4(MatVecArgs p) { \
         matvec_body<TYPE, RPW, 4>(p, jl_smem);                                               \
@@ -70,6 +73,9 @@ extern "C" __global__ __launch_bounds__(256) void jl_dequant(
 #define JL_MATVEC_RES_KERNEL(T, TYPE)                                                               \
     extern "C" __global__ __launch_bounds__(1024) void jl_matvec_##T##_r1_res(MatVecArgs p) {       \
         matvec_body<TYPE, 1, 1, true>(p, jl_smem);                                                  \
+    }                                                                                               \
+    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_##T##_r1_x2_res(MatVecArgs p) {    \
+        matvec_body<TYPE, 1, 2, true>(p, jl_smem);                                                  \
     }                                                                                               \
     extern "C" __global__ __launch_bounds__(1024) void jl_matvec_##T##_r1_x4_res(MatVecArgs p) {    \
         matvec_body<TYPE, 1, 4, true>(p, jl_smem);                                                  \
@@ -90,33 +96,37 @@ JL_MATVEC_KERNEL(q6k, JL_Q6_KS, 1, 1024) JL_MATVEC_KERNEL(q6k, JL_Q6_KS, 2, 512)
 // dynamic LDS = JL_ACT_LDS_BYTES_SHIFTED(k)
 JL_MATVEC_KERNEL(q8_0p, JL_Q8_0P, 1, 1024) JL_MATVEC_KERNEL(q8_0p, JL_Q8_0P, 2, 1024) JL_MATVEC_KERNEL(q8_0p, JL_Q8_0P, 4, 512)
 
-// grid = (row groups, matrices), block = 64..1024
-#define JL_MATVEC_MULTI_FORMS(T, TYPE, SUF, RES)                                                               \
-    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_multi_##T##SUF(MatVecMultiArgs p) {           \
-        matvec_multi_body<TYPE, 1, RES>(p, jl_smem, p.row_bytes);                                              \
-    }                                                                                                          \
-    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_multi_##T##_x4##SUF(MatVecMultiArgs p) {      \
-        matvec_multi_body<TYPE, 4, RES>(p, jl_smem, p.row_bytes);                                              \
-    }                                                                                                          \
-    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_multi_##T##_q##SUF(MatVecMultiArgs p) {       \
-        matvec_multi_body<TYPE, 0, RES>(p, jl_smem, p.row_bytes);                                              \
+// grid = (row groups, matrices), block = 64..1024.  _n: an RMSNorm in front of the quantizer, _a: a gated
+// activation, _na: both; _res: MatVecMultiArgs.resid set
+#define JL_MATVEC_MULTI_PRE(T, TYPE, P, PRE, SUF, RES)                                                             \
+    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_multi_##T##P##SUF(MatVecMultiArgs p) {            \
+        matvec_multi_body<TYPE, 1, RES, PRE>(p, jl_smem);                                             \
+    }                                                                                                              \
+    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_multi_##T##P##_x2##SUF(MatVecMultiArgs p) {       \
+        matvec_multi_body<TYPE, 2, RES, PRE>(p, jl_smem);                                                          \
+    }                                                                                                              \
+    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_multi_##T##P##_x4##SUF(MatVecMultiArgs p) {       \
+        matvec_multi_body<TYPE, 4, RES, PRE>(p, jl_smem);                                             \
     }
-// (_res: MatVecMultiArgs.resid set)
+#define JL_MATVEC_MULTI_FORMS(T, TYPE, SUF, RES)                                                                   \
+    JL_MATVEC_MULTI_PRE(T, TYPE, , 0, SUF, RES) JL_MATVEC_MULTI_PRE(T, TYPE, _n, JL_PRE_NORM, SUF, RES)            \
+    JL_MATVEC_MULTI_PRE(T, TYPE, _a, JL_PRE_ACT, SUF, RES) JL_MATVEC_MULTI_PRE(T, TYPE, _na, JL_PRE_NORM | JL_PRE_ACT, SUF, RES) \
+    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_multi_##T##_q##SUF(MatVecMultiArgs p) {           \
+        matvec_multi_body<TYPE, 0, RES>(p, jl_smem);                                                  \
+    }
 #define JL_MATVEC_MULTI_KERNEL(T, TYPE) JL_MATVEC_MULTI_FORMS(T, TYPE, , false) JL_MATVEC_MULTI_FORMS(T, TYPE, _res, true)
 JL_MATVEC_MULTI_KERNEL(q4k, JL_Q4_K) JL_MATVEC_MULTI_KERNEL(q8_0, JL_Q8_0) JL_MATVEC_MULTI_KERNEL(q6k, JL_Q6_KS)
 JL_MATVEC_MULTI_KERNEL(q8_0p, JL_Q8_0P)
 // The same grid over matrices of different types (the reference's MatVecSegments,
 // jit/gpu/kernels/matvec.go:1411-1431: a block's q, k and v in one launch whatever their
-// formats): the type is uniform per workgroup, so the switch is a scalar branch into the
-// single-type body.
-extern "C" __global__ __launch_bounds__(1024) void jl_matvec_segments(MatVecMultiArgs p) {
-    const int y = blockIdx.y;
-    switch (p.type[y]) {
-    case JL_Q4_K: matvec_multi_body<JL_Q4_K>(p, jl_smem, p.row_bytes_of[y]); break;
-    case JL_Q8_0: matvec_multi_body<JL_Q8_0>(p, jl_smem, p.row_bytes_of[y]); break;
-    case JL_Q6_K: matvec_multi_body<JL_Q6_KS>(p, jl_smem, p.row_bytes_of[y]); break;
+// formats).
+#define JL_MATVEC_SEGMENTS(P, PRE, SUF, RES)                                                                       \
+    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_segments##P##SUF(MatVecMultiArgs p) {             \
+        matvec_segments_body<RES, PRE>(p, jl_smem);                                                                 \
     }
-}
+JL_MATVEC_SEGMENTS(, 0, , false) JL_MATVEC_SEGMENTS(_n, JL_PRE_NORM, , false) JL_MATVEC_SEGMENTS(_a, JL_PRE_ACT, , false)
+JL_MATVEC_SEGMENTS(_na, JL_PRE_NORM | JL_PRE_ACT, , false) JL_MATVEC_SEGMENTS(, 0, _res, true) JL_MATVEC_SEGMENTS(_n, JL_PRE_NORM, _res, true)
+JL_MATVEC_SEGMENTS(_a, JL_PRE_ACT, _res, true) JL_MATVEC_SEGMENTS(_na, JL_PRE_NORM | JL_PRE_ACT, _res, true)
 
 // -------------------------------------------------- few tokens, int8 matrix cores
 extern "C" __global__ __launch_bounds__(256) void jl_few_prep(FewI8PrepArgs p) { few_i8_prep_body(p); }

@@ -543,17 +543,18 @@ template <> struct SlotTraits<JL_Q6_K> {
 // 14.7 with the loads' issue order pinned and the waits checked in the assembly (15, 10, 5, 0
 // loads left in flight before the four dot products): a CU returns its loads in the order they
 // were issued, so the last wavefront's first chunk arrives behind the first wavefront's last.)
-// store(row, total) receives a finished row in lane 63.
+// store(row, total) receives a finished row in lane 63; store.begin(row) is called when the row's work starts.
 template <int TYPE, int RPW, class Store>
 __device__ __forceinline__ void matvec_rows(const uint8_t* w0, int row_bytes, const ActLds& A, int nrows, int r0,
                                             int group_stride, int nslots, int lane,
-                                            typename SlotTraits<TYPE>::W (&w)[RPW], Store store) {
+                                            typename SlotTraits<TYPE>::W (&w)[RPW], Store& store) {
     typedef SlotTraits<TYPE> T;
     float acc[RPW];
 #pragma unroll
     for (int j = 0; j < RPW; j++) acc[j] = 0.f;
     bool preloaded = true;
     for (; r0 < nrows; r0 += group_stride) {
+        store.begin(r0);
         for (int slot = lane; slot < nslots; slot += 64) {
             if (!preloaded) {
 #pragma unroll
@@ -583,6 +584,23 @@ __device__ __forceinline__ float resid_weight(float alpha, const float* gate) {
     if (!gate) return alpha;
     return alpha * (float)(1.0 / (1.0 + exp(-(double)*gate)));
 }
+
+// Where finished rows go.  The residual row is asked for when the row begins: asked for with the sum in hand it is
+// a trip to memory at the end of every launch (0.3-0.4 us).
+struct StoreRows {
+    float* out;
+    __device__ __forceinline__ void begin(int) {}
+    __device__ __forceinline__ void operator()(int r, float t) { out[r] = t; }
+};
+struct StoreRowsRes {
+    float *out, *resid;
+    float wt, base = 0.f;
+    __device__ __forceinline__ void begin(int r) { base = resid ? resid[r] : 0.f; }
+    __device__ __forceinline__ void operator()(int r, float t) {
+        out[r] = t;
+        if (resid) resid[r] = (resid == out ? t : base) + wt * t;
+    }
+};
 
 // One wavefront computes RPW rows at a time and strides over the row groups of
 // a persistent grid.  The first group's weight loads are issued before the
@@ -629,14 +647,11 @@ __device__ __forceinline__ void matvec_body_xp(const MatVecArgs& p, uint8_t* sme
     lds_barrier();   // orders the LDS staging only: the weight loads stay in flight
 
     if constexpr (RES) {
-        float* const resid = p.resid;
-        matvec_rows<TYPE, RPW>(p.w, p.row_bytes, A, p.nrows, r0, group_stride, nslots, lane, w, [&](int r, float t) {
-            p.out[r] = t;
-            resid[r] += resid_weight(p.alpha, p.resid_gate) * t;
-        });
+        StoreRowsRes store{p.out, p.resid, resid_weight(p.alpha, p.resid_gate)};
+        matvec_rows<TYPE, RPW>(p.w, p.row_bytes, A, p.nrows, r0, group_stride, nslots, lane, w, store);
     } else {
-        matvec_rows<TYPE, RPW>(p.w, p.row_bytes, A, p.nrows, r0, group_stride, nslots, lane, w,
-                               [&](int r, float t) { p.out[r] = t; });
+        StoreRows store{p.out};
+        matvec_rows<TYPE, RPW>(p.w, p.row_bytes, A, p.nrows, r0, group_stride, nslots, lane, w, store);
     }
 }
 
@@ -647,6 +662,61 @@ __device__ __forceinline__ void matvec_body(const MatVecArgs& p, uint8_t* smem) 
     matvec_body_xp<TYPE, RPW, XP, RES, PQ>(p, smem);
 }
 
+// f64 sums over lanes by lane moves that cost a vector instruction each (a shuffle through LDS is a
+// hundred cycles, twice a step: 0.4 us of a 6 us launch).
+template <int CTRL> __device__ __forceinline__ double dpp_f64(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const u32 lo = (u32)dpp_i32<CTRL, 0xf>(0, (i32)(u32)b), hi = (u32)dpp_i32<CTRL, 0xf>(0, (i32)(u32)(b >> 32));
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+// Every lane gets the sum over its row of sixteen.
+__device__ __forceinline__ double row_sum_f64(double v) {
+    v += dpp_f64<JL_DPP_QUAD_XOR1>(v);
+    v += dpp_f64<JL_DPP_QUAD_XOR2>(v);
+    v += dpp_f64<JL_DPP_ROW_HALF_MIRROR>(v);
+    v += dpp_f64<JL_DPP_ROW_MIRROR>(v);
+    return v;
+}
+// ... and over the 64 lanes (butterfly order).
+__device__ __forceinline__ double wave_sum_f64(double v) {
+    v = row_sum_f64(v);
+    {
+        const uint64_t b = __builtin_bit_cast(uint64_t, v);
+        const auto l = __builtin_amdgcn_permlane16_swap((u32)b, (u32)b, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap((u32)(b >> 32), (u32)(b >> 32), false, false);
+        v = __builtin_bit_cast(double, ((uint64_t)h[0] << 32) | l[0]) + __builtin_bit_cast(double, ((uint64_t)h[1] << 32) | l[1]);
+    }
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const auto l = __builtin_amdgcn_permlane32_swap((u32)b, (u32)b, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap((u32)(b >> 32), (u32)(b >> 32), false, false);
+    return __builtin_bit_cast(double, ((uint64_t)h[0] << 32) | l[0]) + __builtin_bit_cast(double, ((uint64_t)h[1] << 32) | l[1]);
+}
+// 1 / sqrt(m) in f64: the hardware's estimate and two corrections of it (a step of third order, then Newton's).  A
+// division and a square root are a hundred dependent instructions.  m = +inf gives 0.
+__device__ __forceinline__ double rsqrt_f64(double m) {
+    double y = __builtin_amdgcn_rsq(m);
+    double e = fma(-(m * y), y, 1.0);
+    y = fma(y * e, fma(e, 0.375, 0.5), y);
+    e = fma(-(m * y), y, 1.0);
+    y = fma(y * 0.5, e, y);
+    return m > 1.7e308 ? 0.0 : y;
+}
+// The scale of an RMSNorm, 1 / sqrt(sum of squares / k + eps), from every thread's own sum of squares.  red:
+// nwaves + 1 doubles of LDS.  One wavefront adds the wavefronts' sums and turns them into the scale for all:
+// sixteen of them doing it side by side on four SIMDs made the launch 1.3 us longer.
+__device__ __forceinline__ double rms_scale(double ss, double* red, int nwaves, int wave, int lane, double inv_k, float eps) {
+    ss = wave_sum_f64(ss);
+    if (lane == 0) red[wave] = ss;
+    lds_barrier();                 // (orders LDS only: the first weight loads stay in flight)
+    if (wave == 0) {
+        const double part = red[min(lane & 15, nwaves - 1)];
+        const double tot = row_sum_f64((lane & 15) < nwaves ? part : 0.0);
+        if (lane == 0) red[nwaves] = rsqrt_f64(fma(tot, inv_k, (double)eps));
+    }
+    lds_barrier();
+    return red[nwaves];
+}
+
 // Several matvecs of one type in one launch: grid = (row groups, matrices).  Each
 // workgroup stages its matrix's activation (shared, or its own at xstride; optionally
 // silu(x) * x2 formed on the way into the quantizer) and then is the single-matrix
@@ -654,74 +724,97 @@ __device__ __forceinline__ void matvec_body(const MatVecArgs& p, uint8_t* smem) 
 // q/k/v or gate/up of a block (MatVecPackedGroup, engine/nn/packedgroup.go:13-51), a
 // mixture's experts at decode (MatVecPackedMulti / MatVecPackedGatherAct,
 // engine/nn/packedmulti.go:24,84,93); on this machine the saving is the per-launch cost.
-// Sum over the 64 lanes in f64, butterfly order (every lane gets the sum).
-__device__ __forceinline__ double wave_sum_f64(double v) {
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m, 64);
-    return v;
-}
-
 // XP = 0: the activation comes quantized (MatVecMultiArgs.q / as / s16, one for all matrices):
 // a long gated activation is formed and quantized once by the quantizer kernel instead of by
 // every workgroup (silu and its division for 14336 elements in each of 256 workgroups cost the
 // down projection of a feed-forward block 6 of its 20 us).
 // RES: matrix 0's rows are added into the residual as they are made (entry points of their own,
 // like the single-matrix kernel's).
-template <int TYPE, int XP, bool RES>
-__device__ __forceinline__ void matvec_multi_body_xp(const MatVecMultiArgs& p, uint8_t* smem, int row_bytes) {
+// PRE: what stands in front of the quantizer (entry points of their own: a launch fetches its instructions anew,
+// and registers and branches of a form that is not taken are paid for).
+#define JL_PRE_NORM 1   // RMSNorm(x) * norm_w
+#define JL_PRE_ACT 2    // silu(x) * x2
+// A workgroup's share of the arguments, asked for at once.
+struct MultiNow {
+    float *out, *resid, *norm_out;
+    const uint8_t* w;
+    const float *x, *x2, *norm_w, *resid_gate;
+    double inv_k;
+    float norm_eps, alpha;
+    int nrows, k, per, nwaves, ngroups, row_bytes, type;
+};
+template <bool RES, int PRE, bool SEG>
+__device__ __forceinline__ MultiNow multi_now(const MatVecMultiArgs& p) {
+    const int y = blockIdx.y;
+    MultiNow m;
+    m.out = p.out[y]; m.w = p.w[y]; m.nrows = p.nrows[y];
+    m.k = p.k; m.per = p.per; m.nwaves = p.nwaves; m.ngroups = p.ngroups;
+    m.row_bytes = SEG ? p.row_bytes_of[y] : p.row_bytes;
+    m.type = SEG ? p.type[y] : 0;
+    m.x = p.x;
+    size_t xs = p.xstride;
+    m.x2 = PRE & JL_PRE_ACT ? p.x2 : nullptr;
+    m.resid = RES ? p.resid : nullptr; m.resid_gate = RES ? p.resid_gate : nullptr; m.alpha = RES ? p.alpha : 0.f;
+    m.norm_w = nullptr; m.norm_out = nullptr; m.norm_eps = 0.f; m.inv_k = 0.0;
+    if constexpr ((PRE & JL_PRE_NORM) != 0) {
+        m.norm_w = p.norm_w; m.norm_out = p.norm_out; m.norm_eps = p.norm_eps; m.inv_k = p.inv_k;
+        JL_NOW(m.out, m.w, m.nrows, m.k, m.per, m.nwaves, m.ngroups, m.row_bytes, m.type, m.x, xs, m.x2, m.resid, m.resid_gate, m.alpha,
+               m.norm_w, m.norm_out, m.norm_eps, m.inv_k);
+    } else {
+        JL_NOW(m.out, m.w, m.nrows, m.k, m.per, m.nwaves, m.ngroups, m.row_bytes, m.type, m.x, xs, m.x2, m.resid, m.resid_gate, m.alpha);
+    }
+    m.out = as_global(m.out); m.w = as_global(m.w); m.x = as_global(m.x) + (size_t)y * xs;
+    if constexpr (RES) { m.resid = as_global(m.resid); m.resid_gate = as_global(m.resid_gate); }
+    if constexpr ((PRE & JL_PRE_ACT) != 0) m.x2 = as_global(m.x2) + (size_t)y * xs;
+    if constexpr ((PRE & JL_PRE_NORM) != 0) { m.norm_w = as_global(m.norm_w); m.norm_out = as_global(m.norm_out); }
+    return m;
+}
+
+template <int TYPE, int XP, bool RES, int PRE>
+__device__ __forceinline__ void matvec_multi_body_xp(const MatVecMultiArgs& q, const MultiNow& p, uint8_t* smem) {
+    constexpr bool NORM = (PRE & JL_PRE_NORM) != 0, ACT = (PRE & JL_PRE_ACT) != 0;
     typedef SlotTraits<TYPE> T;
     const int y = blockIdx.y;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = p.nwaves;
     const int nthreads = nwaves * 64;
-    const int nrows = p.nrows[y];
+    const int nrows = p.nrows, row_bytes = p.row_bytes;
     const int nslots = p.k / T::kElems;
     const int group_stride = p.ngroups * nwaves;
     const ActLds A = act_lds_views(smem, p.k);
     int r0 = blockIdx.x * nwaves + wave;
     if ((int)blockIdx.x * nwaves >= nrows) return;   // uniform: this matrix has fewer row groups
-    const uint8_t* w0 = p.w[y];
+    const uint8_t* w0 = p.w;
     if constexpr (XP == 0) {
         typename T::W w[1];
         T::load_w(w0 + (size_t)min(r0, nrows - 1) * row_bytes, min(lane, nslots - 1), w[0]);
-        stage_act_copy<stage_layout_of(TYPE)>(smem, p.q, p.as, p.s16, p.k, nthreads);
+        stage_act_copy<stage_layout_of(TYPE)>(smem, q.q, q.as, q.s16, p.k, nthreads);
         lds_barrier();
-        float* const outp = p.out[y];
+        float* const outp = p.out;
         if constexpr (RES) {
-            float* const resid = y == 0 ? p.resid : nullptr;
-            matvec_rows<TYPE, 1>(w0, row_bytes, A, nrows, r0, group_stride, nslots, lane, w, [&](int r, float t) {
-                outp[r] = t;
-                if (resid) resid[r] += resid_weight(p.alpha, p.resid_gate) * t;
-            });
+            StoreRowsRes store{outp, y == 0 ? p.resid : nullptr, resid_weight(p.alpha, p.resid_gate)};
+            matvec_rows<TYPE, 1>(w0, row_bytes, A, nrows, r0, group_stride, nslots, lane, w, store);
         } else {
-            matvec_rows<TYPE, 1>(w0, row_bytes, A, nrows, r0, group_stride, nslots, lane, w,
-                                 [&](int r, float t) { outp[r] = t; });
+            StoreRows store{outp};
+            matvec_rows<TYPE, 1>(w0, row_bytes, A, nrows, r0, group_stride, nslots, lane, w, store);
         }
         return;
     } else {
-    const float* x = p.x + (size_t)y * p.xstride;
-    const float* x2 = p.x2 ? p.x2 + (size_t)y * p.xstride : nullptr;
+    const float *x = p.x, *x2 = p.x2;
 
     const int n4 = p.k / 4, n4_pad = (n4 + 63) & ~63;
-    f32x4 x0[XP], u0[XP];
+    f32x4 x0[XP], u0[ACT ? XP : 1], nw0[NORM ? XP : 1];   // (nw0: the norm weights of the same groups)
     load_x_groups<XP>(x, p.k, nthreads, x0);
-    if (x2) load_x_groups<XP>(x2, p.k, nthreads, u0);
-    else {
-#pragma unroll
-        for (int i = 0; i < XP; i++) u0[i] = f32x4{1.f, 1.f, 1.f, 1.f};
-    }
-    f32x4 nw0[XP];   // the norm weights of the same groups
-#pragma unroll
-    for (int i = 0; i < XP; i++) nw0[i] = f32x4{1.f, 1.f, 1.f, 1.f};
-    if (p.norm_w) load_x_groups<XP>(p.norm_w, p.k, nthreads, nw0);
+    if constexpr (ACT) load_x_groups<XP>(x2, p.k, nthreads, u0);
+    if constexpr (NORM) load_x_groups<XP>(p.norm_w, p.k, nthreads, nw0);
     __builtin_amdgcn_s_barrier();   // activation loads of the whole workgroup go out first
     typename T::W w[1];
     T::load_w(w0 + (size_t)min(r0, nrows - 1) * row_bytes, min(lane, nslots - 1), w[0]);
     // RMSNorm ahead of the quantizer (the reference's RMSNormQuantRows, jit/gpu/kernels/
     // elem.go:252-267, with its host arithmetic, internal/oracle/oracle.go:230-240): the sum
-    // of squares in f64, scale = 1/sqrt(sum/k + eps), y = f32(f64(x) * scale * f64(w)).
+    // of squares in f64, scale = 1/sqrt(sum/k + eps), y = f32(f64(x) * f64(w) * scale).
     // Every workgroup forms the sum itself: k floats are cheaper than a launch.
-    double nscale = 0.0;
-    if (p.norm_w) {
+    double nscale = 0.0, xw[4];   // xw: x * w of the thread's first group, formed while the scale is on its way
+    if constexpr (NORM) {
         double ss = 0.0;
         int g4 = threadIdx.x;
 #pragma unroll
@@ -733,60 +826,57 @@ __device__ __forceinline__ void matvec_multi_body_xp(const MatVecMultiArgs& p, u
             const f32x4 v = ((const f32x4*)x)[g4];
             ss += (double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z + (double)v.w * v.w;
         }
-        ss = wave_sum_f64(ss);
-        // nwaves partial sums and the scale, behind the staging area (JL_NORM_LDS_BYTES more of
-        // dynamic LDS).  One wavefront turns the sum into the scale: the f64 division and square
-        // root are a hundred dependent instructions, and sixteen wavefronts taking them side by
-        // side on four SIMDs made the launch 1.3 us longer than one taking them for all.
+#pragma unroll
+        for (int i = 0; i < 4; i++) xw[i] = (double)x0[0][i] * (double)nw0[0][i];
+        // (the sums and the scale sit behind the staging area: JL_NORM_LDS_BYTES more of dynamic LDS)
         double* red = (double*)(smem + (((TYPE == JL_Q8_0P ? JL_ACT_LDS_BYTES_SHIFTED(p.k) : JL_ACT_LDS_BYTES(p.k)) + 15) & ~15));
-        if (lane == 0) red[wave] = ss;
-        lds_barrier();                 // (orders LDS only: the first weight loads stay in flight)
-        if (wave == 0) {
-            double tot = 0.0;
-            for (int i = 0; i < nwaves; i++) tot += red[i];
-            if (lane == 0) red[nwaves] = 1.0 / __builtin_sqrt(tot / (double)p.k + (double)p.norm_eps);
-        }
-        lds_barrier();
-        nscale = red[nwaves];
+        nscale = rms_scale(ss, red, nwaves, wave, lane, p.inv_k, p.norm_eps);
     }
-    auto stage_group = [&](int g4, f32x4 v, f32x4 u, f32x4 nw) __attribute__((always_inline)) {
-        if (p.norm_w) {
-            v = f32x4{(float)((double)v.x * nscale * (double)nw.x), (float)((double)v.y * nscale * (double)nw.y),
-                      (float)((double)v.z * nscale * (double)nw.z), (float)((double)v.w * nscale * (double)nw.w)};
+    auto stage_group = [&](int g4, f32x4 v, f32x4 u, f32x4 nw, bool first) __attribute__((always_inline)) {
+        if constexpr (NORM) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = (float)((first ? xw[i] : (double)v[i] * (double)nw[i]) * nscale);
             if (p.norm_out && blockIdx.x == 0 && y == 0 && g4 < n4) ((f32x4*)p.norm_out)[g4] = v;
         }
-        if (x2) v = f32x4{silu_f32(v.x) * u.x, silu_f32(v.y) * u.y, silu_f32(v.z) * u.z, silu_f32(v.w) * u.w};
+        if constexpr (ACT) v = f32x4{silu_f32(v.x) * u.x, silu_f32(v.y) * u.y, silu_f32(v.z) * u.z, silu_f32(v.w) * u.w};
         stage_quantize4<stage_layout_of(TYPE)>(smem, p.k, p.per, g4, v);
     };
     {
+        const f32x4 one = {1.f, 1.f, 1.f, 1.f};
         int g4 = threadIdx.x;
 #pragma unroll
         for (int i = 0; i < XP; i++, g4 += nthreads)
-            if (g4 < n4_pad) stage_group(g4, x0[i], u0[i], nw0[i]);
+            if (g4 < n4_pad) stage_group(g4, x0[i], u0[ACT ? i : 0], nw0[NORM ? i : 0], i == 0);
         for (; g4 < n4_pad; g4 += nthreads)
-            stage_group(g4, ((const f32x4*)x)[min(g4, n4 - 1)],
-                        x2 ? ((const f32x4*)x2)[min(g4, n4 - 1)] : f32x4{1.f, 1.f, 1.f, 1.f},
-                        p.norm_w ? ((const f32x4*)p.norm_w)[min(g4, n4 - 1)] : f32x4{1.f, 1.f, 1.f, 1.f});
+            stage_group(g4, ((const f32x4*)x)[min(g4, n4 - 1)], ACT ? ((const f32x4*)x2)[min(g4, n4 - 1)] : one,
+                        NORM ? ((const f32x4*)p.norm_w)[min(g4, n4 - 1)] : one, false);
     }
     lds_barrier();
 
-    float* const outp = p.out[y];
+    float* const outp = p.out;
     // (a second step of weights requested ahead of the staging, for the launches with an RMSNorm or
     // a gated activation in front, measured slower: gate + up 26.2 -> 32.8 us, down 14.5 -> 16.9)
     if constexpr (RES) {
-        float* const resid = y == 0 ? p.resid : nullptr;
-        matvec_rows<TYPE, 1>(w0, row_bytes, A, nrows, r0, group_stride, nslots, lane, w, [&](int r, float t) {
-            outp[r] = t;
-            if (resid) resid[r] += resid_weight(p.alpha, p.resid_gate) * t;
-        });
+        StoreRowsRes store{outp, y == 0 ? p.resid : nullptr, resid_weight(p.alpha, p.resid_gate)};
+        matvec_rows<TYPE, 1>(w0, row_bytes, A, nrows, r0, group_stride, nslots, lane, w, store);
     } else {
-        matvec_rows<TYPE, 1>(w0, row_bytes, A, nrows, r0, group_stride, nslots, lane, w,
-                             [&](int r, float t) { outp[r] = t; });
+        StoreRows store{outp};
+        matvec_rows<TYPE, 1>(w0, row_bytes, A, nrows, r0, group_stride, nslots, lane, w, store);
     }
     }
 }
 
-template <int TYPE, int XP = 1, bool RES = true>
-__device__ __forceinline__ void matvec_multi_body(const MatVecMultiArgs& p, uint8_t* smem, int row_bytes) {
-    matvec_multi_body_xp<TYPE, XP, RES>(p, smem, row_bytes);
+template <int TYPE, int XP = 1, bool RES = true, int PRE = 0>
+__device__ __forceinline__ void matvec_multi_body(const MatVecMultiArgs& p, uint8_t* smem) {
+    matvec_multi_body_xp<TYPE, XP, RES, PRE>(p, multi_now<RES, PRE, false>(p), smem);
+}
+// Matrices of different types: the type is uniform per workgroup, so the switch is a scalar branch.
+template <bool RES, int PRE>
+__device__ __forceinline__ void matvec_segments_body(const MatVecMultiArgs& p, uint8_t* smem) {
+    const MultiNow m = multi_now<RES, PRE, true>(p);
+    switch (m.type) {
+    case JL_Q4_K: matvec_multi_body_xp<JL_Q4_K, 1, RES, PRE>(p, m, smem); break;
+    case JL_Q8_0: matvec_multi_body_xp<JL_Q8_0, 1, RES, PRE>(p, m, smem); break;
+    case JL_Q6_K: matvec_multi_body_xp<JL_Q6_KS, 1, RES, PRE>(p, m, smem); break;
+    }
 }

@@ -452,7 +452,7 @@ __device__ __forceinline__ void pk_load_x(const PackedMatVecArgs& p, int c, int 
 
 // Quantize (or copy) the chunk's activation into the wavefront's private LDS area.
 // NORM: the second operand is the RMSNorm weight and nscale the row's 1/rms; the normed
-// value is f32(f64(x) * nscale * f64(w)), the reference's host arithmetic
+// value is f32(f64(x) * f64(w) * nscale), the reference's host arithmetic
 // (internal/oracle/oracle.go:230-240).
 template <bool FUSED, bool GATED, bool NORM = false>
 __device__ __forceinline__ void pk_stage_x(const PackedMatVecArgs& p, int c, int lane, const PkX<GATED>& X, uint8_t* my,
@@ -465,8 +465,9 @@ __device__ __forceinline__ void pk_stage_x(const PackedMatVecArgs& p, int c, int
         f32x4 xv = live ? X.v : f32x4{0.f, 0.f, 0.f, 0.f};
         if constexpr (NORM) {
             const f32x4 nw = X.u;
-            xv = f32x4{(float)((double)xv.x * nscale * (double)nw.x), (float)((double)xv.y * nscale * (double)nw.y),
-                       (float)((double)xv.z * nscale * (double)nw.z), (float)((double)xv.w * nscale * (double)nw.w)};
+            // (x * w first, as the row-major form has it)
+            xv = f32x4{(float)((double)xv.x * (double)nw.x * nscale), (float)((double)xv.y * (double)nw.y * nscale),
+                       (float)((double)xv.z * (double)nw.z * nscale), (float)((double)xv.w * (double)nw.w * nscale)};
             if (write_norm && live) ((f32x4*)p.norm_out)[c * 64 + lane] = xv;
         } else if constexpr (GATED) {
             const f32x4 u = live ? X.u : f32x4{0.f, 0.f, 0.f, 0.f};
@@ -551,14 +552,8 @@ __device__ __forceinline__ void packed_matvec_body(const PackedMatVecArgs& p, ui
         for (int i = 0; i < XPRE; i++)
             if ((int)threadIdx.x + i * nthreads < n4) sq(X[i].v);
         for (int g4 = threadIdx.x + XPRE * nthreads; g4 < n4; g4 += nthreads) sq(((const f32x4*)p.x)[g4]);
-        ss = wave_sum_f64(ss);
-        double* nred = (double*)(smem + nwaves * JL_PK_WAVE_LDS);   // the partial-sum area, not in use yet
-        if (lane == 0) nred[wave] = ss;
-        __syncthreads();
-        double tot = 0.0;
-        for (int i = 0; i < nwaves; i++) tot += nred[i];
-        __syncthreads();                                            // all have read before the area is reused
-        nscale = 1.0 / __builtin_sqrt(tot / (double)p.k + (double)p.norm_eps);
+        // (an area of its own, JL_NORM_LDS_BYTES behind the rest)
+        nscale = rms_scale(ss, (double*)(smem + ((JL_PK_LDS_BYTES(nwaves) + 15) & ~15)), nwaves, wave, lane, p.inv_k, p.norm_eps);
         write_norm = p.norm_out != nullptr && blockIdx.x == 0;
     } else {
         __builtin_amdgcn_s_barrier();
@@ -586,8 +581,11 @@ __device__ __forceinline__ void packed_matvec_body(const PackedMatVecArgs& p, ui
 
     float* red = (float*)(smem + nwaves * JL_PK_WAVE_LDS);
     red[wave * JL_PK_RED_STRIDE + lane] = acc;
-    __syncthreads();
     const int j = threadIdx.x & 15;
+    // (the first residual row is on its way over the barrier and the sums)
+    float base = 0.f;
+    if (p.resid) base = p.resid[min(g * RW + (int)(threadIdx.x >> 4), p.nrows - 1)];
+    lds_barrier();
     for (int r = threadIdx.x >> 4; r < RW; r += nwaves * 4) {
         float t = 0.f;
         if (j < nwaves) {
@@ -600,7 +598,7 @@ __device__ __forceinline__ void packed_matvec_body(const PackedMatVecArgs& p, ui
         t += dpp_f32<JL_DPP_ROW_MIRROR, 0xf>(t);
         if (j == 0 && g * RW + r < p.nrows) {
             p.out[g * RW + r] = t;
-            if (p.resid) p.resid[g * RW + r] += p.alpha * t;
+            if (p.resid) p.resid[g * RW + r] = (p.resid == p.out ? t : r < nwaves * 4 ? base : p.resid[g * RW + r]) + p.alpha * t;
         }
     }
 }
@@ -610,14 +608,26 @@ template <int TYPE, int RW, int XPRE, bool GATED, bool NORM = false>
 __device__ __forceinline__ void packed_matvec_multi_body(const PackedMultiArgs& m, uint8_t* smem) {
     const int y = blockIdx.y;
     PackedMatVecArgs p;
-    p.out = m.out[y]; p.qs = m.qs[y]; p.d = m.d[y]; p.sc = m.sc[y];
-    p.x = m.x + (size_t)y * m.xstride;
-    p.x2 = NORM ? m.norm_w : GATED ? m.x2 + (size_t)y * m.xstride : nullptr;
-    p.norm_out = NORM && y == 0 ? m.norm_out : nullptr; p.norm_eps = m.norm_eps;
+    p.out = m.out[y]; p.qs = m.qs[y]; p.d = m.d[y]; p.sc = m.sc[y]; p.row0 = m.row0[y];
+    p.x = m.x; p.x2 = NORM ? m.norm_w : GATED ? m.x2 : nullptr;
+    p.nrows = m.nrows; p.k = m.k; p.stride = m.stride; p.per = m.per; p.nwaves = m.nwaves; p.ngroups = m.ngroups;
+    p.resid = m.resid; p.alpha = m.alpha;
+    const float* gate = m.resid_gate;
+    size_t xs = m.xstride;
+    p.norm_out = nullptr; p.norm_eps = 0.f; p.inv_k = 0.0;
+    if constexpr (NORM) {
+        p.norm_out = m.norm_out; p.norm_eps = m.norm_eps; p.inv_k = m.inv_k;
+        JL_NOW(p.out, p.qs, p.d, p.sc, p.row0, p.x, p.x2, xs, p.nrows, p.k, p.stride, p.per, p.nwaves, p.ngroups, p.resid, p.alpha, gate,
+               p.norm_out, p.norm_eps, p.inv_k);
+        p.norm_out = y == 0 ? as_global(p.norm_out) : nullptr;
+    } else {
+        JL_NOW(p.out, p.qs, p.d, p.sc, p.row0, p.x, p.x2, xs, p.nrows, p.k, p.stride, p.per, p.nwaves, p.ngroups, p.resid, p.alpha, gate);
+    }
+    p.out = as_global(p.out); p.qs = as_global(p.qs); p.d = as_global(p.d); p.sc = as_global(p.sc);
+    p.x = as_global(p.x) + (size_t)y * xs;
+    if constexpr (GATED) p.x2 = as_global(p.x2) + (NORM ? 0 : (size_t)y * xs);
     p.q = nullptr; p.as = nullptr; p.s16 = nullptr;
-    p.nrows = m.nrows; p.k = m.k; p.row0 = m.row0[y]; p.stride = m.stride;
-    p.per = m.per; p.nwaves = m.nwaves; p.ngroups = m.ngroups;
-    p.resid = y == 0 ? m.resid : nullptr;
-    p.alpha = y == 0 && m.resid ? resid_weight(m.alpha, m.resid_gate) : 0.f;
+    p.alpha = y == 0 && p.resid ? resid_weight(p.alpha, as_global(gate)) : 0.f;
+    p.resid = y == 0 ? as_global(p.resid) : nullptr;
     packed_matvec_body<TYPE, RW, XPRE, true, GATED, NORM>(p, smem);
 }
