@@ -35,7 +35,7 @@ struct Tuning {
     int act_split = 0;          // grouped matvec with a gated activation: 1 always quantize it in its own launch, 2 never
     int xpre = 0;               // decode matvec: 1 / 4 float4 groups of x a thread loads ahead of its weights
     int q8pair = 0;             // Q8_0 rows: 2 keeps one block a lane-slot (2-byte-aligned loads)
-    int packed_rw = 0, packed_block = 0, moe_group = 0, moe_logits = 0, moe_q6k_cols = 0;
+    int packed_rw = 0, packed_block = 0, moe_group = 0, moe_logits = 0;
     int moe_shares = 0;
     int gemm_rows = 0;
     int gemm_form = 0;
@@ -44,6 +44,7 @@ struct Tuning {
     int gemm_planes = 0;
     int gemm_few = 0;           // the int8 few-token form: 1 wherever it fits, 2 never
     int few_nt = 0, few_rt = 0, few_waves = 0;
+    int gemm_i8 = 0;            // the int8 tile forms: 1, 2, 3 ask for a shape
     int moe_form = 0;
     int moe_g16 = 0;
     int gemm_fold = 0, gemm_fold_waves = 0;
@@ -834,102 +835,79 @@ int gemm_q4k_launch(jl_ctx* c, float* out, const void* w, const float* x, int nr
                   (unsigned)((rows_left + rows - 1) / rows), rows == 128 ? 512 : 256, gemm_lds_bytes(rows), st, gp);
 }
 
-// Q6_K prefill GEMM on the f16 matrix cores (kernels/gemm_q6k.h): 128-token x 64-row tiles,
-// the Q4_K form's activation prep; a grid that leaves most of the chip idle is widened along
-// K and the partial slabs are added in order.
-constexpr unsigned kGemm6LdsBytes = 2u * 64u * kGemmStride * 2u;   // JL_GEMM6_LDS_BYTES
-
-int gemm_q6k_launch(jl_ctx* c, float* out, const void* w, const float* x, int nrows, int k, int ntok,
-                    hipStream_t st) {
-    const int tok_pad = (ntok + kGemmTile - 1) / kGemmTile * kGemmTile, nsb = k / 256;
-    int rc = gemm_ws_ensure(c, gemm_ws_need(tok_pad, k));
-    if (rc != JL_OK) return rc;
-    uint16_t* bq = (uint16_t*)c->gemm_ws;
-    float* da = (float*)((char*)c->gemm_ws + (size_t)nsb * 2 * (tok_pad / 32) * kGemmAStageBytes);
-    GemmPrepArgs pa;
-    pa.x = x; pa.bq = bq; pa.da = da; pa.ntok = ntok; pa.tok_pad = tok_pad; pa.k = k;
-    void* pp[] = {&pa};
-    rc = launch(c, "jl_gemm_prep_q4k_w16", (unsigned)nsb, (unsigned)(tok_pad / 32), 1024, 0, st, pp);
-    if (rc != JL_OK) return rc;
-    GemmArgs ga;
-    ga.out = out; ga.w = (const uint8_t*)w; ga.bq = bq; ga.da = da;
-    ga.nrows = nrows; ga.k = k; ga.ntok = ntok; ga.tok_pad = tok_pad; ga.row_bytes = nsb * 210;
-    ga.out_stride = nrows; ga.sb_per = 0;
-    void* gp[] = {&ga};
-    const long groups = (long)(tok_pad / kGemmTile) * ((nrows + 63) / 64);
-    int nsplit = c->tune.gemm_split > 0 ? c->tune.gemm_split : (groups <= c->num_cu ? (int)(2 * c->num_cu / groups) : 1);
-    if (nsplit > 8) nsplit = 8;
-    if (nsplit > nsb) nsplit = nsb;
-    if (nsplit > 1) {
-        const int per = (nsb + nsplit - 1) / nsplit;
-        nsplit = (nsb + per - 1) / per;   // no empty split
-        const size_t n = (size_t)ntok * nrows;
-        rc = ws_ensure(c, &c->mx_ws, &c->mx_ws_bytes, n * nsplit * 4);
-        if (rc != JL_OK) return rc;
-        ga.out = (float*)c->mx_ws; ga.sb_per = per;
-        rc = launch(c, "jl_gemm_q6k_r64", (unsigned)(tok_pad / kGemmTile), (unsigned)((nrows + 63) / 64),
-                    256, kGemm6LdsBytes, st, gp, (unsigned)nsplit);
-        if (rc != JL_OK) return rc;
-        SumPartsArgs sa;
-        sa.out = out; sa.part = (const float*)c->mx_ws; sa.n = n; sa.nsplit = nsplit;
-        void* sp[] = {&sa};
-        return launch(c, "jl_sum_parts", (unsigned)((n + 255) / 256), 1, 256, 0, st, sp);
-    }
-    return launch(c, "jl_gemm_q6k_r64", (unsigned)(tok_pad / kGemmTile), (unsigned)((nrows + 63) / 64), 256,
-                  kGemm6LdsBytes, st, gp);
+// The int8 tile forms (kernels/gemm_i8.h): Q8_0, Q4_K and Q6_K with window 32, Q6_K with the k-quant window.
+struct I8Shape { int rt, tw; };
+unsigned gemm_i8_lds(const jl_ctx* c, int type, I8Shape f) {   // JL_GEMM_I8_LDS_BYTES
+    const unsigned planes = type == JL_TYPE_Q6_K ? 2 : 1, rows = 32u * f.rt * (4 / f.tw), mins = type == JL_TYPE_Q4_K;
+    return 2u * (planes * rows * 128u + (c->act_window == 32 ? (mins + 1) * (rows * 16u + 4u * 32u * f.tw * 4u) : 0u));
+}
+bool gemm_i8_applies(const jl_ctx* c, int type, int nrows, int k, int ntok) {
+    if (type != JL_TYPE_Q8_0 && type != JL_TYPE_Q4_K && type != JL_TYPE_Q6_K) return false;
+    if (c->act_window != 32 && !(c->act_window == 256 && type == JL_TYPE_Q6_K)) return false;
+    return k % 128 == 0 && ntok <= 65535 * 4 && (nrows + 63) / 64 <= 65535 && (k + 255) / 256 <= 65535;
+}
+Name gemm_i8_name(const char* pre, const jl_ctx* c, int type, I8Shape f) {
+    Name n;
+    n << pre << "_i8_" << type_info(type)->tag << (c->act_window == 256 ? "w_r" : "_r") << f.rt << "t" << f.tw;
+    return n;
 }
 
-// Q8_0, Q6_K and Q4_K prefill GEMM with the activation window of 32 (kernels/gemm_w32.h): its own
-// prep (fragments in the order of the byte unpack, a token scale per 32), 128-token x 64-row
-// tiles, K split in stages of 128 (Q6_K: whole super-blocks) for small grids.
-constexpr unsigned gemm32_lds_bytes(int planes) {   // JL_GEMM32_LDS_BYTES
-    return (unsigned)planes * 64u * kGemmStride * 2u + 2u * 64u * 4u * 4u + 2u * 4u * kGemmTile * 4u;
-}
-
-int gemm_w32_launch(jl_ctx* c, float* out, int type, const void* w, const float* x, int nrows, int k, int ntok,
-                    hipStream_t st) {
+int gemm_i8_launch(jl_ctx* c, float* out, int type, const void* w, const float* x, int nrows, int k, int ntok, hipStream_t st) {
     const bool q6 = type == JL_TYPE_Q6_K, q4 = type == JL_TYPE_Q4_K;
-    const char* kernel = q6 ? "jl_gemm_q6k_w32" : q4 ? "jl_gemm_q4k_w32" : "jl_gemm_q8_0_w32";
-    const unsigned lds = gemm32_lds_bytes(q6 ? 2 : 1);
-    const int tok_pad = (ntok + kGemmTile - 1) / kGemmTile * kGemmTile, nstage = k / 128;
-    const size_t bq_bytes = (size_t)nstage * (tok_pad / 32) * 8 * 1024, da_bytes = (size_t)(k / 32) * tok_pad * 4;
+    const int tok_pad = (ntok + 127) / 128 * 128, nstage = k / 128;
+    const size_t bq_bytes = (size_t)nstage * (tok_pad / 32) * 4096, da_bytes = (size_t)(k / 32) * tok_pad * 4;
     int rc = gemm_ws_ensure(c, bq_bytes + (q4 ? 2 : 1) * da_bytes);
     if (rc != JL_OK) return rc;
-    uint16_t* bq = (uint16_t*)c->gemm_ws;
-    float* da = (float*)((char*)c->gemm_ws + bq_bytes);
     GemmPrepArgs pa;
-    pa.x = x; pa.bq = bq; pa.da = da; pa.ntok = ntok; pa.tok_pad = tok_pad; pa.k = k;
-    if (q4) pa.dsum = (float*)((char*)da + da_bytes);   // the minimums meet d_a * block sums
+    pa.x = x; pa.bq = (uint16_t*)c->gemm_ws; pa.da = (float*)((char*)c->gemm_ws + bq_bytes);
+    pa.ntok = ntok; pa.tok_pad = tok_pad; pa.k = k; pa.per = c->act_window / 32;
+    if (q4) pa.dsum = (float*)((char*)pa.da + da_bytes);   // the minimums meet d_a * block sums
     void* pp[] = {&pa};
-    rc = launch(c, "jl_gemm_prep_w32", (unsigned)((k + 255) / 256), (unsigned)(tok_pad / 32), 256, 0, st, pp);
+    rc = launch(c, "jl_gemm_i8_prep", (unsigned)((k + 255) / 256), (unsigned)(tok_pad / 32), 1024, 0, st, pp);
     if (rc != JL_OK) return rc;
     GemmArgs ga;
-    ga.out = out; ga.w = (const uint8_t*)w; ga.bq = bq; ga.da = da;
+    ga.out = out; ga.w = (const uint8_t*)w; ga.bq = pa.bq; ga.da = pa.da; ga.dsum = pa.dsum;
     ga.nrows = nrows; ga.k = k; ga.ntok = ntok; ga.tok_pad = tok_pad;
     ga.row_bytes = q6 ? (k / 256) * 210 : q4 ? (k / 256) * 144 : (k / 32) * 34;
-    ga.out_stride = nrows; ga.sb_per = 0; ga.dsum = pa.dsum;
+    ga.out_stride = nrows; ga.sb_per = 0;
     void* gp[] = {&ga};
-    const long groups = (long)(tok_pad / kGemmTile) * ((nrows + 63) / 64);
     const int unit = q6 || q4 ? 2 : 1, nunit = nstage / unit;   // stages a split is made of
-    int nsplit = c->tune.gemm_split > 0 ? c->tune.gemm_split : (groups <= c->num_cu ? (int)(2 * c->num_cu / groups) : 1);
-    if (nsplit > 8) nsplit = 8;
-    if (nsplit > nunit) nsplit = nunit;
+    // Shape and K split by what they should take.  A wavefront's 32 x 32 x 32 block costs its SIMD 0.1 us with two or
+    // three wavefronts there and 0.14 with one; workgroups are resident two (128 x 128: Q8_0 only, the others have no
+    // registers for it) or three (128 x 64; two for the k-quants) a CU; a round costs 1.5 us to begin, the slabs of a
+    // split a launch and a trip through memory.
+    I8Shape f = {2, 4};
+    int nsplit = 1;
+    double best = 1e30;
+    const size_t n = (size_t)ntok * nrows;
+    for (int rt : {4, 2}) {
+        if (c->tune.gemm_i8 > 0 ? rt != (c->tune.gemm_i8 == 1 ? 4 : 2) : rt == 4 && type != JL_TYPE_Q8_0) continue;
+        const long cap = rt == 4 || type != JL_TYPE_Q8_0 ? 2 : 3, groups = (long)((ntok + 127) / 128) * ((nrows + 32 * rt - 1) / (32 * rt));
+        for (int s = 1; s <= 8 && s <= nunit; s++) {
+            if (c->tune.gemm_split > 0 && s != std::min(std::min(c->tune.gemm_split, 8), nunit)) continue;
+            const int per = (nunit + s - 1) / s;
+            if ((nunit + per - 1) / per != s) continue;   // no empty split
+            const long wgs = groups * s, full = wgs / (cap * c->num_cu), left = wgs - full * cap * c->num_cu;
+            const double block = 4 * rt * per * unit;     // of a wavefront
+            double us = full * (1.5 + 0.1 * cap * block);
+            if (left) us += 1.5 + std::max(0.1 * ((left + c->num_cu - 1) / c->num_cu), 0.14) * block;
+            if (s > 1) us += 4.0 + 4e-6 * (s + 1) * n;
+            if (us < best) { best = us; f = {rt, 4}; nsplit = s; }
+        }
+    }
+    const int tt = 32 * f.tw, tr = 32 * f.rt * (4 / f.tw), per = (nunit + nsplit - 1) / nsplit;
     if (nsplit > 1) {
-        const int per = (nunit + nsplit - 1) / nsplit;
-        nsplit = (nunit + per - 1) / per;   // no empty split
-        const size_t n = (size_t)ntok * nrows;
         rc = ws_ensure(c, &c->mx_ws, &c->mx_ws_bytes, n * nsplit * 4);
         if (rc != JL_OK) return rc;
         ga.out = (float*)c->mx_ws; ga.sb_per = per * unit;
-        rc = launch(c, kernel, (unsigned)(tok_pad / kGemmTile), (unsigned)((nrows + 63) / 64), 256, lds, st, gp,
-                    (unsigned)nsplit);
-        if (rc != JL_OK) return rc;
-        SumPartsArgs sa;
-        sa.out = out; sa.part = (const float*)c->mx_ws; sa.n = n; sa.nsplit = nsplit;
-        void* sp[] = {&sa};
-        return launch(c, "jl_sum_parts", (unsigned)((n + 255) / 256), 1, 256, 0, st, sp);
     }
-    return launch(c, kernel, (unsigned)(tok_pad / kGemmTile), (unsigned)((nrows + 63) / 64), 256, lds, st, gp);
+    rc = launch(c, gemm_i8_name("jl_gemm", c, type, f), (unsigned)((ntok + tt - 1) / tt), (unsigned)((nrows + tr - 1) / tr), 256,
+                gemm_i8_lds(c, type, f), st, gp, (unsigned)nsplit);
+    if (rc != JL_OK || nsplit == 1) return rc;
+    SumPartsArgs sa;
+    sa.out = out; sa.part = (const float*)c->mx_ws; sa.n = n; sa.nsplit = nsplit;
+    void* sp[] = {&sa};
+    return launch(c, "jl_sum_parts", (unsigned)((n + 255) / 256), 1, 256, 0, st, sp);
 }
 
 // Few tokens, or few columns an expert, on the int8 matrix cores (kernels/few_i8.h): up to two
@@ -1038,12 +1016,12 @@ int matmul_launch(jl_ctx* c, float* out, int type, const void* w, const float* x
         rc = few_launch(c, f, st);
         if (rc != JL_DECLINED) return rc;
     }
+    if (ntok >= c->gemm_min_tok && c->tune.gemm_form != 9 && ((uintptr_t)w & (type == JL_TYPE_Q4_K ? 15 : 1)) == 0 &&
+        gemm_i8_applies(c, type, nrows, k, ntok))
+        return gemm_i8_launch(c, out, type, w, x, nrows, k, ntok, st);
     const bool gemm = type == JL_TYPE_Q4_K && c->act_window == 256 && ntok >= c->gemm_min_tok &&
                       aligned16(w) && ntok <= 65535 * 4 && kGemmLdsBytes <= c->lds_limit;
     if (gemm) return gemm_q4k_launch(c, out, w, x, nrows, k, ntok, st);
-    if (type == JL_TYPE_Q6_K && c->act_window == 256 && ntok >= c->gemm_min_tok && c->tune.gemm_form != 9 &&
-        ((uintptr_t)w & 1) == 0 && ntok <= 65535 * 4 && (nrows + 63) / 64 <= 65535 && kGemm6LdsBytes <= c->lds_limit)
-        return gemm_q6k_launch(c, out, w, x, nrows, k, ntok, st);   // ("gemm.form" = 9: token by token)
     // Q8_0, a handful of tokens: the grouped dot-product kernel with the tokens as the columns
     // of a single group streams the rows once and beats the 128-token tile (14336 x 4096:
     // 2 tokens 17.4 against 21.7 us token by token, 3 tokens 18.6 against 35.2 for the tile, 8 tokens
@@ -1054,10 +1032,6 @@ int matmul_launch(jl_ctx* c, float* out, int type, const void* w, const float* x
                                nrows, k, st);
         if (rc != JL_DECLINED) return rc;
     }
-    if ((type == JL_TYPE_Q8_0 || type == JL_TYPE_Q6_K || type == JL_TYPE_Q4_K) && c->act_window == 32 &&
-        ntok >= c->gemm_min_tok && c->tune.gemm_form != 9 && k % 128 == 0 && ((uintptr_t)w & 1) == 0 && ntok <= 65535 * 4 &&
-        (nrows + 63) / 64 <= 65535 && gemm32_lds_bytes(2) <= c->lds_limit)
-        return gemm_w32_launch(c, out, type, w, x, nrows, k, ntok, st);
     for (int t = 0; t < ntok; t++) {
         rc = matvec_launch(c, out + (size_t)t * nrows, type, w, x + (size_t)t * k, nullptr, nullptr,
                            nullptr, nrows, k, st);
@@ -1228,24 +1202,18 @@ int packed_matmul_launch(jl_ctx* c, float* out, int type, const PlaneRef& pl, co
     // the matrix-core forms read GGUF rows: the planes are turned back into rows in a workspace
     const bool gemm = type == JL_TYPE_Q4_K && c->act_window == 256 && ntok >= c->gemm_min_tok &&
                       ntok <= 65535 * 4 && kGemmLdsBytes <= c->lds_limit && k / 256 <= 65535;
-    const bool gemm6 = type == JL_TYPE_Q6_K && c->act_window == 256 && ntok >= c->gemm_min_tok &&
-                       c->tune.gemm_form != 9 && ntok <= 65535 * 4 && (nrows + 63) / 64 <= 65535 &&
-                       kGemm6LdsBytes <= c->lds_limit && k / 256 <= 65535;
-    const bool gemm32 = (type == JL_TYPE_Q8_0 || type == JL_TYPE_Q6_K || type == JL_TYPE_Q4_K) && c->act_window == 32 &&
-                        ntok >= c->gemm_min_tok && c->tune.gemm_form != 9 && k % 128 == 0 && ntok <= 65535 * 4 &&
-                        (nrows + 63) / 64 <= 65535 && gemm32_lds_bytes(2) <= c->lds_limit && k / 32 <= 65535;
+    const bool i8 = ntok >= c->gemm_min_tok && c->tune.gemm_form != 9 && gemm_i8_applies(c, type, nrows, k, ntok);
     // Q4_K with the k-quant window: the tiled forms read the planes where they lie; only the
     // few-token forms, which take a lane's operand words straight from GGUF rows, restore rows first
     if (gemm && c->tune.gemm_planes != 2 && !gemm_q4k_few_applies(c, nrows, k, ntok) && (size_t)pl.stride * 4 < ((size_t)1 << 31))
         return gemm_q4k_launch(c, out, nullptr, x, nrows, k, ntok, st, &pl);
-    if (gemm || gemm6 || gemm32) {
+    if (gemm || i8) {
         rc = ws_ensure(c, &c->unpack_ws, &c->unpack_ws_bytes, (size_t)nrows * (size_t)(k / ti->block_elems) * ti->block_bytes);
         if (rc != JL_OK) return rc;
         rc = unpack_launch(c, type, pl, nrows, k, c->unpack_ws, st);
         if (rc != JL_OK) return rc;
-        if (gemm32) return gemm_w32_launch(c, out, type, c->unpack_ws, x, nrows, k, ntok, st);
         return gemm ? gemm_q4k_launch(c, out, c->unpack_ws, x, nrows, k, ntok, st)
-                    : gemm_q6k_launch(c, out, c->unpack_ws, x, nrows, k, ntok, st);
+                    : gemm_i8_launch(c, out, type, c->unpack_ws, x, nrows, k, ntok, st);
     }
     for (int t = 0; t < ntok; t++) {
         rc = packed_matvec_launch(c, out + (size_t)t * nrows, type, pl, x + (size_t)t * k, nullptr, nullptr,
@@ -1253,6 +1221,47 @@ int packed_matmul_launch(jl_ctx* c, float* out, int type, const PlaneRef& pl, co
         if (rc != JL_OK) return rc;
     }
     return JL_OK;
+}
+
+// The int8 tile placed per expert: work list, columns quantized and laid out group by group, tiles.
+int moe_gemm_i8_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1, const float* x,
+                       const float* x2, const uint32_t* src, const uint32_t* start, int n_expert, int ncols, int nrows, int k,
+                       I8Shape f, hipStream_t st) {
+    const TypeInfo* ti = type_info(type);
+    const bool q4 = type == JL_TYPE_Q4_K;
+    const int nslots = ncols / 32 + n_expert + 1, nstage = k / 128, tile = 32 * f.tw;
+    const long tiles_max = ncols / tile + n_expert;
+    if (nslots > 65535 || n_expert > 65535) return JL_DECLINED;
+    const int row_bytes = (k / ti->block_elems) * ti->block_bytes, nmat = bank1 ? 2 : 1, tr = 32 * f.rt * (4 / f.tw);
+    const long work = tiles_max * ((nrows + tr - 1) / tr) * nmat;
+    if (work >= (1L << 31)) return JL_DECLINED;
+    const size_t bq_bytes = (size_t)nstage * nslots * 4096, da_bytes = (size_t)(k / 32) * nslots * 128;
+    const size_t o_wl = bq_bytes + (q4 ? 2 : 1) * da_bytes;
+    int rc = ws_ensure(c, &c->moe_q_ws, &c->moe_q_ws_bytes, o_wl + (size_t)(4 + nslots + tiles_max) * 4);
+    if (rc != JL_OK) return rc;
+    char* ws = (char*)c->moe_q_ws;
+    MoeWorklistArgs wa;
+    wa.start = start; wa.wl = (uint32_t*)(ws + o_wl); wa.n_expert = n_expert; wa.nslots = nslots;
+    wa.tile_log2 = f.tw == 4 ? 7 : 6;
+    void* wp[] = {&wa};
+    rc = launch(c, "jl_moe_worklist", 1, 1, 1024, 0, st, wp);
+    if (rc != JL_OK) return rc;
+    MoeGemmPrepArgs pa;
+    pa.x = x; pa.x2 = x2; pa.src = src; pa.start = start; pa.wl = wa.wl;
+    pa.bq = (uint16_t*)ws; pa.da = (float*)(ws + bq_bytes); pa.k = k; pa.nslots = nslots; pa.per = c->act_window / 32;
+    if (q4) pa.dsum = (float*)(ws + bq_bytes + da_bytes);
+    void* pp[] = {&pa};
+    rc = launch(c, "jl_moe_gemm_i8_prep", (unsigned)((k + 255) / 256), (unsigned)nslots, 1024, 0, st, pp);
+    if (rc != JL_OK) return rc;
+    MoeGemmArgs ga;
+    ga.out[0] = out0; ga.out[1] = out1;
+    ga.bank[0] = (const uint8_t*)bank0; ga.bank[1] = (const uint8_t*)bank1;
+    ga.bq = pa.bq; ga.da = pa.da; ga.dsum = pa.dsum; ga.start = start; ga.wl = wa.wl;
+    ga.sheet_bytes = (size_t)nrows * row_bytes; ga.nrows = nrows; ga.k = k; ga.row_bytes = row_bytes;
+    ga.nslots = nslots; ga.nmat = nmat;
+    void* gp[] = {&ga};
+    const long cap = f.rt == 4 || type != JL_TYPE_Q8_0 ? 2 : 3;
+    return launch(c, gemm_i8_name("jl_moe_gemm", c, type, f), (unsigned)std::min(work, cap * c->num_cu), 1, 256, gemm_i8_lds(c, type, f), st, gp);
 }
 
 // pb0 / pb1: the banks as packed planes (bank0 / bank1 unused then): the per-expert tile kernel
@@ -1290,6 +1299,55 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     const int row_bytes = (k / ti->block_elems) * ti->block_bytes;
     const size_t sheet = (size_t)nrows * row_bytes;
     if (type == JL_TYPE_Q4_K ? sheet % 16 != 0 : sheet % 2 != 0) return JL_DECLINED;
+    // The int8 forms, by columns an expert on average (us of one matrix of 128 experts x 2048 x 768 / 32 x 2048 x 1024 /
+    // 16 x 1024 x 2048, what they replace -> them; "moe.form" = 5 forces the few-token kernel, 6, 7, 8 the tiles of 128
+    // columns x 64 rows, 64 x 128 and 128 x 128):
+    //   Q8_0 window 32    1: 39/16/13 -> 36/15/12   8: 90/29/25 -> 53/21/14   32: 235/71/69 -> 92/30/20   128: 853/238/236 -> 170/56/41
+    //   Q6_K window 32    1: 32/16/15 -> 39/16/12   8: 98/40/31 -> 62/22/15   32: 308/110/89 -> 114/37/25   128: 1065/403/304 -> 254/86/60
+    //   Q6_K window 256   2: 48/20/18 -> 47/19/14   8: 67/27/30 -> 59/21/15   48: 179/47/48 -> 111/38/28    128: 238/81/56 -> 183/61/43
+    // The few-token kernel reads an expert's sheet once for 64 columns and the columns once for every row tile, so it
+    // gives way to the tiles where the columns are the more; a tile of 64 columns needs two workgroups a CU.  With a
+    // column or two an expert Q6_K's dot-product kernel is as fast while rows are short.  Q4_K with the k-quant window
+    // has the forms below; the few-token kernel takes it from nine columns an expert on while the whole bank is small
+    // (gate + up of 24 experts x 512 x 1024, 24 columns 20.8 -> 15.7; 64 x 1024 x 1536, 12 columns 36.6 against 53).
+    {
+        const bool q4w = type == JL_TYPE_Q4_K && c->act_window == 256, q6 = type == JL_TYPE_Q6_K;
+        const int nmat = (planes ? pb1 != nullptr : bank1 != nullptr) ? 2 : 1;
+        const double avg = (double)ncols / n_expert;
+        const long tiles64 = (long)n_expert * nmat * ((nrows + 127) / 128);   // workgroups of a tile of 64 columns an expert
+        const bool align = sheet % (type == JL_TYPE_Q4_K ? 16 : 4) == 0;
+        int form = c->tune.moe_form;
+        if (q6 && !planes && c->act_window == 256 && (form == 3 || form == 4)) form += 2;   // (their Q6_K forms)
+        if (form == 0 && (c->act_window == 32 || c->act_window == 256) && !planes) {
+            if (q4w) form = avg >= 9 && avg <= 40 && (double)n_expert * nmat * nrows * k <= 120e6 ? 5 : 0;
+            else if (q6 && avg < (c->act_window == 32 ? 3 : 2) && k < 2048) form = 0;
+            else if (avg < (q6 && c->act_window == 256 ? 28 : 40)) form = 5;
+            else if (avg < (q6 && c->act_window == 32 ? 64 : 56)) form = tiles64 >= 2 * c->num_cu ? 7 : 5;
+            else form = type == JL_TYPE_Q8_0 && avg >= 64 && tiles64 >= 2 * c->num_cu ? 8 : 6;
+        }
+        if (form == 5 && !align && c->tune.moe_form == 0 && avg >= 6) form = 6;
+        if (form >= 6 && !planes && gemm_i8_applies(c, type, nrows, k, ncols)) {
+            rc = moe_gemm_i8_launch(c, out0, out1, type, bank0, bank1, x, x2, src, start, n_expert, ncols, nrows, k,
+                                    form == 6 ? I8Shape{2, 4} : form == 7 ? I8Shape{2, 2} : I8Shape{4, 4}, st);
+            if (rc != JL_DECLINED) return rc;
+        }
+        if (form == 5 && align && few_fits(c, type, planes, nrows, k, ncols, planes ? pb0->stride : 0)) {
+            FewCall f;
+            f.type = type; f.nrows = nrows; f.k = k; f.ncols = ncols; f.nmat = nmat;
+            f.n_expert = n_expert; f.x = x; f.x2 = x2; f.src = src; f.start = start; f.out[0] = out0; f.out[1] = out1;
+            PlaneRef a{}, b{};
+            if (planes) {
+                a = PlaneRef{pb0->qs, pb0->d, pb0->sc, 0, pb0->stride};
+                if (pb1) b = PlaneRef{pb1->qs, pb1->d, pb1->sc, 0, pb1->stride};
+                f.pl[0] = &a; f.pl[1] = pb1 ? &b : nullptr;
+                f.sheet_words = pb0->sheet_bytes / 4; f.row_step = pb0->sheet_bytes ? 0 : nrows;
+            } else {
+                f.w[0] = bank0; f.w[1] = bank1; f.sheet_bytes = sheet;
+            }
+            rc = few_launch(c, f, st);
+            if (rc != JL_DECLINED) return rc;
+        }
+    }
     // Q4_K with the k-quant activation window can also run on the matrix cores (tuning
     // "moe.form" = 2: groups of 32 columns, a wavefront to itself; 3: groups of 16, the weights
     // decoded in registers, below; 4: the prefill GEMM's tile).  Their vector work does not grow
@@ -1300,37 +1358,31 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     //   1024 rows - / 426 / 489 / 372 / 400 1280 rows - / 501 / 577 / 475 / 435   2048 rows - / 709 / 831 / 639 / 623
     // so form 3 takes over from two columns an expert on average (groups of 32 from ten) and form 4
     // from 72; form 2 is left to "moe.form" = 2.
-    // Q6_K sheets (the down projections of a model whose other experts are Q4_K) have forms 1, 3
-    // and 4 (the Q6_K GEMM's tile); where form 3 does not apply (K too long for LDS) the tile takes
-    // over from "moe.q6k_cols" columns an expert on average, default 12.
     // Form 3: groups of sixteen columns on the 16 x 16 x 32 matrix instruction, the weights decoded
-    // in registers straight into its operand (Q4_K GGUF sheets or packed planes, Q6_K GGUF sheets, the k-quant window; the group's
+    // in registers straight into its operand (Q4_K GGUF sheets or packed planes, the k-quant window; the group's
     // fragments for the whole of K sit in LDS).  Its steady state runs at the rate of a plain read;
-    // the library picks it from two (over planes three) columns an expert on average up to 72, while the
-    // fragments take at most half a CU's LDS (K <= 2304); "moe.form" = 3 forces it wherever they fit.
+    // the library picks it from two (over planes three) columns an expert on average up to 72, wherever
+    // the fragments fit in LDS (one workgroup a CU runs either way: 100 experts x 512 x 2560, six columns, 63 -> 35 us);
+    // "moe.form" = 3 forces it.
     {
         const int nsb = k / 256;
         const size_t frag16 = (size_t)nsb * JL_MOE_G16_LDS_WORDS * 4;   // a token tile's fragments
         const size_t lds16 = frag16 + 16;                               // and the tile counter
         const size_t nslots16 = (size_t)ncols / 16 + (size_t)n_expert + 1;
-        const bool q6k = type == JL_TYPE_Q6_K;   // (GGUF sheets only: plane sheets are Q4_K)
-        const bool can16 = (type == JL_TYPE_Q4_K || (q6k && !planes)) && c->act_window == 256 && lds16 <= c->lds_limit &&
+        const bool can16 = type == JL_TYPE_Q4_K && c->act_window == 256 && lds16 <= c->lds_limit &&
                            (size_t)nrows * row_bytes < ((size_t)1 << 32);
-        // (Q6_K sheets: the decode is 4.5 vector instructions a weight, two matrix instructions a K-step,
-        // and the kernel is bound by them: 62 us for the 2048 x 768 down projections of 128 experts at 64
-        // rows where the dot-product kernel takes 58; with two token tiles a decoded word it costs the
-        // same, so it is picked from six columns an expert, always in groups of 32: 128 rows 68 us against
-        // 97, 256 rows 71 against 139 for the tile, 1024 rows 193 against 195)
-        const bool pick16 = c->tune.moe_form == 0 && 2 * lds16 <= c->lds_limit &&
-                            (long)ncols >= (q6k ? 6L : planes ? 3L : 2L) * n_expert && (long)ncols < (q6k ? 64L : 72L) * n_expert;
+        const bool pick16 = c->tune.moe_form == 0 &&
+                            (long)ncols >= (planes ? 3L : 2L) * n_expert && (long)ncols < 72L * n_expert;
         if (can16 && (c->tune.moe_form == 3 || pick16)) {
-            // up to eight columns an expert the matrix kernel quantizes them itself: no prep launch,
-            // no workspace ("moe.group16" = 1 forces the prep kernel, 2 the fused form)
-            const bool fused = c->tune.moe_g16 == 2 || (c->tune.moe_g16 == 0 && !q6k && (long)ncols <= 8L * n_expert);
-            // from ten columns an expert groups of 32 (two token tiles, a decoded word meets both), so
+            // up to seven columns an expert the matrix kernel quantizes them itself: no prep launch,
+            // no workspace ("moe.group16" = 1 forces the prep kernel, 2 the fused form).  (Eight of many
+            // experts: some have more than sixteen, and the workgroup that reads its sheet twice is the
+            // launch's length: 128 experts, top-8, 128 rows 142 us, in groups of 32 134; 112 rows 115 and 131.)
+            const bool fused = c->tune.moe_g16 == 2 || (c->tune.moe_g16 == 0 && (long)ncols <= (n_expert > 64 ? 7L : 8L) * n_expert);
+            // beyond groups of 32 (two token tiles, a decoded word meets both), so
             // that an expert of 17-32 columns reads its sheet once ("moe.group16" = 3 forces them)
             const bool two = !fused && 2 * frag16 + 16 <= c->lds_limit &&
-                             (c->tune.moe_g16 == 3 || (c->tune.moe_g16 == 0 && (q6k || (long)ncols >= 10L * n_expert)));
+                             (c->tune.moe_g16 == 3 || c->tune.moe_g16 == 0);
             MoeG16PrepArgs pa;
             pa.ws = nullptr;
             if (!fused) {
@@ -1339,7 +1391,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
                 pa.x = x; pa.x2 = x2; pa.src = src; pa.start = start; pa.ws = (uint32_t*)c->moe_q_ws;
                 pa.k = k; pa.n_expert = n_expert; pa.ncols = ncols;
                 void* pp[] = {&pa};
-                rc = launch(c, planes ? "jl_moe_g16_prep_planes" : q6k ? "jl_moe_g16_prep_q6k" : "jl_moe_g16_prep", (unsigned)((ncols + 3) / 4), 1,
+                rc = launch(c, planes ? "jl_moe_g16_prep_planes" : "jl_moe_g16_prep", (unsigned)((ncols + 3) / 4), 1,
                             256, 0, st, pp);
                 if (rc != JL_OK) return rc;
             }
@@ -1388,7 +1440,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
             int ch = planes ? 1 : (nsb <= 3 ? nsb : 2);
             if (c->tune.moe_chunk >= 1 && c->tune.moe_chunk <= 3) ch = std::min(c->tune.moe_chunk, nsb);
             Name name;
-            name << "jl_moe_g16" << (planes ? "p_" : q6k ? "q6_" : "_") << (fused ? (x2 ? 'g' : 'f') : two ? 'd' : 'c') << ch;
+            name << "jl_moe_g16" << (planes ? "p_" : "_") << (fused ? (x2 ? 'g' : 'f') : two ? 'd' : 'c') << ch;
             void* gp[] = {&ga};
             return launch(c, name, (unsigned)grid, 1, (unsigned)(64 * nwaves), (unsigned)(two ? 2 * frag16 + 16 : lds16), st, gp);
         }
@@ -1423,11 +1475,8 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
         return launch(c, "jl_moe_matvec_planes_q4k", (unsigned)((nrows + 63) / 64), (unsigned)n_expert, (unsigned)(a.nwaves * 64),
                       (unsigned)(a.nwaves * 8 * 256), st, params, (unsigned)nmat);   // JL_MOEP_TB columns a pass
     }
-    const bool q6 = type == JL_TYPE_Q6_K;
-    const long q6_cols = c->tune.moe_q6k_cols > 0 ? c->tune.moe_q6k_cols : 12;
-    const bool many_cols = c->tune.moe_form == 0 && (long)ncols >= (q6 ? q6_cols : 10L) * n_expert;   // (Q4_K: 72 and more get here)
-    if ((type == JL_TYPE_Q4_K || q6) && c->act_window == 256 &&
-        (planes || c->tune.moe_form == 4 || many_cols || (!q6 && c->tune.moe_form == 2)) &&
+    const bool many_cols = c->tune.moe_form == 0 && (long)ncols >= 10L * n_expert;   // (72 and more get here)
+    if (type == JL_TYPE_Q4_K && c->act_window == 256 && (planes || c->tune.moe_form == 4 || many_cols || c->tune.moe_form == 2) &&
         4u * 19968u <= c->lds_limit) {   // JL_MOEG_WAVE_LDS
         const int nslots = ncols / 32 + n_expert + 1, nsb = k / 256;
         const int tiles_max = ncols / 128 + n_expert;
@@ -1472,14 +1521,11 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
             return launch(c, "jl_moe_gemm_r64_planes", (unsigned)std::min<long>(work, 2L * c->num_cu), 1, 256,
                           gemm_lds_bytes(64), st, gp);
         }
-        if ((q6 || c->tune.moe_form == 4 || (c->tune.moe_form == 0 && (long)ncols >= 56L * n_expert)) &&
+        if ((c->tune.moe_form == 4 || (c->tune.moe_form == 0 && (long)ncols >= 56L * n_expert)) &&
             kGemmLdsBytes <= c->lds_limit && n_expert <= 65535 && (long)tiles_max * rtiles * ga.nmat < (1L << 31)) {
             const long work = (long)tiles_max * rtiles * ga.nmat;
-            const unsigned grid = (unsigned)std::min<long>(work, (q6 ? 3L : 2L) * c->num_cu);
-            return launch(c, q6 ? "jl_moe_gemm_q6k_r64" : "jl_moe_gemm_r64", grid, 1, 256,
-                          q6 ? kGemm6LdsBytes : gemm_lds_bytes(64), st, gp);
+            return launch(c, "jl_moe_gemm_r64", (unsigned)std::min<long>(work, 2L * c->num_cu), 1, 256, gemm_lds_bytes(64), st, gp);
         }
-        if (q6) return fail(c, JL_ERR_ARG, "moe matvec: %d experts x %ld row tiles do not fit the tile form", n_expert, rtiles);
         return launch(c, "jl_moe_gemm_q4k", (unsigned)((nrows + 255) / 256), (unsigned)nslots, 256, 4u * 19968u, st, gp,
                       (unsigned)ga.nmat);
     }
@@ -1601,9 +1647,14 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     if (e != hipSuccess)
         return bail(JL_ERR_HIP, "hipModuleLoad(" + path + "): " + H->GetErrorString(e));
 
-    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q6k_r64", "jl_gemm_prep_w32", "jl_gemm_q8_0_w32", "jl_gemm_q6k_w32", "jl_gemm_q4k_w32", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_group", "jl_moe_group2", "jl_moe_group2_wide", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_prep_q6k", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_g16q6_c1", "jl_moe_g16q6_c2", "jl_moe_g16q6_c3", "jl_moe_g16q6_f1", "jl_moe_g16q6_f2", "jl_moe_g16q6_f3", "jl_moe_g16q6_g1", "jl_moe_g16q6_g2", "jl_moe_g16q6_g3", "jl_moe_g16q6_d1", "jl_moe_g16q6_d2", "jl_moe_g16q6_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_moe_gemm_q6k_r64", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_silu_mul", "jl_add_rows", "jl_host_in", "jl_host_done", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
+    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_group", "jl_moe_group2", "jl_moe_group2_wide", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_silu_mul", "jl_add_rows", "jl_host_in", "jl_host_done", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
                                       "jl_pack_weights", "jl_unpack_q4k", "jl_unpack_q6k", "jl_unpack_q8_0"};
     names.push_back("jl_few_prep");
+    names.push_back("jl_gemm_i8_prep");
+    names.push_back("jl_moe_gemm_i8_prep");
+    for (const char* pre : {"jl_gemm_i8_", "jl_moe_gemm_i8_"})
+        for (const char* tag : {"q8_0", "q4k", "q6k", "q6kw"})
+            for (const char* shape : {"_r4t4", "_r2t4", "_r2t2"}) names.push_back(std::string(pre) + tag + shape);
     for (const char* tag : {"q4k", "q4kw", "q8_0", "q6k", "q6kw"})
         for (const char* layout : {"rows", "planes"})
             for (const char* size : {"t1r1", "t1r2", "t2r1", "t4r1", "t4r2", "t1r4", "t2r2", "t2r4"})
@@ -1725,7 +1776,7 @@ int jl_set_tuning(jl_ctx* c, const char* key, int value) {
     else if (!strcmp(key, "packed.block")) c->tune.packed_block = value;
     else if (!strcmp(key, "moe.group")) c->tune.moe_group = value;
     else if (!strcmp(key, "moe.logits")) c->tune.moe_logits = value;
-    else if (!strcmp(key, "moe.q6k_cols")) c->tune.moe_q6k_cols = value;
+    else if (!strcmp(key, "moe.q6k_cols")) (void)value;   // (once the column count from which Q6_K took its tile)
     else if (!strcmp(key, "moe.shares")) c->tune.moe_shares = value;
     else if (!strcmp(key, "moe.form")) c->tune.moe_form = value;
     else if (!strcmp(key, "moe.group16")) c->tune.moe_g16 = value;
@@ -1747,6 +1798,7 @@ int jl_set_tuning(jl_ctx* c, const char* key, int value) {
     else if (!strcmp(key, "gemm.prep")) c->tune.gemm_prep = value;
     else if (!strcmp(key, "gemm.planes")) c->tune.gemm_planes = value;
     else if (!strcmp(key, "gemm.few")) c->tune.gemm_few = value;
+    else if (!strcmp(key, "gemm.i8")) c->tune.gemm_i8 = value;
     else if (!strcmp(key, "few.nt")) c->tune.few_nt = value;
     else if (!strcmp(key, "few.rt")) c->tune.few_rt = value;
     else if (!strcmp(key, "few.waves")) c->tune.few_waves = value;

@@ -58,6 +58,7 @@ struct GemmPrepArgs {
     float* da;
     int ntok, tok_pad, k;
     float* dsum = nullptr;   // window 32, optional: d_a * (sum of the block's int8) [k/32][tok_pad]
+    int per = 0;             // the int8 prep: activation window / 32
 };
 
 struct GemmArgs {
@@ -130,6 +131,7 @@ struct MoeWorklistArgs {
     const uint32_t* start;
     uint32_t* wl;
     int n_expert, nslots;
+    int tile_log2 = 7;    // columns a tile
 };
 
 struct MoeGemmPrepArgs {
@@ -141,6 +143,8 @@ struct MoeGemmPrepArgs {
     uint16_t* bq;
     float* da;
     int k, nslots;
+    int per = 0;          // the int8 prep: activation window / 32
+    float* dsum = nullptr;
 };
 
 struct MoeGemmArgs {
@@ -161,6 +165,7 @@ struct MoeGemmArgs {
     const uint32_t* psc[2] = {nullptr, nullptr};
     size_t sheet_words = 0;
     int row_step = 0, pstride = 0;
+    const float* dsum = nullptr;   // the int8 form, Q4_K: d_a * block sums
 };
 
 // Grouped expert matmul, sixteen columns a group (moe_g16_body).  Column group g of expert e is

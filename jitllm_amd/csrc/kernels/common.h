@@ -7,6 +7,7 @@ typedef uint32_t u32;
 typedef int32_t i32;
 typedef u32 u32x2 __attribute__((ext_vector_type(2)));
 typedef u32 u32x4 __attribute__((ext_vector_type(4)));
+typedef i32 i32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // ggml type numbers (the reference's quant.Type, format/quant/types.go:14-55)

@@ -197,7 +197,6 @@ __device__ __forceinline__ void few_put_q6k(u32 d, i32 s0, i32 s1, int g, int r,
     lds[128 + r] = half_bits_to_f32((uint16_t)(d & 0xFFFF)) * 0.25f;
 }
 
-typedef i32 i32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ i32x4 mfma_i8(u32x2 a, u32x2 b, i32x4 c) {
     return __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, a), __builtin_bit_cast(long, b), c, 0, 0, 0);
 }

@@ -5,11 +5,10 @@
 #include "common.h"
 #include "dequant.h"
 #include "few_i8.h"
+#include "gemm_i8.h"
 #include "gemm_q4k.h"
 #include "gemm_q4k_k2.h"
 #include "gemm_q4k_fold.h"
-#include "gemm_q6k.h"
-#include "gemm_w32.h"
 #include "matvec.h"
 #include "moe.h"
 #include "mxfp4.h"
@@ -208,22 +207,54 @@ extern "C" __global__ __launch_bounds__(256, 2) void jl_gemm_q4k_r64(GemmArgs p)
     gemm_split_slice(p);
     gemm_q4k_body<1>(p, jl_smem, blockIdx.x * JL_GEMM_TILE, blockIdx.y * 64);
 }
-// Q6_K with the k-quant window: grid = (tok_pad/128, ceil(nrows/64), K splits), block = 256,
-// dynamic LDS = JL_GEMM6_LDS_BYTES; the activation prep is jl_gemm_prep_q4k
-extern "C" __global__ __launch_bounds__(256, 2) void jl_gemm_q6k_r64(GemmArgs p) {
-    gemm_q6k_split_slice(p);
-    gemm_q6k_body(p, jl_smem, blockIdx.x * JL_GEMM_TILE, blockIdx.y * 64);
+// The int8 form (kernels/gemm_i8.h): prep grid = (ceil(k/256), tok_pad/32), block = 1024; matrix kernel
+// jl_gemm_i8_<type>_<shape>: grid = (token tiles, row tiles, K splits), block = 256, dynamic LDS = JL_GEMM_I8_LDS_BYTES;
+// shape r4t4: 128 tokens x 128 rows, r2t4: 128 x 64, r2t2: 64 x 128.  jl_moe_gemm_i8_...: the same tile per expert.
+extern "C" __global__ __launch_bounds__(1024) void jl_gemm_i8_prep(GemmPrepArgs p) {
+    __shared__ u32 lds[JL_GEMM_I8_PREP_WORDS];
+    gemm_i8_prep_body(p, lds);
 }
-// Q8_0, Q6_K and Q4_K with the activation window of 32: prep grid = (ceil(k/256), tok_pad/32), block = 256;
-// matrix kernel grid = (tok_pad/128, ceil(nrows/64), K splits), block = 256, dynamic LDS =
-// JL_GEMM32_LDS_BYTES(planes)
-extern "C" __global__ __launch_bounds__(256) void jl_gemm_prep_w32(GemmPrepArgs p) {
-    __shared__ u32 sq[32 * 65];
-    gemm_prep_w32_body(p, sq);
+extern "C" __global__ __launch_bounds__(1024) void jl_moe_gemm_i8_prep(MoeGemmPrepArgs p) {
+    __shared__ u32 lds[JL_GEMM_I8_PREP_WORDS];
+    moe_gemm_i8_prep_body(p, lds);
 }
-extern "C" __global__ __launch_bounds__(256, 3) void jl_gemm_q8_0_w32(GemmArgs p) { gemm_w32_body<JL_Q8_0>(p, jl_smem); }
-extern "C" __global__ __launch_bounds__(256, 3) void jl_gemm_q6k_w32(GemmArgs p) { gemm_w32_body<JL_Q6_K>(p, jl_smem); }
-extern "C" __global__ __launch_bounds__(256, 3) void jl_gemm_q4k_w32(GemmArgs p) { gemm_w32_body<JL_Q4_K>(p, jl_smem); }
+template <int TYPE, bool W256, int RT, int TW>
+__device__ __forceinline__ void moe_gemm_i8_tiles(const MoeGemmArgs& p) {
+    constexpr u32 ROWS = 32 * RT * (4 / TW);
+    const u32 rtiles = ((u32)p.nrows + ROWS - 1) / ROWS;
+    const u32 ntiles = p.wl[0];
+    const u32 per_mat = ntiles * rtiles, total = per_mat * (u32)p.nmat;
+    for (u32 idx = blockIdx.x; idx < total; idx += gridDim.x) {   // uniform across the workgroup
+        const u32 mat = idx / per_mat, rem = idx - mat * per_mat;
+        const u32 t = rem / rtiles, rt = rem - t * rtiles;
+        const u32 ent = p.wl[4 + p.nslots + t];
+        const int e = (int)(ent & 0xFFFFu), ctile = (int)(ent >> 16);
+        const u32 c_lo = p.start[e], c_hi = p.start[e + 1];
+        const int slot0 = (int)(c_lo >> 5) + e;
+        GemmArgs g;
+        g.w = p.bank[mat] + (size_t)e * p.sheet_bytes;
+        g.bq = p.bq; g.da = p.da; g.dsum = p.dsum;
+        g.nrows = p.nrows; g.k = p.k; g.row_bytes = p.row_bytes;
+        g.tok_pad = 32 * p.nslots;
+        g.ntok = 32 * slot0 + (int)(c_hi - c_lo);    // tokens are positions in the workspace
+        g.out_stride = p.nrows; g.sb_per = 0;
+        g.out = p.out[mat] + ((ptrdiff_t)c_lo - (ptrdiff_t)32 * slot0) * p.nrows;   // workspace position -> column
+        gemm_i8_body<TYPE, W256, RT, TW>(g, jl_smem, 32 * slot0 + 32 * TW * ctile, (int)(rt * ROWS));
+        __syncthreads();   // the tile's LDS is free for the next one
+    }
+}
+#define JL_GEMM_I8_KERNEL(T, TYPE, W256, RT, TW, OCC)                                                              \
+    extern "C" __global__ __launch_bounds__(256, OCC) void jl_gemm_i8_##T##_r##RT##t##TW(GemmArgs p) {             \
+        gemm_i8_split_slice<TYPE, W256>(p);                                                                        \
+        gemm_i8_body<TYPE, W256, RT, TW>(p, jl_smem, blockIdx.x * 32 * TW, blockIdx.y * 32 * RT * (4 / TW));       \
+    }                                                                                                              \
+    extern "C" __global__ __launch_bounds__(256, OCC) void jl_moe_gemm_i8_##T##_r##RT##t##TW(MoeGemmArgs p) {      \
+        moe_gemm_i8_tiles<TYPE, W256, RT, TW>(p);                                                                  \
+    }
+#define JL_GEMM_I8_SHAPES(T, TYPE, W256, OCC)                                                                      \
+    JL_GEMM_I8_KERNEL(T, TYPE, W256, 4, 4, 2) JL_GEMM_I8_KERNEL(T, TYPE, W256, 2, 4, OCC) JL_GEMM_I8_KERNEL(T, TYPE, W256, 2, 2, OCC)
+JL_GEMM_I8_SHAPES(q8_0, JL_Q8_0, false, 3) JL_GEMM_I8_SHAPES(q4k, JL_Q4_K, false, 2) JL_GEMM_I8_SHAPES(q6k, JL_Q6_K, false, 2)
+JL_GEMM_I8_SHAPES(q6kw, JL_Q6_K, true, 2)
 extern "C" __global__ __launch_bounds__(512) void jl_gemm_q4k_r128(GemmArgs p) {
     gemm_q4k_body<2>(p, jl_smem, blockIdx.x * JL_GEMM_TILE, blockIdx.y * 128);
 }
@@ -340,18 +371,14 @@ extern "C" __global__ __launch_bounds__(256) void jl_moe_g16_prep_planes(MoeG16P
     __shared__ u32 lds[4 * 72];
     moe_g16_prep_body<1>(p, lds);
 }
-extern "C" __global__ __launch_bounds__(256) void jl_moe_g16_prep_q6k(MoeG16PrepArgs p) {
-    __shared__ u32 lds[4 * 72];
-    moe_g16_prep_body<2>(p, lds);
-}
 // _c: fragments from the prep kernel's workspace; _f / _g: the columns (plain / silu(x) * x2) quantized by
-// the kernel itself; _d: groups of 32 columns (two token tiles); g16p: the sheets are packed planes; g16q6: Q6_K rows
+// the kernel itself; _d: groups of 32 columns (two token tiles); g16p: the sheets are packed planes
 #define JL_MOE_G16_FORMS(NAME, KO, CH)                                                                                          \
     extern "C" __global__ __launch_bounds__(512) void jl_moe_##NAME##_c##CH(MoeG16Args p) { moe_g16_body<CH, 0, KO>(p, jl_smem); } \
     extern "C" __global__ __launch_bounds__(512) void jl_moe_##NAME##_f##CH(MoeG16Args p) { moe_g16_body<CH, 1, KO>(p, jl_smem); } \
     extern "C" __global__ __launch_bounds__(512) void jl_moe_##NAME##_g##CH(MoeG16Args p) { moe_g16_body<CH, 2, KO>(p, jl_smem); } \
     extern "C" __global__ __launch_bounds__(512) void jl_moe_##NAME##_d##CH(MoeG16Args p) { moe_g16_body<CH, 0, KO, 2>(p, jl_smem); }
-#define JL_MOE_G16_KERNEL(CH) JL_MOE_G16_FORMS(g16, 0, CH) JL_MOE_G16_FORMS(g16p, 1, CH) JL_MOE_G16_FORMS(g16q6, 2, CH)
+#define JL_MOE_G16_KERNEL(CH) JL_MOE_G16_FORMS(g16, 0, CH) JL_MOE_G16_FORMS(g16p, 1, CH)
 JL_MOE_G16_KERNEL(1) JL_MOE_G16_KERNEL(2) JL_MOE_G16_KERNEL(3)
 // Experts with many columns: the prefill GEMM's 128-token x 64-row tile placed per expert.  An
 // expert's column groups are consecutive slots of the prepared workspace, so to the tile they
@@ -360,7 +387,7 @@ JL_MOE_G16_KERNEL(1) JL_MOE_G16_KERNEL(2) JL_MOE_G16_KERNEL(3)
 // grid = up to two workgroups a CU, block = 256, dynamic LDS as jl_gemm_q4k_r64.
 // PL (Q4_K): the banks are packed planes, an expert's sheet a plane set of its own or a row range
 // of the bank's (MoeGemmArgs.pqs ...); the tile is the plane form of the prefill GEMM's.
-template <int TYPE, bool PL = false>
+template <bool PL>
 __device__ __forceinline__ void moe_gemm_tiles(const MoeGemmArgs& p) {
     const u32 rtiles = (u32)(p.nrows + 63) / 64;
     const u32 ntiles = p.wl[0];
@@ -388,15 +415,12 @@ __device__ __forceinline__ void moe_gemm_tiles(const MoeGemmArgs& p) {
         g.ntok = 32 * slot0 + ncol;                  // tokens are positions in the workspace
         g.out_stride = p.nrows; g.sb_per = 0;
         g.out = p.out[mat] + ((ptrdiff_t)c_lo - (ptrdiff_t)32 * slot0) * p.nrows;   // workspace position -> column
-        if constexpr (TYPE == JL_Q6_K) gemm_q6k_body<true>(g, jl_smem, 32 * slot0 + 128 * ctile, (int)rt * 64);
-        else gemm_q4k_body<1, true, PL>(g, jl_smem, 32 * slot0 + 128 * ctile, (int)rt * 64);
+        gemm_q4k_body<1, true, PL>(g, jl_smem, 32 * slot0 + 128 * ctile, (int)rt * 64);
         __syncthreads();   // the tile's LDS is free for the next one
     }
 }
-extern "C" __global__ __launch_bounds__(256, 2) void jl_moe_gemm_r64(MoeGemmArgs p) { moe_gemm_tiles<JL_Q4_K>(p); }
-extern "C" __global__ __launch_bounds__(256, 2) void jl_moe_gemm_r64_planes(MoeGemmArgs p) { moe_gemm_tiles<JL_Q4_K, true>(p); }
-// Q6_K sheets: dynamic LDS = JL_GEMM6_LDS_BYTES
-extern "C" __global__ __launch_bounds__(256, 2) void jl_moe_gemm_q6k_r64(MoeGemmArgs p) { moe_gemm_tiles<JL_Q6_K>(p); }
+extern "C" __global__ __launch_bounds__(256, 2) void jl_moe_gemm_r64(MoeGemmArgs p) { moe_gemm_tiles<false>(p); }
+extern "C" __global__ __launch_bounds__(256, 2) void jl_moe_gemm_r64_planes(MoeGemmArgs p) { moe_gemm_tiles<true>(p); }
 // grid = 1, block = 1024
 extern "C" __global__ __launch_bounds__(1024) void jl_moe_worklist(MoeWorklistArgs p) {
     __shared__ u32 tot[16];

@@ -1,0 +1,74 @@
+"""The int8 tile kernels (kernels/gemm_i8.h), dense and per expert, at the edges of their tiles: rows and tokens one
+short of, at and one past a tile, K of an odd number of stages, K splits, every shape; against the oracle in f64."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import nmse
+from jitllm_amd import quant, synth
+
+pytestmark = pytest.mark.gpu
+FILL = np.float32(4e30)
+KINDS = [(quant.Q8_0, 32), (quant.Q4_K, 32), (quant.Q6_K, 32), (quant.Q6_K, 256)]
+
+
+@pytest.mark.parametrize("t,window", KINDS, ids=["q8_0", "q4_k", "q6_k", "q6_k-w256"])
+@pytest.mark.parametrize("nrows,k,ntok", [(1, 256, 65), (63, 512, 127), (129, 768, 129), (200, 256, 300), (130, 1280, 66)])
+def test_dense_tiles(dev, devbuf, t, window, nrows, k, ntok):
+    if t == quant.Q8_0 and k == 768:
+        k = 640   # five stages of 128
+    dev.SetActWindow(window)
+    w = synth.random_weights(t, nrows, k, seed=nrows + k)
+    x = np.stack([synth.activations(k, seed=900 + i) * np.float32(1 + i % 3) for i in range(ntok)])
+    want = oracle.matmul_q8act_f64(t, w, x, nrows, k, ntok, window)
+    wd, xd = devbuf(w), devbuf(x)
+    for shape in (0, 1, 2) if t == quant.Q8_0 else (0, 2):
+        for split in (0, 1, 2, 5):
+            dev.set_tuning(gemm__i8=shape, gemm__split=split)
+            o = devbuf(shape=(ntok * nrows + 8,), dtype=np.float32, fill=FILL)
+            assert dev.matmul_dev(o.ptr, t, wd.ptr, xd.ptr, nrows, k, ntok)
+            dev.synchronize()
+            got = o.get()
+            assert np.all(got[ntok * nrows:] == FILL)
+            assert nmse(got[:ntok * nrows].reshape(ntok, nrows), want) <= 1e-10, (shape, split)
+    dev.set_tuning(gemm__i8=0, gemm__split=0)
+    dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("t,window", KINDS, ids=["q8_0", "q4_k", "q6_k", "q6_k-w256"])
+@pytest.mark.parametrize("nrows,k", [(130, 512), (256, 256)])
+def test_tiles_per_expert(dev, devbuf, t, window, nrows, k):
+    """Experts of 0, 1, 31, 64, 65 and 129 columns, two banks, gathered rows, a gated activation; the few-token kernel
+    and every tile."""
+    counts = [1, 0, 31, 64, 65, 129, 0]
+    n_expert, ncols = len(counts), sum(counts)
+    start = np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32)
+    dev.SetActWindow(window)
+    sheet = nrows * quant.row_bytes(t, k)
+    banks = [np.concatenate([synth.random_weights(t, nrows, k, seed=10 * b + e) for e in range(n_expert)]) for b in range(2)]
+    x = np.stack([synth.activations(k, seed=300 + r) for r in range(40)])
+    src = (np.arange(ncols) * 7 % 40).astype(np.uint32)
+    u = np.stack([synth.activations(k, seed=500 + r) for r in range(40)])
+    xg = (x / (1 + np.exp(-x.astype(np.float64))) * u).astype(np.float32)
+    bd, xd, ud, sd, dstart = [devbuf(b) for b in banks], devbuf(x), devbuf(u), devbuf(src), devbuf(start)
+    for gated in (False, True):
+        act = xg if gated else x
+        want = [np.zeros((ncols, nrows)) for _ in banks]
+        for b in range(2):
+            for e in range(n_expert):
+                cols = slice(start[e], start[e + 1])
+                if counts[e]:
+                    want[b][cols] = oracle.matmul_q8act_f64(t, banks[b][e * sheet:(e + 1) * sheet], act[src[cols]], nrows, k, counts[e], window)
+        for form in (0, 5, 6, 7, 8) if t == quant.Q8_0 else (0, 5, 6, 7):
+            dev.set_tuning(moe__form=form)
+            o = [devbuf(shape=(ncols * nrows + 8,), dtype=np.float32, fill=FILL) for _ in banks]
+            assert dev.moe_matvec_dev(o[0].ptr, o[1].ptr, t, bd[0].ptr, bd[1].ptr, xd.ptr, ud.ptr if gated else None, sd.ptr, dstart.ptr,
+                                      n_expert, ncols, nrows, k)
+            dev.synchronize()
+            for b in range(2):
+                got = o[b].get()
+                assert np.all(got[ncols * nrows:] == FILL)
+                # (the gated activation: an exponential of another machine in front of the quantizer)
+                assert nmse(got[:ncols * nrows].reshape(ncols, nrows), want[b]) <= (1e-6 if gated else 1e-10), (gated, form, b)
+    dev.set_tuning(moe__form=0)
+    dev.SetActWindow(32)
