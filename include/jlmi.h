@@ -109,9 +109,10 @@ int jl_synchronize(jl_ctx *ctx);
  * "moe.group" / "moe.logits" / "moe.q6k_cols" / "moe.waves" / "moe.lpr" (forms of the mixture
  * block's other kernels),
  * "mxfp4.split" (K slices of the MXFP4 GEMM), "mxfp4.rows" (96 or 128 rows a tile; 1: the
- * general decode matvec also for one token), "mxfp4.planes" (packed MXFP4: 2 restores rows
- * first, 3 the plane GEMM whatever the grid, 64 / 32 / 16 rows a workgroup of the plane
- * matvec); value 0 restores the built-in choice.  These change launch shapes and f32 summation
+ * general decode matvec also for one token), "mxfp4.few" / "mxfp4.few_min" (the MXFP4
+ * few-token form up to / from this many tokens), "mxfp4.planes" (3 / 4: 64-token tiles of 64 / 96
+ * rows over planes, rows turned into planes first; packed MXFP4: 2 restores rows first,
+ * 64 / 32 / 16 rows a workgroup of the plane matvec); value 0 restores the built-in choice.  These change launch shapes and f32 summation
  * order only.  Two keys change values, both off unless set: "mxfp4.scaled" = 1 runs
  * jl_matmul_mxfp4_packed_bf16_dev on the block-scaled fp8 x fp4 matrix instruction, which
  * quantizes the activations to MX fp8 (rel-L2 about 2.7e-2 against the bf16 activations);

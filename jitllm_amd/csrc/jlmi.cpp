@@ -53,9 +53,10 @@ struct Tuning {
     int moe_lpr = 0;
     int mx_rows = 0;
     int mx_scaled = 0;          // 1: packed MXFP4 matmul on the block-scaled fp8 x fp4 matrix instruction (lossy)
-    int mx_planes = 0;          // packed MXFP4: 2 restores rows first, 3 the plane GEMM whatever the grid; 64 / 32 / 16
-                                // rows a workgroup of the plane matvec
+    int mx_planes = 0;          // packed MXFP4: 2 restores rows first; 64 / 32 / 16 rows a workgroup of the plane
+                                // matvec; rows and planes: 3 / 4 the tiles of 64 / 96 rows
     int mx_split = 0;
+    int mx_few = 0, mx_few_min = 0;   // MXFP4: the few-token form up to / from this many tokens
 };
 
 // The code object's kernels by name.  Looked up on every launch, so without a string to allocate or a tree to
@@ -1647,7 +1648,7 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     if (e != hipSuccess)
         return bail(JL_ERR_HIP, "hipModuleLoad(" + path + "): " + H->GetErrorString(e));
 
-    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_group", "jl_moe_group2", "jl_moe_group2_wide", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_silu_mul", "jl_add_rows", "jl_host_in", "jl_host_done", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
+    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_group", "jl_moe_group2", "jl_moe_group2_wide", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_few_planes_t1", "jl_mxfp4_few_planes_t2", "jl_mxfp4_few_planes_t3", "jl_mxfp4_few_planes_t4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_planes_gemm_r96", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_silu_mul", "jl_add_rows", "jl_host_in", "jl_host_done", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
                                       "jl_pack_weights", "jl_unpack_q4k", "jl_unpack_q6k", "jl_unpack_q8_0"};
     names.push_back("jl_few_prep");
     names.push_back("jl_gemm_i8_prep");
@@ -1785,6 +1786,8 @@ int jl_set_tuning(jl_ctx* c, const char* key, int value) {
     else if (!strcmp(key, "moe.lpr")) c->tune.moe_lpr = value;
     else if (!strcmp(key, "gemm.rows")) c->tune.gemm_rows = value;
     else if (!strcmp(key, "mxfp4.split")) c->tune.mx_split = value;
+    else if (!strcmp(key, "mxfp4.few")) c->tune.mx_few = value;
+    else if (!strcmp(key, "mxfp4.few_min")) c->tune.mx_few_min = value;
     else if (!strcmp(key, "mxfp4.rows")) c->tune.mx_rows = value;
     else if (!strcmp(key, "mxfp4.planes")) c->tune.mx_planes = value;
     else if (!strcmp(key, "mxfp4.scaled")) c->tune.mx_scaled = value;
@@ -2572,6 +2575,77 @@ int jl_layer_ffn_dev(jl_ctx* c, int li, const float* h, float* resid, int n, voi
     return JL_OK;
 }
 
+namespace {
+// Few tokens: 16-row workgroups whose wavefronts split K, in chunks of up to 64 tokens, one launch after a prep
+// that lays the activations out in the order the block decode produces.
+// From where: the kernels for a handful of tokens grow by about a microsecond a token, this one does not, but its
+// prep is a launch (us at 2880 x 2880, rows: 4 tokens 7.4 against 7.3, 8 tokens 11.8 against 7.4; planes: 3 tokens
+// 6.2 against 6.9, 4 tokens 7.0 against 6.8; at 1100 x 1216 the handful's are as fast up to 8).
+// Up to where: a chunk more costs little while the grid is one round of the CUs (rows 2880 x 2880: 128 tokens 16.1
+// against the tiles' 17.5, 192 tokens 21.5 against 18.2; 1100 x 1216: 192 tokens 8.6 against 10.1; planes, whose tiles
+// have no rows to turn: 96 tokens 13.0 against 12.7, 2000 x 4512 12.6 against 15.6).
+bool mx_few_applies(const jl_ctx* c, int nrows, int k, int ntok, bool planes) {
+    if (c->tune.mx_rows == 96 || c->tune.mx_rows == 128 || ntok > 65535) return false;
+    const int form = c->tune.mx_planes;
+    if (form == 3 || form == 4 || (planes && (form == 2 || (form && ntok <= 8)))) return false;
+    const int least = c->tune.mx_few_min > 0 ? c->tune.mx_few_min : (long)nrows * k < 4000000 ? 9 : planes ? 4 : 5;
+    if (ntok < least) return false;
+    if (c->tune.mx_few > 0) return ntok <= c->tune.mx_few;
+    return ntok <= (planes ? 64 : 128) || (ntok <= 256 && (long)((nrows + 15) / 16) * ((ntok + 63) / 64) <= c->num_cu);
+}
+int mx_few_launch(jl_ctx* c, MxGemmArgs& a, const uint16_t* x, hipStream_t st) {
+    const int tiles = (a.ntok + 15) / 16, groups = (a.k + 127) / 128, chunks = (tiles + 3) / 4, nt = (tiles + chunks - 1) / chunks;
+    int rc = gemm_ws_ensure(c, (size_t)groups * 4 * tiles * 1024);
+    if (rc != JL_OK) return rc;
+    MxPrepArgs pa;
+    pa.x = x; pa.xf = (uint16_t*)c->gemm_ws; pa.ntok = a.ntok; pa.tok_pad = 16 * tiles; pa.k = a.k;
+    void* pp[] = {&pa};
+    rc = launch(c, "jl_mxfp4_prep_few", (unsigned)groups, (unsigned)tiles, 256, 0, st, pp);
+    if (rc != JL_OK) return rc;
+    a.x = (const uint16_t*)c->gemm_ws; a.tok_pad = 16 * tiles;
+    void* params[] = {&a};
+    Name name;
+    name << "jl_mxfp4_few_" << (a.qs ? "planes_t" : "t") << nt;
+    return launch(c, name, (unsigned)((a.nrows + 15) / 16), (unsigned)((tiles + nt - 1) / nt), 512, 0, st, params);
+}
+// Tiles of 64 tokens x 64 or 96 rows whose wavefronts split K, the weights taken from planes; rows (w) are turned
+// into planes in the workspace by the launch that lays the activations out.
+// Rows a tile: a round of the CUs takes about 1.36 times as long with 96 (measured at k = 1216 to 4512), so 96 where
+// that saves the rounds (2880 rows: 512 tokens 21.1 -> 17.4 us, 384 tokens of 5000 rows 19.7 against 23.7).
+double mx_tile_rounds(const jl_ctx* c, int nrows, int ntok, int* trows) {
+    auto rounds = [&](int rows) {
+        return (double)(((long)((ntok + 63) / 64) * ((nrows + rows - 1) / rows) + c->num_cu - 1) / c->num_cu);
+    };
+    const double r64 = rounds(64), r96 = 1.36 * rounds(96);
+    *trows = c->tune.mx_planes == 3 ? 64 : c->tune.mx_planes == 4 ? 96 : r96 < r64 ? 96 : 64;
+    return *trows == 96 ? r96 : r64;
+}
+int mx_tile_launch(jl_ctx* c, MxPlanesGemmArgs& a, const uint8_t* w, const uint16_t* x, hipStream_t st) {
+    const int tok_pad = (a.ntok + 63) / 64 * 64, nks = (a.k + 63) / 64, ntt = tok_pad / 32, nblk = a.k / 32;
+    int trows;
+    (void)mx_tile_rounds(c, a.nrows, a.ntok, &trows);
+    const long tiles = (long)(tok_pad / 64) * ((a.nrows + trows - 1) / trows), stride = (a.nrows + 63) / 64 * 64;
+    const long nx = (long)((nks + 3) / 4) * ntt, nw = w ? (stride / 64) * ((nblk + 15) / 16) : 0;
+    if (tiles > 0x7fffffffL / 2 || nx + nw > 0x7fffffffL) return JL_DECLINED;
+    const size_t xa_bytes = (size_t)nks * ntt * 4 * 1024, qs_bytes = w ? (size_t)nblk * 16 * stride : 0;
+    int rc = gemm_ws_ensure(c, xa_bytes + qs_bytes + (w ? (size_t)nblk * stride : 0));
+    if (rc != JL_OK) return rc;
+    MxPlanesPrepArgs pa;
+    pa.x = x; pa.xa = (uint32_t*)c->gemm_ws; pa.ntok = a.ntok; pa.tok_pad = tok_pad; pa.k = a.k;
+    if (w) {
+        pa.w = w; pa.qs = (uint32_t*)((char*)c->gemm_ws + xa_bytes); pa.d = (uint32_t*)((char*)pa.qs + qs_bytes);
+        pa.nrows = a.nrows; pa.stride = (int)stride;
+        a.qs = pa.qs; a.d = pa.d; a.row0 = 0; a.stride = (int)stride;
+    }
+    void* pp[] = {&pa};
+    rc = launch(c, "jl_mxfp4_planes_prep", (unsigned)(nx + nw), 1, 256, 0, st, pp);
+    if (rc != JL_OK) return rc;
+    a.xa = pa.xa; a.tok_pad = tok_pad;
+    void* gp[] = {&a};
+    return launch(c, trows == 96 ? "jl_mxfp4_planes_gemm_r96" : "jl_mxfp4_planes_gemm", (unsigned)(8 * ((tiles + 7) / 8)), 1, 256, (unsigned)(trows / 32 * 16384), st, gp);
+}
+}  // namespace
+
 int jl_matmul_mxfp4_bf16_dev(jl_ctx* c, float* out, const void* w, const uint16_t* x, int nrows, int k,
                              int ntok, void* stream) {
     if (!c) return JL_ERR_ARG;
@@ -2595,38 +2669,11 @@ int jl_matmul_mxfp4_bf16_dev(jl_ctx* c, float* out, const void* w, const uint16_
         // 2880 rows and left 76 CUs without one: 4.65 -> 4.18 us)
         return launch(c, name, (unsigned)((nrows + JL_MX1_RPW - 1) / JL_MX1_RPW), 1, 64, 0, st, params);
     }
+    if (mx_few_applies(c, nrows, k, ntok, false)) return mx_few_launch(c, a, x, st);
     if (ntok <= 8)  // a handful of tokens: stream the rows once, no tile to fill
         return launch(c, "jl_mxfp4_matvec", (unsigned)((nrows + 3) / 4), 1, 256, 0, st, params);
-    if (ntok <= 64 && c->tune.mx_rows != 96 && c->tune.mx_rows != 128) {
-        // few tokens: 16-row workgroups whose wavefronts split K, one launch after a prep
-        // that lays the activations out in the order the block decode produces
-        const int nt = (ntok + 15) / 16, groups = (k + 127) / 128;
-        int rc = gemm_ws_ensure(c, (size_t)groups * 4 * nt * 1024);
-        if (rc != JL_OK) return rc;
-        MxPrepArgs pa;
-        pa.x = x; pa.xf = (uint16_t*)c->gemm_ws; pa.ntok = ntok; pa.tok_pad = 16 * nt; pa.k = k;
-        void* pp[] = {&pa};
-        rc = launch(c, "jl_mxfp4_prep_few", (unsigned)groups, (unsigned)nt, 256, 0, st, pp);
-        if (rc != JL_OK) return rc;
-        a.x = (const uint16_t*)c->gemm_ws; a.tok_pad = 16 * nt;
-        Name name;
-        name << "jl_mxfp4_few_t" << nt;
-        return launch(c, name, (unsigned)((nrows + 15) / 16), 1, 512, 0, st, params);
-    }
-    const unsigned lds = 2u * 128u * 264u * 2u;   // two weight stages [128][264] bf16
-    if (lds > c->lds_limit) return JL_DECLINED;
     // activations into matrix-fragment order (tokens padded to whole tiles, K to whole stages)
     const int tok_pad = (ntok + 127) / 128 * 128, stages = (k + 255) / 256;
-    int rc = gemm_ws_ensure(c, (size_t)stages * (tok_pad / 32) * 16 * 1024);
-    if (rc != JL_OK) return rc;
-    MxPrepArgs pa;
-    pa.x = x; pa.xf = (uint16_t*)c->gemm_ws; pa.ntok = ntok; pa.tok_pad = tok_pad; pa.k = k;
-    void* pp[] = {&pa};
-    rc = launch(c, "jl_mxfp4_prep", (unsigned)stages, (unsigned)(tok_pad / 32), 256, 0, st, pp);
-    if (rc != JL_OK) return rc;
-    a.x = (const uint16_t*)c->gemm_ws; a.tok_pad = tok_pad;
-    // A grid that leaves most CUs idle is widened along K: each split writes partial sums
-    // to a workspace slab and a second kernel adds the slabs in order.
     // rows per tile: 128, or 96 where that takes fewer rounds x rows (2880 rows x 1024 tokens:
     // 184 tiles of 128 rows leave 72 CUs idle for a whole tile, 240 of 96 rows do not)
     auto cost = [&](int rows) {
@@ -2637,13 +2684,37 @@ int jl_matmul_mxfp4_bf16_dev(jl_ctx* c, float* out, const void* w, const uint16_
                       : (cost(96) < cost(128) ? 96 : 128);
     const char* gemm_name = trows == 96 ? "jl_mxfp4_gemm_r96" : "jl_mxfp4_gemm";
     const int tiles = (tok_pad / 128) * ((nrows + trows - 1) / trows);
+    // A grid that leaves most CUs idle is widened along K: each split writes partial sums
+    // to a workspace slab and a second kernel adds the slabs in order.
     int nsplit = c->tune.mx_split > 0 ? c->tune.mx_split : (tiles * 2 <= c->num_cu ? c->num_cu / tiles : 1);
     if (nsplit > 8) nsplit = 8;
     if (nsplit > stages) nsplit = stages;
-    if (nsplit > 1) {
-        const int per = (stages + nsplit - 1) / nsplit;
-        nsplit = (stages + per - 1) / per;   // no empty split
+    int per = (stages + nsplit - 1) / nsplit;
+    nsplit = (stages + per - 1) / per;   // no empty split
+    // These tiles, or the smaller ones of the planes with the rows turned into planes on the way: by their costs as
+    // measured (us; 1100 x 1216 to 5000 x 2048, 64 to 2048 tokens).  These: a stage of K = 256 takes 2.15 with 96 rows
+    // and 2.9 with 128, a split a launch and its slabs; those: 1 a MB of weights and 2.75 a round and 1024 of K.  The
+    // estimates are good to about 8 %, so those only where they win by more (2880 x 2880: 512 tokens 27.9 -> 21.8, 1024
+    // tokens 31.5 against 32.3, 2048 tokens 57 -> 52).
+    int mtrows;
+    const double rounds = mx_tile_rounds(c, nrows, ntok, &mtrows), mb = 1e-6 * nrows * (double)a.row_bytes;
+    const double small_us = 6 + mb + 2.75 * k / 1024 * rounds;
+    const double large_us = 7 + (double)cost(trows) / trows * per * (trows == 96 ? 2.15 : 2.9) +
+                            (nsplit > 1 ? 3.5 + (double)ntok * nrows * nsplit * 4 / 3e6 : 0);
+    const unsigned lds = 2u * 128u * 264u * 2u;   // two weight stages [128][264] bf16
+    if (c->tune.mx_planes == 3 || c->tune.mx_planes == 4 || lds > c->lds_limit || (!c->tune.mx_rows && !c->tune.mx_split && 1.08 * small_us < large_us)) {
+        MxPlanesGemmArgs ga;
+        ga.out = out; ga.nrows = nrows; ga.k = k; ga.ntok = ntok;
+        return mx_tile_launch(c, ga, (const uint8_t*)w, x, st);
     }
+    int rc = gemm_ws_ensure(c, (size_t)stages * (tok_pad / 32) * 16 * 1024);
+    if (rc != JL_OK) return rc;
+    MxPrepArgs pa;
+    pa.x = x; pa.xf = (uint16_t*)c->gemm_ws; pa.ntok = ntok; pa.tok_pad = tok_pad; pa.k = k;
+    void* pp[] = {&pa};
+    rc = launch(c, "jl_mxfp4_prep", (unsigned)stages, (unsigned)(tok_pad / 32), 256, 0, st, pp);
+    if (rc != JL_OK) return rc;
+    a.x = (const uint16_t*)c->gemm_ws; a.tok_pad = tok_pad;
     if (nsplit > 1) {
         const size_t n = (size_t)ntok * nrows;
         rc = ws_ensure(c, &c->mx_ws, &c->mx_ws_bytes, n * nsplit * 4);
@@ -2694,7 +2765,14 @@ int jl_matmul_mxfp4_packed_bf16_dev(jl_ctx* c, float* out, const uint32_t* qs, c
         if (stiles > 0x7fffffffL / 2) return JL_DECLINED;
         return launch(c, "jl_mxfp4_scaled_gemm", (unsigned)(8 * ((stiles + 7) / 8)), 1, 256, 65536, st, gp);
     }
-    if (ntok <= 8 && c->tune.mx_planes != 2) {
+    if (mx_few_applies(c, nrows, k, ntok, true)) {
+        MxGemmArgs a;
+        a.out = out; a.w = nullptr; a.x = x; a.nrows = nrows; a.k = k; a.ntok = ntok; a.row_bytes = 0;
+        a.nsplit = 1; a.part = nullptr; a.tok_pad = 0;
+        a.qs = qs; a.d = d; a.row0 = row; a.stride = stride;
+        return mx_few_launch(c, a, x, st);
+    }
+    if (ntok <= 8 && (c->tune.mx_planes < 2 || c->tune.mx_planes > 4)) {
         // a handful of tokens: the planes are read where they lie, a lane a row
         MxPlanesArgs a;
         a.out = out; a.qs = qs; a.d = d; a.x = (const uint32_t*)x;
@@ -2710,27 +2788,13 @@ int jl_matmul_mxfp4_packed_bf16_dev(jl_ctx* c, float* out, const uint32_t* qs, c
         return launch(c, name, (unsigned)((nrows + rl - 1) / rl), 1, (unsigned)(64 * a.nwaves),
                       (unsigned)(a.nwaves * 8 * 64 * 4), st, params);
     }
-    // a grid of 64 x 64 tiles that gives most CUs a workgroup: the planes feed the matrix
-    // instruction's weight operand as they lie (a plane word is a lane's eight K values)
-    const long tiles = (long)((ntok + 63) / 64) * ((nrows + 63) / 64);
-    if (c->tune.mx_planes != 2 && (c->tune.mx_planes == 3 || 2 * tiles >= c->num_cu) && ntok <= 65535 * 32 &&
-        k % 8 == 0 && 65536u <= c->lds_limit) {
-        const int tok_pad = (ntok + 63) / 64 * 64, nks = (k + 63) / 64, ntt = tok_pad / 32;
-        rc = gemm_ws_ensure(c, (size_t)nks * ntt * 4 * 1024);
-        if (rc != JL_OK) return rc;
-        MxPlanesPrepArgs pa;
-        pa.x = x; pa.xa = (uint32_t*)c->gemm_ws; pa.ntok = ntok; pa.tok_pad = tok_pad; pa.k = k;
-        void* pp[] = {&pa};
-        rc = launch(c, "jl_mxfp4_planes_prep", (unsigned)((nks + 3) / 4), (unsigned)ntt, 256, 0, st, pp);
-        if (rc != JL_OK) return rc;
+    // the planes feed the matrix instruction's weight operand as they lie (a plane word is a lane's eight K values)
+    if (c->tune.mx_planes != 2 && ntok <= 65535 * 32 && 49152u <= c->lds_limit) {
         MxPlanesGemmArgs ga;
-        ga.out = out; ga.qs = qs; ga.d = d; ga.xa = pa.xa;
-        ga.nrows = nrows; ga.k = k; ga.ntok = ntok; ga.tok_pad = tok_pad; ga.row0 = row; ga.stride = stride;
-        void* gp[] = {&ga};
-        if (tiles > 0x7fffffffL / 2) return JL_DECLINED;
-        return launch(c, "jl_mxfp4_planes_gemm", (unsigned)(8 * ((tiles + 7) / 8)), 1, 256, 65536, st, gp);
+        ga.out = out; ga.qs = qs; ga.d = d; ga.nrows = nrows; ga.k = k; ga.ntok = ntok; ga.row0 = row; ga.stride = stride;
+        return mx_tile_launch(c, ga, nullptr, x, st);
     }
-    // fewer tiles: the few-token and tiled forms stage GGUF blocks, so the rows are restored first
+    // (asked for by tuning) the forms over GGUF rows: the rows are restored first
     rc = ws_ensure(c, &c->unpack_ws, &c->unpack_ws_bytes, (size_t)nrows * (size_t)(k / 32) * 17);
     if (rc != JL_OK) return rc;
     rc = unpack_launch(c, JL_TYPE_MXFP4, pl, nrows, k, c->unpack_ws, st);

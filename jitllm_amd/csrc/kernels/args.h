@@ -335,6 +335,10 @@ struct MxGemmArgs {
     int row_bytes;
     int nsplit;           // workgroups along K (grid z); > 1: partial sums go to part
     float* part;          // [nsplit][ntok][nrows], summed by jl_sum_parts
+    // the few-token kernel over packed planes (w unused): rows row0 .. of planes of `stride` rows
+    const uint32_t* qs = nullptr;
+    const uint32_t* d = nullptr;
+    int row0 = 0, stride = 0;
 };
 
 // MXFP4 planes x a handful of bf16 tokens: rows row0 .. row0+nrows of planes of `stride` rows.
@@ -353,6 +357,11 @@ struct MxPlanesPrepArgs {
     const uint16_t* x;    // [ntok][k] bf16 bits
     uint32_t* xa;         // [K-step of 64][token tile of 32][4 matrix K-steps][64 lanes][4 words]
     int ntok, tok_pad, k;
+    // GGUF rows to turn into planes on the way (null: the weights are planes already)
+    const uint8_t* w = nullptr;
+    uint32_t* qs = nullptr;
+    uint32_t* d = nullptr;
+    int nrows = 0, stride = 0;   // stride a multiple of 64
 };
 
 struct MxPlanesGemmArgs {

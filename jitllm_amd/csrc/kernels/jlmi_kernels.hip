@@ -450,7 +450,10 @@ extern "C" __global__ __launch_bounds__(1024) void jl_mxfp4_matvec_planes_r16(Mx
 // block = 256; GEMM grid = 8 * ceil(tiles of 64 x 64 / 8), block = 256, dynamic LDS = 64 KiB
 extern "C" __global__ __launch_bounds__(256) void jl_mxfp4_planes_prep(MxPlanesPrepArgs p) { mx_planes_prep_body(p); }
 extern "C" __global__ __launch_bounds__(256, 2) void jl_mxfp4_planes_gemm(MxPlanesGemmArgs p) {
-    mx_planes_gemm_body(p, (float*)jl_smem);
+    mx_planes_gemm_body<2>(p, (float*)jl_smem);
+}
+extern "C" __global__ __launch_bounds__(256, 2) void jl_mxfp4_planes_gemm_r96(MxPlanesGemmArgs p) {
+    mx_planes_gemm_body<3>(p, (float*)jl_smem);
 }
 // the opt-in block-scaled form over packed planes: prep grid = (ceil(ceil(k/64) / 4), tok_pad/32),
 // block = 256; GEMM grid = 8 * ceil(tiles of 64 x 64 / 8), block = 256, dynamic LDS = 64 KiB
@@ -465,6 +468,10 @@ extern "C" __global__ __launch_bounds__(256) void jl_mxfp4_prep_few(MxPrepArgs p
     extern "C" __global__ __launch_bounds__(512) void jl_mxfp4_few_t##NT(MxGemmArgs p) {       \
         __shared__ __attribute__((aligned(16))) float part[8 * NT * 256];                      \
         mx_few_body<NT>(p, part);                                                              \
+    }                                                                                          \
+    extern "C" __global__ __launch_bounds__(512) void jl_mxfp4_few_planes_t##NT(MxGemmArgs p) { \
+        __shared__ __attribute__((aligned(16))) float part[8 * NT * 256];                      \
+        mx_few_body<NT, true>(p, part);                                                        \
     }
 JL_MX_FEW_KERNEL(1) JL_MX_FEW_KERNEL(2) JL_MX_FEW_KERNEL(3) JL_MX_FEW_KERNEL(4)
 

@@ -483,10 +483,12 @@ __device__ __forceinline__ void mx_planes_matvec_body(const MxPlanesArgs& p, flo
 // conversions with the block's scale.  The word holds elements 4w..4w+3 in its low nibbles and
 // 4w+16..4w+19 in its high ones, and a conversion gives a byte's pair, so the operand's K order
 // is 4w, 4w+16, 4w+1, 4w+17, ...; the prep kernel lays the activation fragments out in that order.
-// A workgroup owns 64 tokens x 64 rows (2 x 2 tiles) and its four wavefronts take the K-steps of
-// 64 (two blocks) in turn: many small workgroups, so a CU holds enough wavefronts to cover the
-// trip to memory; the four partial tiles meet in LDS in wavefront order, wavefront w finishing
-// tile w (red: [wavefront][tile][16][64] floats).
+// A workgroup owns 64 tokens x 32 RT rows (2 x RT tiles) and its four wavefronts take the K-steps
+// of 64 (two blocks) in turn: many small workgroups, so a CU holds enough wavefronts to cover the
+// trip to memory; the four partial tiles meet in LDS in wavefront order, a token tile at a time
+// (red: [wavefront][row tile][16][64] floats).  The activation fragments are most of what a K-step
+// takes from L2, so RT = 3 does more with them (2880 x 2880, 2048 tokens: 50.6 -> 47.6 us) and,
+// chosen where its tiles go into fewer rounds of the CUs, is worth more (512 tokens 21.1 -> 17.4).
 //
 // Tile of workgroup L in a 1-D grid of 8 * ceil(tiles / 8): the hardware deals consecutive
 // workgroups round the eight XCDs, each with an L2 of its own, so XCD x = L % 8 is given a
@@ -501,10 +503,41 @@ __device__ __forceinline__ bool mx_xcd_tile(int ntt64, int nrt, int& tt, int& rt
     return true;
 }
 
-// prep: grid = (ceil(K-steps / 4), tok_pad / 32), block = 256: a wavefront per (K-step, 32 tokens)
-__device__ __forceinline__ void mx_planes_prep_body(const MxPlanesPrepArgs& p) {
-    const int lane = threadIdx.x & 63, nks = (p.k + 63) / 64, ntt = p.tok_pad / 32;
-    const int ks = blockIdx.x * 4 + (threadIdx.x >> 6), tile = blockIdx.y;
+// prep, block = 256: the first ceil(K-steps / 4) * (tok_pad / 32) workgroups lay the activations out, a wavefront per
+// (K-step, 32 tokens); for GGUF rows (p.w) ceil(nrows / 64) * ceil(blocks / 16) more turn the weights into planes of
+// `stride` rows, a wavefront per 64 rows x 4 blocks, a lane a row.  Measured: about 1 us per MB of weights, of which
+// most is the planes' way out to memory and back to the other XCDs (taking the rows through LDS, so that their lines
+// are read side by side, was 1 us slower).  Tiles that read the rows themselves take a scattered 17-byte block per lane
+// and 64 tokens instead: 2880 x 2880, 1024 tokens 48 us against 32.
+__device__ __forceinline__ void mx_planes_prep_body(const MxPlanesPrepArgs& args) {
+    MxPlanesPrepArgs p = args;
+    JL_NOW(p.x, p.xa, p.ntok, p.tok_pad, p.k, p.w, p.qs, p.d, p.nrows, p.stride);
+    p.x = as_global(p.x); p.xa = as_global(p.xa); p.w = as_global(p.w); p.qs = as_global(p.qs); p.d = as_global(p.d);
+    const int lane = threadIdx.x & 63, nks = (p.k + 63) / 64, ntt = p.tok_pad / 32, nkx = (nks + 3) / 4, nx = nkx * ntt;
+    if ((int)blockIdx.x >= nx) {
+        const int g = (int)blockIdx.x - nx, nrt = (p.nrows + 63) / 64, nblk = p.k / 32;
+        const int bt = g / nrt, row = (g - bt * nrt) * 64 + lane, b0 = bt * 16 + 4 * (int)(threadIdx.x >> 6);
+        const uint8_t* wr = p.w + (size_t)min(row, p.nrows - 1) * ((size_t)nblk * 17);
+        u32x4 q[4];
+        uint8_t e[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint8_t* blk = wr + (size_t)min(b0 + i, nblk - 1) * 17;
+            e[i] = blk[0];
+            q[i] = ld16_a1(blk + 1);
+        }
+        // (rows past the last fill the planes up to a whole tile of 64)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (b0 + i >= nblk) break;
+            u32* qd = p.qs + (size_t)(b0 + i) * 4 * p.stride + row;
+#pragma unroll
+            for (int s = 0; s < 4; s++) qd[(size_t)s * p.stride] = q[i][s];
+            ((uint8_t*)p.d)[(size_t)(b0 + i) * p.stride + row] = (uint8_t)(e[i] - 1);
+        }
+        return;
+    }
+    const int tile = (int)blockIdx.x / nkx, ks = ((int)blockIdx.x - tile * nkx) * 4 + (int)(threadIdx.x >> 6);
     if (ks >= nks) return;
     const int t = 32 * tile + (lane & 31), kg = lane >> 5, nblk = p.k / 32;
     u32x4* dst = (u32x4*)p.xa + ((size_t)ks * ntt + tile) * 4 * 64 + lane;
@@ -525,20 +558,24 @@ __device__ __forceinline__ void mx_planes_prep_body(const MxPlanesPrepArgs& p) {
     }
 }
 
-// grid = 8 * ceil(tiles / 8) (mx_xcd_tile), block = 256, dynamic LDS = 64 KiB
-__device__ __forceinline__ void mx_planes_gemm_body(const MxPlanesGemmArgs& p, float* red) {
+// grid = 8 * ceil(tiles / 8) (mx_xcd_tile), block = 256, dynamic LDS = RT * 16 KiB
+template <int RT>
+__device__ __forceinline__ void mx_planes_gemm_body(const MxPlanesGemmArgs& args, float* red) {
+    MxPlanesGemmArgs p = args;
+    JL_NOW(p.out, p.qs, p.d, p.xa, p.nrows, p.k, p.ntok, p.tok_pad, p.row0, p.stride);
+    p.qs = as_global(p.qs); p.d = as_global(p.d); p.out = as_global(p.out); p.xa = as_global(p.xa);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     int tt, rt;
-    if (!mx_xcd_tile(p.tok_pad / 64, (p.nrows + 63) / 64, tt, rt)) return;
-    const int t0 = tt * 64, r0 = rt * 64;
+    if (!mx_xcd_tile(p.tok_pad / 64, (p.nrows + 32 * RT - 1) / (32 * RT), tt, rt)) return;
+    const int t0 = tt * 64, r0 = rt * 32 * RT;
     const int nblk = p.k / 32, nks = (p.k + 63) / 64, ntt = p.tok_pad / 32, kg = lane >> 5;
     const size_t n = (size_t)p.stride, dwords = (n + 3) / 4;
     // every load is a uniform base (scalar registers) plus a 32-bit lane offset
-    u32 qoff[2][2], doff[2];
-    int sh[2];
+    u32 qoff[RT][2], doff[RT];
+    int sh[RT];
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
+    for (int j = 0; j < RT; j++) {
         const u32 row = (u32)p.row0 + (u32)min(r0 + 32 * j + (lane & 31), p.nrows - 1);
         sh[j] = 8 * (int)(row & 3);
         doff[j] = row >> 2;
@@ -548,7 +585,7 @@ __device__ __forceinline__ void mx_planes_gemm_body(const MxPlanesGemmArgs& p, f
     // [row tile][matrix K-step], [row tile][block]; past: the K-step's second block lies beyond K
     // (its codes are zeroed where they are used: a select on the loaded words here would put the
     // wait for the load right behind the load)
-    struct WOps { u32 q[2][4]; u32 d[2][2]; bool past; };
+    struct WOps { u32 q[RT][4]; u32 d[RT][2]; bool past; };
     struct AOps { u32x4 a[2][4]; };                // [token tile][matrix K-step]
     auto load_w = [&](int ks, WOps& o) {
         ks = min(ks, nks - 1);
@@ -560,7 +597,7 @@ __device__ __forceinline__ void mx_planes_gemm_body(const MxPlanesGemmArgs& p, f
             const u32* qb = p.qs + bc * 4 * n;
             const u32* db = p.d + bc * dwords;
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
+            for (int j = 0; j < RT; j++) {
 #pragma unroll
                 for (int s = 0; s < 2; s++) {
                     o.q[j][2 * bi + s] = qb[qoff[j][s]];
@@ -579,18 +616,18 @@ __device__ __forceinline__ void mx_planes_gemm_body(const MxPlanesGemmArgs& p, f
             for (int s4 = 0; s4 < 4; s4++) o.a[i][s4] = *(const u32x4*)(ab + aoff + s4 * 256);
         }
     };
-    f32x16_t acc[2][2];
+    f32x16_t acc[2][RT];
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < RT; j++)
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
     auto compute = [&](const WOps& wo, const AOps& ao) {
 #pragma unroll
         for (int s4 = 0; s4 < 4; s4++) {
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
+            for (int j = 0; j < RT; j++) {
                 const float scale = mx_scale((uint8_t)(((wo.d[j][s4 >> 1] >> sh[j]) & 0xFF) + 1));
                 const u32 q = (s4 >> 1) && wo.past ? 0u : wo.q[j][s4];
                 u32x4 wb;
@@ -632,22 +669,27 @@ __device__ __forceinline__ void mx_planes_gemm_body(const MxPlanesGemmArgs& p, f
         JL_MXP_STEP(5, w1, a0, w2, a1)
     }
 #undef JL_MXP_STEP
+    // a token tile at a time, so that two workgroups' shares of LDS fit a CU; a wavefront finishes a quarter of each tile
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < 2; i++) {
+        if (i) __syncthreads();
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < RT; j++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) red[((wave * 4 + 2 * i + j) * 16 + e) * 64 + lane] = acc[i][j][e];
-    __syncthreads();
-    const int i = wave >> 1, j = wave & 1;
-    const int r = r0 + 32 * j + (lane & 31);
+            for (int e = 0; e < 16; e++) red[((wave * RT + j) * 16 + e) * 64 + lane] = acc[i][j][e];
+        __syncthreads();
 #pragma unroll
-    for (int e = 0; e < 16; e++) {
-        float s = red[((0 * 4 + wave) * 16 + e) * 64 + lane];
+        for (int j = 0; j < RT; j++) {
+            const int r = r0 + 32 * j + (lane & 31);
 #pragma unroll
-        for (int w = 1; w < 4; w++) s += red[((w * 4 + wave) * 16 + e) * 64 + lane];
-        const int t = t0 + 32 * i + 8 * (e >> 2) + 4 * kg + (e & 3);
-        if (r < p.nrows && t < p.ntok) p.out[(size_t)t * p.nrows + r] = s;
+            for (int m = 0; m < 4; m++) {
+                float s = red[(j * 16 + 4 * wave + m) * 64 + lane];
+#pragma unroll
+                for (int w = 1; w < 4; w++) s += red[((w * RT + j) * 16 + 4 * wave + m) * 64 + lane];
+                const int t = t0 + 32 * i + 8 * wave + 4 * kg + m;
+                if (r < p.nrows && t < p.ntok) p.out[(size_t)t * p.nrows + r] = s;
+            }
+        }
     }
 }
 
@@ -850,16 +892,35 @@ __device__ __forceinline__ void mx_prep_few_body(const MxPrepArgs& p) {
     ((u16x8*)p.xf)[(((size_t)G * 4 + j) * ntiles + tile) * 64 + lane] = o;
 }
 
-// grid = ceil(nrows / 16), block = 512, static LDS = 8 x NT x 1 KiB; p.x is the prep's
-// workspace, p.tok_pad = 16 * NT.
-template <int NT>
-__device__ __forceinline__ void mx_few_body(const MxGemmArgs& p, float* part) {
+// PL: the weights are packed planes, read where they lie: word j of a block is a plane of its own, so a K-step's
+// load is sixteen rows' words side by side for each of the four blocks.  (Restoring rows first was a launch of 5 us
+// in front: 2880 x 2880, 64 tokens 14.5 us.)  Workgroups go round the eight XCDs in the order of their ids: each XCD
+// is given a run of consecutive row tiles, whose words share lines.
+// grid = (ceil(nrows / 16), token chunks of 16 NT), block = 512, static LDS = 8 x NT x 1 KiB; p.x is the prep's
+// workspace, p.tok_pad = 16 * (its token tiles).
+template <int NT, bool PL = false>
+__device__ __forceinline__ void mx_few_body(const MxGemmArgs& args, float* part) {
+    MxGemmArgs p = args;
+    if constexpr (PL) {
+        JL_NOW(p.out, p.x, p.qs, p.d, p.nrows, p.k, p.ntok, p.tok_pad, p.row0, p.stride);
+        p.qs = as_global(p.qs); p.d = as_global(p.d);
+    } else {
+        JL_NOW(p.out, p.x, p.w, p.nrows, p.k, p.ntok, p.tok_pad, p.row_bytes);
+        p.w = as_global(p.w);
+    }
+    p.out = as_global(p.out); p.x = as_global(p.x);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, kq = lane >> 4;
-    const int r0 = blockIdx.x * 16;
+    int rtile = blockIdx.x;
+    if (PL && (gridDim.x & 7) == 0) rtile = (rtile & 7) * (int)(gridDim.x >> 3) + (rtile >> 3);
+    const int r0 = rtile * 16, tile0 = blockIdx.y * NT, ntiles = p.tok_pad / 16;
     const int nblk = p.k / 32, ngroups = (nblk + 3) / 4;
-    const uint8_t* wrow = p.w + (size_t)min(r0 + r16, p.nrows - 1) * p.row_bytes;
-    const u32x4* xf = (const u32x4*)p.x;
+    const int row = min(r0 + r16, p.nrows - 1);
+    const uint8_t* wrow = PL ? nullptr : p.w + (size_t)row * p.row_bytes;
+    const u32* xw = (const u32*)p.x;
+    const u32x4* xf = (const u32x4*)xw;
+    const size_t pst = (size_t)p.stride, dst = (pst + 3) / 4;
+    const u32 prow = (u32)(p.row0 + row), dsh = 8 * (prow & 3);
 
     f32x4 out[NT];
 #pragma unroll
@@ -867,10 +928,16 @@ __device__ __forceinline__ void mx_few_body(const MxGemmArgs& p, float* part) {
 
     struct W { u32x4 q; u32 e; };
     auto load_w = [&](int G, W& w) {
-        const int b = 4 * G + kq;
-        const uint8_t* blk = wrow + (size_t)min(b, nblk - 1) * 17;
-        w.e = blk[0];
-        w.q = ld16_a1(blk + 1);
+        const int b = min(4 * G + kq, nblk - 1);
+        if constexpr (PL) {
+            const u32* q = p.qs + (size_t)b * 4 * pst + prow;
+            w.q = u32x4{q[0], q[pst], q[2 * pst], q[3 * pst]};
+            w.e = p.d[(size_t)b * dst + (prow >> 2)];   // four rows' exponents: taken apart where they are used
+        } else {
+            const uint8_t* blk = wrow + (size_t)b * 17;
+            w.e = blk[0];
+            w.q = ld16_a1(blk + 1);
+        }
         // (a block past the end of K reads the row's last block; its codes are zeroed where they
         // are used.  A select on the loaded words here puts the wait for the load right behind
         // the load, and so does a copy of one register set into the other at the loop's end: the
@@ -882,9 +949,9 @@ __device__ __forceinline__ void mx_few_body(const MxGemmArgs& p, float* part) {
         bf16x8 af[4 * NT];
 #pragma unroll
         for (int i = 0; i < 4 * NT; i++)
-            af[i] = __builtin_bit_cast(bf16x8, xf[((size_t)G * 4 * NT + i) * 64 + lane]);
+            af[i] = __builtin_bit_cast(bf16x8, xf[(((size_t)G * 4 + i / NT) * ntiles + min(tile0 + i % NT, ntiles - 1)) * 64 + lane]);
         __builtin_amdgcn_sched_barrier(0);
-        const float scale = mx_scale((uint8_t)wcur.e);
+        const float scale = mx_scale(PL ? (uint8_t)(((wcur.e >> dsh) & 0xFF) + 1) : (uint8_t)wcur.e);
         const bool past = 4 * G + kq >= nblk;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -930,7 +997,7 @@ __device__ __forceinline__ void mx_few_body(const MxGemmArgs& p, float* part) {
         if (r < p.nrows) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int tok = 16 * t + 4 * (l >> 4) + i;
+                const int tok = 16 * (tile0 + t) + 4 * (l >> 4) + i;
                 if (tok < p.ntok) p.out[(size_t)tok * p.nrows + r] = s[i];
             }
         }

@@ -238,6 +238,43 @@ def test_mxfp4_packed_matmul_every_exponent_one_token(dev, devbuf):
     assert np.all(np.isfinite(want)) and np.allclose(got, want, rtol=2e-6, atol=0)
 
 
+@pytest.mark.parametrize("packed", [False, True], ids=["rows", "planes"])
+@pytest.mark.parametrize("shape", [(2, 17, 32), (9, 129, 160), (65, 100, 544), (130, 127, 96), (193, 65, 2080), (257, 200, 480)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("form", ["few", "tile64", "tile96"])
+def test_mxfp4_forms_at_their_edges(dev, devbuf, shape, packed, form):
+    """The few-token kernel in token chunks and the small tiles in both heights, over GGUF rows (turned into planes on
+    the way) and over a row range of planes: ragged tokens, rows and K (half K-steps, part groups of blocks)."""
+    from jitllm_amd.device import Packed
+    ntok, nrows, k = shape
+    t, pad = quant.MXFP4, 5
+    w = synth.quantized_weights(t, nrows + 2 * pad, k, seed=nrows)
+    xb, xf = to_bf16(np.stack([synth.activations(k, seed=70 + i) for i in range(ntok)]))
+    want = xf.astype(np.float64) @ oracle.dequant(t, w, (nrows + 2 * pad) * k).reshape(-1, k)[pad:pad + nrows].astype(np.float64).T
+    dw, dx = devbuf(w), devbuf(xb)
+    out = devbuf(shape=(ntok * nrows + 8,), dtype=np.float32, fill=np.float32(2e30))
+    tuning = {"few": {"mxfp4__few": 4096, "mxfp4__few_min": 2}, "tile64": {"mxfp4__planes": 3}, "tile96": {"mxfp4__planes": 4}}[form]
+    dev.set_tuning(**tuning)
+    try:
+        n0 = dev.launch_count()
+        if packed:
+            nq, nd, _ = dev.packed_words(t, nrows + 2 * pad, k)
+            qs, d = devbuf(shape=(nq,), dtype=np.uint32), devbuf(shape=(nd,), dtype=np.uint32)
+            assert dev.pack_weights_dev(t, dw.ptr, nrows + 2 * pad, k, qs.ptr, d.ptr, None)
+            n0 = dev.launch_count()
+            assert dev.matmul_mxfp4_packed_bf16_dev(out.ptr, Packed(qs.ptr, d.ptr, None, pad, nrows + 2 * pad), dx.ptr, nrows, k, ntok)
+        else:
+            assert dev.matmul_mxfp4_bf16_dev(out.ptr, dw.ptr + pad * (k // 32) * 17, dx.ptr, nrows, k, ntok)
+        dev.synchronize()
+        assert dev.launch_count() - n0 == (1 if ntok <= 8 and form != "few" and not packed else 2)
+    finally:
+        dev.set_tuning(**{k_: 0 for k_ in tuning})
+    got = out.get()
+    assert np.all(got[ntok * nrows:] == np.float32(2e30))
+    got = got[:ntok * nrows].reshape(ntok, nrows)
+    assert nmse(got, want) <= 1e-10 and rel_l2(got, want) <= 1e-3
+
+
 # ------------------------------------------------------------------ block-scaled form (opt-in)
 def mx_fp8_activations(xf):
     """The opt-in form's activation quantizer restated in numpy: per token and block of 32 a
