@@ -1265,20 +1265,17 @@ int moe_gemm_i8_launch(jl_ctx* c, float* out0, float* out1, int type, const void
     return launch(c, gemm_i8_name("jl_moe_gemm", c, type, f), (unsigned)std::min(work, cap * c->num_cu), 1, 256, gemm_i8_lds(c, type, f), st, gp);
 }
 
-// pb0 / pb1: the banks as packed planes (bank0 / bank1 unused then): the per-expert tile kernel
-// reads an expert's sheet where it lies in the bank's pages.
-int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1,
-                      const float* x, const float* x2, const uint32_t* src, const uint32_t* start,
-                      int n_expert, int ncols, int nrows, int k, hipStream_t st, const jl_packed_bank* pb0,
-                      const jl_packed_bank* pb1) {
-    const TypeInfo* ti = nullptr;
-    int rc = matvec_check(c, type, nrows, k, &ti);
-    if (rc != JL_OK) return rc;
-    const bool planes = pb0 != nullptr;
-    if (!out0 || (!planes && !bank0) || !x || !start || n_expert <= 0 || ncols <= 0)
-        return fail(c, JL_ERR_ARG, "moe matvec: bad operand");
+// What a grouped matmul asks of its one or two banks of n_expert sheets of nrows x k, whichever kernel serves them
+// and whether or not anything is grouped: GGUF rows (bank0, bank1) or packed planes (pb0, pb1).  `two` says that the
+// call has a second output.  Reads nothing of the device, so it can go in front of everything else.
+int moe_banks_check(jl_ctx* c, int type, bool planes, const void* bank0, const void* bank1, const jl_packed_bank* pb0,
+                    const jl_packed_bank* pb1, bool two, int n_expert, int nrows, int k) {
+    const TypeInfo* ti = type_info(type);
+    if (!ti) return JL_DECLINED;
+    if (nrows <= 0 || k <= 0 || n_expert <= 0) return fail(c, JL_ERR_ARG, "moe matvec: %d experts of %d x %d", n_expert, nrows, k);
+    if ((planes ? pb1 != nullptr : bank1 != nullptr) != two) return fail(c, JL_ERR_ARG, "moe matvec: second matrix needs both bank and out");
     if (planes) {
-        if ((pb1 == nullptr) != (out1 == nullptr)) return fail(c, JL_ERR_ARG, "moe matvec: second matrix needs both bank and out");
+        if (!pb0) return fail(c, JL_ERR_ARG, "moe matvec: null bank");
         for (const jl_packed_bank* b : {pb0, pb1}) {
             if (!b) continue;
             if (!b->qs || !b->d || !b->sc || b->stride <= 0) return fail(c, JL_ERR_ARG, "moe matvec: null plane");
@@ -1289,17 +1286,34 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
                             n_expert, nrows);
             if (b->sheet_bytes != pb0->sheet_bytes || b->stride != pb0->stride) return JL_DECLINED;   // one layout a launch
         }
-        // plane sheets are served by the tile form (Q4_K, the k-quant window)
+        // plane sheets are served in Q4_K with the k-quant window
         if (type != JL_TYPE_Q4_K || c->act_window != 256) return JL_DECLINED;
         if ((size_t)pb0->stride * 4 >= ((size_t)1 << 31)) return JL_DECLINED;
-    } else if ((bank1 == nullptr) != (out1 == nullptr)) {
-        return fail(c, JL_ERR_ARG, "moe matvec: second matrix needs both bank and out");
+    } else {
+        if (!bank0) return fail(c, JL_ERR_ARG, "moe matvec: null bank");
+        if (!aligned16(bank0) || (bank1 && !aligned16(bank1))) return JL_DECLINED;
     }
-    if (!aligned16(x) || (x2 && !aligned16(x2)) || k % 256 != 0 || n_expert > 65535 || ncols > 65535) return JL_DECLINED;
-    if (!planes && (!aligned16(bank0) || (bank1 && !aligned16(bank1)))) return JL_DECLINED;
+    if (k % 256 != 0 || n_expert > 65535) return JL_DECLINED;
+    const size_t sheet = (size_t)nrows * (size_t)(k / ti->block_elems) * ti->block_bytes;
+    return (type == JL_TYPE_Q4_K ? sheet % 16 : sheet % 2) != 0 ? JL_DECLINED : JL_OK;
+}
+
+// pb0 / pb1: the banks as packed planes (bank0 / bank1 unused then): the per-expert kernels
+// read an expert's sheet where it lies in the bank's pages.
+int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1,
+                      const float* x, const float* x2, const uint32_t* src, const uint32_t* start,
+                      int n_expert, int ncols, int nrows, int k, hipStream_t st, const jl_packed_bank* pb0,
+                      const jl_packed_bank* pb1) {
+    const TypeInfo* ti = nullptr;
+    int rc = matvec_check(c, type, nrows, k, &ti);
+    if (rc != JL_OK) return rc;
+    const bool planes = pb0 != nullptr;
+    if (!out0 || !x || !start || ncols <= 0) return fail(c, JL_ERR_ARG, "moe matvec: bad operand");
+    rc = moe_banks_check(c, type, planes, bank0, bank1, pb0, pb1, out1 != nullptr, n_expert, nrows, k);
+    if (rc != JL_OK) return rc;
+    if (!aligned16(x) || (x2 && !aligned16(x2)) || ncols > 65535) return JL_DECLINED;
     const int row_bytes = (k / ti->block_elems) * ti->block_bytes;
     const size_t sheet = (size_t)nrows * row_bytes;
-    if (type == JL_TYPE_Q4_K ? sheet % 16 != 0 : sheet % 2 != 0) return JL_DECLINED;
     // The int8 forms, by columns an expert on average (us of one matrix of 128 experts x 2048 x 768 / 32 x 2048 x 1024 /
     // 16 x 1024 x 2048, what they replace -> them; "moe.form" = 5 forces the few-token kernel, 6, 7, 8 the tiles of 128
     // columns x 64 rows, 64 x 128 and 128 x 128):
@@ -2281,31 +2295,48 @@ int dense_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate
     return launch(c, "jl_add_rows", (unsigned)((n_embd / 4 + 255) / 256), (unsigned)n, 256, 0, st, rp);
 }
 
+// Everything the steps of a routed block ask of the caller's operands, asked before anything is enqueued and whether or
+// not the steps run (a block of one expert has nothing to group or combine).  Reads nothing of the device.
+int moe_ffn_check(jl_ctx* c, const float* resid, int type, int down_type, const void* gate_bank, const void* up_bank,
+                  const void* down_bank, const jl_packed_bank* pg, const jl_packed_bank* pu, const jl_packed_bank* pd,
+                  const float* x, int rows, int k_used, int n_expert, int n_ffn, int n_embd) {
+    if (rows <= 0 || k_used <= 0 || n_expert <= 0 || n_ffn <= 0 || n_embd <= 0) return fail(c, JL_ERR_ARG, "moe ffn: bad shape");
+    if (!resid || !x) return fail(c, JL_ERR_ARG, "moe ffn: null operand");
+    if (n_expert > 1024 || k_used > 16 || n_ffn % 256 != 0 || n_embd % 256 != 0) return JL_DECLINED;
+    int rc = moe_banks_check(c, type, pg != nullptr, gate_bank, up_bank, pg, pu, true, n_expert, n_ffn, n_embd);
+    if (rc == JL_OK) rc = moe_banks_check(c, down_type, pg != nullptr, down_bank, nullptr, pd, nullptr, false, n_expert, n_embd, n_ffn);
+    if (rc != JL_OK) return rc;
+    return aligned16(x) && aligned16(resid) && (size_t)rows * k_used <= 65535 ? JL_OK : JL_DECLINED;
+}
+
 int moe_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate_bank, const void* up_bank,
             const void* down_bank, const jl_packed_bank* pg, const jl_packed_bank* pu, const jl_packed_bank* pd,
             const float* x, const uint32_t* sel, int sel_stride, const float* wt, int rows, int k_used, int n_expert,
             int n_ffn, int n_embd, void* stream) {
     if (!c) return JL_ERR_ARG;
-    if (rows <= 0 || k_used <= 0 || n_expert <= 0 || n_ffn <= 0 || n_embd <= 0)
-        return fail(c, JL_ERR_ARG, "moe ffn: bad shape");
-    if (n_expert > 1024 || k_used > 16 || n_ffn % 256 != 0 || n_embd % 256 != 0) return JL_DECLINED;
-    HIP_TRY(c, H->SetDevice(c->device));
-    hipStream_t st = pick_stream(c, stream);
+    if (!sel || !wt || sel_stride < k_used) return fail(c, JL_ERR_ARG, "moe ffn: bad selection");
+    int rc = moe_ffn_check(c, resid, type, down_type, gate_bank, up_bank, down_bank, pg, pu, pd, x, rows, k_used, n_expert, n_ffn, n_embd);
+    if (rc != JL_OK) return rc;
+    const bool planes = pg != nullptr;
     const size_t ncols = (size_t)rows * k_used;
+    HIP_TRY(c, H->SetDevice(c->device));
+    const TypeInfo* ti = nullptr;
+    if ((rc = matvec_check(c, type, n_ffn, n_embd, &ti)) != JL_OK || (rc = matvec_check(c, down_type, n_embd, n_ffn, &ti)) != JL_OK) return rc;
+    hipStream_t st = pick_stream(c, stream);
     MoeWs w;
-    int rc = moe_ws(c, rows, k_used, n_expert, n_ffn, n_embd, &w);
+    rc = moe_ws(c, rows, k_used, n_expert, n_ffn, n_embd, &w);
     if (rc != JL_OK) return rc;
     uint32_t *start = w.start, *perm = w.perm, *pos = w.pos;
     float *g = w.g, *u = w.u, *y = w.y;
-    // one expert: every row is its column, nothing to group
-    if (n_expert == 1 && k_used == 1 && (!pg || (!pg->sheet_bytes && !pu->sheet_bytes && !pd->sheet_bytes)) && moe_dense_wanted(c)) {
+    // one expert: every row is its column, nothing to group (and no selection to read: every id is 0)
+    if (n_expert == 1 && k_used == 1 && (!planes || (!pg->sheet_bytes && !pd->sheet_bytes)) && moe_dense_wanted(c)) {
         PlaneRef a{}, b{}, d{};
-        if (pg) {
+        if (planes) {
             a = PlaneRef{pg->qs, pg->d, pg->sc, 0, pg->stride}; b = PlaneRef{pu->qs, pu->d, pu->sc, 0, pu->stride};
             d = PlaneRef{pd->qs, pd->d, pd->sc, 0, pd->stride};
         }
-        rc = dense_ffn(c, resid, type, down_type, gate_bank, up_bank, down_bank, pg ? &a : nullptr, pg ? &b : nullptr, pg ? &d : nullptr,
-                       x, wt, rows, n_ffn, n_embd, g, u, y, st);
+        rc = dense_ffn(c, resid, type, down_type, gate_bank, up_bank, down_bank, planes ? &a : nullptr, planes ? &b : nullptr,
+                       planes ? &d : nullptr, x, wt, rows, n_ffn, n_embd, g, u, y, st);
         if (rc != JL_DECLINED) return rc;
     }
     rc = jl_moe_group_dev(c, sel, sel_stride, rows, k_used, n_expert, start, perm, pos, st);
@@ -2333,13 +2364,15 @@ int moe_block(jl_ctx* c, float* resid, int type, int down_type, const void* gate
               uint32_t* sel, float* wt, void* stream) {
     if (rows <= 0 || k_used <= 0 || n_expert <= 0 || n_ffn <= 0 || n_embd <= 0 || !router || !x || !resid)
         return fail(c, JL_ERR_ARG, "moe block: bad operand");
-    if (n_expert > 1024 || k_used > 16 || k_used > n_expert || n_ffn % 256 != 0 || n_embd % 256 != 0) return JL_DECLINED;
+    if (k_used > n_expert) return JL_DECLINED;
+    int rc = moe_ffn_check(c, resid, type, down_type, gate_bank, up_bank, down_bank, pg, pu, pd, x, rows, k_used, n_expert, n_ffn, n_embd);
+    if (rc != JL_OK) return rc;
     HIP_TRY(c, H->SetDevice(c->device));
     hipStream_t st = pick_stream(c, stream);
     const int sel_stride = k_used + 1;
     auto up256 = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const size_t o_sel = up256((size_t)rows * n_expert * 4), o_wt = o_sel + up256((size_t)rows * sel_stride * 4);
-    int rc = ws_ensure(c, &c->moe_route_ws, &c->moe_route_ws_bytes, o_wt + up256((size_t)rows * k_used * 4));
+    rc = ws_ensure(c, &c->moe_route_ws, &c->moe_route_ws_bytes, o_wt + up256((size_t)rows * k_used * 4));
     if (rc != JL_OK) return rc;
     float* logits = (float*)c->moe_route_ws;
     if (!sel) sel = (uint32_t*)((char*)c->moe_route_ws + o_sel);

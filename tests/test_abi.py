@@ -230,3 +230,60 @@ def test_grouped_host_forms_argument_checks_without_a_gpu():
     assert grp(2, x=None) < 0
     assert grp(2) < 0 and b"no device" in lib.jl_last_error(ctx)
     lib.jl_ctx_destroy(ctx)
+
+
+@pytest.mark.parametrize("n_expert", [1, 4])
+def test_routed_block_argument_checks_without_a_gpu(n_expert):
+    """Every form of the routed feed-forward block on a context bound to no device: what an operand must be is asked
+    before anything runs, also where one expert leaves nothing to group; a good call fails at the device."""
+    import ctypes as C
+    lib = _lib.load()
+    ctx = C.c_void_p()
+    opts = _lib.Options(-1, 256, None)
+    assert lib.jl_ctx_create(C.byref(ctx), C.byref(opts)) == _lib.OK and ctx.value
+    E, F, rows, t = 512, 256, 2, quant.Q4_K
+    P = 1 << 20   # addresses that nothing reads: no call gets past its checks
+    bank = lambda nrows, **kw: _lib.PackedBank(kw.get("qs", P), kw.get("d", P), kw.get("sc", P), kw.get("sheet", 0),
+                                               kw.get("stride", n_expert * nrows))
+
+    def ffn(gate=P, up=P, down=P, down_t=t, x=P, resid=P, sel=P, sel_stride=2, wt=P, t=t, n_ffn=F):
+        return lib.jl_moe_ffn_types_dev(ctx, resid, t, down_t, gate, up, down, x, sel, sel_stride, wt, rows, 1, n_expert, n_ffn, E, None)
+
+    def block(gate=P, up=P, down=P, down_t=t, x=P, resid=P, t=t, n_ffn=F, router=P):
+        return lib.jl_moe_block_dev(ctx, resid, t, down_t, gate, up, down, 0, router, x, rows, 1,
+                                    n_expert, n_ffn, E, None, None, None)
+
+    def packed(gate=None, up=None, down=None, x=P, resid=P, sel=P, sel_stride=2, wt=P, t=t):
+        g, u, d = (gate or bank(F)), (up or bank(F)), (down or bank(E))
+        return lib.jl_moe_ffn_packed_dev(ctx, resid, t, C.byref(g), C.byref(u), C.byref(d), x, sel, sel_stride, wt, rows, 1, n_expert, F, E, None)
+
+    def packed_block(gate=None, up=None, down=None, x=P, resid=P, t=t):
+        g, u, d = (gate or bank(F)), (up or bank(F)), (down or bank(E))
+        return lib.jl_moe_block_packed_dev(ctx, resid, t, C.byref(g), C.byref(u), C.byref(d), 0, P, x, rows, 1, n_expert, F, E, None, None, None)
+
+    ERR_ARG, ERR_HIP = -1, -2
+    for call in (ffn, block):
+        assert call() == ERR_HIP
+        for null in ("gate", "up", "down", "x", "resid"):
+            assert call(**{null: None}) == ERR_ARG, null
+        for off in ("gate", "up", "down", "x", "resid"):
+            assert call(**{off: P + 4}) == _lib.DECLINED, off
+        assert call(t=99) == _lib.DECLINED and call(down_t=99) == _lib.DECLINED and call(n_ffn=F + 32) == _lib.DECLINED
+    for call in (ffn, packed):
+        assert call(sel=None) == ERR_ARG and call(wt=None) == ERR_ARG and call(sel_stride=0) == ERR_ARG
+    for call in (packed, packed_block):
+        assert call() == ERR_HIP
+        for m, nrows in (("gate", F), ("up", F), ("down", E)):
+            for null in ("qs", "d", "sc"):
+                assert call(**{m: bank(nrows, **{null: None})}) == ERR_ARG, (m, null)
+                assert call(**{m: bank(nrows, **{null: P + 2})}) == _lib.DECLINED, (m, null)
+            # planes that do not hold the bank's rows; a second bank laid out otherwise than the first
+            assert call(**{m: bank(nrows, stride=n_expert * nrows - 1)}) == ERR_ARG, m
+            assert call(**{m: bank(nrows, stride=nrows - 1, sheet=1 << 20)}) == ERR_ARG, m
+        assert call(up=bank(F, stride=n_expert * F + 1)) == _lib.DECLINED
+        assert call(x=None) == ERR_ARG and call(resid=None) == ERR_ARG
+        assert call(x=P + 4) == _lib.DECLINED and call(resid=P + 4) == _lib.DECLINED
+        assert call(t=quant.Q8_0) == _lib.DECLINED             # plane banks: Q4_K
+    assert lib.jl_set_act_window(ctx, 32) == _lib.OK
+    assert packed() == _lib.DECLINED and packed_block() == _lib.DECLINED   # and the k-quant window
+    lib.jl_ctx_destroy(ctx)
