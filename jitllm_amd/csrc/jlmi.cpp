@@ -2262,8 +2262,13 @@ int dense_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate
     auto few = [&](int t, const void* w, const PlaneRef* p, int nrows, int k) {
         return n <= 64 && few_fits(c, t, planes, nrows, k, n, planes ? p->stride : 0) && (planes || ((uintptr_t)w & (t == JL_TYPE_Q4_K ? 15 : 3)) == 0);
     };
+    // (vectors of four floats are read from x and added to resid; rows longer than the decode kernels take are not
+    // served whatever the number of tokens)
+    if (n > 65535 || n_embd % 4 || n_ffn % 4 || !aligned16(x) || !aligned16(resid)) return JL_DECLINED;
+    const TypeInfo* ti = nullptr;
     int rc;
-    if (n > 65535 || n_embd % 4 || n_ffn % 4) return JL_DECLINED;
+    if (!planes && ((rc = matvec_check(c, type, n_ffn, n_embd, &ti)) != JL_OK || (rc = matvec_check(c, down_type, n_embd, n_ffn, &ti)) != JL_OK))
+        return rc;
     if (few(type, gate, pg, n_ffn, n_embd) && few(type, up, pu, n_ffn, n_embd) && (!planes || (pg->row == pu->row && pg->stride == pu->stride))) {
         FewCall f;
         f.type = type; f.nrows = n_ffn; f.k = n_embd; f.ncols = n; f.nmat = 2; f.x = x;

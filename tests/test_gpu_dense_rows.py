@@ -44,3 +44,35 @@ def test_dense_block_rows(dev, devbuf, t, down_t, packed, n):
     finally:
         dev.ReleaseLayers(0, 1)
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("n", [2, 65])
+@pytest.mark.parametrize("packed", [False, True], ids=["rows", "planes"])
+def test_dense_block_rows_off_their_alignment(dev, devbuf, packed, n):
+    """Rows whose vectors of four floats do not begin on 16 bytes are declined; a residual that does not is served
+    row by row, with the values of an aligned one; rows the decode kernels decline for their length are declined."""
+    E, F, t = 256, 512, quant.Q8_0
+    dev.SetActWindow(32)
+    mats = [(t, synth.quantized_weights(t, r, k, seed=r + k), r, k) for r, k in ((F, E), (F, E), (E, F))]
+    ops = [_planes(*m) for m in mats] if packed else [m[1] for m in mats]
+    h = np.stack([synth.activations(E, seed=20 + i) for i in range(n)])
+    r0 = np.stack([synth.activations(E, seed=90 + i) for i in range(n)])
+    hd, hoff = devbuf(h), devbuf(np.concatenate([[0], h.ravel()]).astype(np.float32))
+    roff = devbuf(np.concatenate([[0], r0.ravel(), [7]]).astype(np.float32))
+    assert dev.PrepLayer(0, _lib.LAYER_DENSE, t, E, F, *ops)
+    try:
+        want = devbuf(r0)
+        assert not dev.layer_ffn_dev(0, hoff.ptr + 4, want.ptr, n)
+        for i in range(n):
+            assert dev.layer_ffn_dev(0, hd.ptr + 4 * E * i, want.ptr + 4 * E * i, 1)
+        assert dev.layer_ffn_dev(0, hd.ptr, roff.ptr + 4, n)
+        dev.synchronize()
+        got = roff.get()
+        assert got[0] == 0 and got[-1] == 7
+        assert np.array_equal(got[1:-1].view(np.uint32), want.get().ravel().view(np.uint32))
+        if not packed:
+            long = 131072
+            assert dev.PrepLayer(0, _lib.LAYER_DENSE, t, E, long, *[np.zeros(E * long // 32 * 34, np.uint8)] * 3)
+            assert not dev.layer_ffn_dev(0, hd.ptr, want.ptr, 1) and not dev.layer_ffn_dev(0, hd.ptr, want.ptr, n)
+    finally:
+        dev.ReleaseLayers(0, 1)
