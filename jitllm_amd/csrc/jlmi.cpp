@@ -3172,8 +3172,8 @@ int jl_matvec_packed_group(jl_ctx* c, int n, float* const* outs, const int* type
         i = e;
     }
     if (rc == JL_OK && resid) rc = host_result_copy(c, o_rd, rd, (size_t)rows[0]);
-    if (resid) host_out(o_rd, resid, (size_t)rows[0]);
     for (int i = 0; i < n; i++) host_out(o_out[i], outs[i], (size_t)rows[i]);
+    if (resid) host_out(o_rd, resid, (size_t)rows[0]);   // last: the sum is what stays where resid is also an output
     return host_io_end(c, rc);
 }
 
