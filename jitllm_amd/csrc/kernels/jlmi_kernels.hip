@@ -461,22 +461,21 @@ extern "C" __global__ __launch_bounds__(256) void jl_mxfp4_scaled_prep(MxScaledP
 extern "C" __global__ __launch_bounds__(256, 2) void jl_mxfp4_scaled_gemm(MxScaledGemmArgs p) {
     mx_scaled_gemm_body(p, (float*)jl_smem);
 }
-// 9..64 tokens: prep grid = (ceil(k/128), tiles of 16 tokens), block = 256; kernel grid =
-// ceil(nrows/16), block = 512; _t<NT>: up to 16 NT tokens
+// A few tokens: prep grid = (ceil(k/128), tiles of 16 tokens), block = 256; kernel grid = (ceil(nrows/16), chunks),
+// block = 512; _t<NT>: up to 16 NT tokens, _c<NT>: chunks of 16 NT of more
 extern "C" __global__ __launch_bounds__(256) void jl_mxfp4_prep_few(MxPrepArgs p) { mx_prep_few_body(p); }
-#define JL_MX_FEW_KERNEL(NT)                                                                   \
-    extern "C" __global__ __launch_bounds__(512) void jl_mxfp4_few_t##NT(MxGemmArgs p) {       \
+#define JL_MX_FEW_KERNEL(NAME, NT, PL, CHUNKS)                                                 \
+    extern "C" __global__ __launch_bounds__(512) void jl_mxfp4_few_##NAME(MxGemmArgs p) {      \
         __shared__ __attribute__((aligned(16))) float part[8 * NT * 256];                      \
-        mx_few_body<NT>(p, part);                                                              \
-    }                                                                                          \
-    extern "C" __global__ __launch_bounds__(512) void jl_mxfp4_few_planes_t##NT(MxGemmArgs p) { \
-        __shared__ __attribute__((aligned(16))) float part[8 * NT * 256];                      \
-        mx_few_body<NT, true>(p, part);                                                        \
+        mx_few_body<NT, PL, CHUNKS>(p, part);                                                  \
     }
-JL_MX_FEW_KERNEL(1) JL_MX_FEW_KERNEL(2) JL_MX_FEW_KERNEL(3) JL_MX_FEW_KERNEL(4)
+JL_MX_FEW_KERNEL(t1, 1, false, false) JL_MX_FEW_KERNEL(t2, 2, false, false)
+JL_MX_FEW_KERNEL(t3, 3, false, false) JL_MX_FEW_KERNEL(t4, 4, false, false)
+JL_MX_FEW_KERNEL(c3, 3, false, true) JL_MX_FEW_KERNEL(c4, 4, false, true)
+JL_MX_FEW_KERNEL(planes_t1, 1, true, false) JL_MX_FEW_KERNEL(planes_t2, 2, true, false)
+JL_MX_FEW_KERNEL(planes_t3, 3, true, false) JL_MX_FEW_KERNEL(planes_t4, 4, true, false)
+JL_MX_FEW_KERNEL(planes_c3, 3, true, true) JL_MX_FEW_KERNEL(planes_c4, 4, true, true)
 
-// n words of `value`: the selection and weight tables of a dense block run as a mixture of one
-// expert (a kernel, not a memset, so that a caller may capture it).  grid = ceil(n / 256), block = 256
 // A Q4_K weight is d * sc * q - dmin * m with sc, m <= 63 and q <= 15: a super-block whose
 // |d| * 945 + |dmin| * 63 passes the largest f16 cannot be folded (a NaN or infinite scale
 // fails the comparison and is flagged too).  grid = ceil(nblocks/256), block = 256.

@@ -862,10 +862,10 @@ __device__ __forceinline__ void sum_parts_body(const SumPartsArgs& p) {
 }
 
 // ---------------------------------------------------------------- few tokens
-// 9..64 tokens: the weights (4.4 MB at 2880 x 2880) should be read once and nothing else
-// should cost; the tiled GEMM above needs a K split with a second launch there.  The scheme
-// of the Q4_K few-token kernel: v_mfma_f32_16x16x32_bf16 (16 tokens x 16 rows, K = 32), a
-// workgroup owns 16 rows and all tokens, its eight wavefronts split K and meet in LDS.
+// From a handful of tokens to a few chunks of 64 (mx_few_applies in jlmi.cpp): the weights (4.4 MB at
+// 2880 x 2880) should be read once and nothing else should cost; the tiled GEMM above needs a K split
+// with a second launch there.  v_mfma_f32_16x16x32_bf16 (16 tokens x 16 rows, K = 32), a
+// workgroup owns 16 rows and a chunk of tokens, its eight wavefronts split K and meet in LDS.
 // K is walked in groups of four blocks (128 weights).  Lane (row r = lane % 16, kq = lane / 16)
 // loads block 4 G + kq of its row whole (16 code bytes + the exponent) and K-step j of the
 // group takes code word j of every lane: a step mixes four blocks, each lane converting its
@@ -896,9 +896,14 @@ __device__ __forceinline__ void mx_prep_few_body(const MxPrepArgs& p) {
 // load is sixteen rows' words side by side for each of the four blocks.  (Restoring rows first was a launch of 5 us
 // in front: 2880 x 2880, 64 tokens 14.5 us.)  Workgroups go round the eight XCDs in the order of their ids: each XCD
 // is given a run of consecutive row tiles, whose words share lines.
+// Up to 64 tokens are one chunk of NT token tiles, so a fragment's place is the group's base and a constant.  CHUNKS:
+// more tokens in chunks of NT tiles, the tiles of all of them side by side in the workspace (us with that form's
+// run-time strides for every count -> one chunk by constants: 2880 x 2880, 64 tokens rows 11.0 -> 9.5, planes 10.6 -> 8.9;
+// 33 tokens 9.5 -> 8.6 and 9.0 -> 8.0; 9 tokens 7.5 -> 7.1 and 6.8 -> 6.5; 5760 x 2880, 64 tokens 15.5 -> 14.0 and
+// 13.6 -> 11.9).
 // grid = (ceil(nrows / 16), token chunks of 16 NT), block = 512, static LDS = 8 x NT x 1 KiB; p.x is the prep's
-// workspace, p.tok_pad = 16 * (its token tiles).
-template <int NT, bool PL = false>
+// workspace, p.tok_pad = 16 * (its token tiles), 16 NT without CHUNKS.
+template <int NT, bool PL, bool CHUNKS>
 __device__ __forceinline__ void mx_few_body(const MxGemmArgs& args, float* part) {
     MxGemmArgs p = args;
     if constexpr (PL) {
@@ -913,7 +918,7 @@ __device__ __forceinline__ void mx_few_body(const MxGemmArgs& args, float* part)
     const int r16 = lane & 15, kq = lane >> 4;
     int rtile = blockIdx.x;
     if (PL && (gridDim.x & 7) == 0) rtile = (rtile & 7) * (int)(gridDim.x >> 3) + (rtile >> 3);
-    const int r0 = rtile * 16, tile0 = blockIdx.y * NT, ntiles = p.tok_pad / 16;
+    const int r0 = rtile * 16, tile0 = CHUNKS ? blockIdx.y * NT : 0, ntiles = CHUNKS ? p.tok_pad / 16 : NT;
     const int nblk = p.k / 32, ngroups = (nblk + 3) / 4;
     const int row = min(r0 + r16, p.nrows - 1);
     const uint8_t* wrow = PL ? nullptr : p.w + (size_t)row * p.row_bytes;
@@ -949,7 +954,7 @@ __device__ __forceinline__ void mx_few_body(const MxGemmArgs& args, float* part)
         bf16x8 af[4 * NT];
 #pragma unroll
         for (int i = 0; i < 4 * NT; i++)
-            af[i] = __builtin_bit_cast(bf16x8, xf[(((size_t)G * 4 + i / NT) * ntiles + min(tile0 + i % NT, ntiles - 1)) * 64 + lane]);
+            af[i] = __builtin_bit_cast(bf16x8, xf[(((size_t)G * 4 + i / NT) * ntiles + (CHUNKS ? min(tile0 + i % NT, ntiles - 1) : i % NT)) * 64 + lane]);
         __builtin_amdgcn_sched_barrier(0);
         const float scale = mx_scale(PL ? (uint8_t)(((wcur.e >> dsh) & 0xFF) + 1) : (uint8_t)wcur.e);
         const bool past = 4 * G + kq >= nblk;

@@ -275,6 +275,42 @@ def test_mxfp4_forms_at_their_edges(dev, devbuf, shape, packed, form):
     assert nmse(got, want) <= 1e-10 and rel_l2(got, want) <= 1e-3
 
 
+@pytest.mark.parametrize("packed", [False, True], ids=["rows", "planes"])
+def test_mxfp4_few_tokens_one_chunk_and_several(dev, devbuf, packed):
+    """The few-token kernel at every count of token tiles, one chunk (up to 64 tokens) and the first chunked ones: a
+    token's sums do not depend on how many share the launch, so its bits are those of the call of sixteen tokens that
+    holds it (which the test above holds to the f64 product)."""
+    from jitllm_amd.device import Packed
+    t, nrows, k, most = quant.MXFP4, 37, 1184, 160
+    w = synth.quantized_weights(t, nrows, k, seed=3)
+    xb, xf = to_bf16(np.stack([synth.activations(k, seed=170 + i) for i in range(most)]))
+    dw, dx = devbuf(w), devbuf(xb)
+    nq, nd, _ = dev.packed_words(t, nrows, k)
+    qs, d = devbuf(shape=(nq,), dtype=np.uint32), devbuf(shape=(nd,), dtype=np.uint32)
+    assert dev.pack_weights_dev(t, dw.ptr, nrows, k, qs.ptr, d.ptr, None)
+
+    def run(x0, ntok):
+        out = devbuf(shape=(ntok * nrows + 8,), dtype=np.float32, fill=np.float32(2e30))
+        x = dx.ptr + x0 * k * 2
+        if packed:
+            assert dev.matmul_mxfp4_packed_bf16_dev(out.ptr, Packed(qs.ptr, d.ptr, None, 0, nrows), x, nrows, k, ntok)
+        else:
+            assert dev.matmul_mxfp4_bf16_dev(out.ptr, dw.ptr, x, nrows, k, ntok)
+        dev.synchronize()
+        got = out.get()
+        assert np.all(got[ntok * nrows:] == np.float32(2e30))
+        return got[:ntok * nrows].reshape(ntok, nrows)
+
+    dev.set_tuning(mxfp4__few=4096, mxfp4__few_min=2)
+    try:
+        want = np.concatenate([run(i, 16) for i in range(0, most, 16)])
+        assert nmse(want, xf.astype(np.float64) @ oracle.dequant(t, w, nrows * k).reshape(nrows, k).astype(np.float64).T) <= 1e-10
+        for ntok in (2, 15, 17, 32, 33, 48, 49, 63, 64, 65, 80, 81, 96, 97, 128, 129, 160):
+            assert np.array_equal(run(0, ntok).view(np.uint32), want[:ntok].view(np.uint32)), ntok
+    finally:
+        dev.set_tuning(mxfp4__few=0, mxfp4__few_min=0)
+
+
 # ------------------------------------------------------------------ block-scaled form (opt-in)
 def mx_fp8_activations(xf):
     """The opt-in form's activation quantizer restated in numpy: per token and block of 32 a
