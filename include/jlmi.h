@@ -341,8 +341,12 @@ int jl_matmul_dev(jl_ctx *ctx, float *out, int type, const void *w, const float 
                   int nrows, int k, int ntok, void *stream);
 
 /* nn.LayerDevice.Reserve(maxRows, maxK) (engine/nn/device.go:1096-1176): size the
- * prefill workspace for up to max_tok tokens of max_k features now, so later
- * calls allocate nothing. */
+ * prefill workspaces for up to max_tok tokens of max_k features now, so that later calls of
+ * jl_matmul_dev and jl_matmul_mxfp4_bf16_dev within them allocate nothing, whatever their rows
+ * (nor do their packed forms, but for the ones that restore rows from planes).  Where the
+ * fastest form of a shape needs room that grows with its rows -- MXFP4 rows turned into planes,
+ * more K slices than two rounds of the chip hold -- such a call takes one that fits;
+ * jl_reserve_shape makes the room for one shape's fastest form. */
 int jl_reserve(jl_ctx *ctx, int max_tok, int max_k);
 
 /* nn.LayerDevice.PrepLayer / Layers / ReleaseLayers (engine/nn/device.go:1096-1176) for the

@@ -169,6 +169,8 @@ struct jl_ctx {
     // prefill GEMM workspace (quantized activations in stage layout), grown on demand
     void* gemm_ws = nullptr;
     size_t gemm_ws_bytes = 0;
+    std::vector<std::pair<int, int>> reserved;   // (tokens, features) jl_reserve has sized the workspaces for
+
     void* w16_ws = nullptr;   // expanded weights of the two-pass GEMM
     size_t w16_ws_bytes = 0;
 
@@ -620,6 +622,16 @@ size_t gemm_ws_need(int ntok, int k) {
 
 int gemm_ws_ensure(jl_ctx* c, size_t need) { return grow(c, &c->gemm_ws, &c->gemm_ws_bytes, need); }
 
+// Calls jl_reserve covers allocate nothing, whatever their rows: a workspace that grows with the rows is then only
+// used as far as it is there.  K slices: the Q4_K and MXFP4 forms cut a grid to at most two rounds of the CUs, whose
+// tiles this many bytes hold; the int8 tiles, whose rule has no such bound, keep to it where it is all there is.
+bool reserved_for(const jl_ctx* c, int ntok, int k) {
+    for (const auto& r : c->reserved)
+        if (ntok <= r.first && k <= r.second) return true;
+    return false;
+}
+size_t slab_reserve(const jl_ctx* c) { return (size_t)c->num_cu * 256 * 128 * 4; }
+
 constexpr size_t kGemmW16StageVecs = 1152;   // JL_GEMM_W16_STAGE_VECS
 constexpr unsigned kGemmW16LdsBytes = 2u * 1152u * 16u + 2u * kGemmTile * 4u;
 
@@ -880,7 +892,7 @@ int gemm_i8_launch(jl_ctx* c, float* out, int type, const void* w, const float* 
     I8Shape f = {2, 4};
     int nsplit = 1;
     double best = 1e30;
-    const size_t n = (size_t)ntok * nrows;
+    const size_t n = (size_t)ntok * nrows, most = reserved_for(c, ntok, k) ? slab_reserve(c) : (size_t)-1;
     for (int rt : {4, 2}) {
         if (c->tune.gemm_i8 > 0 ? rt != (c->tune.gemm_i8 == 1 ? 4 : 2) : rt == 4 && type != JL_TYPE_Q8_0) continue;
         const long cap = rt == 4 || type != JL_TYPE_Q8_0 ? 2 : 3, groups = (long)((ntok + 127) / 128) * ((nrows + 32 * rt - 1) / (32 * rt));
@@ -888,6 +900,7 @@ int gemm_i8_launch(jl_ctx* c, float* out, int type, const void* w, const float* 
             if (c->tune.gemm_split > 0 && s != std::min(std::min(c->tune.gemm_split, 8), nunit)) continue;
             const int per = (nunit + s - 1) / s;
             if ((nunit + per - 1) / per != s) continue;   // no empty split
+            if (s > 1 && n * s * 4 > most) continue;
             const long wgs = groups * s, full = wgs / (cap * c->num_cu), left = wgs - full * cap * c->num_cu;
             const double block = 4 * rt * per * unit;     // of a wavefront
             double us = full * (1.5 + 0.1 * cap * block);
@@ -2097,7 +2110,11 @@ int jl_reserve(jl_ctx* c, int max_tok, int max_k) {
     // the k-quant prep's layout and the window-32 prep's (fragments + two scale planes)
     const size_t tok_pad = ((size_t)max_tok + 255) / 256 * 256;
     const size_t w32 = (size_t)(max_k / 128) * (tok_pad / 32) * 8 * 1024 + 2 * (size_t)(max_k / 32) * tok_pad * 4;
-    return gemm_ws_ensure(c, std::max(gemm_ws_need(max_tok, max_k), w32));
+    int rc = gemm_ws_ensure(c, std::max(gemm_ws_need(max_tok, max_k), w32));
+    if (rc == JL_OK) rc = ws_ensure(c, &c->mx_ws, &c->mx_ws_bytes, slab_reserve(c));
+    if (rc != JL_OK) return rc;
+    c->reserved.push_back({max_tok, max_k});
+    return JL_OK;
 }
 
 int jl_reserve_shape(jl_ctx* c, int type, int nrows, int k, int ntok, int packed) {
@@ -2658,6 +2675,9 @@ double mx_tile_rounds(const jl_ctx* c, int nrows, int ntok, int* trows) {
     *trows = c->tune.mx_planes == 3 ? 64 : c->tune.mx_planes == 4 ? 96 : r96 < r64 ? 96 : 64;
     return *trows == 96 ? r96 : r64;
 }
+size_t mx_tile_xa_bytes(int k, int ntok) { return (size_t)((k + 63) / 64) * ((ntok + 63) / 64 * 2) * 4 * 1024; }
+// rows turned into planes: codes and exponents of rows in whole runs of 64
+size_t mx_tile_plane_bytes(int nrows, int k) { return (size_t)(k / 32) * 17 * ((nrows + 63) / 64 * 64); }
 int mx_tile_launch(jl_ctx* c, MxPlanesGemmArgs& a, const uint8_t* w, const uint16_t* x, hipStream_t st) {
     const int tok_pad = (a.ntok + 63) / 64 * 64, nks = (a.k + 63) / 64, ntt = tok_pad / 32, nblk = a.k / 32;
     int trows;
@@ -2665,8 +2685,8 @@ int mx_tile_launch(jl_ctx* c, MxPlanesGemmArgs& a, const uint8_t* w, const uint1
     const long tiles = (long)(tok_pad / 64) * ((a.nrows + trows - 1) / trows), stride = (a.nrows + 63) / 64 * 64;
     const long nx = (long)((nks + 3) / 4) * ntt, nw = w ? (stride / 64) * ((nblk + 15) / 16) : 0;
     if (tiles > 0x7fffffffL / 2 || nx + nw > 0x7fffffffL) return JL_DECLINED;
-    const size_t xa_bytes = (size_t)nks * ntt * 4 * 1024, qs_bytes = w ? (size_t)nblk * 16 * stride : 0;
-    int rc = gemm_ws_ensure(c, xa_bytes + qs_bytes + (w ? (size_t)nblk * stride : 0));
+    const size_t xa_bytes = mx_tile_xa_bytes(a.k, a.ntok), qs_bytes = (size_t)nblk * 16 * stride;
+    int rc = gemm_ws_ensure(c, xa_bytes + (w ? mx_tile_plane_bytes(a.nrows, a.k) : 0));
     if (rc != JL_OK) return rc;
     MxPlanesPrepArgs pa;
     pa.x = x; pa.xa = (uint32_t*)c->gemm_ws; pa.ntok = a.ntok; pa.tok_pad = tok_pad; pa.k = a.k;
@@ -2740,7 +2760,10 @@ int jl_matmul_mxfp4_bf16_dev(jl_ctx* c, float* out, const void* w, const uint16_
     const double large_us = 7 + (double)cost(trows) / trows * per * (trows == 96 ? 2.15 : 2.9) +
                             (nsplit > 1 ? 3.5 + (double)ntok * nrows * nsplit * 4 / 3e6 : 0);
     const unsigned lds = 2u * 128u * 264u * 2u;   // two weight stages [128][264] bf16
-    if (c->tune.mx_planes == 3 || c->tune.mx_planes == 4 || lds > c->lds_limit || (!c->tune.mx_rows && !c->tune.mx_split && 1.08 * small_us < large_us)) {
+    // (the planes of a reserved call have to fit what is there; jl_reserve_shape, a dry run, makes them room)
+    const bool room = !reserved_for(c, ntok, k) || call_dry_run(c) || mx_tile_xa_bytes(k, ntok) + mx_tile_plane_bytes(nrows, k) <= c->gemm_ws_bytes;
+    if (c->tune.mx_planes == 3 || c->tune.mx_planes == 4 || lds > c->lds_limit ||
+        (room && !c->tune.mx_rows && !c->tune.mx_split && 1.08 * small_us < large_us)) {
         MxPlanesGemmArgs ga;
         ga.out = out; ga.nrows = nrows; ga.k = k; ga.ntok = ntok;
         return mx_tile_launch(c, ga, (const uint8_t*)w, x, st);
