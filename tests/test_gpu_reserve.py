@@ -11,11 +11,11 @@ from jitllm_amd.hipmem import mem_info
 pytestmark = pytest.mark.gpu
 
 # (MXFP4 512 x 2880 x 2880: its fastest form turns the rows into planes; most others are cut along K)
-SHAPES = [(quant.MXFP4, 32, 300, 5760, 5760), (quant.MXFP4, 32, 512, 2880, 2880), (quant.MXFP4, 32, 200, 640, 4096),
-          (quant.MXFP4, 32, 40, 2880, 2880), (quant.Q8_0, 32, 300, 512, 5888), (quant.Q8_0, 32, 500, 4096, 4096),
-          (quant.Q8_0, 32, 2, 512, 2048), (quant.Q4_K, 32, 130, 512, 4096), (quant.Q6_K, 32, 130, 512, 4096),
-          (quant.Q6_K, 256, 130, 512, 4096), (quant.Q4_K, 256, 512, 4096, 2048), (quant.Q4_K, 256, 100, 512, 4096),
-          (quant.Q4_K, 256, 20, 512, 4096)]
+SHAPES = [(quant.MXFP4, 32, 300, 5760, 2880), (quant.MXFP4, 32, 512, 2880, 2880), (quant.MXFP4, 32, 200, 640, 3072),
+          (quant.MXFP4, 32, 40, 2880, 2880), (quant.Q8_0, 32, 300, 512, 3072), (quant.Q8_0, 32, 500, 4096, 2944),
+          (quant.Q8_0, 32, 2, 512, 2048), (quant.Q4_K, 32, 130, 512, 3072), (quant.Q6_K, 32, 130, 512, 3072),
+          (quant.Q6_K, 256, 130, 512, 3072), (quant.Q4_K, 256, 512, 4096, 2048), (quant.Q4_K, 256, 100, 512, 3072),
+          (quant.Q4_K, 256, 20, 512, 3072)]
 
 
 def _operands(devbuf, t, ntok, nrows, k):
@@ -40,7 +40,13 @@ def _run(d, o, t, window, wd, xd, nrows, k, ntok):
 
 def test_reserved_calls_allocate_nothing(dev, devbuf):
     with Device(device=0, act_window=32) as grows, Device(device=0, act_window=32) as held:
-        held.Reserve(512, 5888)
+        # (a kernel with spilled registers takes memory of the runtime's on a stream's first launch of it)
+        wd, xd, (a, b) = _operands(devbuf, quant.MXFP4, 70, 200, 256)
+        for form in (3, 4):
+            held.set_tuning(mxfp4__planes=form)
+            _run(held, a, quant.MXFP4, 32, wd, xd, 200, 256, 70)
+        held.set_tuning(mxfp4__planes=0)
+        held.Reserve(512, 3072)
         for t, window, ntok, nrows, k in SHAPES:
             wd, xd, (a, b) = _operands(devbuf, t, ntok, nrows, k)
             want = _run(grows, a, t, window, wd, xd, nrows, k, ntok)
