@@ -245,8 +245,8 @@ int jl_matvec_q8_dev(jl_ctx *ctx, float *out, int type, const void *w, const int
  * internal/oracle/moe.go:361-370; the logit is jl_moe_logits_dev with one expert row).
  * norm_w, when set, puts an RMSNorm in
  * front of everything, the reference's RMSNormQuantRows (jit/gpu/kernels/elem.go:252-267)
- * with the arithmetic of its host form (internal/oracle/oracle.go:230-240): the activation
- * is f32(f64(x) * 1/sqrt(mean(x^2) + norm_eps) * f64(norm_w)), mean in f64; norm_out, when
+ * in the f64 of its host form (internal/oracle/oracle.go:230-240): the activation
+ * is f32(f64(x) * f64(norm_w) * 1/sqrt(mean(x^2) + norm_eps)), mean in f64; norm_out, when
  * set, receives that normed vector.  One launch, whatever the mix of types (the reference's
  * MatVecSegments, jit/gpu/kernels/matvec.go:1411-1431). */
 #define JL_MAX_GROUP 4
@@ -290,8 +290,8 @@ int jl_matvec_gather_dev(jl_ctx *ctx, float *const *outs, int type, const void *
  * resid[r] += alpha * out[0][r] (MVGroup.Resid, engine/nn/packedgroup.go:32-36), alpha
  * times sigmoid(*resid_gate) when resid_gate is given, as in jl_matvec_group_dev; norm_w,
  * when given (never together with up: JL_DECLINED), puts RMSNorm(x_j, norm_w, norm_eps) in
- * front of the quantizer (RMSNormQuantRows, jit/gpu/kernels/elem.go:252-267, with the host
- * arithmetic of internal/oracle/oracle.go:230-240) and norm_out, if not null, receives
+ * front of the quantizer (RMSNormQuantRows, jit/gpu/kernels/elem.go:252-267, in f64 as in
+ * jl_matvec_group_dev) and norm_out, if not null, receives
  * matrix 0's normed activation.  m <= 16, one launch. */
 int jl_matvec_packed_multi_dev(jl_ctx *ctx, float *const *outs, int type, const uint32_t *const *qs,
                                const uint32_t *const *d, const uint32_t *const *sc, const int *row0,

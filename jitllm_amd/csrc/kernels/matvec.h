@@ -810,8 +810,10 @@ __device__ __forceinline__ void matvec_multi_body_xp(const MatVecMultiArgs& q, c
     typename T::W w[1];
     T::load_w(w0 + (size_t)min(r0, nrows - 1) * row_bytes, min(lane, nslots - 1), w[0]);
     // RMSNorm ahead of the quantizer (the reference's RMSNormQuantRows, jit/gpu/kernels/
-    // elem.go:252-267, with its host arithmetic, internal/oracle/oracle.go:230-240): the sum
-    // of squares in f64, scale = 1/sqrt(sum/k + eps), y = f32(f64(x) * f64(w) * scale).
+    // elem.go:252-267): the sum of squares in f64, scale = 1/sqrt(sum/k + eps), y = f32(f64(x) *
+    // f64(w) * scale).  The reference's host form (internal/oracle/oracle.go:230-240) is f32(f64(x) *
+    // scale * f64(w)): x * w, a product of two f32, is exact in f64 and there before the scale is, so
+    // this has one f64 rounding where that has two; the f32 differs where it sits on a rounding boundary.
     // Every workgroup forms the sum itself: k floats are cheaper than a launch.
     double nscale = 0.0, xw[4];   // xw: x * w of the thread's first group, formed while the scale is on its way
     if constexpr (NORM) {

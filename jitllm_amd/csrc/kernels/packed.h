@@ -452,8 +452,8 @@ __device__ __forceinline__ void pk_load_x(const PackedMatVecArgs& p, int c, int 
 
 // Quantize (or copy) the chunk's activation into the wavefront's private LDS area.
 // NORM: the second operand is the RMSNorm weight and nscale the row's 1/rms; the normed
-// value is f32(f64(x) * f64(w) * nscale), the reference's host arithmetic
-// (internal/oracle/oracle.go:230-240).
+// value is f32(f64(x) * f64(w) * nscale), the product that is exact in f64 first, as in matvec.h
+// (internal/oracle/oracle.go:230-240 has x * scale * w).
 template <bool FUSED, bool GATED, bool NORM = false>
 __device__ __forceinline__ void pk_stage_x(const PackedMatVecArgs& p, int c, int lane, const PkX<GATED>& X, uint8_t* my,
                                            double nscale = 0.0, bool write_norm = false) {
