@@ -90,23 +90,25 @@ int jl_synchronize(jl_ctx *ctx);
  * (rows per wavefront: 1, 2, 4), "matvec.block" (threads per workgroup), "matvec.grid"
  * (workgroups), "matvec.q8pair" (2: Q8_0
  * rows one block a lane-slot even where the two-block form with 4-byte-aligned loads applies),
- * "matvec.xpre" (1 / 4: float4 groups of the activation a thread loads ahead of its weights),
+ * "matvec.xpre" (1 / 2 / 4: float4 groups of the activation a thread loads ahead of its weights),
  * "matvec.act_split" (1: a group's gated activation is formed and quantized once, by a launch of
  * its own, instead of by every workgroup), "gemm.min_tok"
  * (fewest tokens sent to the matrix-core GEMM), "gemm.form" (1: 128 x 64 tiles, 2: 256 x 128
  * tiles, 3: two-pass, 4: up to 64 tokens on the int8 matrix cores, 5: 32 rows x 64 tokens a
  * workgroup, 6: 128 x 64 tiles over the whole of K on two groups of wavefronts, 9: token by
  * token), "gemm.few" (form 4: 1 for any number of tokens, 2 never), "few.nt" / "few.rt" /
- * "few.waves" (its token tiles, row tiles and wavefronts a workgroup), "gemm.rows" (64 or 128),
+ * "few.waves" (its token tiles, row tiles and wavefronts a workgroup), "gemm.i8" (the int8 tiles of
+ * Q8_0: 1 / 2 for 128 x 128 / 128 tokens x 64 rows), "gemm.rows" (64 or 128),
  * "gemm.split" (K slices), "gemm.prep" (4: the four-wavefront activation prep), "gemm.planes"
  * (2: restore rows from planes before the GEMM), "packed.rw" (rows per wavefront of the
  * packed-plane matvec: 16, 32, 64), "packed.block" (its threads per workgroup), "moe.shares"
  * (row shares an expert's matrix is split into), "moe.form" (grouped matmul: 1 dot products,
- * 2 / 3 groups of 32 / 16 columns on the matrix cores, 4 the prefill tile per expert),
+ * 2 / 3 groups of 32 / 16 columns on the matrix cores, 4 the prefill tile per expert, 5 the int8
+ * few-token kernel, 6 / 7 / 8 the int8 tiles of 128 columns x 64 rows, 64 x 128 and (Q8_0) 128 x 128),
  * "moe.group16" (form 3: 1 a prep kernel quantizes the columns, 2 the matrix kernel does, 3 groups
  * of 32 columns),
  * "moe.chunk" (form 3: super-blocks a step, 1-3),
- * "moe.group" / "moe.logits" / "moe.q6k_cols" / "moe.waves" / "moe.lpr" (forms of the mixture
+ * "moe.group" / "moe.logits" / "moe.waves" / "moe.lpr" (forms of the mixture
  * block's other kernels),
  * "mxfp4.split" (K slices of the MXFP4 GEMM), "mxfp4.rows" (96 or 128 rows a tile; 1: the
  * general decode matvec also for one token), "mxfp4.few" / "mxfp4.few_min" (the MXFP4

@@ -33,7 +33,7 @@ const HipApi* H = nullptr;  // the process-wide HIP runtime, resolved by the fir
 struct Tuning {
     int rpw = 0, block = 0, grid = 0;
     int act_split = 0;          // grouped matvec with a gated activation: 1 always quantize it in its own launch, 2 never
-    int xpre = 0;               // decode matvec: 1 / 4 float4 groups of x a thread loads ahead of its weights
+    int xpre = 0;               // decode matvec: 1 / 2 / 4 float4 groups of x a thread loads ahead of its weights
     int q8pair = 0;             // Q8_0 rows: 2 keeps one block a lane-slot (2-byte-aligned loads)
     int packed_rw = 0, packed_block = 0, moe_group = 0, moe_logits = 0;
     int moe_shares = 0;
@@ -44,7 +44,7 @@ struct Tuning {
     int gemm_planes = 0;
     int gemm_few = 0;           // the int8 few-token form: 1 wherever it fits, 2 never
     int few_nt = 0, few_rt = 0, few_waves = 0;
-    int gemm_i8 = 0;            // the int8 tile forms: 1, 2, 3 ask for a shape
+    int gemm_i8 = 0;            // the int8 tile forms, Q8_0: 1 / 2 ask for 128 x 128 / 128 x 64 tiles
     int moe_form = 0;
     int moe_g16 = 0;
     int gemm_fold = 0, gemm_fold_waves = 0;
@@ -894,7 +894,7 @@ int gemm_i8_launch(jl_ctx* c, float* out, int type, const void* w, const float* 
     double best = 1e30;
     const size_t n = (size_t)ntok * nrows, most = reserved_for(c, ntok, k) ? slab_reserve(c) : (size_t)-1;
     for (int rt : {4, 2}) {
-        if (c->tune.gemm_i8 > 0 ? rt != (c->tune.gemm_i8 == 1 ? 4 : 2) : rt == 4 && type != JL_TYPE_Q8_0) continue;
+        if (type != JL_TYPE_Q8_0 ? rt == 4 : c->tune.gemm_i8 > 0 && rt != (c->tune.gemm_i8 == 1 ? 4 : 2)) continue;
         const long cap = rt == 4 || type != JL_TYPE_Q8_0 ? 2 : 3, groups = (long)((ntok + 127) / 128) * ((nrows + 32 * rt - 1) / (32 * rt));
         for (int s = 1; s <= 8 && s <= nunit; s++) {
             if (c->tune.gemm_split > 0 && s != std::min(std::min(c->tune.gemm_split, 8), nunit)) continue;
@@ -1329,7 +1329,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     const size_t sheet = (size_t)nrows * row_bytes;
     // The int8 forms, by columns an expert on average (us of one matrix of 128 experts x 2048 x 768 / 32 x 2048 x 1024 /
     // 16 x 1024 x 2048, what they replace -> them; "moe.form" = 5 forces the few-token kernel, 6, 7, 8 the tiles of 128
-    // columns x 64 rows, 64 x 128 and 128 x 128):
+    // columns x 64 rows, 64 x 128 and, Q8_0, 128 x 128):
     //   Q8_0 window 32    1: 39/16/13 -> 36/15/12   8: 90/29/25 -> 53/21/14   32: 235/71/69 -> 92/30/20   128: 853/238/236 -> 170/56/41
     //   Q6_K window 32    1: 32/16/15 -> 39/16/12   8: 98/40/31 -> 62/22/15   32: 308/110/89 -> 114/37/25   128: 1065/403/304 -> 254/86/60
     //   Q6_K window 256   2: 48/20/18 -> 47/19/14   8: 67/27/30 -> 59/21/15   48: 179/47/48 -> 111/38/28    128: 238/81/56 -> 183/61/43
@@ -1356,7 +1356,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
         if (form == 5 && !align && c->tune.moe_form == 0 && avg >= 6) form = 6;
         if (form >= 6 && !planes && gemm_i8_applies(c, type, nrows, k, ncols)) {
             rc = moe_gemm_i8_launch(c, out0, out1, type, bank0, bank1, x, x2, src, start, n_expert, ncols, nrows, k,
-                                    form == 6 ? I8Shape{2, 4} : form == 7 ? I8Shape{2, 2} : I8Shape{4, 4}, st);
+                                    form == 7 ? I8Shape{2, 2} : form == 8 && type == JL_TYPE_Q8_0 ? I8Shape{4, 4} : I8Shape{2, 4}, st);
             if (rc != JL_DECLINED) return rc;
         }
         if (form == 5 && align && few_fits(c, type, planes, nrows, k, ncols, planes ? pb0->stride : 0)) {
@@ -1680,9 +1680,14 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     names.push_back("jl_few_prep");
     names.push_back("jl_gemm_i8_prep");
     names.push_back("jl_moe_gemm_i8_prep");
-    for (const char* pre : {"jl_gemm_i8_", "jl_moe_gemm_i8_"})
-        for (const char* tag : {"q8_0", "q4k", "q6k", "q6kw"})
-            for (const char* shape : {"_r4t4", "_r2t4", "_r2t2"}) names.push_back(std::string(pre) + tag + shape);
+    for (const char* tag : {"q8_0", "q4k", "q6k", "q6kw"})
+        for (const char* form : {"jl_gemm_i8_%s_r2t4", "jl_moe_gemm_i8_%s_r2t4", "jl_moe_gemm_i8_%s_r2t2"}) {
+            char nm[64];
+            snprintf(nm, sizeof nm, form, tag);
+            names.push_back(nm);
+        }
+    names.push_back("jl_gemm_i8_q8_0_r4t4");
+    names.push_back("jl_moe_gemm_i8_q8_0_r4t4");
     for (const char* tag : {"q4k", "q4kw", "q8_0", "q6k", "q6kw"})
         for (const char* layout : {"rows", "planes"})
             for (const char* size : {"t1r1", "t1r2", "t2r1", "t4r1", "t4r2", "t1r4", "t2r2", "t2r4"})
@@ -1804,7 +1809,7 @@ int jl_set_tuning(jl_ctx* c, const char* key, int value) {
     else if (!strcmp(key, "packed.block")) c->tune.packed_block = value;
     else if (!strcmp(key, "moe.group")) c->tune.moe_group = value;
     else if (!strcmp(key, "moe.logits")) c->tune.moe_logits = value;
-    else if (!strcmp(key, "moe.q6k_cols")) (void)value;   // (once the column count from which Q6_K took its tile)
+    else if (!strcmp(key, "moe.q6k_cols")) (void)value;   // (accepted, without effect)
     else if (!strcmp(key, "moe.shares")) c->tune.moe_shares = value;
     else if (!strcmp(key, "moe.form")) c->tune.moe_form = value;
     else if (!strcmp(key, "moe.group16")) c->tune.moe_g16 = value;
