@@ -22,17 +22,19 @@ def test_dense_tiles(dev, devbuf, t, window, nrows, k, ntok):
     x = np.stack([synth.activations(k, seed=900 + i) * np.float32(1 + i % 3) for i in range(ntok)])
     want = oracle.matmul_q8act_f64(t, w, x, nrows, k, ntok, window)
     wd, xd = devbuf(w), devbuf(x)
-    for shape in (0, 1, 2) if t == quant.Q8_0 else (0, 2):
-        for split in (0, 1, 2, 5):
-            dev.set_tuning(gemm__i8=shape, gemm__split=split)
-            o = devbuf(shape=(ntok * nrows + 8,), dtype=np.float32, fill=FILL)
-            assert dev.matmul_dev(o.ptr, t, wd.ptr, xd.ptr, nrows, k, ntok)
-            dev.synchronize()
-            got = o.get()
-            assert np.all(got[ntok * nrows:] == FILL)
-            assert nmse(got[:ntok * nrows].reshape(ntok, nrows), want) <= 1e-10, (shape, split)
-    dev.set_tuning(gemm__i8=0, gemm__split=0)
-    dev.SetActWindow(32)
+    try:
+        for shape in (0, 1, 2) if t == quant.Q8_0 else (0, 2):
+            for split in (0, 1, 2, 5):
+                dev.set_tuning(gemm__i8=shape, gemm__split=split)
+                o = devbuf(shape=(ntok * nrows + 8,), dtype=np.float32, fill=FILL)
+                assert dev.matmul_dev(o.ptr, t, wd.ptr, xd.ptr, nrows, k, ntok)
+                dev.synchronize()
+                got = o.get()
+                assert np.all(got[ntok * nrows:] == FILL)
+                assert nmse(got[:ntok * nrows].reshape(ntok, nrows), want) <= 1e-10, (shape, split)
+    finally:
+        dev.set_tuning(gemm__i8=0, gemm__split=0)
+        dev.SetActWindow(32)
 
 
 @pytest.mark.parametrize("t,window", KINDS, ids=["q8_0", "q4_k", "q6_k", "q6_k-w256"])
@@ -51,24 +53,26 @@ def test_tiles_per_expert(dev, devbuf, t, window, nrows, k):
     u = np.stack([synth.activations(k, seed=500 + r) for r in range(40)])
     xg = (x / (1 + np.exp(-x.astype(np.float64))) * u).astype(np.float32)
     bd, xd, ud, sd, dstart = [devbuf(b) for b in banks], devbuf(x), devbuf(u), devbuf(src), devbuf(start)
-    for gated in (False, True):
-        act = xg if gated else x
-        want = [np.zeros((ncols, nrows)) for _ in banks]
-        for b in range(2):
-            for e in range(n_expert):
-                cols = slice(start[e], start[e + 1])
-                if counts[e]:
-                    want[b][cols] = oracle.matmul_q8act_f64(t, banks[b][e * sheet:(e + 1) * sheet], act[src[cols]], nrows, k, counts[e], window)
-        for form in (0, 5, 6, 7, 8) if t == quant.Q8_0 else (0, 5, 6, 7):
-            dev.set_tuning(moe__form=form)
-            o = [devbuf(shape=(ncols * nrows + 8,), dtype=np.float32, fill=FILL) for _ in banks]
-            assert dev.moe_matvec_dev(o[0].ptr, o[1].ptr, t, bd[0].ptr, bd[1].ptr, xd.ptr, ud.ptr if gated else None, sd.ptr, dstart.ptr,
-                                      n_expert, ncols, nrows, k)
-            dev.synchronize()
+    try:
+        for gated in (False, True):
+            act = xg if gated else x
+            want = [np.zeros((ncols, nrows)) for _ in banks]
             for b in range(2):
-                got = o[b].get()
-                assert np.all(got[ncols * nrows:] == FILL)
-                # (the gated activation: an exponential of another machine in front of the quantizer)
-                assert nmse(got[:ncols * nrows].reshape(ncols, nrows), want[b]) <= (1e-6 if gated else 1e-10), (gated, form, b)
-    dev.set_tuning(moe__form=0)
-    dev.SetActWindow(32)
+                for e in range(n_expert):
+                    cols = slice(start[e], start[e + 1])
+                    if counts[e]:
+                        want[b][cols] = oracle.matmul_q8act_f64(t, banks[b][e * sheet:(e + 1) * sheet], act[src[cols]], nrows, k, counts[e], window)
+            for form in (0, 5, 6, 7, 8) if t == quant.Q8_0 else (0, 5, 6, 7):
+                dev.set_tuning(moe__form=form)
+                o = [devbuf(shape=(ncols * nrows + 8,), dtype=np.float32, fill=FILL) for _ in banks]
+                assert dev.moe_matvec_dev(o[0].ptr, o[1].ptr, t, bd[0].ptr, bd[1].ptr, xd.ptr, ud.ptr if gated else None, sd.ptr, dstart.ptr,
+                                          n_expert, ncols, nrows, k)
+                dev.synchronize()
+                for b in range(2):
+                    got = o[b].get()
+                    assert np.all(got[ncols * nrows:] == FILL)
+                    # (the gated activation: an exponential of another machine in front of the quantizer)
+                    assert nmse(got[:ncols * nrows].reshape(ncols, nrows), want[b]) <= (1e-6 if gated else 1e-10), (gated, form, b)
+    finally:
+        dev.set_tuning(moe__form=0)
+        dev.SetActWindow(32)

@@ -542,10 +542,12 @@ def test_grouped_matvec_over_packed_expert_sheets(dev, devbuf, layout, nrows, k)
     xd, dstart, dperm = devbuf(x), devbuf(start), devbuf(perm[:used].copy())
     o0 = devbuf(shape=(used * nrows + 8,), dtype=np.float32, fill=np.float32(4e30))
     o1 = devbuf(shape=(used * nrows + 8,), dtype=np.float32, fill=np.float32(4e30))
-    # the dot-product form over planes, the library's pick, groups of sixteen columns (columns from a
+    # the int8 few-token kernel (its own pick of tiles, then tiles of several rows and tokens), the dot-product
+    # form over planes, the library's pick, groups of sixteen columns (columns from a
     # prep kernel, then quantized by the matrix kernel itself), then the tile
-    for form in (1, 0, 3, 13, 23, 4):
-        dev.set_tuning(moe__form=form % 10, moe__group16={3: 1, 13: 2, 23: 3}.get(form, 0))
+    for form in (5, 105, 205, 305, 1, 0, 3, 13, 23, 4):
+        nt, rt = {105: (1, 4), 205: (2, 4), 305: (4, 2)}.get(form, (0, 0))
+        dev.set_tuning(moe__form=form % 10, moe__group16={3: 1, 13: 2, 23: 3}.get(form, 0), few__nt=nt, few__rt=rt)
         o0.put(np.full(used * nrows + 8, 4e30, np.float32))
         o1.put(np.full(used * nrows + 8, 4e30, np.float32))
         assert dev.moe_matvec_packed_dev(o0.ptr, o1.ptr, t, pb0, pb1, xd.ptr, None, dperm.ptr, dstart.ptr, n_expert,
@@ -555,7 +557,7 @@ def test_grouped_matvec_over_packed_expert_sheets(dev, devbuf, layout, nrows, k)
         assert np.all(g0[used * nrows:] == np.float32(4e30)) and np.all(g1[used * nrows:] == np.float32(4e30))
         assert nmse(g0[:used * nrows].reshape(used, nrows), want0) <= 1e-10, form
         assert nmse(g1[:used * nrows].reshape(used, nrows), want1) <= 1e-10, form
-    dev.set_tuning(moe__form=0, moe__group16=0)
+    dev.set_tuning(moe__form=0, moe__group16=0, few__nt=0, few__rt=0)
     # the tile form over the same weights as GGUF banks: the same integers, the same epilogue
     b0, b1 = devbuf(bank0), devbuf(bank1)
     r0 = devbuf(shape=(used * nrows,), dtype=np.float32, fill=0)
