@@ -11,6 +11,7 @@
 #include <dlfcn.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -1278,6 +1279,48 @@ int moe_gemm_i8_launch(jl_ctx* c, float* out0, float* out1, int type, const void
     return launch(c, gemm_i8_name("jl_moe_gemm", c, type, f), (unsigned)std::min(work, cap * c->num_cu), 1, 256, gemm_i8_lds(c, type, f), st, gp);
 }
 
+// Blocks of rows an expert's matrix is cut into by the groups-of-columns kernels ("moe.form" = 3): one workgroup of eight
+// wavefronts a CU (the same age on every SIMD, tiles handed out as they get to them: two younger workgroups of four
+// measured 4 % slower), so the grid runs in rounds of CUs workgroups; among the splits of the rows into blocks the one
+// with the least rounds x tiles a wavefront, the fewest blocks among equals (every block fills LDS anew).  Experts that
+// can have a column: at most one a column.  "moe.waves" = 4: the two-workgroup form.
+int moe_g16_blocks(const jl_ctx* c, int nrows, int n_expert, int ncols, int nmat, int nwaves) {
+    const int tiles = (nrows + 15) / 16, sets = (tiles + nwaves - 1) / nwaves;
+    if (c->tune.moe_shares > 0) return std::min(c->tune.moe_shares, sets);
+    const long slots = (nwaves == 4 ? 2L : 1L) * c->num_cu, n_act = std::min<long>(n_expert, ncols);
+    int best = 1;
+    long best_cost = -1;
+    for (int nb = 1; nb <= sets && nb <= 64; nb++) {
+        const long per_wave = (sets + nb - 1) / nb, rounds = ((long)nb * n_act * nmat + slots - 1) / slots, cost = rounds * per_wave;
+        if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = nb; }
+    }
+    return best;
+}
+
+// Q4_K GGUF banks with the k-quant window, 9 to 40 columns an expert on average: whether the int8 few-token kernel takes
+// less time than groups of 32 columns, by what each has to do (us; fitted to 276 launches, 8 to 128 experts of 512 x 512
+// to 2816 x 2048, one and two matrices, to 10 % each).  The few-token kernel: a prep of the columns and the bank's elements
+// by the token tiles of a pass, once more for the experts that overflow it.  Groups of 32: rounds of workgroups, an XCD's
+// experts on its own CUs, each a fill of LDS and its tiles, again for the experts of more than 32 (one of them can be
+// the launch's length).  Chosen so, a launch takes 1.1 % more than the better of the two on average, at most 23;
+// never the few-token kernel: 18 on average; up to 120e6 elements of the bank: 5.7, at most 80 (28 x 1792 x 1280,
+// 38 columns 60.6 us against 36.1; 40 x 768 x 1536 twice, 20 columns 43 against 26).
+bool moe_q4k_few(const jl_ctx* c, int n_expert, int ncols, int nmat, int nrows, int k) {
+    const double avg = (double)ncols / n_expert, nsb = k / 256;
+    if (avg < 9 || avg > 40) return false;
+    const auto over = [&](int n) { return 0.5 * std::erfc((n + 0.5 - avg) / std::sqrt(2 * avg)); };   // an expert's columns pass n
+    const int tiles = (nrows + 15) / 16;
+    const long cut = moe_g16_blocks(c, nrows, n_expert, ncols, nmat, 8), tiles_wg = (tiles + cut - 1) / cut;
+    const long blocks = (tiles + tiles_wg - 1) / tiles_wg, cus_xcd = std::max(1, c->num_cu / 8);
+    const long rounds = (blocks * nmat * ((n_expert + 7) / 8) + cus_xcd - 1) / cus_xcd;
+    const double p = over(32), again = 0.4 * (1 - std::pow(1 - p, n_expert)) + 0.6 * p;
+    const double groups = rounds * (1 + again) * (0.96 * nsb + tiles_wg / 8.0 * (0.71 * nsb + 1.6));
+    const int nt = avg <= 16 ? 1 : avg <= 32 ? 2 : 4;
+    const double few = 0.5 + 0.95e-6 * ncols * k +   // (what its prep takes longer)
+                       1e-6 * n_expert * nmat * (double)nrows * k * (1 + over(16 * nt)) * (nt == 1 ? 0.157 : nt == 2 ? 0.241 : 0.495);
+    return few < groups;
+}
+
 // What a grouped matmul asks of its one or two banks of n_expert sheets of nrows x k, whichever kernel serves them
 // and whether or not anything is grouped: GGUF rows (bank0, bank1) or packed planes (pb0, pb1).  `two` says that the
 // call has a second output.  Reads nothing of the device, so it can go in front of everything else.
@@ -1336,8 +1379,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     // The few-token kernel reads an expert's sheet once for 64 columns and the columns once for every row tile, so it
     // gives way to the tiles where the columns are the more; a tile of 64 columns needs two workgroups a CU.  With a
     // column or two an expert Q6_K's dot-product kernel is as fast while rows are short.  Q4_K with the k-quant window
-    // has the forms below; the few-token kernel takes it from nine columns an expert on while the whole bank is small
-    // (gate + up of 24 experts x 512 x 1024, 24 columns 20.8 -> 15.7; 64 x 1024 x 1536, 12 columns 36.6 against 53).
+    // has the forms below, and the few-token kernel where moe_q4k_few finds it faster.
     {
         const bool q4w = type == JL_TYPE_Q4_K && c->act_window == 256, q6 = type == JL_TYPE_Q6_K;
         const int nmat = (planes ? pb1 != nullptr : bank1 != nullptr) ? 2 : 1;
@@ -1347,7 +1389,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
         int form = c->tune.moe_form;
         if (q6 && !planes && c->act_window == 256 && (form == 3 || form == 4)) form += 2;   // (their Q6_K forms)
         if (form == 0 && (c->act_window == 32 || c->act_window == 256) && !planes) {
-            if (q4w) form = avg >= 9 && avg <= 40 && (double)n_expert * nmat * nrows * k <= 120e6 ? 5 : 0;
+            if (q4w) form = moe_q4k_few(c, n_expert, ncols, nmat, nrows, k) ? 5 : 0;
             else if (q6 && avg < (c->act_window == 32 ? 3 : 2) && k < 2048) form = 0;
             else if (avg < (q6 && c->act_window == 256 ? 28 : 40)) form = 5;
             else if (avg < (q6 && c->act_window == 32 ? 64 : 56)) form = tiles64 >= 2 * c->num_cu ? 7 : 5;
@@ -1402,11 +1444,14 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
         const bool pick16 = c->tune.moe_form == 0 &&
                             (long)ncols >= (planes ? 3L : 2L) * n_expert && (long)ncols < 72L * n_expert;
         if (can16 && (c->tune.moe_form == 3 || pick16)) {
-            // up to seven columns an expert the matrix kernel quantizes them itself: no prep launch,
-            // no workspace ("moe.group16" = 1 forces the prep kernel, 2 the fused form).  (Eight of many
-            // experts: some have more than sixteen, and the workgroup that reads its sheet twice is the
-            // launch's length: 128 experts, top-8, 128 rows 142 us, in groups of 32 134; 112 rows 115 and 131.)
-            const bool fused = c->tune.moe_g16 == 2 || (c->tune.moe_g16 == 0 && (long)ncols <= (n_expert > 64 ? 7L : 8L) * n_expert);
+            // up to eight columns an expert the matrix kernel quantizes them itself: no prep launch,
+            // no workspace ("moe.group16" = 1 forces the prep kernel, 2 the fused form).  (An expert of more than
+            // sixteen is read twice, and that workgroup can be the launch's length; how often one is depends on the
+            // routing.  Gate + up / down of 768 x 2048, means of eight random routings, fused against groups of 32:
+            // 8 columns, 64 experts 31.4 / 18.3 against 37.5 / 24.2, 96 72 / 32 against 75 / 40, 112 64 / 52 against
+            // 64 / 63, 128 68 / 32 against 69 / 38; 9 columns, 64 34 / 20 against 38 / 24, 112 72 / 55 against 64 / 63,
+            // 128 75 / 36 against 70 / 38.)
+            const bool fused = c->tune.moe_g16 == 2 || (c->tune.moe_g16 == 0 && (long)ncols <= 8L * n_expert);
             // beyond groups of 32 (two token tiles, a decoded word meets both), so
             // that an expert of 17-32 columns reads its sheet once ("moe.group16" = 3 forces them)
             const bool two = !fused && 2 * frag16 + 16 <= c->lds_limit &&
@@ -1436,26 +1481,9 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
                 ga.row_step = pb0->sheet_bytes ? 0 : nrows;
                 ga.pstride = pb0->stride;
             }
-            // One workgroup of eight wavefronts a CU (the same age on every SIMD, tiles handed out as
-            // they get to them: two younger workgroups of four measured 4 % slower), so the grid runs
-            // in rounds of CUs workgroups; among the splits of the rows into blocks the one with the
-            // least rounds x tiles a wavefront, the fewest blocks among equals (every block fills LDS
-            // anew).  Experts that can have a column: at most one a column.  "moe.waves" = 4: the
-            // two-workgroup form.
             const int nmat = (planes ? pb1 != nullptr : bank1 != nullptr) ? 2 : 1, tiles = (nrows + 15) / 16;
             const int nwaves = !two && c->tune.moe_waves == 4 ? 4 : 8;
-            const long wgs_cu = nwaves == 4 ? 2 : 1;
-            const int sets = (tiles + nwaves - 1) / nwaves;
-            const long n_act = std::min<long>(n_expert, ncols);
-            int best_blocks = 1;
-            long best_cost = -1;
-            for (int nb = 1; nb <= sets && nb <= 64; nb++) {
-                const long per_wave = (sets + nb - 1) / nb;
-                const long rounds = ((long)nb * n_act * nmat + wgs_cu * c->num_cu - 1) / (wgs_cu * c->num_cu);
-                const long cost = rounds * per_wave;
-                if (best_cost < 0 || cost < best_cost) { best_cost = cost; best_blocks = nb; }
-            }
-            if (c->tune.moe_shares > 0) best_blocks = std::min(c->tune.moe_shares, sets);
+            const int best_blocks = moe_g16_blocks(c, nrows, n_expert, ncols, nmat, nwaves);
             ga.tiles_wg = (tiles + best_blocks - 1) / best_blocks;   // handed out inside the workgroup as its wavefronts get to them
             ga.blocks = (tiles + ga.tiles_wg - 1) / ga.tiles_wg;
             ga.nmat = nmat; ga.n_expert = n_expert; ga.nwaves = nwaves;
