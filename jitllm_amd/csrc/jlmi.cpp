@@ -2664,22 +2664,84 @@ int jl_layer_ffn_dev(jl_ctx* c, int li, const float* h, float* resid, int n, voi
 }
 
 namespace {
+// Rows a tile: a round of the CUs takes about 1.36 times as long with 96 (measured at k = 1216 to 4512), so 96 where
+// that saves the rounds (2880 rows: 512 tokens 21.1 -> 17.4 us, 384 tokens of 5000 rows 19.7 against 23.7).
+double mx_tile_rounds(const jl_ctx* c, int nrows, int ntok, int* trows) {
+    auto rounds = [&](int rows) {
+        return (double)(((long)((ntok + 63) / 64) * ((nrows + rows - 1) / rows) + c->num_cu - 1) / c->num_cu);
+    };
+    const double r64 = rounds(64), r96 = 1.36 * rounds(96);
+    *trows = c->tune.mx_planes == 3 ? 64 : c->tune.mx_planes == 4 ? 96 : r96 < r64 ? 96 : 64;
+    return *trows == 96 ? r96 : r64;
+}
+
+// More than a handful of tokens over GGUF rows: tiles of 128 tokens x 128 or 96 rows that read them, K split over
+// `split` workgroups of `per` stages, or the smaller tiles of the planes with the rows turned into planes on the way; by
+// their costs as measured (us; 1100 x 1216 to 5000 x 2048, 64 to 2048 tokens).  The former: a stage of K = 256 takes 2.15
+// with 96 rows and 2.9 with 128, a split a launch and its slabs; the latter: 1 a MB of weights and 2.75 a round and 1024
+// of K.
+struct MxRowsPlan {
+    int trows, split, per;
+    double rows_us, planes_us;
+};
+MxRowsPlan mx_rows_plan(const jl_ctx* c, int nrows, int k, int ntok) {
+    MxRowsPlan p;
+    const int ttok = (ntok + 127) / 128, stages = (k + 255) / 256;
+    // rows per tile: 128, or 96 where that takes fewer rounds x rows (2880 rows x 1024 tokens:
+    // 184 tiles of 128 rows leave 72 CUs idle for a whole tile, 240 of 96 rows do not)
+    auto cost = [&](int rows) {
+        const long t = (long)ttok * ((nrows + rows - 1) / rows);
+        return ((t + c->num_cu - 1) / c->num_cu) * rows;
+    };
+    p.trows = c->tune.mx_rows == 96 || c->tune.mx_rows == 128 ? c->tune.mx_rows : (cost(96) < cost(128) ? 96 : 128);
+    const long tiles = (long)ttok * ((nrows + p.trows - 1) / p.trows);
+    // A grid that leaves most CUs idle is widened along K: each split writes partial sums
+    // to a workspace slab and a second kernel adds the slabs in order.
+    long split = c->tune.mx_split > 0 ? c->tune.mx_split : (tiles * 2 <= c->num_cu ? c->num_cu / tiles : 1);
+    split = std::min(split, std::min(8L, (long)stages));
+    p.per = (int)((stages + split - 1) / split);
+    p.split = (stages + p.per - 1) / p.per;   // no empty split
+    int mtrows;
+    const double rounds = mx_tile_rounds(c, nrows, ntok, &mtrows), mb = 1e-6 * nrows * (double)(k / 32 * 17);
+    p.planes_us = 6 + mb + 2.75 * k / 1024 * rounds;
+    p.rows_us = 7 + (double)cost(p.trows) / p.trows * p.per * (p.trows == 96 ? 2.15 : 2.9) +
+                (p.split > 1 ? 3.5 + (double)ntok * nrows * p.split * 4 / 3e6 : 0);
+    return p;
+}
+
 // Few tokens: 16-row workgroups whose wavefronts split K, in chunks of up to 64 tokens, one launch after a prep
 // that lays the activations out in the order the block decode produces.
-// From where: the kernels for a handful of tokens grow by about a microsecond a token, this one does not, but its
-// prep is a launch (us at 2880 x 2880, rows: 4 tokens 7.4 against 7.3, 8 tokens 11.8 against 7.4; planes: 3 tokens
-// 6.2 against 6.9, 4 tokens 7.0 against 6.8; at 1100 x 1216 the handful's are as fast up to 8).
-// Up to where: a chunk more costs little while the grid is one round of the CUs (rows 2880 x 2880: 128 tokens 16.1
-// against the tiles' 17.5, 192 tokens 21.5 against 18.2; 1100 x 1216: 192 tokens 8.6 against 10.1; planes, whose tiles
-// have no rows to turn: 96 tokens 13.0 against 12.7, 2000 x 4512 12.6 against 15.6).
+// From where: the kernels for a handful of tokens grow with the tokens, this one does not, but its prep is a launch.
+// Over rows a token more costs what a round of their workgroups does, four rows each, on all CUs (us, these against this
+// one: one round 1024 x 2880, 8 tokens 5.9 and 7.0; two 2048 x 1024, 6 and 8 tokens 4.4 and 4.9, 5.2 and 4.9, 2048 x 2048,
+// 6 and 8 tokens 5.2 and 5.9, 6.2 and 5.9; three 2880 x 1440, 5 tokens 5.5 and 5.5, 2880 x 2880 8.8 and 7.0; six 5760 x
+// 2880, 3 tokens 11.0 and 9.4, 2 tokens 8.5 and 9.3); over planes what K does (1024 x 1024, 4 and 5 tokens 4.4 and 4.5, 4.7
+// and 4.6; 2880 x 1440, 3 and 4 tokens 4.5 and 4.8, 5.0 and 4.9; 1024 x 2880, 2 and 3 tokens 4.6 and 5.2, 5.4 and 5.3; matrices of
+// a few tens of kilobytes keep the one launch, 130 x 256, 4 and 5 tokens 4.0 and 4.1, 4.4 and 4.2).
+// Up to where: 64 tokens are one chunk.  More, up to 128 tokens, or 256 while the chunks are one round of the CUs: over
+// rows while that is estimated faster than the tiles -- 4 and 0.48 a token tile and 1024 of K for each round, a tenth
+// more with several chunks (2880 x 2880, 128 tokens 16.3 against 17.8; 2880 x 14336, 80 tokens 46 against 28, 5760 x 5760,
+// 128 tokens 35 against 27, 512 x 8192, 128 tokens 24.2 against 20.5 for the tiles) --, over planes, whose tiles have
+// no rows to turn, only while they are one round (2880 x 2880, 96 tokens 13.0 against 12.8; 512 x 8192, 256 tokens 20.7
+// against 24.5; K slices over rows restored from the planes are no match for either: 2880 x 14336, 96 tokens 57 against 36).
 bool mx_few_applies(const jl_ctx* c, int nrows, int k, int ntok, bool planes) {
     if (c->tune.mx_rows == 96 || c->tune.mx_rows == 128 || ntok > 65535) return false;
     const int form = c->tune.mx_planes;
     if (form == 3 || form == 4 || (planes && (form == 2 || (form && ntok <= 8)))) return false;
-    const int least = c->tune.mx_few_min > 0 ? c->tune.mx_few_min : (long)nrows * k < 4000000 ? 9 : planes ? 4 : 5;
+    int least = c->tune.mx_few_min;
+    if (least <= 0) {
+        const long rounds = ((nrows + 3) / 4 + (long)c->num_cu - 1) / c->num_cu;
+        least = planes ? ((long)nrows * k < 200000 ? 9 : k <= 1024 ? 5 : k < 2048 ? 4 : 3) : rounds == 1 ? 9 : rounds == 2 ? 7 : rounds == 3 ? 5 : 3;
+    }
     if (ntok < least) return false;
     if (c->tune.mx_few > 0) return ntok <= c->tune.mx_few;
-    return ntok <= (planes ? 64 : 128) || (ntok <= 256 && (long)((nrows + 15) / 16) * ((ntok + 63) / 64) <= c->num_cu);
+    if (ntok <= 64) return true;
+    const int tiles = (ntok + 15) / 16, chunks = (tiles + 3) / 4, nt = (tiles + chunks - 1) / chunks;
+    const long wgs = (long)((nrows + 15) / 16) * ((tiles + nt - 1) / nt), rounds = (wgs + c->num_cu - 1) / c->num_cu;
+    if (ntok > 256 || (rounds > 1 && (planes || ntok > 128))) return false;
+    if (planes) return true;
+    const MxRowsPlan p = mx_rows_plan(c, nrows, k, ntok);
+    return 1.1 * (4 + 0.48e-3 * k * nt * rounds) < std::min(p.rows_us, p.planes_us);
 }
 int mx_few_launch(jl_ctx* c, MxGemmArgs& a, const uint16_t* x, hipStream_t st) {
     const int tiles = (a.ntok + 15) / 16, groups = (a.k + 127) / 128, chunks = (tiles + 3) / 4, nt = (tiles + chunks - 1) / chunks;
@@ -2698,16 +2760,6 @@ int mx_few_launch(jl_ctx* c, MxGemmArgs& a, const uint16_t* x, hipStream_t st) {
 }
 // Tiles of 64 tokens x 64 or 96 rows whose wavefronts split K, the weights taken from planes; rows (w) are turned
 // into planes in the workspace by the launch that lays the activations out.
-// Rows a tile: a round of the CUs takes about 1.36 times as long with 96 (measured at k = 1216 to 4512), so 96 where
-// that saves the rounds (2880 rows: 512 tokens 21.1 -> 17.4 us, 384 tokens of 5000 rows 19.7 against 23.7).
-double mx_tile_rounds(const jl_ctx* c, int nrows, int ntok, int* trows) {
-    auto rounds = [&](int rows) {
-        return (double)(((long)((ntok + 63) / 64) * ((nrows + rows - 1) / rows) + c->num_cu - 1) / c->num_cu);
-    };
-    const double r64 = rounds(64), r96 = 1.36 * rounds(96);
-    *trows = c->tune.mx_planes == 3 ? 64 : c->tune.mx_planes == 4 ? 96 : r96 < r64 ? 96 : 64;
-    return *trows == 96 ? r96 : r64;
-}
 size_t mx_tile_xa_bytes(int k, int ntok) { return (size_t)((k + 63) / 64) * ((ntok + 63) / 64 * 2) * 4 * 1024; }
 // rows turned into planes: codes and exponents of rows in whole runs of 64
 size_t mx_tile_plane_bytes(int nrows, int k) { return (size_t)(k / 32) * 17 * ((nrows + 63) / 64 * 64); }
@@ -2765,38 +2817,16 @@ int jl_matmul_mxfp4_bf16_dev(jl_ctx* c, float* out, const void* w, const uint16_
         return launch(c, "jl_mxfp4_matvec", (unsigned)((nrows + 3) / 4), 1, 256, 0, st, params);
     // activations into matrix-fragment order (tokens padded to whole tiles, K to whole stages)
     const int tok_pad = (ntok + 127) / 128 * 128, stages = (k + 255) / 256;
-    // rows per tile: 128, or 96 where that takes fewer rounds x rows (2880 rows x 1024 tokens:
-    // 184 tiles of 128 rows leave 72 CUs idle for a whole tile, 240 of 96 rows do not)
-    auto cost = [&](int rows) {
-        const long t = (long)(tok_pad / 128) * ((nrows + rows - 1) / rows);
-        return ((t + c->num_cu - 1) / c->num_cu) * rows;
-    };
-    const int trows = c->tune.mx_rows == 96 || c->tune.mx_rows == 128 ? c->tune.mx_rows
-                      : (cost(96) < cost(128) ? 96 : 128);
+    const MxRowsPlan plan = mx_rows_plan(c, nrows, k, ntok);
+    const int trows = plan.trows, nsplit = plan.split;
     const char* gemm_name = trows == 96 ? "jl_mxfp4_gemm_r96" : "jl_mxfp4_gemm";
-    const int tiles = (tok_pad / 128) * ((nrows + trows - 1) / trows);
-    // A grid that leaves most CUs idle is widened along K: each split writes partial sums
-    // to a workspace slab and a second kernel adds the slabs in order.
-    int nsplit = c->tune.mx_split > 0 ? c->tune.mx_split : (tiles * 2 <= c->num_cu ? c->num_cu / tiles : 1);
-    if (nsplit > 8) nsplit = 8;
-    if (nsplit > stages) nsplit = stages;
-    int per = (stages + nsplit - 1) / nsplit;
-    nsplit = (stages + per - 1) / per;   // no empty split
-    // These tiles, or the smaller ones of the planes with the rows turned into planes on the way: by their costs as
-    // measured (us; 1100 x 1216 to 5000 x 2048, 64 to 2048 tokens).  These: a stage of K = 256 takes 2.15 with 96 rows
-    // and 2.9 with 128, a split a launch and its slabs; those: 1 a MB of weights and 2.75 a round and 1024 of K.  The
-    // estimates are good to about 8 %, so those only where they win by more (2880 x 2880: 512 tokens 27.9 -> 21.8, 1024
-    // tokens 31.5 against 32.3, 2048 tokens 57 -> 52).
-    int mtrows;
-    const double rounds = mx_tile_rounds(c, nrows, ntok, &mtrows), mb = 1e-6 * nrows * (double)a.row_bytes;
-    const double small_us = 6 + mb + 2.75 * k / 1024 * rounds;
-    const double large_us = 7 + (double)cost(trows) / trows * per * (trows == 96 ? 2.15 : 2.9) +
-                            (nsplit > 1 ? 3.5 + (double)ntok * nrows * nsplit * 4 / 3e6 : 0);
+    // (the estimates are good to about 8 %, so planes only where they win by more: 2880 x 2880, 512 tokens 27.9 -> 21.8,
+    // 1024 tokens 31.5 against 32.3, 2048 tokens 57 -> 52)
     const unsigned lds = 2u * 128u * 264u * 2u;   // two weight stages [128][264] bf16
     // (the planes of a reserved call have to fit what is there; jl_reserve_shape, a dry run, makes them room)
     const bool room = !reserved_for(c, ntok, k) || call_dry_run(c) || mx_tile_xa_bytes(k, ntok) + mx_tile_plane_bytes(nrows, k) <= c->gemm_ws_bytes;
     if (c->tune.mx_planes == 3 || c->tune.mx_planes == 4 || lds > c->lds_limit ||
-        (room && !c->tune.mx_rows && !c->tune.mx_split && 1.08 * small_us < large_us)) {
+        (room && !c->tune.mx_rows && !c->tune.mx_split && 1.08 * plan.planes_us < plan.rows_us)) {
         MxPlanesGemmArgs ga;
         ga.out = out; ga.nrows = nrows; ga.k = k; ga.ntok = ntok;
         return mx_tile_launch(c, ga, (const uint8_t*)w, x, st);
