@@ -942,7 +942,8 @@ struct FewCall {
 bool few_fits(const jl_ctx* c, int type, bool planes, int nrows, int k, int ncols, int stride) {
     const TypeInfo* ti = type_info(type);
     if (!ti || c->tune.gemm_few == 2 || k % ti->block_elems || ncols > 65535 * 4 || (k + 255) / 256 > 65535) return false;
-    if (planes) return (size_t)stride * 4 * 8 < ((size_t)1 << 32);
+    if (planes)   // (a lane's offset: up to twelve planes of Q6_K's, the whole D plane of Q8_0's)
+        return (size_t)stride * 4 * 12 < ((size_t)1 << 32) && (type != JL_TYPE_Q8_0 || (size_t)(k / 32) * (((size_t)stride + 1) / 2) * 4 < ((size_t)1 << 32));
     if (type == JL_TYPE_Q8_0 && k % 64) return false;   // (rows on 4-byte boundaries)
     return (size_t)nrows * (size_t)(k / ti->block_elems) * ti->block_bytes < ((size_t)1 << 32);
 }
