@@ -406,8 +406,11 @@ int matvec_launch(jl_ctx* c, float* out, int type, const void* w, const float* x
     // sixteen wavefronts a CU for the k-quants, whose registers leave room for no more (a second round of workgroups
     // quantizes x again: Q6_K 10822 x 768 7.0 us -> 5.6, 14336 x 4096 10.2 -> 8.6), as two workgroups of eight, which
     // cover each other's barriers (9988 x 5120 Q6_K 9.4 against 10.3 as one; 6000 x 4096 Q4_K 4.5 and 4.5);
-    // Q8_0: two workgroups of twelve, or, up to two rounds of them, one of sixteen wavefronts (14336 x 4096 10.2
-    // against 10.6, 8192 x 4096 7.3 against 6.8).
+    // Q8_0: two workgroups of twelve, or, up to two rounds of them, one of sixteen wavefronts (8192 x 4096 7.3 against
+    // 6.8); from forty rows a CU with the two-block form, K = 3584 to 5120, two of eight (weights from memory, eight
+    // against twelve: 14336 x 4096 11.8 and 12.4, 12800 x 5120 14.7 and 15.7, 10240 x 3584 8.0 and 9.3; from cache the
+    // same, 10.3 and 10.5, 12.1 and 12.5, 6.6 and 7.2; outside that range the ones gain what the others lose: 14336 x 2560
+    // 8.1 and 8.4, from cache 6.8 and 6.3, 14336 x 14336 41.6 and 39.4).
     int rpw = c->tune.rpw, block = c->tune.block;
     if (rpw <= 0 || resid || !x) rpw = 1;   // (the kernels with the residual add or a quantized activation: one row a wavefront)
     if (rpw != 1 && rpw != 2 && rpw != 4) return fail(c, JL_ERR_ARG, "matvec: rpw=%d", rpw);
@@ -415,7 +418,8 @@ int matvec_launch(jl_ctx* c, float* out, int type, const void* w, const float* x
     const bool small = nrows <= 16 * c->num_cu;
     const bool one_per_cu = small || (type == JL_TYPE_Q8_0 && pair && nrows <= 32 * c->num_cu && k >= 4096);
     if (block <= 0)
-        block = small ? 64 * std::max(8, (nrows + c->num_cu - 1) / c->num_cu) : one_per_cu ? 1024 : type == JL_TYPE_Q8_0 ? 768 : 512;
+        block = small ? 64 * std::max(8, (nrows + c->num_cu - 1) / c->num_cu) : one_per_cu ? 1024 :
+                type == JL_TYPE_Q8_0 && !(pair && nrows >= 40 * c->num_cu && k >= 3584 && k <= 5120) ? 768 : 512;
     if (block % 64 != 0 || block > 1024) return fail(c, JL_ERR_ARG, "matvec: block=%d", block);
     if (block > matvec_max_block(type, rpw, pair)) block = matvec_max_block(type, rpw, pair);
     const int rows_per_block = (block / 64) * rpw;
