@@ -890,10 +890,15 @@ int gemm_i8_launch(jl_ctx* c, float* out, int type, const void* w, const float* 
     ga.out_stride = nrows; ga.sb_per = 0;
     void* gp[] = {&ga};
     const int unit = q6 || q4 ? 2 : 1, nunit = nstage / unit;   // stages a split is made of
-    // Shape and K split by what they should take.  A wavefront's 32 x 32 x 32 block costs its SIMD 0.1 us with two or
-    // three wavefronts there and 0.14 with one; workgroups are resident two (128 x 128: Q8_0 only, the others have no
-    // registers for it) or three (128 x 64; two for the k-quants) a CU; a round costs 1.5 us to begin, the slabs of a
-    // split a launch and a trip through memory.
+    // Shape and K split by what they should take.  A wavefront's 32 x 32 x 32 block costs its SIMD `many` us with two or
+    // three wavefronts there and `alone` with one; workgroups are resident two (128 x 128: Q8_0 only, the others have no
+    // registers for it) or three (128 x 64; two for the k-quants) a CU; the slabs of a split a launch (hidden under the
+    // tail of the tiles) and a trip through memory.  Fitted to 19 shapes (1024 x 4096 to 14336 x 4096, 100 to 2048 tokens)
+    // of every type at 1 to 8 splits, 6 % each; the pick is within 5 % of the best split at all but eight of the 76.  (One
+    // pair of constants for every type left the k-quants uncut: window 32, 512 tokens of 4096 x 4096 Q4_K 62 against 52
+    // in two, Q6_K 80 against 66, 900 tokens of 1700 x 8192 112 against 85 and 143 against 105.)
+    const double many = type == JL_TYPE_Q8_0 ? 0.088 : q4 ? 0.114 : c->act_window == 32 ? 0.160 : 0.097;
+    const double alone = type == JL_TYPE_Q8_0 ? 0.125 : q4 ? 0.177 : c->act_window == 32 ? 0.241 : 0.131;
     I8Shape f = {2, 4};
     int nsplit = 1;
     double best = 1e30;
@@ -908,9 +913,9 @@ int gemm_i8_launch(jl_ctx* c, float* out, int type, const void* w, const float* 
             if (s > 1 && n * s * 4 > most) continue;
             const long wgs = groups * s, full = wgs / (cap * c->num_cu), left = wgs - full * cap * c->num_cu;
             const double block = 4 * rt * per * unit;     // of a wavefront
-            double us = full * (1.5 + 0.1 * cap * block);
-            if (left) us += 1.5 + std::max(0.1 * ((left + c->num_cu - 1) / c->num_cu), 0.14) * block;
-            if (s > 1) us += 4.0 + 4e-6 * (s + 1) * n;
+            double us = full * (0.15 + many * cap * block);
+            if (left) us += 0.15 + std::max(many * ((left + c->num_cu - 1) / c->num_cu), alone) * block;
+            if (s > 1) us += 0.25 + 1.16e-6 * (s + 1) * n;
             if (us < best) { best = us; f = {rt, 4}; nsplit = s; }
         }
     }
