@@ -23,6 +23,7 @@ struct HipApi {
     hipError_t (*ModuleLoad)(hipModule_t*, const char*) = nullptr;
     hipError_t (*ModuleUnload)(hipModule_t) = nullptr;
     hipError_t (*ModuleGetFunction)(hipFunction_t*, hipModule_t, const char*) = nullptr;
+    hipError_t (*FuncGetAttribute)(int*, hipFunction_attribute, hipFunction_t) = nullptr;
     hipError_t (*ModuleLaunchKernel)(hipFunction_t, unsigned, unsigned, unsigned, unsigned, unsigned,
                                      unsigned, unsigned, hipStream_t, void**, void**) = nullptr;
     hipError_t (*Malloc)(void**, size_t) = nullptr;
@@ -72,6 +73,7 @@ inline const HipApi* hip_api(std::string* why) {
             JL_SYM(ModuleLoad, "hipModuleLoad");
             JL_SYM(ModuleUnload, "hipModuleUnload");
             JL_SYM(ModuleGetFunction, "hipModuleGetFunction");
+            JL_SYM(FuncGetAttribute, "hipFuncGetAttribute");
             JL_SYM(ModuleLaunchKernel, "hipModuleLaunchKernel");
             JL_SYM(Malloc, "hipMalloc");
             JL_SYM(Free, "hipFree");

@@ -165,6 +165,7 @@ struct jl_ctx {
     int gemm_min_tok = 3;  // below this a per-token matvec loop is as fast (3.8 us a token against 8.9 us for up to 16)
     int num_cu = 0;
     size_t lds_limit = 0;
+    uint8_t few_simd[5][2][4][3] = {};   // wavefronts a SIMD holds of jl_few_*: form, planes, token tiles - 1, row tiles / 2 (0: not built)
     std::atomic<unsigned long long> launches{0};   // kernels launched so far (jl_launch_count)
 
     // prefill GEMM workspace (quantized activations in stage layout), grown on demand
@@ -957,6 +958,71 @@ bool few_fits(const jl_ctx* c, int type, bool planes, int nrows, int k, int ncol
     return (size_t)nrows * (size_t)(k / ti->block_elems) * ti->block_bytes < ((size_t)1 << 32);
 }
 
+int few_form(int type, bool w256) { return type == JL_TYPE_Q8_0 ? 2 : type == JL_TYPE_Q4_K ? w256 : 3 + w256; }
+
+// A workgroup's token tiles (of 16), row tiles (of 16) and wavefronts, over which K is dealt.
+struct FewShape { int nt, rt, nw; };
+
+// Token tiles: what the (average) group fills.  Two rules for the other two.
+//
+// One group: the least of an estimate, in units of a wavefront's step of 256 alone on its SIMD.  Workgroups of eight or
+// four wavefronts run in rounds of `cap` a CU (registers and LDS), the last with what is left; a round takes `e` (its
+// start, the reduction) and ceil(K / 256 / wavefronts) steps, a step a serial chain (longer with more row tiles) and a
+// part of each wavefront the SIMD holds.  Fitted to 34 shapes (1024 x 1024 to 14336 x 4096) of every type, window and
+// layout at 8, 24, 40 and 64 tokens over everything that is built: the pick is 1 to 4 % behind the best on average.
+// Against always eight wavefronts, and row tiles where most CUs kept a workgroup, geometric means over them: 8 and 24
+// tokens 1 to 4 % faster, 64 tokens 7 to 10 %, the worst loss 11 % and the largest gain 66 %: a workgroup over a round's
+// end costs a whole round (rows of 9216 x 1280, window 32, 64 tokens: Q6_K 25.9 against 15.6).  (Three, five and six wavefronts are the best of some shapes and, estimated so, the worst of others: 5120 x
+// 5120 Q6_K, 64 tokens, five 38.6, eight 25.7.)  Three token tiles: 33 to 48 tokens took four (40 tokens 22 % faster, never slower).
+//
+// Groups of a mixture (grid: rows, banks, experts; most groups part empty): row tiles as many as leave most CUs a
+// workgroup, eight wavefronts.  More rows a workgroup share the activations' loads, and over planes widen the weights'
+// (14336 x 4096 / 4096 x 4096, us, row tiles 1 / 2 / 4: Q8_0 planes 16 tokens 28.8 20.6 18.7 / 11.6 11.3 14.7; Q4_K
+// planes 20.1 15.4 14.4 / 8.4 9.4 12.6; Q4_K rows 18.2 16.4 - / 8.5 10.2 -; Q8_0 rows 64 tokens 39.3 35.0 - /
+// 13.5 18.0 -).
+FewShape few_shape(const jl_ctx* c, int type, bool w256, bool planes, int nrows, int k, int ncols, bool groups, int n_expert, int nmat) {
+    const int nsb = (k + 255) / 256, form = few_form(type, w256);
+    const long avg = ((long)ncols + n_expert - 1) / n_expert, sheets = (long)n_expert * nmat, cus = c->num_cu;
+    FewShape f = {1, 1, std::min(8, nsb)};
+    if (groups) f.nt = avg <= 16 ? 1 : avg <= 32 ? 2 : 4;
+    else f.nt = (int)std::min<long>((avg + 15) / 16, 4);
+    if (c->tune.few_nt) f.nt = c->tune.few_nt;
+    if (groups) {
+        if (planes ? (nrows + 31) / 32 * sheets >= cus : f.nt != 2 && (type == JL_TYPE_Q4_K || f.nt == 4) && (nrows + 31) / 32 * sheets >= cus)
+            f.rt = 2;
+        if (planes && f.nt <= 2 && (f.nt == 2 || type != JL_TYPE_Q6_K) && (nrows + 63) / 64 * sheets * 10 >= cus * 7) f.rt = 4;
+    } else {
+        // (One token tile: steps are short and mostly the weights' way, which over rows leads through LDS and over planes
+        // gets wider loads with more row tiles.)
+        const bool one = f.nt == 1;
+        const double e = one ? 0.5 : 3, more = !one ? 1.6 : planes ? 1.2 : 1.8, longer = one ? 2 : 1.5;
+        double best = 1e30;
+        for (int w : {8, 4}) {
+            const int nw = std::min(w, nsb);
+            double part = 0.25 * nw, chain = 1;
+            for (int rt : {1, 2, 4}) {
+                const int simd = f.nt > 4 ? 0 : c->few_simd[form][planes][f.nt - 1][rt / 2];
+                if (!simd || nrows < rt) break;
+                const size_t lds = std::max(nw * JL_FEW_WAVE_BYTES(type, planes, rt), JL_FEW_RED_BYTES(nw, f.nt, rt));
+                if (lds > c->lds_limit) break;
+                const long cap = std::max<long>(1, std::min<long>(4 * simd / nw, (long)(c->lds_limit / lds)));
+                const long wgs = (nrows + 16 * rt - 1) / (16 * rt) * sheets, full = wgs / (cap * cus), left = (wgs - full * cap * cus + cus - 1) / cus;
+                const int steps = (nsb + nw - 1) / nw;
+                double t = full * (e + steps * (chain + part * cap));
+                if (left) t += e + steps * (chain + part * left);
+                if (t < best) { best = t; f.rt = rt; f.nw = nw; }
+                part *= more; chain *= longer;
+            }
+        }
+    }
+    if (c->tune.few_rt) f.rt = c->tune.few_rt;
+    if (nrows < f.rt) f.rt = 1;
+    if (c->tune.few_waves) f.nw = std::min(c->tune.few_waves, nsb);
+    else if (c->tune.few_rt || groups) f.nw = std::min(8, nsb);
+    while (f.nw > 1 && (size_t)f.nw * JL_FEW_WAVE_BYTES(type, planes, f.rt) > c->lds_limit) f.nw--;
+    return f;
+}
+
 int few_launch(jl_ctx* c, const FewCall& f, hipStream_t st) {
     const bool planes = f.pl[0] != nullptr;
     const TypeInfo* ti = type_info(f.type);
@@ -990,23 +1056,8 @@ int few_launch(jl_ctx* c, const FewCall& f, hipStream_t st) {
     if (planes) { a.prow0 = f.pl[0]->row; a.pstride = f.pl[0]->stride; }
     a.nrows = f.nrows; a.k = f.k; a.row_bytes = (f.k / ti->block_elems) * ti->block_bytes;
     a.ncols = f.ncols; a.nslots = nslots; a.nch = nch;
-    // Token tiles a workgroup: what the (average) group fills.  Row tiles: more rows a workgroup share the
-    // activations' loads, and over planes widen the weights' (measured at 14336 x 4096 / 4096 x 4096, us, row
-    // tiles 1 / 2 / 4: Q8_0 planes 16 tokens 28.8 20.6 18.7 / 11.6 11.3 14.7; Q4_K planes 20.1 15.4 14.4 /
-    // 8.4 9.4 12.6; Q4_K rows 18.2 16.4 - / 8.5 10.2 -; Q8_0 rows 64 tokens 39.3 35.0 - / 13.5 18.0 -): as
-    // many as leave most CUs a workgroup.
-    const long avg = ((long)f.ncols + f.n_expert - 1) / f.n_expert;
-    const int nt = c->tune.few_nt ? c->tune.few_nt : avg <= 16 ? 1 : avg <= 32 ? 2 : 4;
-    const long sheets = (long)f.n_expert * f.nmat, cus = c->num_cu;
-    int rt = 1;
-    if (planes ? (f.nrows + 31) / 32 * sheets >= cus : nt != 2 && (f.type == JL_TYPE_Q4_K || nt == 4) && (f.nrows + 31) / 32 * sheets >= cus)
-        rt = 2;
-    if (planes && nt <= 2 && (nt == 2 || f.type != JL_TYPE_Q6_K) && (f.nrows + 63) / 64 * sheets * 10 >= cus * 7) rt = 4;
-    if (c->tune.few_rt) rt = c->tune.few_rt;
-    if (f.nrows < rt) rt = 1;
-    int nw = c->tune.few_waves ? c->tune.few_waves : 8;
-    if (nw > nch / 2) nw = nch / 2;
-    while (nw > 1 && (size_t)nw * JL_FEW_WAVE_BYTES(f.type, planes, rt) > c->lds_limit) nw--;
+    const FewShape sh = few_shape(c, f.type, w256, planes, f.nrows, f.k, f.ncols, f.start != nullptr, f.n_expert, f.nmat);
+    const int nt = sh.nt, rt = sh.rt, nw = sh.nw;
     a.nwaves = nw;
     const unsigned lds = (unsigned)std::max(nw * JL_FEW_WAVE_BYTES(f.type, planes, rt), JL_FEW_RED_BYTES(nw, nt, rt));
     if (lds > c->lds_limit) return JL_DECLINED;
@@ -1728,7 +1779,7 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     names.push_back("jl_moe_gemm_i8_q8_0_r4t4");
     for (const char* tag : {"q4k", "q4kw", "q8_0", "q6k", "q6kw"})
         for (const char* layout : {"rows", "planes"})
-            for (const char* size : {"t1r1", "t1r2", "t2r1", "t4r1", "t4r2", "t1r4", "t2r2", "t2r4"})
+            for (const char* size : {"t1r1", "t1r2", "t2r1", "t3r1", "t3r2", "t4r1", "t4r2", "t1r4", "t2r2", "t2r4"})
                 if (layout[0] == 'p' || (strcmp(size, "t1r4") && strcmp(size, "t2r2") && strcmp(size, "t2r4"))) names.push_back(std::string("jl_few_") + tag + "_" + layout + "_" + size);
     for (const char* tag : {"q4k", "q8_0", "q6k"})
         for (int rw : {16, 32, 64})
@@ -1768,6 +1819,21 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
             return bail(JL_ERR_HIP, "hipModuleGetFunction(" + n + "): " + H->GetErrorString(e));
         c->fn.add(n, f);
     }
+    for (int form = 0; form < 5; form++)
+        for (int planes = 0; planes < 2; planes++)
+            for (int nt = 1; nt <= 4; nt++)
+                for (int rt : {1, 2, 4}) {
+                    const char* tags[] = {"q4k", "q4kw", "q8_0", "q6k", "q6kw"};   // (few_form)
+                    Name n;
+                    n << "jl_few_" << tags[form] << (planes ? "_planes" : "_rows") << "_t" << nt << "r" << rt;
+                    const hipFunction_t f = c->fn.find(n);
+                    int regs = 0;
+                    if (!f) continue;
+                    e = H->FuncGetAttribute(&regs, HIP_FUNC_ATTRIBUTE_NUM_REGS, f);
+                    if (e != hipSuccess) return bail(JL_ERR_HIP, std::string("hipFuncGetAttribute(") + (const char*)n + "): " + H->GetErrorString(e));
+                    // (a SIMD's 512 registers a lane, in blocks of eight)
+                    c->few_simd[form][planes][nt - 1][rt / 2] = (uint8_t)std::max(1, std::min(8, 512 / std::max(8, (regs + 7) / 8 * 8)));
+                }
     {
         uint32_t tab[2 * 17];
         for (uint32_t n = 0; n <= 16; n++) { tab[2 * n] = 0; tab[2 * n + 1] = n; }

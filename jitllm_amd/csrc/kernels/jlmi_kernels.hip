@@ -136,7 +136,8 @@ extern "C" __global__ __launch_bounds__(256) void jl_few_prep(FewI8PrepArgs p) {
     }
 #define JL_FEW_SIZES(T, TYPE, P, PL, W256)                                                                      \
     JL_FEW_KERNEL(T, TYPE, P, PL, 1, 1, W256) JL_FEW_KERNEL(T, TYPE, P, PL, 1, 2, W256)                         \
-    JL_FEW_KERNEL(T, TYPE, P, PL, 2, 1, W256) JL_FEW_KERNEL(T, TYPE, P, PL, 4, 1, W256)                         \
+    JL_FEW_KERNEL(T, TYPE, P, PL, 2, 1, W256) JL_FEW_KERNEL(T, TYPE, P, PL, 3, 1, W256)                         \
+    JL_FEW_KERNEL(T, TYPE, P, PL, 3, 2, W256) JL_FEW_KERNEL(T, TYPE, P, PL, 4, 1, W256)                         \
     JL_FEW_KERNEL(T, TYPE, P, PL, 4, 2, W256)
 #define JL_FEW_WIDE(T, TYPE, W256)                                                                              \
     JL_FEW_KERNEL(T, TYPE, planes, true, 1, 4, W256) JL_FEW_KERNEL(T, TYPE, planes, true, 2, 2, W256)           \

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(1, 16, 256), (3, 37, 1280), (16, 100, 2816), (17, 130, 1024), (33, 48, 512), (64, 200, 2304), (5, 33, 160),
           (20, 50, 320), (7, 64, 832)]
 # (token tiles, row tiles): the built-in choice and every compiled pair
-TILES = [(0, 0), (1, 1), (1, 2), (2, 1), (4, 1), (4, 2), (1, 4), (2, 2), (2, 4)]
+TILES = [(0, 0), (1, 1), (1, 2), (2, 1), (3, 1), (3, 2), (4, 1), (4, 2), (1, 4), (2, 2), (2, 4)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
@@ -54,6 +54,28 @@ def test_few_tokens_rows_and_planes(dev, devbuf, t, window, shape):
     finally:
         dev.set_tuning(gemm__few=0, few__nt=0, few__rt=0)
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("rows", [1, 2])
+@pytest.mark.parametrize("waves", [1, 3, 4, 8])
+def test_few_tokens_three_tiles_dealt_over_wavefronts(dev, devbuf, waves, rows):
+    """K of eleven super-blocks over fewer wavefronts than that, the last round part empty; 33, 47 and 48 tokens."""
+    t, nrows, k = quant.Q4_K, 70, 2816
+    w = synth.random_weights(t, nrows, k, seed=3)
+    x = np.stack([synth.activations(k, seed=i) for i in range(48)])
+    want = oracle.matmul_q8act_f64(t, w, x, nrows, k, 48, 32)
+    wd, xd = devbuf(w), devbuf(x)
+    try:
+        dev.set_tuning(few__waves=waves, few__rt=rows)
+        for ntok in (33, 47, 48):
+            out = devbuf(np.full(ntok * nrows + 8, 3e30, np.float32))
+            assert dev.matmul_dev(out.ptr, t, wd.ptr, xd.ptr, nrows, k, ntok)
+            dev.synchronize()
+            got = out.get()
+            assert np.all(got[ntok * nrows:] == np.float32(3e30))
+            assert nmse(got[:ntok * nrows].reshape(ntok, nrows), want[:ntok]) <= 1e-10
+    finally:
+        dev.set_tuning(few__waves=0, few__rt=0)
 
 
 @pytest.mark.parametrize("t,nrows,k", [(quant.Q8_0, 65, 32), (quant.Q8_0, 130, 544), (quant.Q4_K, 63, 256), (quant.Q6_K, 129, 768),
