@@ -2787,13 +2787,14 @@ MxRowsPlan mx_rows_plan(const jl_ctx* c, int nrows, int k, int ntok) {
 
 // Few tokens: 16-row workgroups whose wavefronts split K, in chunks of up to 64 tokens, one launch after a prep
 // that lays the activations out in the order the block decode produces.
-// From where: the kernels for a handful of tokens grow with the tokens, this one does not, but its prep is a launch.
-// Over rows a token more costs what a round of their workgroups does, four rows each, on all CUs (us, these against this
-// one: one round 1024 x 2880, 8 tokens 5.9 and 7.0; two 2048 x 1024, 6 and 8 tokens 4.4 and 4.9, 5.2 and 4.9, 2048 x 2048,
-// 6 and 8 tokens 5.2 and 5.9, 6.2 and 5.9; three 2880 x 1440, 5 tokens 5.5 and 5.5, 2880 x 2880 8.8 and 7.0; six 5760 x
-// 2880, 3 tokens 11.0 and 9.4, 2 tokens 8.5 and 9.3); over planes what K does (1024 x 1024, 4 and 5 tokens 4.4 and 4.5, 4.7
-// and 4.6; 2880 x 1440, 3 and 4 tokens 4.5 and 4.8, 5.0 and 4.9; 1024 x 2880, 2 and 3 tokens 4.6 and 5.2, 5.4 and 5.3; matrices of
-// a few tens of kilobytes keep the one launch, 130 x 256, 4 and 5 tokens 4.0 and 4.1, 4.4 and 4.2).
+// From where: the kernels for a handful of tokens grow with the tokens, this one does not, but it is two launches, which a
+// host that issues calls one after the other cannot do in less than 6.7 us.  From three tokens, so, where the one launch
+// is estimated to take more than that and more than this form: over rows a token costs what a round of their workgroups
+// does, four rows each, on all CUs, over planes what K and the matrix do (fitted to 17 shapes, 512 x 512 to 12288 x 2048,
+// 2 to 8 tokens, 6 % each).  Device us, these against this one: rows 2880 x 2880, 3 and 5 tokens 6.5 and 6.8, 8.9 and 6.9,
+// 5760 x 2880, 3 tokens 11.3 and 9.3; planes 5760 x 2880, 3 tokens 9.1 and 7.0, 3413 x 1536, 5 and 8 tokens 6.0 and 5.4,
+// 7.5 and 5.4.  (By device time alone it would begin earlier: planes 2124 x 1120, 5 tokens 5.5 and 4.7, but call by call
+// 5.4 and 6.8.)
 // Up to where: 64 tokens are one chunk.  More, up to 128 tokens, or 256 while the chunks are one round of the CUs: over
 // rows while that is estimated faster than the tiles -- 4 and 0.48 a token tile and 1024 of K for each round, a tenth
 // more with several chunks (2880 x 2880, 128 tokens 16.3 against 17.8; 2880 x 14336, 80 tokens 46 against 28, 5760 x 5760,
@@ -2804,12 +2805,14 @@ bool mx_few_applies(const jl_ctx* c, int nrows, int k, int ntok, bool planes) {
     if (c->tune.mx_rows == 96 || c->tune.mx_rows == 128 || ntok > 65535) return false;
     const int form = c->tune.mx_planes;
     if (form == 3 || form == 4 || (planes && (form == 2 || (form && ntok <= 8)))) return false;
-    int least = c->tune.mx_few_min;
-    if (least <= 0) {
-        const long rounds = ((nrows + 3) / 4 + (long)c->num_cu - 1) / c->num_cu;
-        least = planes ? ((long)nrows * k < 200000 ? 9 : k <= 1024 ? 5 : k < 2048 ? 4 : 3) : rounds == 1 ? 9 : rounds == 2 ? 7 : rounds == 3 ? 5 : 3;
+    if (c->tune.mx_few_min > 0) {
+        if (ntok < c->tune.mx_few_min) return false;
+    } else if (ntok <= 8) {
+        const long r4 = ((nrows + 3) / 4 + (long)c->num_cu - 1) / c->num_cu, r16 = ((nrows + 15) / 16 + (long)c->num_cu - 1) / c->num_cu;
+        const double one = planes ? 3.25 + ntok * (0.04 + 0.17e-3 * k + 0.062e-6 * nrows * k) : 2 + ntok * (0.1 + 0.13e-3 * k * r4);
+        const double two = 3.85 + (planes ? 0.61e-3 : 0.95e-3) * k * r16;
+        if (ntok < 3 || one < std::max(6.7, two)) return false;
     }
-    if (ntok < least) return false;
     if (c->tune.mx_few > 0) return ntok <= c->tune.mx_few;
     if (ntok <= 64) return true;
     const int tiles = (ntok + 15) / 16, chunks = (tiles + 3) / 4, nt = (tiles + chunks - 1) / chunks;
