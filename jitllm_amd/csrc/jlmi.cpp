@@ -966,14 +966,15 @@ struct FewShape { int nt, rt, nw; };
 // Token tiles: what the (average) group fills.  Two rules for the other two.
 //
 // One group: the least of an estimate, in units of a wavefront's step of 256 alone on its SIMD.  Workgroups of eight or
-// four wavefronts run in rounds of `cap` a CU (registers and LDS), the last with what is left; a round takes `e` (its
+// four wavefronts run in rounds of `cap` a CU (registers of the fullest SIMD, and LDS), the last with what is left; a round takes `e` (its
 // start, the reduction) and ceil(K / 256 / wavefronts) steps, a step a serial chain (longer with more row tiles) and a
 // part of each wavefront the SIMD holds.  Fitted to 34 shapes (1024 x 1024 to 14336 x 4096) of every type, window and
-// layout at 8, 24, 40 and 64 tokens over everything that is built: the pick is 1 to 4 % behind the best on average.
+// layout at 8, 24, 40 and 64 tokens over everything that is built: the pick is 1 to 3 % behind the best on average.
 // Against always eight wavefronts, and row tiles where most CUs kept a workgroup, geometric means over them: 8 and 24
-// tokens 1 to 4 % faster, 64 tokens 7 to 10 %, the worst loss 11 % and the largest gain 66 %: a workgroup over a round's
-// end costs a whole round (rows of 9216 x 1280, window 32, 64 tokens: Q6_K 25.9 against 15.6).  (Three, five and six wavefronts are the best of some shapes and, estimated so, the worst of others: 5120 x
-// 5120 Q6_K, 64 tokens, five 38.6, eight 25.7.)  Three token tiles: 33 to 48 tokens took four (40 tokens 22 % faster, never slower).
+// tokens 2 to 4 % faster, 64 tokens 9 %, the worst loss 11 % and the largest gain 66 %: a workgroup over a round's end
+// costs a whole round (rows of 9216 x 1280, window 32, 64 tokens: Q6_K 25.7 against 15.5).  (Three, five and six
+// wavefronts are the best of some shapes and, estimated so, the worst of others: 5120 x 5120 Q6_K, 64 tokens, five 38.6,
+// eight 25.7.)  Three token tiles: 33 to 48 tokens took four (40 tokens 24 % faster, never slower).
 //
 // Groups of a mixture (grid: rows, banks, experts; most groups part empty): row tiles as many as leave most CUs a
 // workgroup, eight wavefronts.  More rows a workgroup share the activations' loads, and over planes widen the weights'
@@ -992,10 +993,8 @@ FewShape few_shape(const jl_ctx* c, int type, bool w256, bool planes, int nrows,
             f.rt = 2;
         if (planes && f.nt <= 2 && (f.nt == 2 || type != JL_TYPE_Q6_K) && (nrows + 63) / 64 * sheets * 10 >= cus * 7) f.rt = 4;
     } else {
-        // (One token tile: steps are short and mostly the weights' way, which over rows leads through LDS and over planes
-        // gets wider loads with more row tiles.)
-        const bool one = f.nt == 1;
-        const double e = one ? 0.5 : 3, more = !one ? 1.6 : planes ? 1.2 : 1.8, longer = one ? 2 : 1.5;
+        // (over planes more row tiles get wider loads of the weights, which is most of a step with one token tile)
+        const double e = planes && f.nt <= 2 ? 0.5 : 3, more = !planes ? 1.6 : f.nt == 1 ? 1.2 : 1.4;
         double best = 1e30;
         for (int w : {8, 4}) {
             const int nw = std::min(w, nsb);
@@ -1005,13 +1004,13 @@ FewShape few_shape(const jl_ctx* c, int type, bool w256, bool planes, int nrows,
                 if (!simd || nrows < rt) break;
                 const size_t lds = std::max(nw * JL_FEW_WAVE_BYTES(type, planes, rt), JL_FEW_RED_BYTES(nw, f.nt, rt));
                 if (lds > c->lds_limit) break;
-                const long cap = std::max<long>(1, std::min<long>(4 * simd / nw, (long)(c->lds_limit / lds)));
+                const long cap = std::max<long>(1, std::min<long>(simd / ((nw + 3) / 4), (long)(c->lds_limit / lds)));
                 const long wgs = (nrows + 16 * rt - 1) / (16 * rt) * sheets, full = wgs / (cap * cus), left = (wgs - full * cap * cus + cus - 1) / cus;
                 const int steps = (nsb + nw - 1) / nw;
                 double t = full * (e + steps * (chain + part * cap));
                 if (left) t += e + steps * (chain + part * left);
                 if (t < best) { best = t; f.rt = rt; f.nw = nw; }
-                part *= more; chain *= longer;
+                part *= more; chain *= 2;
             }
         }
     }
