@@ -5,20 +5,22 @@
 // that.  v_mfma_i32_16x16x32_i8 takes a quantized weight as it is -- no conversion to f16, no scale
 // multiplied in -- so what is left for the vector unit is the unpacking of nibbles (none for Q8_0)
 // and, for every 16 rows x 16 tokens x 32 of K, the conversion of four int32 sums and their two
-// scales: 12 to 20 instructions against 420 to 544 bytes of weights, under the memory time up to
-// about 64 tokens.  The 128-token tiles (gemm_q6k.h, gemm_w32.h) spend the same on 12 tokens as on
-// 128 and add K slices in a second launch.
+// scales: 18 to 23 vector instructions a matrix instruction.  A 128-token tile (gemm_i8.h) spends
+// the same on 12 tokens as on 128 and adds K slices in a second launch.  Counters at 16 tokens (14336 x 4096,
+// Q6_K 4096 x 14336 at 12; kernel alone, traced): Q4_K rows 12.8 us and planes 11.6, Q6_K rows 15.6, Q8_0
+// rows 14.9; the vector unit issues 21 to 33 % of the time, the matrix cores 4 to 7 %, wavefronts wait for
+// data 38 to 49 %, L1 answers 8.6 to 14.8 of 42 to 51 thousand cycles.  What is left is the serial chain of a
+// wavefront's few steps (a super-block's weights, through LDS, matrix instruction, scales) behind the prep's launch.
 //
 //   * A workgroup owns 16 RT rows and up to 16 NT columns; its wavefronts split K (wavefront w takes
 //     super-blocks w, w + nwaves, ...: a row's bytes are asked for side by side) and their partial tiles
 //     are added through LDS in wavefront order: one launch after the prep.
-//   * The next bound after memory is the CU's L1: a vector load costs it one access for every 64-byte
-//     line that a quad of ADJACENT lanes touches, so the matrix operand's own lane order (lane % 16 = row)
-//     costs 64 accesses a 1 KiB load where 16 would do (Q4_K rows 14336 x 4096, 16 tokens: 192 accesses a
-//     chunk of 128 x 16 rows, L1 busy for 60 % of 14 us; Q8_0 446, 43 of 69 thousand clocks).  GGUF rows are
-//     therefore loaded along the row, 16 bytes a lane, and change lanes through the wavefront's own corner
-//     of LDS; over planes a lane loads one word of RT consecutive rows (so row tile j of a workgroup is rows
-//     RT r + j), and the four header words of a Q4_K super-block are one load by the four lane groups.
+//   * L1 would be the next bound after memory: a vector load costs it one access for every 64-byte line that a
+//     quad of ADJACENT lanes touches, so the matrix operand's own lane order (lane % 16 = row) would cost 64
+//     accesses a 1 KiB load where 16 do.  GGUF rows are therefore loaded along the row, 16 bytes a lane, and
+//     change lanes through the wavefront's own corner of LDS; over planes a lane loads one word of RT
+//     consecutive rows (so row tile j of a workgroup is rows RT r + j), and the four header words of a Q4_K
+//     super-block are one load by the four lane groups.
 //   * Lane (r = lane % 16, g = lane / 16) holds, for a block of 32, eight values of row r, in an order of
 //     the weights' own (jl_few_order), and the prep lays the int8 activations out to match: four blocks'
 //     values in two 16-byte loads, their scales in one.

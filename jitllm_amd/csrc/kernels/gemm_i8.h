@@ -11,12 +11,15 @@
 // as two int8 operands, 128 * hi + lo, whose sums are put together as integers.
 //
 // What bounds it.  Window 32: both scales change every 32 of K, so an output element costs three vector
-// instructions a block (convert, times d_a, multiply-add with d) and the matrix cores wait for the vector unit.
-// As f16 operands (which this replaces) it was two, and slower all the same: a loop of two f16 matrix instructions
-// and 32 vector instructions takes what one int8 and 48 take (180 against 174 ns a SIMD, three wavefronts; the
-// chip holds 1.9 GHz under the first and 2.2 under the second), and f16 operands cost twice the LDS and L1 bytes and
-// the conversion of every weight.  Window 256: the matrix cores, two instructions a block, and the making
-// of Q6_K's two operands, which every workgroup of 128 tokens does anew.
+// instructions a block (convert, times d_a, multiply-add with d) and the matrix cores wait for the vector unit: Q8_0,
+// 2048 tokens x 4096 -> 14336, 53 vector instructions a matrix instruction, the vector unit issuing all of the time, the
+// matrix cores 16 % (and L1, mostly the weights' narrow loads, 0.70 of 0.72 million cycles a CU); Q6_K, two operands and
+// two matrix instructions a block, 41 each, 86 % and 16 %.  As f16 operands (which this replaces: 460 us, now 384) it was
+// two an element beside two matrix instructions, and twice the LDS and L1 bytes and the conversion of every weight: in
+// registers alone that loop is the shorter (two f16 matrix instructions and 32 vector instructions 189 ns a SIMD with
+// three wavefronts, one int8 and 48 215, nothing of it hidden), as a kernel not.  Window 256 (551 us as f16 operands,
+// 14336 -> 4096, now 400): 12 vector instructions a matrix instruction, most of them the making of Q6_K's two operands,
+// which every workgroup of 128 tokens does anew; vector unit 43 %, matrix cores 27 %, L1 0.66 of 0.85 million cycles.
 //
 // A workgroup of four wavefronts owns 32 TW tokens x 32 RT (4 / TW) rows, a wavefront 32 tokens x 32 RT rows.  A stage is
 // 128 of K: the 256 threads turn the rows' bytes into operands in LDS (thread = row, block of 32), one stage ahead of
