@@ -334,9 +334,10 @@ int jl_matvec_packed_group(jl_ctx *ctx, int n, float *const *outs, const int *ty
 
 /* JIT.MatMulPacked / MatMul semantics on resident operands (engine/nn/packedmm.go:23,
  * matmul.go:27): x [ntok][k] f32 -> out [ntok][nrows], every token quantized on
- * its own.  Q4_K with the 256 window runs the matrix-core GEMM (quantize-and-
- * lay-out kernel, then the GEMM kernel, in a workspace the context owns); other
- * cases run one fused matvec launch per token, which the reference also falls
+ * its own.  From two (Q8_0) or three tokens a quantize-and-lay-out kernel and a matrix-core
+ * kernel, in a workspace the context owns: up to 64 tokens the int8 few-token kernel, any
+ * window; more on f16 tiles (Q4_K, window 256) or int8 tiles (window 32; Q6_K also 256).
+ * Other cases run one fused matvec launch per token, which the reference also falls
  * back to (engine/model/prefill.go:1036-1041).  The workspace grows on demand
  * (a device allocation); jl_reserve sizes it ahead of time. */
 int jl_matmul_dev(jl_ctx *ctx, float *out, int type, const void *w, const float *x,
@@ -375,9 +376,9 @@ int jl_reserve(jl_ctx *ctx, int max_tok, int max_k);
  * jl_layer_ffn_dev runs block li for n rows: h [n][n_embd] in, resid [n][n_embd] updated, both in
  * device memory (they may be one buffer, as they are for a block with its norm in front: every
  * launch that reads a row of h has been enqueued before the one that adds to it).  One row runs the
- * decode kernels (two launches for a dense block), more rows the grouped kernels of the mixture
- * block (a dense block is a mixture of one expert that every row selects with weight 1; with
- * norm_w set its rows run one at a time).  The values are those of the pointer-form entry points
+ * decode kernels (two launches for a dense block); more rows of a dense block two few-token
+ * matmuls (up to 64 rows) or three prefill GEMMs (with norm_w set its rows run one at a time), of
+ * a mixture its grouped kernels.  The values are those of the pointer-form entry points
  * on the same operands, bit for bit.  Workspaces are the context's (calls on one context are
  * serialized by the caller).
  *
@@ -473,10 +474,11 @@ int jl_matvec_packed_q8_dev(jl_ctx *ctx, float *out, int type, const uint32_t *q
                             const int8_t *q, const float *as, const float *sum16, int nrows,
                             int k, void *stream);
 
-/* JIT.MatMulPacked on resident planes (engine/nn/packedmm.go:23-139).  Q4_K with the
- * 256 window and enough tokens restores the row range to GGUF order in a workspace the
- * context owns and runs the matrix-core GEMM on it; other cases run one packed matvec
- * launch per token. */
+/* JIT.MatMulPacked on resident planes (engine/nn/packedmm.go:23-139).  From two (Q8_0) or
+ * three tokens up to 64 the int8 few-token kernel reads the planes where they lie, and so do
+ * the Q4_K tiles of the 256 window; the int8 tiles, and the Q4_K form for grids of a round of 32-row
+ * workgroups, take the row range restored to GGUF order in a workspace the context owns.
+ * Other cases run one packed matvec launch per token. */
 int jl_matmul_packed_dev(jl_ctx *ctx, float *out, int type, const uint32_t *qs, const uint32_t *d,
                          const uint32_t *sc, int row, int stride, const float *x, int nrows,
                          int k, int ntok, void *stream);
@@ -492,12 +494,10 @@ int jl_matmul_mxfp4_bf16_dev(jl_ctx *ctx, float *out, const void *w, const uint1
 
 /* The same over packed MXFP4 planes (jit/gpu/kernels/pack.go:543-575: QS the code bytes
  * four words a block, D the exponent minus one four rows a word; sizes from
- * jl_packed_words, no SC plane): rows row .. row+nrows of planes of `stride` rows.  Up to
- * 8 tokens read the planes where they lie, a lane a row; so do more tokens when tiles of
- * 64 tokens x 64 rows give at least half the CUs a workgroup (a plane word is a lane's
- * eight K values of the matrix instruction's weight operand); the shapes between restore
- * the row range to GGUF blocks in a workspace the context owns and run the few-token and
- * tiled forms on it.  The value of a block is that of the GGUF block it was packed from. */
+ * jl_packed_words, no SC plane): rows row .. row+nrows of planes of `stride` rows.  Every
+ * number of tokens reads the planes where they lie: a handful a lane a row, up to 64 (and more
+ * on a grid of one round) the few-token form, beyond tiles of 64 tokens x 64 or 96 rows (a
+ * plane word is a lane's eight K values of the matrix instruction's weight operand).  The value of a block is that of the GGUF block it was packed from. */
 int jl_matmul_mxfp4_packed_bf16_dev(jl_ctx *ctx, float *out, const uint32_t *qs, const uint32_t *d,
                                     int row, int stride, const uint16_t *x, int nrows, int k,
                                     int ntok, void *stream);
@@ -582,8 +582,7 @@ int jl_moe_grouped(jl_ctx *ctx, float *resid, int type, const void *gate_bank, c
                    const void *down_bank, const float *x, const uint32_t *sel, int sel_stride,
                    const float *wt, int rows, int k_used, int n_expert, int n_ffn, int n_embd);
 
-/* jl_moe_matvec_dev over banks of packed planes: the per-expert matrix-core tile reads every
- * sheet where it lies (Q4_K with the activation window of 256; anything else JL_DECLINED).
+/* jl_moe_matvec_dev over banks of packed planes, every sheet read where it lies (Q4_K with the activation window of 256; anything else JL_DECLINED).
  * bank1 / out1 may be null; both banks must share one layout (sheet_bytes, stride). */
 int jl_moe_matvec_packed_dev(jl_ctx *ctx, float *out0, float *out1, int type,
                              const jl_packed_bank *bank0, const jl_packed_bank *bank1, const float *x,
