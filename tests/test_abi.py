@@ -36,7 +36,7 @@ def test_context_creation_fails_loudly_without_a_gpu():
     ctx = C.c_void_p()
     opts = _lib.Options(0, 32, b"/nonexistent/code_object.hsaco")
     rc = lib.jl_ctx_create(C.byref(ctx), C.byref(opts))
-    assert rc < 0 and not ctx.value           # no device here, or no such code object on a GPU box
+    assert rc < 0 and not ctx.value           # no device here, or no such code object on a machine with one
     assert lib.jl_last_error(None)
 
 
