@@ -2221,7 +2221,7 @@ int jl_reserve(jl_ctx* c, int max_tok, int max_k) {
     int rc = gemm_ws_ensure(c, std::max(gemm_ws_need(max_tok, max_k), w32));
     if (rc == JL_OK) rc = ws_ensure(c, &c->mx_ws, &c->mx_ws_bytes, slab_reserve(c));
     if (rc != JL_OK) return rc;
-    c->reserved.push_back({max_tok, max_k});
+    if (!reserved_for(c, max_tok, max_k)) c->reserved.push_back({max_tok, max_k});
     return JL_OK;
 }
 
