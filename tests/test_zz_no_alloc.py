@@ -97,6 +97,26 @@ def test_static_matmul_on_a_stream_of_the_callers(dev, devbuf):
     dev.SetActWindow(32)
 
 
+@pytest.mark.parametrize("t,window,nrows,k,ntok", [(quant.Q8_0, 32, 1184, 9472, 1960), (quant.Q6_K, 256, 1248, 7168, 1568),
+                                                   (quant.Q4_K, 32, 1648, 7168, 1296)])
+def test_static_matmul_where_the_fastest_slices_would_not_fit(dev, devbuf, t, window, nrows, k, ntok):
+    """Seven K slices (Q8_0 five) would be the fastest and do not fit the array behind the activations: as many as
+    fit are taken, and the call that may allocate takes the same ones (equal bits)."""
+    dev.SetActWindow(window)
+    w = synth.random_weights(t, nrows, k, seed=8)
+    x = np.tile(np.stack([synth.activations(k, seed=i) for i in range(8)]), (ntok // 8, 1))
+    wd, xd = devbuf(w), devbuf(x)
+    want, got = devbuf(shape=(ntok * nrows,), dtype=np.float32, fill=POISON), devbuf(shape=(ntok * nrows + 64,), dtype=np.float32, fill=POISON)
+    assert dev.matmul_dev(want.ptr, t, wd.ptr, xd.ptr, nrows, k, ntok)
+    assert dev.matmul_static_dev(got.ptr, t, wd.ptr, xd.ptr, nrows, k, ntok)
+    dev.synchronize()
+    a, b = want.get(), got.get()
+    assert np.array_equal(a, b[:ntok * nrows]) and np.all(b[ntok * nrows:] == np.float32(POISON)) and np.all(np.abs(a) < 1e30)
+    for buf in (wd, xd, want, got):
+        buf.free()
+    dev.SetActWindow(32)
+
+
 def test_static_matmul_refuses_what_does_not_fit(dev, devbuf):
     """A shape whose activation fragments alone exceed the array: a clear error, and the
     output untouched."""
