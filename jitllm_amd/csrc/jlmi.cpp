@@ -607,7 +607,7 @@ int ws_ensure(jl_ctx* c, void** buf, size_t* have, size_t need);
 int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1,
                       const float* x, const float* x2, const uint32_t* src, const uint32_t* start,
                       int n_expert, int ncols, int nrows, int k, hipStream_t st,
-                      const jl_packed_bank* pb0 = nullptr, const jl_packed_bank* pb1 = nullptr);
+                      const jl_packed_bank* pb0 = nullptr, const jl_packed_bank* pb1 = nullptr, int nsrc = 0);
 
 // plane banks of a mixture: from this many columns an expert (on average) the matrix-core tile
 // per expert takes over from the dot-product form ("moe.form" = 1 / 4 forces one)
@@ -1362,28 +1362,23 @@ int moe_g16_blocks(const jl_ctx* c, int nrows, int n_expert, int ncols, int nmat
     return best;
 }
 
-// Q4_K GGUF banks with the k-quant window, 9 to 40 columns an expert on average: whether the int8 few-token kernel takes
-// less time than groups of 32 columns, by what each has to do (us; fitted to 276 launches, 8 to 128 experts of 512 x 512
-// to 2816 x 2048, one and two matrices, to 10 % each).  The few-token kernel: a prep of the columns and the bank's elements
-// by the token tiles of a pass, once more for the experts that overflow it.  Groups of 32: rounds of workgroups, an XCD's
-// experts on its own CUs, each a fill of LDS and its tiles, again for the experts of more than 32 (one of them can be
-// the launch's length).  Chosen so, a launch takes 1.1 % more than the better of the two on average, at most 23;
-// never the few-token kernel: 18 on average; up to 120e6 elements of the bank: 5.7, at most 80 (28 x 1792 x 1280,
-// 38 columns 60.6 us against 36.1; 40 x 768 x 1536 twice, 20 columns 43 against 26).
-bool moe_q4k_few(const jl_ctx* c, int n_expert, int ncols, int nmat, int nrows, int k) {
-    const double avg = (double)ncols / n_expert, nsb = k / 256;
-    if (avg < 9 || avg > 40) return false;
+// Banks with the k-quant window, more than eight columns an expert on average: whether the int8 few-token kernel takes less
+// time than the columns against decoded rows (kernels/moe_cols.h), us by what each has to do (millions of the banks'
+// elements, a pass of the columns a time; super-blocks of a row, the chain of a small grid), fitted to 38 (Q4_K) and 19
+// (Q6_K) shapes, 8 to 128 experts of 512 x 1024 to 2816 x 1024 at 3 to 64 columns.  Chosen so, a launch takes 0.5 % (Q4_K)
+// and 1.3 % (Q6_K) more than the best of every form on average from twelve columns on, at most 24 (8 x 512 x 1024, 32
+// columns 13.3 us against 10.7) and 46 %; always the columns 1.9 %, always the few-token kernel 49, groups of 32 41 %.
+bool moe_few_faster(int type, int n_expert, int ncols, int nmat, int nrows, int k) {
+    const double avg = (double)ncols / n_expert, nsb = k / 256, melem = 1e-6 * n_expert * nmat * (double)nrows * k;
     const auto over = [&](int n) { return 0.5 * std::erfc((n + 0.5 - avg) / std::sqrt(2 * avg)); };   // an expert's columns pass n
-    const int tiles = (nrows + 15) / 16;
-    const long cut = moe_g16_blocks(c, nrows, n_expert, ncols, nmat, 8), tiles_wg = (tiles + cut - 1) / cut;
-    const long blocks = (tiles + tiles_wg - 1) / tiles_wg, cus_xcd = std::max(1, c->num_cu / 8);
-    const long rounds = (blocks * nmat * ((n_expert + 7) / 8) + cus_xcd - 1) / cus_xcd;
-    const double p = over(32), again = 0.4 * (1 - std::pow(1 - p, n_expert)) + 0.6 * p;
-    const double groups = rounds * (1 + again) * (0.96 * nsb + tiles_wg / 8.0 * (0.71 * nsb + 1.6));
     const int nt = avg <= 16 ? 1 : avg <= 32 ? 2 : 4;
-    const double few = 0.5 + 0.95e-6 * ncols * k +   // (what its prep takes longer)
-                       1e-6 * n_expert * nmat * (double)nrows * k * (1 + over(16 * nt)) * (nt == 1 ? 0.157 : nt == 2 ? 0.241 : 0.495);
-    return few < groups;
+    const double passes = melem * (1 + over(16 * nt));
+    if (type == JL_TYPE_Q4_K) {
+        if (avg >= 32) return false;
+        const double few = 5.3 + 1.15 * (0.5 + 0.95e-6 * ncols * k + passes * (nt == 1 ? 0.157 : 0.241));
+        return few < std::max(7 + 1.1 * nsb, 5.5 + 0.155 * melem) * (1 + 0.3 * over(32));
+    }
+    return 6.0 + passes * (nt == 1 ? 0.267 : nt == 2 ? 0.377 : 0.76) < 8.6 + 0.81 * nsb + melem * (0.247 + 0.113 * over(32) + 0.475 * over(64));
 }
 
 // What a grouped matmul asks of its one or two banks of n_expert sheets of nrows x k, whichever kernel serves them
@@ -1419,12 +1414,61 @@ int moe_banks_check(jl_ctx* c, int type, bool planes, const void* bank0, const v
     return (type == JL_TYPE_Q4_K ? sheet % 16 : sheet % 2) != 0 ? JL_DECLINED : JL_OK;
 }
 
+// The columns of an expert against rows decoded in registers (kernels/moe_cols.h): the source rows quantized once each
+// (nsrc of them, src naming each column's; nsrc = 0: not known, a record a column), then the matrices.
+int moe_cols_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1, const jl_packed_bank* pb0,
+                    const jl_packed_bank* pb1, const float* x, const float* x2, const uint32_t* src, const uint32_t* start, int n_expert,
+                    int ncols, int nrows, int k, int nsrc, hipStream_t st) {
+    const TypeInfo* ti = type_info(type);
+    const bool q6 = type == JL_TYPE_Q6_K, planes = pb0 != nullptr, mapped = src && nsrc > 0 && nsrc <= ncols;
+    const size_t nsb = (size_t)k / 256, nrec = mapped ? nsrc : ncols, rec = q6 ? 256 : 512;
+    const int nmat = (planes ? pb1 != nullptr : bank1 != nullptr) ? 2 : 1;
+    const unsigned lds = q6       ? 2u * 64u * 256u + 128u * (208u + 16u + 2u) + 64u * 4u   // JL_MC_Q6_LDS
+                         : planes ? 2u * 64u * (512u + 32u + 4u)                          // JL_MC_PLANES_LDS
+                                  : 2u * (64u * 256u + 128u * 144u + 64u * 36u);          // JL_MC_Q4_LDS
+    // (32-bit offsets in the kernels: records, and half a super-block's words of every row of the planes)
+    if (nrec * nsb * rec >= ((size_t)1 << 32) || (planes && (size_t)pb0->stride >= ((size_t)1 << 25)) || lds > c->lds_limit) return JL_DECLINED;
+    const double avg = (double)ncols / n_expert;
+    const long rblocks = (nrows + 127) / 128, shares = avg <= 48 ? 1 : (long)(avg * 1.2 / 64) + 1, items = rblocks * shares * nmat * n_expert;
+    if (items >= (1L << 30)) return JL_DECLINED;
+    const size_t o_aug = nrec * nsb * rec, o_da = o_aug + (q6 ? 0 : nrec * nsb * 32);
+    int rc = ws_ensure(c, &c->moe_q_ws, &c->moe_q_ws_bytes, o_da + nrec * nsb * 4);
+    if (rc != JL_OK) return rc;
+    char* ws = (char*)c->moe_q_ws;
+    const char* tag = q6 ? "q6k" : planes ? "q4k_planes" : "q4k";
+    MoeColsPrepArgs pa;
+    pa.x = x; pa.x2 = x2; pa.src = mapped ? nullptr : src; pa.rec = (uint32_t*)ws; pa.aug = (uint32_t*)(ws + o_aug); pa.da = (float*)(ws + o_da);
+    pa.k = k; pa.nrec = (int)nrec;
+    void* pp[] = {&pa};
+    Name name;
+    name << "jl_moe_cols_prep_" << tag;
+    rc = launch(c, name, (unsigned)((nrec * nsb + 15) / 16), 1, 256, 0, st, pp);
+    if (rc != JL_OK) return rc;
+    MoeColsArgs ga;
+    ga.out[0] = out0; ga.out[1] = out1;
+    ga.bank[0] = (const uint8_t*)bank0; ga.bank[1] = (const uint8_t*)bank1;
+    if (planes) {
+        const jl_packed_bank* pbs[2] = {pb0, pb1};
+        for (int m = 0; m < nmat; m++) { ga.pqs[m] = pbs[m]->qs; ga.pd[m] = pbs[m]->d; ga.psc[m] = pbs[m]->sc; }
+        ga.sheet_words = pb0->sheet_bytes / 4;
+        ga.row_step = pb0->sheet_bytes ? 0 : nrows;
+        ga.pstride = pb0->stride;
+    }
+    ga.rec = (const uint8_t*)ws; ga.aug = (const uint8_t*)ws + o_aug; ga.da = pa.da; ga.map = mapped ? src : nullptr; ga.start = start;
+    ga.nrows = nrows; ga.k = k; ga.row_bytes = (k / ti->block_elems) * ti->block_bytes; ga.sheet_bytes = (size_t)nrows * ga.row_bytes;
+    ga.nmat = nmat; ga.rblocks = (int)rblocks; ga.shares = (int)shares; ga.items = (int)items;
+    void* gp[] = {&ga};
+    Name gname;
+    gname << "jl_moe_cols_" << tag;
+    return launch(c, gname, (unsigned)((items + 7) / 8 * 8), 1, 256, lds, st, gp);
+}
+
 // pb0 / pb1: the banks as packed planes (bank0 / bank1 unused then): the per-expert kernels
 // read an expert's sheet where it lies in the bank's pages.
 int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1,
                       const float* x, const float* x2, const uint32_t* src, const uint32_t* start,
                       int n_expert, int ncols, int nrows, int k, hipStream_t st, const jl_packed_bank* pb0,
-                      const jl_packed_bank* pb1) {
+                      const jl_packed_bank* pb1, int nsrc) {
     const TypeInfo* ti = nullptr;
     int rc = matvec_check(c, type, nrows, k, &ti);
     if (rc != JL_OK) return rc;
@@ -1454,13 +1498,22 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
         int form = c->tune.moe_form;
         if (q6 && !planes && c->act_window == 256 && (form == 3 || form == 4)) form += 2;   // (their Q6_K forms)
         if (form == 0 && (c->act_window == 32 || c->act_window == 256) && !planes) {
-            if (q4w) form = moe_q4k_few(c, n_expert, ncols, nmat, nrows, k) ? 5 : 0;
+            if (q4w) form = ncols <= 8L * n_expert ? 0 : moe_few_faster(type, n_expert, ncols, nmat, nrows, k) ? 5 : 9;
+            else if (q6 && c->act_window == 256 && avg > 8 && avg < 60) form = moe_few_faster(type, n_expert, ncols, nmat, nrows, k) ? 5 : 9;
             else if (q6 && avg < (c->act_window == 32 ? 3 : 2) && k < 2048) form = 0;
             else if (avg < (q6 && c->act_window == 256 ? 28 : 40)) form = 5;
             else if (avg < (q6 && c->act_window == 32 ? 64 : 56)) form = tiles64 >= 2 * c->num_cu ? 7 : 5;
             else form = type == JL_TYPE_Q8_0 && avg >= 64 && tiles64 >= 2 * c->num_cu ? 8 : 6;
         }
+        // Planes (gate + up + down of 128 x 768 x 2048 and 32 x 1024 x 2048, the block's us, the forms below against columns):
+        // 12 columns 149 / 74 against 159 / 70, 16 157 / 75 against 167 / 72, 25 248 / 92 against 194 / 80, 48 363 / 135
+        // against 275 / 105, 64 384 / 151 against 380 / 138, 128 (the second) 219 against 208.
+        if (form == 0 && q4w && planes && ncols >= 16L * n_expert) form = 9;
         if (form == 5 && !align && c->tune.moe_form == 0 && avg >= 6) form = 6;
+        if (form == 9 && c->act_window == 256 && (type == JL_TYPE_Q4_K || (q6 && !planes))) {
+            rc = moe_cols_launch(c, out0, out1, type, bank0, bank1, pb0, pb1, x, x2, src, start, n_expert, ncols, nrows, k, nsrc, st);
+            if (rc != JL_DECLINED) return rc;
+        }
         if (form >= 6 && !planes && gemm_i8_applies(c, type, nrows, k, ncols)) {
             rc = moe_gemm_i8_launch(c, out0, out1, type, bank0, bank1, x, x2, src, start, n_expert, ncols, nrows, k,
                                     form == 7 ? I8Shape{2, 2} : form == 8 && type == JL_TYPE_Q8_0 ? I8Shape{4, 4} : I8Shape{2, 4}, st);
@@ -1491,8 +1544,9 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     //   16 rows 73 / 155 / 85 / - / -       64 rows 133 / 210 / 110 / - / -     128 rows 191 / 223 / 130 / 137 / 302
     //   192 rows - / 232 / 171 / 147 / 309  256 rows 333 / 238 / 187 / 157 / 315  512 rows - / 301 / 281 / 243 / 352
     //   1024 rows - / 426 / 489 / 372 / 400 1280 rows - / 501 / 577 / 475 / 435   2048 rows - / 709 / 831 / 639 / 623
-    // so form 3 takes over from two columns an expert on average (groups of 32 from ten) and form 4
-    // from 72; form 2 is left to "moe.form" = 2.
+    // so form 3 takes over from two columns an expert on average.  Above eight the columns against decoded rows
+    // ("moe.form" = 9, above) have replaced groups of 32 and form 4 over GGUF rows (777 rows: 339 -> 234 us), and over planes
+    // from sixteen; form 4 is left to what they decline, form 2 to "moe.form" = 2.
     // Form 3: groups of sixteen columns on the 16 x 16 x 32 matrix instruction, the weights decoded
     // in registers straight into its operand (Q4_K GGUF sheets or packed planes, the k-quant window; the group's
     // fragments for the whole of K sit in LDS).  Its steady state runs at the rate of a plain read;
@@ -1773,6 +1827,8 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     names.push_back("jl_few_prep");
     names.push_back("jl_gemm_i8_prep");
     names.push_back("jl_moe_gemm_i8_prep");
+    for (const char* tag : {"q4k", "q4k_planes", "q6k"})
+        for (const char* form : {"jl_moe_cols_", "jl_moe_cols_prep_"}) names.push_back(std::string(form) + tag);
     for (const char* tag : {"q8_0", "q4k", "q6k", "q6kw"})
         for (const char* form : {"jl_gemm_i8_%s_r2t4", "jl_moe_gemm_i8_%s_r2t4", "jl_moe_gemm_i8_%s_r2t2"}) {
             char nm[64];
@@ -2478,7 +2534,7 @@ int moe_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate_b
     if (rc != JL_OK) return rc;
     // gate and up: columns read the routed rows of x
     rc = moe_matvec_launch(c, g, u, type, gate_bank, up_bank, x, nullptr, perm, start, n_expert, (int)ncols, n_ffn, n_embd, st,
-                           pg, pu);
+                           pg, pu, rows);
     if (rc != JL_OK) return rc;
     // down: the activation of column c is silu(g[c]) * u[c]
     rc = moe_matvec_launch(c, y, nullptr, down_type, down_bank, nullptr, g, u, nullptr, start, n_expert, (int)ncols, n_embd, n_ffn, st,

@@ -168,6 +168,32 @@ struct MoeGemmArgs {
     const float* dsum = nullptr;   // the int8 form, Q4_K: d_a * block sums
 };
 
+// Grouped expert matmul for experts of some tens of columns (kernels/moe_cols.h): rec [record][k/256][512 or 256 bytes],
+// aug [record][k/256][32 bytes], da [record][k/256].
+struct MoeColsPrepArgs {
+    const float* x;
+    const float* x2;        // null: plain activation, else silu(x) * x2
+    const uint32_t* src;    // null: record r is row r of x
+    uint32_t* rec;
+    uint32_t* aug;
+    float* da;
+    int k, nrec;
+};
+struct MoeColsArgs {
+    float* out[2];
+    const uint8_t* bank[2];
+    const uint32_t* pqs[2] = {nullptr, nullptr};   // packed planes, as in MoeG16Args
+    const uint32_t* pd[2] = {nullptr, nullptr};
+    const uint32_t* psc[2] = {nullptr, nullptr};
+    const uint8_t* rec;
+    const uint8_t* aug;
+    const float* da;
+    const uint32_t* map;    // column -> record (null: its own)
+    const uint32_t* start;
+    size_t sheet_bytes, sheet_words = 0;
+    int nrows, k, row_bytes, nmat, rblocks, shares, items, row_step = 0, pstride = 0;
+};
+
 // Grouped expert matmul, sixteen columns a group (moe_g16_body).  Column group g of expert e is
 // slot (start[e] >> 4) + e + g of the prepared workspace; a slot holds, for every super-block,
 // JL_MOE_G16_SB_WORDS words: eight matrix fragments of 64 lanes x 16 bytes (half, K-step), the

@@ -11,6 +11,7 @@
 #include "gemm_q4k_fold.h"
 #include "matvec.h"
 #include "moe.h"
+#include "moe_cols.h"
 #include "mxfp4.h"
 #include "packed.h"
 #include "quantize.h"
@@ -342,6 +343,11 @@ JL_MOE_KERNEL(q6k, JL_Q6_K, 16) JL_MOE_KERNEL(q6k, JL_Q6_K, 32) JL_MOE_KERNEL(q6
 extern "C" __global__ __launch_bounds__(512) void jl_moe_matvec_planes_q4k(MoePlanesArgs p) {
     moe_matvec_planes_body(p, jl_smem);
 }
+// experts of some tens of columns (kernels/moe_cols.h): prep grid = ceil(records * k/256 / 16); matrices: dynamic LDS = JL_MC_LDS_BYTES
+#define JL_MOE_COLS(T, KO)                                                                                                         \
+    extern "C" __global__ __launch_bounds__(256) void jl_moe_cols_prep_##T(MoeColsPrepArgs p) { moe_cols_prep_body<KO>(p); }      \
+    extern "C" __global__ __launch_bounds__(256, 2) void jl_moe_cols_##T(MoeColsArgs p) { moe_cols_body<KO>(p, jl_smem); }
+JL_MOE_COLS(q4k, 0) JL_MOE_COLS(q4k_planes, 1) JL_MOE_COLS(q6k, 2)
 // grid = (ceil(n_embd/256), rows), block = 256
 extern "C" __global__ __launch_bounds__(256) void jl_moe_combine(MoeCombineArgs p) {
     __shared__ float swt[16];

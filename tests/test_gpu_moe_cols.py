@@ -1,0 +1,88 @@
+"""The grouped matmul that decodes its rows in registers (kernels/moe_cols.h) at the edges of its tiles: experts of 0, 1, 31,
+33, 64, 65 and 129 columns, rows of one tile less, exactly and more, one super-block of K, an odd and an even number of
+them; GGUF rows and packed planes, one bank and two, gathered rows, a gated activation; against the oracle in f64."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import nmse
+from jitllm_amd import quant, synth
+
+pytestmark = pytest.mark.gpu
+FILL = np.float32(4e30)
+COUNTS = [1, 0, 31, 33, 64, 65, 129, 0]
+
+
+@pytest.mark.parametrize("t,layout", [(quant.Q4_K, "rows"), (quant.Q4_K, "one"), (quant.Q4_K, "sheets"), (quant.Q6_K, "rows")],
+                         ids=["q4_k", "q4_k-planes", "q4_k-sheets", "q6_k"])
+@pytest.mark.parametrize("nrows,k", [(1, 256), (130, 512), (96, 768), (257, 1024)])
+def test_columns_against_decoded_rows(dev, devbuf, t, layout, nrows, k):
+    from test_gpu_moe import _pack_bank
+    n_expert, ncols = len(COUNTS), sum(COUNTS)
+    start = np.concatenate([[0], np.cumsum(COUNTS)]).astype(np.uint32)
+    dev.SetActWindow(256)
+    sheet = nrows * quant.row_bytes(t, k)
+    banks = [np.concatenate([synth.random_weights(t, nrows, k, seed=10 * b + e) for e in range(n_expert)]) for b in range(2)]
+    x = np.stack([synth.activations(k, seed=300 + r) * np.float32(1 + r % 3) for r in range(40)])
+    u = np.stack([synth.activations(k, seed=500 + r) for r in range(40)])
+    src = (np.arange(ncols) * 7 % 40).astype(np.uint32)
+    xg = (x / (1 + np.exp(-x.astype(np.float64))) * u).astype(np.float32)
+    xd, ud, sd, dstart = devbuf(x), devbuf(u), devbuf(src), devbuf(start)
+    hold = [_pack_bank(dev, devbuf, t, b, n_expert, nrows, k, layout) if layout != "rows" else (devbuf(b), None) for b in banks]
+    try:
+        dev.set_tuning(moe__form=9)
+        for gated in (False, True):
+            act = xg if gated else x
+            o = [devbuf(shape=(ncols * nrows + 8,), dtype=np.float32, fill=FILL) for _ in banks]
+            args = (xd.ptr, ud.ptr if gated else None, sd.ptr, dstart.ptr, n_expert, ncols, nrows, k)
+            if layout == "rows":
+                assert dev.moe_matvec_dev(o[0].ptr, o[1].ptr, t, hold[0][0].ptr, hold[1][0].ptr, *args)
+            else:
+                assert dev.moe_matvec_packed_dev(o[0].ptr, o[1].ptr, t, hold[0][0], hold[1][0], *args)
+            dev.synchronize()
+            for b in range(2):
+                want = np.zeros((ncols, nrows))
+                for e in range(n_expert):
+                    cols = slice(start[e], start[e + 1])
+                    if COUNTS[e]:
+                        want[cols] = oracle.matmul_q8act_f64(t, banks[b][e * sheet:(e + 1) * sheet], act[src[cols]], nrows, k, COUNTS[e], 256)
+                got = o[b].get()
+                assert np.all(got[ncols * nrows:] == FILL)
+                # (the gated activation: an exponential of another machine in front of the quantizer)
+                assert nmse(got[:ncols * nrows].reshape(ncols, nrows), want) <= (1e-6 if gated else 1e-10), (gated, b)
+    finally:
+        dev.set_tuning(moe__form=0)
+        dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("down", [quant.Q4_K, quant.Q6_K], ids=["q4_k", "q6_k"])
+def test_block_with_source_rows_quantized_once(dev, devbuf, down):
+    """The routed block, where a source row's record serves all of its columns: the bits of a record a column."""
+    rows, k_used, n_expert, n_ffn, n_embd = 75, 3, 6, 512, 768
+    rng = np.random.default_rng(5)
+    sel = np.stack([rng.permutation(n_expert)[:k_used] for _ in range(rows)]).astype(np.uint32)
+    perm = np.argsort(sel.reshape(-1), kind="stable")
+    start = np.concatenate([[0], np.cumsum(np.bincount(sel.reshape(-1), minlength=n_expert))]).astype(np.uint32)
+    ncols = rows * k_used
+    dev.SetActWindow(256)
+    bank = lambda t, nrows, k, s: devbuf(np.concatenate([synth.random_weights(t, nrows, k, seed=s + e) for e in range(n_expert)]))
+    gate, up, dn = bank(quant.Q4_K, n_ffn, n_embd, 0), bank(quant.Q4_K, n_ffn, n_embd, 50), bank(down, n_embd, n_ffn, 90)
+    x = np.stack([synth.activations(n_embd, seed=700 + r) for r in range(rows)])
+    wt = np.full((rows, k_used), 1 / k_used, np.float32)
+    xd, sd, wd, start_d = devbuf(x), devbuf(sel), devbuf(wt), devbuf(start)
+    perm_d, pos_d = devbuf((perm // k_used).astype(np.uint32)), devbuf(np.argsort(perm, kind="stable").astype(np.uint32))
+    try:
+        dev.set_tuning(moe__form=9)
+        r = devbuf(np.zeros((rows, n_embd), np.float32))
+        assert dev.moe_ffn_dev(r.ptr, quant.Q4_K, gate.ptr, up.ptr, dn.ptr, xd.ptr, sd.ptr, k_used, wd.ptr, rows, k_used, n_expert, n_ffn,
+                               n_embd, down_type=down)
+        g, u, y = (devbuf(shape=(ncols, n), dtype=np.float32) for n in (n_ffn, n_ffn, n_embd))
+        want = devbuf(np.zeros((rows, n_embd), np.float32))
+        assert dev.moe_matvec_dev(g.ptr, u.ptr, quant.Q4_K, gate.ptr, up.ptr, xd.ptr, None, perm_d.ptr, start_d.ptr, n_expert, ncols, n_ffn, n_embd)
+        assert dev.moe_matvec_dev(y.ptr, None, down, dn.ptr, None, g.ptr, u.ptr, None, start_d.ptr, n_expert, ncols, n_embd, n_ffn)
+        assert dev.moe_combine_dev(want.ptr, y.ptr, wd.ptr, sd.ptr, k_used, pos_d.ptr, rows, k_used, n_embd)
+        dev.synchronize()
+        assert np.array_equal(r.get().view(np.uint32), want.get().view(np.uint32))
+    finally:
+        dev.set_tuning(moe__form=0)
+        dev.SetActWindow(32)
