@@ -321,10 +321,8 @@ extern "C" __global__ __launch_bounds__(1024) void jl_moe_group(MoeGroupArgs p) 
     __shared__ __attribute__((aligned(16))) uint16_t skeys[JL_MOE_GROUP_KEYS];
     moe_group_body(p, scount, skeys);
 }
-// the linear-time form: one workgroup of 1024 threads, dynamic LDS = JL_MOE_GROUP2_LDS(experts)
-extern "C" __global__ __launch_bounds__(1024) void jl_moe_group2(MoeGroupArgs p) { moe_group2_body<uint16_t>(p, jl_smem); }
-// more than 65535 pairs: 32-bit counts, dynamic LDS = 16 * experts * 4 + (experts + 17) * 4
-extern "C" __global__ __launch_bounds__(1024) void jl_moe_group2_wide(MoeGroupArgs p) { moe_group2_body<u32>(p, jl_smem); }
+// the linear-time form: a workgroup of 1024 threads for 1024 pairs, dynamic LDS = JL_MOE_GROUP2_LDS(experts)
+extern "C" __global__ __launch_bounds__(1024) void jl_moe_group2(MoeGroupArgs p) { moe_group2_body(p, jl_smem); }
 // grid = (ceil(k/4/256), ncols), block = 256
 extern "C" __global__ __launch_bounds__(256) void jl_moe_quant(MoeQuantArgs p) { moe_quant_body(p); }
 // grid = (row shares, n_expert, matrices), block = 512, dynamic LDS = 8 staged columns

@@ -240,67 +240,76 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& p, u32* scoun
     }
 }
 
-// The same sort in time linear in the pairs (the form above compares every pair with every
-// expert, all on one CU: 11 us at 512 pairs and 128 experts, 234 us at 16,384 pairs).  The
-// pair list is cut into sixteen contiguous shares, one per wavefront, walked in runs of 64.
-// Inside a run every lane finds the lanes that hold its expert with one ballot per bit of the
-// expert id, which gives its rank among them and their number; the share's running count of
-// the expert (an LDS table the wavefront owns, so its accesses execute in order) gives the
-// pairs before the run.  A thread per expert then turns the sixteen share counts into offsets,
-// the expert totals are scanned, and a pair's column is its expert's first column + the
-// expert's pairs in earlier shares + its rank in its own share: (row, slot) order inside an
-// expert, no atomics.  The rank waits in pos[] between the passes (the same thread writes
-// and reads it).  grid = 1, block = 1024, dynamic LDS = JL_MOE_GROUP2_LDS(nexp).
-#define JL_MOE_GROUP2_LDS(nexp) (16 * (nexp) * 2 + ((nexp) + 1 + 16) * 4)
-// CNT: the type of a share's per-expert counts and of their running sums over the sixteen
-// shares: uint16_t while the whole pair list has at most 65535 pairs (no sum can pass that),
-// u32 above.  Dynamic LDS = 16 * nexp * sizeof(CNT) + (nexp + 17) * 4.
-template <typename CNT>
+// The same sort in time linear in the pairs, a workgroup for every 1024 of them (the form above compares every pair with
+// every expert, all on one CU: 11 us at 512 pairs and 128 experts, 234 us at 16,384 pairs).  A workgroup's pairs are
+// sixteen runs of 64, one a wavefront.  Inside a run every lane finds the lanes that hold its expert with one ballot per
+// bit of the expert id, which gives its rank among them and their number; a thread per expert turns the sixteen runs'
+// counts into offsets.  What the earlier workgroups' pairs hold of an expert, and all pairs together, every workgroup
+// counts for itself (an LDS atomic a pair; no order needed): no workgroup waits for another.  A pair's column is its
+// expert's first column + the expert's pairs in earlier workgroups and runs + its rank in its run: (row, slot) order inside
+// an expert.  One workgroup that walked its sixteen shares run after run took 15.4 us at 6216 pairs, with keys and ranks in
+// registers 12.8 (its ballots alone are 6 us of one CU's issue slots); now 6.6 (512 pairs 4.8 as before).
+// grid = ceil(pairs / 1024), block = 1024, dynamic LDS = JL_MOE_GROUP2_LDS(nexp).
+#define JL_MOE_GROUP2_LDS(nexp) (16 * (nexp) * 2 + (2 * (nexp) + 16) * 4)
 __device__ __forceinline__ void moe_group2_body(const MoeGroupArgs& p, uint8_t* smem) {
-    const int npairs = p.rows * p.k_used, nexp = p.n_expert;
-    const int nruns = (npairs + 63) / 64, runs_per = (nruns + 15) / 16;
-    CNT* scnt = (CNT*)smem;                                            // [16][nexp]
-    u32* sstart = (u32*)(scnt + 16 * nexp);                            // [nexp + 1]
-    u32* stot = sstart + nexp + 1;                                     // [16] wavefront totals
+    const int npairs = p.rows * p.k_used, nexp = p.n_expert, lo = (int)blockIdx.x * 1024;
+    u32* sbefore = (u32*)smem;                // [nexp] pairs of earlier workgroups, then a pair's expert's first column here
+    u32* srest = sbefore + nexp;              // [nexp] the other pairs
+    u32* stot = srest + nexp;                 // [16] wavefront totals
+    uint16_t* scnt = (uint16_t*)(stot + 16);  // [16][nexp]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const bool one = gridDim.x == 1;
     int nbits = 0;
     while ((1 << nbits) < nexp) nbits++;
-    for (int i = tid; i < 16 * nexp; i += 1024) scnt[i] = 0;
+    // i / k_used = i * inv >> 32 for i < 65536 (k_used = 1: inv wraps to 0)
+    const u32 inv = 0xFFFFFFFFu / (u32)p.k_used + 1u;
+    const bool quick = npairs <= 65536 && p.k_used > 1;
+    auto row_of = [&](int i) { return quick ? (int)__umulhi((u32)i, inv) : i / p.k_used; };
+    auto key_of = [&](int i) {
+        const int r = row_of(i);
+        return p.sel[(size_t)r * p.sel_stride + (i - r * p.k_used)];
+    };
+    const int i = lo + tid;
+    u32 e = 0;
+    if (i < npairs) e = key_of(i);
+    for (int j = tid; j < 2 * nexp; j += 1024) sbefore[j] = 0;
+    for (int j = tid; j < 8 * nexp; j += 1024) ((u32*)scnt)[j] = 0;
     __syncthreads();
-    const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;   // lanes below this one
-    CNT* mine = scnt + wave * nexp;
-    const int run_lo = min(wave * runs_per, nruns), run_hi = min(run_lo + runs_per, nruns);
-    auto key_of = [&](int i) { return p.sel[(i / p.k_used) * p.sel_stride + i % p.k_used]; };
-    for (int run = run_lo; run < run_hi; run++) {
-        const int i = run * 64 + lane;
-        u32 e = 0;
-        bool valid = i < npairs;
-        if (valid) {
-            e = key_of(i);
-            valid = e < (u32)nexp;   // an id no expert has: the pair is left out, as in the form above
-        }
-        uint64_t m = __ballot(valid);
-        for (int b = 0; b < nbits; b++) {
-            const bool bit = (e >> b) & 1;
-            const uint64_t bal = __ballot(bit);
-            m &= bit ? bal : ~bal;
-        }
-        if (valid) {
-            const u32 before = mine[e];
-            p.pos[i] = before + (u32)__builtin_popcountll(m & lt);
-            if ((m & lt) == 0) mine[e] = (CNT)(before + (u32)__builtin_popcountll(m));
+    const bool valid = i < npairs && e < (u32)nexp;   // an id no expert has: the pair is left out, as in the form above
+    if (!valid) e = 0;
+    if (!one) {
+        for (int j0 = tid; j0 < npairs; j0 += 8 * 1024) {   // eight keys on their way at a time
+            u32 key[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) key[u] = key_of(min(j0 + 1024 * u, npairs - 1));
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int j = j0 + 1024 * u;
+                if (j < npairs && key[u] < (u32)nexp) atomicAdd(j < lo ? &sbefore[key[u]] : &srest[key[u]], 1u);
+            }
         }
     }
+    const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;   // lanes below this one
+    uint64_t m = __ballot(valid);
+    for (int b = 0; b < nbits; b++) {
+        const bool bit = (e >> b) & 1;
+        const uint64_t bal = __ballot(bit);
+        m &= bit ? bal : ~bal;
+    }
+    const u32 rank = (u32)__builtin_popcountll(m & lt);
+    uint16_t* mine = scnt + wave * nexp;
+    if (valid && rank == 0) mine[e] = (uint16_t)__builtin_popcountll(m);
     __syncthreads();
-    // per expert: counts of successive shares -> pairs in earlier shares; the total goes to the scan
+    // per expert: counts of successive runs -> pairs in earlier runs
     u32 total = 0;
     if (tid < nexp) {
 #pragma unroll
         for (int w = 0; w < 16; w++) {
             const u32 c = scnt[w * nexp + tid];
-            scnt[w * nexp + tid] = (CNT)total;
+            scnt[w * nexp + tid] = (uint16_t)total;
             total += c;
         }
+        if (!one) total = sbefore[tid] + srest[tid];
     }
     // exclusive scan of the totals over experts (thread = expert; nexp <= 1024)
     u32 v = total;
@@ -313,18 +322,16 @@ __device__ __forceinline__ void moe_group2_body(const MoeGroupArgs& p, uint8_t* 
     __syncthreads();
     for (int w = 0; w < wave; w++) v += stot[w];
     if (tid < nexp) {
-        sstart[tid] = v - total;
-        p.start[tid] = v - total;
-        if (tid == nexp - 1) p.start[nexp] = v;
+        sbefore[tid] += v - total;
+        if (blockIdx.x == 0) {
+            p.start[tid] = v - total;
+            if (tid == nexp - 1) p.start[nexp] = v;
+        }
     }
     __syncthreads();
-    for (int run = run_lo; run < run_hi; run++) {
-        const int i = run * 64 + lane;
-        if (i >= npairs) continue;
-        const u32 e = key_of(i);
-        if (e >= (u32)nexp) continue;
-        const u32 col = sstart[e] + mine[e] + p.pos[i];
-        p.perm[col] = (u32)(i / p.k_used);
+    if (valid) {
+        const u32 col = sbefore[e] + mine[e] + rank;
+        p.perm[col] = (u32)row_of(i);
         p.pos[i] = col;
     }
 }
