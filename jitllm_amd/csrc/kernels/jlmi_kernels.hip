@@ -311,9 +311,13 @@ extern "C" __global__ __launch_bounds__(128) void jl_moe_logits(MoeLogitsArgs p)
     moe_logits_body<1>(p, part);
 }
 // many tokens: grid = (ceil(experts / 8), ceil(tokens / JL_LOGITS_TOK)), block = 128
-extern "C" __global__ __launch_bounds__(128) void jl_moe_logits_e8(MoeLogitsArgs p) {
-    __shared__ float part[JL_LOGITS_TOK * 128];
+extern "C" __global__ __launch_bounds__(128, 4) void jl_moe_logits_e8(MoeLogitsArgs p) {
+    __shared__ float part[2 * JL_LOGITS_TOK * 128];
     moe_logits_body<8>(p, part);
+}
+extern "C" __global__ __launch_bounds__(128, 4) void jl_moe_logits_e8_f16(MoeLogitsArgs p) {
+    __shared__ float part[2 * JL_LOGITS_TOK * 128];
+    moe_logits_body<8, true>(p, part);
 }
 // one workgroup of 1024 threads (n_expert <= 1024)
 extern "C" __global__ __launch_bounds__(1024) void jl_moe_group(MoeGroupArgs p) {

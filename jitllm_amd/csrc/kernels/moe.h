@@ -1356,10 +1356,11 @@ __device__ __forceinline__ void moe_combine_body(const MoeCombineArgs& p, float*
 // taking thread j + s at s = 64, 32, ..., 1.  One workgroup per expert row and group of
 // JL_LOGITS_TOK tokens: the row is read once for all of them.
 // With many tokens the launch is bound by re-reading x from L2 for every expert row (2048
-// tokens x 128 experts x k = 2048: 114 us), so there a workgroup takes EB = 8 expert rows
-// for its eight tokens and every x value loaded meets eight weights (grid.x = ceil(rows/EB)).
+// tokens x 128 experts x k = 2048: 88 us), so there a workgroup takes EB = 8 expert rows
+// for its eight tokens and every x value loaded meets eight weights (grid.x = ceil(rows/EB)): 34 us, a
+// product and a sum an instruction each (12 us of issue), four wavefronts a SIMD.
 #define JL_LOGITS_TOK 8
-template <int EB>
+template <int EB, bool F16 = false>
 __device__ __forceinline__ void moe_logits_body(const MoeLogitsArgs& p, float* part) {
     const int r0 = blockIdx.x * EB, t0 = blockIdx.y * JL_LOGITS_TOK, tid = threadIdx.x;
     const int nt = min(JL_LOGITS_TOK, p.ntok - t0), k = p.k;
@@ -1368,35 +1369,79 @@ __device__ __forceinline__ void moe_logits_body(const MoeLogitsArgs& p, float* p
     for (int e = 0; e < EB; e++)
 #pragma unroll
         for (int t = 0; t < JL_LOGITS_TOK; t++) acc[e][t] = 0.f;
-    // a trip: element i0 + tid of every row and token; the ragged last trip (k % 128 != 0) adds +0 where
-    // the row has ended, the whole ones carry neither the select nor the clamp (a third of the
-    // loop's vector instructions, and the kernel issues vector instructions most of its time)
-    auto trip = [&](int i0, auto RAGGED) {
-        constexpr bool ragged = decltype(RAGGED)::value != 0;
-        const int i = i0 + tid, ic = ragged ? min(i, k - 1) : i;
-        float w[EB], xv[JL_LOGITS_TOK];
+    if constexpr (EB == 1) {
+        // a trip: element i0 + tid of every row and token; the ragged last trip (k % 128 != 0) adds +0 where
+        // the row has ended, the whole ones carry neither the select nor the clamp (a third of the
+        // loop's vector instructions, and the kernel issues vector instructions most of its time)
+        auto trip = [&](int i0, auto RAGGED) {
+            constexpr bool ragged = decltype(RAGGED)::value != 0;
+            const int i = i0 + tid, ic = ragged ? min(i, k - 1) : i;
+            float w, xv[JL_LOGITS_TOK];
+            const size_t at = (size_t)r0 * k + ic;
+            w = p.f16 ? half_bits_to_f32(((const uint16_t*)p.w)[at]) : ((const float*)p.w)[at];
 #pragma unroll
-        for (int e = 0; e < EB; e++) {
-            const size_t at = (size_t)min(r0 + e, p.n_expert - 1) * k + ic;
-            w[e] = p.f16 ? half_bits_to_f32(((const uint16_t*)p.w)[at]) : ((const float*)p.w)[at];
+            for (int t = 0; t < JL_LOGITS_TOK; t++) xv[t] = p.x[(size_t)(t0 + min(t, nt - 1)) * k + ic];
+#pragma unroll
+            for (int t = 0; t < JL_LOGITS_TOK; t++) {
+                const float prod = w * xv[t];
+                acc[0][t] = acc[0][t] + (!ragged || i < k ? prod : 0.f);
+            }
+        };
+        const int kfull = k & ~127;
+        // unrolled so that the loads of several trips are in flight together; the sums stay in order
+#pragma unroll 16
+        for (int i0 = 0; i0 < kfull; i0 += 128) trip(i0, GemmIntC<0>{});
+        if (kfull < k) trip(kfull, GemmIntC<1>{});
+    } else {
+        // Every row's base in scalar registers and one lane offset for all sixteen loads of a trip, the next trip's
+        // loads on their way while this one's 64 products are added: two vector instructions a product and nothing
+        // beside them (the clamped form with a select a product: 24.9 us at 777 tokens x 128 experts x 2048, this 16.8).
+        const float* xp[JL_LOGITS_TOK];
+        const char* wp[EB];
+        constexpr int es = F16 ? 2 : 4;
+#pragma unroll
+        for (int t = 0; t < JL_LOGITS_TOK; t++) xp[t] = p.x + (size_t)(t0 + min(t, nt - 1)) * k;
+#pragma unroll
+        for (int e = 0; e < EB; e++) wp[e] = (const char*)p.w + (size_t)min(r0 + e, p.n_expert - 1) * k * es;
+        float w[EB], xv[JL_LOGITS_TOK], wn[EB], xn[JL_LOGITS_TOK];
+        const int trips = (k + 127) >> 7;
+        auto load = [&](float (&a)[EB], float (&b)[JL_LOGITS_TOK], int trip) __attribute__((always_inline)) {
+            const u32 i = (u32)min(128 * trip + tid, k - 1);
+#pragma unroll
+            for (int e = 0; e < EB; e++) {
+                if constexpr (F16) a[e] = half_bits_to_f32(*(const uint16_t*)(wp[e] + 2 * i));
+                else a[e] = *(const float*)(wp[e] + 4 * i);
+            }
+#pragma unroll
+            for (int t = 0; t < JL_LOGITS_TOK; t++) b[t] = *(const float*)((const char*)xp[t] + 4 * i);
+        };
+        load(w, xv, 0);
+        for (int trip = 0; trip + 1 < trips; trip++) {
+            load(wn, xn, trip + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < EB; e++) {
+#pragma unroll
+                for (int t = 0; t < JL_LOGITS_TOK; t++) {
+                    const float prod = w[e] * xv[t];
+                    acc[e][t] = acc[e][t] + prod;
+                }
+                __builtin_amdgcn_sched_barrier(0);   // (products not formed far ahead of their sums, in registers of their own)
+            }
+#pragma unroll
+            for (int e = 0; e < EB; e++) w[e] = wn[e];
+#pragma unroll
+            for (int t = 0; t < JL_LOGITS_TOK; t++) xv[t] = xn[t];
         }
-#pragma unroll
-        for (int t = 0; t < JL_LOGITS_TOK; t++) xv[t] = p.x[(size_t)(t0 + min(t, nt - 1)) * k + ic];
+        const bool in = 128 * (trips - 1) + tid < k;   // in the ragged last trip a lane past the row's end adds +0
 #pragma unroll
         for (int e = 0; e < EB; e++)
 #pragma unroll
             for (int t = 0; t < JL_LOGITS_TOK; t++) {
                 const float prod = w[e] * xv[t];
-                acc[e][t] = acc[e][t] + (!ragged || i < k ? prod : 0.f);
+                acc[e][t] = acc[e][t] + (in ? prod : 0.f);
             }
-    };
-    const int kfull = k & ~127;
-    // unrolled so that the loads of several trips are in flight together; the sums stay in order
-#pragma unroll EB == 1 ? 16 : 2
-    // (the eight-row form keeps the select in every trip: without it the same loop measured 34.4 us
-    // against 29.3 at 1024 tokens, the one-row form 5.96 against 6.8 at 64)
-    for (int i0 = 0; i0 < kfull; i0 += 128) trip(i0, GemmIntC<EB == 1 ? 0 : 1>{});
-    if (kfull < k) trip(kfull, GemmIntC<1>{});
+    }
     // The tree, one token per 16 lanes: lane j of a token's row takes the partial sums the
     // tree would bring to thread j by s = 16 (levels 64, 32, 16: seven adds in tree order),
     // then levels 8..1 are lane moves inside the 16-lane row (lane j reads lane j + s).
@@ -1406,11 +1451,11 @@ __device__ __forceinline__ void moe_logits_body(const MoeLogitsArgs& p, float* p
     const int tk = tid >> 4, j = tid & 15;
 #pragma unroll
     for (int e = 0; e < EB; e++) {
-        if (e) __syncthreads();
+        float* buf = part + (e & 1) * (JL_LOGITS_TOK * 128);   // (two in turn: one barrier a row)
 #pragma unroll
-        for (int t = 0; t < JL_LOGITS_TOK; t++) part[t * 128 + tid] = acc[e][t];
+        for (int t = 0; t < JL_LOGITS_TOK; t++) buf[t * 128 + tid] = acc[e][t];
         __syncthreads();
-        const float* q = part + tk * 128 + j;
+        const float* q = buf + tk * 128 + j;
         const float a0 = q[0] + q[64], a32 = q[32] + q[96], a16 = q[16] + q[80], a48 = q[48] + q[112];
         const float b0 = a0 + a32, b16 = a16 + a48;
         float v = b0 + b16;
