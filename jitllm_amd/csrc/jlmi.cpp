@@ -1346,18 +1346,25 @@ int moe_gemm_i8_launch(jl_ctx* c, float* out0, float* out1, int type, const void
 
 // Blocks of rows an expert's matrix is cut into by the groups-of-columns kernels ("moe.form" = 3): one workgroup of eight
 // wavefronts a CU (the same age on every SIMD, tiles handed out as they get to them: two younger workgroups of four
-// measured 4 % slower), so the grid runs in rounds of CUs workgroups; among the splits of the rows into blocks the one
-// with the least rounds x tiles a wavefront, the fewest blocks among equals (every block fills LDS anew).  Experts that
-// can have a column: at most one a column.  "moe.waves" = 4: the two-workgroup form.
-int moe_g16_blocks(const jl_ctx* c, int nrows, int n_expert, int ncols, int nmat, int nwaves) {
+// measured 4 % slower).  An expert is worked on by XCD e % 8 alone, so the grid runs in rounds of that XCD's CUs, a round
+// taking its fill of LDS and the tiles a wavefront has: the split that is estimated least, the fewest blocks among equals.
+// Fitted to 19 shapes (8 to 128 experts of 512 x 1024 to 2304 x 768) at 2, 4, 6 and 8 columns an expert and every number of
+// blocks, 9 % each; the pick is 0.6 % behind the best on average, at most 19 (rounds of all CUs without the fill, the rule
+// before: 5.7, at most 64: 46 x 1536 x 1024 twice, eight columns, twelve blocks 41 us, two 25.4).  "moe.waves" = 4: the
+// two-workgroup form.
+int moe_g16_blocks(const jl_ctx* c, int nrows, int k, int n_expert, int ncols, int nmat, int nwaves) {
     const int tiles = (nrows + 15) / 16, sets = (tiles + nwaves - 1) / nwaves;
     if (c->tune.moe_shares > 0) return std::min(c->tune.moe_shares, sets);
-    const long slots = (nwaves == 4 ? 2L : 1L) * c->num_cu, n_act = std::min<long>(n_expert, ncols);
+    // (experts that can have a column: at most one a column)
+    const long slots = std::max(1, c->num_cu / 8) * (nwaves == 4 ? 2L : 1L), n_xcd = (std::min<long>(n_expert, ncols) + 7) / 8;
+    const double nsb = k / 256, fill = 1.62 + (0.22 + 0.074 * std::min(16.0, (double)ncols / n_expert)) * nsb, tile = 0.19 + 0.6 * nsb;
     int best = 1;
-    long best_cost = -1;
+    double best_cost = 1e30;
     for (int nb = 1; nb <= sets && nb <= 64; nb++) {
-        const long per_wave = (sets + nb - 1) / nb, rounds = ((long)nb * n_act * nmat + slots - 1) / slots, cost = rounds * per_wave;
-        if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = nb; }
+        const long tiles_wg = (tiles + nb - 1) / nb, blocks = (tiles + tiles_wg - 1) / tiles_wg;
+        const long per_wave = (tiles_wg + nwaves - 1) / nwaves, rounds = (blocks * nmat * n_xcd + slots - 1) / slots;
+        const double cost = rounds * (fill + per_wave * tile);
+        if (cost < best_cost) { best_cost = cost; best = nb; }
     }
     return best;
 }
@@ -1602,7 +1609,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
             }
             const int nmat = (planes ? pb1 != nullptr : bank1 != nullptr) ? 2 : 1, tiles = (nrows + 15) / 16;
             const int nwaves = !two && c->tune.moe_waves == 4 ? 4 : 8;
-            const int best_blocks = moe_g16_blocks(c, nrows, n_expert, ncols, nmat, nwaves);
+            const int best_blocks = moe_g16_blocks(c, nrows, k, n_expert, ncols, nmat, nwaves);
             ga.tiles_wg = (tiles + best_blocks - 1) / best_blocks;   // handed out inside the workgroup as its wavefronts get to them
             ga.blocks = (tiles + ga.tiles_wg - 1) / ga.tiles_wg;
             ga.nmat = nmat; ga.n_expert = n_expert; ga.nwaves = nwaves;
