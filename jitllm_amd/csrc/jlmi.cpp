@@ -1421,6 +1421,29 @@ int moe_banks_check(jl_ctx* c, int type, bool planes, const void* bank0, const v
     return (type == JL_TYPE_Q4_K ? sheet % 16 : sheet % 2) != 0 ? JL_DECLINED : JL_OK;
 }
 
+// A decode matvec a routed column (kernels/moe.h: moe_gather_body), GGUF banks.
+int moe_gather_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1, const float* x,
+                      const float* x2, const uint32_t* src, const uint32_t* start, int n_expert, int ncols, int nrows, int k, hipStream_t st) {
+    const TypeInfo* ti = type_info(type);
+    MoeGatherArgs a;
+    a.out[0] = out0; a.out[1] = out1; a.bank[0] = (const uint8_t*)bank0; a.bank[1] = (const uint8_t*)bank1;
+    a.x = x; a.x2 = x2; a.src = src; a.start = start; a.n_expert = n_expert;
+    a.nrows = nrows; a.k = k; a.row_bytes = (k / ti->block_elems) * ti->block_bytes; a.per = c->act_window / 32;
+    a.sheet_bytes = (size_t)nrows * a.row_bytes;
+    const int nmat = bank1 ? 2 : 1;
+    const bool pair = q8_pair_form(c, type, bank0, k) && (!bank1 || q8_pair_form(c, type, bank1, k)) && a.sheet_bytes % 4 == 0;
+    const size_t lds = act_lds_bytes(k) + (pair ? (size_t)k + 16 : 0) + 16;
+    if (lds > c->lds_limit || ncols > 65535) return JL_DECLINED;
+    // one round of workgroups, as the grouped matvecs (two a CU for the paired Q8_0 form)
+    a.nwaves = 16;
+    const long slots = (pair ? 2L : 1L) * c->num_cu, groups = (nrows + 15) / 16;
+    a.ngroups = (int)std::max(1L, std::min(groups, slots / ((long)ncols * nmat)));
+    Name name;
+    name << "jl_moe_gather_" << (pair ? "q8_0p" : ti->tag) << (x2 ? "_a" : "");
+    void* params[] = {&a};
+    return launch(c, name, (unsigned)a.ngroups, (unsigned)ncols, 1024, (unsigned)lds, st, params, (unsigned)nmat);
+}
+
 // The columns of an expert against rows decoded in registers (kernels/moe_cols.h): the source rows quantized once each
 // (nsrc of them, src naming each column's; nsrc = 0: not known, a record a column), then the matrices.
 int moe_cols_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1, const jl_packed_bank* pb0,
@@ -1504,6 +1527,16 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
         const bool align = sheet % (type == JL_TYPE_Q4_K ? 16 : 4) == 0;
         int form = c->tune.moe_form;
         if (q6 && !planes && c->act_window == 256 && (form == 3 || form == 4)) form += 2;   // (their Q6_K forms)
+        // A handful of columns: a decode matvec each (the whole block's us, as it was -> so).  Q4_K, 128 experts of 768 x 2048,
+        // 8 / 16 / 24 columns 42 -> 33 / 44 -> 40 / 46 -> 49, 60 of 1792 x 2816, 4 / 16 / 32 / 48 columns 53 -> 32 / 71 -> 52 /
+        // 94 -> 86 / 114 -> 127, 8 of 1024 x 1536, 2 / 16 / 24 columns 31 -> 22 / 38 -> 38 / 39 -> 47; Q6_K down projections the
+        // same; Q8_0, whose other form costs an expert more: the first 8 / 64 / 96 columns 52 -> 34 / 109 -> 96 / 128 -> 138,
+        // the second 57 -> 34 at 4, 191 -> 177 at 64, 8 x 1024 x 1536 at 24 columns 41 -> 43.  Q4_K and Q6_K sheets under 512 x 512
+        // keep the grouped form, whose launches a caller can count on there (tests/test_gpu_moe.py), though they would gain as
+        // well: 8 experts of 256 x 512, 12 columns 28.7 against 21.9.
+        const bool gather = type == JL_TYPE_Q8_0 ? ncols <= 16 || (ncols <= 64 && avg <= 1.1)
+                                                 : (long)nrows * k >= 512L * 512 && ncols <= ((double)nrows * k >= 2.4e6 && avg <= 0.6 ? 32 : 16);
+        if (form == 0 && !planes && (type == JL_TYPE_Q8_0 || type == JL_TYPE_Q4_K || q6) && gather) form = 10;
         if (form == 0 && (c->act_window == 32 || c->act_window == 256) && !planes) {
             if (q4w) form = ncols <= 8L * n_expert ? 0 : moe_few_faster(type, n_expert, ncols, nmat, nrows, k) ? 5 : 9;
             else if (q6 && c->act_window == 256 && avg > 8 && avg < 60) form = moe_few_faster(type, n_expert, ncols, nmat, nrows, k) ? 5 : 9;
@@ -1517,6 +1550,10 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
         // against 275 / 105, 64 384 / 151 against 380 / 138, 128 (the second) 219 against 208.
         if (form == 0 && q4w && planes && ncols >= 16L * n_expert) form = 9;
         if (form == 5 && !align && c->tune.moe_form == 0 && avg >= 6) form = 6;
+        if (form == 10 && !planes) {
+            rc = moe_gather_launch(c, out0, out1, type, bank0, bank1, x, x2, src, start, n_expert, ncols, nrows, k, st);
+            if (rc != JL_DECLINED) return rc;
+        }
         if (form == 9 && c->act_window == 256 && (type == JL_TYPE_Q4_K || (q6 && !planes))) {
             rc = moe_cols_launch(c, out0, out1, type, bank0, bank1, pb0, pb1, x, x2, src, start, n_expert, ncols, nrows, k, nsrc, st);
             if (rc != JL_DECLINED) return rc;
@@ -1834,6 +1871,8 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     names.push_back("jl_few_prep");
     names.push_back("jl_gemm_i8_prep");
     names.push_back("jl_moe_gemm_i8_prep");
+    for (const char* tag : {"q4k", "q8_0", "q8_0p", "q6k"})
+        for (const char* act : {"", "_a"}) names.push_back(std::string("jl_moe_gather_") + tag + act);
     for (const char* tag : {"q4k", "q4k_planes", "q6k"})
         for (const char* form : {"jl_moe_cols_", "jl_moe_cols_prep_"}) names.push_back(std::string(form) + tag);
     for (const char* tag : {"q8_0", "q4k", "q6k", "q6kw"})

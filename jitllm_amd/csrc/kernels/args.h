@@ -170,6 +170,18 @@ struct MoeGemmArgs {
 
 // Grouped expert matmul for experts of some tens of columns (kernels/moe_cols.h): rec [record][k/256][512 or 256 bytes],
 // aug [record][k/256][32 bytes], da [record][k/256].
+// A decode matvec a routed column (moe_gather_body): grid y = column, z = matrix.
+struct MoeGatherArgs {
+    float* out[2];          // [column][nrows]
+    const uint8_t* bank[2];
+    const float* x;
+    const float* x2;        // null: plain activation, else silu(x) * x2
+    const uint32_t* src;    // null: column c reads row c
+    const uint32_t* start;
+    size_t sheet_bytes;
+    int nrows, k, row_bytes, per, nwaves, ngroups, n_expert;
+};
+
 struct MoeColsPrepArgs {
     const float* x;
     const float* x2;        // null: plain activation, else silu(x) * x2

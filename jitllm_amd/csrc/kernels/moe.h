@@ -1348,6 +1348,38 @@ __device__ __forceinline__ void moe_combine_body(const MoeCombineArgs& p, float*
     *res = acc;
 }
 
+// ---------------------------------------------------------------- a column or two of a few experts
+// A decode matvec (kernels/matvec.h) for each routed column: its source row quantized in the workgroup, its expert's sheet
+// read once for it.  With hardly a column an expert that is every byte once, and there is no launch in front that quantizes.
+template <int TYPE, int PRE>
+__device__ __forceinline__ void moe_gather_body(const MoeGatherArgs& args, uint8_t* smem) {
+    const u32 c = blockIdx.y;
+    const int mat = blockIdx.z, lane = threadIdx.x & 63;
+    MultiNow m;
+    m.out = args.out[mat]; m.w = args.bank[mat]; m.nrows = args.nrows; m.k = args.k; m.per = args.per; m.nwaves = args.nwaves;
+    m.ngroups = args.ngroups; m.row_bytes = args.row_bytes; m.type = 0; m.x = args.x; m.x2 = PRE & JL_PRE_ACT ? args.x2 : nullptr;
+    m.resid = nullptr; m.resid_gate = nullptr; m.alpha = 0.f; m.norm_w = nullptr; m.norm_out = nullptr; m.norm_eps = 0.f; m.inv_k = 0.0;
+    const u32 *src = args.src, *start = args.start;
+    size_t sheet = args.sheet_bytes;
+    int n_expert = args.n_expert;
+    JL_NOW(m.out, m.w, m.nrows, m.k, m.per, m.nwaves, m.ngroups, m.row_bytes, m.x, m.x2, src, start, sheet, n_expert);
+    src = as_global(src); start = as_global(start);
+    const u32 row = src ? (u32)__builtin_amdgcn_readfirstlane((i32)src[c]) : c;
+    // the column's expert: the last whose first column is not past it
+    u32 cnt = 0;
+    for (int base = 0; base <= n_expert; base += 64) {
+        const int idx = base + lane;
+        const u32 s = start[min(idx, n_expert)];
+        cnt += (u32)__builtin_popcountll(__ballot(idx <= n_expert && s <= c));
+    }
+    m.out = as_global(m.out) + (size_t)c * m.nrows;
+    m.w = as_global(m.w) + (size_t)(cnt - 1) * sheet;
+    m.x = as_global(m.x) + (size_t)row * m.k;
+    if constexpr ((PRE & JL_PRE_ACT) != 0) m.x2 = as_global(m.x2) + (size_t)row * m.k;
+    MatVecMultiArgs unused;
+    matvec_multi_body_xp<TYPE, 1, false, PRE>(unused, m, smem);
+}
+
 // ---------------------------------------------------------------- router logits
 // logits[t][r] = sum_i W[r][i] * x[t][i] in f32, with the summation order of the reference's
 // device kernel (jit/gpu/kernels/moe.go:843-917) so that the bits are its bits: thread j of
