@@ -1421,13 +1421,14 @@ int moe_banks_check(jl_ctx* c, int type, bool planes, const void* bank0, const v
     return (type == JL_TYPE_Q4_K ? sheet % 16 : sheet % 2) != 0 ? JL_DECLINED : JL_OK;
 }
 
-// A decode matvec a routed column (kernels/moe.h: moe_gather_body), GGUF banks.
-int moe_gather_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1, const float* x,
-                      const float* x2, const uint32_t* src, const uint32_t* start, int n_expert, int ncols, int nrows, int k, hipStream_t st) {
+// A decode matvec a routed column (kernels/moe.h: moe_gather_body), GGUF banks.  start null: column c is pair c of sel.
+int moe_gather_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1, const float* x, const float* x2,
+                      const uint32_t* src, const uint32_t* start, const uint32_t* sel, int sel_stride, int k_used, int n_expert, int ncols,
+                      int nrows, int k, hipStream_t st) {
     const TypeInfo* ti = type_info(type);
     MoeGatherArgs a;
     a.out[0] = out0; a.out[1] = out1; a.bank[0] = (const uint8_t*)bank0; a.bank[1] = (const uint8_t*)bank1;
-    a.x = x; a.x2 = x2; a.src = src; a.start = start; a.n_expert = n_expert;
+    a.x = x; a.x2 = x2; a.src = src; a.start = start; a.sel = sel; a.sel_stride = sel_stride; a.k_used = k_used; a.n_expert = n_expert;
     a.nrows = nrows; a.k = k; a.row_bytes = (k / ti->block_elems) * ti->block_bytes; a.per = c->act_window / 32;
     a.sheet_bytes = (size_t)nrows * a.row_bytes;
     const int nmat = bank1 ? 2 : 1;
@@ -1442,6 +1443,56 @@ int moe_gather_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     name << "jl_moe_gather_" << (pair ? "q8_0p" : ti->tag) << (x2 ? "_a" : "");
     void* params[] = {&a};
     return launch(c, name, (unsigned)a.ngroups, (unsigned)ncols, 1024, (unsigned)lds, st, params, (unsigned)nmat);
+}
+
+// Whether a block's pairs go without grouping (moe_gather_ffn).  What that saves is two launches and the grouped kernels' setup; what
+// it costs is a sheet read once more for every pair that shares its expert with another, so the line is a number of such pairs,
+// the rows' choices taken as evenly spread.  The whole block, grouped -> so, us, pairs that share in brackets: Q4_K 128 experts
+// top-8 of 768 x 2048 with Q6_K down 35 -> 24 (0), 43 -> 27 (0.5), 56 -> 36 (3), 82 -> 63 (12), 96 -> 97 (27); 60 top-4 of 1792 x
+// 2816 33 -> 25 (0), 127 -> 117 (21), 142 -> 178 (44); 8 top-2 of 2048 x 2816 28 -> 20 (0), 50 -> 40 (9), 48 -> 49 (13); 32 top-4 of
+// 1024 x 2048 47 -> 37 (11), 53 -> 54 (23).  Q8_0, whose grouped form costs more: 60 top-4 of 1792 x 2816 36 -> 27 (0), 174 -> 159
+// (21), 221 -> 250 (44); 32 top-4 of 1024 x 2048 57 -> 43 (11), 80 -> 70 (36), 84 -> 86 (50); 8 top-2 of 2048 x 2816 51 -> 45 (9),
+// 59 -> 57 (13), 63 -> 66 (16: three pairs an expert, where the grouped form reads a sheet a third as often); Q6_K the same,
+// 128 experts top-8 of 768 x 2048 119 -> 114 (27), 155 -> 190 (92).
+// Q4_K and Q6_K sheets under 512 x 512 keep the grouped form, whose launches a caller can count on there
+// (tests/test_gpu_moe.py), though they would gain as well.
+bool moe_gather_ffn_wanted(int type, int rows, int k_used, int n_expert, int n_ffn, int n_embd) {
+    const double pairs = (double)rows * k_used;
+    if (pairs > 256 || pairs > 2.5 * n_expert || (type != JL_TYPE_Q8_0 && (long)n_ffn * n_embd < 512L * 512)) return false;
+    const double touched = n_expert * (1.0 - std::pow(1.0 - std::min(1.0, (double)k_used / n_expert), rows));
+    return pairs - touched <= (type == JL_TYPE_Q4_K ? 18 : 32);
+}
+
+// A routed block of a handful of pairs without its grouping and combine: the pairs themselves are the columns of gate + up,
+// and the down projections of a row's pairs are one matvec that adds into the residual stream.  JL_DECLINED (nothing
+// enqueued) where the activations of a row do not fit LDS.
+int moe_gather_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate, const void* up, const void* down, const float* x,
+                   const uint32_t* sel, int sel_stride, const float* wt, int rows, int k_used, int n_expert, int n_ffn, int n_embd,
+                   float* g, float* u, hipStream_t st) {
+    const TypeInfo* ti = type_info(down_type);
+    MoeGatherDownArgs a;
+    a.resid = resid; a.bank = (const uint8_t*)down; a.g = g; a.u = u; a.sel = sel; a.wt = wt;
+    a.nrows = n_embd; a.k = n_ffn; a.row_bytes = (n_ffn / ti->block_elems) * ti->block_bytes; a.per = c->act_window / 32;
+    a.sheet_bytes = (size_t)n_embd * a.row_bytes;
+    a.n_expert = n_expert; a.sel_stride = sel_stride; a.k_used = k_used;
+    const long kk = (long)k_used * n_ffn;
+    if (kk > 65536 || act_lds_bytes((int)kk) + 256 > c->lds_limit || act_lds_bytes(n_embd) + 256 > c->lds_limit) return JL_DECLINED;
+    const bool pair = q8_pair_form(c, down_type, down, (int)kk) && n_ffn % 64 == 0 && a.row_bytes % 4 == 0 &&
+                      act_lds_bytes((int)kk) + (size_t)kk + 256 <= c->lds_limit;
+    const size_t lds = act_lds_bytes((int)kk) + (pair ? (size_t)kk + 16 : 0) + 16 + 128;
+    const uint32_t row_slots = (uint32_t)(n_ffn / (down_type == JL_TYPE_Q8_0 && !pair ? 32 : 64));
+    a.slots_inv = 0xFFFFFFFFu / row_slots + 1u;
+    int rc = moe_gather_launch(c, g, u, type, gate, up, x, nullptr, nullptr, nullptr, sel, sel_stride, k_used, n_expert, rows * k_used,
+                               n_ffn, n_embd, st);
+    if (rc != JL_OK) return rc;
+    // (eight and four wavefronts a workgroup: the same at one row, 2 and 9 us slower at 32 pairs)
+    a.nwaves = 16;
+    const long slots = (pair ? 2L : 1L) * c->num_cu, groups = (n_embd + 15) / 16;
+    a.ngroups = (int)std::max(1L, std::min(groups, slots / rows));
+    Name name;
+    name << "jl_moe_gather_" << (pair ? "q8_0p" : ti->tag) << "_down";
+    void* params[] = {&a};
+    return launch(c, name, (unsigned)a.ngroups, (unsigned)rows, 1024, (unsigned)lds, st, params);
 }
 
 // The columns of an expert against rows decoded in registers (kernels/moe_cols.h): the source rows quantized once each
@@ -1551,7 +1602,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
         if (form == 0 && q4w && planes && ncols >= 16L * n_expert) form = 9;
         if (form == 5 && !align && c->tune.moe_form == 0 && avg >= 6) form = 6;
         if (form == 10 && !planes) {
-            rc = moe_gather_launch(c, out0, out1, type, bank0, bank1, x, x2, src, start, n_expert, ncols, nrows, k, st);
+            rc = moe_gather_launch(c, out0, out1, type, bank0, bank1, x, x2, src, start, nullptr, 0, 1, n_expert, ncols, nrows, k, st);
             if (rc != JL_DECLINED) return rc;
         }
         if (form == 9 && c->act_window == 256 && (type == JL_TYPE_Q4_K || (q6 && !planes))) {
@@ -1872,7 +1923,7 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     names.push_back("jl_gemm_i8_prep");
     names.push_back("jl_moe_gemm_i8_prep");
     for (const char* tag : {"q4k", "q8_0", "q8_0p", "q6k"})
-        for (const char* act : {"", "_a"}) names.push_back(std::string("jl_moe_gather_") + tag + act);
+        for (const char* act : {"", "_a", "_down"}) names.push_back(std::string("jl_moe_gather_") + tag + act);
     for (const char* tag : {"q4k", "q4k_planes", "q6k"})
         for (const char* form : {"jl_moe_cols_", "jl_moe_cols_prep_"}) names.push_back(std::string(form) + tag);
     for (const char* tag : {"q8_0", "q4k", "q6k", "q6kw"})
@@ -2568,6 +2619,11 @@ int moe_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate_b
         }
         rc = dense_ffn(c, resid, type, down_type, gate_bank, up_bank, down_bank, planes ? &a : nullptr, planes ? &b : nullptr,
                        planes ? &d : nullptr, x, wt, rows, n_ffn, n_embd, g, u, y, st);
+        if (rc != JL_DECLINED) return rc;
+    }
+    if (!planes && (c->tune.moe_form == 11 || (c->tune.moe_form == 0 && moe_gather_ffn_wanted(type, rows, k_used, n_expert, n_ffn, n_embd)))) {
+        rc = moe_gather_ffn(c, resid, type, down_type, gate_bank, up_bank, down_bank, x, sel, sel_stride, wt, rows, k_used, n_expert, n_ffn,
+                            n_embd, g, u, st);
         if (rc != JL_DECLINED) return rc;
     }
     rc = jl_moe_group_dev(c, sel, sel_stride, rows, k_used, n_expert, start, perm, pos, st);

@@ -177,9 +177,23 @@ struct MoeGatherArgs {
     const float* x;
     const float* x2;        // null: plain activation, else silu(x) * x2
     const uint32_t* src;    // null: column c reads row c
-    const uint32_t* start;
+    const uint32_t* start;  // null: column c is pair c of sel, which reads row c / k_used
+    const uint32_t* sel;    // [row][sel_stride]
     size_t sheet_bytes;
-    int nrows, k, row_bytes, per, nwaves, ngroups, n_expert;
+    int nrows, k, row_bytes, per, nwaves, ngroups, n_expert, sel_stride, k_used;
+};
+
+// resid[row] += sum over the row's pairs of wt * (down sheet of the pair's expert . silu(g) u)  (moe_gather_down_body):
+// grid y = row.
+struct MoeGatherDownArgs {
+    float* resid;           // [row][nrows]
+    const uint8_t* bank;
+    const float *g, *u;     // [pair][k]
+    const uint32_t* sel;    // [row][sel_stride]
+    const float* wt;        // [row][k_used]
+    size_t sheet_bytes;
+    uint32_t slots_inv;     // 2^32 / (slots of a sheet's row), rounded up
+    int nrows, k, row_bytes, per, nwaves, ngroups, n_expert, sel_stride, k_used;
 };
 
 struct MoeColsPrepArgs {

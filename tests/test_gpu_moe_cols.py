@@ -123,3 +123,49 @@ def test_a_matvec_a_column(dev, devbuf, t, window, nrows, k):
                 assert nmse(got[:ncols * nrows].reshape(ncols, nrows), want) <= (1e-6 if gated else 1e-10), (gated, b)
     finally:
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("t,down,window,n_expert,k_used,rows,n_ffn,n_embd,pair", [
+    (quant.Q4_K, quant.Q6_K, 256, 40, 8, 1, 512, 512, 0),       # fewer slots than two chunks of lanes; one row
+    (quant.Q4_K, quant.Q4_K, 256, 9, 3, 3, 1280, 1792, 0),      # ragged chunks, more row groups than workgroups a row
+    (quant.Q4_K, quant.Q4_K, 32, 33, 1, 2, 768, 2304, 0),       # one pair a row
+    (quant.Q6_K, quant.Q6_K, 32, 20, 2, 5, 512, 512, 0),
+    (quant.Q8_0, quant.Q8_0, 32, 20, 16, 2, 256, 256, 0),       # sixteen pairs, the paired form
+    (quant.Q8_0, quant.Q8_0, 32, 12, 4, 3, 1024, 768, 2),       # banks that are not on four bytes: the plain form
+    (quant.Q8_0, quant.Q6_K, 32, 12, 5, 3, 768, 1024, 0),
+], ids=lambda v: str(v))
+def test_block_of_pairs(dev, devbuf, t, down, window, n_expert, k_used, rows, n_ffn, n_embd, pair):
+    """The routed block without grouping and combine: a selection with a stride of its own, the first and the last expert
+    in use, an id no expert has (it adds nothing), the residual added to and nothing behind it touched."""
+    from test_gpu_moe import _oracle_block
+    rng = np.random.default_rng(7)
+    sel = np.full((rows, k_used + 2), 0xFFFFFFFF, np.uint32)
+    for r in range(rows):
+        sel[r, :k_used] = rng.permutation(n_expert)[:k_used]
+    sel[0, 0], sel[-1, k_used - 1] = (0, n_expert - 1) if k_used > 1 or rows > 1 else (0, 0)
+    if rows > 2:
+        sel[1, 0] = n_expert + 3
+    wt = (rng.random((rows, k_used)) / k_used).astype(np.float32)
+    bank = lambda ty, nr, k, s: np.concatenate([synth.random_weights(ty, nr, k, seed=s + e) for e in range(n_expert)])
+    banks = [bank(t, n_ffn, n_embd, 0), bank(t, n_ffn, n_embd, 100), bank(down, n_embd, n_ffn, 200)]
+    x = np.stack([synth.activations(n_embd, seed=900 + r) for r in range(rows)])
+    start = rng.standard_normal((rows, n_embd)).astype(np.float32)
+    want = start + _oracle_block(t, *banks, x, sel, wt, n_expert, n_ffn, n_embd, window, td=down)
+    dev.SetActWindow(window)
+    hold = [devbuf(b) for b in banks]
+    xd, sd, wd = devbuf(x), devbuf(sel), devbuf(wt)
+    try:
+        dev.set_tuning(moe__form=11, q8pair=pair)
+        resid = devbuf(np.concatenate([start.reshape(-1), np.full(8, FILL)]))
+        before = dev.launch_count()
+        assert dev.moe_ffn_dev(resid.ptr, t, *[b.ptr for b in hold], xd.ptr, sd.ptr, k_used + 2, wd.ptr, rows, k_used, n_expert,
+                               n_ffn, n_embd, down_type=down)
+        dev.synchronize()
+        assert dev.launch_count() - before == 2
+        got = resid.get()
+        assert np.all(got[rows * n_embd:] == FILL)
+        # (an exponential of another machine in front of the second quantizer, as for the other forms)
+        assert nmse(got[:rows * n_embd].reshape(rows, n_embd), want) <= 1e-6
+    finally:
+        dev.set_tuning(moe__form=0, q8pair=0)
+        dev.SetActWindow(32)
