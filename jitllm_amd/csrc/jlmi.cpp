@@ -1421,6 +1421,23 @@ int moe_banks_check(jl_ctx* c, int type, bool planes, const void* bank0, const v
     return (type == JL_TYPE_Q4_K ? sheet % 16 : sheet % 2) != 0 ? JL_DECLINED : JL_OK;
 }
 
+// Lanes a row for the gather kernels: of 64, 32 and 16 (8: rows of eight slots at most) the width that leaves the fewest without a slot while every CU still gets
+// a workgroup.
+// Whole block, us, 64 -> 32 / 16 lanes for gate + up: Q4_K, 32 slots a row (K 2048), 8 / 32 / 96 pairs of 128 experts 22.6 -> 21.8 /
+// 20.8, 36.6 -> 31.2 / 31.7, 95.7 -> 76.4 / 77.3; 44 slots (three of sixteen lanes), 16 / 60 pairs of 60 43.5 -> 42.6 / 40.1, 116 ->
+// 114 / 103; too few workgroups, 2 pairs of 24 experts of 1280 rows, 40 slots, 18.2 -> 19.4 / 19.7.  Q8_0 gains only while a lane
+// has one slot: 28 slots 70 -> 66 / 67, 44 slots 59.7 -> 63.4 / 63.6.
+int gather_lanes(const jl_ctx* c, int type, int nslots, int nrows, long matvecs) {
+    int best = 64;
+    double most = nslots / (64.0 * ((nslots + 63) / 64));
+    for (int lanes = 32; lanes >= (nslots <= 8 ? 8 : 16); lanes /= 2) {
+        const double used = nslots / ((double)lanes * ((nslots + lanes - 1) / lanes));
+        const int rows = 16 * (64 / lanes);
+        if (used > most && (type != JL_TYPE_Q8_0 || nslots <= lanes) && (nrows + rows - 1) / rows * matvecs >= c->num_cu) best = lanes, most = used;
+    }
+    return best;
+}
+
 // A decode matvec a routed column (kernels/moe.h: moe_gather_body), GGUF banks.  start null: column c is pair c of sel.
 int moe_gather_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1, const float* x, const float* x2,
                       const uint32_t* src, const uint32_t* start, const uint32_t* sel, int sel_stride, int k_used, int n_expert, int ncols,
@@ -1437,30 +1454,32 @@ int moe_gather_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     if (lds > c->lds_limit || ncols > 65535) return JL_DECLINED;
     // one round of workgroups, as the grouped matvecs (two a CU for the paired Q8_0 form)
     a.nwaves = 16;
-    const long slots = (pair ? 2L : 1L) * c->num_cu, groups = (nrows + 15) / 16;
+    const int lpr = gather_lanes(c, type, k / (type == JL_TYPE_Q8_0 && !pair ? 32 : 64), nrows, (long)ncols * nmat), per_group = 16 * (64 / lpr);
+    const long slots = (pair ? 2L : 1L) * c->num_cu, groups = (nrows + per_group - 1) / per_group;
     a.ngroups = (int)std::max(1L, std::min(groups, slots / ((long)ncols * nmat)));
     Name name;
-    name << "jl_moe_gather_" << (pair ? "q8_0p" : ti->tag) << (x2 ? "_a" : "");
+    name << "jl_moe_gather_" << (pair ? "q8_0p" : ti->tag) << (x2 ? "_a" : "") << "_l" << lpr;
     void* params[] = {&a};
     return launch(c, name, (unsigned)a.ngroups, (unsigned)ncols, 1024, (unsigned)lds, st, params, (unsigned)nmat);
 }
 
-// Whether a block's pairs go without grouping (moe_gather_ffn).  What that saves is two launches and the grouped kernels' setup; what
-// it costs is a sheet read once more for every pair that shares its expert with another, so the line is a number of such pairs,
-// the rows' choices taken as evenly spread.  The whole block, grouped -> so, us, pairs that share in brackets: Q4_K 128 experts
-// top-8 of 768 x 2048 with Q6_K down 35 -> 24 (0), 43 -> 27 (0.5), 56 -> 36 (3), 82 -> 63 (12), 96 -> 97 (27); 60 top-4 of 1792 x
-// 2816 33 -> 25 (0), 127 -> 117 (21), 142 -> 178 (44); 8 top-2 of 2048 x 2816 28 -> 20 (0), 50 -> 40 (9), 48 -> 49 (13); 32 top-4 of
-// 1024 x 2048 47 -> 37 (11), 53 -> 54 (23).  Q8_0, whose grouped form costs more: 60 top-4 of 1792 x 2816 36 -> 27 (0), 174 -> 159
-// (21), 221 -> 250 (44); 32 top-4 of 1024 x 2048 57 -> 43 (11), 80 -> 70 (36), 84 -> 86 (50); 8 top-2 of 2048 x 2816 51 -> 45 (9),
-// 59 -> 57 (13), 63 -> 66 (16: three pairs an expert, where the grouped form reads a sheet a third as often); Q6_K the same,
-// 128 experts top-8 of 768 x 2048 119 -> 114 (27), 155 -> 190 (92).
+// Whether a block's pairs go without grouping (moe_gather_ffn).  That saves two launches and the grouped kernels' setup, 13 us, and
+// reads a sheet again for every pair that shares its expert with another, but at 6.5 TB/s (from L2 and the memory-side cache where
+// it is read again) against the 3.65 that the grouped kernels make of a few columns a sheet; the rows' choices are taken as evenly
+// spread.  The whole block, grouped -> so, us, at pairs: Q4_K 128 experts top-8 of 768 x 2048 with Q6_K down 35 -> 22 (8), 56 -> 30
+// (32), 97 -> 79 (96), 122 -> 118 (192), 134 -> 163 (320: grouped); 60 top-4 of 1792 x 2816 33 -> 25 (4), 127 -> 98 (60), 142 -> 146
+// (92), 138 -> 162 (120: grouped); 8 top-2 of 2048 x 2816 28 -> 20 (2), 50 -> 36 (16), 49 -> 51 (24: grouped); 32 top-4 of 1024 x
+// 2048 47 -> 31 (32), 49 -> 44 (64), 49 -> 58 (80: grouped).  Q8_0 60 top-4 of 1792 x 2816 36 -> 27 (4), 174 -> 159 (60), 221 -> 250 (92:
+// grouped); 32 top-4 of 1024 x 2048, Q6_K down, 57 -> 41 (32), 80 -> 66 (64), 84 -> 99 (96: grouped).
 // Q4_K and Q6_K sheets under 512 x 512 keep the grouped form, whose launches a caller can count on there
 // (tests/test_gpu_moe.py), though they would gain as well.
-bool moe_gather_ffn_wanted(int type, int rows, int k_used, int n_expert, int n_ffn, int n_embd) {
-    const double pairs = (double)rows * k_used;
-    if (pairs > 256 || pairs > 2.5 * n_expert || (type != JL_TYPE_Q8_0 && (long)n_ffn * n_embd < 512L * 512)) return false;
+bool moe_gather_ffn_wanted(int type, int down_type, int rows, int k_used, int n_expert, int n_ffn, int n_embd) {
+    const double pairs = (double)rows * k_used, sheet = (double)n_ffn * n_embd;
+    if (pairs > 256 || (type != JL_TYPE_Q8_0 && sheet < 512.0 * 512.0)) return false;
+    const TypeInfo *t = type_info(type), *d = type_info(down_type);
+    const double mb = sheet * 1e-6 * (2.0 * t->block_bytes / t->block_elems + (double)d->block_bytes / d->block_elems);
     const double touched = n_expert * (1.0 - std::pow(1.0 - std::min(1.0, (double)k_used / n_expert), rows));
-    return pairs - touched <= (type == JL_TYPE_Q4_K ? 18 : 32);
+    return pairs * mb / 6.5 < 13.0 + touched * mb / 3.65;
 }
 
 // A routed block of a handful of pairs without its grouping and combine: the pairs themselves are the columns of gate + up,
@@ -1487,10 +1506,11 @@ int moe_gather_ffn(jl_ctx* c, float* resid, int type, int down_type, const void*
     if (rc != JL_OK) return rc;
     // (eight and four wavefronts a workgroup: the same at one row, 2 and 9 us slower at 32 pairs)
     a.nwaves = 16;
-    const long slots = (pair ? 2L : 1L) * c->num_cu, groups = (n_embd + 15) / 16;
+    const int lpr = gather_lanes(c, down_type, (int)row_slots * k_used, n_embd, rows), per_group = 16 * (64 / lpr);
+    const long slots = (pair ? 2L : 1L) * c->num_cu, groups = (n_embd + per_group - 1) / per_group;
     a.ngroups = (int)std::max(1L, std::min(groups, slots / rows));
     Name name;
-    name << "jl_moe_gather_" << (pair ? "q8_0p" : ti->tag) << "_down";
+    name << "jl_moe_gather_" << (pair ? "q8_0p" : ti->tag) << "_down_l" << lpr;
     void* params[] = {&a};
     return launch(c, name, (unsigned)a.ngroups, (unsigned)rows, 1024, (unsigned)lds, st, params);
 }
@@ -1578,7 +1598,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
         const bool align = sheet % (type == JL_TYPE_Q4_K ? 16 : 4) == 0;
         int form = c->tune.moe_form;
         if (q6 && !planes && c->act_window == 256 && (form == 3 || form == 4)) form += 2;   // (their Q6_K forms)
-        // A handful of columns: a decode matvec each (the whole block's us, as it was -> so).  Q4_K, 128 experts of 768 x 2048,
+        // A handful of columns: a decode matvec each (the whole block's us with both of its matvecs, as it was -> so, at 64 lanes a row).  Q4_K, 128 experts of 768 x 2048,
         // 8 / 16 / 24 columns 42 -> 33 / 44 -> 40 / 46 -> 49, 60 of 1792 x 2816, 4 / 16 / 32 / 48 columns 53 -> 32 / 71 -> 52 /
         // 94 -> 86 / 114 -> 127, 8 of 1024 x 1536, 2 / 16 / 24 columns 31 -> 22 / 38 -> 38 / 39 -> 47; Q6_K down projections the
         // same; Q8_0, whose other form costs an expert more: the first 8 / 64 / 96 columns 52 -> 34 / 109 -> 96 / 128 -> 138,
@@ -1923,7 +1943,8 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     names.push_back("jl_gemm_i8_prep");
     names.push_back("jl_moe_gemm_i8_prep");
     for (const char* tag : {"q4k", "q8_0", "q8_0p", "q6k"})
-        for (const char* act : {"", "_a", "_down"}) names.push_back(std::string("jl_moe_gather_") + tag + act);
+        for (const char* act : {"", "_a", "_down"})
+            for (const char* lpr : {"_l8", "_l16", "_l32", "_l64"}) names.push_back(std::string("jl_moe_gather_") + tag + act + lpr);
     for (const char* tag : {"q4k", "q4k_planes", "q6k"})
         for (const char* form : {"jl_moe_cols_", "jl_moe_cols_prep_"}) names.push_back(std::string(form) + tag);
     for (const char* tag : {"q8_0", "q4k", "q6k", "q6kw"})
@@ -2621,7 +2642,7 @@ int moe_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate_b
                        planes ? &d : nullptr, x, wt, rows, n_ffn, n_embd, g, u, y, st);
         if (rc != JL_DECLINED) return rc;
     }
-    if (!planes && (c->tune.moe_form == 11 || (c->tune.moe_form == 0 && moe_gather_ffn_wanted(type, rows, k_used, n_expert, n_ffn, n_embd)))) {
+    if (!planes && (c->tune.moe_form == 11 || (c->tune.moe_form == 0 && moe_gather_ffn_wanted(type, down_type, rows, k_used, n_expert, n_ffn, n_embd)))) {
         rc = moe_gather_ffn(c, resid, type, down_type, gate_bank, up_bank, down_bank, x, sel, sel_stride, wt, rows, k_used, n_expert, n_ffn,
                             n_embd, g, u, st);
         if (rc != JL_DECLINED) return rc;

@@ -347,10 +347,11 @@ extern "C" __global__ __launch_bounds__(512) void jl_moe_matvec_planes_q4k(MoePl
 }
 // a matvec a routed column: grid = (row groups, columns, matrices), block = 1024, dynamic LDS as jl_matvec_multi_*; the down
 // projections of a row's pairs: grid = (row groups, rows), block <= 1024, 128 bytes of LDS behind the staging area
-#define JL_MOE_GATHER(T, TYPE)                                                                                                    \
-    extern "C" __global__ __launch_bounds__(1024) void jl_moe_gather_##T(MoeGatherArgs p) { moe_gather_body<TYPE, 0>(p, jl_smem); } \
-    extern "C" __global__ __launch_bounds__(1024) void jl_moe_gather_##T##_a(MoeGatherArgs p) { moe_gather_body<TYPE, JL_PRE_ACT>(p, jl_smem); } \
-    extern "C" __global__ __launch_bounds__(1024) void jl_moe_gather_##T##_down(MoeGatherDownArgs p) { moe_gather_down_body<TYPE>(p, jl_smem); }
+#define JL_MOE_GATHER_L(T, TYPE, L)                                                                                                            \
+    extern "C" __global__ __launch_bounds__(1024) void jl_moe_gather_##T##_l##L(MoeGatherArgs p) { moe_gather_body<TYPE, 0, L>(p, jl_smem); }         \
+    extern "C" __global__ __launch_bounds__(1024) void jl_moe_gather_##T##_a_l##L(MoeGatherArgs p) { moe_gather_body<TYPE, JL_PRE_ACT, L>(p, jl_smem); } \
+    extern "C" __global__ __launch_bounds__(1024) void jl_moe_gather_##T##_down_l##L(MoeGatherDownArgs p) { moe_gather_down_body<TYPE, L>(p, jl_smem); }
+#define JL_MOE_GATHER(T, TYPE) JL_MOE_GATHER_L(T, TYPE, 8) JL_MOE_GATHER_L(T, TYPE, 16) JL_MOE_GATHER_L(T, TYPE, 32) JL_MOE_GATHER_L(T, TYPE, 64)
 JL_MOE_GATHER(q4k, JL_Q4_K) JL_MOE_GATHER(q8_0, JL_Q8_0) JL_MOE_GATHER(q8_0p, JL_Q8_0P) JL_MOE_GATHER(q6k, JL_Q6_KS)
 // experts of some tens of columns (kernels/moe_cols.h): prep grid = ceil(records * k/256 / 16); matrices: dynamic LDS = JL_MC_LDS_BYTES
 #define JL_MOE_COLS(T, KO)                                                                                                         \

@@ -1349,41 +1349,74 @@ __device__ __forceinline__ void moe_combine_body(const MoeCombineArgs& p, float*
 // ---------------------------------------------------------------- a column or two of a few experts
 // A decode matvec (kernels/matvec.h) for each routed column: its source row quantized in the workgroup, its expert's sheet
 // read once for it.  With hardly a column an expert that is every byte once, and there is no launch in front that quantizes.
-template <int TYPE, int PRE>
+// A row takes LPR lanes, a wavefront's step 64 / LPR rows.
+template <int TYPE, int PRE, int LPR>
 __device__ __forceinline__ void moe_gather_body(const MoeGatherArgs& args, uint8_t* smem) {
+    constexpr bool ACT = (PRE & JL_PRE_ACT) != 0;
+    constexpr int RPS = 64 / LPR;
+    typedef SlotTraits<TYPE> T;
     const u32 c = blockIdx.y;
-    const int mat = blockIdx.z, lane = threadIdx.x & 63;
-    MultiNow m;
-    m.out = args.out[mat]; m.w = args.bank[mat]; m.nrows = args.nrows; m.k = args.k; m.per = args.per; m.nwaves = args.nwaves;
-    m.ngroups = args.ngroups; m.row_bytes = args.row_bytes; m.type = 0; m.x = args.x; m.x2 = PRE & JL_PRE_ACT ? args.x2 : nullptr;
-    m.resid = nullptr; m.resid_gate = nullptr; m.alpha = 0.f; m.norm_w = nullptr; m.norm_out = nullptr; m.norm_eps = 0.f; m.inv_k = 0.0;
-    const u32 *src = args.src, *start = args.start, *sel = args.sel;
-    size_t sheet = args.sheet_bytes;
-    int n_expert = args.n_expert, ku = args.k_used, sel_stride = args.sel_stride;
-    JL_NOW(m.out, m.w, m.nrows, m.k, m.per, m.nwaves, m.ngroups, m.row_bytes, m.x, m.x2, src, start, sel, sheet, n_expert, ku, sel_stride);
-    src = as_global(src); start = as_global(start); sel = as_global(sel);
+    const int mat = blockIdx.z, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float* out = args.out[mat];
+    const uint8_t* w0 = args.bank[mat];
+    MoeGatherArgs p = args;
+    JL_NOW(out, w0, p.x, p.x2, p.src, p.start, p.sel, p.sheet_bytes, p.nrows, p.k, p.row_bytes, p.per, p.nwaves, p.ngroups, p.n_expert,
+           p.sel_stride, p.k_used);
+    const u32 *src = as_global(p.src), *start = as_global(p.start), *sel = as_global(p.sel);
+    const int nrows = p.nrows, k = p.k, nthreads = p.nwaves * 64, nslots = k / T::kElems;
     u32 row, e;
     if (!start) {
-        row = c / (u32)ku;
+        row = c / (u32)p.k_used;
         // (an id no expert has: its weight is none, see moe_gather_down_body)
-        e = min((u32)__builtin_amdgcn_readfirstlane((i32)sel[row * (u32)sel_stride + (c - row * (u32)ku)]), (u32)n_expert - 1u);
+        e = min((u32)__builtin_amdgcn_readfirstlane((i32)sel[row * (u32)p.sel_stride + (c - row * (u32)p.k_used)]), (u32)p.n_expert - 1u);
     } else {
         row = src ? (u32)__builtin_amdgcn_readfirstlane((i32)src[c]) : c;
         // the column's expert: the last whose first column is not past it
         u32 cnt = 0;
-        for (int base = 0; base <= n_expert; base += 64) {
+        for (int base = 0; base <= p.n_expert; base += 64) {
             const int idx = base + lane;
-            const u32 s = start[min(idx, n_expert)];
-            cnt += (u32)__builtin_popcountll(__ballot(idx <= n_expert && s <= c));
+            const u32 s = start[min(idx, p.n_expert)];
+            cnt += (u32)__builtin_popcountll(__ballot(idx <= p.n_expert && s <= c));
         }
         e = cnt - 1;
     }
-    m.out = as_global(m.out) + (size_t)c * m.nrows;
-    m.w = as_global(m.w) + (size_t)e * sheet;
-    m.x = as_global(m.x) + (size_t)row * m.k;
-    if constexpr ((PRE & JL_PRE_ACT) != 0) m.x2 = as_global(m.x2) + (size_t)row * m.k;
-    MatVecMultiArgs unused;
-    matvec_multi_body_xp<TYPE, 1, false, PRE>(unused, m, smem);
+    out = as_global(out) + (size_t)c * nrows;
+    w0 = as_global(w0) + (size_t)e * p.sheet_bytes;
+    const float *x = as_global(p.x) + (size_t)row * k, *x2 = ACT ? as_global(p.x2) + (size_t)row * k : nullptr;
+    const ActLds A = act_lds_views(smem, k);
+    const int n4 = k / 4, n4_pad = (n4 + 63) & ~63;
+    f32x4 x0[1], u0[1];
+    load_x_groups<1>(x, k, nthreads, x0);
+    if constexpr (ACT) load_x_groups<1>(x2, k, nthreads, u0);
+    __builtin_amdgcn_s_barrier();   // activation loads of the whole workgroup go out first
+    const int sub = lane / LPR, l = lane % LPR;
+    int r0 = (blockIdx.x * p.nwaves + wave) * RPS;
+    typename T::W w;
+    T::load_w(w0 + (size_t)min(r0 + sub, nrows - 1) * p.row_bytes, min(l, nslots - 1), w);
+    auto stage_group = [&](int g4, f32x4 v, f32x4 f) __attribute__((always_inline)) {
+        if constexpr (ACT) v = f32x4{silu_f32(v.x) * f.x, silu_f32(v.y) * f.y, silu_f32(v.z) * f.z, silu_f32(v.w) * f.w};
+        stage_quantize4<stage_layout_of(TYPE)>(smem, k, p.per, g4, v);
+    };
+    int g4 = threadIdx.x;
+    if (g4 < n4_pad) stage_group(g4, x0[0], u0[0]);
+    for (g4 += nthreads; g4 < n4_pad; g4 += nthreads)
+        stage_group(g4, ((const f32x4*)x)[min(g4, n4 - 1)], ACT ? ((const f32x4*)x2)[min(g4, n4 - 1)] : f32x4{0.f, 0.f, 0.f, 0.f});
+    lds_barrier();
+    bool preloaded = true;
+    for (; r0 < nrows; r0 += p.ngroups * p.nwaves * RPS) {   // (uniform: every row group of a wavefront takes part in its sums)
+        const uint8_t* wr = w0 + (size_t)min(r0 + sub, nrows - 1) * p.row_bytes;
+        float acc = 0.f;
+        for (int slot = l; slot < nslots; slot += LPR) {
+            if (!preloaded) T::load_w(wr, slot, w);
+            preloaded = false;
+            typename T::Act a;
+            T::load_act(A, slot, a);
+            acc += T::dot(w, slot, a);
+        }
+        preloaded = false;
+        const float t = group_sum<LPR>(acc);
+        if (l == LPR - 1 && r0 + sub < nrows) out[r0 + sub] = t;
+    }
 }
 
 // The down projections of a row's pairs and their weighted sum into the residual stream, one matvec a row: its K is the
@@ -1391,10 +1424,10 @@ __device__ __forceinline__ void moe_gather_body(const MoeGatherArgs& args, uint8
 // wt * (its slots of a pair).  Neither a column a pair is stored nor added up by a launch behind: one row through 128 experts of
 // 768 x 2048, top-8, Q6_K down: 8.2 us, and 3.6 of combine after it, and 4.1 of grouping in front of the pairs, are now one
 // launch (the whole block 35 -> 24 us).
-template <int TYPE>
+template <int TYPE, int LPR>
 __device__ __forceinline__ void moe_gather_down_body(const MoeGatherDownArgs& args, uint8_t* smem) {
     typedef SlotTraits<TYPE> T;
-    constexpr int XP = 2;
+    constexpr int XP = 2, RPS = 64 / LPR;
     MoeGatherDownArgs p = args;
     JL_NOW(p.resid, p.bank, p.g, p.u, p.sel, p.wt, p.sheet_bytes, p.slots_inv, p.nrows, p.k, p.row_bytes, p.per, p.nwaves, p.ngroups,
            p.n_expert, p.sel_stride, p.k_used);
@@ -1410,7 +1443,8 @@ __device__ __forceinline__ void moe_gather_down_body(const MoeGatherDownArgs& ar
     // behind the staging area: a pair's expert and its weight (an id no expert has: none)
     u32* se = (u32*)(smem + (((TYPE == JL_Q8_0P ? JL_ACT_LDS_BYTES_SHIFTED(k) : JL_ACT_LDS_BYTES(k)) + 15) & ~15));
     float* sw = (float*)(se + 16);
-    const int s0 = min(lane, nslots - 1), pair0 = (int)__umulhi((u32)s0, p.slots_inv);   // the lane's first slot and its pair
+    const int sub = lane / LPR, l = lane % LPR;
+    const int s0 = min(l, nslots - 1), pair0 = (int)__umulhi((u32)s0, p.slots_inv);   // the lane's first slot and its pair
     const u32 e0 = min(sel[pair0], last);
     const int mine = min((int)threadIdx.x, p.k_used - 1);
     const u32 em = sel[mine];
@@ -1421,9 +1455,9 @@ __device__ __forceinline__ void moe_gather_down_body(const MoeGatherDownArgs& ar
     load_x_groups<XP>(g, k, nthreads, x0);
     load_x_groups<XP>(u, k, nthreads, u0);
     __builtin_amdgcn_s_barrier();   // activation loads of the whole workgroup go out first
-    int r0 = blockIdx.x * p.nwaves + wave;
+    int r0 = (blockIdx.x * p.nwaves + wave) * RPS;
     typename T::W w;
-    T::load_w(bank + (size_t)e0 * p.sheet_bytes + (size_t)min(r0, nrows - 1) * p.row_bytes, s0 - pair0 * row_slots, w);
+    T::load_w(bank + (size_t)e0 * p.sheet_bytes + (size_t)min(r0 + sub, nrows - 1) * p.row_bytes, s0 - pair0 * row_slots, w);
     if ((int)threadIdx.x < p.k_used) {
         se[threadIdx.x] = min(em, last);
         sw[threadIdx.x] = em <= last ? wm : 0.f;
@@ -1440,20 +1474,21 @@ __device__ __forceinline__ void moe_gather_down_body(const MoeGatherDownArgs& ar
     lds_barrier();
 
     bool preloaded = true;
-    for (; r0 < nrows; r0 += p.ngroups * p.nwaves) {
-        const float base = resid[r0];
+    for (; r0 < nrows; r0 += p.ngroups * p.nwaves * RPS) {
+        const int r = min(r0 + sub, nrows - 1);
+        const float base = resid[r];
         float acc = 0.f;
-        for (int slot = lane; slot < nslots; slot += 64) {
+        for (int slot = l; slot < nslots; slot += LPR) {
             const int pair = (int)__umulhi((u32)slot, p.slots_inv), s = slot - pair * row_slots;
-            if (!preloaded) T::load_w(bank + (size_t)se[pair] * p.sheet_bytes + (size_t)r0 * p.row_bytes, s, w);
+            if (!preloaded) T::load_w(bank + (size_t)se[pair] * p.sheet_bytes + (size_t)r * p.row_bytes, s, w);
             preloaded = false;
             typename T::Act a;
             T::load_act(A, slot, a);
             acc = fmaf(sw[pair], T::dot(w, s, a), acc);
         }
         preloaded = false;
-        const float t = wave_sum_to_lane63(acc);
-        if (lane == 63) resid[r0] = base + t;
+        const float t = group_sum<LPR>(acc);
+        if (l == LPR - 1 && r0 + sub < nrows) resid[r] = base + t;
     }
 }
 

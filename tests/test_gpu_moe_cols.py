@@ -133,6 +133,10 @@ def test_a_matvec_a_column(dev, devbuf, t, window, nrows, k):
     (quant.Q8_0, quant.Q8_0, 32, 20, 16, 2, 256, 256, 0),       # sixteen pairs, the paired form
     (quant.Q8_0, quant.Q8_0, 32, 12, 4, 3, 1024, 768, 2),       # banks that are not on four bytes: the plain form
     (quant.Q8_0, quant.Q6_K, 32, 12, 5, 3, 768, 1024, 0),
+    (quant.Q4_K, quant.Q4_K, 256, 6, 4, 24, 768, 512, 0),       # eight lanes a row, several rows a step, the last step ragged
+    (quant.Q4_K, quant.Q6_K, 32, 6, 2, 40, 512, 1024, 0),       # sixteen and eight
+    (quant.Q4_K, quant.Q4_K, 256, 6, 2, 20, 1024, 2816, 0),     # sixteen lanes of three slots, the last without one for some
+    (quant.Q6_K, quant.Q8_0, 32, 6, 2, 20, 768, 2048, 0),       # 32
 ], ids=lambda v: str(v))
 def test_block_of_pairs(dev, devbuf, t, down, window, n_expert, k_used, rows, n_ffn, n_embd, pair):
     """The routed block without grouping and combine: a selection with a stride of its own, the first and the last expert
