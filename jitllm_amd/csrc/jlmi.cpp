@@ -52,6 +52,7 @@ struct Tuning {
     int moe_chunk = 0;
     int moe_waves = 0;
     int moe_lpr = 0;
+    int matvec_lanes = 0;
     int mx_rows = 0;
     int mx_scaled = 0;          // 1: packed MXFP4 matmul on the block-scaled fp8 x fp4 matrix instruction (lossy)
     int mx_planes = 0;          // packed MXFP4: 2 restores rows first; 64 / 32 / 16 rows a workgroup of the plane
@@ -388,6 +389,16 @@ int matvec_check(jl_ctx* c, int type, int nrows, int k, const TypeInfo** ti_out)
     return JL_OK;
 }
 
+// Lanes a row for the decode matvecs: a row of at most 32 (16) slots takes 32 (16) lanes of a wavefront, which then has two (four)
+// rows a step; the same sums in the same order (the lanes left out added zeros).  From eight rows a CU; below, the launch is
+// its ramp.  us, 64 lanes -> 32 -> 16, weights in turn: Q4_K 8192 x 1024 4.8 -> 3.4 -> 3.1 (the host's launch), 32768 x 1024 11.5 ->
+// 7.4 -> 5.5, 8192 x 2048 5.0 -> 4.2, 16384 x 2048 7.9 -> 5.9, 65536 x 2048 22.6 -> 15.5; Q6_K 8192 x 1024 5.8 -> 4.2 -> 3.5, 16384 x 2048
+// 10.2 -> 8.2; Q8_0 16384 x 1024 6.9 -> 5.3 -> 5.8, 65536 x 1024 20.9 -> 15.3 -> 14.4, 16384 x 2048 9.0 -> 8.6.
+int matvec_lanes(const jl_ctx* c, int slots, long rows) {
+    const int lanes = c->tune.matvec_lanes ? c->tune.matvec_lanes : rows <= 8L * c->num_cu ? 64 : slots <= 16 ? 16 : 32;
+    return slots <= lanes ? lanes : 64;
+}
+
 int matvec_launch(jl_ctx* c, float* out, int type, const void* w, const float* x, const int8_t* q,
                   const float* as, const float* s16, int nrows, int k, hipStream_t st, float* resid = nullptr,
                   float alpha = 0.f, const float* resid_gate = nullptr) {
@@ -401,9 +412,9 @@ int matvec_launch(jl_ctx* c, float* out, int type, const void* w, const float* x
     if (type == JL_TYPE_Q4_K && !aligned16(w)) return JL_DECLINED;
     if (((uintptr_t)w & 1) != 0) return JL_DECLINED;
 
-    // Shape choice, from sweeps on MI355X: one row per wavefront.  At most sixteen rows a CU: one workgroup a CU of as
+    // Shape choice, from sweeps on MI355X: one row (or step of rows) per wavefront.  At most sixteen a CU: one workgroup a CU of as
     // many wavefronts as it has rows, eight at least (the workgroup quantizes x; Q4_K 1500 x 13312 on eight 6.9 us, on
-    // sixteen 7.8; 3000 x 11008 on twelve 6.2 and 6.6).  Taller ones: a persistent grid over the row groups with
+    // sixteen 7.8; 3000 x 11008 on twelve 6.2 and 6.6; 6144 x 2048 two rows a step, 4.1 as two workgroups a CU, so 3.3).  Taller ones: a persistent grid over the row groups with
     // sixteen wavefronts a CU for the k-quants, whose registers leave room for no more (a second round of workgroups
     // quantizes x again: Q6_K 10822 x 768 7.0 us -> 5.6, 14336 x 4096 10.2 -> 8.6), as two workgroups of eight, which
     // cover each other's barriers (9988 x 5120 Q6_K 9.4 against 10.3 as one; 6000 x 4096 Q4_K 4.5 and 4.5);
@@ -416,14 +427,19 @@ int matvec_launch(jl_ctx* c, float* out, int type, const void* w, const float* x
     if (rpw <= 0 || resid || !x) rpw = 1;   // (the kernels with the residual add or a quantized activation: one row a wavefront)
     if (rpw != 1 && rpw != 2 && rpw != 4) return fail(c, JL_ERR_ARG, "matvec: rpw=%d", rpw);
     const bool pair = q8_pair_form(c, type, w, k);
-    const bool small = nrows <= 16 * c->num_cu;
+    const int slots = k / (type == JL_TYPE_Q8_0 && !pair ? 32 : 64);
+    int lanes = rpw == 1 && x && !resid ? matvec_lanes(c, slots, nrows) : 64;
+    const int steps = (nrows + 64 / lanes - 1) / (64 / lanes);   // of a wavefront, all rows
+    const bool small = steps <= 16 * c->num_cu;
     const bool one_per_cu = small || (type == JL_TYPE_Q8_0 && pair && nrows <= 32 * c->num_cu && k >= 4096);
     if (block <= 0)
-        block = small ? 64 * std::max(8, (nrows + c->num_cu - 1) / c->num_cu) : one_per_cu ? 1024 :
+        block = small ? 64 * std::max(8, (steps + c->num_cu - 1) / c->num_cu) : one_per_cu ? 1024 :
                 type == JL_TYPE_Q8_0 && !(pair && nrows >= 40 * c->num_cu && k >= 3584 && k <= 5120) ? 768 : 512;
     if (block % 64 != 0 || block > 1024) return fail(c, JL_ERR_ARG, "matvec: block=%d", block);
     if (block > matvec_max_block(type, rpw, pair)) block = matvec_max_block(type, rpw, pair);
-    const int rows_per_block = (block / 64) * rpw;
+    const int xpre = x_groups(c, k, block);
+    if (xpre != 1) lanes = 64;   // (a tuned workgroup: rows that short are one group a thread otherwise)
+    const int rows_per_block = (block / 64) * rpw * (64 / lanes);
     long groups = ((long)nrows + rows_per_block - 1) / rows_per_block;
     long grid = c->tune.grid > 0 ? c->tune.grid : (long)c->num_cu * (one_per_cu && rpw == 1 ? 1 : 2);
     if (grid > groups) grid = groups;
@@ -443,9 +459,9 @@ int matvec_launch(jl_ctx* c, float* out, int type, const void* w, const float* x
     a.nwaves = block / 64;
     a.ngroups = (int)grid;
     a.resid = resid; a.alpha = alpha; a.resid_gate = resid ? resid_gate : nullptr;
-    const int xpre = x_groups(c, k, block);
     Name name;
     name << "jl_matvec_" << (pair ? "q8_0p" : ti->tag) << "_r" << rpw << (!x ? "_pq" : xpre == 4 ? "_x4" : xpre == 2 ? "_x2" : "") << (resid ? "_res" : "");
+    if (lanes != 64) name << "_l" << lanes;
     void* params[] = {&a};
     unsigned lds = (unsigned)(act_lds_bytes(k) + (pair ? (size_t)k + 16 : 0));
     return launch(c, name, (unsigned)grid, 1, (unsigned)block, lds, st, params);
@@ -493,17 +509,27 @@ int matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, const vo
     // workgroups stages (norms, gates) the activation once more (us, with 512 workgroups for every type -> now:
     // gate + up with a norm in front Q4_K 2048 / 7168 7.9 -> 6.7, 4096 / 14336 13.0 -> 12.3, Q6_K 1536 / 4608 9.6 -> 7.1;
     // q + k + v of a 4096 k-quant block 8.2 -> 6.1); never more row groups than a matrix has.
-    const int nwaves = 16;
+    const int nwaves = 16, xpre = x_groups(c, k, nwaves * 64);
+    int lanes = 64;
+    if (!x2 && !resid && (types || xpre == 1) && (m > 1 || types || norm_w)) {
+        long total = 0;
+        bool plain8 = false;   // (the mixed-type kernel reads Q8_0 rows a block a slot)
+        for (int i = 0; i < m; i++) {
+            total += rows[i];
+            plain8 |= (types ? types[i] : type) == JL_TYPE_Q8_0 && !pair;
+        }
+        lanes = matvec_lanes(c, k / (plain8 ? 32 : 64), total);
+    }
+    const int step = nwaves * (64 / lanes);
     const long slots = c->tune.grid > 0 ? c->tune.grid : (pair ? 2L : 1L) * c->num_cu;
-    long lo = 1, gx = ((long)max_rows + nwaves - 1) / nwaves;
+    long lo = 1, gx = ((long)max_rows + step - 1) / step;
     while (lo < gx) {   // the largest gx whose workgroups with work are at most `slots`
         const long mid = (lo + gx + 1) / 2;
         long n = 0;
-        for (int i = 0; i < m; i++) n += std::min(mid, ((long)rows[i] + nwaves - 1) / nwaves);
+        for (int i = 0; i < m; i++) n += std::min(mid, ((long)rows[i] + step - 1) / step);
         if (n <= slots) lo = mid; else gx = mid - 1;
     }
     a.nwaves = nwaves; a.ngroups = (int)gx;
-    const int xpre = x_groups(c, k, nwaves * 64);
     Name name;
     // "matvec.act_split" = 1: a gated activation shared by the group's matrices is formed and
     // quantized once, by the quantizer kernel, and the matvec stages the int8 copy (the same
@@ -552,6 +578,7 @@ int matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, const vo
     if (types) name << "jl_matvec_segments";
     else name << "jl_matvec_multi_" << (pair ? "q8_0p" : ti->tag);
     name << (norm_w ? x2 ? "_na" : "_n" : x2 ? "_a" : "") << (types || xpre == 1 ? "" : xpre == 4 ? "_x4" : "_x2") << (resid ? "_res" : "");
+    if (lanes != 64) name << "_l" << lanes;
     void* params[] = {&a};
     // (+ 16 to round the staging area up, + JL_NORM_LDS_BYTES for the RMSNorm's partial sums)
     unsigned lds = (unsigned)(act_lds_bytes(k) + (pair ? (size_t)k + 16 : 0) + 16 + 160);
@@ -1977,6 +2004,14 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     for (int rpw : {1, 2, 4})
         for (const char* xp : {"_x2", "_x4"}) names.push_back("jl_matvec_q8_0p_r" + std::to_string(rpw) + xp);
     for (const char* tag : {"q4k", "q8_0", "q6k", "q8_0p"}) names.push_back(std::string("jl_matvec_") + tag + "_r1_x2_res");
+    for (const char* lanes : {"_l32", "_l16"}) {
+        for (const char* tag : {"q4k", "q8_0", "q6k", "q8_0p"})
+            for (const char* form : {"jl_matvec_%s_r1", "jl_matvec_multi_%s", "jl_matvec_multi_%s_n"}) {
+                std::string n(form);
+                names.push_back(n.replace(n.find("%s"), 2, tag) + lanes);
+            }
+        for (const char* pre : {"", "_n"}) names.push_back(std::string("jl_matvec_segments") + pre + lanes);
+    }
     for (const char* tag : {"q4k", "q8_0", "q6k", "q8_0p"}) {
         for (const char* res : {"", "_res"}) {
             for (const char* pre : {"", "_n", "_a", "_na"})
@@ -2097,6 +2132,7 @@ int jl_set_tuning(jl_ctx* c, const char* key, int value) {
     else if (!strcmp(key, "moe.group16")) c->tune.moe_g16 = value;
     else if (!strcmp(key, "moe.chunk")) c->tune.moe_chunk = value;
     else if (!strcmp(key, "moe.waves")) c->tune.moe_waves = value;
+    else if (!strcmp(key, "matvec.lanes")) c->tune.matvec_lanes = value;
     else if (!strcmp(key, "moe.lpr")) c->tune.moe_lpr = value;
     else if (!strcmp(key, "gemm.rows")) c->tune.gemm_rows = value;
     else if (!strcmp(key, "mxfp4.split")) c->tune.mx_split = value;

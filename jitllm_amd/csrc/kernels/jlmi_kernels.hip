@@ -128,6 +128,28 @@ JL_MATVEC_SEGMENTS(, 0, , false) JL_MATVEC_SEGMENTS(_n, JL_PRE_NORM, , false) JL
 JL_MATVEC_SEGMENTS(_na, JL_PRE_NORM | JL_PRE_ACT, , false) JL_MATVEC_SEGMENTS(, 0, _res, true) JL_MATVEC_SEGMENTS(_n, JL_PRE_NORM, _res, true)
 JL_MATVEC_SEGMENTS(_a, JL_PRE_ACT, _res, true) JL_MATVEC_SEGMENTS(_na, JL_PRE_NORM | JL_PRE_ACT, _res, true)
 
+// The same with 32 or 16 lanes a row, for rows of at most that many slots
+#define JL_MATVEC_LANES(T, TYPE, L)                                                                                \
+    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_##T##_r1_l##L(MatVecArgs p) {                     \
+        matvec_body<TYPE, 1, 1, false, false, L>(p, jl_smem);                                                      \
+    }                                                                                                              \
+    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_multi_##T##_l##L(MatVecMultiArgs p) {             \
+        matvec_multi_body<TYPE, 1, false, 0, L>(p, jl_smem);                                                       \
+    }                                                                                                              \
+    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_multi_##T##_n_l##L(MatVecMultiArgs p) {           \
+        matvec_multi_body<TYPE, 1, false, JL_PRE_NORM, L>(p, jl_smem);                                             \
+    }
+#define JL_MATVEC_LANES_TYPES(L)                                                                                   \
+    JL_MATVEC_LANES(q4k, JL_Q4_K, L) JL_MATVEC_LANES(q8_0, JL_Q8_0, L) JL_MATVEC_LANES(q6k, JL_Q6_KS, L)           \
+    JL_MATVEC_LANES(q8_0p, JL_Q8_0P, L)                                                                            \
+    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_segments_l##L(MatVecMultiArgs p) {                \
+        matvec_segments_body<false, 0, L>(p, jl_smem);                                                             \
+    }                                                                                                              \
+    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_segments_n_l##L(MatVecMultiArgs p) {              \
+        matvec_segments_body<false, JL_PRE_NORM, L>(p, jl_smem);                                                   \
+    }
+JL_MATVEC_LANES_TYPES(32) JL_MATVEC_LANES_TYPES(16)
+
 // -------------------------------------------------- few tokens, int8 matrix cores
 extern "C" __global__ __launch_bounds__(256) void jl_few_prep(FewI8PrepArgs p) { few_i8_prep_body(p); }
 // jl_few_<type>_<rows | planes>_t<token tiles>r<row tiles>: grid = (row tiles, experts, matrices)

@@ -531,6 +531,19 @@ template <> struct SlotTraits<JL_Q6_K> {
 };
 
 
+// Sum over the LPR consecutive lanes of a row group (LPR = 4 to 64); the
+// total is valid in the group's last lane.
+template <int LPR>
+__device__ __forceinline__ float group_sum(float v) {
+    v += dpp_f32<JL_DPP_QUAD_XOR1, 0xf>(v);
+    v += dpp_f32<JL_DPP_QUAD_XOR2, 0xf>(v);
+    if (LPR >= 8) v += dpp_f32<JL_DPP_ROW_HALF_MIRROR, 0xf>(v);
+    if (LPR >= 16) v += dpp_f32<JL_DPP_ROW_MIRROR, 0xf>(v);
+    if (LPR >= 32) v += dpp_f32<JL_DPP_ROW_BCAST15, 0xa>(v);
+    if (LPR >= 64) v += dpp_f32<JL_DPP_ROW_BCAST31, 0xc>(v);
+    return v;
+}
+
 // The row loop of one wavefront: rows r0, r0 + group_stride, ... (RPW at a time), each row's
 // slots dealt to the lanes in chunks of 64.  w holds the first step's weights, loaded by the
 // caller before the activation was staged; every later step's loads are issued when the step
@@ -543,23 +556,28 @@ template <> struct SlotTraits<JL_Q6_K> {
 // 14.7 with the loads' issue order pinned and the waits checked in the assembly (15, 10, 5, 0
 // loads left in flight before the four dot products): a CU returns its loads in the order they
 // were issued, so the last wavefront's first chunk arrives behind the first wavefront's last.)
-// store(row, total) receives a finished row in lane 63; store.begin(row) is called when the row's work starts.
-template <int TYPE, int RPW, class Store>
+// store(row, total) receives a finished row in its last lane; store.begin(row) is called when the row's work starts.
+// LPR: lanes a row.  A row of K <= 2048 has 32 slots at most and left half of a wavefront without loads: two (four) rows
+// a step there, the same sums (a lane without a slot adds zero).
+template <int TYPE, int RPW, int LPR = 64, class Store>
 __device__ __forceinline__ void matvec_rows(const uint8_t* w0, int row_bytes, const ActLds& A, int nrows, int r0,
                                             int group_stride, int nslots, int lane,
                                             typename SlotTraits<TYPE>::W (&w)[RPW], Store& store) {
     typedef SlotTraits<TYPE> T;
+    static_assert(RPW == 1 || LPR == 64, "several rows a step: by lanes or by registers");
+    const int sub = LPR == 64 ? 0 : lane / LPR, l = LPR == 64 ? lane : lane % LPR;
     float acc[RPW];
 #pragma unroll
     for (int j = 0; j < RPW; j++) acc[j] = 0.f;
     bool preloaded = true;
-    for (; r0 < nrows; r0 += group_stride) {
-        store.begin(r0);
-        for (int slot = lane; slot < nslots; slot += 64) {
+    for (; r0 < nrows; r0 += group_stride) {   // (uniform)
+        const int r = LPR == 64 ? r0 : min(r0 + sub, nrows - 1);
+        store.begin(r);
+        for (int slot = l; slot < nslots; slot += LPR) {
             if (!preloaded) {
 #pragma unroll
                 for (int j = 0; j < RPW; j++)
-                    T::load_w(w0 + (size_t)min(r0 + j, nrows - 1) * row_bytes, slot, w[j]);
+                    T::load_w(w0 + (size_t)min(r + j, nrows - 1) * row_bytes, slot, w[j]);
             }
             preloaded = false;
             typename T::Act a;
@@ -570,8 +588,8 @@ __device__ __forceinline__ void matvec_rows(const uint8_t* w0, int row_bytes, co
         preloaded = false;
 #pragma unroll
         for (int j = 0; j < RPW; j++) {
-            const float t = wave_sum_to_lane63(acc[j]);
-            if (lane == 63 && r0 + j < nrows) store(r0 + j, t);
+            const float t = group_sum<LPR>(acc[j]);
+            if (l == LPR - 1 && r0 + sub + j < nrows) store(r + j, t);
             acc[j] = 0.f;
         }
     }
@@ -611,15 +629,15 @@ struct StoreRowsRes {
 // gate's f64 exponential compiled into the plain kernel behind a branch, the plain matvecs ran
 // 10-20 % slower, Q8_0 14336 x 4096 14.2 against 11.8 us).
 // PQ: the activation comes quantized (MatVecArgs.q / as / s16) and is only copied into LDS.
-template <int TYPE, int RPW, int XP, bool RES, bool PQ>
+template <int TYPE, int RPW, int XP, bool RES, bool PQ, int LPR = 64>
 __device__ __forceinline__ void matvec_body_xp(const MatVecArgs& p, uint8_t* smem) {
     typedef SlotTraits<TYPE> T;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = p.nwaves;
     const int nslots = p.k / T::kElems;
-    const int rows_per_block = nwaves * RPW;
+    const int rows_per_block = nwaves * RPW * (64 / LPR), sub = LPR == 64 ? 0 : lane / LPR;
     const int group_stride = p.ngroups * rows_per_block;
     const ActLds A = act_lds_views(smem, p.k);
-    int r0 = blockIdx.x * rows_per_block + wave * RPW;
+    int r0 = blockIdx.x * rows_per_block + wave * RPW * (64 / LPR);
 
     // The activation loads go first, for the whole workgroup: a CU serves its vector
     // loads in the order they were issued whichever wavefront issued them, so every
@@ -636,10 +654,10 @@ __device__ __forceinline__ void matvec_body_xp(const MatVecArgs& p, uint8_t* sme
 
     typename T::W w[RPW];
     {
-        const int s = min(lane, nslots - 1);
+        const int s = min(LPR == 64 ? lane : lane % LPR, nslots - 1);
 #pragma unroll
         for (int j = 0; j < RPW; j++)
-            T::load_w(p.w + (size_t)min(r0 + j, p.nrows - 1) * p.row_bytes, s, w[j]);
+            T::load_w(p.w + (size_t)min(r0 + sub + j, p.nrows - 1) * p.row_bytes, s, w[j]);
     }
     constexpr int SH = stage_layout_of(TYPE);
     if constexpr (!PQ) stage_act_quantize<SH, XP>(smem, p.x, p.k, p.per, x0, nwaves * 64);
@@ -648,18 +666,18 @@ __device__ __forceinline__ void matvec_body_xp(const MatVecArgs& p, uint8_t* sme
 
     if constexpr (RES) {
         StoreRowsRes store{p.out, p.resid, resid_weight(p.alpha, p.resid_gate)};
-        matvec_rows<TYPE, RPW>(p.w, p.row_bytes, A, p.nrows, r0, group_stride, nslots, lane, w, store);
+        matvec_rows<TYPE, RPW, LPR>(p.w, p.row_bytes, A, p.nrows, r0, group_stride, nslots, lane, w, store);
     } else {
         StoreRows store{p.out};
-        matvec_rows<TYPE, RPW>(p.w, p.row_bytes, A, p.nrows, r0, group_stride, nslots, lane, w, store);
+        matvec_rows<TYPE, RPW, LPR>(p.w, p.row_bytes, A, p.nrows, r0, group_stride, nslots, lane, w, store);
     }
 }
 
 // XP = 1: a vector of at most one float4 group a thread; 4: longer ones (the host picks the
 // entry point; one body compiled for both behind a branch ran the short-vector case 10 % slower).
-template <int TYPE, int RPW, int XP = 1, bool RES = false, bool PQ = false>
+template <int TYPE, int RPW, int XP = 1, bool RES = false, bool PQ = false, int LPR = 64>
 __device__ __forceinline__ void matvec_body(const MatVecArgs& p, uint8_t* smem) {
-    matvec_body_xp<TYPE, RPW, XP, RES, PQ>(p, smem);
+    matvec_body_xp<TYPE, RPW, XP, RES, PQ, LPR>(p, smem);
 }
 
 // f64 sums over lanes by lane moves that cost a vector instruction each (a shuffle through LDS is a
@@ -770,7 +788,7 @@ __device__ __forceinline__ MultiNow multi_now(const MatVecMultiArgs& p) {
     return m;
 }
 
-template <int TYPE, int XP, bool RES, int PRE>
+template <int TYPE, int XP, bool RES, int PRE, int LPR = 64>
 __device__ __forceinline__ void matvec_multi_body_xp(const MatVecMultiArgs& q, const MultiNow& p, uint8_t* smem) {
     constexpr bool NORM = (PRE & JL_PRE_NORM) != 0, ACT = (PRE & JL_PRE_ACT) != 0;
     typedef SlotTraits<TYPE> T;
@@ -779,10 +797,11 @@ __device__ __forceinline__ void matvec_multi_body_xp(const MatVecMultiArgs& q, c
     const int nthreads = nwaves * 64;
     const int nrows = p.nrows, row_bytes = p.row_bytes;
     const int nslots = p.k / T::kElems;
-    const int group_stride = p.ngroups * nwaves;
+    constexpr int RPS = 64 / LPR;   // rows a step
+    const int group_stride = p.ngroups * nwaves * RPS, sub = LPR == 64 ? 0 : lane / LPR;
     const ActLds A = act_lds_views(smem, p.k);
-    int r0 = blockIdx.x * nwaves + wave;
-    if ((int)blockIdx.x * nwaves >= nrows) return;   // uniform: this matrix has fewer row groups
+    int r0 = (blockIdx.x * nwaves + wave) * RPS;
+    if ((int)blockIdx.x * nwaves * RPS >= nrows) return;   // uniform: this matrix has fewer row groups
     const uint8_t* w0 = p.w;
     if constexpr (XP == 0) {
         typename T::W w[1];
@@ -808,7 +827,7 @@ __device__ __forceinline__ void matvec_multi_body_xp(const MatVecMultiArgs& q, c
     if constexpr (NORM) load_x_groups<XP>(p.norm_w, p.k, nthreads, nw0);
     __builtin_amdgcn_s_barrier();   // activation loads of the whole workgroup go out first
     typename T::W w[1];
-    T::load_w(w0 + (size_t)min(r0, nrows - 1) * row_bytes, min(lane, nslots - 1), w[0]);
+    T::load_w(w0 + (size_t)min(r0 + sub, nrows - 1) * row_bytes, min(LPR == 64 ? lane : lane % LPR, nslots - 1), w[0]);
     // RMSNorm ahead of the quantizer (the reference's RMSNormQuantRows, jit/gpu/kernels/
     // elem.go:252-267): the sum of squares in f64, scale = 1/sqrt(sum/k + eps), y = f32(f64(x) *
     // f64(w) * scale).  The reference's host form (internal/oracle/oracle.go:230-240) is f32(f64(x) *
@@ -860,25 +879,25 @@ __device__ __forceinline__ void matvec_multi_body_xp(const MatVecMultiArgs& q, c
     // a gated activation in front, measured slower: gate + up 26.2 -> 32.8 us, down 14.5 -> 16.9)
     if constexpr (RES) {
         StoreRowsRes store{outp, y == 0 ? p.resid : nullptr, resid_weight(p.alpha, p.resid_gate)};
-        matvec_rows<TYPE, 1>(w0, row_bytes, A, nrows, r0, group_stride, nslots, lane, w, store);
+        matvec_rows<TYPE, 1, LPR>(w0, row_bytes, A, nrows, r0, group_stride, nslots, lane, w, store);
     } else {
         StoreRows store{outp};
-        matvec_rows<TYPE, 1>(w0, row_bytes, A, nrows, r0, group_stride, nslots, lane, w, store);
+        matvec_rows<TYPE, 1, LPR>(w0, row_bytes, A, nrows, r0, group_stride, nslots, lane, w, store);
     }
     }
 }
 
-template <int TYPE, int XP = 1, bool RES = true, int PRE = 0>
+template <int TYPE, int XP = 1, bool RES = true, int PRE = 0, int LPR = 64>
 __device__ __forceinline__ void matvec_multi_body(const MatVecMultiArgs& p, uint8_t* smem) {
-    matvec_multi_body_xp<TYPE, XP, RES, PRE>(p, multi_now<RES, PRE, false>(p), smem);
+    matvec_multi_body_xp<TYPE, XP, RES, PRE, LPR>(p, multi_now<RES, PRE, false>(p), smem);
 }
 // Matrices of different types: the type is uniform per workgroup, so the switch is a scalar branch.
-template <bool RES, int PRE>
+template <bool RES, int PRE, int LPR = 64>
 __device__ __forceinline__ void matvec_segments_body(const MatVecMultiArgs& p, uint8_t* smem) {
     const MultiNow m = multi_now<RES, PRE, true>(p);
     switch (m.type) {
-    case JL_Q4_K: matvec_multi_body_xp<JL_Q4_K, 1, RES, PRE>(p, m, smem); break;
-    case JL_Q8_0: matvec_multi_body_xp<JL_Q8_0, 1, RES, PRE>(p, m, smem); break;
-    case JL_Q6_K: matvec_multi_body_xp<JL_Q6_KS, 1, RES, PRE>(p, m, smem); break;
+    case JL_Q4_K: matvec_multi_body_xp<JL_Q4_K, 1, RES, PRE, LPR>(p, m, smem); break;
+    case JL_Q8_0: matvec_multi_body_xp<JL_Q8_0, 1, RES, PRE, LPR>(p, m, smem); break;
+    case JL_Q6_K: matvec_multi_body_xp<JL_Q6_KS, 1, RES, PRE, LPR>(p, m, smem); break;
     }
 }

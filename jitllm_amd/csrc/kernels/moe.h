@@ -334,19 +334,6 @@ __device__ __forceinline__ void moe_group2_body(const MoeGroupArgs& p, uint8_t* 
     }
 }
 
-// Sum over the LPR consecutive lanes of a row group (LPR = 16, 32 or 64); the
-// total is valid in the group's last lane.
-template <int LPR>
-__device__ __forceinline__ float group_sum(float v) {
-    v += dpp_f32<JL_DPP_QUAD_XOR1, 0xf>(v);
-    v += dpp_f32<JL_DPP_QUAD_XOR2, 0xf>(v);
-    if (LPR >= 8) v += dpp_f32<JL_DPP_ROW_HALF_MIRROR, 0xf>(v);
-    if (LPR >= 16) v += dpp_f32<JL_DPP_ROW_MIRROR, 0xf>(v);
-    if (LPR >= 32) v += dpp_f32<JL_DPP_ROW_BCAST15, 0xa>(v);
-    if (LPR >= 64) v += dpp_f32<JL_DPP_ROW_BCAST31, 0xc>(v);
-    return v;
-}
-
 // ------------------------------------------------- grouped matvec, packed planes
 // The dot-product form over banks of packed planes, for a handful of columns an expert (a small
 // prefill batch through a mixture: 64 rows top-8 of 128 experts is four columns an expert).

@@ -227,3 +227,46 @@ def test_shared_expert_add_gated_by_a_device_logit(dev, devbuf, layout):
     # the device's f64 exp may differ from numpy's in its last bit, which can move the f32 weight by one ulp
     assert np.max(np.abs(got - want)) <= 2.0 ** -22 * np.max(np.abs(yh))
     dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("k", [32, 512, 1024, 1088, 1536, 2048])
+@pytest.mark.parametrize("t", [quant.Q4_K, quant.Q6_K, quant.Q8_0], ids=["q4_k", "q6_k", "q8_0"])
+def test_short_rows_on_part_of_the_lanes(dev, devbuf, t, k):
+    """Rows of at most 32 (16) slots take 32 (16) lanes, two (four) of them a step: the bits of a row a wavefront, for a row
+    count that leaves the last step ragged, fewer rows than a step, one matrix and several, a norm in front, mixed types."""
+    if t != quant.Q8_0 and k % 256:
+        pytest.skip("k-quants: whole super-blocks")
+    window = 32
+    dev.SetActWindow(window)
+    rows = [2051, 1, 67]
+    ws = [synth.quantized_weights(t, r, k, seed=40 + i) for i, r in enumerate(rows)]
+    x, nw = synth.activations(k, seed=3), np.linspace(0.5, 1.5, k, dtype=np.float32)
+    dws, dx, dnw = [devbuf(w) for w in ws], devbuf(x), devbuf(nw)
+    other = quant.Q8_0 if t != quant.Q8_0 else quant.Q4_K if k % 256 == 0 else None
+    got = {}
+    try:
+        for lanes in (64, 32, 16, 0):
+            dev.set_tuning(lanes=lanes)
+            res = []
+            for r, w in zip(rows, dws):
+                o = devbuf(shape=(r + 4,), dtype=np.float32, fill=np.float32(6e30))
+                assert dev.matvec_dev(o.ptr, t, w.ptr, dx.ptr, r, k)
+                res.append(o)
+            types = [[t] * 3] + ([[t, t, other]] if other else [])
+            for ty in types:
+                hold = [devbuf(synth.quantized_weights(q, r, k, seed=40 + i)) for i, (q, r) in enumerate(zip(ty, rows))]
+                for norm in (None, dnw.ptr):
+                    outs = [devbuf(shape=(r + 4,), dtype=np.float32, fill=np.float32(6e30)) for r in rows]
+                    assert dev.matvec_group_dev([o.ptr for o in outs], ty, [h.ptr for h in hold], rows, dx.ptr, k, norm_w=norm, norm_eps=1e-5)
+                    dev.synchronize()
+                    res += outs
+            dev.synchronize()
+            got[lanes] = [o.get() for o in res]
+    finally:
+        dev.set_tuning(lanes=0)
+    for i, r in enumerate(rows):
+        if r > 1:   # (one row alone can be a sum that cancels: its error is bounded against its terms, not its value; its bits below)
+            assert nmse(got[64][i][:r], _want(t, ws[i], x, r, k, window)) <= 1e-10
+    for lanes in (32, 16, 0):
+        for i, (a, b) in enumerate(zip(got[lanes], got[64])):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (lanes, i)
