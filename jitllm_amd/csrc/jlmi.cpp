@@ -1498,11 +1498,13 @@ int moe_gather_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
 // (92), 138 -> 162 (120: grouped); 8 top-2 of 2048 x 2816 28 -> 20 (2), 50 -> 36 (16), 49 -> 51 (24: grouped); 32 top-4 of 1024 x
 // 2048 47 -> 31 (32), 49 -> 44 (64), 49 -> 58 (80: grouped).  Q8_0 60 top-4 of 1792 x 2816 36 -> 27 (4), 174 -> 159 (60), 221 -> 250 (92:
 // grouped); 32 top-4 of 1024 x 2048, Q6_K down, 57 -> 41 (32), 80 -> 66 (64), 84 -> 99 (96: grouped).
-// Q4_K and Q6_K sheets under 512 x 512 keep the grouped form, whose launches a caller can count on there
+// Over planes (Q4_K) 128 top-8 of 768 x 2048 36 -> 21 (8), 63 -> 44 (64), 83 -> 68 (128), 108 -> 108 (256: grouped); 60 top-4 of 1792 x
+// 2816 39 -> 24 (4), 108 -> 100 (64), 143 -> 171 (128: grouped); 8 top-2 of 1024 x 1536 30 -> 16 (2), 42 -> 29 (32).
+// Q4_K and Q6_K rows of sheets under 512 x 512 keep the grouped form, whose launches a caller can count on there
 // (tests/test_gpu_moe.py), though they would gain as well.
-bool moe_gather_ffn_wanted(int type, int down_type, int rows, int k_used, int n_expert, int n_ffn, int n_embd) {
+bool moe_gather_ffn_wanted(int type, int down_type, bool planes, int rows, int k_used, int n_expert, int n_ffn, int n_embd) {
     const double pairs = (double)rows * k_used, sheet = (double)n_ffn * n_embd;
-    if (pairs > 256 || (type != JL_TYPE_Q8_0 && sheet < 512.0 * 512.0)) return false;
+    if (pairs > 256 || (!planes && type != JL_TYPE_Q8_0 && sheet < 512.0 * 512.0)) return false;
     const TypeInfo *t = type_info(type), *d = type_info(down_type);
     const double mb = sheet * 1e-6 * (2.0 * t->block_bytes / t->block_elems + (double)d->block_bytes / d->block_elems);
     const double touched = n_expert * (1.0 - std::pow(1.0 - std::min(1.0, (double)k_used / n_expert), rows));
@@ -1540,6 +1542,45 @@ int moe_gather_ffn(jl_ctx* c, float* resid, int type, int down_type, const void*
     name << "jl_moe_gather_" << (pair ? "q8_0p" : ti->tag) << "_down_l" << lpr;
     void* params[] = {&a};
     return launch(c, name, (unsigned)a.ngroups, (unsigned)rows, 1024, (unsigned)lds, st, params);
+}
+
+// The same over packed planes.  Rows a workgroup and its wavefronts as the packed matvecs have them (other widths and eight against
+// sixteen wavefronts: within 4 % at 8 to 128 pairs, sixteen-row runs from 32 pairs up to 40 % slower).
+int moe_planes_gather_ffn(jl_ctx* c, float* resid, const jl_packed_bank* pg, const jl_packed_bank* pu, const jl_packed_bank* pd, const float* x,
+                          const uint32_t* sel, int sel_stride, const float* wt, int rows, int k_used, int n_expert, int n_ffn, int n_embd,
+                          float* g, float* u, hipStream_t st) {
+    if (k_used > 16 || (long)rows * k_used > 65535 || (long)k_used * n_ffn > (1L << 24)) return JL_DECLINED;
+    auto width = [&](int nrows, long matvecs) {   // rows a workgroup: the widest run that still gives three CUs in four a workgroup
+        int rw = c->tune.packed_rw;
+        if (rw != 16 && rw != 32 && rw != 64)
+            for (rw = 64; rw > 16 && matvecs * ((nrows + rw - 1) / rw) < c->num_cu * 3 / 4;) rw >>= 1;
+        return rw;
+    };
+    auto waves = [&](long groups, int nchunks) { return std::min(nchunks, c->tune.packed_block > 0 ? c->tune.packed_block / 64 : groups <= c->num_cu ? 16 : 8); };
+    MoePlanesGatherArgs a;
+    a.out[0] = g; a.out[1] = u;
+    a.qs[0] = pg->qs; a.d[0] = pg->d; a.sc[0] = pg->sc; a.qs[1] = pu->qs; a.d[1] = pu->d; a.sc[1] = pu->sc;
+    a.x = x; a.sel = sel; a.sheet_words = pg->sheet_bytes / 4; a.row_step = pg->sheet_bytes ? 0 : n_ffn; a.stride = pg->stride;
+    a.nrows = n_ffn; a.k = n_embd; a.per = c->act_window / 32; a.n_expert = n_expert; a.sel_stride = sel_stride; a.k_used = k_used;
+    const int pairs = rows * k_used, rw = width(n_ffn, 2L * pairs);
+    a.ngroups = (n_ffn + rw - 1) / rw;
+    a.nwaves = waves(2L * pairs * a.ngroups, n_embd / 256);
+    Name name;
+    name << "jl_moe_planes_gather_w" << rw;
+    void* params[] = {&a};
+    int rc = launch(c, name, (unsigned)a.ngroups, (unsigned)pairs, 64u * a.nwaves, (unsigned)(a.nwaves * (384 + 65 * 4)), st, params, 2);   // JL_PK_LDS_BYTES
+    if (rc != JL_OK) return rc;
+    MoePlanesDownArgs b;
+    b.resid = resid; b.qs = pd->qs; b.d = pd->d; b.sc = pd->sc; b.g = g; b.u = u; b.sel = sel; b.wt = wt;
+    b.sheet_words = pd->sheet_bytes / 4; b.row_step = pd->sheet_bytes ? 0 : n_embd; b.stride = pd->stride;
+    b.nrows = n_embd; b.k = n_ffn; b.per = c->act_window / 32; b.n_expert = n_expert; b.sel_stride = sel_stride; b.k_used = k_used;
+    const int dw = width(n_embd, rows);
+    b.ngroups = (n_embd + dw - 1) / dw;
+    b.nwaves = waves((long)rows * b.ngroups, k_used * (n_ffn / 256));
+    Name dname;
+    dname << "jl_moe_planes_down_w" << dw;
+    void* dparams[] = {&b};
+    return launch(c, dname, (unsigned)b.ngroups, (unsigned)rows, 64u * b.nwaves, (unsigned)(b.nwaves * (384 + 65 * 4)), st, dparams);
 }
 
 // The columns of an expert against rows decoded in registers (kernels/moe_cols.h): the source rows quantized once each
@@ -1972,6 +2013,8 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     for (const char* tag : {"q4k", "q8_0", "q8_0p", "q6k"})
         for (const char* act : {"", "_a", "_down"})
             for (const char* lpr : {"_l8", "_l16", "_l32", "_l64"}) names.push_back(std::string("jl_moe_gather_") + tag + act + lpr);
+    for (const char* rw : {"16", "32", "64"})
+        for (const char* form : {"jl_moe_planes_gather_w", "jl_moe_planes_down_w"}) names.push_back(std::string(form) + rw);
     for (const char* tag : {"q4k", "q4k_planes", "q6k"})
         for (const char* form : {"jl_moe_cols_", "jl_moe_cols_prep_"}) names.push_back(std::string(form) + tag);
     for (const char* tag : {"q8_0", "q4k", "q6k", "q6kw"})
@@ -2678,7 +2721,12 @@ int moe_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate_b
                        planes ? &d : nullptr, x, wt, rows, n_ffn, n_embd, g, u, y, st);
         if (rc != JL_DECLINED) return rc;
     }
-    if (!planes && (c->tune.moe_form == 11 || (c->tune.moe_form == 0 && moe_gather_ffn_wanted(type, down_type, rows, k_used, n_expert, n_ffn, n_embd)))) {
+    const bool gather = c->tune.moe_form == 11 || (c->tune.moe_form == 0 && moe_gather_ffn_wanted(type, down_type, planes, rows, k_used, n_expert, n_ffn, n_embd));
+    if (gather && planes) {
+        rc = moe_planes_gather_ffn(c, resid, pg, pu, pd, x, sel, sel_stride, wt, rows, k_used, n_expert, n_ffn, n_embd, g, u, st);
+        if (rc != JL_DECLINED) return rc;
+    }
+    if (gather && !planes) {
         rc = moe_gather_ffn(c, resid, type, down_type, gate_bank, up_bank, down_bank, x, sel, sel_stride, wt, rows, k_used, n_expert, n_ffn,
                             n_embd, g, u, st);
         if (rc != JL_DECLINED) return rc;

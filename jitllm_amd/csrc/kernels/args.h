@@ -196,6 +196,25 @@ struct MoeGatherDownArgs {
     int nrows, k, row_bytes, per, nwaves, ngroups, n_expert, sel_stride, k_used;
 };
 
+// The same two steps over packed planes: column = pair of sel; sheet_words, row_step: from an expert's planes, rows to the next's.
+struct MoePlanesGatherArgs {
+    float* out[2];          // [pair][nrows]
+    const uint32_t *qs[2], *d[2], *sc[2];
+    const float* x;         // [row][k]
+    const uint32_t* sel;
+    size_t sheet_words;
+    int nrows, k, row_step, stride, per, nwaves, ngroups, n_expert, sel_stride, k_used;
+};
+struct MoePlanesDownArgs {
+    float* resid;           // [row][nrows]
+    const uint32_t *qs, *d, *sc;
+    const float *g, *u;     // [pair][k]
+    const uint32_t* sel;
+    const float* wt;        // [row][k_used]
+    size_t sheet_words;
+    int nrows, k, row_step, stride, per, nwaves, ngroups, n_expert, sel_stride, k_used;
+};
+
 struct MoeColsPrepArgs {
     const float* x;
     const float* x2;        // null: plain activation, else silu(x) * x2

@@ -12,6 +12,7 @@
 #include "matvec.h"
 #include "moe.h"
 #include "moe_cols.h"
+#include "moe_planes.h"
 #include "mxfp4.h"
 #include "packed.h"
 #include "quantize.h"
@@ -375,6 +376,15 @@ extern "C" __global__ __launch_bounds__(512) void jl_moe_matvec_planes_q4k(MoePl
     extern "C" __global__ __launch_bounds__(1024) void jl_moe_gather_##T##_down_l##L(MoeGatherDownArgs p) { moe_gather_down_body<TYPE, L>(p, jl_smem); }
 #define JL_MOE_GATHER(T, TYPE) JL_MOE_GATHER_L(T, TYPE, 8) JL_MOE_GATHER_L(T, TYPE, 16) JL_MOE_GATHER_L(T, TYPE, 32) JL_MOE_GATHER_L(T, TYPE, 64)
 JL_MOE_GATHER(q4k, JL_Q4_K) JL_MOE_GATHER(q8_0, JL_Q8_0) JL_MOE_GATHER(q8_0p, JL_Q8_0P) JL_MOE_GATHER(q6k, JL_Q6_KS)
+// over planes: grid = (ceil(nrows/RW), pairs, 2) and (ceil(nrows/RW), rows), block <= 1024, dynamic LDS = JL_PK_LDS_BYTES
+#define JL_MOE_PLANES_GATHER(RW)                                                                                          \
+    extern "C" __global__ __launch_bounds__(1024) void jl_moe_planes_gather_w##RW(MoePlanesGatherArgs p) {                \
+        moe_planes_gather_body<RW, 1>(p, jl_smem);                                                                        \
+    }                                                                                                                     \
+    extern "C" __global__ __launch_bounds__(1024) void jl_moe_planes_down_w##RW(MoePlanesDownArgs p) {                    \
+        moe_planes_down_body<RW, 2>(p, jl_smem);                                                                          \
+    }
+JL_MOE_PLANES_GATHER(16) JL_MOE_PLANES_GATHER(32) JL_MOE_PLANES_GATHER(64)
 // experts of some tens of columns (kernels/moe_cols.h): prep grid = ceil(records * k/256 / 16); matrices: dynamic LDS = JL_MC_LDS_BYTES
 #define JL_MOE_COLS(T, KO)                                                                                                         \
     extern "C" __global__ __launch_bounds__(256) void jl_moe_cols_prep_##T(MoeColsPrepArgs p) { moe_cols_prep_body<KO>(p); }      \

@@ -137,6 +137,10 @@ def test_a_matvec_a_column(dev, devbuf, t, window, nrows, k):
     (quant.Q4_K, quant.Q6_K, 32, 6, 2, 40, 512, 1024, 0),       # sixteen and eight
     (quant.Q4_K, quant.Q4_K, 256, 6, 2, 20, 1024, 2816, 0),     # sixteen lanes of three slots, the last without one for some
     (quant.Q6_K, quant.Q8_0, 32, 6, 2, 20, 768, 2048, 0),       # 32
+    (quant.Q4_K, quant.Q4_K, 256, 12, 8, 1, 512, 768, "one"),   # packed planes, the three widths of a run of rows
+    (quant.Q4_K, quant.Q4_K, 256, 12, 3, 3, 1280, 1792, "sheets"),
+    (quant.Q4_K, quant.Q4_K, 256, 7, 2, 40, 256, 1024, "one"),
+    (quant.Q4_K, quant.Q4_K, 256, 7, 4, 16, 768, 512, "sheets"),
 ], ids=lambda v: str(v))
 def test_block_of_pairs(dev, devbuf, t, down, window, n_expert, k_used, rows, n_ffn, n_embd, pair):
     """The routed block without grouping and combine: a selection with a stride of its own, the first and the last expert
@@ -156,14 +160,20 @@ def test_block_of_pairs(dev, devbuf, t, down, window, n_expert, k_used, rows, n_
     start = rng.standard_normal((rows, n_embd)).astype(np.float32)
     want = start + _oracle_block(t, *banks, x, sel, wt, n_expert, n_ffn, n_embd, window, td=down)
     dev.SetActWindow(window)
-    hold = [devbuf(b) for b in banks]
+    planes = isinstance(pair, str)
+    if planes:
+        from test_gpu_moe import _pack_bank
+        hold = [_pack_bank(dev, devbuf, t, b, n_expert, r, k, pair) for b, (r, k) in zip(banks, [(n_ffn, n_embd)] * 2 + [(n_embd, n_ffn)])]
+    else:
+        hold = [devbuf(b) for b in banks]
     xd, sd, wd = devbuf(x), devbuf(sel), devbuf(wt)
     try:
-        dev.set_tuning(moe__form=11, q8pair=pair)
+        dev.set_tuning(moe__form=11, q8pair=0 if planes else pair)
         resid = devbuf(np.concatenate([start.reshape(-1), np.full(8, FILL)]))
         before = dev.launch_count()
-        assert dev.moe_ffn_dev(resid.ptr, t, *[b.ptr for b in hold], xd.ptr, sd.ptr, k_used + 2, wd.ptr, rows, k_used, n_expert,
-                               n_ffn, n_embd, down_type=down)
+        args = (xd.ptr, sd.ptr, k_used + 2, wd.ptr, rows, k_used, n_expert, n_ffn, n_embd)
+        assert dev.moe_ffn_packed_dev(resid.ptr, t, *[b[0] for b in hold], *args) if planes else \
+            dev.moe_ffn_dev(resid.ptr, t, *[b.ptr for b in hold], *args, down_type=down)
         dev.synchronize()
         assert dev.launch_count() - before == 2
         got = resid.get()
