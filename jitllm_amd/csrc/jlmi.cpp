@@ -631,10 +631,12 @@ int resident_weight(jl_ctx* c, const void* w, size_t bytes, void** dev) {
 }
 
 int ws_ensure(jl_ctx* c, void** buf, size_t* have, size_t need);
+// The work lists a block's grouping made for tiles of 64 and of 128 columns.
+struct MoeLists { uint32_t* wl[2]; int nslots; };
 int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1,
                       const float* x, const float* x2, const uint32_t* src, const uint32_t* start,
                       int n_expert, int ncols, int nrows, int k, hipStream_t st,
-                      const jl_packed_bank* pb0 = nullptr, const jl_packed_bank* pb1 = nullptr, int nsrc = 0);
+                      const jl_packed_bank* pb0 = nullptr, const jl_packed_bank* pb1 = nullptr, int nsrc = 0, const MoeLists* lists = nullptr);
 
 // plane banks of a mixture: from this many columns an expert (on average) the matrix-core tile
 // per expert takes over from the dot-product form ("moe.form" = 1 / 4 forces one)
@@ -1333,7 +1335,7 @@ int packed_matmul_launch(jl_ctx* c, float* out, int type, const PlaneRef& pl, co
 // The int8 tile placed per expert: work list, columns quantized and laid out group by group, tiles.
 int moe_gemm_i8_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1, const float* x,
                        const float* x2, const uint32_t* src, const uint32_t* start, int n_expert, int ncols, int nrows, int k,
-                       I8Shape f, hipStream_t st) {
+                       I8Shape f, hipStream_t st, const MoeLists* lists) {
     const TypeInfo* ti = type_info(type);
     const bool q4 = type == JL_TYPE_Q4_K;
     const int nslots = ncols / 32 + n_expert + 1, nstage = k / 128, tile = 32 * f.tw;
@@ -1351,8 +1353,8 @@ int moe_gemm_i8_launch(jl_ctx* c, float* out0, float* out1, int type, const void
     wa.start = start; wa.wl = (uint32_t*)(ws + o_wl); wa.n_expert = n_expert; wa.nslots = nslots;
     wa.tile_log2 = f.tw == 4 ? 7 : 6;
     void* wp[] = {&wa};
-    rc = launch(c, "jl_moe_worklist", 1, 1, 1024, 0, st, wp);
-    if (rc != JL_OK) return rc;
+    if (lists && lists->nslots == nslots) wa.wl = lists->wl[wa.tile_log2 - 6];   // (made by the grouping)
+    else if ((rc = launch(c, "jl_moe_worklist", 1, 1, 1024, 0, st, wp)) != JL_OK) return rc;
     MoeGemmPrepArgs pa;
     pa.x = x; pa.x2 = x2; pa.src = src; pa.start = start; pa.wl = wa.wl;
     pa.bq = (uint16_t*)ws; pa.da = (float*)(ws + bq_bytes); pa.k = k; pa.nslots = nslots; pa.per = c->act_window / 32;
@@ -1637,7 +1639,7 @@ int moe_cols_launch(jl_ctx* c, float* out0, float* out1, int type, const void* b
 int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1,
                       const float* x, const float* x2, const uint32_t* src, const uint32_t* start,
                       int n_expert, int ncols, int nrows, int k, hipStream_t st, const jl_packed_bank* pb0,
-                      const jl_packed_bank* pb1, int nsrc) {
+                      const jl_packed_bank* pb1, int nsrc, const MoeLists* lists) {
     const TypeInfo* ti = nullptr;
     int rc = matvec_check(c, type, nrows, k, &ti);
     if (rc != JL_OK) return rc;
@@ -1699,7 +1701,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
         }
         if (form >= 6 && !planes && gemm_i8_applies(c, type, nrows, k, ncols)) {
             rc = moe_gemm_i8_launch(c, out0, out1, type, bank0, bank1, x, x2, src, start, n_expert, ncols, nrows, k,
-                                    form == 7 ? I8Shape{2, 2} : form == 8 && type == JL_TYPE_Q8_0 ? I8Shape{4, 4} : I8Shape{2, 4}, st);
+                                    form == 7 ? I8Shape{2, 2} : form == 8 && type == JL_TYPE_Q8_0 ? I8Shape{4, 4} : I8Shape{2, 4}, st, lists);
             if (rc != JL_DECLINED) return rc;
         }
         if (form == 5 && align && few_fits(c, type, planes, nrows, k, ncols, planes ? pb0->stride : 0)) {
@@ -2546,9 +2548,9 @@ int jl_moe_logits_dev(jl_ctx* c, float* logits, int wtype, const void* w, const 
                   pick_stream(c, stream), params);
 }
 
-int jl_moe_group_dev(jl_ctx* c, const uint32_t* sel, int sel_stride, int rows, int k_used, int n_expert,
-                     uint32_t* start, uint32_t* perm, uint32_t* pos, void* stream) {
-    if (!c) return JL_ERR_ARG;
+namespace {
+int moe_group_launch(jl_ctx* c, const uint32_t* sel, int sel_stride, int rows, int k_used, int n_expert, uint32_t* start, uint32_t* perm,
+                     uint32_t* pos, MoeLists* lists, hipStream_t st) {
     if (!sel || !start || !perm || !pos || rows <= 0 || k_used <= 0 || sel_stride < k_used)
         return fail(c, JL_ERR_ARG, "moe group: bad operand");
     if (n_expert <= 0 || n_expert > 1024) return JL_DECLINED;
@@ -2560,9 +2562,20 @@ int jl_moe_group_dev(jl_ctx* c, const uint32_t* sel, int sel_stride, int rows, i
     // the linear-time form, a workgroup for 1024 pairs (moe.group = 1 forces the one that compares every pair with every
     // expert)
     const size_t npairs = (size_t)rows * k_used, lds2 = 16 * (size_t)n_expert * 2 + (2 * (size_t)n_expert + 16) * 4;   // JL_MOE_GROUP2_LDS
-    if (c->tune.moe_group != 1 && lds2 <= c->lds_limit && npairs <= 0x7fffffffu - 8192)
-        return launch(c, "jl_moe_group2", (unsigned)((npairs + 1023) / 1024), 1, 1024, (unsigned)lds2, pick_stream(c, stream), params);
-    return launch(c, "jl_moe_group", 1, 1, 1024, 0, pick_stream(c, stream), params);
+    if (c->tune.moe_group != 1 && lds2 <= c->lds_limit && npairs <= 0x7fffffffu - 8192) {
+        if (lists->nslots) { a.wl[0] = lists->wl[0]; a.wl[1] = lists->wl[1]; a.nslots = lists->nslots; }
+        return launch(c, "jl_moe_group2", (unsigned)((npairs + 1023) / 1024), 1, 1024, (unsigned)lds2, st, params);
+    }
+    lists->nslots = 0;   // (this form makes none)
+    return launch(c, "jl_moe_group", 1, 1, 1024, 0, st, params);
+}
+}  // namespace
+
+int jl_moe_group_dev(jl_ctx* c, const uint32_t* sel, int sel_stride, int rows, int k_used, int n_expert,
+                     uint32_t* start, uint32_t* perm, uint32_t* pos, void* stream) {
+    if (!c) return JL_ERR_ARG;
+    MoeLists none{};
+    return moe_group_launch(c, sel, sel_stride, rows, k_used, n_expert, start, perm, pos, &none, pick_stream(c, stream));
 }
 
 int jl_moe_matvec_dev(jl_ctx* c, float* out0, float* out1, int type, const void* bank0, const void* bank1,
@@ -2606,20 +2619,23 @@ namespace {
 struct MoeWs {
     uint32_t *start, *perm, *pos;
     float *g, *u, *y;
+    MoeLists lists;
 };
 int moe_ws(jl_ctx* c, int rows, int k_used, int n_expert, int n_ffn, int n_embd, MoeWs* w) {
     const size_t ncols = (size_t)rows * k_used;
     auto up256 = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const size_t o_start = 0, o_perm = up256((size_t)(n_expert + 1) * 4), o_pos = o_perm + up256(ncols * 4);
     const size_t o_g = o_pos + up256(ncols * 4), o_u = o_g + up256(ncols * n_ffn * 4);
-    const size_t o_y = o_u + up256(ncols * n_ffn * 4), total = o_y + up256(ncols * n_embd * 4);
-    int rc = ws_ensure(c, &c->moe_ws, &c->moe_ws_bytes, total);
+    const size_t o_y = o_u + up256(ncols * n_ffn * 4), o_wl = o_y + up256(ncols * n_embd * 4);
+    const size_t nslots = ncols / 32 + n_expert + 1, list = up256((4 + nslots + ncols / 64 + n_expert) * 4);
+    int rc = ws_ensure(c, &c->moe_ws, &c->moe_ws_bytes, o_wl + 2 * list);
     if (rc != JL_OK) return rc;
     char* ws = (char*)c->moe_ws;
     w->start = (uint32_t*)(ws + o_start);
     w->perm = (uint32_t*)(ws + o_perm);
     w->pos = (uint32_t*)(ws + o_pos);
     w->g = (float*)(ws + o_g); w->u = (float*)(ws + o_u); w->y = (float*)(ws + o_y);
+    w->lists = MoeLists{{(uint32_t*)(ws + o_wl), (uint32_t*)(ws + o_wl + list)}, (int)nslots};
     return JL_OK;
 }
 
@@ -2731,15 +2747,17 @@ int moe_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate_b
                             n_embd, g, u, st);
         if (rc != JL_DECLINED) return rc;
     }
-    rc = jl_moe_group_dev(c, sel, sel_stride, rows, k_used, n_expert, start, perm, pos, st);
+    // (the work lists where a matvec may take the int8 tiles)
+    if (planes || ncols < 8 * (size_t)n_expert || (type == JL_TYPE_Q4_K && down_type == JL_TYPE_Q4_K && c->act_window == 256)) w.lists.nslots = 0;
+    rc = moe_group_launch(c, sel, sel_stride, rows, k_used, n_expert, start, perm, pos, &w.lists, st);
     if (rc != JL_OK) return rc;
     // gate and up: columns read the routed rows of x
     rc = moe_matvec_launch(c, g, u, type, gate_bank, up_bank, x, nullptr, perm, start, n_expert, (int)ncols, n_ffn, n_embd, st,
-                           pg, pu, rows);
+                           pg, pu, rows, &w.lists);
     if (rc != JL_OK) return rc;
     // down: the activation of column c is silu(g[c]) * u[c]
     rc = moe_matvec_launch(c, y, nullptr, down_type, down_bank, nullptr, g, u, nullptr, start, n_expert, (int)ncols, n_embd, n_ffn, st,
-                           pd, nullptr);
+                           pd, nullptr, 0, &w.lists);
     if (rc != JL_OK) return rc;
     return jl_moe_combine_dev(c, resid, y, wt, sel, sel_stride, pos, rows, k_used, n_embd, st);
 }

@@ -308,6 +308,8 @@ struct MoeGroupArgs {
     uint32_t* perm;
     uint32_t* pos;
     int sel_stride, rows, k_used, n_expert;
+    uint32_t* wl[2] = {};   // null, or the work lists (MoeWorklistArgs) of tiles of 64 and of 128 columns
+    int nslots = 0;
 };
 
 // Router: softmax over all experts, the k largest by (score descending, index ascending),

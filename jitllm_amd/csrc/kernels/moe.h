@@ -326,6 +326,34 @@ __device__ __forceinline__ void moe_group2_body(const MoeGroupArgs& p, uint8_t* 
             if (tid == nexp - 1) p.start[nexp] = v;
         }
     }
+    // The work lists of the tile forms (moe_worklist_body, n_expert <= 1024), both at once: a launch of its own takes 4.4 us
+    // and the two matvecs of a block would each make one.
+    if (blockIdx.x == 0 && p.wl[0]) {   // uniform
+        const u32 e = (u32)tid, c_lo = v - total, s0 = (c_lo >> 5) + e, ng = (total + 31) >> 5;
+        u32 nt = 0;
+        if (tid < nexp) {
+            nt = (total + 63) >> 6 | ((total + 127) >> 7) << 16;
+            const u32 s1 = tid + 1 < nexp ? (v >> 5) + e + 1 : (u32)p.nslots;
+            for (u32 s = s0; s < s1; s++) p.wl[0][4 + s] = p.wl[1][4 + s] = s - s0 < ng ? e : 0xFFFFFFFFu;
+        }
+        u32 t = nt;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const u32 o = __shfl_up(t, off, 64);
+            if (lane >= off) t += o;
+        }
+        __syncthreads();   // (the totals of the scan above have been read)
+        if (lane == 63) stot[wave] = t;
+        __syncthreads();
+        for (int w = 0; w < wave; w++) t += stot[w];
+#pragma unroll
+        for (int l = 0; l < 2; l++) {
+            const u32 n = nt >> (16 * l) & 0xFFFF, first = (t >> (16 * l) & 0xFFFF) - n;
+            u32* tiles = p.wl[l] + 4 + p.nslots + first;
+            for (u32 j = 0; j < n; j++) tiles[j] = e | (j << 16);
+            if (tid == nexp - 1) p.wl[l][0] = first + n;
+        }
+    }
     __syncthreads();
     if (valid) {
         const u32 col = sbefore[e] + mine[e] + rank;

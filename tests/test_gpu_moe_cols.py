@@ -183,3 +183,46 @@ def test_block_of_pairs(dev, devbuf, t, down, window, n_expert, k_used, rows, n_
     finally:
         dev.set_tuning(moe__form=0, q8pair=0)
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("t,down,window,form", [(quant.Q8_0, quant.Q6_K, 32, 6), (quant.Q8_0, quant.Q8_0, 32, 8), (quant.Q4_K, quant.Q6_K, 32, 7),
+                                                (quant.Q6_K, quant.Q6_K, 256, 6)], ids=lambda v: str(v))
+@pytest.mark.parametrize("rows", [90, 700])
+def test_block_with_work_lists_from_the_grouping(dev, devbuf, t, down, window, form, rows):
+    """The tiles of a block from the work lists its grouping made: the bits of the separate calls, whose matvecs make their own;
+    experts nobody chose (the last among them), one of most rows, one and several workgroups of pairs."""
+    k_used, n_expert, n_ffn, n_embd = 2, 9, 256, 512
+    rng = np.random.default_rng(rows)
+    sel = np.stack([rng.choice([1, 2, 4, 5, 7], 2, replace=False) for _ in range(rows)]).astype(np.uint32)
+    sel[: rows * 2 // 3, 0], sel[: rows * 2 // 3, 1] = 4, 1 + 4 * (np.arange(rows * 2 // 3) % 2)
+    perm = np.argsort(sel.reshape(-1), kind="stable")
+    start = np.concatenate([[0], np.cumsum(np.bincount(sel.reshape(-1), minlength=n_expert))]).astype(np.uint32)
+    ncols = rows * k_used
+    dev.SetActWindow(window)
+    bank = lambda ty, nrows, k, s: devbuf(np.concatenate([synth.random_weights(ty, nrows, k, seed=s + e) for e in range(n_expert)]))
+    gate, up, dn = bank(t, n_ffn, n_embd, 0), bank(t, n_ffn, n_embd, 50), bank(down, n_embd, n_ffn, 90)
+    x = np.stack([synth.activations(n_embd, seed=700 + r) for r in range(rows)])
+    wt = rng.random((rows, k_used)).astype(np.float32)
+    xd, sd, wd, start_d = devbuf(x), devbuf(sel), devbuf(wt), devbuf(start)
+    perm_d, pos_d = devbuf((perm // k_used).astype(np.uint32)), devbuf(np.argsort(perm, kind="stable").astype(np.uint32))
+    try:
+        dev.set_tuning(moe__form=form)
+        r = devbuf(np.zeros((rows, n_embd), np.float32))
+        g, u, y = (devbuf(shape=(ncols, n), dtype=np.float32) for n in (n_ffn, n_ffn, n_embd))
+        want = devbuf(np.zeros((rows, n_embd), np.float32))
+        before = dev.launch_count()
+        assert dev.moe_matvec_dev(g.ptr, u.ptr, t, gate.ptr, up.ptr, xd.ptr, None, perm_d.ptr, start_d.ptr, n_expert, ncols, n_ffn, n_embd)
+        assert dev.moe_matvec_dev(y.ptr, None, down, dn.ptr, None, g.ptr, u.ptr, None, start_d.ptr, n_expert, ncols, n_embd, n_ffn)
+        separate = dev.launch_count() - before + 2
+        assert dev.moe_combine_dev(want.ptr, y.ptr, wd.ptr, sd.ptr, k_used, pos_d.ptr, rows, k_used, n_embd)
+        for _ in range(2):
+            r.put(np.zeros((rows, n_embd), np.float32))
+            before = dev.launch_count()
+            assert dev.moe_ffn_dev(r.ptr, t, gate.ptr, up.ptr, dn.ptr, xd.ptr, sd.ptr, k_used, wd.ptr, rows, k_used, n_expert, n_ffn,
+                                   n_embd, down_type=down)
+            assert dev.launch_count() - before == separate - 2   # two work lists less
+            dev.synchronize()
+            assert np.array_equal(r.get().view(np.uint32), want.get().view(np.uint32))
+    finally:
+        dev.set_tuning(moe__form=0)
+        dev.SetActWindow(32)
