@@ -900,6 +900,53 @@ Name gemm_i8_name(const char* pre, const jl_ctx* c, int type, I8Shape f) {
     return n;
 }
 
+size_t gemm_i8_acts(int type, int ntok, int k) {   // bytes of the activations' fragments and scales
+    const size_t tok_pad = ((size_t)ntok + 127) / 128 * 128;
+    return (size_t)(k / 128) * (tok_pad / 32) * 4096 + (type == JL_TYPE_Q4_K ? 2 : 1) * (size_t)(k / 32) * tok_pad * 4;
+}
+// The tile and the slices of K of a launch, and what the tiles should take.
+struct I8Plan { I8Shape f; int nsplit; double us; };
+I8Plan gemm_i8_plan(const jl_ctx* c, int type, int nrows, int k, int ntok) {
+    const bool q6 = type == JL_TYPE_Q6_K, q4 = type == JL_TYPE_Q4_K;
+    const int nstage = k / 128;
+    const int unit = q6 || q4 ? 2 : 1, nunit = nstage / unit;   // stages a split is made of
+    // Shape and K split by what they should take.  A wavefront's 32 x 32 x 32 block costs its SIMD `many` us with two or
+    // three wavefronts there and `alone` with one; workgroups are resident two (128 x 128: Q8_0 only, the others have no
+    // registers for it) or three (128 x 64; two for the k-quants) a CU; the slabs of a split a launch (hidden under the
+    // tail of the tiles) and a trip through memory.  Fitted to 19 shapes (1024 x 4096 to 14336 x 4096, 100 to 2048 tokens)
+    // of every type at 1 to 8 splits, 6 % each; the pick is within 5 % of the best split at all but eight of the 76.  (One
+    // pair of constants for every type left the k-quants uncut: window 32, 512 tokens of 4096 x 4096 Q4_K 62 against 52
+    // in two, Q6_K 80 against 66, 900 tokens of 1700 x 8192 112 against 85 and 143 against 105.)
+    const double many = type == JL_TYPE_Q8_0 ? 0.088 : q4 ? 0.114 : c->act_window == 32 ? 0.160 : 0.097;
+    const double alone = type == JL_TYPE_Q8_0 ? 0.125 : q4 ? 0.177 : c->act_window == 32 ? 0.241 : 0.131;
+    I8Shape f = {2, 4};
+    int nsplit = 1;
+    double best = 1e30;
+    // Slabs as far as the static array has room for them behind the activations, in every call, so that a call that may
+    // not allocate is served where one without slices fits, with the slices of the call that may (without that bound one
+    // drawn shape in thirteen was refused for its slices; by the estimate it costs 0.3 % on average).
+    const size_t n = (size_t)ntok * nrows, acts = (gemm_i8_acts(type, ntok, k) + 255) & ~(size_t)255;
+    size_t most = acts < jl_static_scratch_bytes() ? jl_static_scratch_bytes() - acts : 0;
+    if (reserved_for(c, ntok, k)) most = std::min(most, slab_reserve(c));
+    for (int rt : {4, 2}) {
+        if (type != JL_TYPE_Q8_0 ? rt == 4 : c->tune.gemm_i8 > 0 && rt != (c->tune.gemm_i8 == 1 ? 4 : 2)) continue;
+        const long cap = rt == 4 || type != JL_TYPE_Q8_0 ? 2 : 3, groups = (long)((ntok + 127) / 128) * ((nrows + 32 * rt - 1) / (32 * rt));
+        for (int s = 1; s <= 8 && s <= nunit; s++) {
+            if (c->tune.gemm_split > 0 && s != std::min(std::min(c->tune.gemm_split, 8), nunit)) continue;
+            const int per = (nunit + s - 1) / s;
+            if ((nunit + per - 1) / per != s) continue;   // no empty split
+            if (s > 1 && n * s * 4 > most) continue;
+            const long wgs = groups * s, full = wgs / (cap * c->num_cu), left = wgs - full * cap * c->num_cu;
+            const double block = 4 * rt * per * unit;     // of a wavefront
+            double us = full * (0.15 + many * cap * block);
+            if (left) us += 0.15 + std::max(many * ((left + c->num_cu - 1) / c->num_cu), alone) * block;
+            if (s > 1) us += 0.25 + 1.16e-6 * (s + 1) * n;
+            if (us < best) { best = us; f = {rt, 4}; nsplit = s; }
+        }
+    }
+    return {f, nsplit, best};
+}
+
 int gemm_i8_launch(jl_ctx* c, float* out, int type, const void* w, const float* x, int nrows, int k, int ntok, hipStream_t st) {
     const bool q6 = type == JL_TYPE_Q6_K, q4 = type == JL_TYPE_Q4_K;
     const int tok_pad = (ntok + 127) / 128 * 128, nstage = k / 128;
@@ -920,40 +967,10 @@ int gemm_i8_launch(jl_ctx* c, float* out, int type, const void* w, const float* 
     ga.out_stride = nrows; ga.sb_per = 0;
     void* gp[] = {&ga};
     const int unit = q6 || q4 ? 2 : 1, nunit = nstage / unit;   // stages a split is made of
-    // Shape and K split by what they should take.  A wavefront's 32 x 32 x 32 block costs its SIMD `many` us with two or
-    // three wavefronts there and `alone` with one; workgroups are resident two (128 x 128: Q8_0 only, the others have no
-    // registers for it) or three (128 x 64; two for the k-quants) a CU; the slabs of a split a launch (hidden under the
-    // tail of the tiles) and a trip through memory.  Fitted to 19 shapes (1024 x 4096 to 14336 x 4096, 100 to 2048 tokens)
-    // of every type at 1 to 8 splits, 6 % each; the pick is within 5 % of the best split at all but eight of the 76.  (One
-    // pair of constants for every type left the k-quants uncut: window 32, 512 tokens of 4096 x 4096 Q4_K 62 against 52
-    // in two, Q6_K 80 against 66, 900 tokens of 1700 x 8192 112 against 85 and 143 against 105.)
-    const double many = type == JL_TYPE_Q8_0 ? 0.088 : q4 ? 0.114 : c->act_window == 32 ? 0.160 : 0.097;
-    const double alone = type == JL_TYPE_Q8_0 ? 0.125 : q4 ? 0.177 : c->act_window == 32 ? 0.241 : 0.131;
-    I8Shape f = {2, 4};
-    int nsplit = 1;
-    double best = 1e30;
-    // Slabs as far as the static array has room for them behind the activations, in every call, so that a call that may
-    // not allocate is served where one without slices fits, with the slices of the call that may (without that bound one
-    // drawn shape in thirteen was refused for its slices; by the estimate it costs 0.3 % on average).
-    const size_t n = (size_t)ntok * nrows, acts = (bq_bytes + (q4 ? 2 : 1) * da_bytes + 255) & ~(size_t)255;
-    size_t most = acts < jl_static_scratch_bytes() ? jl_static_scratch_bytes() - acts : 0;
-    if (reserved_for(c, ntok, k)) most = std::min(most, slab_reserve(c));
-    for (int rt : {4, 2}) {
-        if (type != JL_TYPE_Q8_0 ? rt == 4 : c->tune.gemm_i8 > 0 && rt != (c->tune.gemm_i8 == 1 ? 4 : 2)) continue;
-        const long cap = rt == 4 || type != JL_TYPE_Q8_0 ? 2 : 3, groups = (long)((ntok + 127) / 128) * ((nrows + 32 * rt - 1) / (32 * rt));
-        for (int s = 1; s <= 8 && s <= nunit; s++) {
-            if (c->tune.gemm_split > 0 && s != std::min(std::min(c->tune.gemm_split, 8), nunit)) continue;
-            const int per = (nunit + s - 1) / s;
-            if ((nunit + per - 1) / per != s) continue;   // no empty split
-            if (s > 1 && n * s * 4 > most) continue;
-            const long wgs = groups * s, full = wgs / (cap * c->num_cu), left = wgs - full * cap * c->num_cu;
-            const double block = 4 * rt * per * unit;     // of a wavefront
-            double us = full * (0.15 + many * cap * block);
-            if (left) us += 0.15 + std::max(many * ((left + c->num_cu - 1) / c->num_cu), alone) * block;
-            if (s > 1) us += 0.25 + 1.16e-6 * (s + 1) * n;
-            if (us < best) { best = us; f = {rt, 4}; nsplit = s; }
-        }
-    }
+    const I8Plan plan = gemm_i8_plan(c, type, nrows, k, ntok);
+    const I8Shape f = plan.f;
+    const int nsplit = plan.nsplit;
+    const size_t n = (size_t)ntok * nrows;
     const int tt = 32 * f.tw, tr = 32 * f.rt * (4 / f.tw), per = (nunit + nsplit - 1) / nsplit;
     if (nsplit > 1) {
         rc = ws_ensure(c, &c->mx_ws, &c->mx_ws_bytes, n * nsplit * 4);
@@ -995,7 +1012,7 @@ bool few_fits(const jl_ctx* c, int type, bool planes, int nrows, int k, int ncol
 int few_form(int type, bool w256) { return type == JL_TYPE_Q8_0 ? 2 : type == JL_TYPE_Q4_K ? w256 : 3 + w256; }
 
 // A workgroup's token tiles (of 16), row tiles (of 16) and wavefronts, over which K is dealt.
-struct FewShape { int nt, rt, nw; };
+struct FewShape { int nt, rt, nw; double us = 0; };   // us: what launch and prep should take (more than 64 tokens)
 
 // Token tiles: what the (average) group fills.  Two rules for the other two.
 //
@@ -1027,26 +1044,48 @@ FewShape few_shape(const jl_ctx* c, int type, bool w256, bool planes, int nrows,
             f.rt = 2;
         if (planes && f.nt <= 2 && (f.nt == 2 || type != JL_TYPE_Q6_K) && (nrows + 63) / 64 * sheets * 10 >= cus * 7) f.rt = 4;
     } else {
-        // (over planes more row tiles get wider loads of the weights, which is most of a step with one token tile)
-        const double e = planes && f.nt <= 2 ? 0.5 : 3, more = !planes ? 1.6 : f.nt == 1 ? 1.2 : 1.4;
-        double best = 1e30;
-        for (int w : {8, 4}) {
-            const int nw = std::min(w, nsb);
-            double part = 0.25 * nw, chain = 1;
-            for (int rt : {1, 2, 4}) {
-                const int simd = f.nt > 4 ? 0 : c->few_simd[form][planes][f.nt - 1][rt / 2];
-                if (!simd || nrows < rt) break;
-                const size_t lds = std::max(nw * JL_FEW_WAVE_BYTES(type, planes, rt), JL_FEW_RED_BYTES(nw, f.nt, rt));
-                if (lds > c->lds_limit) break;
-                const long cap = std::max<long>(1, std::min<long>(simd / ((nw + 3) / 4), (long)(c->lds_limit / lds)));
-                const long wgs = (nrows + 16 * rt - 1) / (16 * rt) * sheets, full = wgs / (cap * cus), left = (wgs - full * cap * cus + cus - 1) / cus;
-                const int steps = (nsb + nw - 1) / nw;
-                double t = full * (e + steps * (chain + part * cap));
-                if (left) t += e + steps * (chain + part * left);
-                if (t < best) { best = t; f.rt = rt; f.nw = nw; }
-                part *= more; chain *= 2;
+        // More than 64 tokens: the token tiles a workgroup takes by time, us: the prep, rounds of `start`, steps of a chain and of
+        // the wavefronts the SIMD holds, both longer with every token tile.  Fitted to 12 shapes (1024 x 1024 to 14336 x 4096) at
+        // 32 to 512 tokens with one to four token tiles (the prep's first term from 64 tokens on), 6 to 10 % each; the pick is
+        // 1.5 to 3 % behind the best.
+        static const struct { double start, chain0, chain1, part0, part1; } cost[5][2] = {   // [few_form()][planes]
+            {{2.16, 0.53, 0.12, 0.00, 0.23}, {3.74, 0.82, 0.04, 0.00, 0.24}}, {{2.51, 0.36, 0.17, 0.06, 0.21}, {3.86, 0.37, 0.27, 0.23, 0.12}},
+            {{1.88, 0.55, 0.19, 0.13, 0.16}, {3.90, 0.07, 0.17, 0.48, 0.16}}, {{1.92, 0.14, 0.52, 0.39, 0.14}, {3.41, 0.77, 0.36, 0.36, 0.18}},
+            {{1.99, 0.12, 0.47, 0.36, 0.11}, {3.68, 0.66, 0.29, 0.37, 0.12}}};
+        const auto& q = cost[form][planes];
+        const int nt_lo = avg > 64 && !c->tune.few_nt ? 1 : f.nt, nt_hi = f.nt;
+        f.us = 1e30;
+        for (int nt = nt_lo; nt <= nt_hi; nt++) {
+            const long tgroups = ((avg + 15) / 16 + nt - 1) / nt;
+            // (over planes more row tiles get wider loads of the weights, which is most of a step with one token tile)
+            const double e = planes && nt <= 2 ? 0.5 : 3, more = !planes ? 1.6 : nt == 1 ? 1.2 : 1.4;
+            double best = 1e30, us = 0;
+            FewShape g = {nt, 1, std::min(8, nsb)};
+            for (int w : {8, 4}) {
+                const int nw = std::min(w, nsb);
+                double part = 0.25 * nw, chain = 1;
+                for (int rt : {1, 2, 4}) {
+                    const int simd = nt > 4 ? 0 : c->few_simd[form][planes][nt - 1][rt / 2];
+                    if (!simd || nrows < rt) break;
+                    const size_t lds = std::max(nw * JL_FEW_WAVE_BYTES(type, planes, rt), JL_FEW_RED_BYTES(nw, nt, rt));
+                    if (lds > c->lds_limit) break;
+                    const long cap = std::max<long>(1, std::min<long>(simd / ((nw + 3) / 4), (long)(c->lds_limit / lds)));
+                    const long wgs = (nrows + 16 * rt - 1) / (16 * rt) * sheets * tgroups, full = wgs / (cap * cus), left = (wgs - full * cap * cus + cus - 1) / cus;
+                    const int steps = (nsb + nw - 1) / nw;
+                    double t = full * (e + steps * (chain + part * cap));
+                    if (left) t += e + steps * (chain + part * left);
+                    if (t < best) {
+                        best = t; g.rt = rt; g.nw = nw;
+                        const long rounds = full + (left > 0);
+                        us = rounds * (q.start + steps * chain * (q.chain0 + q.chain1 * nt)) + steps * part * (full * cap + left) * (q.part0 + q.part1 * nt);
+                    }
+                    part *= more; chain *= 2;
+                }
             }
+            us += (planes ? 5.2 : 6.4) + (planes ? 1.9e-6 : 1.7e-6) * avg * k;
+            if (best < 1e30 && us < f.us) { f = g; f.us = us; }
         }
+        if (f.us == 1e30) f = {f.nt, 1, std::min(8, nsb), 1e30};
     }
     if (c->tune.few_rt) f.rt = c->tune.few_rt;
     if (nrows < f.rt) f.rt = 1;
@@ -1092,12 +1131,14 @@ int few_launch(jl_ctx* c, const FewCall& f, hipStream_t st) {
     const FewShape sh = few_shape(c, f.type, w256, planes, f.nrows, f.k, f.ncols, f.start != nullptr, f.n_expert, f.nmat);
     const int nt = sh.nt, rt = sh.rt, nw = sh.nw;
     a.nwaves = nw;
+    const int ntile = (f.ncols + 15) / 16, tgroups = (ntile + nt - 1) / nt;
+    a.tgroup = f.start ? 0 : (ntile + tgroups - 1) / tgroups;
     const unsigned lds = (unsigned)std::max(nw * JL_FEW_WAVE_BYTES(f.type, planes, rt), JL_FEW_RED_BYTES(nw, nt, rt));
     if (lds > c->lds_limit) return JL_DECLINED;
     Name name;
     name << "jl_few_" << ti->tag << (w256 ? "w_" : "_") << (planes ? "planes" : "rows") << "_t" << nt << "r" << rt;
     void* ap[] = {&a};
-    return launch(c, name, (unsigned)((f.nrows + 16 * rt - 1) / (16 * rt)), (unsigned)f.n_expert, (unsigned)(64 * nw), lds, st, ap,
+    return launch(c, name, (unsigned)((f.nrows + 16 * rt - 1) / (16 * rt)), (unsigned)(f.start ? f.n_expert : tgroups), (unsigned)(64 * nw), lds, st, ap,
                   (unsigned)f.nmat);
 }
 
@@ -1105,7 +1146,29 @@ int few_launch(jl_ctx* c, const FewCall& f, hipStream_t st) {
 bool few_applies(const jl_ctx* c, int type, bool planes, int nrows, int k, int ntok, int stride) {
     if (!few_fits(c, type, planes, nrows, k, ntok, stride)) return false;
     if (c->tune.gemm_few == 1 || (c->tune.gemm_form == 4 && ntok <= 64)) return true;
-    if (c->tune.gemm_form != 0 || ntok > 64) return false;
+    if (c->tune.gemm_form != 0) return false;
+    if (ntok > 64) {
+        // Beyond one group of 64 the groups of tokens are workgroups of their own, and the weights' bytes come again from L2:
+        // where the estimate is below a tiled GEMM's (which pays its slices of K, their sum and, over planes, the rows made anew).
+        // Against those, us: Q8_0 2048 x 2048 96 tokens 18.2 -> 10.0, 4096 x 4096 256 planes 39.5 -> 29.2; Q4_K window 32 8192 x 2048
+        // 128 29.4 -> 20.7, 1024 x 1024 512 22 -> 14; Q6_K 4096 x 4096 128 26.1 -> 23.8, window 32 32.2 -> 25.9; Q4_K 2048 x 8192 96
+        // 27.4 -> 19.9, planes 34.4 -> 20.5.  The tiles stay, 14336 x 4096: Q8_0 rows 128 tokens 42.8 (51.9 so).
+        // (A twelfth off the tiles' estimate for both errors.)
+        if (ntok > 1024 || ntok < c->gemm_min_tok || c->tune.gemm_few || c->tune.gemm_split || c->tune.gemm_i8) return false;
+        const size_t need = (size_t)((k + 255) / 256 * 2) * ((ntok + 15) / 16) * 2560;
+        if (need > jl_static_scratch_bytes()) return false;
+        const bool w256 = type == JL_TYPE_Q4_K && c->act_window == 256;
+        double tiles = 1e30;
+        if (w256 && gemm_q4k_few_applies(c, nrows, k, ntok)) {
+            const long groups = (long)((nrows + 31) / 32) * ((ntok + 63) / 64), rounds = (groups + c->num_cu - 1) / c->num_cu;
+            tiles = 8.9 + 3.2e-6 * ntok * k + 0.5 * rounds * (k / 256);   // (over planes 3 us and more above that: one choice for both layouts)
+        } else if (!w256 && gemm_i8_applies(c, type, nrows, k, ntok)) {
+            const I8Plan p = gemm_i8_plan(c, type, nrows, k, ntok);
+            tiles = 11.7 + 1e-6 * ((ntok + 127) / 128 * 128) * k + 1.03 * p.us + (p.nsplit > 1 ? 1.8 : 0) + (planes ? 4.3 + 0.16e-6 * nrows * k : 0);
+        }
+        if (tiles == 1e30) return false;   // (nothing to be measured against: as before)
+        return few_shape(c, type, type != JL_TYPE_Q8_0 && c->act_window == 256, planes && !w256, nrows, k, ntok, false, 1, 1).us < 0.92 * tiles;
+    }
     // (two tokens: two matvecs are as fast for the k-quants, not for Q8_0: 21 against 22 us, 9.6 against 10.6)
     return ntok >= (type == JL_TYPE_Q8_0 ? 2 : c->gemm_min_tok);
 }

@@ -114,6 +114,7 @@ struct FewI8Args {
     size_t sheet_bytes, sheet_words;
     int nrows, k, row_bytes, ncols, nslots, nch, nwaves;
     int prow0, row_step, pstride;
+    int tgroup;             // start null: token tiles a workgroup, grid y = the groups of them
 };
 
 // Mixture block on the matrix cores (Q4_K, activation window 256).  An expert's columns are

@@ -527,10 +527,9 @@ __device__ __forceinline__ void few_planes_half(int c, const FewPlaneW<TYPE>* W,
     }
 }
 
-// grid = (ceil(nrows / (16 RT)), experts, matrices), block = 64 * p.nwaves, dynamic LDS: JL_FEW_LDS_BYTES.
+// grid = (ceil(nrows / (16 RT)), experts or token groups, matrices), block = 64 * p.nwaves, dynamic LDS: JL_FEW_LDS_BYTES.
 template <int TYPE, bool PL, int NT, int RT, bool W256>
 __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem) {
-    const int e = blockIdx.y;
     FewI8Args p;   // the matrix's arguments, asked for at once
     {
         const int mat = blockIdx.z;
@@ -541,14 +540,14 @@ __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem
         p.sheet_bytes = PL ? 0 : args.sheet_bytes; p.sheet_words = PL ? args.sheet_words : 0;
         p.row_step = PL ? args.row_step : 0; p.prow0 = PL ? args.prow0 : 0; p.pstride = PL ? args.pstride : 0;
         p.nrows = args.nrows; p.k = args.k; p.row_bytes = PL ? 0 : args.row_bytes; p.ncols = args.ncols; p.nslots = args.nslots;
-        p.nch = args.nch; p.nwaves = args.nwaves;
+        p.nch = args.nch; p.nwaves = args.nwaves; p.tgroup = args.tgroup;
         if constexpr (PL) {
             JL_NOW(p.out[0], p.pqs[0], p.pd[0], p.psc[0], p.resid, p.bq, p.da, p.ds, p.start, p.sheet_words, p.row_step, p.prow0, p.pstride,
-                   p.nrows, p.k, p.ncols, p.nslots, p.nch, p.nwaves);
+                   p.nrows, p.k, p.ncols, p.nslots, p.nch, p.nwaves, p.tgroup);
             p.pqs[0] = as_global(p.pqs[0]); p.pd[0] = as_global(p.pd[0]); p.psc[0] = as_global(p.psc[0]);
         } else {
             JL_NOW(p.out[0], p.w[0], p.resid, p.bq, p.da, p.ds, p.start, p.sheet_bytes, p.nrows, p.k, p.row_bytes, p.ncols, p.nslots, p.nch,
-                   p.nwaves);
+                   p.nwaves, p.tgroup);
             p.w[0] = as_global(p.w[0]);
         }
         p.out[0] = as_global(p.out[0]); p.resid = as_global(p.resid); p.bq = as_global(p.bq); p.da = as_global(p.da); p.ds = as_global(p.ds);
@@ -556,6 +555,7 @@ __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem
     }
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nw = p.nwaves;
     const int r16 = lane & 15, g = lane >> 4;
+    const int e = p.start ? blockIdx.y : 0;
     u32 col0 = 0, ncol = (u32)p.ncols;
     if (p.start) {
         col0 = (u32)__builtin_amdgcn_readfirstlane((i32)p.start[e]);
@@ -573,7 +573,10 @@ __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem
     uint8_t* st = (uint8_t*)sc + JL_FEW_SC_BYTES * RT;   // GGUF rows: the staged super-block
     // Q6_K: the lane groups that hold a block's first run of sixteen
     const u32 m0 = g < 2 ? 0xFFFFFFFFu : 0u;
-    const u32 ntile = (ncol + 15) >> 4, slot0 = (col0 >> 4) + (u32)e;
+    const u32 t_lo = p.start ? 0u : blockIdx.y * (u32)p.tgroup;
+    const u32 ntile = p.start ? (ncol + 15) >> 4 : min((ncol + 15) >> 4, t_lo + (u32)p.tgroup);
+    ncol = min(ncol, 16u * ntile);   // (a last tile of NT past the group's: not this workgroup's to store)
+    const u32 slot0 = (col0 >> 4) + (u32)e;
 
     FewPlaneAddr pa;
     FewRowAddr<TYPE, RT> ra;
@@ -610,7 +613,7 @@ __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem
         }
     }
 
-    for (u32 t0 = 0; t0 < ntile; t0 += NT) {
+    for (u32 t0 = t_lo; t0 < ntile; t0 += NT) {
         f32x4 acc[RT][NT];
 #pragma unroll
         for (int rt = 0; rt < RT; rt++)

@@ -92,3 +92,36 @@ def test_planes_to_rows_round_trip(dev, devbuf, t, nrows, k):
         dev.synchronize()
         got = dst.get()
         assert np.array_equal(got[:n * rb], src[lo * rb:(lo + n) * rb]) and np.all(got[n * rb:] == 0xEE)
+
+
+@pytest.mark.parametrize("ntok,nrows,k", [(65, 200, 256), (97, 77, 2304), (130, 16, 1024), (200, 1030, 1152)], ids=lambda v: str(v))
+@pytest.mark.parametrize("window", [32, 256])
+@pytest.mark.parametrize("t", [quant.Q8_0, quant.Q4_K, quant.Q6_K], ids=["q8_0", "q4_k", "q6_k"])
+def test_more_than_one_group_of_tokens(dev, devbuf, t, window, ntok, nrows, k):
+    """Groups of tokens on workgroups of their own: token tiles the groups do not divide (a last tile that belongs to the next
+    group is not stored twice), one token in the last, the library's own choice; rows and planes."""
+    if k % quant.block_elems(t) or (t == quant.Q8_0 and window == 256):
+        pytest.skip("K is not a whole number of this type's blocks")
+    dev.SetActWindow(window)
+    w = synth.random_weights(t, nrows, k, seed=ntok)
+    x = np.stack([synth.activations(k, seed=100 + i) * np.float32(1 + i % 7) for i in range(ntok)])
+    want = oracle.matmul_q8act_f64(t, w, x, nrows, k, ntok, window)
+    wd, xd = devbuf(w), devbuf(x)
+    planes = [devbuf(np.zeros(max(n, 4), np.uint32)) for n in quant.packed_words(t, nrows, k)]
+    assert dev.pack_weights_dev(t, wd.ptr, nrows, k, *[p.ptr for p in planes])
+    try:
+        for nt in (0, 1, 2, 3, 4):
+            dev.set_tuning(gemm__few=1 if nt else 0, few__nt=nt)
+            for packed in (False, True):
+                out = devbuf(np.full(ntok * nrows + 8, 3e30, np.float32))
+                if packed:
+                    assert dev.matmul_packed_dev(out.ptr, t, Packed(*[p.ptr for p in planes], 0, nrows), xd.ptr, nrows, k, ntok)
+                else:
+                    assert dev.matmul_dev(out.ptr, t, wd.ptr, xd.ptr, nrows, k, ntok)
+                dev.synchronize()
+                got = out.get()
+                assert np.all(got[ntok * nrows:] == np.float32(3e30)), "wrote past the output"
+                assert nmse(got[:ntok * nrows].reshape(ntok, nrows), want) <= 1e-10, (nt, packed)
+    finally:
+        dev.set_tuning(gemm__few=0, few__nt=0)
+        dev.SetActWindow(32)
