@@ -1012,7 +1012,7 @@ bool few_fits(const jl_ctx* c, int type, bool planes, int nrows, int k, int ncol
 int few_form(int type, bool w256) { return type == JL_TYPE_Q8_0 ? 2 : type == JL_TYPE_Q4_K ? w256 : 3 + w256; }
 
 // A workgroup's token tiles (of 16), row tiles (of 16) and wavefronts, over which K is dealt.
-struct FewShape { int nt, rt, nw; double us = 0; };   // us: what launch and prep should take (more than 64 tokens)
+struct FewShape { int nt, rt, nw; double us = 0; };   // us: what launch and prep should take (one matrix)
 
 // Token tiles: what the (average) group fills.  Two rules for the other two.
 //
@@ -1044,16 +1044,19 @@ FewShape few_shape(const jl_ctx* c, int type, bool w256, bool planes, int nrows,
             f.rt = 2;
         if (planes && f.nt <= 2 && (f.nt == 2 || type != JL_TYPE_Q6_K) && (nrows + 63) / 64 * sheets * 10 >= cus * 7) f.rt = 4;
     } else {
-        // More than 64 tokens: the token tiles a workgroup takes by time, us: the prep, rounds of `start`, steps of a chain and of
+        // More than one token tile: the token tiles a workgroup takes by time, us: the prep, rounds of `start`, steps of a chain and of
         // the wavefronts the SIMD holds, both longer with every token tile.  Fitted to 12 shapes (1024 x 1024 to 14336 x 4096) at
-        // 32 to 512 tokens with one to four token tiles (the prep's first term from 64 tokens on), 6 to 10 % each; the pick is
-        // 1.5 to 3 % behind the best.
+        // 32 to 512 tokens with one to four token tiles 6 to 10 % each; the pick is 1.5
+        // to 3 % behind the best.  Up to 64 tokens a split has to promise a seventh more, and Q8_0 planes, where the fit is worst, have
+        // none (17 to 64 tokens, against all of them in one workgroup: Q4_K planes 1526 x 5120, 52 tokens 16.3 -> 12.5, Q6_K 1114 x
+        // 10752, 57 tokens 29.6 -> 21.9; most shapes keep the one).
         static const struct { double start, chain0, chain1, part0, part1; } cost[5][2] = {   // [few_form()][planes]
             {{2.16, 0.53, 0.12, 0.00, 0.23}, {3.74, 0.82, 0.04, 0.00, 0.24}}, {{2.51, 0.36, 0.17, 0.06, 0.21}, {3.86, 0.37, 0.27, 0.23, 0.12}},
             {{1.88, 0.55, 0.19, 0.13, 0.16}, {3.90, 0.07, 0.17, 0.48, 0.16}}, {{1.92, 0.14, 0.52, 0.39, 0.14}, {3.41, 0.77, 0.36, 0.36, 0.18}},
             {{1.99, 0.12, 0.47, 0.36, 0.11}, {3.68, 0.66, 0.29, 0.37, 0.12}}};
         const auto& q = cost[form][planes];
-        const int nt_lo = avg > 64 && !c->tune.few_nt ? 1 : f.nt, nt_hi = f.nt;
+        const int nt_lo = avg > (planes && type == JL_TYPE_Q8_0 ? 64 : 16) && !c->tune.few_nt ? 1 : f.nt, nt_hi = f.nt;
+        double least = 1e30;
         f.us = 1e30;
         for (int nt = nt_lo; nt <= nt_hi; nt++) {
             const long tgroups = ((avg + 15) / 16 + nt - 1) / nt;
@@ -1083,9 +1086,10 @@ FewShape few_shape(const jl_ctx* c, int type, bool w256, bool planes, int nrows,
                 }
             }
             us += (planes ? 5.2 : 6.4) + (planes ? 1.9e-6 : 1.7e-6) * avg * k;
-            if (best < 1e30 && us < f.us) { f = g; f.us = us; }
+            const double weighed = avg <= 64 && nt < nt_hi ? 1.15 * us : us;
+            if (best < 1e30 && weighed < least) { least = weighed; f = g; f.us = us; }
         }
-        if (f.us == 1e30) f = {f.nt, 1, std::min(8, nsb), 1e30};
+        if (least == 1e30) f = {nt_hi, 1, std::min(8, nsb), 1e30};
     }
     if (c->tune.few_rt) f.rt = c->tune.few_rt;
     if (nrows < f.rt) f.rt = 1;
