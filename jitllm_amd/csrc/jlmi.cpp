@@ -529,6 +529,10 @@ int matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, const vo
         for (int i = 0; i < m; i++) n += std::min(mid, ((long)rows[i] + step - 1) / step);
         if (n <= slots) lo = mid; else gx = mid - 1;
     }
+    // (one matrix for several activations, a token each: a row group's workgroups on one XCD, whose L2 then holds its rows)
+    bool same = m > 1 && gx > 8;
+    for (int i = 1; i < m && same; i++) same = ws[i] == ws[0];
+    if (same) gx &= ~7L;
     a.nwaves = nwaves; a.ngroups = (int)gx;
     Name name;
     // "matvec.act_split" = 1: a gated activation shared by the group's matrices is formed and
@@ -1146,6 +1150,59 @@ int few_launch(jl_ctx* c, const FewCall& f, hipStream_t st) {
                   (unsigned)f.nmat);
 }
 
+int packed_matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, const PlaneRef* pls, const float* x, size_t xstride, const float* up,
+                               float* resid, float alpha, const float* resid_gate, const float* norm_w, float norm_eps, float* norm_out, int nrows,
+                               int k, hipStream_t st);
+// A few tokens as that many decode matvecs in one launch (each reads the weights, the later ones from L2).
+int tokens_matvec_launch(jl_ctx* c, float* out, int type, const void* w, const PlaneRef* pl, const float* x, int nrows, int k, int ntok, hipStream_t st) {
+    float* outs[JL_MAX_MULTI];
+    const void* ws[JL_MAX_MULTI];
+    PlaneRef pls[JL_MAX_MULTI];
+    int rows[JL_MAX_MULTI];
+    for (int t = 0; t < ntok; t++) {
+        outs[t] = out + (size_t)t * nrows; ws[t] = w; rows[t] = nrows;
+        if (pl) pls[t] = *pl;
+    }
+    return pl ? packed_matvec_multi_launch(c, type, ntok, outs, pls, x, k, nullptr, nullptr, 0.f, nullptr, nullptr, 0.f, nullptr, nrows, k, st)
+              : matvec_multi_launch(c, type, ntok, outs, ws, rows, x, k, nullptr, nullptr, 0.f, k, st);
+}
+// Where: the few-token form is two launches, this is one.  Over rows a workgroup's sixteen wavefronts make `passes` steps of their
+// lanes a row, each a chain of trips (Q8_0, two workgroups a CU: at least its bytes); over planes a wavefront goes through its share
+// of K, longer with wider runs of rows, and longer where eight does not divide the runs (a run's workgroups then share no XCD).
+// Two tokens of a k-quant always (they were two launches of the matvec), else up to eight where that is an eighth (planes: a fifth) below the
+// few-token estimate.  us, before -> so: Q4_K 4096 x 4096 2 / 4 tokens 8.9 -> 6.3 / 9.2 -> 8.6, 2048 x 2048 8 tokens 8.9 -> 6.2, 14336 x
+// 4096 2 tokens 16.3 -> 12.1, 4 tokens 16.5 (18.1 so); Q6_K 4096 x 14336 2 tokens 24.0 -> 16.1; Q8_0 planes 4096 x 4096 2 / 4 tokens
+// 13.0 -> 8.0 / 12.9 (9.0 so).
+bool tokens_matvec_wanted(const jl_ctx* c, int type, bool planes, int nrows, int k, int ntok, int stride) {
+    if (ntok < 2 || ntok > JL_MAX_MULTI) return false;
+    if (c->tune.gemm_few == 3) return true;
+    if (ntok > 8 || c->tune.gemm_few || c->tune.gemm_form || c->gemm_min_tok != 3) return false;
+    if (ntok == 2 && type != JL_TYPE_Q8_0) return true;
+    if (!few_fits(c, type, planes, nrows, k, ntok, stride)) return false;
+    const TypeInfo* ti = type_info(type);
+    const bool q8 = type == JL_TYPE_Q8_0;
+    const long cus = c->num_cu;
+    const double mb = 1e-6 * nrows * ((double)k / ti->block_elems * ti->block_bytes);
+    double us;
+    if (!planes) {   // (matvec_multi_launch)
+        const int slots = (k + 63) / 64, lanes = matvec_lanes(c, slots, (long)nrows * ntok), step = 16 * (64 / lanes);
+        const long groups = (nrows + step - 1) / step;
+        long gx = std::min(groups, std::max(1L, (q8 ? 2 : 1) * cus / ntok));
+        if (gx > 8) gx &= ~7L;
+        const double trips = (double)((groups + gx - 1) / gx) * ((slots + lanes - 1) / lanes);
+        us = q8 ? std::max(4.3 + 0.125 * ntok * mb, 4.3 + (slots > 64 ? 2.2 : 1.5) * trips) : 4.3 + (type == JL_TYPE_Q4_K ? 1.0 : 1.28) * trips;
+    } else {         // (packed_matvec_multi_launch)
+        int rw = 64;
+        while (rw > 16 && (long)ntok * ((nrows + rw - 1) / rw) < cus * 3 / 4) rw >>= 1;
+        const long runs = (nrows + rw - 1) / rw, wgs = runs * ntok;
+        const int nch = (k + 255) / 256, nw = std::min(nch, wgs <= cus ? 16 : 8);
+        const double trips = (double)((wgs + (nw > 8 ? 1 : 3) * cus - 1) / ((nw > 8 ? 1 : 3) * cus)) * ((nch + nw - 1) / nw);
+        const bool whole = runs % 8 == 0;
+        us = std::max(4.3 + (whole ? 0.12 : 0.2) * ntok * mb, 4.5 + trips * (rw == 64 ? 3.1 : rw == 32 ? 2.2 : 1.8) * (whole ? 1 : 1.3));
+    }
+    return us < (planes ? 0.78 : 0.87) * few_shape(c, type, !q8 && c->act_window == 256, planes, nrows, k, ntok, false, 1, 1).us;
+}
+
 // Where the int8 few-token form serves a plain matmul.
 bool few_applies(const jl_ctx* c, int type, bool planes, int nrows, int k, int ntok, int stride) {
     if (!few_fits(c, type, planes, nrows, k, ntok, stride)) return false;
@@ -1186,6 +1243,10 @@ int matmul_launch(jl_ctx* c, float* out, int type, const void* w, const float* x
     if (rc != JL_OK) return rc;
     if (!out || !w || !x || ntok <= 0) return fail(c, JL_ERR_ARG, "matmul: bad operand");
     if (!aligned16(x) || (k % 4) != 0) return JL_DECLINED;
+    if (tokens_matvec_wanted(c, type, false, nrows, k, ntok, 0)) {
+        rc = tokens_matvec_launch(c, out, type, w, nullptr, x, nrows, k, ntok, st);
+        if (rc != JL_DECLINED) return rc;
+    }
     if (few_applies(c, type, false, nrows, k, ntok, 0) && ((uintptr_t)w & (type == JL_TYPE_Q4_K ? 15 : 3)) == 0) {
         FewCall f;
         f.type = type; f.nrows = nrows; f.k = k; f.ncols = ntok; f.w[0] = w; f.x = x; f.out[0] = out;
@@ -1369,6 +1430,10 @@ int packed_matmul_launch(jl_ctx* c, float* out, int type, const PlaneRef& pl, co
     if (rc != JL_OK) return rc;
     if (!out || !x || ntok <= 0) return fail(c, JL_ERR_ARG, "packed matmul: bad operand");
     if (!aligned16(x) || (k % 4) != 0) return JL_DECLINED;
+    if (tokens_matvec_wanted(c, type, true, nrows, k, ntok, pl.stride)) {
+        rc = tokens_matvec_launch(c, out, type, nullptr, &pl, x, nrows, k, ntok, st);
+        if (rc != JL_DECLINED) return rc;
+    }
     if (few_applies(c, type, true, nrows, k, ntok, pl.stride)) {
         FewCall f;
         f.type = type; f.nrows = nrows; f.k = k; f.ncols = ntok; f.pl[0] = &pl; f.x = x; f.out[0] = out;
@@ -3530,7 +3595,7 @@ int jl_matmul(jl_ctx* c, float* out, int type, const void* w, size_t wbytes, con
     if ((rc = host_io_begin(c, nx, no)) != JL_OK) return rc;
     rc = stage_in(c, 0, x, nx);
     const float* xd = nullptr;
-    if (rc == JL_OK) rc = host_io_go(c, &xd, few_applies(c, type, false, nrows, k, ntok, 0));
+    if (rc == JL_OK) rc = host_io_go(c, &xd, few_applies(c, type, false, nrows, k, ntok, 0) && !tokens_matvec_wanted(c, type, false, nrows, k, ntok, 0));
     if (rc == JL_OK) rc = matmul_launch(c, host_results(c), type, wd, xd, nrows, k, ntok, c->stream);
     host_out(0, out, no);
     return host_io_end(c, rc);
@@ -3706,7 +3771,7 @@ int jl_matmul_packed(jl_ctx* c, float* out, int type, const uint32_t* qs, const 
     if ((rc = host_io_begin(c, nx, no)) != JL_OK) return rc;
     rc = stage_in(c, 0, x, nx);
     const float* xd = nullptr;
-    if (rc == JL_OK) rc = host_io_go(c, &xd, few_applies(c, type, true, nrows, k, ntok, pl.stride));
+    if (rc == JL_OK) rc = host_io_go(c, &xd, few_applies(c, type, true, nrows, k, ntok, pl.stride) && !tokens_matvec_wanted(c, type, true, nrows, k, ntok, pl.stride));
     if (rc == JL_OK) rc = ntok == 1 ? packed_matvec_launch(c, host_results(c), type, pl, xd, nullptr,
                                           nullptr, nullptr, nrows, k, c->stream)
                    : packed_matmul_launch(c, host_results(c), type, pl, xd, nrows, k,

@@ -125,3 +125,33 @@ def test_more_than_one_group_of_tokens(dev, devbuf, t, window, ntok, nrows, k):
     finally:
         dev.set_tuning(gemm__few=0, few__nt=0)
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("ntok,nrows,k", [(2, 16, 256), (2, 700, 2048), (3, 4100, 1024), (8, 1030, 4352), (16, 37, 1280)], ids=lambda v: str(v))
+@pytest.mark.parametrize("t", [quant.Q8_0, quant.Q4_K, quant.Q6_K], ids=["q8_0", "q4_k", "q6_k"])
+def test_a_few_tokens_as_matvecs_in_one_launch(dev, devbuf, t, ntok, nrows, k):
+    """One launch, and the values of the decode matvec token by token, over rows and planes; a plane set's row range."""
+    dev.SetActWindow(32)
+    w = synth.random_weights(t, nrows, k, seed=ntok)
+    x = np.stack([synth.activations(k, seed=100 + i) * np.float32(1 + i % 7) for i in range(ntok)])
+    want = oracle.matmul_q8act_f64(t, w, x, nrows, k, ntok, 32)
+    wd, xd = devbuf(w), devbuf(x)
+    planes = [devbuf(np.zeros(max(n, 4), np.uint32)) for n in quant.packed_words(t, nrows, k)]
+    assert dev.pack_weights_dev(t, wd.ptr, nrows, k, *[p.ptr for p in planes])
+    lo, part = 3, nrows - 5
+    try:
+        dev.set_tuning(gemm__few=3)
+        for packed, r0, n in ((False, 0, nrows), (True, 0, nrows), (True, lo, part)):
+            out = devbuf(np.full(ntok * n + 8, 3e30, np.float32))
+            before = dev.launch_count()
+            if packed:
+                assert dev.matmul_packed_dev(out.ptr, t, Packed(*[p.ptr for p in planes], r0, nrows), xd.ptr, n, k, ntok)
+            else:
+                assert dev.matmul_dev(out.ptr, t, wd.ptr, xd.ptr, n, k, ntok)
+            assert dev.launch_count() == before + 1
+            dev.synchronize()
+            got = out.get()
+            assert np.all(got[ntok * n:] == np.float32(3e30)), "wrote past the output"
+            assert nmse(got[:ntok * n].reshape(ntok, n), want[:, r0:r0 + n]) <= 1e-10, (packed, r0)
+    finally:
+        dev.set_tuning(gemm__few=0)
