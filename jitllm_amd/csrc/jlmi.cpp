@@ -1618,6 +1618,7 @@ int moe_gather_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     const int lpr = gather_lanes(c, type, k / (type == JL_TYPE_Q8_0 && !pair ? 32 : 64), nrows, (long)ncols * nmat), per_group = 16 * (64 / lpr);
     const long slots = (pair ? 2L : 1L) * c->num_cu, groups = (nrows + per_group - 1) / per_group;
     a.ngroups = (int)std::max(1L, std::min(groups, slots / ((long)ncols * nmat)));
+    if (!start && !sel && a.ngroups > 8) a.ngroups &= ~7;   // (one matrix: a row group's workgroups on one XCD)
     Name name;
     name << "jl_moe_gather_" << (pair ? "q8_0p" : ti->tag) << (x2 ? "_a" : "") << "_l" << lpr;
     void* params[] = {&a};
@@ -1672,6 +1673,7 @@ int moe_gather_ffn(jl_ctx* c, float* resid, int type, int down_type, const void*
     const int lpr = gather_lanes(c, down_type, (int)row_slots * k_used, n_embd, rows), per_group = 16 * (64 / lpr);
     const long slots = (pair ? 2L : 1L) * c->num_cu, groups = (n_embd + per_group - 1) / per_group;
     a.ngroups = (int)std::max(1L, std::min(groups, slots / rows));
+    if (!sel && a.ngroups > 8) a.ngroups &= ~7;
     Name name;
     name << "jl_moe_gather_" << (pair ? "q8_0p" : ti->tag) << "_down_l" << lpr;
     void* params[] = {&a};
@@ -2794,6 +2796,27 @@ int dense_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate
     int rc;
     if (!planes && ((rc = matvec_check(c, type, n_ffn, n_embd, &ti)) != JL_OK || (rc = matvec_check(c, down_type, n_embd, n_ffn, &ti)) != JL_OK))
         return rc;
+    // Two to four rows: a decode matvec a row and matrix, two launches (moe_gather_ffn with no selection) where the few-token form's
+    // four are slower: 9 us + 0.12 (Q8_0 0.14) a MB of weights and row, against 15.5 + 0.28 a MB less a tenth.  Rows, us, before -> so:
+    // Q4_K 1024 / 4096 2, 4 rows 16.3 -> 10.1, 17.1 -> 11.1; 4096 / 14336 2 rows 42.4 -> 33.5, 3 rows 42.5 (48.3 so);
+    // Q6_K 2048 / 8192 3 rows 28.4 -> 25.3, 4 rows 29.1 (27.0 so, left); Q8_0 2048 / 8192 2 rows 26.1 -> 18.0; Q4_K planes 1280 / 5120
+    // 2 rows 19.1 -> 12.4.  (From five rows on only the smallest blocks gain, 16.9 -> 14.5 at eight rows of 1024 / 4096, and a row's bits
+    // there are those of a longer run, tests/test_gpu_layer.py.)
+    if (n >= 2 && n <= 4 && moe_dense_wanted(c) && !c->tune.gemm_form && !c->tune.gemm_few && !c->tune.few_nt && !c->tune.few_rt) {
+        const TypeInfo *t = type_info(type), *d = type_info(down_type);
+        const double mb = 1e-6 * n_ffn * n_embd * (2.0 * t->block_bytes / t->block_elems + (double)d->block_bytes / d->block_elems);
+        if (mb * ((type == JL_TYPE_Q8_0 ? 0.14 : 0.12) * n - 0.25) < 4.4) {
+            if (!planes && n_ffn % 64 == 0 && n_embd % 64 == 0 && aligned16(gate) && aligned16(up) && aligned16(down)) {
+                rc = moe_gather_ffn(c, resid, type, down_type, gate, up, down, x, nullptr, 0, wt, n, 1, 1, n_ffn, n_embd, g, u, st);
+                if (rc != JL_DECLINED) return rc;
+            } else if (planes && type == JL_TYPE_Q4_K && down_type == JL_TYPE_Q4_K && pg->stride == pu->stride && !pg->row && !pu->row && !pd->row) {
+                const jl_packed_bank bg = {pg->qs, pg->d, pg->sc, 0, pg->stride}, bu = {pu->qs, pu->d, pu->sc, 0, pu->stride},
+                                     bd = {pd->qs, pd->d, pd->sc, 0, pd->stride};
+                rc = moe_planes_gather_ffn(c, resid, &bg, &bu, &bd, x, nullptr, 0, wt, n, 1, 1, n_ffn, n_embd, g, u, st);
+                if (rc != JL_DECLINED) return rc;
+            }
+        }
+    }
     if (few(type, gate, pg, n_ffn, n_embd) && few(type, up, pu, n_ffn, n_embd) && (!planes || (pg->row == pu->row && pg->stride == pu->stride))) {
         FewCall f;
         f.type = type; f.nrows = n_ffn; f.k = n_embd; f.ncols = n; f.nmat = 2; f.x = x;

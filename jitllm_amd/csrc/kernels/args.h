@@ -179,7 +179,7 @@ struct MoeGatherArgs {
     const float* x2;        // null: plain activation, else silu(x) * x2
     const uint32_t* src;    // null: column c reads row c
     const uint32_t* start;  // null: column c is pair c of sel, which reads row c / k_used
-    const uint32_t* sel;    // [row][sel_stride]
+    const uint32_t* sel;    // [row][sel_stride]; null as well: one expert, column c reads row c
     size_t sheet_bytes;
     int nrows, k, row_bytes, per, nwaves, ngroups, n_expert, sel_stride, k_used;
 };
@@ -190,14 +190,14 @@ struct MoeGatherDownArgs {
     float* resid;           // [row][nrows]
     const uint8_t* bank;
     const float *g, *u;     // [pair][k]
-    const uint32_t* sel;    // [row][sel_stride]
-    const float* wt;        // [row][k_used]
+    const uint32_t* sel;    // [row][sel_stride]; null: expert 0 (k_used 1)
+    const float* wt;        // [row][k_used]; null: 1
     size_t sheet_bytes;
     uint32_t slots_inv;     // 2^32 / (slots of a sheet's row), rounded up
     int nrows, k, row_bytes, per, nwaves, ngroups, n_expert, sel_stride, k_used;
 };
 
-// The same two steps over packed planes: column = pair of sel; sheet_words, row_step: from an expert's planes, rows to the next's.
+// The same two steps over packed planes: column = pair of sel (null: column c reads row c, expert 0); sheet_words, row_step: from an expert's planes, rows to the next's.
 struct MoePlanesGatherArgs {
     float* out[2];          // [pair][nrows]
     const uint32_t *qs[2], *d[2], *sc[2];

@@ -1380,7 +1380,9 @@ __device__ __forceinline__ void moe_gather_body(const MoeGatherArgs& args, uint8
     const u32 *src = as_global(p.src), *start = as_global(p.start), *sel = as_global(p.sel);
     const int nrows = p.nrows, k = p.k, nthreads = p.nwaves * 64, nslots = k / T::kElems;
     u32 row, e;
-    if (!start) {
+    if (!start && !sel) {
+        row = c; e = 0;
+    } else if (!start) {
         row = c / (u32)p.k_used;
         // (an id no expert has: its weight is none, see moe_gather_down_body)
         e = min((u32)__builtin_amdgcn_readfirstlane((i32)sel[row * (u32)p.sel_stride + (c - row * (u32)p.k_used)]), (u32)p.n_expert - 1u);
@@ -1449,8 +1451,9 @@ __device__ __forceinline__ void moe_gather_down_body(const MoeGatherDownArgs& ar
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nthreads = p.nwaves * 64;
     const int row_slots = p.k / T::kElems, nslots = row_slots * p.k_used, k = p.k * p.k_used, nrows = p.nrows;
     const size_t tok = blockIdx.y;
-    const u32* sel = as_global(p.sel) + tok * p.sel_stride;
-    const float *wt = as_global(p.wt) + tok * p.k_used, *g = as_global(p.g) + tok * k, *u = as_global(p.u) + tok * k;
+    // (no selection: one expert; no weights: one)
+    const u32* sel = p.sel ? as_global(p.sel) + tok * p.sel_stride : nullptr;
+    const float *wt = p.wt ? as_global(p.wt) + tok * p.k_used : nullptr, *g = as_global(p.g) + tok * k, *u = as_global(p.u) + tok * k;
     const uint8_t* bank = as_global(p.bank);
     float* resid = as_global(p.resid) + tok * nrows;
     const u32 last = (u32)p.n_expert - 1u;
@@ -1460,10 +1463,10 @@ __device__ __forceinline__ void moe_gather_down_body(const MoeGatherDownArgs& ar
     float* sw = (float*)(se + 16);
     const int sub = lane / LPR, l = lane % LPR;
     const int s0 = min(l, nslots - 1), pair0 = (int)__umulhi((u32)s0, p.slots_inv);   // the lane's first slot and its pair
-    const u32 e0 = min(sel[pair0], last);
+    const u32 e0 = sel ? min(sel[pair0], last) : 0u;
     const int mine = min((int)threadIdx.x, p.k_used - 1);
-    const u32 em = sel[mine];
-    const float wm = wt[mine];
+    const u32 em = sel ? sel[mine] : 0u;
+    const float wm = wt ? wt[mine] : 1.f;
 
     const int n4 = k / 4, n4_pad = (n4 + 63) & ~63;
     f32x4 x0[XP], u0[XP];

@@ -21,9 +21,9 @@ __device__ __forceinline__ void moe_planes_gather_body(const MoePlanesGatherArgs
     size_t words = m.sheet_words;
     int row_step = m.row_step, ku = m.k_used, sel_stride = m.sel_stride, n_expert = m.n_expert;
     JL_NOW(p.out, p.qs, p.d, p.sc, p.x, p.nrows, p.k, p.stride, p.per, p.nwaves, p.ngroups, sel, words, row_step, ku, sel_stride, n_expert);
-    const u32 row = c / (u32)ku;
-    // (an id no expert has: its weight is none, see below)
-    const u32 e = min((u32)__builtin_amdgcn_readfirstlane((i32)as_global(sel)[row * (u32)sel_stride + (c - row * (u32)ku)]), (u32)n_expert - 1u);
+    const u32 row = sel ? c / (u32)ku : c;
+    // (no selection: one matrix; an id no expert has: its weight is none, see below)
+    const u32 e = !sel ? 0u : min((u32)__builtin_amdgcn_readfirstlane((i32)as_global(sel)[row * (u32)sel_stride + (c - row * (u32)ku)]), (u32)n_expert - 1u);
     p.out = as_global(p.out) + (size_t)c * p.nrows;
     p.qs = as_global(p.qs) + (size_t)e * words; p.d = as_global(p.d) + (size_t)e * words; p.sc = as_global(p.sc) + (size_t)e * words;
     p.row0 = (int)e * row_step;
@@ -38,16 +38,16 @@ __device__ __forceinline__ void moe_planes_down_body(const MoePlanesDownArgs& ar
            m.n_expert, m.sel_stride, m.k_used);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwaves = m.nwaves;
     const size_t tok = blockIdx.y;
-    const u32* sel = as_global(m.sel) + tok * m.sel_stride;
-    const float* wt = as_global(m.wt) + tok * m.k_used;
+    const u32* sel = m.sel ? as_global(m.sel) + tok * m.sel_stride : nullptr;   // (null: expert 0)
+    const float* wt = m.wt ? as_global(m.wt) + tok * m.k_used : nullptr;        // (null: 1)
     float* resid = as_global(m.resid) + tok * m.nrows;
     int g = blockIdx.x;
     if ((m.ngroups & 7) == 0) g = (g & 7) * (m.ngroups >> 3) + (g >> 3);   // (neighbouring row runs to one XCD, as above)
     const int rl = lane % RW, b0 = lane / RW * NB, rr = min(g * RW + rl, m.nrows - 1);
     // lane i holds pair i's expert and weight (an id no expert has: none)
-    const u32 last = (u32)m.n_expert - 1u, id = sel[min(lane, m.k_used - 1)];
+    const u32 last = (u32)m.n_expert - 1u, id = sel ? sel[min(lane, m.k_used - 1)] : 0u;
     const u32 ids = min(id, last);
-    const float wts = id <= last ? wt[min(lane, m.k_used - 1)] : 0.f;
+    const float wts = id > last ? 0.f : wt ? wt[min(lane, m.k_used - 1)] : 1.f;
 
     const int row_chunks = m.k / 256, nchunks = row_chunks * m.k_used;
     PackedMatVecArgs p;   // the activation: the row's gated columns one behind the other

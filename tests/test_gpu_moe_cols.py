@@ -226,3 +226,45 @@ def test_block_with_work_lists_from_the_grouping(dev, devbuf, t, down, window, f
     finally:
         dev.set_tuning(moe__form=0)
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("t,down,window,rows,n_ffn,n_embd,packed", [
+    (quant.Q4_K, quant.Q6_K, 256, 2, 1280, 768, False), (quant.Q6_K, quant.Q6_K, 32, 3, 512, 1024, False),
+    (quant.Q8_0, quant.Q8_0, 32, 4, 448, 320, False), (quant.Q4_K, quant.Q4_K, 256, 4, 768, 512, True),
+    (quant.Q4_K, quant.Q4_K, 256, 2, 2304, 256, True)], ids=lambda v: str(v))
+def test_dense_block_of_a_few_rows(dev, devbuf, t, down, window, rows, n_ffn, n_embd, packed):
+    """A dense block's two to four rows in two launches: one expert, no selection; the residual added to and nothing behind it."""
+    from test_gpu_moe import _oracle_block, _pack_bank
+    w = [synth.random_weights(t, n_ffn, n_embd, seed=1), synth.random_weights(t, n_ffn, n_embd, seed=2), synth.random_weights(down, n_embd, n_ffn, seed=3)]
+    x = np.stack([synth.activations(n_embd, seed=900 + r) for r in range(rows)])
+    start = np.stack([synth.activations(n_embd, seed=30 + r) for r in range(rows)])
+    sel, wt = np.zeros((rows, 2), np.uint32), np.full((rows, 1), 0.75, np.float32)
+    want = start + _oracle_block(t, *w, x, sel, wt, 1, n_ffn, n_embd, window, td=down)
+    dev.SetActWindow(window)
+    xd, sd, wd = devbuf(x), devbuf(sel), devbuf(wt)
+    try:
+        resid = devbuf(np.concatenate([start.reshape(-1), np.full(8, FILL)]))
+        args = (xd.ptr, sd.ptr, 2, wd.ptr, rows, 1, 1, n_ffn, n_embd)
+        before = dev.launch_count()
+        if packed:
+            hold = [_pack_bank(dev, devbuf, t, b, 1, r, k, "one") for b, (r, k) in zip(w, [(n_ffn, n_embd)] * 2 + [(n_embd, n_ffn)])]
+            before = dev.launch_count()
+            assert dev.moe_ffn_packed_dev(resid.ptr, t, *[b[0] for b in hold], *args)
+        else:
+            hold = [devbuf(b) for b in w]
+            if t == quant.Q8_0:   # (a mixture takes K in 256s: the dense block by its handle, weight one)
+                want = start + _oracle_block(t, *w, x, sel, np.ones_like(wt), 1, n_ffn, n_embd, window, td=down)
+                from jitllm_amd import _lib
+                assert dev.PrepLayer(0, _lib.LAYER_DENSE, t, n_embd, n_ffn, *w)
+                before = dev.launch_count()
+                assert dev.layer_ffn_dev(0, xd.ptr, resid.ptr, rows)
+            else:
+                assert dev.moe_ffn_dev(resid.ptr, t, *[b.ptr for b in hold], *args, down_type=down)
+        dev.synchronize()
+        assert dev.launch_count() - before == 2
+        got = resid.get()
+        assert np.all(got[rows * n_embd:] == FILL)
+        assert nmse(got[:rows * n_embd].reshape(rows, n_embd), want) <= 1e-6
+    finally:
+        dev.ReleaseLayers(0, 1)
+        dev.SetActWindow(32)
