@@ -321,11 +321,23 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
             stage(GemmIntC<1>{}, step + 1);
         }
     } else {
-        i32x16 acc[2][NPL];
-        f32x4 dav[4], dsv[4];
-        float pd = 0.f, pm = 0.f;   // the row scales of the tile whose sums wait in the other accumulator
+        // One operand: the sums start at the bits of M = 1.5 * 2^23, so that what comes out of the matrix core IS the float M + P
+        // (|P| <= 32 * 127 * 128 < 2^22), and P * d = fma(M + P, d, -M d) with -M d exact (d has 17 bits at most): no conversion.
+        constexpr bool MAGIC = NPL == 1;
+        i32x16 first = {0};
+        if constexpr (MAGIC) {
 #pragma unroll
-        for (int pl = 0; pl < NPL; pl++) acc[1][pl] = zero;
+            for (int e = 0; e < 16; e++) first[e] = 0x4B400000;
+            asm volatile("" : "+v"(first));   // (held in registers: as a constant it is moved in anew for every instruction)
+        }
+        // Three wavefronts a SIMD (Q8_0, two row tiles): a tile's scaling right behind its own matrix instruction, whose latency the
+        // other wavefronts fill; a second accumulator would be spilled.
+        constexpr bool ONE = MAGIC && !Q4 && RT == 2;
+        i32x16 acc[ONE ? 1 : 2][NPL];
+        f32x4 dav[4], dsv[4];
+        float pd = 0.f, pm = 0.f, pc = 0.f;   // the row scales of the tile whose sums wait in the other accumulator; -M * pd
+#pragma unroll
+        for (int pl = 0; pl < NPL; pl++) acc[ONE ? 0 : 1][pl] = zero;
 #pragma unroll
         for (int i = 0; i < 4; i++) { dav[i] = f32x4{0.f, 0.f, 0.f, 0.f}; dsv[i] = f32x4{0.f, 0.f, 0.f, 0.f}; }
         // o += the sums y, scaled; next: where the token scales of the block behind lie, which take each quarter's
@@ -335,8 +347,13 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
             for (int i = 0; i < 4; i++) {
 #pragma unroll
                 for (int e = 4 * i; e < 4 * i + 4; e++) {
-                    const i32 v = NPL == 2 ? (y[0][e] << 7) + y[NPL - 1][e] : y[0][e];
-                    o[e] = fmaf((float)v * dav[i][e & 3], pd, o[e]);
+                    if constexpr (MAGIC) {
+                        const i32 v = y[0][e];   // (a copy: bit_cast of a vector's element takes another element's bits)
+                        o[e] = fmaf(fmaf(__builtin_bit_cast(float, v), pd, pc), dav[i][e & 3], o[e]);
+                    } else {
+                        const i32 v = (y[0][e] << 7) + y[NPL - 1][e];
+                        o[e] = fmaf((float)v * dav[i][e & 3], pd, o[e]);
+                    }
                     if constexpr (Q4) o[e] = fmaf(dsv[i][e & 3], pm, o[e]);
                 }
                 if constexpr (decltype(MOVE)::value) {
@@ -368,13 +385,37 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
             for (int n = 0; n < 4 * RT; n++) {
                 const int b = n / RT, j = n % RT;
                 if (n + 1 < 4 * RT) read_w(n + 1);
+                if constexpr (ONE) {
+                    if (j == 0) {
 #pragma unroll
-                for (int pl = 0; pl < NPL; pl++) acc[n & 1][pl] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ring[b], wf[n & 1][pl], zero, 0, 0, 0);
+                        for (int i = 0; i < 4; i++) {
+                            dav[i] = *(const f32x4*)(sDa + b * 32 * TW + 8 * i);
+                            if constexpr (Q4) dsv[i] = *(const f32x4*)(sDs + b * 32 * TW + 8 * i);
+                        }
+                    }
+                    acc[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ring[b], wf[n & 1][0], first, 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    pd = dd[j][b];
+                    pc = -12582912.f * pd;
+                    if constexpr (Q4) pm = dm[j][b];
+                    if (j == RT - 1) {
+                        ring[b] = a_frag(nstep, b);
+                        part(nxt, step + 1, b);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    scale(GemmIntC<0>{}, acc[0], out[j], nullptr, nullptr);
+                    __builtin_amdgcn_sched_barrier(0);
+                    continue;
+                }
+#pragma unroll
+                for (int pl = 0; pl < NPL; pl++)
+                    acc[n & 1][pl] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ring[b], wf[n & 1][pl], MAGIC ? first : zero, 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 // the tile before
                 if (j == 0) scale(GemmIntC<1>{}, acc[1], out[RT - 1], sDa + b * 32 * TW, sDs + b * 32 * TW);
                 else scale(GemmIntC<0>{}, acc[(n + 1) & 1], out[j - 1], nullptr, nullptr);
                 pd = dd[j][b];
+                if constexpr (MAGIC) pc = -12582912.f * pd;
                 if constexpr (Q4) pm = dm[j][b];
                 if (j == RT - 1) {
                     ring[b] = a_frag(nstep, b);
@@ -384,7 +425,7 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
             }
             lds_barrier();
         }
-        scale(GemmIntC<0>{}, acc[1], out[RT - 1], nullptr, nullptr);
+        if constexpr (!ONE) scale(GemmIntC<0>{}, acc[1], out[RT - 1], nullptr, nullptr);
     }
     // store: lane = row (contiguous in memory), register = token
 #pragma unroll
