@@ -45,7 +45,7 @@ struct Tuning {
     int gemm_planes = 0;
     int gemm_few = 0;           // the int8 few-token form: 1 wherever it fits, 2 never
     int few_nt = 0, few_rt = 0, few_waves = 0;
-    int gemm_i8 = 0;            // the int8 tile forms, Q8_0: 1 / 2 ask for 128 x 128 / 128 x 64 tiles
+    int gemm_i8 = 0;            // the int8 tile forms, Q8_0: 1 / 2 / 3 ask for 128 x 128 / 128 x 64 / 256 x 128 tiles
     int moe_form = 0;
     int moe_g16 = 0;
     int gemm_fold = 0, gemm_fold_waves = 0;
@@ -890,7 +890,7 @@ int gemm_q4k_launch(jl_ctx* c, float* out, const void* w, const float* x, int nr
 // The int8 tile forms (kernels/gemm_i8.h): Q8_0, Q4_K and Q6_K with window 32, Q6_K with the k-quant window.
 struct I8Shape { int rt, tw; };
 unsigned gemm_i8_lds(const jl_ctx* c, int type, I8Shape f) {   // JL_GEMM_I8_LDS_BYTES
-    const unsigned planes = type == JL_TYPE_Q6_K ? 2 : 1, rows = 32u * f.rt * (4 / f.tw), mins = type == JL_TYPE_Q4_K;
+    const unsigned planes = type == JL_TYPE_Q6_K ? 2 : 1, rows = 32u * f.rt * (f.tw < 4 ? 4 / f.tw : 1), mins = type == JL_TYPE_Q4_K;
     return 2u * (planes * rows * 128u + (c->act_window == 32 ? (mins + 1) * (rows * 16u + 4u * 32u * f.tw * 4u) : 0u));
 }
 bool gemm_i8_applies(const jl_ctx* c, int type, int nrows, int k, int ntok) {
@@ -921,8 +921,14 @@ I8Plan gemm_i8_plan(const jl_ctx* c, int type, int nrows, int k, int ntok) {
     // of every type at 1 to 8 splits, 6 % each; the pick is within 5 % of the best split at all but eight of the 76.  (One
     // pair of constants for every type left the k-quants uncut: window 32, 512 tokens of 4096 x 4096 Q4_K 62 against 52
     // in two, Q6_K 80 against 66, 900 tokens of 1700 x 8192 112 against 85 and 143 against 105.)
-    const double many = type == JL_TYPE_Q8_0 ? 0.088 : q4 ? 0.114 : c->act_window == 32 ? 0.160 : 0.097;
-    const double alone = type == JL_TYPE_Q8_0 ? 0.125 : q4 ? 0.177 : c->act_window == 32 ? 0.241 : 0.131;
+    // (Q8_0's and Q4_K's since their sums come as floats: 512 to 2048 tokens of five shapes.)  Q8_0, 256 tokens x 128 rows on eight
+    // wavefronts, one workgroup a CU: a weight's narrow loads, which fill L1 under the 128-token tile (0.70 of 0.67 million cycles), serve
+    // twice the tokens; 2048 tokens of 4096 x 14336 330 -> 303, 1024 of 14336 x 4096 177 -> 160, 512 93 -> 85, but 1500 of 8192 x 2048,
+    // a round and a half, 84 (90 so).
+    struct Shape { int rt, tw, cap; double many, alone; };
+    static const Shape q8_shapes[] = {{4, 8, 1, 0.073, 0.146}, {4, 4, 2, 0.081, 0.115}, {2, 4, 3, 0.086, 0.122}};
+    const Shape one = {2, 4, 2, q4 ? 0.106 : c->act_window == 32 ? 0.160 : 0.097, q4 ? 0.165 : c->act_window == 32 ? 0.241 : 0.131};
+    const bool q8 = type == JL_TYPE_Q8_0;
     I8Shape f = {2, 4};
     int nsplit = 1;
     double best = 1e30;
@@ -932,9 +938,11 @@ I8Plan gemm_i8_plan(const jl_ctx* c, int type, int nrows, int k, int ntok) {
     const size_t n = (size_t)ntok * nrows, acts = (gemm_i8_acts(type, ntok, k) + 255) & ~(size_t)255;
     size_t most = acts < jl_static_scratch_bytes() ? jl_static_scratch_bytes() - acts : 0;
     if (reserved_for(c, ntok, k)) most = std::min(most, slab_reserve(c));
-    for (int rt : {4, 2}) {
-        if (type != JL_TYPE_Q8_0 ? rt == 4 : c->tune.gemm_i8 > 0 && rt != (c->tune.gemm_i8 == 1 ? 4 : 2)) continue;
-        const long cap = rt == 4 || type != JL_TYPE_Q8_0 ? 2 : 3, groups = (long)((ntok + 127) / 128) * ((nrows + 32 * rt - 1) / (32 * rt));
+    for (int i = 0; i < (q8 ? 3 : 1); i++) {
+        const Shape& h = q8 ? q8_shapes[i] : one;
+        if (q8 && c->tune.gemm_i8 > 0 && i != c->tune.gemm_i8 % 3) continue;
+        const int rt = h.rt, waves = h.tw / 4;   // (of a workgroup on a SIMD)
+        const long cap = h.cap, groups = (long)((ntok + 32 * h.tw - 1) / (32 * h.tw)) * ((nrows + 32 * rt - 1) / (32 * rt));
         for (int s = 1; s <= 8 && s <= nunit; s++) {
             if (c->tune.gemm_split > 0 && s != std::min(std::min(c->tune.gemm_split, 8), nunit)) continue;
             const int per = (nunit + s - 1) / s;
@@ -942,10 +950,10 @@ I8Plan gemm_i8_plan(const jl_ctx* c, int type, int nrows, int k, int ntok) {
             if (s > 1 && n * s * 4 > most) continue;
             const long wgs = groups * s, full = wgs / (cap * c->num_cu), left = wgs - full * cap * c->num_cu;
             const double block = 4 * rt * per * unit;     // of a wavefront
-            double us = full * (0.15 + many * cap * block);
-            if (left) us += 0.15 + std::max(many * ((left + c->num_cu - 1) / c->num_cu), alone) * block;
+            double us = full * (0.15 + h.many * waves * cap * block);
+            if (left) us += 0.15 + std::max(h.many * waves * ((left + c->num_cu - 1) / c->num_cu), h.alone) * block;
             if (s > 1) us += 0.25 + 1.16e-6 * (s + 1) * n;
-            if (us < best) { best = us; f = {rt, 4}; nsplit = s; }
+            if (us < best) { best = us; f = {rt, h.tw}; nsplit = s; }
         }
     }
     return {f, nsplit, best};
@@ -975,13 +983,13 @@ int gemm_i8_launch(jl_ctx* c, float* out, int type, const void* w, const float* 
     const I8Shape f = plan.f;
     const int nsplit = plan.nsplit;
     const size_t n = (size_t)ntok * nrows;
-    const int tt = 32 * f.tw, tr = 32 * f.rt * (4 / f.tw), per = (nunit + nsplit - 1) / nsplit;
+    const int tt = 32 * f.tw, tr = 32 * f.rt, per = (nunit + nsplit - 1) / nsplit;
     if (nsplit > 1) {
         rc = ws_ensure(c, &c->mx_ws, &c->mx_ws_bytes, n * nsplit * 4);
         if (rc != JL_OK) return rc;
         ga.out = (float*)c->mx_ws; ga.sb_per = per * unit;
     }
-    rc = launch(c, gemm_i8_name("jl_gemm", c, type, f), (unsigned)((ntok + tt - 1) / tt), (unsigned)((nrows + tr - 1) / tr), 256,
+    rc = launch(c, gemm_i8_name("jl_gemm", c, type, f), (unsigned)((ntok + tt - 1) / tt), (unsigned)((nrows + tr - 1) / tr), 64u * f.tw,
                 gemm_i8_lds(c, type, f), st, gp, (unsigned)nsplit);
     if (rc != JL_OK || nsplit == 1) return rc;
     SumPartsArgs sa;
@@ -2160,6 +2168,7 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
             names.push_back(nm);
         }
     names.push_back("jl_gemm_i8_q8_0_r4t4");
+    names.push_back("jl_gemm_i8_q8_0_r4t8");
     names.push_back("jl_moe_gemm_i8_q8_0_r4t4");
     for (const char* tag : {"q4k", "q4kw", "q8_0", "q6k", "q6kw"})
         for (const char* layout : {"rows", "planes"})

@@ -10,19 +10,18 @@
 // v_mfma_i32_32x32x32_i8 takes a block of 32 a time, exactly.  Q6_K's weight is sc * (q - 32), thirteen bits: it goes in
 // as two int8 operands, 128 * hi + lo, whose sums are put together as integers.
 //
-// What bounds it.  Window 32: both scales change every 32 of K, so an output element costs three vector
-// instructions a block (convert, times d_a, multiply-add with d) and the matrix cores wait for the vector unit: Q8_0,
-// 2048 tokens x 4096 -> 14336, 53 vector instructions a matrix instruction, the vector unit issuing all of the time, the
-// matrix cores 16 % (and L1, mostly the weights' narrow loads, 0.70 of 0.72 million cycles a CU); Q6_K, two operands and
-// two matrix instructions a block, 41 each, 86 % and 16 %.  As f16 operands (which this replaces: 460 us, now 384) it was
-// two an element beside two matrix instructions, and twice the LDS and L1 bytes and the conversion of every weight: in
-// registers alone that loop is the shorter (two f16 matrix instructions and 32 vector instructions 189 ns a SIMD with
-// three wavefronts, one int8 and 48 215, nothing of it hidden), as a kernel not.  Window 256 (551 us as f16 operands,
-// 14336 -> 4096, now 400): 12 vector instructions a matrix instruction, most of them the making of Q6_K's two operands,
-// which every workgroup of 128 tokens does anew; vector unit 43 %, matrix cores 27 %, L1 0.66 of 0.85 million cycles.
+// What bounds it.  Window 32: both scales change every 32 of K, so an output element costs vector instructions a block.  Q8_0 and
+// Q4_K: two, since the sums leave the matrix core as floats (below); with a conversion, a product and a multiply-add it was
+// three, 53 vector instructions a matrix instruction with everything else, now 37.  Q8_0, 2048 tokens x 4096 -> 14336, tiles of
+// 256 tokens x 128 rows: the vector unit issues 76 % of the time and the matrix instructions take most of the rest, the two do
+// not overlap on a SIMD; L1 0.35 of 0.69 million cycles (0.70 of 0.67 under tiles of 128 tokens, whose weights' narrow loads bound
+// it then): 320 us, 363 before, 460 as f16 operands.  Q6_K, two operands and two matrix instructions a block, 41 vector instructions
+// each, 86 % and 16 %.  Window 256 (551 us as f16 operands, 14336 -> 4096, now 400): 12 vector instructions a matrix instruction, most of
+// them the making of Q6_K's two operands, which every workgroup of 128 tokens does anew; vector unit 43 %, matrix cores 27 %, L1
+// 0.66 of 0.85 million cycles.
 //
-// A workgroup of four wavefronts owns 32 TW tokens x 32 RT (4 / TW) rows, a wavefront 32 tokens x 32 RT rows.  A stage is
-// 128 of K: the 256 threads turn the rows' bytes into operands in LDS (thread = row, block of 32), one stage ahead of
+// A workgroup of four wavefronts (TW = 8: eight) owns 32 TW tokens x 32 RT (4 / TW) rows, a wavefront 32 tokens x 32 RT rows.  A
+// stage is 128 of K: the threads turn the rows' bytes into operands in LDS (thread = row, block of 32), one stage ahead of
 // the matrix work and dealt over it, two buffers and one barrier a stage.  A tile's scaling runs under the next
 // tile's matrix instruction.  Rows sit on lanes (stores are contiguous), tokens on registers; activation fragments
 // come from L2 into a register ring a stage ahead.
@@ -117,7 +116,7 @@ template <> struct GemmI8Raw<JL_Q6_K> { u32x4 q[2], h[2]; u32 d; };   // d: the 
 template <int TYPE, bool W256, int RT, int TW>
 __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, int t0, int r0) {
     constexpr bool Q6 = TYPE == JL_Q6_K, Q4 = TYPE == JL_Q4_K;
-    constexpr int NPL = Q6 ? 2 : 1, ROWS = 32 * RT * (4 / TW), NB = ROWS / 64;
+    constexpr int NPL = Q6 ? 2 : 1, NW = TW > 4 ? TW : 4, ROWS = 32 * RT * (NW / TW), NB = ROWS / (16 * NW);
     constexpr int BUF = JL_GEMM_I8_BUF_BYTES(NPL, ROWS, TW, !W256, Q4), O_D = NPL * ROWS * 128, O_DA = O_D + ROWS * 16,
                   O_M = O_DA + 4 * 32 * TW * 4, O_DS = O_M + ROWS * 16;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -129,7 +128,7 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
     const int qb = tid & 3;
     const uint8_t* wrow[NB];
 #pragma unroll
-    for (int i = 0; i < NB; i++) wrow[i] = p.w + (size_t)min(r0 + (tid >> 2) + 64 * i, p.nrows - 1) * p.row_bytes;
+    for (int i = 0; i < NB; i++) wrow[i] = p.w + (size_t)min(r0 + (tid >> 2) + 16 * NW * i, p.nrows - 1) * p.row_bytes;
     GemmI8Raw<TYPE> raw[NB];
     float rda[2] = {0.f, 0.f}, rds[2] = {0.f, 0.f};
     auto load_w = [&](int step, int i) __attribute__((always_inline)) {
@@ -161,8 +160,8 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
     auto load_scales = [&](int step) __attribute__((always_inline)) {
         step = min(step, nsteps - 1);
 #pragma unroll
-        for (int u = 0; u < TW / 2; u++) {
-            const int idx = tid + 256 * u, b = idx / (32 * TW), t = min(t0 + idx % (32 * TW), p.tok_pad - 1);
+        for (int u = 0; u < 2 * TW / NW; u++) {
+            const int idx = tid + 64 * NW * u, b = idx / (32 * TW), t = min(t0 + idx % (32 * TW), p.tok_pad - 1);
             rda[u] = p.da[(size_t)(4 * step + b) * p.tok_pad + t];
             if constexpr (Q4) rds[u] = p.dsum[(size_t)(4 * step + b) * p.tok_pad + t];
         }
@@ -170,7 +169,7 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
     // Half h of the thread's block of row set i of stage `step`, as operand bytes in `buf`; with h = 0 its scales.
     auto slice = [&](uint8_t* buf, int step, int i, int h) __attribute__((always_inline)) {
         const GemmI8Raw<TYPE>& r = raw[i];
-        const int row = (tid >> 2) + 64 * i;
+        const int row = (tid >> 2) + 16 * NW * i;
         uint8_t* dst = buf + row * 128 + 16 * ((2 * qb + h) ^ (row & 7));
         float *sD = (float*)(buf + O_D) + row * 4 + qb, *sM = (float*)(buf + O_M) + row * 4 + qb;
         if constexpr (Q6) {
@@ -211,9 +210,9 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
     };
     auto put_scales = [&](uint8_t* buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < TW / 2; u++) {
-            ((float*)(buf + O_DA))[tid + 256 * u] = rda[u];
-            if constexpr (Q4) ((float*)(buf + O_DS))[tid + 256 * u] = rds[u];
+        for (int u = 0; u < 2 * TW / NW; u++) {
+            ((float*)(buf + O_DA))[tid + 64 * NW * u] = rda[u];
+            if constexpr (Q4) ((float*)(buf + O_DS))[tid + 64 * NW * u] = rds[u];
         }
     };
     // Part b (0..3) of the work that readies stage `step` in `buf`, and its places refilled with the stage behind it.

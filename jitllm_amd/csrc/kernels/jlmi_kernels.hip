@@ -282,6 +282,10 @@ __device__ __forceinline__ void moe_gemm_i8_tiles(const MoeGemmArgs& p) {
     JL_GEMM_I8_DENSE(T, TYPE, W256, 2, 4, OCC) JL_GEMM_I8_MOE(T, TYPE, W256, 2, 4, OCC) JL_GEMM_I8_MOE(T, TYPE, W256, 2, 2, OCC)
 JL_GEMM_I8_SHAPES(q8_0, JL_Q8_0, false, 3) JL_GEMM_I8_SHAPES(q4k, JL_Q4_K, false, 2) JL_GEMM_I8_SHAPES(q6k, JL_Q6_K, false, 2)
 JL_GEMM_I8_SHAPES(q6kw, JL_Q6_K, true, 2)
+extern "C" __global__ __launch_bounds__(512) void jl_gemm_i8_q8_0_r4t8(GemmArgs p) {
+    gemm_i8_split_slice<JL_Q8_0, false>(p);
+    gemm_i8_body<JL_Q8_0, false, 4, 8>(p, jl_smem, blockIdx.x * 256, blockIdx.y * 128);
+}
 JL_GEMM_I8_DENSE(q8_0, JL_Q8_0, false, 4, 4, 2) JL_GEMM_I8_MOE(q8_0, JL_Q8_0, false, 4, 4, 2)
 extern "C" __global__ __launch_bounds__(512) void jl_gemm_q4k_r128(GemmArgs p) {
     gemm_q4k_body<2>(p, jl_smem, blockIdx.x * JL_GEMM_TILE, blockIdx.y * 128);

@@ -76,3 +76,25 @@ def test_tiles_per_expert(dev, devbuf, t, window, nrows, k):
     finally:
         dev.set_tuning(moe__form=0)
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("nrows,k,ntok", [(1, 128, 257), (127, 640, 255), (129, 512, 513), (300, 1280, 256)])
+def test_tiles_of_256_tokens(dev, devbuf, nrows, k, ntok):
+    """Q8_0, 256 tokens x 128 rows on eight wavefronts: one token past a tile and one short of it, a wavefront and more without a
+    token of theirs, rows that end inside a tile, one stage of K; K slices."""
+    dev.SetActWindow(32)
+    w = synth.random_weights(quant.Q8_0, nrows, k, seed=nrows + k)
+    x = np.stack([synth.activations(k, seed=900 + i) * np.float32(1 + i % 3) for i in range(ntok)])
+    want = oracle.matmul_q8act_f64(quant.Q8_0, w, x, nrows, k, ntok, 32)
+    wd, xd = devbuf(w), devbuf(x)
+    try:
+        for split in (1, 3):
+            dev.set_tuning(gemm__i8=3, gemm__split=split)
+            o = devbuf(shape=(ntok * nrows + 8,), dtype=np.float32, fill=FILL)
+            assert dev.matmul_dev(o.ptr, quant.Q8_0, wd.ptr, xd.ptr, nrows, k, ntok)
+            dev.synchronize()
+            got = o.get()
+            assert np.all(got[ntok * nrows:] == FILL)
+            assert nmse(got[:ntok * nrows].reshape(ntok, nrows), want) <= 1e-10, split
+    finally:
+        dev.set_tuning(gemm__i8=0, gemm__split=0)
