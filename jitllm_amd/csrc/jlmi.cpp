@@ -1801,7 +1801,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     // The few-token kernel reads an expert's sheet once for 64 columns and the columns once for every row tile, so it
     // gives way to the tiles where the columns are the more; a tile of 64 columns needs two workgroups a CU.  With a
     // column or two an expert Q6_K's dot-product kernel is as fast while rows are short.  Q4_K with the k-quant window
-    // has the forms below, and the few-token kernel where moe_q4k_few finds it faster.
+    // has the forms below, and the few-token kernel where moe_few_faster finds it faster.
     {
         const bool q4w = type == JL_TYPE_Q4_K && c->act_window == 256, q6 = type == JL_TYPE_Q6_K;
         const int nmat = (planes ? pb1 != nullptr : bank1 != nullptr) ? 2 : 1;

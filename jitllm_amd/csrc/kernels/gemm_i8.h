@@ -321,8 +321,9 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
         }
     } else {
         // One operand: the sums start at the bits of M = 1.5 * 2^23, so that what comes out of the matrix core IS the float M + P
-        // (|P| <= 32 * 127 * 128 < 2^22), and P * d = fma(M + P, d, -M d) with -M d exact (d has 17 bits at most): no conversion.
-        constexpr bool MAGIC = NPL == 1;
+        // (|P| <= 32 * 127 * 128 < 2^22), and P * d = fma(M + P, d, -M d) with -M d exact (d has 17 bits at most): no conversion.  (A
+        // scale that is infinite makes its row NaN, where the product had made it infinite or NaN.)
+        constexpr bool MAGIC = NPL == 1 && !(Q4 && TW == 2);   // (that tile has no sixteen registers to spare)
         i32x16 first = {0};
         if constexpr (MAGIC) {
 #pragma unroll
@@ -350,7 +351,7 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
                         const i32 v = y[0][e];   // (a copy: bit_cast of a vector's element takes another element's bits)
                         o[e] = fmaf(fmaf(__builtin_bit_cast(float, v), pd, pc), dav[i][e & 3], o[e]);
                     } else {
-                        const i32 v = (y[0][e] << 7) + y[NPL - 1][e];
+                        const i32 v = NPL == 2 ? (y[0][e] << 7) + y[NPL - 1][e] : y[0][e];
                         o[e] = fmaf((float)v * dav[i][e & 3], pd, o[e]);
                     }
                     if constexpr (Q4) o[e] = fmaf(dsv[i][e & 3], pm, o[e]);
