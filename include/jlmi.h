@@ -96,15 +96,17 @@ int jl_synchronize(jl_ctx *ctx);
  * (fewest tokens sent to the matrix-core GEMM), "gemm.form" (1: 128 x 64 tiles, 2: 256 x 128
  * tiles, 3: two-pass, 4: up to 64 tokens on the int8 matrix cores, 5: 32 rows x 64 tokens a
  * workgroup, 6: 128 x 64 tiles over the whole of K on two groups of wavefronts, 9: token by
- * token), "gemm.few" (form 4: 1 for any number of tokens, 2 never), "few.nt" / "few.rt" /
+ * token), "gemm.few" (1: form 4 for any number of tokens, 2: never,
+ * 3: a decode matvec a token in one launch, up to eight), "few.nt" / "few.rt" /
  * "few.waves" (its token tiles, row tiles and wavefronts a workgroup), "gemm.i8" (the int8 tiles of
- * Q8_0: 1 / 2 for 128 x 128 / 128 tokens x 64 rows), "gemm.rows" (64 or 128),
+ * Q8_0: 1 / 2 / 3 for 128 x 128 / 128 tokens x 64 rows / 256 x 128), "matvec.lanes" (lanes a row of a decode matvec: 16, 32, 64), "gemm.rows" (64 or 128),
  * "gemm.split" (K slices), "gemm.prep" (4: the four-wavefront activation prep), "gemm.planes"
  * (2: restore rows from planes before the GEMM), "packed.rw" (rows per wavefront of the
  * packed-plane matvec: 16, 32, 64), "packed.block" (its threads per workgroup), "moe.shares"
- * (row shares an expert's matrix is split into), "moe.form" (grouped matmul: 1 dot products,
+ * (row shares an expert's matrix is split into), "moe.form" (grouped matmul: 10 a decode matvec a column, 1 dot products,
  * 2 / 3 groups of 32 / 16 columns on the matrix cores, 4 the prefill tile per expert, 5 the int8
- * few-token kernel, 6 / 7 / 8 the int8 tiles of 128 columns x 64 rows, 64 x 128 and (Q8_0) 128 x 128),
+ * few-token kernel, 6 / 7 / 8 the int8 tiles of 128 columns x 64 rows, 64 x 128 and (Q8_0) 128 x 128,
+ * 9 columns against rows decoded in registers; a routed block: 11 a handful of pairs without grouping),
  * "moe.group16" (form 3: 1 a prep kernel quantizes the columns, 2 the matrix kernel does, 3 groups
  * of 32 columns),
  * "moe.chunk" (form 3: super-blocks a step, 1-3),
@@ -335,8 +337,9 @@ int jl_matvec_packed_group(jl_ctx *ctx, int n, float *const *outs, const int *ty
 /* JIT.MatMulPacked / MatMul semantics on resident operands (engine/nn/packedmm.go:23,
  * matmul.go:27): x [ntok][k] f32 -> out [ntok][nrows], every token quantized on
  * its own.  From two (Q8_0) or three tokens a quantize-and-lay-out kernel and a matrix-core
- * kernel, in a workspace the context owns: up to 64 tokens the int8 few-token kernel, any
- * window; more on f16 tiles (Q4_K, window 256) or int8 tiles (window 32; Q6_K also 256).
+ * kernel, in a workspace the context owns: few tokens (up to 64, and more where it is estimated
+ * faster) the int8 few-token kernel, any window; more on f16 tiles (Q4_K, window 256) or int8 tiles (window 32;
+ * Q6_K also 256).  Up to eight tokens may run as a decode matvec each, in one launch and without a workspace.
  * Other cases run one fused matvec launch per token, which the reference also falls
  * back to (engine/model/prefill.go:1036-1041).  The workspace grows on demand
  * (a device allocation); jl_reserve sizes it ahead of time. */
@@ -376,8 +379,8 @@ int jl_reserve(jl_ctx *ctx, int max_tok, int max_k);
  * jl_layer_ffn_dev runs block li for n rows: h [n][n_embd] in, resid [n][n_embd] updated, both in
  * device memory (they may be one buffer, as they are for a block with its norm in front: every
  * launch that reads a row of h has been enqueued before the one that adds to it).  One row runs the
- * decode kernels (two launches for a dense block); more rows of a dense block two few-token
- * matmuls (up to 64 rows) or three prefill GEMMs (with norm_w set its rows run one at a time), of
+ * decode kernels (two launches for a dense block); more rows of a dense block decode matvecs in two
+ * launches (up to four rows), two few-token matmuls (up to 64) or three prefill GEMMs (with norm_w set its rows run one at a time), of
  * a mixture its grouped kernels.  The values are those of the pointer-form entry points
  * on the same operands, bit for bit.  Workspaces are the context's (calls on one context are
  * serialized by the caller).
@@ -475,7 +478,7 @@ int jl_matvec_packed_q8_dev(jl_ctx *ctx, float *out, int type, const uint32_t *q
                             int k, void *stream);
 
 /* JIT.MatMulPacked on resident planes (engine/nn/packedmm.go:23-139).  From two (Q8_0) or
- * three tokens up to 64 the int8 few-token kernel reads the planes where they lie, and so do
+ * three tokens the int8 few-token kernel (up to 64 tokens, and more where it is estimated faster) reads the planes where they lie, and so do
  * the Q4_K tiles of the 256 window; the int8 tiles, and the Q4_K form for grids of a round of 32-row
  * workgroups, take the row range restored to GGUF order in a workspace the context owns.
  * Other cases run one packed matvec launch per token. */

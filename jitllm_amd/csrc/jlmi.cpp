@@ -43,7 +43,7 @@ struct Tuning {
     int gemm_split = 0;
     int gemm_prep = 0;
     int gemm_planes = 0;
-    int gemm_few = 0;           // the int8 few-token form: 1 wherever it fits, 2 never
+    int gemm_few = 0;           // the int8 few-token form: 1 wherever it fits, 2 never; 3: decode matvecs in one launch
     int few_nt = 0, few_rt = 0, few_waves = 0;
     int gemm_i8 = 0;            // the int8 tile forms, Q8_0: 1 / 2 / 3 ask for 128 x 128 / 128 x 64 / 256 x 128 tiles
     int moe_form = 0;

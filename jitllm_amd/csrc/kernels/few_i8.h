@@ -15,6 +15,10 @@
 //   * A workgroup owns 16 RT rows and up to 16 NT columns; its wavefronts split K (wavefront w takes
 //     super-blocks w, w + nwaves, ...: a row's bytes are asked for side by side) and their partial tiles
 //     are added through LDS in wavefront order: one launch after the prep.
+//   * More tokens than a workgroup's columns: groups of tgroup token tiles on grid y, each of which reads the weights
+//     again (from L2 while the groups of a row tile run together).  64 tokens in smaller groups where more workgroups are
+//     worth it (1.025 over 17 to 64 tokens), and beyond 64 where the estimates put it before the tiles: 208 drawn
+//     matmuls of 60 to 780 tokens 1.175 times as fast as without.
 //   * L1 would be the next bound after memory: a vector load costs it one access for every 64-byte line that a
 //     quad of ADJACENT lanes touches, so the matrix operand's own lane order (lane % 16 = row) would cost 64
 //     accesses a 1 KiB load where 16 do.  GGUF rows are therefore loaded along the row, 16 bytes a lane, and
