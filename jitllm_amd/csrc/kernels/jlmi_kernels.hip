@@ -394,12 +394,8 @@ JL_MOE_PLANES_GATHER(16) JL_MOE_PLANES_GATHER(32) JL_MOE_PLANES_GATHER(64)
     extern "C" __global__ __launch_bounds__(256) void jl_moe_cols_prep_##T(MoeColsPrepArgs p) { moe_cols_prep_body<KO>(p); }      \
     extern "C" __global__ __launch_bounds__(256, 2) void jl_moe_cols_##T(MoeColsArgs p) { moe_cols_body<KO>(p, jl_smem); }
 JL_MOE_COLS(q4k, 0) JL_MOE_COLS(q4k_planes, 1) JL_MOE_COLS(q6k, 2)
-// grid = (ceil(n_embd/256), rows), block = 256
-extern "C" __global__ __launch_bounds__(256) void jl_moe_combine(MoeCombineArgs p) {
-    __shared__ float swt[16];
-    __shared__ u32 spos[16];
-    moe_combine_body(p, swt, spos);
-}
+// grid = (ceil(n_embd/4/256), rows), block = 256
+extern "C" __global__ __launch_bounds__(256) void jl_moe_combine(MoeCombineArgs p) { moe_combine_body(p); }
 
 // ------------------------------------------------------------------- MXFP4
 // grid = (ceil(ntok/128), ceil(nrows/128), K splits), block = 256, dynamic LDS = 4 stages of 128 x 272 B

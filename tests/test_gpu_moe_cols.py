@@ -268,3 +268,25 @@ def test_dense_block_of_a_few_rows(dev, devbuf, t, down, window, rows, n_ffn, n_
     finally:
         dev.ReleaseLayers(0, 1)
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("k_used,n_embd", [(1, 4), (2, 1020), (8, 1024), (9, 1028), (16, 2052)])
+def test_combine_bits(dev, devbuf, k_used, n_embd):
+    """The weighted sum at the edges of its groups of eight experts and of its workgroups of 1024 columns: one f32 product and
+    one f32 addition an expert, ascending ids, ids that are equal in slot order (bit for bit)."""
+    rows = 3
+    rng = np.random.default_rng(k_used)
+    sel = rng.permuted(np.tile(np.arange(20, dtype=np.uint32), (rows, 1)), axis=1)[:, :k_used + 2].copy()
+    sel[1, :k_used] = 7
+    wt = rng.random((rows, k_used), dtype=np.float32)
+    pos = rng.permutation(rows * k_used).astype(np.uint32)
+    y = rng.standard_normal((rows * k_used, n_embd)).astype(np.float32)
+    resid = rng.standard_normal((rows, n_embd)).astype(np.float32)
+    want = resid.copy()
+    for r in range(rows):
+        for s in np.argsort(sel[r, :k_used], kind="stable"):
+            want[r] = want[r] + wt[r, s] * y[pos[r * k_used + s]]
+    rd, yd, wd, sd, pd = devbuf(resid), devbuf(y), devbuf(wt), devbuf(sel), devbuf(pos)
+    assert dev.moe_combine_dev(rd.ptr, yd.ptr, wd.ptr, sd.ptr, k_used + 2, pd.ptr, rows, k_used, n_embd)
+    dev.synchronize()
+    assert np.array_equal(rd.get().view(np.uint32), want.view(np.uint32))
