@@ -529,7 +529,8 @@ int jl_moe_route_dev(jl_ctx *ctx, const float *logits, int rows, int n_expert, i
  * jit/gpu/tier/grouppairs_test.go:91-122, with unit 1): sel [rows][sel_stride] holds
  * each row's k_used expert ids first.  Fills start [n_expert+1] (first column of each
  * expert's run), perm [rows*k_used] (column -> row) and pos [rows*k_used]
- * (pair r*k_used+s -> column); experts ascending, pairs in (row, slot) order. */
+ * (pair r*k_used+s -> column); experts ascending, pairs in (row, slot) order.  A pair whose id
+ * no expert has is left out: its pos, and perm from start[n_expert] on, are not written. */
 int jl_moe_group_dev(jl_ctx *ctx, const uint32_t *sel, int sel_stride, int rows, int k_used,
                      int n_expert, uint32_t *start, uint32_t *perm, uint32_t *pos, void *stream);
 
@@ -538,8 +539,9 @@ int jl_moe_group_dev(jl_ctx *ctx, const uint32_t *sel, int sel_stride, int rows,
  * engine/nn/packedmulti.go:24,93): for every column c of expert e,
  *   out0[c][0:nrows] = bank0 sheet e . act(c)   (and out1 / bank1 when given),
  * act(c) = x[src[c]] (src NULL: x[c]) or silu(x[..]) * x2[..] when x2 is given.  A bank
- * is n_expert sheets of nrows x k GGUF rows back to back.  ncols = start[n_expert], the
- * number of columns (rows * k_used).  Activations are quantized per column exactly as
+ * is n_expert sheets of nrows x k GGUF rows back to back.  ncols = the number of columns (rows *
+ * k_used); columns from start[n_expert] on belong to no expert and what out holds of them is
+ * undefined.  Activations are quantized per column exactly as
  * jl_matvec_dev does, once, into a workspace the context owns (grown on demand). */
 int jl_moe_matvec_dev(jl_ctx *ctx, float *out0, float *out1, int type, const void *bank0,
                       const void *bank1, const float *x, const float *x2, const uint32_t *src,
@@ -557,6 +559,7 @@ int jl_moe_combine_dev(jl_ctx *ctx, float *resid, const float *y, const float *w
  * (engine/model/moe.go:510-761): group, gate and up in one launch, act(gate)*up fused
  * into the down launch's quantizer, combine into resid [rows][n_embd] (accumulated).
  * gate/up banks: n_expert sheets of n_ffn x n_embd; down bank: n_embd x n_ffn.
+ * A pair whose id no expert has adds nothing.
  * Intermediates live in a workspace the context owns (grown on demand). */
 int jl_moe_ffn_dev(jl_ctx *ctx, float *resid, int type, const void *gate_bank,
                    const void *up_bank, const void *down_bank, const float *x,

@@ -1957,7 +1957,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
         MoeQuantArgs qa;
         qa.x = x; qa.x2 = x2; qa.src = src;
         qa.q = nullptr; qa.as = nullptr; qa.s16 = nullptr; qa.chunked = (uint32_t*)c->moe_q_ws;
-        qa.k = k; qa.per = c->act_window / 32;
+        qa.k = k; qa.per = c->act_window / 32; qa.start = start; qa.n_expert = n_expert;
         void* qparams[] = {&qa};
         rc = launch(c, "jl_moe_quant", (unsigned)((k / 4 + 255) / 256), (unsigned)ncols, 256, 0, st, qparams);
         if (rc != JL_OK) return rc;
@@ -2060,7 +2060,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     MoeQuantArgs qa;
     qa.x = x; qa.x2 = x2; qa.src = src;
     qa.q = (int8_t*)qws; qa.as = (float*)(qws + o_as); qa.s16 = (float*)(qws + o_s16);
-    qa.k = k; qa.per = c->act_window / 32;
+    qa.k = k; qa.per = c->act_window / 32; qa.start = start; qa.n_expert = n_expert;
     void* qparams[] = {&qa};
     rc = launch(c, "jl_moe_quant", (unsigned)((k / 4 + 255) / 256), (unsigned)ncols, 256, 0, st, qparams);
     if (rc != JL_OK) return rc;
@@ -2740,9 +2740,10 @@ int jl_moe_matvec_packed_dev(jl_ctx* c, float* out0, float* out1, int type, cons
                              pick_stream(c, stream), bank0, bank1);
 }
 
-int jl_moe_combine_dev(jl_ctx* c, float* resid, const float* y, const float* wt, const uint32_t* sel,
-                       int sel_stride, const uint32_t* pos, int rows, int k_used, int n_embd, void* stream) {
-    if (!c) return JL_ERR_ARG;
+namespace {
+// last_id: ids past it are no expert's and add nothing.
+int moe_combine_launch(jl_ctx* c, float* resid, const float* y, const float* wt, const uint32_t* sel, int sel_stride, const uint32_t* pos,
+                       int rows, int k_used, int n_embd, uint32_t last_id, hipStream_t st) {
     if (!resid || !y || !wt || !sel || !pos || rows <= 0 || n_embd <= 0)
         return fail(c, JL_ERR_ARG, "moe combine: bad operand");
     if (k_used <= 0 || k_used > 16 || sel_stride < k_used || rows > 65535) return JL_DECLINED;
@@ -2750,10 +2751,17 @@ int jl_moe_combine_dev(jl_ctx* c, float* resid, const float* y, const float* wt,
     HIP_TRY(c, H->SetDevice(c->device));
     MoeCombineArgs a;
     a.resid = resid; a.y = y; a.wt = wt; a.sel = sel; a.pos = pos;
-    a.sel_stride = sel_stride; a.k_used = k_used; a.n_embd = n_embd;
+    a.sel_stride = sel_stride; a.k_used = k_used; a.n_embd = n_embd; a.last_id = last_id;
     void* params[] = {&a};
-    return launch(c, "jl_moe_combine", (unsigned)((n_embd / 4 + 255) / 256), (unsigned)rows, 256, 0,
-                  pick_stream(c, stream), params);
+    return launch(c, "jl_moe_combine", (unsigned)((n_embd / 4 + 255) / 256), (unsigned)rows, 256, 0, st, params);
+}
+}  // namespace
+
+// (how many experts there are is not known here: every id counts)
+int jl_moe_combine_dev(jl_ctx* c, float* resid, const float* y, const float* wt, const uint32_t* sel,
+                       int sel_stride, const uint32_t* pos, int rows, int k_used, int n_embd, void* stream) {
+    if (!c) return JL_ERR_ARG;
+    return moe_combine_launch(c, resid, y, wt, sel, sel_stride, pos, rows, k_used, n_embd, 0xFFFFFFFFu, pick_stream(c, stream));
 }
 
 namespace {
@@ -2923,7 +2931,7 @@ int moe_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate_b
     rc = moe_matvec_launch(c, y, nullptr, down_type, down_bank, nullptr, g, u, nullptr, start, n_expert, (int)ncols, n_embd, n_ffn, st,
                            pd, nullptr, 0, &w.lists);
     if (rc != JL_OK) return rc;
-    return jl_moe_combine_dev(c, resid, y, wt, sel, sel_stride, pos, rows, k_used, n_embd, st);
+    return moe_combine_launch(c, resid, y, wt, sel, sel_stride, pos, rows, k_used, n_embd, (uint32_t)n_expert - 1u, st);
 }
 
 // The whole block from the hidden state on: router logits, softmax + top-k, the routed

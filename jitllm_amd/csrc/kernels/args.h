@@ -343,6 +343,8 @@ struct MoeQuantArgs {
     float* as;
     float* s16;
     int k, per;
+    const uint32_t* start;  // [n_expert + 1]: columns from start[n_expert] on belong to no expert and are left alone
+    int n_expert;
     // chunked form (q, as, s16 unused): column c's 256-element chunk i as 88 consecutive words at
     // chunked + (c * k/256 + i) * 88 -- 64 of int8 values, 8 scales, 16 half-block sums -- so a
     // reader addresses everything it needs of a (column, chunk) from one base
@@ -386,8 +388,9 @@ struct MoeCombineArgs {
     const float* y;         // [ncols][n_embd]
     const float* wt;        // [rows][k_used]
     const uint32_t* sel;    // [rows][sel_stride]
-    const uint32_t* pos;    // [rows*k_used]
+    const uint32_t* pos;    // [rows*k_used]; not read for an id that no expert has
     int sel_stride, k_used, n_embd;
+    uint32_t last_id;       // ids past this one are no expert's and add nothing
 };
 
 // MXFP4 weights x bf16 activations: out [ntok][nrows] f32.

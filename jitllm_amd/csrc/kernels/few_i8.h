@@ -68,12 +68,16 @@ __device__ __forceinline__ void few_i8_prep_body(const FewI8PrepArgs& args) {
     const u32 c = blockIdx.y * 4 + wave;
     if (c >= (u32)p.ncols) return;   // whole wavefronts, no barrier below
     const int ch = blockIdx.x, g4 = ch * 64 + lane;
-    const size_t row = p.src ? p.src[c] : c;
+    // (a column of no expert -- the grouping leaves ids that no expert has out -- has no source row either)
+    const u32 ncols = p.start ? p.start[p.n_expert] : (u32)p.ncols;
+    u32 row = p.src ? p.src[c] : c;
+    if (c >= ncols) row = 0;
     const bool live = g4 < p.k / 4;
     const int gc = live ? g4 : p.k / 4 - 1;
     f32x4 v = ((const f32x4*)(p.x + row * (size_t)p.k))[gc];
     f32x4 u = {0.f, 0.f, 0.f, 0.f};
     if (p.x2) u = ((const f32x4*)(p.x2 + row * (size_t)p.k))[gc];
+    if (c >= ncols) return;   // the whole wavefront
     u32 slot = c >> 4, i = c & 15;
     if (p.start) {
         // the column's expert: the last whose first column is not past it

@@ -470,7 +470,9 @@ __device__ __forceinline__ void moe_matvec_planes_body(const MoePlanesArgs& p, u
 // grid = (ceil(k/4/256), ncols), block = 256: one thread per four elements of a column.
 __device__ __forceinline__ void moe_quant_body(const MoeQuantArgs& p) {
     const size_t c = blockIdx.y;
+    const u32 ncols = p.start[p.n_expert];
     const size_t src = p.src ? p.src[c] : c;
+    if (c >= ncols) return;   // uniform
     const int g4 = blockIdx.x * 256 + threadIdx.x;
     const bool live = g4 < p.k / 4;
     f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -935,6 +937,7 @@ __device__ __forceinline__ void moe_g16_prep_body(const MoeG16PrepArgs& p, u32* 
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) c_lo = max(c_lo, (u32)__shfl_xor((int)c_lo, off, 64));
     const int e = (int)cnt - 1;
+    if (e >= p.n_expert) return;   // (the whole wavefront: a column of no expert, whose source row nobody wrote)
     const u32 rel = c - c_lo;
     const size_t slot = (size_t)(c_lo >> 4) + (size_t)e + (rel >> 4);
     const int i = (int)(rel & 15);
@@ -1328,7 +1331,7 @@ __device__ __forceinline__ void moe_g16_body(const MoeG16Args& p, uint8_t* smem)
 // of mostly cached reads), 64 rows 5.2 -> 4.9.
 __device__ __forceinline__ void moe_combine_body(const MoeCombineArgs& args) {
     MoeCombineArgs p = args;
-    JL_NOW(p.resid, p.y, p.wt, p.sel, p.pos, p.sel_stride, p.k_used, p.n_embd);
+    JL_NOW(p.resid, p.y, p.wt, p.sel, p.pos, p.sel_stride, p.k_used, p.n_embd, p.last_id);
     const u32 r = blockIdx.y;
     const int ku = p.k_used, lane = threadIdx.x & 63;
     const int n4 = p.n_embd >> 2, n = blockIdx.x * 256 + threadIdx.x, nc = min(n, n4 - 1);
@@ -1338,6 +1341,7 @@ __device__ __forceinline__ void moe_combine_body(const MoeCombineArgs& args) {
     const i32 mine = (i32)as_global(p.sel)[(size_t)r * p.sel_stride + slot];
     const float wt = as_global(p.wt)[(size_t)r * ku + slot];
     const i32 at = (i32)as_global(p.pos)[(size_t)r * ku + slot];
+    const int have = (int)__builtin_popcountll(__ballot(lane < ku && (u32)mine <= p.last_id));   // (the other ids' ranks are behind these)
     f32x4 acc = res[nc];
     int rank = 0;   // a stable rank: equal ids (not a valid routing) keep their slot order
     for (int j = 0; j < ku; j++) {
@@ -1348,14 +1352,14 @@ __device__ __forceinline__ void moe_combine_body(const MoeCombineArgs& args) {
     const i32 spos = __builtin_amdgcn_ds_permute(to, at), swt = __builtin_amdgcn_ds_permute(to, __builtin_bit_cast(i32, wt));
     // eight experts' rows requested together (a loop of load, add, load, ... is a chain of trips to
     // memory), added in ascending expert order
-    for (int i0 = 0; i0 < ku; i0 += 8) {
+    for (int i0 = 0; i0 < have; i0 += 8) {
         f32x4 y[8];
 #pragma unroll
         for (int b = 0; b < 8; b++)
-            y[b] = (y4 + (size_t)(u32)__builtin_amdgcn_readlane(spos, min(i0 + b, ku - 1)) * n4)[nc];
+            y[b] = (y4 + (size_t)(u32)__builtin_amdgcn_readlane(spos, min(i0 + b, have - 1)) * n4)[nc];
 #pragma unroll
         for (int b = 0; b < 8; b++) {
-            if (i0 + b < ku) {   // uniform
+            if (i0 + b < have) {   // uniform
                 const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(swt, i0 + b));
                 acc = f32x4{acc.x + w * y[b].x, acc.y + w * y[b].y, acc.z + w * y[b].z, acc.w + w * y[b].w};
             }
@@ -1387,10 +1391,14 @@ __device__ __forceinline__ void moe_gather_body(const MoeGatherArgs& args, uint8
         row = c; e = 0;
     } else if (!start) {
         row = c / (u32)p.k_used;
-        // (an id no expert has: its weight is none, see moe_gather_down_body)
+        // (an id no expert has: the last sheet, for a pair that adds nothing, see moe_gather_down_body)
         e = min((u32)__builtin_amdgcn_readfirstlane((i32)sel[row * (u32)p.sel_stride + (c - row * (u32)p.k_used)]), (u32)p.n_expert - 1u);
     } else {
+        // (a column of no expert -- the grouping leaves ids that no expert has out -- has no source row either: the first row and
+        // the last sheet, for a result that nobody reads.  start[n_expert] is on its way with src[c].)
+        const u32 ncols = (u32)__builtin_amdgcn_readfirstlane((i32)start[p.n_expert]);
         row = src ? (u32)__builtin_amdgcn_readfirstlane((i32)src[c]) : c;
+        if (c >= ncols) row = 0;
         // the column's expert: the last whose first column is not past it
         u32 cnt = 0;
         for (int base = 0; base <= p.n_expert; base += 64) {
@@ -1398,7 +1406,7 @@ __device__ __forceinline__ void moe_gather_body(const MoeGatherArgs& args, uint8
             const u32 s = start[min(idx, p.n_expert)];
             cnt += (u32)__builtin_popcountll(__ballot(idx <= p.n_expert && s <= c));
         }
-        e = cnt - 1;
+        e = min(cnt - 1, (u32)p.n_expert - 1u);
     }
     out = as_global(out) + (size_t)c * nrows;
     w0 = as_global(w0) + (size_t)e * p.sheet_bytes;
@@ -1461,7 +1469,7 @@ __device__ __forceinline__ void moe_gather_down_body(const MoeGatherDownArgs& ar
     float* resid = as_global(p.resid) + tok * nrows;
     const u32 last = (u32)p.n_expert - 1u;
     const ActLds A = act_lds_views(smem, k);
-    // behind the staging area: a pair's expert and its weight (an id no expert has: none)
+    // behind the staging area: a pair's id and its weight (an id no expert has: the last sheet is read for it and nothing added)
     u32* se = (u32*)(smem + (((TYPE == JL_Q8_0P ? JL_ACT_LDS_BYTES_SHIFTED(k) : JL_ACT_LDS_BYTES(k)) + 15) & ~15));
     float* sw = (float*)(se + 16);
     const int sub = lane / LPR, l = lane % LPR;
@@ -1480,8 +1488,8 @@ __device__ __forceinline__ void moe_gather_down_body(const MoeGatherDownArgs& ar
     typename T::W w;
     T::load_w(bank + (size_t)e0 * p.sheet_bytes + (size_t)min(r0 + sub, nrows - 1) * p.row_bytes, s0 - pair0 * row_slots, w);
     if ((int)threadIdx.x < p.k_used) {
-        se[threadIdx.x] = min(em, last);
-        sw[threadIdx.x] = em <= last ? wm : 0.f;
+        se[threadIdx.x] = em;
+        sw[threadIdx.x] = wm;
     }
     auto stage_group = [&](int g4, f32x4 v, f32x4 f) __attribute__((always_inline)) {
         v = f32x4{silu_f32(v.x) * f.x, silu_f32(v.y) * f.y, silu_f32(v.z) * f.z, silu_f32(v.w) * f.w};
@@ -1501,11 +1509,13 @@ __device__ __forceinline__ void moe_gather_down_body(const MoeGatherDownArgs& ar
         float acc = 0.f;
         for (int slot = l; slot < nslots; slot += LPR) {
             const int pair = (int)__umulhi((u32)slot, p.slots_inv), s = slot - pair * row_slots;
-            if (!preloaded) T::load_w(bank + (size_t)se[pair] * p.sheet_bytes + (size_t)r * p.row_bytes, s, w);
+            const u32 id = se[pair];
+            if (!preloaded) T::load_w(bank + (size_t)min(id, last) * p.sheet_bytes + (size_t)r * p.row_bytes, s, w);
             preloaded = false;
             typename T::Act a;
             T::load_act(A, slot, a);
-            acc = fmaf(sw[pair], T::dot(w, s, a), acc);
+            const float more = fmaf(sw[pair], T::dot(w, s, a), acc);
+            acc = id <= last ? more : acc;
         }
         preloaded = false;
         const float t = group_sum<LPR>(acc);

@@ -22,7 +22,7 @@ __device__ __forceinline__ void moe_planes_gather_body(const MoePlanesGatherArgs
     int row_step = m.row_step, ku = m.k_used, sel_stride = m.sel_stride, n_expert = m.n_expert;
     JL_NOW(p.out, p.qs, p.d, p.sc, p.x, p.nrows, p.k, p.stride, p.per, p.nwaves, p.ngroups, sel, words, row_step, ku, sel_stride, n_expert);
     const u32 row = sel ? c / (u32)ku : c;
-    // (no selection: one matrix; an id no expert has: its weight is none, see below)
+    // (no selection: one matrix; an id no expert has: the last sheet, for a pair that adds nothing, see below)
     const u32 e = !sel ? 0u : min((u32)__builtin_amdgcn_readfirstlane((i32)as_global(sel)[row * (u32)sel_stride + (c - row * (u32)ku)]), (u32)n_expert - 1u);
     p.out = as_global(p.out) + (size_t)c * p.nrows;
     p.qs = as_global(p.qs) + (size_t)e * words; p.d = as_global(p.d) + (size_t)e * words; p.sc = as_global(p.sc) + (size_t)e * words;
@@ -44,10 +44,9 @@ __device__ __forceinline__ void moe_planes_down_body(const MoePlanesDownArgs& ar
     int g = blockIdx.x;
     if ((m.ngroups & 7) == 0) g = (g & 7) * (m.ngroups >> 3) + (g >> 3);   // (neighbouring row runs to one XCD, as above)
     const int rl = lane % RW, b0 = lane / RW * NB, rr = min(g * RW + rl, m.nrows - 1);
-    // lane i holds pair i's expert and weight (an id no expert has: none)
-    const u32 last = (u32)m.n_expert - 1u, id = sel ? sel[min(lane, m.k_used - 1)] : 0u;
-    const u32 ids = min(id, last);
-    const float wts = id > last ? 0.f : wt ? wt[min(lane, m.k_used - 1)] : 1.f;
+    // lane i holds pair i's id and weight (an id no expert has: the last sheet is read for it and nothing added)
+    const u32 last = (u32)m.n_expert - 1u, ids = sel ? sel[min(lane, m.k_used - 1)] : 0u;
+    const float wts = wt ? wt[min(lane, m.k_used - 1)] : 1.f;
 
     const int row_chunks = m.k / 256, nchunks = row_chunks * m.k_used;
     PackedMatVecArgs p;   // the activation: the row's gated columns one behind the other
@@ -64,13 +63,15 @@ __device__ __forceinline__ void moe_planes_down_body(const MoePlanesDownArgs& ar
     float acc = 0.f;
     auto chunk = [&](int c, const PkX<true>& Xc) __attribute__((always_inline)) {
         const int pair = c / row_chunks, cc = c - pair * row_chunks;   // (uniform)
-        const size_t e = (u32)__builtin_amdgcn_readlane((i32)ids, pair);
+        const u32 id = (u32)__builtin_amdgcn_readlane((i32)ids, pair);
+        const size_t e = min(id, last);
         p.qs = qs + e * m.sheet_words; p.d = d + e * m.sheet_words; p.sc = sc + e * m.sheet_words;
         const int row = (int)e * m.row_step + rr;
         PkWQ4K<NB> w;
         pk_load<NB>(p, cc, b0, row, w);
         pk_stage_x<true, true>(p, c, lane, Xc, my);
-        acc = fmaf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(i32, wts), pair)), pk_dot<NB>(p, w, cc, b0, row, A), acc);
+        const float more = fmaf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(i32, wts), pair)), pk_dot<NB>(p, w, cc, b0, row, A), acc);
+        acc = id <= last ? more : acc;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };

@@ -290,3 +290,51 @@ def test_combine_bits(dev, devbuf, k_used, n_embd):
     assert dev.moe_combine_dev(rd.ptr, yd.ptr, wd.ptr, sd.ptr, k_used + 2, pd.ptr, rows, k_used, n_embd)
     dev.synchronize()
     assert np.array_equal(rd.get().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("t,down,window,forms", [
+    (quant.Q4_K, quant.Q4_K, 256, ((0, 0), (1, 0), (2, 0), (3, 1), (3, 2), (3, 3), (4, 0), (5, 0), (9, 0), (10, 0), (11, 0))),
+    (quant.Q4_K, quant.Q6_K, 256, ((0, 0), (5, 0), (9, 0), (10, 0), (11, 0))), (quant.Q8_0, quant.Q8_0, 32, ((0, 0), (1, 0), (5, 0), (6, 0), (10, 0), (11, 0))),
+    (quant.Q4_K, "one", 256, ((0, 0), (1, 0), (3, 1), (4, 0), (5, 0), (9, 0), (11, 0)))], ids=["q4_k", "q4_k-q6_k", "q8_0", "planes"])
+@pytest.mark.parametrize("rows", [2, 40, 600])
+def test_ids_that_no_expert_has(dev, devbuf, t, down, window, forms, rows):
+    """Pairs whose id no expert has add nothing, in every form of the block, with one workgroup of pairs and with several: the
+    grouping leaves them out, so the columns behind the last expert's have no source row and a pair no column.  The last
+    expert is nobody's and holds an infinite scale, which must reach no row."""
+    from test_gpu_moe import _oracle_block, _pack_bank
+    n_expert, k_used, n_ffn, n_embd, period = 5, 3, 512, 256, 8
+    planes = isinstance(down, str)
+    td = t if planes else down
+    rng = np.random.default_rng(11)
+    some = np.stack([rng.permutation(n_expert - 1)[:k_used] for _ in range(period)]).astype(np.uint32)
+    some[0, 1], some[1, 0], some[3, 2], some[4], some[6, 0] = 0xFFFFFFFF, n_expert, 70000, n_expert + 1, 0x80000000
+    wts = (rng.random((period, k_used)) / k_used).astype(np.float32)
+    xs = np.stack([synth.activations(n_embd, seed=900 + r) for r in range(period)])
+    bank = lambda ty, nr, k, s: np.concatenate([synth.random_weights(ty, nr, k, seed=s + e) for e in range(n_expert)])
+    banks = [bank(t, n_ffn, n_embd, 0), bank(t, n_ffn, n_embd, 100), bank(td, n_embd, n_ffn, 200)]
+    want = _oracle_block(t, *banks, xs, some, wts, n_expert, n_ffn, n_embd, window, td=td)
+    last = banks[2][(n_expert - 1) * (len(banks[2]) // n_expert):].reshape(-1, quant.BLOCK[td][1])
+    d = {quant.Q4_K: 0, quant.Q6_K: 208, quant.Q8_0: 0}[td]
+    last[:, d], last[:, d + 1] = 0x00, 0x7C
+    at = np.arange(rows) % period
+    dev.SetActWindow(window)
+    hold = [_pack_bank(dev, devbuf, t, b, n_expert, r, k, "one") for b, (r, k) in zip(banks, [(n_ffn, n_embd)] * 2 + [(n_embd, n_ffn)])] if planes else \
+        [devbuf(b) for b in banks]
+    xd, sd, wd = devbuf(xs[at]), devbuf(some[at]), devbuf(wts[at])
+    try:
+        for form, g16 in forms:
+            if form in (10, 11) and rows > 40:
+                continue
+            dev.set_tuning(moe__form=form, moe__group16=g16)
+            resid = devbuf(np.concatenate([np.zeros(rows * n_embd, np.float32), np.full(8, FILL)]))
+            args = (xd.ptr, sd.ptr, k_used, wd.ptr, rows, k_used, n_expert, n_ffn, n_embd)
+            assert dev.moe_ffn_packed_dev(resid.ptr, t, *[b[0] for b in hold], *args) if planes else \
+                dev.moe_ffn_dev(resid.ptr, t, *[b.ptr for b in hold], *args, down_type=down)
+            dev.synchronize()
+            got = resid.get()
+            assert np.all(got[rows * n_embd:] == FILL)
+            # (an exponential of another machine in front of the second quantizer, as for the other tests of a block)
+            assert nmse(got[:rows * n_embd].reshape(rows, n_embd), want[at]) <= 1e-6, (form, g16)
+    finally:
+        dev.set_tuning(moe__form=0, moe__group16=0)
+        dev.SetActWindow(32)
