@@ -112,6 +112,37 @@ template <> struct GemmI8Raw<JL_Q8_0> { u32x4 q[2]; u32 d; };
 template <> struct GemmI8Raw<JL_Q4_K> { u32x4 q[2], h; };
 template <> struct GemmI8Raw<JL_Q6_K> { u32x4 q[2], h[2]; u32 d; };   // d: the super-block's | the run's two scales << 16
 
+// One sum out[t][r] of a window-32 tile, block by block as integers turned to f32, row: the weight row's first block.
+template <int TYPE>
+__device__ __forceinline__ float gemm_i8_one(const GemmArgs& p, const uint8_t* row, int t) {
+    const u32x4* a = (const u32x4*)p.bq + ((size_t)(t >> 5) * 4) * 64 + (t & 31);
+    float o = 0.f;
+#pragma unroll 1
+    for (int b = 0; b < p.k / 32; b++) {
+        const u32x4* f = a + ((size_t)(b >> 2) * (p.tok_pad >> 5) * 4 + (b & 3)) * 64;
+        const uint8_t* blk = TYPE == JL_Q4_K ? row + (size_t)(b >> 3) * 144 : row + (size_t)b * 34;
+        const uint8_t* q = TYPE == JL_Q4_K ? blk + 16 + 32 * ((b & 7) >> 1) : blk + 2;
+        i32 P = 0;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const u32x4 w = ld16_a2(q + 16 * h), v = f[32 * h];
+#pragma unroll
+            for (int c = 0; c < 4; c++) P = dot4(TYPE == JL_Q4_K ? (w[c] >> (4 * (b & 1))) & 0x0F0F0F0Fu : w[c], v[c], P);
+        }
+        const size_t at = (size_t)b * p.tok_pad + t;
+        if constexpr (TYPE == JL_Q4_K) {
+            const u32x4 h = ld16_a2(blk);
+            u32 sc, mn;
+            scale_min_k4(b & 7, h.y, h.z, h.w, sc, mn);
+            o = fmaf((float)P * p.da[at], half_bits_to_f32((uint16_t)(h.x & 0xFFFF)) * (float)sc, o);
+            o = fmaf(p.dsum[at], -(half_bits_to_f32((uint16_t)(h.x >> 16)) * (float)mn), o);
+        } else {
+            o = fmaf((float)P * p.da[at], half_bits_to_f32(ld2(blk)), o);
+        }
+    }
+    return o;
+}
+
 // t0, r0: the tile's first token and row.
 template <int TYPE, bool W256, int RT, int TW>
 __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, int t0, int r0) {
@@ -119,6 +150,10 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
     constexpr int NPL = Q6 ? 2 : 1, NW = TW > 4 ? TW : 4, ROWS = 32 * RT * (NW / TW), NB = ROWS / (16 * NW);
     constexpr int BUF = JL_GEMM_I8_BUF_BYTES(NPL, ROWS, TW, !W256, Q4), O_D = NPL * ROWS * 128, O_DA = O_D + ROWS * 16,
                   O_M = O_DA + 4 * 32 * TW * 4, O_DS = O_M + ROWS * 16;
+    // One operand, window 32: the sums start at the bits of M = 1.5 * 2^23, so that what comes out of the matrix core IS the float
+    // M + P (|P| <= 32 * 127 * 128 < 2^22), and P * d = fma(M + P, d, -M d) with -M d exact (d has 17 bits at most): no
+    // conversion.  (A row with a scale that is infinite comes out as NaN so: it is summed again where it is stored.)
+    constexpr bool MAGIC = !W256 && NPL == 1 && !(Q4 && TW == 2);   // (that tile has no sixteen registers to spare)
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), tg = wave % TW, rg = wave / TW;
     const bool live = t0 + 32 * tg < p.ntok;                   // else no token of its 32 exists
@@ -320,10 +355,6 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
             stage(GemmIntC<1>{}, step + 1);
         }
     } else {
-        // One operand: the sums start at the bits of M = 1.5 * 2^23, so that what comes out of the matrix core IS the float M + P
-        // (|P| <= 32 * 127 * 128 < 2^22), and P * d = fma(M + P, d, -M d) with -M d exact (d has 17 bits at most): no conversion.  (A
-        // scale that is infinite makes its row NaN, where the product had made it infinite or NaN.)
-        constexpr bool MAGIC = NPL == 1 && !(Q4 && TW == 2);   // (that tile has no sixteen registers to spare)
         i32x16 first = {0};
         if constexpr (MAGIC) {
 #pragma unroll
@@ -436,6 +467,20 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
         for (int e = 0; e < 16; e++) {
             const int t = t0 + 32 * tg + 8 * (e >> 2) + 4 * kg + (e & 3);
             if (t < p.ntok) p.out[(size_t)t * p.out_stride + r] = out[j][e];
+        }
+    }
+    // MAGIC: an infinite scale makes a row's every sum NaN, whatever the token.  The decode matvec and the few-token kernel give
+    // the product's infinities there, and NaN where it has none.
+    if constexpr (MAGIC) {
+#pragma unroll
+        for (int j = 0; j < RT; j++) {
+            const int r = r0 + row0 + 32 * j + arow;
+            if (r >= p.nrows || !__builtin_isnan(out[j][0])) continue;
+#pragma unroll 1
+            for (int e = 0; e < 16; e++) {
+                const int t = t0 + 32 * tg + 8 * (e >> 2) + 4 * kg + (e & 3);
+                if (t < p.ntok) p.out[(size_t)t * p.out_stride + r] = gemm_i8_one<TYPE>(p, p.w + (size_t)r * p.row_bytes, t);
+            }
         }
     }
 }

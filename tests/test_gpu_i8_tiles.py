@@ -98,3 +98,53 @@ def test_tiles_of_256_tokens(dev, devbuf, nrows, k, ntok):
             assert nmse(got[:ntok * nrows].reshape(ntok, nrows), want) <= 1e-10, split
     finally:
         dev.set_tuning(gemm__i8=0, gemm__split=0)
+
+
+@pytest.mark.parametrize("t", [quant.Q8_0, quant.Q4_K], ids=["q8_0", "q4_k"])
+@pytest.mark.parametrize("ntok", [1, 3, 40, 300])
+def test_scales_that_are_no_numbers(dev, devbuf, t, ntok):
+    """A block whose scale is infinite makes its row infinite with the scale's sign, two of opposite sign or a NaN make it NaN, in every kernel (matvec, few tokens, tiles, K slices, tiles per expert); the other rows as ever."""
+    nrows, k, window = 131, 768, 32
+    dev.SetActWindow(window)
+    w = synth.random_weights(t, nrows, k, seed=3)
+    # (weights, scales and activations above zero: a block's products have one sign)
+    x = np.abs(np.stack([synth.activations(k, seed=900 + i) for i in range(ntok)])) + np.float32(0.1)
+    b = w.reshape(nrows, -1, quant.BLOCK[t][1])
+    if t == quant.Q4_K:
+        b[:, :, 4:16] |= 1      # every sub-block's scale at least one
+        b[:, :, 8:12] &= 0x3F   # (minimums: six bits)
+    else:
+        b[:, :, 2:] = b[:, :, 2:] & 0x7F | 1
+    inf, ninf, nan = (0x00, 0x7C), (0x00, 0xFC), (0x00, 0x7E)
+    b[5, 0, :2], b[64, 1, :2], b[127, 2, :2], b[130, 1, :2] = inf, ninf, nan, inf
+    b[100, 0, :2], b[100, 2, :2] = inf, ninf
+    want = oracle.matmul_q8act_f64(t, w, x, nrows, k, ntok, window)
+    want[:, [5, 64, 100, 127, 130]] = np.inf, -np.inf, np.nan, np.nan, np.inf   # (the oracle forms Q8_0 with a bias: NaN there)
+    wd, xd = devbuf(w), devbuf(x)
+    start = devbuf(np.array([0, 0, ntok], np.uint32))
+    bank = devbuf(np.concatenate([w, w]))
+
+    def check(o, what):
+        dev.synchronize()
+        got = o.get()[:ntok * nrows].reshape(ntok, nrows)
+        assert np.array_equal(np.isnan(got), np.isnan(want)), what
+        assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want)), what
+        ok = np.isfinite(want)
+        assert nmse(got[ok], want[ok]) <= 1e-10, what
+    try:
+        with np.errstate(invalid="ignore"):
+            for few, shape, split in ((0, 0, 0), (1, 0, 0), (2, 0, 0), (2, 0, 2), (2, 1, 0), (2, 2, 3), (2, 3, 0)):
+                if shape in (1, 3) and t != quant.Q8_0:
+                    continue
+                dev.set_tuning(gemm__few=few, gemm__i8=shape, gemm__split=split)
+                o = devbuf(shape=(ntok * nrows + 8,), dtype=np.float32, fill=FILL)
+                assert dev.matmul_dev(o.ptr, t, wd.ptr, xd.ptr, nrows, k, ntok)
+                check(o, (few, shape, split))
+            for form in (0, 5, 6, 7, 8) if t == quant.Q8_0 else (0, 5, 6, 7):
+                dev.set_tuning(gemm__few=0, gemm__i8=0, gemm__split=0, moe__form=form)
+                o = devbuf(shape=(ntok * nrows + 8,), dtype=np.float32, fill=FILL)
+                assert dev.moe_matvec_dev(o.ptr, None, t, bank.ptr, None, xd.ptr, None, None, start.ptr, 2, ntok, nrows, k)
+                check(o, form)
+    finally:
+        dev.set_tuning(gemm__few=0, gemm__i8=0, gemm__split=0, moe__form=0)
+        dev.SetActWindow(32)
