@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+template <int V> struct GemmIntC { static constexpr int value = V; };
+
 typedef uint32_t u32;
 typedef int32_t i32;
 typedef u32 u32x2 __attribute__((ext_vector_type(2)));

@@ -36,7 +36,7 @@
 //     4 (q - 32) as an int8 (six bits at the top of the byte, sign bit flipped), the 1/4 goes into d.
 //   * Q4_K: the minimums meet d_a * (sum of the block's a).
 //   * With the k-quant window (W256) one d_a covers a super-block: Q6_K and Q4_K sum integers (sc * dot,
-//     m * sum of a) in v_mad_i32_i24 over the whole chunk and turn to f32 once.
+//     m * sum of a) in v_mad_i32_i24 over the super-block and turn to f32 once.
 //
 // start / slots: column group g of expert e is slot start[e]/16 + e + g, as in the mixture's other
 // kernels; a plain matrix is one expert whose columns are the tokens (start null).
@@ -230,13 +230,16 @@ template <int TYPE, bool W256> struct FewA {
     }
 };
 
-// Four blocks of RT row tiles against NT slots.  m0: all ones in the lane groups of a block's first run (Q6_K).
-template <int TYPE, bool PL, int NT, int RT, bool W256>
+// Four blocks of RT row tiles against NT slots: half H of a super-block.  m0: all ones in the lane groups of a block's first
+// run (Q6_K).  P, M (W256): the super-block's integer sums, scaled once, behind its second half, the larger product d P unrounded.
+// (Scaled after each half, d P rounded first, and the wavefronts' sums added one after the other: NMSE against 64 bits at K = 4096
+// 8.8e-15 for Q4_K, so 6.5e-15, the tiles 7.5e-15; Q6_K 5.3e-15, so 3.9e-15, the tiles 4.8e-15.  And half as many scalings: Q4_K
+// 14336 x 4096, 48 tokens 24.4 -> 21.5 us, Q6_K 4096 x 4096, 96 tokens 17.6 -> 16.4.)
+template <int TYPE, bool PL, int NT, int RT, bool W256, int H>
 __device__ __forceinline__ void few_blocks(const FewR<TYPE, PL>* R, const float* sc, const FewA<TYPE, W256>* X, u32 m0, int g,
-                                           f32x4 (*acc)[NT]) {
+                                           i32x4 (*P)[NT], i32x4 (*M)[NT], f32x4 (*acc)[NT]) {
     const i32x4 zero = {0, 0, 0, 0};
-    i32x4 P[RT][NT], M[RT][NT];
-    if constexpr (W256)
+    if constexpr (W256 && H == 0)
 #pragma unroll
         for (int rt = 0; rt < RT; rt++)
 #pragma unroll
@@ -300,7 +303,7 @@ __device__ __forceinline__ void few_blocks(const FewR<TYPE, PL>* R, const float*
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (W256)
+    if constexpr (W256 && H == 1)
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             const float* scr = sc + rt * (JL_FEW_SC_BYTES / 4);
@@ -311,8 +314,9 @@ __device__ __forceinline__ void few_blocks(const FewR<TYPE, PL>* R, const float*
             for (int t = 0; t < NT; t++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    float v = d4[i] * (float)P[rt][t][i];
-                    if constexpr (TYPE == JL_Q4_K) v = fmaf(-n4[i], (float)M[rt][t][i], v);
+                    float v;
+                    if constexpr (TYPE == JL_Q4_K) v = fmaf(d4[i], (float)P[rt][t][i], -(n4[i] * (float)M[rt][t][i]));
+                    else v = d4[i] * (float)P[rt][t][i];
                     acc[rt][t][i] = fmaf(v, X[t].d1, acc[rt][t][i]);
                 }
         }
@@ -623,6 +627,7 @@ __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem
 
     for (u32 t0 = t_lo; t0 < ntile; t0 += NT) {
         f32x4 acc[RT][NT];
+        i32x4 P[RT][NT], M[RT][NT];
 #pragma unroll
         for (int rt = 0; rt < RT; rt++)
 #pragma unroll
@@ -646,11 +651,12 @@ __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem
             FewA<TYPE, W256> X0[NT], X1[NT];
             auto pin = [&]() { few_pin(va); few_pin(vd); few_pin(pa.vg); few_pin(pa.vh); few_pin(pa.vr); };
             auto load_w = [&](int c, FewPlaneW<TYPE>* W) { few_planes_load<TYPE, RT>(p, m, c, pa, g, W); };
-            auto compute = [&](int c, const FewPlaneW<TYPE>* W, const FewA<TYPE, W256>* X) {
+            auto compute = [&](auto H, int sb, const FewPlaneW<TYPE>* W, const FewA<TYPE, W256>* X) {
+                constexpr int h = decltype(H)::value;
                 FewR<TYPE, true> R[RT];
-                few_planes_half<TYPE, RT, W256>(c, W, sc, g, r16, R);
+                few_planes_half<TYPE, RT, W256>(2 * sb + h, W, sc, g, r16, R);
                 few_lds_fence();
-                few_blocks<TYPE, true, NT, RT, W256>(R, sc, X, m0, g, acc);
+                few_blocks<TYPE, true, NT, RT, W256, h>(R, sc, X, m0, g, P, M, acc);
                 few_lds_fence();
             };
             // (super-blocks w, w + nwaves, ... of wavefront w, the halves in turn: the order of the rows' form,
@@ -664,18 +670,18 @@ __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem
                     pin();
                     if (AHEAD) load_a(2 * sb + 1, X1); else load_a(2 * sb, X0);
                     load_w(2 * sb + 1, W1);
-                    compute(2 * sb, W0, X0);
+                    compute(GemmIntC<0>{}, sb, W0, X0);
                     pin();
                     if (AHEAD) load_a(2 * (sb + nw), X0); else load_a(2 * sb + 1, X0);
                     load_w(2 * (sb + nw), W0);
-                    compute(2 * sb + 1, W1, AHEAD ? X1 : X0);
+                    compute(GemmIntC<1>{}, sb, W1, AHEAD ? X1 : X0);
                 }
                 pin();
                 if (AHEAD) load_a(2 * sb + 1, X1); else load_a(2 * sb, X0);
                 load_w(2 * sb + 1, W1);
-                compute(2 * sb, W0, X0);
+                compute(GemmIntC<0>{}, sb, W0, X0);
                 if (!AHEAD) load_a(2 * sb + 1, X0);
-                compute(2 * sb + 1, W1, AHEAD ? X1 : X0);
+                compute(GemmIntC<1>{}, sb, W1, AHEAD ? X1 : X0);
             }
         } else {
             // A super-block's registers are free once it is staged, so one set is enough: stage, ask for the
@@ -694,11 +700,12 @@ __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem
 #pragma unroll
                 for (int rt = 0; rt < RT; rt++) { few_pin(ra.tail[rt]); few_pin(ra.mine[rt]); }
             };
-            auto half = [&](int sb, int h, const FewA<TYPE, W256>* X) {
+            auto half = [&](int sb, auto H, const FewA<TYPE, W256>* X) {
+                constexpr int h = decltype(H)::value;
                 FewR<TYPE, false> R[RT];
                 few_rows_half<TYPE, RT, W256>(p, sb, h, ra, st, sc, g, r16, R);
                 few_lds_fence();
-                few_blocks<TYPE, false, NT, RT, W256>(R, sc, X, m0, g, acc);
+                few_blocks<TYPE, false, NT, RT, W256, h>(R, sc, X, m0, g, P, M, acc);
                 few_lds_fence();
             };
             auto unit = [&](int sb, int next) {   // next < 0: the last
@@ -709,13 +716,13 @@ __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem
                 if constexpr (NT == 1) {
                     load_a(2 * sb + 1, X1);
                     if (next >= 0) few_rows_load<TYPE, RT>(p, m.w, next, ra, W);
-                    half(sb, 0, X0);
-                    half(sb, 1, X1);
+                    half(sb, GemmIntC<0>{}, X0);
+                    half(sb, GemmIntC<1>{}, X1);
                 } else {
-                    half(sb, 0, X0);
+                    half(sb, GemmIntC<0>{}, X0);
                     load_a(2 * sb + 1, X0);
                     if (next >= 0) few_rows_load<TYPE, RT>(p, m.w, next, ra, W);
-                    half(sb, 1, X0);
+                    half(sb, GemmIntC<1>{}, X0);
                 }
             };
             const int nsb = p.nch / 2;
@@ -752,8 +759,13 @@ __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem
         const u32 left = ncol - t0 * 16;
         for (int i = threadIdx.x; i < 16 * NT * 16 * RT; i += nw * 64) {
             const int tok = i / (16 * RT), rr = i % (16 * RT);
+            // (by pairs: one after the other the eight additions round four and a half times a result's size, so three)
+            const float* at = red + tok * RS + rr;
+            constexpr int W = 16 * NT * RS;
             float v = 0.f;
-            for (int q = 0; q < nw; q++) v += red[(q * 16 * NT + tok) * RS + rr];
+            int q = 0;
+            for (; q + 4 <= nw; q += 4, at += 4 * W) v += (at[0] + at[W]) + (at[2 * W] + at[3 * W]);
+            for (; q < nw; q++, at += W) v += at[0];
             if ((u32)tok < left && r0 + rr < p.nrows) {
                 const size_t o = (size_t)(col0 + t0 * 16 + tok) * p.nrows + r0 + rr;
                 if (p.out[0]) p.out[0][o] = v;

@@ -160,7 +160,6 @@ __device__ __forceinline__ void gemm_prep_q4k_body(const GemmPrepArgs& p, u32* l
 }
 
 // -------------------------------------------------------------------- main
-template <int V> struct GemmIntC { static constexpr int value = V; };
 
 // f(GemmIntC<I>{}) for I = 0..N-1 with I a compile-time constant inside f: register arrays
 // indexed by it stay in registers.

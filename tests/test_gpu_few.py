@@ -155,3 +155,31 @@ def test_a_few_tokens_as_matvecs_in_one_launch(dev, devbuf, t, ntok, nrows, k):
             assert nmse(got[:ntok * n].reshape(ntok, n), want[:, r0:r0 + n]) <= 1e-10, (packed, r0)
     finally:
         dev.set_tuning(gemm__few=0)
+
+
+# A rounding of a sum whose mantissa is spread evenly over its logarithm: 2^-46 / 12 of [1, 2)'s mean square 1.5 / ln 2.
+ROUNDING = 2.0 ** -46 / 12 / (1.5 / np.log(2))
+
+
+@pytest.mark.parametrize("t", [quant.Q4_K, quant.Q6_K], ids=["q4_k", "q6_k"])
+def test_few_tokens_round_once_a_super_block(dev, devbuf, t):
+    """The k-quant window, 56 super-blocks over eight wavefronts: no more roundings than one scaling a super-block, a chain of
+    seven and a tree of eight make, counted in a result's size -- d P (Q4_K: d P - dmin M, whose second product is 2.7 of it
+    for weights spread as N(0, s)), four for the chain's sums that grow to an eighth, one a level.  Half as many again for what
+    the count leaves out; scaled by halves and added one after the other it was 13 (Q6_K) and 19."""
+    nrows, k, ntok = 256, 14336, 70
+    units = 1 + 4 + 3 + (2.7 if t == quant.Q4_K else 0)
+    w = synth.quantized_weights(t, nrows, k, seed=5)
+    x = np.stack([synth.activations(k, seed=300 + i) for i in range(ntok)])
+    wd, xd = devbuf(w), devbuf(x)
+    dev.SetActWindow(256)
+    try:
+        want = oracle.matmul_q8act_f64(t, w, x, nrows, k, ntok, 256)
+        dev.set_tuning(gemm__few=1, few__waves=8)
+        out = devbuf(shape=(ntok, nrows), dtype=np.float32)
+        assert dev.matmul_dev(out.ptr, t, wd.ptr, xd.ptr, nrows, k, ntok)
+        dev.synchronize()
+        assert nmse(out.get(), want) <= 1.5 * units * ROUNDING
+    finally:
+        dev.set_tuning(gemm__few=0, few__waves=0)
+        dev.SetActWindow(32)
