@@ -467,12 +467,17 @@ int matvec_launch(jl_ctx* c, float* out, int type, const void* w, const float* x
     return launch(c, name, (unsigned)grid, 1, (unsigned)block, lds, st, params);
 }
 
+// The forms for several tokens or routed pairs: Q6_K has one for the k-quant window.
+const char* q6_tag(const jl_ctx* c, int type) { return type == JL_TYPE_Q6_K && c->act_window == 256 ? "q6kw" : type_info(type)->tag; }
+
 // m matrices of one type in one launch (kernels/matvec.h, matvec_multi_body).
+// tokens: one plain matrix for m activations (tokens_matvec_launch).
 // types: null when every matrix is of `type`; else the type of each (the mixed-type kernel).
 int matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, const void* const* ws, const int* rows,
                         const float* x, size_t xstride, const float* x2, float* resid, float alpha, int k,
                         hipStream_t st, const float* norm_w = nullptr, float norm_eps = 0.f,
-                        float* norm_out = nullptr, const int* types = nullptr, const float* resid_gate = nullptr) {
+                        float* norm_out = nullptr, const int* types = nullptr, const float* resid_gate = nullptr,
+                        bool tokens = false) {
     if (m < 1 || m > JL_MAX_MULTI) return fail(c, JL_ERR_ARG, "matvec multi: %d matrices", m);
     const TypeInfo* ti = nullptr;
     const TypeInfo* tis[JL_MAX_MULTI];
@@ -580,7 +585,7 @@ int matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, const vo
         return launch(c, name, (unsigned)gx, (unsigned)m, nwaves * 64, lds, st, params);
     }
     if (types) name << "jl_matvec_segments";
-    else name << "jl_matvec_multi_" << (pair ? "q8_0p" : ti->tag);
+    else name << "jl_matvec_multi_" << (pair ? "q8_0p" : tokens && type == JL_TYPE_Q4_K ? "q4kf" : tokens ? q6_tag(c, type) : ti->tag);
     name << (norm_w ? x2 ? "_na" : "_n" : x2 ? "_a" : "") << (types || xpre == 1 ? "" : xpre == 4 ? "_x4" : "_x2") << (resid ? "_res" : "");
     if (lanes != 64) name << "_l" << lanes;
     void* params[] = {&a};
@@ -1160,7 +1165,7 @@ int few_launch(jl_ctx* c, const FewCall& f, hipStream_t st) {
 
 int packed_matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, const PlaneRef* pls, const float* x, size_t xstride, const float* up,
                                float* resid, float alpha, const float* resid_gate, const float* norm_w, float norm_eps, float* norm_out, int nrows,
-                               int k, hipStream_t st);
+                               int k, hipStream_t st, bool tokens = false);
 // A few tokens as that many decode matvecs in one launch (each reads the weights, the later ones from L2).
 int tokens_matvec_launch(jl_ctx* c, float* out, int type, const void* w, const PlaneRef* pl, const float* x, int nrows, int k, int ntok, hipStream_t st) {
     float* outs[JL_MAX_MULTI];
@@ -1171,8 +1176,8 @@ int tokens_matvec_launch(jl_ctx* c, float* out, int type, const void* w, const P
         outs[t] = out + (size_t)t * nrows; ws[t] = w; rows[t] = nrows;
         if (pl) pls[t] = *pl;
     }
-    return pl ? packed_matvec_multi_launch(c, type, ntok, outs, pls, x, k, nullptr, nullptr, 0.f, nullptr, nullptr, 0.f, nullptr, nrows, k, st)
-              : matvec_multi_launch(c, type, ntok, outs, ws, rows, x, k, nullptr, nullptr, 0.f, k, st);
+    return pl ? packed_matvec_multi_launch(c, type, ntok, outs, pls, x, k, nullptr, nullptr, 0.f, nullptr, nullptr, 0.f, nullptr, nrows, k, st, true)
+              : matvec_multi_launch(c, type, ntok, outs, ws, rows, x, k, nullptr, nullptr, 0.f, k, st, nullptr, 0.f, nullptr, nullptr, nullptr, true);
 }
 // Where: the few-token form is two launches, this is one.  Over rows a workgroup's sixteen wavefronts make `passes` steps of their
 // lanes a row, each a chain of trips (Q8_0, two workgroups a CU: at least its bytes); over planes a wavefront goes through its share
@@ -1186,6 +1191,9 @@ bool tokens_matvec_wanted(const jl_ctx* c, int type, bool planes, int nrows, int
     if (c->tune.gemm_few == 3) return true;
     if (ntok > 8 || c->tune.gemm_few || c->tune.gemm_form || c->gemm_min_tok != 3) return false;
     if (ntok == 2 && type != JL_TYPE_Q8_0) return true;
+    // (Q6_K over planes, and short rows under a shorter window: the matvec's sums round more than the few-token kernel's, NMSE
+    // against 64 bits 8.3e-15 and 4.8e-15 for eight tokens at K = 2048 over planes, 4.6e-15 and 4.3e-15 for three at K = 512)
+    if (type == JL_TYPE_Q6_K && (planes || (c->act_window != 256 && k < 1024))) return false;
     if (!few_fits(c, type, planes, nrows, k, ntok, stride)) return false;
     const TypeInfo* ti = type_info(type);
     const bool q8 = type == JL_TYPE_Q8_0;
@@ -1366,7 +1374,7 @@ int packed_matvec_launch(jl_ctx* c, float* out, int type, const PlaneRef& pl, co
 int packed_matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, const PlaneRef* pls,
                                const float* x, size_t xstride, const float* up, float* resid, float alpha,
                                const float* resid_gate, const float* norm_w, float norm_eps, float* norm_out,
-                               int nrows, int k, hipStream_t st) {
+                               int nrows, int k, hipStream_t st, bool tokens) {
     if (m < 1 || m > JL_MAX_MULTI) return fail(c, JL_ERR_ARG, "packed multi: %d matrices", m);
     // the norm precedes gate and up, the gated activation precedes down: never both
     if (norm_w && (up || !aligned16(norm_w) || (norm_out && !aligned16(norm_out)))) return JL_DECLINED;
@@ -1404,7 +1412,7 @@ int packed_matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, c
     a.nrows = nrows; a.k = k; a.stride = pls[0].stride; a.per = c->act_window / 32;
     a.nwaves = nw; a.ngroups = (nrows + rw - 1) / rw;
     Name name;
-    name << "jl_matvec_packed_multi_" << (up ? "act_" : norm_w ? "norm_" : "") << ti->tag << "_w" << rw;
+    name << "jl_matvec_packed_multi_" << (up ? "act_" : norm_w ? "norm_" : "") << (tokens && type == JL_TYPE_Q4_K ? "q4kf" : ti->tag) << "_w" << rw;
     void* params[] = {&a};
     return launch(c, name, (unsigned)a.ngroups, (unsigned)m, (unsigned)(nw * 64),
                   (unsigned)(nw * (384 + 65 * 4) + (norm_w ? 16 + 160 : 0)), st, params);   // JL_PK_LDS_BYTES + JL_NORM_LDS_BYTES
@@ -1628,7 +1636,7 @@ int moe_gather_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     a.ngroups = (int)std::max(1L, std::min(groups, slots / ((long)ncols * nmat)));
     if (!start && !sel && a.ngroups > 8) a.ngroups &= ~7;   // (one matrix: a row group's workgroups on one XCD)
     Name name;
-    name << "jl_moe_gather_" << (pair ? "q8_0p" : ti->tag) << (x2 ? "_a" : "") << "_l" << lpr;
+    name << "jl_moe_gather_" << (pair ? "q8_0p" : q6_tag(c, type)) << (x2 ? "_a" : "") << "_l" << lpr;
     void* params[] = {&a};
     return launch(c, name, (unsigned)a.ngroups, (unsigned)ncols, 1024, (unsigned)lds, st, params, (unsigned)nmat);
 }
@@ -1683,7 +1691,7 @@ int moe_gather_ffn(jl_ctx* c, float* resid, int type, int down_type, const void*
     a.ngroups = (int)std::max(1L, std::min(groups, slots / rows));
     if (!sel && a.ngroups > 8) a.ngroups &= ~7;
     Name name;
-    name << "jl_moe_gather_" << (pair ? "q8_0p" : ti->tag) << "_down_l" << lpr;
+    name << "jl_moe_gather_" << (pair ? "q8_0p" : q6_tag(c, down_type)) << "_down_l" << lpr;
     void* params[] = {&a};
     return launch(c, name, (unsigned)a.ngroups, (unsigned)rows, 1024, (unsigned)lds, st, params);
 }
@@ -2154,11 +2162,14 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     names.push_back("jl_few_prep");
     names.push_back("jl_gemm_i8_prep");
     names.push_back("jl_moe_gemm_i8_prep");
-    for (const char* tag : {"q4k", "q8_0", "q8_0p", "q6k"})
+    for (const char* tag : {"q4k", "q8_0", "q8_0p", "q6k", "q6kw"})
         for (const char* act : {"", "_a", "_down"})
             for (const char* lpr : {"_l8", "_l16", "_l32", "_l64"}) names.push_back(std::string("jl_moe_gather_") + tag + act + lpr);
     for (const char* rw : {"16", "32", "64"})
         for (const char* form : {"jl_moe_planes_gather_w", "jl_moe_planes_down_w"}) names.push_back(std::string(form) + rw);
+    for (const char* tag : {"q4kf", "q6kw"})
+        for (const char* form : {"", "_x2", "_x4", "_l32", "_l16"}) names.push_back(std::string("jl_matvec_multi_") + tag + form);
+    for (const char* rw : {"16", "32", "64"}) names.push_back(std::string("jl_matvec_packed_multi_q4kf_w") + rw);
     for (const char* tag : {"q4k", "q4k_planes", "q6k"})
         for (const char* form : {"jl_moe_cols_", "jl_moe_cols_prep_"}) names.push_back(std::string(form) + tag);
     for (const char* tag : {"q8_0", "q4k", "q6k", "q6kw"})

@@ -118,6 +118,8 @@ JL_MATVEC_KERNEL(q8_0p, JL_Q8_0P, 1, 1024) JL_MATVEC_KERNEL(q8_0p, JL_Q8_0P, 2, 
 #define JL_MATVEC_MULTI_KERNEL(T, TYPE) JL_MATVEC_MULTI_FORMS(T, TYPE, , false) JL_MATVEC_MULTI_FORMS(T, TYPE, _res, true)
 JL_MATVEC_MULTI_KERNEL(q4k, JL_Q4_K) JL_MATVEC_MULTI_KERNEL(q8_0, JL_Q8_0) JL_MATVEC_MULTI_KERNEL(q6k, JL_Q6_KS)
 JL_MATVEC_MULTI_KERNEL(q8_0p, JL_Q8_0P)
+// One matrix for several tokens
+JL_MATVEC_MULTI_PRE(q4kf, JL_Q4_KF, , 0, , false) JL_MATVEC_MULTI_PRE(q6kw, JL_Q6_KW, , 0, , false)
 // The same grid over matrices of different types (the reference's MatVecSegments,
 // jit/gpu/kernels/matvec.go:1411-1431: a block's q, k and v in one launch whatever their
 // formats).
@@ -150,6 +152,12 @@ JL_MATVEC_SEGMENTS(_a, JL_PRE_ACT, _res, true) JL_MATVEC_SEGMENTS(_na, JL_PRE_NO
         matvec_segments_body<false, JL_PRE_NORM, L>(p, jl_smem);                                                   \
     }
 JL_MATVEC_LANES_TYPES(32) JL_MATVEC_LANES_TYPES(16)
+#define JL_MATVEC_TOKENS_LANES(T, TYPE, L)                                                                         \
+    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_multi_##T##_l##L(MatVecMultiArgs p) {             \
+        matvec_multi_body<TYPE, 1, false, 0, L>(p, jl_smem);                                                       \
+    }
+JL_MATVEC_TOKENS_LANES(q4kf, JL_Q4_KF, 32) JL_MATVEC_TOKENS_LANES(q4kf, JL_Q4_KF, 16)
+JL_MATVEC_TOKENS_LANES(q6kw, JL_Q6_KW, 32) JL_MATVEC_TOKENS_LANES(q6kw, JL_Q6_KW, 16)
 
 // -------------------------------------------------- few tokens, int8 matrix cores
 extern "C" __global__ __launch_bounds__(256) void jl_few_prep(FewI8PrepArgs p) { few_i8_prep_body(p); }
@@ -209,6 +217,11 @@ JL_PACKED_KERNEL(q6k, JL_Q6_K, 64, 4) JL_PACKED_KERNEL(q6k, JL_Q6_K, 32, 4) JL_P
 JL_PACKED_MULTI_KERNEL(q4k, JL_Q4_K, 64, 4) JL_PACKED_MULTI_KERNEL(q4k, JL_Q4_K, 32, 4) JL_PACKED_MULTI_KERNEL(q4k, JL_Q4_K, 16, 4)
 JL_PACKED_MULTI_KERNEL(q8_0, JL_Q8_0, 64, 2) JL_PACKED_MULTI_KERNEL(q8_0, JL_Q8_0, 32, 4) JL_PACKED_MULTI_KERNEL(q8_0, JL_Q8_0, 16, 4)
 JL_PACKED_MULTI_KERNEL(q6k, JL_Q6_K, 64, 4) JL_PACKED_MULTI_KERNEL(q6k, JL_Q6_K, 32, 4) JL_PACKED_MULTI_KERNEL(q6k, JL_Q6_K, 16, 4)
+#define JL_PACKED_TOKENS_KERNEL(RW)                                                                             \
+    extern "C" __global__ __launch_bounds__(1024) void jl_matvec_packed_multi_q4kf_w##RW(PackedMultiArgs p) {   \
+        packed_matvec_multi_body<JL_Q4_KF, RW, 4, false>(p, jl_smem);                                           \
+    }
+JL_PACKED_TOKENS_KERNEL(64) JL_PACKED_TOKENS_KERNEL(32) JL_PACKED_TOKENS_KERNEL(16)   // (one matrix for several tokens)
 
 // ------------------------------------------------------------ prefill GEMM
 // grid = (k/256, tok_pad/4), block = 256: one wavefront per (token, super-block)
@@ -379,7 +392,7 @@ extern "C" __global__ __launch_bounds__(512) void jl_moe_matvec_planes_q4k(MoePl
     extern "C" __global__ __launch_bounds__(1024) void jl_moe_gather_##T##_a_l##L(MoeGatherArgs p) { moe_gather_body<TYPE, JL_PRE_ACT, L>(p, jl_smem); } \
     extern "C" __global__ __launch_bounds__(1024) void jl_moe_gather_##T##_down_l##L(MoeGatherDownArgs p) { moe_gather_down_body<TYPE, L>(p, jl_smem); }
 #define JL_MOE_GATHER(T, TYPE) JL_MOE_GATHER_L(T, TYPE, 8) JL_MOE_GATHER_L(T, TYPE, 16) JL_MOE_GATHER_L(T, TYPE, 32) JL_MOE_GATHER_L(T, TYPE, 64)
-JL_MOE_GATHER(q4k, JL_Q4_K) JL_MOE_GATHER(q8_0, JL_Q8_0) JL_MOE_GATHER(q8_0p, JL_Q8_0P) JL_MOE_GATHER(q6k, JL_Q6_KS)
+JL_MOE_GATHER(q4k, JL_Q4_KF) JL_MOE_GATHER(q8_0, JL_Q8_0) JL_MOE_GATHER(q8_0p, JL_Q8_0P) JL_MOE_GATHER(q6k, JL_Q6_KS) JL_MOE_GATHER(q6kw, JL_Q6_KW)
 // over planes: grid = (ceil(nrows/RW), pairs, 2) and (ceil(nrows/RW), rows), block <= 1024, dynamic LDS = JL_PK_LDS_BYTES
 #define JL_MOE_PLANES_GATHER(RW)                                                                                          \
     extern "C" __global__ __launch_bounds__(1024) void jl_moe_planes_gather_w##RW(MoePlanesGatherArgs p) {                \

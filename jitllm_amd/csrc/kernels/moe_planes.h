@@ -28,7 +28,7 @@ __device__ __forceinline__ void moe_planes_gather_body(const MoePlanesGatherArgs
     p.qs = as_global(p.qs) + (size_t)e * words; p.d = as_global(p.d) + (size_t)e * words; p.sc = as_global(p.sc) + (size_t)e * words;
     p.row0 = (int)e * row_step;
     p.x = as_global(p.x) + (size_t)row * p.k;
-    packed_matvec_body<JL_Q4_K, RW, XPRE, true>(p, smem);
+    packed_matvec_body<JL_Q4_KF, RW, XPRE, true>(p, smem);
 }
 template <int RW, int XPRE>
 __device__ __forceinline__ void moe_planes_down_body(const MoePlanesDownArgs& args, uint8_t* smem) {
@@ -67,7 +67,7 @@ __device__ __forceinline__ void moe_planes_down_body(const MoePlanesDownArgs& ar
         const size_t e = min(id, last);
         p.qs = qs + e * m.sheet_words; p.d = d + e * m.sheet_words; p.sc = sc + e * m.sheet_words;
         const int row = (int)e * m.row_step + rr;
-        PkWQ4K<NB> w;
+        PkWQ4KF<NB> w;
         pk_load<NB>(p, cc, b0, row, w);
         pk_stage_x<true, true>(p, c, lane, Xc, my);
         const float more = fmaf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(i32, wts), pair)), pk_dot<NB>(p, w, cc, b0, row, A), acc);

@@ -318,9 +318,9 @@ __device__ __forceinline__ void pk_load(const PackedMatVecArgs& p, int c, int b0
         for (int j = 0; j < 4; j++) w.q[i][j] = qs[(size_t)(i * 4 + j) * st];
 }
 
-template <int NB>
-__device__ __forceinline__ float pk_dot(const PackedMatVecArgs&, const PkWQ4K<NB>& w, int, int b0, int,
-                                        const PkAct& A) {
+// F: the larger product enters its difference unrounded, as in the rows' form for several tokens (JL_Q4_KF).
+template <bool F, int NB>
+__device__ __forceinline__ float pk_dot_q4k(const PkWQ4K<NB>& w, int b0, const PkAct& A) {
     const u32 M = 0x0F0F0F0Fu;
     const float d = half_bits_to_f32((uint16_t)(w.d & 0xFFFF));
     const float dmin = half_bits_to_f32((uint16_t)(w.d >> 16));
@@ -341,10 +341,22 @@ __device__ __forceinline__ float pk_dot(const PackedMatVecArgs&, const PkWQ4K<NB
         dt = dot4((w.q[i][2] >> 4) & M, a1.z, dt);
         dt = dot4((w.q[i][3] >> 4) & M, a1.w, dt);
         const float sa = A.ss[2 * s] + A.ss[2 * s + 1];
-        const float v = (float)dt * (d * (float)sc) - sa * (dmin * (float)m);
+        const float dsc = d * (float)sc, bias = sa * (dmin * (float)m);
+        const float v = F ? fmaf((float)dt, dsc, -bias) : (float)dt * dsc - bias;
         acc = fmaf(v, A.da[s], acc);
     }
     return acc;
+}
+template <int NB>
+__device__ __forceinline__ float pk_dot(const PackedMatVecArgs&, const PkWQ4K<NB>& w, int, int b0, int,
+                                        const PkAct& A) {
+    return pk_dot_q4k<false>(w, b0, A);
+}
+template <int NB> struct PkWQ4KF : PkWQ4K<NB> {};
+template <int NB>
+__device__ __forceinline__ float pk_dot(const PackedMatVecArgs&, const PkWQ4KF<NB>& w, int, int b0, int,
+                                        const PkAct& A) {
+    return pk_dot_q4k<true>((const PkWQ4K<NB>&)w, b0, A);
 }
 
 template <int NB>
@@ -424,6 +436,7 @@ __device__ __forceinline__ float pk_dot(const PackedMatVecArgs&, const PkWQ6K<NB
 
 template <int TYPE, int NB> struct PkTraits;
 template <int NB> struct PkTraits<JL_Q4_K, NB> { typedef PkWQ4K<NB> W; };
+template <int NB> struct PkTraits<JL_Q4_KF, NB> { typedef PkWQ4KF<NB> W; };
 template <int NB> struct PkTraits<JL_Q8_0, NB> { typedef PkWQ8<NB> W; };
 template <int NB> struct PkTraits<JL_Q6_K, NB> { typedef PkWQ6K<NB> W; };
 

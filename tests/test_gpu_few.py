@@ -183,3 +183,37 @@ def test_few_tokens_round_once_a_super_block(dev, devbuf, t):
     finally:
         dev.set_tuning(gemm__few=0, few__waves=0)
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("t", [quant.Q4_K, quant.Q6_K], ids=["q4_k", "q6_k"])
+def test_tokens_side_by_side_round_no_more_than_the_few_token_kernel(dev, devbuf, t):
+    """The k-quant window, decode matvecs of eight tokens and of routed columns at K = 2048: roundings counted as above -- Q6_K two
+    products a super-block and three levels of a tree of eight; Q4_K d P - dmin M and half of two products a slot and the five
+    levels of 32 slots.  (Every run of Q6_K scaled for itself made 8.5, both products of Q4_K rounded 13.4.)"""
+    nrows, k, ntok = 1500, 2048, 8
+    units = 2 + 3 if t == quant.Q6_K else 2.7 + 1 + 1 + 5
+    w = synth.quantized_weights(t, nrows, k, seed=6)
+    x = np.stack([synth.activations(k, seed=300 + i) for i in range(ntok)])
+    start = np.array([0, ntok], np.uint32)
+    wd, xd, sd = devbuf(w), devbuf(x), devbuf(start)
+    planes = [devbuf(np.zeros(max(n, 4), np.uint32)) for n in quant.packed_words(t, nrows, k)]
+    assert dev.pack_weights_dev(t, wd.ptr, nrows, k, *[p.ptr for p in planes])
+    dev.SetActWindow(256)
+    try:
+        want = oracle.matmul_q8act_f64(t, w, x, nrows, k, ntok, 256)
+        dev.set_tuning(gemm__few=3, moe__form=10)
+        for form in ("rows", "columns") + (("planes",) if t == quant.Q4_K else ()):
+            out = devbuf(shape=(ntok, nrows), dtype=np.float32)
+            before = dev.launch_count()
+            if form == "rows":
+                assert dev.matmul_dev(out.ptr, t, wd.ptr, xd.ptr, nrows, k, ntok)
+            elif form == "planes":
+                assert dev.matmul_packed_dev(out.ptr, t, Packed(*[p.ptr for p in planes], 0, nrows), xd.ptr, nrows, k, ntok)
+            else:
+                assert dev.moe_matvec_dev(out.ptr, None, t, wd.ptr, None, xd.ptr, None, None, sd.ptr, 1, ntok, nrows, k)
+            assert dev.launch_count() == before + 1
+            dev.synchronize()
+            assert nmse(out.get(), want) <= 1.5 * units * ROUNDING, form
+    finally:
+        dev.set_tuning(gemm__few=0, moe__form=0)
+        dev.SetActWindow(32)
