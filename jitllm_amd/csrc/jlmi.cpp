@@ -1641,10 +1641,13 @@ int moe_gather_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     return launch(c, name, (unsigned)a.ngroups, (unsigned)ncols, 1024, (unsigned)lds, st, params, (unsigned)nmat);
 }
 
-// Whether a block's pairs go without grouping (moe_gather_ffn).  That saves two launches and the grouped kernels' setup, 13 us, and
-// reads a sheet again for every pair that shares its expert with another, but at 6.5 TB/s (from L2 and the memory-side cache where
-// it is read again) against the 3.65 that the grouped kernels make of a few columns a sheet; the rows' choices are taken as evenly
-// spread.  The whole block, grouped -> so, us, at pairs: Q4_K 128 experts top-8 of 768 x 2048 with Q6_K down 35 -> 22 (8), 56 -> 30
+// Whether a block's pairs go without grouping (moe_gather_ffn).  That saves two launches and the grouped kernels' setup, and reads a
+// sheet again for every pair that shares its expert with another, but faster (from L2 and the memory-side cache where it is read
+// again) than the grouped kernels, which make 5 TB/s of a few columns a sheet, over planes 7 and a longer setup; the rows' choices
+// are taken as evenly spread.  Fitted to 862 (Q4_K, k-quant window), 450 (planes) and 1724 (the others) blocks, 2 to 128 experts of
+// 768 x 2048 to 14336 x 4096 at 1 to 32 rows: 0.7, 2.4 and 0.6 % behind the better of the two, at most 9, 4 and 11 % slower than
+// grouped.  (One line for all, 6.5 and 3.65 TB/s and 13 us: 16 experts top-4 of 14336 x 4096, six rows 273 -> 349 us, planes of
+// 4096 x 4096 221 -> 267 at 64 experts and sixteen.)  The whole block, grouped -> so, us, at pairs: Q4_K 128 experts top-8 of 768 x 2048 with Q6_K down 35 -> 22 (8), 56 -> 30
 // (32), 97 -> 79 (96), 122 -> 118 (192), 134 -> 163 (320: grouped); 60 top-4 of 1792 x 2816 33 -> 25 (4), 127 -> 98 (60), 142 -> 146
 // (92), 138 -> 162 (120: grouped); 8 top-2 of 2048 x 2816 28 -> 20 (2), 50 -> 36 (16), 49 -> 51 (24: grouped); 32 top-4 of 1024 x
 // 2048 47 -> 31 (32), 49 -> 44 (64), 49 -> 58 (80: grouped).  Q8_0 60 top-4 of 1792 x 2816 36 -> 27 (4), 174 -> 159 (60), 221 -> 250 (92:
@@ -1653,13 +1656,16 @@ int moe_gather_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
 // 2816 39 -> 24 (4), 108 -> 100 (64), 143 -> 171 (128: grouped); 8 top-2 of 1024 x 1536 30 -> 16 (2), 42 -> 29 (32).
 // Q4_K and Q6_K rows of sheets under 512 x 512 keep the grouped form, whose launches a caller can count on there
 // (tests/test_gpu_moe.py), though they would gain as well.
-bool moe_gather_ffn_wanted(int type, int down_type, bool planes, int rows, int k_used, int n_expert, int n_ffn, int n_embd) {
+bool moe_gather_ffn_wanted(const jl_ctx* c, int type, int down_type, bool planes, int rows, int k_used, int n_expert, int n_ffn, int n_embd) {
     const double pairs = (double)rows * k_used, sheet = (double)n_ffn * n_embd;
     if (pairs > 256 || (!planes && type != JL_TYPE_Q8_0 && sheet < 512.0 * 512.0)) return false;
     const TypeInfo *t = type_info(type), *d = type_info(down_type);
     const double mb = sheet * 1e-6 * (2.0 * t->block_bytes / t->block_elems + (double)d->block_bytes / d->block_elems);
     const double touched = n_expert * (1.0 - std::pow(1.0 - std::min(1.0, (double)k_used / n_expert), rows));
-    return pairs * mb / 6.5 < 13.0 + touched * mb / 3.65;
+    struct { double again, grouped, setup; } q = {8, 5.6, 14};
+    if (planes) q = {7.5, 7, 20};
+    else if (type == JL_TYPE_Q4_K && c->act_window == 256) q = {6.5, 5, 18};
+    return pairs * mb / q.again < q.setup + touched * mb / q.grouped;
 }
 
 // A routed block of a handful of pairs without its grouping and combine: the pairs themselves are the columns of gate + up,
@@ -1825,8 +1831,17 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
         // the second 57 -> 34 at 4, 191 -> 177 at 64, 8 x 1024 x 1536 at 24 columns 41 -> 43.  Q4_K and Q6_K sheets under 512 x 512
         // keep the grouped form, whose launches a caller can count on there (tests/test_gpu_moe.py), though they would gain as
         // well: 8 experts of 256 x 512, 12 columns 28.7 against 21.9.
-        const bool gather = type == JL_TYPE_Q8_0 ? ncols <= 16 || (ncols <= 64 && avg <= 1.1)
-                                                 : (long)nrows * k >= 512L * 512 && ncols <= ((double)nrows * k >= 2.4e6 && avg <= 0.6 ? 32 : 16);
+        // It reads a sheet again for every column that shares it, which shows where sheets are large: at 6 TB/s, against the
+        // few-token kernel's 4 for the sheets that have a column (taken as evenly spread) and 5 us of prep.  us, that kernel / so:
+        // Q6_K 4096 x 14336, 2 experts, 6 / 16 columns 32 / 58, 33 / 92, 4 experts 16 columns 56 / 103.  Q4_K with the k-quant window
+        // has a slower one: 14336 x 4096 twice, 4 experts, 8 / 12 columns 92 / 70, 93 / 113; one matrix the same on average.  (512
+        // and 256 launches, 2 to 16 experts of 1024 x 2048 to 14336 x 4096, 2 to 32 columns: 1.3 and 1.9 % behind the better of
+        // the two; by the columns alone 7.5 and 2.4.)
+        const double mb = 1e-6 * nmat * sheet, reads = mb * ncols;
+        const bool shared = q4w ? ncols > 8 && nmat == 2 && reads >= 280
+                                : reads / 6 >= 5 + mb / 4 * n_expert * (1 - std::pow(1 - 1.0 / n_expert, ncols));
+        const bool gather = !shared && (type == JL_TYPE_Q8_0 ? ncols <= 16 || (ncols <= 64 && avg <= 1.1)
+                                                 : (long)nrows * k >= 512L * 512 && ncols <= ((double)nrows * k >= 2.4e6 && avg <= 0.6 ? 32 : 16));
         if (form == 0 && !planes && (type == JL_TYPE_Q8_0 || type == JL_TYPE_Q4_K || q6) && gather) form = 10;
         if (form == 0 && (c->act_window == 32 || c->act_window == 256) && !planes) {
             if (q4w) form = ncols <= 8L * n_expert ? 0 : moe_few_faster(type, n_expert, ncols, nmat, nrows, k) ? 5 : 9;
@@ -2920,7 +2935,7 @@ int moe_ffn(jl_ctx* c, float* resid, int type, int down_type, const void* gate_b
                        planes ? &d : nullptr, x, wt, rows, n_ffn, n_embd, g, u, y, st);
         if (rc != JL_DECLINED) return rc;
     }
-    const bool gather = c->tune.moe_form == 11 || (c->tune.moe_form == 0 && moe_gather_ffn_wanted(type, down_type, planes, rows, k_used, n_expert, n_ffn, n_embd));
+    const bool gather = c->tune.moe_form == 11 || (c->tune.moe_form == 0 && moe_gather_ffn_wanted(c, type, down_type, planes, rows, k_used, n_expert, n_ffn, n_embd));
     if (gather && planes) {
         rc = moe_planes_gather_ffn(c, resid, pg, pu, pd, x, sel, sel_stride, wt, rows, k_used, n_expert, n_ffn, n_embd, g, u, st);
         if (rc != JL_DECLINED) return rc;

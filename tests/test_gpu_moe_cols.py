@@ -338,3 +338,48 @@ def test_ids_that_no_expert_has(dev, devbuf, t, down, window, forms, rows):
     finally:
         dev.set_tuning(moe__form=0, moe__group16=0)
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("t,window,nrows,k,counts,launches", [
+    (quant.Q6_K, 256, 2048, 4096, [9, 7], 2), (quant.Q8_0, 32, 2048, 4096, [9, 7], 2), (quant.Q4_K, 32, 4096, 4096, [9, 7], 2),
+    (quant.Q6_K, 256, 1024, 1024, [1, 2, 1, 1], 1), (quant.Q8_0, 32, 4096, 2048, [1] * 8, 1)],
+    ids=lambda v: str(v))
+def test_columns_that_share_a_large_sheet(dev, devbuf, t, window, nrows, k, counts, launches):
+    """Columns that share sheets of some megabytes are not given a decode matvec each, which would read a sheet again for every
+    one of them (two launches); small sheets and columns of their own are (one)."""
+    n_expert, ncols = len(counts), sum(counts)
+    start = np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32)
+    sheet = nrows * quant.row_bytes(t, k)
+    banks = [np.concatenate([synth.random_weights(t, nrows, k, seed=20 * b + e) for e in range(n_expert)]) for b in range(2)]
+    x = np.stack([synth.activations(k, seed=40 + r) for r in range(ncols)])
+    bd, xd, sd = [devbuf(b) for b in banks], devbuf(x), devbuf(start)
+    dev.SetActWindow(window)
+    try:
+        o = [devbuf(shape=(ncols, nrows), dtype=np.float32, fill=FILL) for _ in banks]
+        before = dev.launch_count()
+        assert dev.moe_matvec_dev(o[0].ptr, o[1].ptr, t, bd[0].ptr, bd[1].ptr, xd.ptr, None, None, sd.ptr, n_expert, ncols, nrows, k)
+        made = dev.launch_count() - before
+        dev.synchronize()
+        assert made == launches
+        e = n_expert - 1
+        for b in range(2):
+            want = oracle.matmul_q8act_f64(t, banks[b][e * sheet:], x[start[e]:], nrows, k, counts[e], window)
+            assert nmse(o[b].get()[start[e]:], want) <= 1e-10
+    finally:
+        dev.SetActWindow(32)
+
+
+def test_pairs_that_share_large_sheets_are_grouped(dev, devbuf):
+    """16 experts, top-4: six rows' pairs, which share sheets of 7.8 MB, are grouped; two rows' hardly share any and are not.
+    (Blocks of zeros: the residual stays.)"""
+    n_expert, k_used, n_ffn, n_embd = 16, 4, 2048, 3584
+    bank = devbuf(np.zeros(n_expert * n_ffn * quant.row_bytes(quant.Q8_0, n_embd), np.uint8))
+    for rows, pairs_alone in ((6, False), (2, True)):
+        sel = np.stack([np.random.default_rng(r).permutation(n_expert)[:k_used] for r in range(rows)]).astype(np.uint32)
+        start = np.stack([synth.activations(n_embd, seed=30 + r) for r in range(rows)])
+        xd, sd, wd, resid = devbuf(start), devbuf(sel), devbuf(np.full((rows, k_used), 0.25, np.float32)), devbuf(start)
+        before = dev.launch_count()
+        assert dev.moe_ffn_dev(resid.ptr, quant.Q8_0, bank.ptr, bank.ptr, bank.ptr, xd.ptr, sd.ptr, k_used, wd.ptr, rows, k_used, n_expert, n_ffn, n_embd)
+        assert (dev.launch_count() - before == 2) == pairs_alone
+        dev.synchronize()
+        assert np.array_equal(resid.get(), start)
