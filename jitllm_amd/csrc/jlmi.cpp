@@ -2733,7 +2733,9 @@ int moe_group_launch(jl_ctx* c, const uint32_t* sel, int sel_stride, int rows, i
     const size_t npairs = (size_t)rows * k_used, lds2 = 16 * (size_t)n_expert * 2 + (2 * (size_t)n_expert + 16) * 4;   // JL_MOE_GROUP2_LDS
     if (c->tune.moe_group != 1 && lds2 <= c->lds_limit && npairs <= 0x7fffffffu - 8192) {
         if (lists->nslots) { a.wl[0] = lists->wl[0]; a.wl[1] = lists->wl[1]; a.nslots = lists->nslots; }
-        return launch(c, "jl_moe_group2", (unsigned)((npairs + 1023) / 1024), 1, 1024, (unsigned)lds2, st, params);
+        const size_t n1024 = (npairs + 1023) / 1024;
+        a.chunks = (int)((n1024 + c->num_cu - 1) / c->num_cu);
+        return launch(c, "jl_moe_group2", (unsigned)((n1024 + a.chunks - 1) / a.chunks), 1, 1024, (unsigned)lds2, st, params);
     }
     lists->nslots = 0;   // (this form makes none)
     return launch(c, "jl_moe_group", 1, 1, 1024, 0, st, params);

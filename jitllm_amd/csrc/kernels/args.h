@@ -309,6 +309,7 @@ struct MoeGroupArgs {
     uint32_t* perm;
     uint32_t* pos;
     int sel_stride, rows, k_used, n_expert;
+    int chunks = 1;         // 1024s of pairs a workgroup (moe_group2_body)
     uint32_t* wl[2] = {};   // null, or the work lists (MoeWorklistArgs) of tiles of 64 and of 128 columns
     int nslots = 0;
 };

@@ -247,10 +247,12 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& p, u32* scoun
 // expert's first column + the expert's pairs in earlier workgroups and runs + its rank in its run: (row, slot) order inside
 // an expert.  One workgroup that walked its sixteen shares run after run took 15.4 us at 6216 pairs, with keys and ranks in
 // registers 12.8 (its ballots alone are 6 us of one CU's issue slots); now 6.6 (512 pairs 4.8 as before).
-// grid = ceil(pairs / 1024), block = 1024, dynamic LDS = JL_MOE_GROUP2_LDS(nexp).
+// The counting is every workgroup's own walk over all pairs, so there are no more workgroups than CUs: from 262144 pairs on
+// each takes several 1024s (p.chunks; one each, four million pairs took 11.8 ms, one workgroup alone 7.3, so 1.0).
+// grid = ceil(pairs / (1024 chunks)), block = 1024, dynamic LDS = JL_MOE_GROUP2_LDS(nexp).
 #define JL_MOE_GROUP2_LDS(nexp) (16 * (nexp) * 2 + (2 * (nexp) + 16) * 4)
 __device__ __forceinline__ void moe_group2_body(const MoeGroupArgs& p, uint8_t* smem) {
-    const int npairs = p.rows * p.k_used, nexp = p.n_expert, lo = (int)blockIdx.x * 1024;
+    const int npairs = p.rows * p.k_used, nexp = p.n_expert, lo = (int)blockIdx.x * 1024 * p.chunks;
     u32* sbefore = (u32*)smem;                // [nexp] pairs of earlier workgroups, then a pair's expert's first column here
     u32* srest = sbefore + nexp;              // [nexp] the other pairs
     u32* stot = srest + nexp;                 // [16] wavefront totals
@@ -288,27 +290,36 @@ __device__ __forceinline__ void moe_group2_body(const MoeGroupArgs& p, uint8_t* 
         }
     }
     const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;   // lanes below this one
-    uint64_t m = __ballot(valid);
-    for (int b = 0; b < nbits; b++) {
-        const bool bit = (e >> b) & 1;
-        const uint64_t bal = __ballot(bit);
-        m &= bit ? bal : ~bal;
-    }
-    const u32 rank = (u32)__builtin_popcountll(m & lt);
     uint16_t* mine = scnt + wave * nexp;
-    if (valid && rank == 0) mine[e] = (uint16_t)__builtin_popcountll(m);
-    __syncthreads();
-    // per expert: counts of successive runs -> pairs in earlier runs
-    u32 total = 0;
-    if (tid < nexp) {
-#pragma unroll
-        for (int w = 0; w < 16; w++) {
-            const u32 c = scnt[w * nexp + tid];
-            scnt[w * nexp + tid] = (uint16_t)total;
-            total += c;
+    // a pair's rank among its expert's in its run, and the run's number of them
+    auto rank_of = [&](u32 e, bool valid) {
+        uint64_t m = __ballot(valid);
+        for (int b = 0; b < nbits; b++) {
+            const bool bit = (e >> b) & 1;
+            const uint64_t bal = __ballot(bit);
+            m &= bit ? bal : ~bal;
         }
-        if (!one) total = sbefore[tid] + srest[tid];
-    }
+        const u32 rank = (u32)__builtin_popcountll(m & lt);
+        if (valid && rank == 0) mine[e] = (uint16_t)__builtin_popcountll(m);
+        return rank;
+    };
+    // per expert: counts of successive runs -> pairs in earlier runs; all of the sixteen's are returned
+    auto runs = [&]() {
+        u32 total = 0;
+        if (tid < nexp) {
+#pragma unroll
+            for (int w = 0; w < 16; w++) {
+                const u32 c = scnt[w * nexp + tid];
+                scnt[w * nexp + tid] = (uint16_t)total;
+                total += c;
+            }
+        }
+        return total;
+    };
+    const u32 rank = rank_of(e, valid);
+    __syncthreads();
+    u32 here = runs(), total = here;
+    if (tid < nexp && !one) total = sbefore[tid] + srest[tid];
     // exclusive scan of the totals over experts (thread = expert; nexp <= 1024)
     u32 v = total;
 #pragma unroll
@@ -359,6 +370,28 @@ __device__ __forceinline__ void moe_group2_body(const MoeGroupArgs& p, uint8_t* 
         const u32 col = sbefore[e] + mine[e] + rank;
         p.perm[col] = (u32)row_of(i);
         p.pos[i] = col;
+    }
+    // very many pairs: the workgroup's further 1024s, one after the other
+    for (int c = 1; c < p.chunks; c++) {
+        const u32 at = (u32)lo + 1024u * c + tid;
+        const int i = (int)at;
+        u32 e = 0;
+        if (at < (u32)npairs) e = key_of(i);
+        __syncthreads();   // (the 1024 before have been placed)
+        if (tid < nexp) sbefore[tid] += here;
+        for (int j = tid; j < 8 * nexp; j += 1024) ((u32*)scnt)[j] = 0;
+        __syncthreads();
+        const bool valid = at < (u32)npairs && e < (u32)nexp;
+        if (!valid) e = 0;
+        const u32 rank = rank_of(e, valid);
+        __syncthreads();
+        here = runs();
+        __syncthreads();
+        if (valid) {
+            const u32 col = sbefore[e] + mine[e] + rank;
+            p.perm[col] = (u32)row_of(i);
+            p.pos[i] = col;
+        }
     }
 }
 

@@ -70,6 +70,28 @@ def test_grouping_is_bit_exact(dev, devbuf, mode, rows, n_expert, k_used, form):
     dev.set_tuning(moe__group=0)
 
 
+@pytest.mark.parametrize("rows,n_expert,k_used", [(32777, 128, 8), (75000, 1000, 16), (40000, 7, 7)])
+def test_grouping_with_several_1024s_a_workgroup(dev, devbuf, rows, n_expert, k_used):
+    """More pairs than a workgroup a CU takes at 1024 each: two and five of them a workgroup, the last one and the last workgroup
+    ragged; ids that no expert has among them (their pairs are left out)."""
+    rng = np.random.default_rng(rows)
+    sel = np.ascontiguousarray(rng.integers(0, n_expert, (rows, k_used)).astype(np.uint32))
+    sel[rng.integers(0, rows, 50), rng.integers(0, k_used, 50)] = n_expert + 5
+    flat = sel.reshape(-1)
+    order = np.argsort(flat, kind="stable")
+    order = order[flat[order] < n_expert]
+    want_start = np.concatenate([[0], np.cumsum(np.bincount(flat[flat < n_expert], minlength=n_expert))]).astype(np.uint32)
+    want_pos = np.full(flat.size, 99, np.uint32)
+    want_pos[order] = np.arange(order.size)
+    sd, start = devbuf(sel), devbuf(shape=(n_expert + 1,), dtype=np.uint32, fill=99)
+    perm, pos = (devbuf(shape=(flat.size,), dtype=np.uint32, fill=99) for _ in range(2))
+    assert dev.moe_group_dev(sd.ptr, k_used, rows, k_used, n_expert, start.ptr, perm.ptr, pos.ptr)
+    dev.synchronize()
+    assert np.array_equal(start.get(), want_start)
+    assert np.array_equal(perm.get()[:order.size], (order // k_used).astype(np.uint32)) and np.all(perm.get()[order.size:] == 99)
+    assert np.array_equal(pos.get(), want_pos)
+
+
 @functools.lru_cache(maxsize=8)
 def _banks(t, n_expert, nrows, k, seed, planted):
     make = synth.random_weights if planted else synth.quantized_weights
