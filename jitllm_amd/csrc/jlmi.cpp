@@ -325,7 +325,7 @@ int x_groups(const jl_ctx* c, int k, int threads) {
 hipStream_t pick_stream(jl_ctx* c, void* s) { return s ? (hipStream_t)s : c->stream; }
 
 // LDS of the decode matvec: int8 activations, a scale per 32, a sum per 16
-size_t act_lds_bytes(int k) { return (size_t)k + (size_t)(k / 32) * 4 + (size_t)(k / 16) * 4; }
+size_t act_lds_bytes(int k) { return JL_ACT_LDS_BYTES((size_t)k); }
 
 // Q8_0 rows in the form that takes two blocks a lane-slot with every load 4-byte aligned
 // (kernels/matvec.h): rows on 4-byte boundaries, an even number of blocks a row, room in
@@ -589,8 +589,8 @@ int matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, const vo
     name << (norm_w ? x2 ? "_na" : "_n" : x2 ? "_a" : "") << (types || xpre == 1 ? "" : xpre == 4 ? "_x4" : "_x2") << (resid ? "_res" : "");
     if (lanes != 64) name << "_l" << lanes;
     void* params[] = {&a};
-    // (+ 16 to round the staging area up, + JL_NORM_LDS_BYTES for the RMSNorm's partial sums)
-    unsigned lds = (unsigned)(act_lds_bytes(k) + (pair ? (size_t)k + 16 : 0) + 16 + 160);
+    // (+ 16 to round the staging area up)
+    unsigned lds = (unsigned)(act_lds_bytes(k) + (pair ? (size_t)k + 16 : 0) + 16 + JL_NORM_LDS_BYTES);
     return launch(c, name, (unsigned)gx, (unsigned)m, nwaves * 64, lds, st, params);
 }
 
@@ -1366,7 +1366,7 @@ int packed_matvec_launch(jl_ctx* c, float* out, int type, const PlaneRef& pl, co
     name << "jl_matvec_packed_" << (x ? "" : "q8_") << ti->tag << "_w" << rw;
     void* params[] = {&a};
     return launch(c, name, (unsigned)((nrows + rw - 1) / rw), 1, (unsigned)(nw * 64),
-                  (unsigned)(nw * (384 + 65 * 4)), st, params);  // JL_PK_LDS_BYTES
+                  (unsigned)JL_PK_LDS_BYTES(nw), st, params);
 }
 
 // m packed matvecs of one type and shape in one launch (grid.y = matrix): each with its
@@ -1415,7 +1415,7 @@ int packed_matvec_multi_launch(jl_ctx* c, int type, int m, float* const* outs, c
     name << "jl_matvec_packed_multi_" << (up ? "act_" : norm_w ? "norm_" : "") << (tokens && type == JL_TYPE_Q4_K ? "q4kf" : ti->tag) << "_w" << rw;
     void* params[] = {&a};
     return launch(c, name, (unsigned)a.ngroups, (unsigned)m, (unsigned)(nw * 64),
-                  (unsigned)(nw * (384 + 65 * 4) + (norm_w ? 16 + 160 : 0)), st, params);   // JL_PK_LDS_BYTES + JL_NORM_LDS_BYTES
+                  (unsigned)(JL_PK_LDS_BYTES(nw) + (norm_w ? 16 + JL_NORM_LDS_BYTES : 0)), st, params);
 }
 
 // MXFP4 planes (QS and D only): rows row .. row+nrows of a buffer of `stride` rows.
@@ -1726,7 +1726,7 @@ int moe_planes_gather_ffn(jl_ctx* c, float* resid, const jl_packed_bank* pg, con
     Name name;
     name << "jl_moe_planes_gather_w" << rw;
     void* params[] = {&a};
-    int rc = launch(c, name, (unsigned)a.ngroups, (unsigned)pairs, 64u * a.nwaves, (unsigned)(a.nwaves * (384 + 65 * 4)), st, params, 2);   // JL_PK_LDS_BYTES
+    int rc = launch(c, name, (unsigned)a.ngroups, (unsigned)pairs, 64u * a.nwaves, (unsigned)JL_PK_LDS_BYTES(a.nwaves), st, params, 2);
     if (rc != JL_OK) return rc;
     MoePlanesDownArgs b;
     b.resid = resid; b.qs = pd->qs; b.d = pd->d; b.sc = pd->sc; b.g = g; b.u = u; b.sel = sel; b.wt = wt;
@@ -1738,7 +1738,7 @@ int moe_planes_gather_ffn(jl_ctx* c, float* resid, const jl_packed_bank* pg, con
     Name dname;
     dname << "jl_moe_planes_down_w" << dw;
     void* dparams[] = {&b};
-    return launch(c, dname, (unsigned)b.ngroups, (unsigned)rows, 64u * b.nwaves, (unsigned)(b.nwaves * (384 + 65 * 4)), st, dparams);
+    return launch(c, dname, (unsigned)b.ngroups, (unsigned)rows, 64u * b.nwaves, (unsigned)JL_PK_LDS_BYTES(b.nwaves), st, dparams);
 }
 
 // The columns of an expert against rows decoded in registers (kernels/moe_cols.h): the source rows quantized once each
@@ -1748,11 +1748,9 @@ int moe_cols_launch(jl_ctx* c, float* out0, float* out1, int type, const void* b
                     int ncols, int nrows, int k, int nsrc, hipStream_t st) {
     const TypeInfo* ti = type_info(type);
     const bool q6 = type == JL_TYPE_Q6_K, planes = pb0 != nullptr, mapped = src && nsrc > 0 && nsrc <= ncols;
-    const size_t nsb = (size_t)k / 256, nrec = mapped ? nsrc : ncols, rec = q6 ? 256 : 512;
+    const size_t nsb = (size_t)k / 256, nrec = mapped ? nsrc : ncols, rec = JL_MC_REC(q6);
     const int nmat = (planes ? pb1 != nullptr : bank1 != nullptr) ? 2 : 1;
-    const unsigned lds = q6       ? 2u * 64u * 256u + 128u * (208u + 16u + 2u) + 64u * 4u   // JL_MC_Q6_LDS
-                         : planes ? 2u * 64u * (512u + 32u + 4u)                          // JL_MC_PLANES_LDS
-                                  : 2u * (64u * 256u + 128u * 144u + 64u * 36u);          // JL_MC_Q4_LDS
+    const unsigned lds = q6 ? JL_MC_Q6_LDS : planes ? JL_MC_PLANES_LDS : JL_MC_Q4_LDS;
     // (32-bit offsets in the kernels: records, and half a super-block's words of every row of the planes)
     if (nrec * nsb * rec >= ((size_t)1 << 32) || (planes && (size_t)pb0->stride >= ((size_t)1 << 25)) || lds > c->lds_limit) return JL_DECLINED;
     const double avg = (double)ncols / n_expert;
@@ -2730,7 +2728,7 @@ int moe_group_launch(jl_ctx* c, const uint32_t* sel, int sel_stride, int rows, i
     void* params[] = {&a};
     // the linear-time form, a workgroup for 1024 pairs (moe.group = 1 forces the one that compares every pair with every
     // expert)
-    const size_t npairs = (size_t)rows * k_used, lds2 = 16 * (size_t)n_expert * 2 + (2 * (size_t)n_expert + 16) * 4;   // JL_MOE_GROUP2_LDS
+    const size_t npairs = (size_t)rows * k_used, lds2 = JL_MOE_GROUP2_LDS((size_t)n_expert);
     if (c->tune.moe_group != 1 && lds2 <= c->lds_limit && npairs <= 0x7fffffffu - 8192) {
         if (lists->nslots) { a.wl[0] = lists->wl[0]; a.wl[1] = lists->wl[1]; a.nslots = lists->nslots; }
         const size_t n1024 = (npairs + 1023) / 1024;

@@ -4,6 +4,20 @@
 #pragma once
 #include <stdint.h>
 
+// ---- dynamic LDS of the decode matvecs, as the kernels divide it and the host asks for it
+// Bytes of LDS the staging area needs for a k-element activation.
+#define JL_ACT_LDS_BYTES(k) ((k) + ((k) / 32) * 4 + ((k) / 16) * 4)
+// the grouped kernels' RMSNorm: up to sixteen partial sums and the scale, behind the staging area
+#define JL_NORM_LDS_BYTES 160
+// ... and with the second copy of the int8 values that the Q8_0 pair form reads (k % 64 == 0)
+#define JL_ACT_LDS_BYTES_SHIFTED(k) (JL_ACT_LDS_BYTES(k) + (k) + 16)
+// A wavefront's private LDS: 256 int8 activations, 8 scales, 16 half-block sums.
+#define JL_PK_WAVE_LDS 384
+// Dynamic LDS of a workgroup of `nw` wavefronts: the private areas, then the
+// partial sums [nw][64], rows one word apart in banks.
+#define JL_PK_RED_STRIDE 65
+#define JL_PK_LDS_BYTES(nw) ((nw) * (JL_PK_WAVE_LDS + JL_PK_RED_STRIDE * 4))
+
 struct MatVecArgs {
     float* out;          // [nrows]
     const uint8_t* w;    // GGUF row-major blocks
@@ -169,8 +183,6 @@ struct MoeGemmArgs {
     const float* dsum = nullptr;   // the int8 form, Q4_K: d_a * block sums
 };
 
-// Grouped expert matmul for experts of some tens of columns (kernels/moe_cols.h): rec [record][k/256][512 or 256 bytes],
-// aug [record][k/256][32 bytes], da [record][k/256].
 // A decode matvec a routed column (moe_gather_body): grid y = column, z = matrix.
 struct MoeGatherArgs {
     float* out[2];          // [column][nrows]
@@ -216,6 +228,18 @@ struct MoePlanesDownArgs {
     int nrows, k, row_step, stride, per, nwaves, ngroups, n_expert, sel_stride, k_used;
 };
 
+// Grouped expert matmul for experts of some tens of columns (kernels/moe_cols.h): rec [record][k/256][512 or 256 bytes],
+// aug [record][k/256][32 bytes], da [record][k/256].
+// A column's record of one super-block: the operand pieces of sixteen bytes in the order the weights decode to
+// (Q4_K: f16, piece 2 ks + kg of K-step ks = 0..15; Q6_K: int8, piece 8 kg + ks, ks = 0..7).
+#define JL_MC_REC(q6) ((q6) ? 256 : 512)
+// its dynamic LDS: Q4_K rows (columns by halves of a super-block, rows as they lie), Q6_K rows, Q4_K planes
+#define JL_MC_A (64 * 256)      // half a super-block of 64 columns
+#define JL_MC_W (128 * 144)
+#define JL_MC_Q4_LDS (2 * JL_MC_A + 2 * JL_MC_W + 2 * (64 * 32 + 64 * 4))
+#define JL_MC_Q6_W (128 * 208)
+#define JL_MC_Q6_LDS (2 * 64 * 256 + JL_MC_Q6_W + 128 * 16 + 128 * 2 + 64 * 4)
+#define JL_MC_PLANES_LDS (2 * (64 * 512 + 64 * 32 + 64 * 4))
 struct MoeColsPrepArgs {
     const float* x;
     const float* x2;        // null: plain activation, else silu(x) * x2
@@ -303,6 +327,8 @@ struct GemmW16Args {
 // Mixture-of-experts grouping: sel [rows][sel_stride] expert ids (the first k_used of
 // each row are the selection) -> start [n_expert+1], perm [rows*k_used] (column ->
 // row), pos [rows*k_used] (pair -> column).
+// Dynamic LDS of the linear-time form (moe_group2_body).
+#define JL_MOE_GROUP2_LDS(nexp) (16 * (nexp) * 2 + (2 * (nexp) + 16) * 4)
 struct MoeGroupArgs {
     const uint32_t* sel;
     uint32_t* start;

@@ -31,13 +31,6 @@ struct ActLds {
     const uint8_t* a2;   // the Q8_0 pair form only: a second copy of a[], two bytes further on
 };
 
-// Bytes of LDS the staging area needs for a k-element activation.
-#define JL_ACT_LDS_BYTES(k) ((k) + ((k) / 32) * 4 + ((k) / 16) * 4)
-// the grouped kernels' RMSNorm: up to sixteen partial sums and the scale, behind the staging area
-#define JL_NORM_LDS_BYTES 160
-// ... and with the second copy of the int8 values that the Q8_0 pair form reads (k % 64 == 0)
-#define JL_ACT_LDS_BYTES_SHIFTED(k) (JL_ACT_LDS_BYTES(k) + (k) + 16)
-
 __device__ __forceinline__ ActLds act_lds_views(uint8_t* smem, int k) {
     ActLds v;
     v.a = smem;

@@ -250,7 +250,6 @@ __device__ __forceinline__ void moe_group_body(const MoeGroupArgs& p, u32* scoun
 // The counting is every workgroup's own walk over all pairs, so there are no more workgroups than CUs: from 262144 pairs on
 // each takes several 1024s (p.chunks; one each, four million pairs took 11.8 ms, one workgroup alone 7.3, so 1.0).
 // grid = ceil(pairs / (1024 chunks)), block = 1024, dynamic LDS = JL_MOE_GROUP2_LDS(nexp).
-#define JL_MOE_GROUP2_LDS(nexp) (16 * (nexp) * 2 + (2 * (nexp) + 16) * 4)
 __device__ __forceinline__ void moe_group2_body(const MoeGroupArgs& p, uint8_t* smem) {
     const int npairs = p.rows * p.k_used, nexp = p.n_expert, lo = (int)blockIdx.x * 1024 * p.chunks;
     u32* sbefore = (u32*)smem;                // [nexp] pairs of earlier workgroups, then a pair's expert's first column here

@@ -21,10 +21,6 @@
 
 #pragma clang fp contract(off)
 
-// A column's record of one super-block: the operand pieces of sixteen bytes in the order the weights decode to
-// (Q4_K: f16, piece 2 ks + kg of K-step ks = 0..15; Q6_K: int8, piece 8 kg + ks, ks = 0..7).
-#define JL_MC_REC(q6) ((q6) ? 256 : 512)
-
 // KO: 0 Q4_K GGUF rows, 1 Q4_K planes, 2 Q6_K rows.  A wavefront takes four (record, super-block) tasks.
 template <int KO>
 __device__ __forceinline__ void moe_cols_prep_body(const MoeColsPrepArgs& args) {
@@ -129,9 +125,6 @@ __device__ __forceinline__ void mc_store(const MoeColsArgs& p, const f32x16 (&ou
 
 // Q4_K rows.  G: groups of 32 columns (n columns exist).  The rows' bytes come to LDS as they lie, 144 contiguous bytes a
 // row (straight into registers, a lane a row, is sixteen bytes of 64 lines an instruction), and each wavefront reads its own.
-#define JL_MC_A (64 * 256)      // half a super-block of 64 columns
-#define JL_MC_W (128 * 144)
-#define JL_MC_Q4_LDS (2 * JL_MC_A + 2 * JL_MC_W + 2 * (64 * 32 + 64 * 4))
 template <int G>
 __device__ __forceinline__ void moe_cols_q4_tile(const MoeColsArgs& p, uint8_t* smem, int e, int mat, int r0, u32 c0, int n) {
     constexpr int O_W = 2 * JL_MC_A, O_AUG = O_W + 2 * JL_MC_W, O_DA = O_AUG + 2 * 64 * 32;
@@ -287,8 +280,6 @@ __device__ __forceinline__ void moe_cols_q4_tile(const MoeColsArgs& p, uint8_t* 
 
 // Q6_K rows: 210-byte blocks lie on two-byte boundaries, so the rows' bytes come through registers (sixteen bytes a lane along
 // the row), a super-block ahead, and are laid down in LDS when the one before has been used.
-#define JL_MC_Q6_W (128 * 208)
-#define JL_MC_Q6_LDS (2 * 64 * 256 + JL_MC_Q6_W + 128 * 16 + 128 * 2 + 64 * 4)
 template <int G>
 __device__ __forceinline__ void moe_cols_q6_tile(const MoeColsArgs& p, uint8_t* smem, int e, int mat, int r0, u32 c0, int n) {
     constexpr int A_SB = 64 * 256, O_W = 2 * A_SB, O_D = O_W + JL_MC_Q6_W + 128 * 16, O_DA = O_D + 128 * 2;
@@ -423,7 +414,6 @@ __device__ __forceinline__ void moe_cols_q6_tile(const MoeColsArgs& p, uint8_t* 
 
 // Q4_K planes: a lane's words of its row straight into registers, a super-block ahead (every request is 32 rows' words of a plane).
 struct MoeColsPlaneWords { u32x4 h, q[4]; };   // (d, dmin) and the words of six-bit fields; words of K-steps 4 v ..
-#define JL_MC_PLANES_LDS (2 * (64 * 512 + 64 * 32 + 64 * 4))
 template <int G>
 __device__ __forceinline__ void moe_cols_planes_tile(const MoeColsArgs& p, uint8_t* smem, int e, int mat, int r0, u32 c0, int n) {
     constexpr int REC = 512, BUF = 64 * REC, O_AUG = 2 * BUF, AUG = 64 * 32, O_DA = O_AUG + 2 * AUG, NW = 20,

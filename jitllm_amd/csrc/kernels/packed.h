@@ -287,13 +287,6 @@ __device__ __forceinline__ void unpack_body(const UnpackArgs& p, uint8_t* lds) {
 
 // ---------------------------------------------------------------- matvec
 
-// A wavefront's private LDS: 256 int8 activations, 8 scales, 16 half-block sums.
-#define JL_PK_WAVE_LDS 384
-// Dynamic LDS of a workgroup of `nw` wavefronts: the private areas, then the
-// partial sums [nw][64], rows one word apart in banks.
-#define JL_PK_RED_STRIDE 65
-#define JL_PK_LDS_BYTES(nw) ((nw) * (JL_PK_WAVE_LDS + JL_PK_RED_STRIDE * 4))
-
 struct PkAct {
     const u32x4* a;    // int8 activations of the chunk, 16 per vector
     const float* da;   // [8]
