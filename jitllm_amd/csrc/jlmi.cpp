@@ -1190,6 +1190,9 @@ bool tokens_matvec_wanted(const jl_ctx* c, int type, bool planes, int nrows, int
     if (ntok < 2 || ntok > JL_MAX_MULTI) return false;
     if (c->tune.gemm_few == 3) return true;
     if (ntok > 8 || c->tune.gemm_few || c->tune.gemm_form || c->gemm_min_tok != 3) return false;
+    // (Short rows over planes, where one launch takes wider runs and a lane the more blocks of a row: NMSE against 64 bits at K =
+    // 256 to 512, Q6_K two tokens 5.5e-15 and two launches 4.0e-15, Q8_0 three 5.2e-15 and the few-token kernel 4.3e-15.)
+    if (planes && k < 1024 && type != JL_TYPE_Q4_K) return false;
     if (ntok == 2 && type != JL_TYPE_Q8_0) return true;
     // (Q6_K over planes, and short rows under a shorter window: the matvec's sums round more than the few-token kernel's, NMSE
     // against 64 bits 8.3e-15 and 4.8e-15 for eight tokens at K = 2048 over planes, 4.6e-15 and 4.3e-15 for three at K = 512)

@@ -217,3 +217,29 @@ def test_tokens_side_by_side_round_no_more_than_the_few_token_kernel(dev, devbuf
     finally:
         dev.set_tuning(gemm__few=0, moe__form=0)
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("t,ntok", [(quant.Q6_K, 2), (quant.Q8_0, 3)], ids=["q6_k", "q8_0"])
+def test_short_rows_over_planes_keep_their_kernels(dev, devbuf, t, ntok):
+    """Under K = 1024, two tokens of Q6_K are the decode matvec's bits token by token and three of Q8_0 the few-token kernel's: side
+    by side in one launch they round more."""
+    nrows, k = 8192, 512
+    w = synth.quantized_weights(t, nrows, k, seed=7)
+    x = np.stack([synth.activations(k, seed=300 + i) for i in range(ntok)])
+    wd, xd = devbuf(w), devbuf(x)
+    planes = [devbuf(np.zeros(max(n, 4), np.uint32)) for n in quant.packed_words(t, nrows, k)]
+    assert dev.pack_weights_dev(t, wd.ptr, nrows, k, *[p.ptr for p in planes])
+    p = Packed(*[p.ptr for p in planes], 0, nrows)
+    out, want = (devbuf(shape=(ntok, nrows), dtype=np.float32) for _ in range(2))
+    assert dev.matmul_packed_dev(out.ptr, t, p, xd.ptr, nrows, k, ntok)
+    try:
+        if t == quant.Q6_K:
+            for i in range(ntok):
+                assert dev.matvec_packed_dev(want.ptr + i * nrows * 4, t, p, xd.ptr + i * k * 4, nrows, k)
+        else:
+            dev.set_tuning(gemm__few=1)
+            assert dev.matmul_packed_dev(want.ptr, t, p, xd.ptr, nrows, k, ntok)
+        dev.synchronize()
+        assert np.array_equal(out.get().view(np.uint32), want.get().view(np.uint32))
+    finally:
+        dev.set_tuning(gemm__few=0)
