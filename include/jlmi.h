@@ -97,7 +97,7 @@ int jl_synchronize(jl_ctx *ctx);
  * tiles, 3: two-pass, 4: up to 64 tokens on the int8 matrix cores, 5: 32 rows x 64 tokens a
  * workgroup, 6: 128 x 64 tiles over the whole of K on two groups of wavefronts, 9: token by
  * token), "gemm.few" (1: form 4 for any number of tokens, 2: never,
- * 3: a decode matvec a token in one launch, up to eight), "few.nt" / "few.rt" /
+ * 3: a decode matvec a token in one launch, up to sixteen), "few.nt" / "few.rt" /
  * "few.waves" (its token tiles, row tiles and wavefronts a workgroup), "gemm.i8" (the int8 tiles of
  * Q8_0: 1 / 2 / 3 for 128 x 128 / 128 tokens x 64 rows / 256 x 128), "matvec.lanes" (lanes a row of a decode matvec: 16, 32, 64), "gemm.rows" (64 or 128),
  * "gemm.split" (K slices), "gemm.prep" (4: the four-wavefront activation prep), "gemm.planes"
@@ -339,7 +339,9 @@ int jl_matvec_packed_group(jl_ctx *ctx, int n, float *const *outs, const int *ty
  * its own.  From two (Q8_0) or three tokens a quantize-and-lay-out kernel and a matrix-core
  * kernel, in a workspace the context owns: few tokens (up to 64, and more where it is estimated
  * faster) the int8 few-token kernel, any window; more on f16 tiles (Q4_K, window 256) or int8 tiles (window 32;
- * Q6_K also 256).  Up to eight tokens may run as a decode matvec each, in one launch and without a workspace.
+ * Q6_K also 256).  Up to eight tokens may run as a decode matvec each, in one launch and without a workspace (Q6_K over
+ * planes: two).  Which kernel serves is chosen by shape, number of tokens and layout, so a token's result agrees
+ * between calls to f32 rounding and not bit for bit.
  * Other cases run one fused matvec launch per token, which the reference also falls
  * back to (engine/model/prefill.go:1036-1041).  The workspace grows on demand
  * (a device allocation); jl_reserve sizes it ahead of time. */
@@ -560,6 +562,9 @@ int jl_moe_combine_dev(jl_ctx *ctx, float *resid, const float *y, const float *w
  * into the down launch's quantizer, combine into resid [rows][n_embd] (accumulated).
  * gate/up banks: n_expert sheets of n_ffn x n_embd; down bank: n_embd x n_ffn.
  * A pair whose id no expert has adds nothing.
+ * A handful of pairs (at most 256, where that is estimated faster) has neither grouping nor combine: a decode matvec a pair,
+ * then one a row over all of its pairs' gated columns, whose weighted sum runs over the pairs in slot order and is added
+ * to resid once.  Its bits are not those of the calls above one after the other, which add expert after expert.
  * Intermediates live in a workspace the context owns (grown on demand). */
 int jl_moe_ffn_dev(jl_ctx *ctx, float *resid, int type, const void *gate_bank,
                    const void *up_bank, const void *down_bank, const float *x,
