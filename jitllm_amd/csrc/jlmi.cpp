@@ -59,6 +59,7 @@ struct Tuning {
                                 // matvec; rows and planes: 3 / 4 the tiles of 64 / 96 rows
     int mx_split = 0;
     int mx_few = 0, mx_few_min = 0;   // MXFP4: the few-token form up to / from this many tokens
+    int mx_one = 0;                   // ... in one launch: 1 never, 11 / 12 wherever it can be, that many row tiles a workgroup
 };
 
 // The code object's kernels by name.  Looked up on every launch, so without a string to allocate or a tree to
@@ -2176,6 +2177,9 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_logits_e8_f16", "jl_moe_group", "jl_moe_group2", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_few_planes_t1", "jl_mxfp4_few_planes_t2", "jl_mxfp4_few_planes_t3", "jl_mxfp4_few_planes_t4", "jl_mxfp4_few_c3", "jl_mxfp4_few_c4", "jl_mxfp4_few_planes_c3", "jl_mxfp4_few_planes_c4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_planes_gemm_r96", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_silu_mul", "jl_add_rows", "jl_host_in", "jl_host_done", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
                                       "jl_pack_weights", "jl_unpack_q4k", "jl_unpack_q6k", "jl_unpack_q8_0"};
     names.push_back("jl_few_prep");
+    for (const char* pl : {"", "planes_"})
+        for (int nt = 1; nt <= 4; nt++)
+            for (int rt = 1; rt <= 2; rt++) names.push_back(std::string("jl_mxfp4_one_") + pl + "t" + std::to_string(nt) + "r" + std::to_string(rt));
     names.push_back("jl_gemm_i8_prep");
     names.push_back("jl_moe_gemm_i8_prep");
     for (const char* tag : {"q4k", "q8_0", "q8_0p", "q6k", "q6kw"})
@@ -2353,6 +2357,7 @@ int jl_set_tuning(jl_ctx* c, const char* key, int value) {
     else if (!strcmp(key, "mxfp4.split")) c->tune.mx_split = value;
     else if (!strcmp(key, "mxfp4.few")) c->tune.mx_few = value;
     else if (!strcmp(key, "mxfp4.few_min")) c->tune.mx_few_min = value;
+    else if (!strcmp(key, "mxfp4.one")) c->tune.mx_one = value;
     else if (!strcmp(key, "mxfp4.rows")) c->tune.mx_rows = value;
     else if (!strcmp(key, "mxfp4.planes")) c->tune.mx_planes = value;
     else if (!strcmp(key, "mxfp4.scaled")) c->tune.mx_scaled = value;
@@ -3302,6 +3307,63 @@ bool mx_few_applies(const jl_ctx* c, int nrows, int k, int ntok, bool planes) {
     const MxRowsPlan p = mx_rows_plan(c, nrows, k, ntok);
     return 1.1 * (4 + 0.48e-3 * k * nt * rounds) < std::min(p.rows_us, p.planes_us);
 }
+// The same tiles in one launch that takes the activations as they lie (mx_one_body): how many row tiles a workgroup owns, 0: another
+// form.  Its workgroups bring all activations to their CU, so one of more row tiles is worth it where it saves a round; where LDS
+// (128 KB from five units of 16 tokens x 1024 of K on) leaves a CU one workgroup, a started round counts whole.  us, fitted to 12
+// shapes, 512 x 512 to 12288 x 2048, 2 to 256 tokens (rows 5 %, planes 8), beside what else serves: two launches 5 to 5.8 and a slope, a
+// decode matvec a token over rows, tiles.  Two launches -> one: 2880 x 2880 rows, 3 / 16 / 64 tokens 7.5 -> 6.4, 8.2 -> 6.6, 11.0 ->
+// 10.0, planes 8.0 -> 5.7, 7.4 -> 5.9, 10.3 -> 9.2; 5760 x 5760 planes, 16 and 64 tokens 12.5 -> 9.9, 21.3 -> 15.6; 1024 x 1024, 16
+// tokens 6.2 -> 3.9.  More than 64 tokens while the chunks are one round: 2880 x 2880 rows, 128 tokens 18.0 -> 13.0; two
+// rounds lose (5305 x 3520 planes, 128 tokens 16.8 against 21.2).  Two launches stay where the rounds are several and full: 12288 x 2048
+// rows, 64 tokens 16.2 against 17.3.
+double mx_one_us(const jl_ctx* c, int nrows, int k, int ntok, bool planes, int rt, double* rounds) {
+    const int tiles = (ntok + 15) / 16, chunks = (tiles + 3) / 4, nt = (tiles + chunks - 1) / chunks;
+    const double wgs = (double)((nrows + 16 * rt - 1) / (16 * rt)) * ((tiles + nt - 1) / nt), full = wgs / c->num_cu, kk = k / 1024.0;
+    const bool two = 2 * JL_MX_ONE_LDS(k, nt) <= 160 * 1024;   // workgroups a CU
+    *rounds = two ? std::max(1.0, full) : std::ceil(full);
+    const double us = planes ? 2.4 + *rounds * (rt == 1 ? 1.1 + kk * (0.62 + 0.4 * (nt - 1)) : 1.0 + kk * (1.0 + 0.435 * (nt - 1)))
+                             : rt == 1 ? 2.6 + *rounds * (0.3 + kk * (1.2 + 0.385 * (nt - 1))) : 3.2 + *rounds * (kk * (2.03 + 0.46 * (nt - 1)) - 0.4);
+    return !two && full > 1 ? 1.15 * us : us;
+}
+int mx_one_rows(const jl_ctx* c, int nrows, int k, int ntok, bool planes) {
+    const int form = c->tune.mx_one, tiles = (ntok + 15) / 16, chunks = (tiles + 3) / 4, nt = (tiles + chunks - 1) / chunks;
+    // (a lane's place among the activations is 32 bits)
+    if (form == 1 || ntok < 2 || chunks > 65535 || (size_t)ntok * k >= ((size_t)1 << 31) || (unsigned)JL_MX_ONE_LDS(k, nt) > c->lds_limit) return 0;
+    if (form == 11 || form == 12) return form - 10;
+    const int pf = c->tune.mx_planes;
+    if (c->tune.mx_rows || c->tune.mx_split || c->tune.mx_few > 0 || c->tune.mx_few_min > 0 || pf == 3 || pf == 4) return 0;
+    if (planes && (pf == 2 || (pf && ntok <= 8))) return 0;
+    double r1, r2;
+    const double us1 = mx_one_us(c, nrows, k, ntok, planes, 1, &r1), us2 = mx_one_us(c, nrows, k, ntok, planes, 2, &r2);
+    const double us = std::min(us1, us2), kk = k / 1024.0;
+    const int rt = us1 <= us2 ? 1 : 2;
+    double other;
+    if (ntok <= 8 && !mx_few_applies(c, nrows, k, ntok, planes)) {
+        if (planes) return rt;
+        const long r4 = ((nrows + 3) / 4 + (long)c->num_cu - 1) / c->num_cu;
+        other = (3.2 + ntok * (0.1 + 0.13e-3 * k * r4)) / 1.08;
+    } else {
+        const double full = std::max(1.0, (double)((nrows + 15) / 16) * ((tiles + nt - 1) / nt) / c->num_cu), r = 0.5 * (full + std::ceil(full));
+        const double two = planes ? 5.8 + r * kk * (0.63 + 0.31 * (nt - 1)) : 5.0 + r * kk * (1.21 + 0.31 * (nt - 1));
+        other = two;
+        if (ntok > 64) {
+            if ((rt == 1 ? r1 : r2) > 1) return 0;
+            int trows;
+            const MxRowsPlan p = mx_rows_plan(c, nrows, k, ntok);
+            other = planes ? 6 + 2.75 * kk * mx_tile_rounds(c, nrows, ntok, &trows) : std::min(p.rows_us, p.planes_us);
+            if (mx_few_applies(c, nrows, k, ntok, planes)) other = std::min(other, two);
+        }
+    }
+    return us < other ? rt : 0;
+}
+int mx_one_launch(jl_ctx* c, MxGemmArgs& a, int rt, hipStream_t st) {
+    const int tiles = (a.ntok + 15) / 16, chunks = (tiles + 3) / 4, nt = (tiles + chunks - 1) / chunks;
+    const unsigned lds = JL_MX_ONE_LDS(a.k, nt);
+    void* params[] = {&a};
+    Name name;
+    name << "jl_mxfp4_one_" << (a.qs ? "planes_t" : "t") << nt << 'r' << rt;
+    return launch(c, name, (unsigned)((a.nrows + 16 * rt - 1) / (16 * rt)), (unsigned)((tiles + nt - 1) / nt), 512, lds, st, params);
+}
 int mx_few_launch(jl_ctx* c, MxGemmArgs& a, const uint16_t* x, hipStream_t st) {
     const int tiles = (a.ntok + 15) / 16, groups = (a.k + 127) / 128, chunks = (tiles + 3) / 4, nt = (tiles + chunks - 1) / chunks;
     int rc = gemm_ws_ensure(c, (size_t)groups * 4 * tiles * 1024);
@@ -3371,6 +3433,7 @@ int jl_matmul_mxfp4_bf16_dev(jl_ctx* c, float* out, const void* w, const uint16_
         // 2880 rows and left 76 CUs without one: 4.65 -> 4.18 us)
         return launch(c, name, (unsigned)((nrows + JL_MX1_RPW - 1) / JL_MX1_RPW), 1, 64, 0, st, params);
     }
+    if (const int rt = mx_one_rows(c, nrows, k, ntok, false)) return mx_one_launch(c, a, rt, st);
     if (mx_few_applies(c, nrows, k, ntok, false)) return mx_few_launch(c, a, x, st);
     if (ntok <= 8)  // a handful of tokens: stream the rows once, no tile to fill
         return launch(c, "jl_mxfp4_matvec", (unsigned)((nrows + 3) / 4), 1, 256, 0, st, params);
@@ -3448,11 +3511,13 @@ int jl_matmul_mxfp4_packed_bf16_dev(jl_ctx* c, float* out, const uint32_t* qs, c
         if (stiles > 0x7fffffffL / 2) return JL_DECLINED;
         return launch(c, "jl_mxfp4_scaled_gemm", (unsigned)(8 * ((stiles + 7) / 8)), 1, 256, 65536, st, gp);
     }
-    if (mx_few_applies(c, nrows, k, ntok, true)) {
+    const int one = mx_one_rows(c, nrows, k, ntok, true);
+    if (one || mx_few_applies(c, nrows, k, ntok, true)) {
         MxGemmArgs a;
         a.out = out; a.w = nullptr; a.x = x; a.nrows = nrows; a.k = k; a.ntok = ntok; a.row_bytes = 0;
         a.nsplit = 1; a.part = nullptr; a.tok_pad = 0;
         a.qs = qs; a.d = d; a.row0 = row; a.stride = stride;
+        if (one) return mx_one_launch(c, a, one, st);
         return mx_few_launch(c, a, x, st);
     }
     if (ntok <= 8 && (c->tune.mx_planes < 2 || c->tune.mx_planes > 4)) {

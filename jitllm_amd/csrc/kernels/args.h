@@ -430,6 +430,10 @@ struct MxPrepArgs {
     int ntok, tok_pad, k;
 };
 
+// The one-launch few-token kernel (mx_one_body): token tiles of a group of activations (4 KB) a wavefront has room for, as many as
+// it works on at most (two row tiles' sums have to fit); dynamic LDS of its eight wavefronts.
+#define JL_MX_ONE_SLOTS(k, nt) (((k) + 1023) / 1024 * (nt) < 4 ? ((k) + 1023) / 1024 * (nt) : 4)
+#define JL_MX_ONE_LDS(k, nt) (8 * 4096 * JL_MX_ONE_SLOTS(k, nt))
 struct MxGemmArgs {
     float* out;
     const uint8_t* w;     // GGUF row-major MXFP4 blocks (17 bytes per 32)

@@ -83,6 +83,17 @@ __device__ __forceinline__ void lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
+// Loads that write LDS directly: sixteen (four) bytes a lane from a uniform base plus a 32-bit lane offset to LDS at `to` + 16 (4) *
+// lane.  The compiler does not count them: wait_loads<N> waits until at most N of the wavefront's loads are out.
+__device__ __forceinline__ void load_lds16(const uint8_t* base, u32 off, u32 to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(base) : "memory", "m0");
+}
+__device__ __forceinline__ void load_lds4(const uint8_t* base, u32 off, u32 to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(to), "v"(off), "s"(base) : "memory", "m0");
+}
+template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+__device__ __forceinline__ u32 lds_address(const void* q) { return (u32)(uintptr_t)(const __attribute__((address_space(3))) void*)q; }
+
 // Q4_K / Q5_K 6-bit scale and minimum of sub-block j from the 12 packed bytes,
 // given as three little-endian words (format/quant/dequant.go:360-365).
 __device__ __forceinline__ void scale_min_k4(int j, u32 s0, u32 s1, u32 s2, u32& sc, u32& m) {

@@ -540,6 +540,12 @@ JL_MX_FEW_KERNEL(c3, 3, false, true) JL_MX_FEW_KERNEL(c4, 4, false, true)
 JL_MX_FEW_KERNEL(planes_t1, 1, true, false) JL_MX_FEW_KERNEL(planes_t2, 2, true, false)
 JL_MX_FEW_KERNEL(planes_t3, 3, true, false) JL_MX_FEW_KERNEL(planes_t4, 4, true, false)
 JL_MX_FEW_KERNEL(planes_c3, 3, true, true) JL_MX_FEW_KERNEL(planes_c4, 4, true, true)
+// the same in one launch: kernel grid = (ceil(nrows / (16 RT)), chunks of 16 NT tokens), block = 512, dynamic LDS = JL_MX_ONE_LDS(k, NT)
+#define JL_MX_ONE_KERNEL(NT, RT)                                                                                                                       \
+    extern "C" __global__ __launch_bounds__(512) void jl_mxfp4_one_t##NT##r##RT(MxGemmArgs p) { mx_one_body<NT, RT, false>(p, jl_smem); }               \
+    extern "C" __global__ __launch_bounds__(512) void jl_mxfp4_one_planes_t##NT##r##RT(MxGemmArgs p) { mx_one_body<NT, RT, true>(p, jl_smem); }
+JL_MX_ONE_KERNEL(1, 1) JL_MX_ONE_KERNEL(2, 1) JL_MX_ONE_KERNEL(3, 1) JL_MX_ONE_KERNEL(4, 1)
+JL_MX_ONE_KERNEL(1, 2) JL_MX_ONE_KERNEL(2, 2) JL_MX_ONE_KERNEL(3, 2) JL_MX_ONE_KERNEL(4, 2)
 
 // A Q4_K weight is d * sc * q - dmin * m with sc, m <= 63 and q <= 15: a super-block whose
 // |d| * 945 + |dmin| * 63 passes the largest f16 cannot be folded (a NaN or infinite scale

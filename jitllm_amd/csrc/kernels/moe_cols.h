@@ -75,16 +75,6 @@ __device__ __forceinline__ void moe_cols_prep_body(const MoeColsPrepArgs& args) 
     }
 }
 
-// sixteen bytes a lane from a uniform base plus a 32-bit lane offset into LDS at `to` + 16 * lane
-__device__ __forceinline__ void mc_load_lds(const uint8_t* base, u32 off, u32 to) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(base) : "memory", "m0");
-}
-__device__ __forceinline__ void mc_load_lds4(const uint8_t* base, u32 off, u32 to) {   // four bytes a lane
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(to), "v"(off), "s"(base) : "memory", "m0");
-}
-template <int N> __device__ __forceinline__ void mc_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-__device__ __forceinline__ u32 lds_address(const void* q) { return (u32)(uintptr_t)(const __attribute__((address_space(3))) void*)q; }
-
 // Bytes b0 and b1 of w, integers up to 63, as a pair of f16: (1024 + n) by its bits, then m * n + a in one exact step.
 __device__ __forceinline__ f16x2 mc_pair(u32 w, int b0, int b1, f16x2 m, f16x2 a) {
     const u32 v = __builtin_amdgcn_perm(0x64646464u, w, 0x04000400u | (u32)b0 | ((u32)b1 << 16));
@@ -162,15 +152,15 @@ __device__ __forceinline__ void moe_cols_q4_tile(const MoeColsArgs& p, uint8_t* 
         const uint8_t* base = p.rec + (size_t)h * 256;
         const u32 to = lds0 + (h & 1) * JL_MC_A + 1024 * NA * wave;
 #pragma unroll
-        for (int i = 0; i < NA; i++) mc_load_lds(base, aoff[i], __builtin_amdgcn_readfirstlane(to + 1024 * i));
+        for (int i = 0; i < NA; i++) load_lds16(base, aoff[i], __builtin_amdgcn_readfirstlane(to + 1024 * i));
     };
     auto load_w = [&](int sb) __attribute__((always_inline)) {
         const uint8_t* base = sheet + (size_t)sb * 144;
         const u32 to = lds0 + O_W + (sb & 1) * JL_MC_W + 4096 * wave;
 #pragma unroll
-        for (int i = 0; i < 4; i++) mc_load_lds(base, woff[i], __builtin_amdgcn_readfirstlane(to + 1024 * i));
-        mc_load_lds(xbase + (size_t)sb * xstep, xoff, __builtin_amdgcn_readfirstlane(lds0 + xto + (sb & 1) * xpar));
-        if (wave == 0) mc_load_lds4((const uint8_t*)p.da + (size_t)sb * 4, doff, __builtin_amdgcn_readfirstlane(lds0 + O_DA + (sb & 1) * 256));
+        for (int i = 0; i < 4; i++) load_lds16(base, woff[i], __builtin_amdgcn_readfirstlane(to + 1024 * i));
+        load_lds16(xbase + (size_t)sb * xstep, xoff, __builtin_amdgcn_readfirstlane(lds0 + xto + (sb & 1) * xpar));
+        if (wave == 0) load_lds4((const uint8_t*)p.da + (size_t)sb * 4, doff, __builtin_amdgcn_readfirstlane(lds0 + O_DA + (sb & 1) * 256));
     };
     load_a(0);
     load_w(0);
@@ -196,9 +186,9 @@ __device__ __forceinline__ void moe_cols_q4_tile(const MoeColsArgs& p, uint8_t* 
         for (int hf = 0; hf < 2; hf++) {
             // This half's columns, and with the first half the super-block's weights, have arrived everywhere; the place of
             // the half before is free.  (The requests behind them that may be out: the next super-block's weights.)
-            if (hf == 0 || !more) mc_wait<0>();
-            else if (wave == 0) mc_wait<NS + 1>();
-            else mc_wait<NS>();
+            if (hf == 0 || !more) wait_loads<0>();
+            else if (wave == 0) wait_loads<NS + 1>();
+            else wait_loads<NS>();
             lds_barrier();
             if (hf == 0 || more) load_a(2 * sb + hf + 1);
             if (hf == 0 && more) load_w(sb + 1);
@@ -326,7 +316,7 @@ __device__ __forceinline__ void moe_cols_q6_tile(const MoeColsArgs& p, uint8_t* 
         const uint8_t* base = p.rec + (size_t)sb * 256;
         const u32 to = lds0 + (sb & 1) * A_SB + 1024 * NA * wave;
 #pragma unroll
-        for (int i = 0; i < NA; i++) mc_load_lds(base, aoff[i], __builtin_amdgcn_readfirstlane(to + 1024 * i));
+        for (int i = 0; i < NA; i++) load_lds16(base, aoff[i], __builtin_amdgcn_readfirstlane(to + 1024 * i));
     };
     load_a(0);
     load_w(0);
@@ -338,7 +328,7 @@ __device__ __forceinline__ void moe_cols_q6_tile(const MoeColsArgs& p, uint8_t* 
     const u32 place = (u32)l32 * 256 + 16 * ((8 * kg) ^ (l32 & 15));
     const i32x16 zero = {0};
     for (int sb = 0; sb < nsb; sb++) {
-        mc_wait<0>();    // this super-block's columns (in LDS) and weights (in registers) are here
+        wait_loads<0>();    // this super-block's columns (in LDS) and weights (in registers) are here
         lds_barrier();   // ... everywhere, and the one before has been used
         put_w();
         if (sb + 1 < nsb) load_a(sb + 1);
@@ -408,7 +398,7 @@ __device__ __forceinline__ void moe_cols_q6_tile(const MoeColsArgs& p, uint8_t* 
         __builtin_amdgcn_sched_barrier(0);
     }
     mc_store<G>(p, out, mat, r0 + 32 * wave + l32, kg, c0, n);
-    mc_wait<0>();
+    wait_loads<0>();
     lds_barrier();   // LDS is free for the next columns
 }
 
@@ -455,7 +445,7 @@ __device__ __forceinline__ void moe_cols_planes_tile(const MoeColsArgs& p, uint8
         const uint8_t* base = p.rec + (size_t)sb * REC;
         const u32 to = lds0 + (sb & 1) * BUF + 8 * G * REC * wave;
 #pragma unroll
-        for (int i = 0; i < NI; i++) mc_load_lds(base, voff[i], __builtin_amdgcn_readfirstlane(to + 1024 * i));
+        for (int i = 0; i < NI; i++) load_lds16(base, voff[i], __builtin_amdgcn_readfirstlane(to + 1024 * i));
     };
     // block sums (thread = column tid / 4, eight bytes) and scales (thread = column), through registers
     const u32 arec = (u32)__shfl((int)crec, 16 * wave + (lane >> 2), 64);

@@ -1008,3 +1008,164 @@ __device__ __forceinline__ void mx_few_body(const MxGemmArgs& args, float* part)
         }
     }
 }
+
+// ---------------------------------------------------------------- few tokens, one launch
+// The same tiles without a prep: the activations reach LDS as they lie, by loads that write LDS directly, and what is
+// rearranged is the weights' nibbles, of which a step has eight a lane.  A wavefront takes groups of four blocks (128 of K)
+// of its own; a group's activations are 256 bytes a token, sixteen pieces of sixteen bytes, piece P of token t at place
+// P ^ t % 16, so that a step's reads (one piece of sixteen tokens) spread over the banks.  Step c of a group: lane (token or
+// row r = lane % 16, kq = lane / 16) supplies elements 8 c .. 8 c + 7 of block 4 G + kq, one piece of the activations and,
+// of the weights, the low (c < 2) or high nibbles of code words 2 (c % 2) and 2 (c % 2) + 1.
+//
+// What bounds it: the trips -- weights and the first groups' activations, asked for together, then NBUF groups a trip -- and
+// the activations, of which every workgroup brings all to its CU (2880 x 2880, 64 tokens: 369 KB, 2.4 us of L1's 64 bytes a
+// cycle).
+//
+// grid = (ceil(nrows / (16 RT)), token chunks of 16 NT), block = 512, dynamic LDS = JL_MX_ONE_LDS(k, NT); p.x as the caller
+// has it (sixteen-byte aligned).
+template <int NT, int RT, bool PL>
+__device__ __forceinline__ void mx_one_body(const MxGemmArgs& args, uint8_t* smem) {
+    MxGemmArgs p = args;
+    if constexpr (PL) {
+        JL_NOW(p.out, p.x, p.qs, p.d, p.nrows, p.k, p.ntok, p.row0, p.stride);
+        p.qs = as_global(p.qs); p.d = as_global(p.d);
+    } else {
+        JL_NOW(p.out, p.x, p.w, p.nrows, p.k, p.ntok, p.row_bytes);
+        p.w = as_global(p.w);
+    }
+    p.out = as_global(p.out);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, kq = lane >> 4;
+    int rtile = blockIdx.x;
+    if (PL && (gridDim.x & 7) == 0) rtile = (rtile & 7) * (int)(gridDim.x >> 3) + (rtile >> 3);
+    const int r0 = rtile * 16 * RT, t0 = blockIdx.y * 16 * NT;
+    const int nblk = p.k / 32, ngroups = (nblk + 3) / 4, mine_bytes = 4096 * JL_MX_ONE_SLOTS(p.k, NT);
+    const u32 mine = (u32)(wave * mine_bytes);
+    const u32 lds0 = lds_address(smem) + mine;
+    const size_t pst = (size_t)p.stride, dst = (pst + 3) / 4;
+    const uint8_t* wrow[RT];
+    u32 prow[RT];
+#pragma unroll
+    for (int j = 0; j < RT; j++) {
+        const int row = min(r0 + 16 * j + r16, p.nrows - 1);
+        wrow[j] = PL ? nullptr : p.w + (size_t)row * p.row_bytes;
+        prow[j] = (u32)(p.row0 + row);
+    }
+    // activations: four tokens an instruction (past the last: the last again)
+    u32 xrow[4 * NT];
+#pragma unroll
+    for (int n = 0; n < 4 * NT; n++) xrow[n] = (u32)min(t0 + 4 * n + (lane >> 4), p.ntok - 1) * (u32)(2 * p.k);
+    auto load_x = [&](int G, int t, u32 slot) __attribute__((always_inline)) {   // token tile t of group G
+#pragma unroll
+        for (int n = 0; n < 4; n++) {
+            const u32 piece = (u32)((lane & 15) ^ (4 * n + (lane >> 4)));
+            load_lds16((const uint8_t*)p.x, xrow[4 * t + n] + min(256 * (u32)G + 16 * piece, (u32)(2 * p.k - 16)),
+                       __builtin_amdgcn_readfirstlane(lds0 + slot + 1024 * n));
+        }
+    };
+    struct W { u32x4 q; u32 e; };
+    auto load_w = [&](int G, int j, W& w) __attribute__((always_inline)) {
+        const int b = min(4 * G + kq, nblk - 1);
+        if constexpr (PL) {
+            const u32* q = p.qs + (size_t)b * 4 * pst + prow[j];
+            w.q = u32x4{q[0], q[pst], q[2 * pst], q[3 * pst]};
+            w.e = p.d[(size_t)b * dst + (prow[j] >> 2)];   // four rows' exponents: taken apart where they are used
+        } else {
+            const uint8_t* blk = wrow[j] + (size_t)b * 17;
+            w.e = blk[0];
+            w.q = ld16_a1(blk + 1);
+        }
+    };
+    f32x4 out[RT][NT];
+#pragma unroll
+    for (int j = 0; j < RT; j++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) out[j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint8_t* A = smem + mine + 256 * r16;
+    u32 place[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) place[c] = 16 * (u32)((4 * kq + c) ^ r16);
+
+    // four of the wavefront's groups (all of K = 4096) have their weights asked for together
+    for (int G0 = wave; G0 < ngroups; G0 += 32) {
+        const int nunit = min(4, (ngroups - G0 + 7) / 8) * NT;   // units of a token tile of a group, four on their way
+        W w[4][RT];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (G0 + 8 * i < ngroups)
+#pragma unroll
+                for (int j = 0; j < RT; j++) load_w(G0 + 8 * i, j, w[i][j]);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (u < nunit) load_x(G0 + 8 * (u / NT), u % NT, 4096 * u);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int G = G0 + 8 * i;
+            if (G >= ngroups) break;   // uniform
+            const bool past = 4 * G + kq >= nblk;
+            u32x4 wv[RT][4];
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                const int u = i * NT + t;
+                if (u + 3 < nunit) wait_loads<12>();   // (uniform)
+                else if (u + 2 < nunit) wait_loads<8>();
+                else if (u + 1 < nunit) wait_loads<4>();
+                else wait_loads<0>();
+                bf16x8 af[4];
+#pragma unroll
+                for (int c = 0; c < 4; c++) af[c] = *(const bf16x8*)(A + 4096 * (u & 3) + place[c]);
+                if (t == 0) {
+#pragma unroll
+                    for (int j = 0; j < RT; j++) {
+                        const float scale = mx_scale(PL ? (uint8_t)(((w[i][j].e >> (8 * (prow[j] & 3))) & 0xFF) + 1) : (uint8_t)w[i][j].e);
+#pragma unroll
+                        for (int c = 0; c < 4; c++)
+#pragma unroll
+                            for (int h = 0; h < 2; h++) {
+                                const u32 q = past ? 0u : w[i][j].q[2 * (c & 1) + h];
+                                const u32 nib = (c < 2 ? q : q >> 4) & 0x0F0F0F0Fu, pr = nib | (nib >> 4);   // bytes 0, 2: elements (0, 1), (2, 3)
+                                wv[j][c][2 * h] = __builtin_bit_cast(u32, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(pr, scale, 0));
+                                wv[j][c][2 * h + 1] = __builtin_bit_cast(u32, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(pr, scale, 2));
+                            }
+                    }
+                }
+                if (4 * G + 4 > nblk) {   // uniform: K ends inside the group
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+                        if (past) af[c] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the fragments are in registers: their place is free
+                if (u + 4 < nunit) load_x(G0 + 8 * ((u + 4) / NT), (u + 4) % NT, 4096 * (u & 3));
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+#pragma unroll
+                    for (int j = 0; j < RT; j++)
+                        out[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[c], __builtin_bit_cast(bf16x8, wv[j][c]), out[j][t], 0, 0, 0);
+            }
+        }
+    }
+
+    // the eight K shares, added in wavefront order; part [tile][lane] of four floats in each wavefront's own place
+    f32x4* pv = (f32x4*)(smem + mine);
+#pragma unroll
+    for (int j = 0; j < RT; j++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) pv[(j * NT + t) * 64 + lane] = out[j][t];
+    __syncthreads();
+    for (int o = tid; o < RT * NT * 64; o += 512) {
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < 8; w++) {
+            const f32x4 v = *(const f32x4*)(smem + w * mine_bytes + 16 * o);
+            s = f32x4{s.x + v.x, s.y + v.y, s.z + v.z, s.w + v.w};
+        }
+        const int jt = o >> 6, l = o & 63, r = r0 + 16 * (jt / NT) + (l & 15);
+        if (r < p.nrows) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int tok = t0 + 16 * (jt % NT) + 4 * (l >> 4) + i;
+                if (tok < p.ntok) p.out[(size_t)tok * p.nrows + r] = s[i];
+            }
+        }
+    }
+}

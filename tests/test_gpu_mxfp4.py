@@ -311,6 +311,46 @@ def test_mxfp4_few_tokens_one_chunk_and_several(dev, devbuf, packed):
         dev.set_tuning(mxfp4__few=0, mxfp4__few_min=0)
 
 
+@pytest.mark.parametrize("k", [32, 160, 1024, 1184, 4128], ids=str)
+@pytest.mark.parametrize("packed", [False, True], ids=["rows", "planes"])
+def test_mxfp4_few_tokens_in_one_launch(dev, devbuf, packed, k):
+    """The form that takes the activations as they lie: one and two row tiles a workgroup, every count of token tiles, rows and
+    tokens that fill no tile, K that ends inside a group of four blocks and K of more than a wavefront's four groups.  The
+    last token holds an infinity in its last block: it reaches that token's sums alone, as in the plain product."""
+    from jitllm_amd.device import Packed
+    t, pad = quant.MXFP4, 3
+    for nrows, ntok in ((1, 2), (15, 16), (16, 17), (33, 48), (50, 64), (37, 65), (64, 200)):
+        w = synth.quantized_weights(t, nrows + 2 * pad, k, seed=5)
+        wd = oracle.dequant(t, w, (nrows + 2 * pad) * k).reshape(-1, k)[pad:pad + nrows].astype(np.float64)
+        x = np.stack([synth.activations(k, seed=900 + i) for i in range(ntok)])
+        x[-1, k - 5] = np.inf
+        xb, xf = to_bf16(x)
+        dw, dx = devbuf(w), devbuf(xb)
+        nq, nd, _ = dev.packed_words(t, nrows + 2 * pad, k)
+        qs, d = devbuf(shape=(nq,), dtype=np.uint32), devbuf(shape=(nd,), dtype=np.uint32)
+        assert dev.pack_weights_dev(t, dw.ptr, nrows + 2 * pad, k, qs.ptr, d.ptr, None)
+        with np.errstate(invalid="ignore"):
+            want = xf.astype(np.float64) @ wd.T
+        for form in (11, 12):
+            out = devbuf(shape=(ntok * nrows + 8,), dtype=np.float32, fill=np.float32(2e30))
+            dev.set_tuning(mxfp4__one=form)
+            try:
+                n0 = dev.launch_count()
+                if packed:
+                    assert dev.matmul_mxfp4_packed_bf16_dev(out.ptr, Packed(qs.ptr, d.ptr, None, pad, nrows + 2 * pad), dx.ptr, nrows, k, ntok)
+                else:
+                    assert dev.matmul_mxfp4_bf16_dev(out.ptr, dw.ptr + pad * (k // 32) * 17, dx.ptr, nrows, k, ntok)
+                dev.synchronize()
+                assert dev.launch_count() - n0 == 1
+            finally:
+                dev.set_tuning(mxfp4__one=0)
+            got = out.get()
+            assert np.all(got[ntok * nrows:] == np.float32(2e30))
+            got = got[:ntok * nrows].reshape(ntok, nrows)
+            assert nmse(got[:-1], want[:-1]) <= 1e-10, (nrows, ntok, form)
+            assert np.array_equal(got[-1].astype(np.float64), want[-1], equal_nan=True), (nrows, ntok, form)
+
+
 # ------------------------------------------------------------------ block-scaled form (opt-in)
 def mx_fp8_activations(xf):
     """The opt-in form's activation quantizer restated in numpy: per token and block of 32 a
