@@ -1145,7 +1145,7 @@ __device__ __forceinline__ void mx_one_body(const MxGemmArgs& args, uint8_t* sme
         }
     }
 
-    // the eight K shares, added in wavefront order; part [tile][lane] of four floats in each wavefront's own place
+    // the eight K shares, added by pairs; part [tile][lane] of four floats in each wavefront's own place
     f32x4* pv = (f32x4*)(smem + mine);
 #pragma unroll
     for (int j = 0; j < RT; j++)
@@ -1153,12 +1153,14 @@ __device__ __forceinline__ void mx_one_body(const MxGemmArgs& args, uint8_t* sme
         for (int t = 0; t < NT; t++) pv[(j * NT + t) * 64 + lane] = out[j][t];
     __syncthreads();
     for (int o = tid; o < RT * NT * 64; o += 512) {
-        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        f32x4 v[8];
 #pragma unroll
-        for (int w = 0; w < 8; w++) {
-            const f32x4 v = *(const f32x4*)(smem + w * mine_bytes + 16 * o);
-            s = f32x4{s.x + v.x, s.y + v.y, s.z + v.z, s.w + v.w};
-        }
+        for (int w = 0; w < 8; w++) v[w] = *(const f32x4*)(smem + w * mine_bytes + 16 * o);
+#pragma unroll
+        for (int h = 1; h < 8; h *= 2)
+#pragma unroll
+            for (int w = 0; w < 8; w += 2 * h) v[w] = f32x4{v[w].x + v[w + h].x, v[w].y + v[w + h].y, v[w].z + v[w + h].z, v[w].w + v[w + h].w};
+        const f32x4 s = v[0];
         const int jt = o >> 6, l = o & 63, r = r0 + 16 * (jt / NT) + (l & 15);
         if (r < p.nrows) {
 #pragma unroll
