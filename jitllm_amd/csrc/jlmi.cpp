@@ -58,6 +58,7 @@ struct Tuning {
     int mx_planes = 0;          // packed MXFP4: 2 restores rows first; 64 / 32 / 16 rows a workgroup of the plane
                                 // matvec; rows and planes: 3 / 4 the tiles of 64 / 96 rows
     int mx_split = 0;
+    int gemm_tall = 0;   // Q8_0, 256 tokens x 128 rows: 1 no tiles of 64 rows, 2 + n those behind n of 128
     int mx_few = 0, mx_few_min = 0;   // MXFP4: the few-token form up to / from this many tokens
     int mx_one = 0;                   // ... in one launch: 1 never, 11 / 12 wherever it can be, that many row tiles a workgroup
 };
@@ -915,7 +916,7 @@ size_t gemm_i8_acts(int type, int ntok, int k) {   // bytes of the activations' 
     return (size_t)(k / 128) * (tok_pad / 32) * 4096 + (type == JL_TYPE_Q4_K ? 2 : 1) * (size_t)(k / 32) * tok_pad * 4;
 }
 // The tile and the slices of K of a launch, and what the tiles should take.
-struct I8Plan { I8Shape f; int nsplit; double us; };
+struct I8Plan { I8Shape f; int nsplit; double us; int tall; };
 I8Plan gemm_i8_plan(const jl_ctx* c, int type, int nrows, int k, int ntok) {
     const bool q6 = type == JL_TYPE_Q6_K, q4 = type == JL_TYPE_Q4_K;
     const int nstage = k / 128;
@@ -936,7 +937,7 @@ I8Plan gemm_i8_plan(const jl_ctx* c, int type, int nrows, int k, int ntok) {
     const Shape one = {2, 4, 2, q4 ? 0.106 : c->act_window == 32 ? 0.160 : 0.097, q4 ? 0.165 : c->act_window == 32 ? 0.241 : 0.131};
     const bool q8 = type == JL_TYPE_Q8_0;
     I8Shape f = {2, 4};
-    int nsplit = 1;
+    int nsplit = 1, tall = 1 << 24;
     double best = 1e30;
     // Slabs as far as the static array has room for them behind the activations, in every call, so that a call that may
     // not allocate is served where one without slices fits, with the slices of the call that may (without that bound one
@@ -959,10 +960,18 @@ I8Plan gemm_i8_plan(const jl_ctx* c, int type, int nrows, int k, int ntok) {
             double us = full * (0.15 + h.many * waves * cap * block);
             if (left) us += 0.15 + std::max(h.many * waves * ((left + c->num_cu - 1) / c->num_cu), h.alone) * block;
             if (s > 1) us += 0.25 + 1.16e-6 * (s + 1) * n;
-            if (us < best) { best = us; f = {rt, h.tw}; nsplit = s; }
+            // 256 tokens x 128 rows: a last round of at most half of the CUs gives its rows to tiles of 64 instead, which take 0.59 of a
+            // tile's time and fill it (2048 tokens of 14336 x 4096, 3.5 rounds: 334 -> 322)
+            int high = 1 << 24;
+            if (h.tw == 8 && s == 1 && full && left && c->tune.gemm_tall != 1) {
+                const long ttiles = (ntok + 255) / 256, tall_n = full * c->num_cu / ttiles, low = ((nrows - 128 * tall_n + 63) / 64) * ttiles;
+                const double mixed = full * (0.15 + h.many * waves * block) + 0.15 + 0.59 * h.many * waves * block;
+                if (low <= c->num_cu && mixed < us) us = mixed, high = (int)tall_n;
+            }
+            if (us < best) { best = us; f = {rt, h.tw}; nsplit = s; tall = high; }
         }
     }
-    return {f, nsplit, best};
+    return {f, nsplit, best, c->tune.gemm_tall > 1 ? c->tune.gemm_tall - 2 : tall};
 }
 
 int gemm_i8_launch(jl_ctx* c, float* out, int type, const void* w, const float* x, int nrows, int k, int ntok, hipStream_t st) {
@@ -995,7 +1004,12 @@ int gemm_i8_launch(jl_ctx* c, float* out, int type, const void* w, const float* 
         if (rc != JL_OK) return rc;
         ga.out = (float*)c->mx_ws; ga.sb_per = per * unit;
     }
-    rc = launch(c, gemm_i8_name("jl_gemm", c, type, f), (unsigned)((ntok + tt - 1) / tt), (unsigned)((nrows + tr - 1) / tr), 64u * f.tw,
+    int rtiles = (nrows + tr - 1) / tr;
+    if (f.tw == 8 && plan.tall < rtiles) {
+        ga.tall = plan.tall;
+        rtiles = plan.tall + (nrows - 128 * plan.tall + 63) / 64;
+    }
+    rc = launch(c, gemm_i8_name("jl_gemm", c, type, f), (unsigned)((ntok + tt - 1) / tt), (unsigned)rtiles, 64u * f.tw,
                 gemm_i8_lds(c, type, f), st, gp, (unsigned)nsplit);
     if (rc != JL_OK || nsplit == 1) return rc;
     SumPartsArgs sa;
@@ -2357,6 +2371,7 @@ int jl_set_tuning(jl_ctx* c, const char* key, int value) {
     else if (!strcmp(key, "mxfp4.split")) c->tune.mx_split = value;
     else if (!strcmp(key, "mxfp4.few")) c->tune.mx_few = value;
     else if (!strcmp(key, "mxfp4.few_min")) c->tune.mx_few_min = value;
+    else if (!strcmp(key, "gemm.tall")) c->tune.gemm_tall = value;
     else if (!strcmp(key, "mxfp4.one")) c->tune.mx_one = value;
     else if (!strcmp(key, "mxfp4.rows")) c->tune.mx_rows = value;
     else if (!strcmp(key, "mxfp4.planes")) c->tune.mx_planes = value;

@@ -85,6 +85,7 @@ struct GemmArgs {
     int out_stride;      // floats between tokens in out
     int sb_per;          // K split: super-blocks per blockIdx.z (0 = whole K), out = slab z of [gridDim.z][ntok][out_stride]
     const float* dsum = nullptr;   // window 32, Q4_K: the prep's d_a * block sums
+    int tall = 1 << 24;   // Q8_0, 256 tokens x 128 rows: row tiles of 128, those behind them are of 64
     // the weights as packed planes (the kernels' plane forms; w is unused then): QS, D and SC
     // planes of a buffer of pstride rows, this launch's first row at prow0 (nrows counted from
     // it), its first super-block psb0 (a K split moves it)

@@ -147,7 +147,10 @@ __device__ __forceinline__ float gemm_i8_one(const GemmArgs& p, const uint8_t* r
 template <int TYPE, bool W256, int RT, int TW>
 __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, int t0, int r0) {
     constexpr bool Q6 = TYPE == JL_Q6_K, Q4 = TYPE == JL_Q4_K;
-    constexpr int NPL = Q6 ? 2 : 1, NW = TW > 4 ? TW : 4, ROWS = 32 * RT * (NW / TW), NB = ROWS / (16 * NW);
+    constexpr int NPL = Q6 ? 2 : 1, NW = TW > 4 ? TW : 4, ROWS = 32 * RT * (NW / TW);
+    constexpr bool HALVES = ROWS < 16 * NW;   // fewer blocks than threads: two threads a block of 32, sixteen bytes each
+    constexpr int NB = HALVES ? 1 : ROWS / (16 * NW);
+    static_assert(!HALVES || TYPE == JL_Q8_0, "two threads a block: Q8_0");
     constexpr int BUF = JL_GEMM_I8_BUF_BYTES(NPL, ROWS, TW, !W256, Q4), O_D = NPL * ROWS * 128, O_DA = O_D + ROWS * 16,
                   O_M = O_DA + 4 * 32 * TW * 4, O_DS = O_M + ROWS * 16;
     // One operand, window 32: the sums start at the bits of M = 1.5 * 2^23, so that what comes out of the matrix core IS the float
@@ -160,10 +163,10 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
     const int arow = lane & 31, kg = lane >> 5;
     const int nsteps = p.k / 128;
     // this thread's share of a weight stage: block (run) qb of rows tid / 4 + 64 i
-    const int qb = tid & 3;
+    const int qb = HALVES ? (tid >> 1) & 3 : tid & 3, myrow = HALVES ? tid >> 3 : tid >> 2;
     const uint8_t* wrow[NB];
 #pragma unroll
-    for (int i = 0; i < NB; i++) wrow[i] = p.w + (size_t)min(r0 + (tid >> 2) + 16 * NW * i, p.nrows - 1) * p.row_bytes;
+    for (int i = 0; i < NB; i++) wrow[i] = p.w + (size_t)min(r0 + myrow + 16 * NW * i, p.nrows - 1) * p.row_bytes;
     GemmI8Raw<TYPE> raw[NB];
     float rda[2] = {0.f, 0.f}, rds[2] = {0.f, 0.f};
     auto load_w = [&](int step, int i) __attribute__((always_inline)) {
@@ -187,8 +190,8 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
         } else {
             const uint8_t* blk = wrow[i] + (size_t)(4 * step + qb) * 34;
             r.d = ld2(blk);
-            r.q[0] = ld16_a2(blk + 2);
-            r.q[1] = ld16_a2(blk + 18);
+            r.q[0] = ld16_a2(blk + 2 + (HALVES ? 16 * (tid & 1) : 0));
+            if constexpr (!HALVES) r.q[1] = ld16_a2(blk + 18);
         }
     };
     // window 32: the stage's token scales, 4 blocks x 32 TW tokens
@@ -204,8 +207,8 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
     // Half h of the thread's block of row set i of stage `step`, as operand bytes in `buf`; with h = 0 its scales.
     auto slice = [&](uint8_t* buf, int step, int i, int h) __attribute__((always_inline)) {
         const GemmI8Raw<TYPE>& r = raw[i];
-        const int row = (tid >> 2) + 16 * NW * i;
-        uint8_t* dst = buf + row * 128 + 16 * ((2 * qb + h) ^ (row & 7));
+        const int row = myrow + 16 * NW * i;
+        uint8_t* dst = buf + row * 128 + 16 * ((2 * qb + (HALVES ? tid & 1 : h)) ^ (row & 7));
         float *sD = (float*)(buf + O_D) + row * 4 + qb, *sM = (float*)(buf + O_M) + row * 4 + qb;
         if constexpr (Q6) {
             const int nsh = 4 * (qb >> 1), hsh = (2 * qb - 4) & 31;
@@ -255,6 +258,9 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
         if constexpr (NB == 2) {
             slice(buf, step, b >> 1, b & 1);
             if (b & 1) load_w(step + 1, b >> 1);
+        } else if constexpr (HALVES) {
+            if (b == 0) slice(buf, step, 0, 0);   // (both of a block's threads store its scale)
+            if (b == 0) load_w(step + 1, 0);
         } else {
             if (b < 2) slice(buf, step, 0, b);
             if (b == 1) load_w(step + 1, 0);
@@ -363,7 +369,7 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
         }
         // Three wavefronts a SIMD (Q8_0, two row tiles): a tile's scaling right behind its own matrix instruction, whose latency the
         // other wavefronts fill; a second accumulator would be spilled.
-        constexpr bool ONE = MAGIC && !Q4 && RT == 2;
+        constexpr bool ONE = MAGIC && !Q4 && RT == 2 && TW == 4;
         i32x16 acc[ONE ? 1 : 2][NPL];
         f32x4 dav[4], dsv[4];
         float pd = 0.f, pm = 0.f, pc = 0.f;   // the row scales of the tile whose sums wait in the other accumulator; -M * pd

@@ -297,7 +297,9 @@ JL_GEMM_I8_SHAPES(q8_0, JL_Q8_0, false, 3) JL_GEMM_I8_SHAPES(q4k, JL_Q4_K, false
 JL_GEMM_I8_SHAPES(q6kw, JL_Q6_K, true, 2)
 extern "C" __global__ __launch_bounds__(512) void jl_gemm_i8_q8_0_r4t8(GemmArgs p) {
     gemm_i8_split_slice<JL_Q8_0, false>(p);
-    gemm_i8_body<JL_Q8_0, false, 4, 8>(p, jl_smem, blockIdx.x * 256, blockIdx.y * 128);
+    const int y = blockIdx.y;
+    if (y < p.tall) gemm_i8_body<JL_Q8_0, false, 4, 8>(p, jl_smem, blockIdx.x * 256, y * 128);
+    else gemm_i8_body<JL_Q8_0, false, 2, 8>(p, jl_smem, blockIdx.x * 256, 64 * (y + p.tall));   // (128 tall + 64 (y - tall))
 }
 JL_GEMM_I8_DENSE(q8_0, JL_Q8_0, false, 4, 4, 2) JL_GEMM_I8_MOE(q8_0, JL_Q8_0, false, 4, 4, 2)
 extern "C" __global__ __launch_bounds__(512) void jl_gemm_q4k_r128(GemmArgs p) {

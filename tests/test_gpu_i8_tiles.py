@@ -78,6 +78,35 @@ def test_tiles_per_expert(dev, devbuf, t, window, nrows, k):
         dev.SetActWindow(32)
 
 
+@pytest.mark.parametrize("nrows,k,ntok", [(1, 256, 256), (65, 640, 255), (191, 128, 513), (300, 1280, 257)])
+def test_tiles_of_64_rows_behind_those_of_128(dev, devbuf, nrows, k, ntok):
+    """Q8_0, 256 tokens: none, some and all of the rows in tiles of 64 rows (two threads a block of weights); a row whose scale
+    is infinite among them.  Every value is the tile of 128 rows' bit for bit."""
+    dev.SetActWindow(32)
+    w = synth.random_weights(quant.Q8_0, nrows, k, seed=nrows + k)
+    w.reshape(nrows, -1)[-1, 34:36] = (0x00, 0x7C)   # an infinite scale in the last row's second block
+    x = np.stack([synth.activations(k, seed=900 + i) * np.float32(1 + i % 3) for i in range(ntok)])
+    wd, xd = devbuf(w), devbuf(x)
+    want = oracle.matmul_q8act_f64(quant.Q8_0, w, x, nrows, k, ntok, 32)
+    try:
+        ref = None
+        for tall in [1] + [2 + n for n in range((nrows + 127) // 128 + 1)]:
+            dev.set_tuning(gemm__i8=3, gemm__split=1, gemm__tall=tall)
+            o = devbuf(shape=(ntok * nrows + 8,), dtype=np.float32, fill=FILL)
+            assert dev.matmul_dev(o.ptr, quant.Q8_0, wd.ptr, xd.ptr, nrows, k, ntok)
+            dev.synchronize()
+            got = o.get()
+            assert np.all(got[ntok * nrows:] == FILL)
+            got = got[:ntok * nrows].reshape(ntok, nrows)
+            ref = got if ref is None else ref
+            assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), tall
+        if nrows > 1:
+            assert nmse(ref[:, :-1], want[:, :-1]) <= 1e-10
+        assert np.all(np.isinf(ref[:, -1]) | np.isnan(ref[:, -1]))
+    finally:
+        dev.set_tuning(gemm__i8=0, gemm__split=0, gemm__tall=0)
+
+
 @pytest.mark.parametrize("nrows,k,ntok", [(1, 128, 257), (127, 640, 255), (129, 512, 513), (300, 1280, 256)])
 def test_tiles_of_256_tokens(dev, devbuf, nrows, k, ntok):
     """Q8_0, 256 tokens x 128 rows on eight wavefronts: one token past a tile and one short of it, a wavefront and more without a
