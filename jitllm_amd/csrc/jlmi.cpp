@@ -2188,7 +2188,7 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     if (e != hipSuccess)
         return bail(JL_ERR_HIP, "hipModuleLoad(" + path + "): " + H->GetErrorString(e));
 
-    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e8", "jl_moe_logits_e8_f16", "jl_moe_group", "jl_moe_group2", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_few_planes_t1", "jl_mxfp4_few_planes_t2", "jl_mxfp4_few_planes_t3", "jl_mxfp4_few_planes_t4", "jl_mxfp4_few_c3", "jl_mxfp4_few_c4", "jl_mxfp4_few_planes_c3", "jl_mxfp4_few_planes_c4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_planes_gemm_r96", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_silu_mul", "jl_add_rows", "jl_host_in", "jl_host_done", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
+    std::vector<std::string> names = {"jl_quantize_act", "jl_dequant", "jl_matvec_q4k_r1_pq", "jl_matvec_q4k_r1_pq_res", "jl_matvec_q8_0_r1_pq", "jl_matvec_q8_0_r1_pq_res", "jl_matvec_q6k_r1_pq", "jl_matvec_q6k_r1_pq_res", "jl_matvec_q8_0p_r1_pq", "jl_matvec_q8_0p_r1_pq_res", "jl_matvec_q4k_r1_res", "jl_matvec_q4k_r1_x4_res", "jl_matvec_q8_0_r1_res", "jl_matvec_q8_0_r1_x4_res", "jl_matvec_q6k_r1_res", "jl_matvec_q6k_r1_x4_res", "jl_matvec_q8_0p_r1_res", "jl_matvec_q8_0p_r1_x4_res", "jl_matvec_q8_0p_r1", "jl_matvec_q8_0p_r2", "jl_matvec_q8_0p_r4", "jl_gemm_prep_q4k", "jl_gemm_prep_q4k_w16", "jl_gemm_q4k_r64", "jl_gemm_q4k_r128", "jl_gemm_q4k_wide", "jl_gemm_prep_q4k_fold", "jl_gemm_q4k_fold_wide", "jl_gemm_q4k_fold_wide4", "jl_gemm_q4k_k2", "jl_gemm_q4k_k2_planes", "jl_gemm_prep_q4k_planes", "jl_gemm_q4k_r64_planes", "jl_gemm_q4k_wide_planes", "jl_gemm_w16_prep_q4k", "jl_gemm_q4k_w16", "jl_gemm_q4k_few32", "jl_moe_route", "jl_moe_route_g2", "jl_moe_route_g4", "jl_moe_logits", "jl_moe_logits_e2", "jl_moe_logits_e2_f16", "jl_moe_logits_e4", "jl_moe_logits_e4_f16", "jl_moe_logits_e8", "jl_moe_logits_e8_f16", "jl_moe_group", "jl_moe_group2", "jl_moe_quant", "jl_moe_matvec_planes_q4k", "jl_moe_combine", "jl_moe_worklist", "jl_moe_gemm_prep", "jl_moe_gemm_prep_planes", "jl_moe_gemm_q4k", "jl_moe_g16_prep", "jl_moe_g16_prep_planes", "jl_moe_g16_c1", "jl_moe_g16_c2", "jl_moe_g16_c3", "jl_moe_g16_f1", "jl_moe_g16_f2", "jl_moe_g16_f3", "jl_moe_g16_g1", "jl_moe_g16_g2", "jl_moe_g16_g3", "jl_moe_g16_d1", "jl_moe_g16_d2", "jl_moe_g16_d3", "jl_moe_g16p_c1", "jl_moe_g16p_c2", "jl_moe_g16p_c3", "jl_moe_g16p_f1", "jl_moe_g16p_f2", "jl_moe_g16p_f3", "jl_moe_g16p_g1", "jl_moe_g16p_g2", "jl_moe_g16p_g3", "jl_moe_g16p_d1", "jl_moe_g16p_d2", "jl_moe_g16p_d3", "jl_moe_gemm_r64", "jl_moe_gemm_r64_planes", "jl_mxfp4_prep", "jl_mxfp4_prep_few", "jl_mxfp4_few_t1", "jl_mxfp4_few_t2", "jl_mxfp4_few_t3", "jl_mxfp4_few_t4", "jl_mxfp4_few_planes_t1", "jl_mxfp4_few_planes_t2", "jl_mxfp4_few_planes_t3", "jl_mxfp4_few_planes_t4", "jl_mxfp4_few_c3", "jl_mxfp4_few_c4", "jl_mxfp4_few_planes_c3", "jl_mxfp4_few_planes_c4", "jl_mxfp4_gemm", "jl_mxfp4_gemm_r96", "jl_mxfp4_matvec", "jl_mxfp4_matvec1_b1", "jl_mxfp4_matvec1_b2", "jl_mxfp4_matvec1_b3", "jl_mxfp4_scaled_prep", "jl_mxfp4_scaled_gemm", "jl_mxfp4_planes_prep", "jl_mxfp4_planes_gemm", "jl_mxfp4_planes_gemm_r96", "jl_mxfp4_matvec_planes_r64", "jl_mxfp4_matvec_planes_r32", "jl_mxfp4_matvec_planes_r16", "jl_unpack_mxfp4", "jl_sum_parts", "jl_silu_mul", "jl_add_rows", "jl_host_in", "jl_host_done", "jl_q4k_fold_range", "jl_probe_read", "jl_probe_empty", "jl_probe_wait", "jl_probe_mfma", "jl_probe_mfma_v5",
                                       "jl_pack_weights", "jl_unpack_q4k", "jl_unpack_q6k", "jl_unpack_q8_0"};
     names.push_back("jl_few_prep");
     for (const char* pl : {"", "planes_"})
@@ -2727,15 +2727,23 @@ int jl_moe_logits_dev(jl_ctx* c, float* logits, int wtype, const void* w, const 
     a.w = w; a.x = x; a.logits = logits; a.n_expert = n_expert; a.k = k; a.ntok = ntok;
     a.f16 = wtype == JL_TYPE_F16;
     void* params[] = {&a};
-    // eight expert rows a workgroup once that still gives every CU a workgroup (us, a row a workgroup / eight; 128 experts
-    // x 2048: 128 tokens 9.1 / 9.0, 256 14.1 / 9.6, 2048 88 / 34; 32 x 2048: 512 tokens 8.9 / 9.0; 64 x 2880: 192 tokens
-    // 8.5 / 11.4, 256 12.3 / 11.4; tuning "moe.logits" = 1 / 8 forces a form)
-    const long blocked = (long)((n_expert + 7) / 8) * ((ntok + 7) / 8);
-    if (c->tune.moe_logits == 8 || (c->tune.moe_logits == 0 && blocked >= c->num_cu))
-        return launch(c, a.f16 ? "jl_moe_logits_e8_f16" : "jl_moe_logits_e8", (unsigned)((n_expert + 7) / 8), (unsigned)((ntok + 7) / 8), 128, 0,
-                      pick_stream(c, stream), params);
-    return launch(c, "jl_moe_logits", (unsigned)n_expert, (unsigned)((ntok + 7) / 8), 128, 0,   // JL_LOGITS_TOK
-                  pick_stream(c, stream), params);
+    // Expert rows a workgroup takes: more of them meet an x value loaded once, fewer are more workgroups, whose wavefronts hide each
+    // other's dependent adds.  us by 1 / 2 / 4 / 8 rows, x from memory: 128 experts x 2048, 64 tokens 5.3 / 6.0 / 6.7 / 9.4, 128 9.2 /
+    // 6.4 / 7.2 / 9.6, 256 13.6 / 9.0 / 7.7 / 10.3, 512 22 / 14.6 / 11.7 / 11.6, 1024 47 / 31 / 23 / 18.9; 64 x 2048, 512 tokens 14.5 /
+    // 10.1 / 7.7 / 10.3; 87 x 1024, 1024 tokens 29 / 12.3 / 9.5 / 10.0; 16 x 2816, 1024 tokens 18.6 / 10.8 / 11.5 / 14.1.  Tuning
+    // "moe.logits" = 1 / 2 / 4 / 8 forces a form.
+    int eb = c->tune.moe_logits;
+    if (eb != 1 && eb != 2 && eb != 4 && eb != 8) {
+        const auto a_cu = [&](int e) { return (double)((n_expert + e - 1) / e) * ((ntok + 7) / 8) / c->num_cu; };
+        eb = a_cu(1) <= 4 ? 1 : a_cu(2) <= 5 ? 2 : a_cu(4) <= std::max(5.75, 11776.0 / k) ? 4 : 8;
+    }
+    const unsigned gx = (unsigned)std::min(8, (ntok + 7) / 8);   // token groups side by side
+    if (eb > 1) {
+        Name name;
+        name << "jl_moe_logits_e" << eb << (a.f16 ? "_f16" : "");
+        return launch(c, name, gx, (unsigned)((n_expert + eb - 1) / eb), 128, 0, pick_stream(c, stream), params, (unsigned)((ntok + 63) / 64));
+    }
+    return launch(c, "jl_moe_logits", gx, (unsigned)n_expert, 128, 0, pick_stream(c, stream), params, (unsigned)((ntok + 63) / 64));   // JL_LOGITS_TOK
 }
 
 namespace {

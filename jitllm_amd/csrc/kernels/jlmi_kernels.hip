@@ -347,20 +347,19 @@ extern "C" __global__ __launch_bounds__(256, 2) void jl_gemm_q4k_w16(GemmW16Args
 extern "C" __global__ __launch_bounds__(64) void jl_moe_route(MoeRouteArgs p) { moe_route_body<16>(p); }
 extern "C" __global__ __launch_bounds__(64) void jl_moe_route_g2(MoeRouteArgs p) { moe_route_body<2>(p); }
 extern "C" __global__ __launch_bounds__(64) void jl_moe_route_g4(MoeRouteArgs p) { moe_route_body<4>(p); }
-// grid = (experts, ceil(tokens / JL_LOGITS_TOK)), block = 128
+// grid = (token groups, 8 at most, experts, ceil(token groups / 8)), block = 128; a group is JL_LOGITS_TOK tokens
 extern "C" __global__ __launch_bounds__(128) void jl_moe_logits(MoeLogitsArgs p) {
     __shared__ float part[JL_LOGITS_TOK * 128];
     moe_logits_body<1>(p, part);
 }
-// many tokens: grid = (ceil(experts / 8), ceil(tokens / JL_LOGITS_TOK)), block = 128
-extern "C" __global__ __launch_bounds__(128, 4) void jl_moe_logits_e8(MoeLogitsArgs p) {
-    __shared__ float part[2 * JL_LOGITS_TOK * 128];
-    moe_logits_body<8>(p, part);
-}
-extern "C" __global__ __launch_bounds__(128, 4) void jl_moe_logits_e8_f16(MoeLogitsArgs p) {
-    __shared__ float part[2 * JL_LOGITS_TOK * 128];
-    moe_logits_body<8, true>(p, part);
-}
+// more tokens: grid = (..., ceil(experts / EB), ...)
+#define JL_MOE_LOGITS(NAME, EB, F16)                                                        \
+    extern "C" __global__ __launch_bounds__(128, 4) void jl_moe_logits_##NAME(MoeLogitsArgs p) {  \
+        __shared__ float part[2 * JL_LOGITS_TOK * 128];                                     \
+        moe_logits_body<EB, F16>(p, part);                                                  \
+    }
+JL_MOE_LOGITS(e2, 2, false) JL_MOE_LOGITS(e2_f16, 2, true) JL_MOE_LOGITS(e4, 4, false) JL_MOE_LOGITS(e4_f16, 4, true)
+JL_MOE_LOGITS(e8, 8, false) JL_MOE_LOGITS(e8_f16, 8, true)
 // one workgroup of 1024 threads (n_expert <= 1024)
 extern "C" __global__ __launch_bounds__(1024) void jl_moe_group(MoeGroupArgs p) {
     __shared__ u32 scount[2048];

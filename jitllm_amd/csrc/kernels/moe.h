@@ -1569,7 +1569,9 @@ __device__ __forceinline__ void moe_gather_down_body(const MoeGatherDownArgs& ar
 #define JL_LOGITS_TOK 8
 template <int EB, bool F16 = false>
 __device__ __forceinline__ void moe_logits_body(const MoeLogitsArgs& p, float* part) {
-    const int r0 = blockIdx.x * EB, t0 = blockIdx.y * JL_LOGITS_TOK, tid = threadIdx.x;
+    // (workgroups go round the eight XCDs in the order of their ids: a token group's rows of x are fetched into one L2)
+    const int r0 = blockIdx.y * EB, t0 = (blockIdx.x + 8 * blockIdx.z) * JL_LOGITS_TOK, tid = threadIdx.x;
+    if (t0 >= p.ntok) return;   // uniform
     const int nt = min(JL_LOGITS_TOK, p.ntok - t0), k = p.k;
     float acc[EB][JL_LOGITS_TOK];
 #pragma unroll
@@ -1600,17 +1602,18 @@ __device__ __forceinline__ void moe_logits_body(const MoeLogitsArgs& p, float* p
         for (int i0 = 0; i0 < kfull; i0 += 128) trip(i0, GemmIntC<0>{});
         if (kfull < k) trip(kfull, GemmIntC<1>{});
     } else {
-        // Every row's base in scalar registers and one lane offset for all sixteen loads of a trip, the next trip's
-        // loads on their way while this one's 64 products are added: two vector instructions a product and nothing
-        // beside them (the clamped form with a select a product: 24.9 us at 777 tokens x 128 experts x 2048, this 16.8).
+        // Every row's base in scalar registers and one lane offset for all sixteen loads of a trip: two vector instructions a
+        // product and nothing beside them.  The next trip's loads are on their way while this one's products are added, the
+        // two sets of registers in turn (copied from one to the other 128 experts x 2048, 1024 tokens took 21.7 us, 20.9 so; three sets
+        // 20.6, but 1024 wide 13.6 against 13.3).
         const float* xp[JL_LOGITS_TOK];
         const char* wp[EB];
-        constexpr int es = F16 ? 2 : 4;
+        constexpr int es = F16 ? 2 : 4, NS = 2;
 #pragma unroll
         for (int t = 0; t < JL_LOGITS_TOK; t++) xp[t] = p.x + (size_t)(t0 + min(t, nt - 1)) * k;
 #pragma unroll
         for (int e = 0; e < EB; e++) wp[e] = (const char*)p.w + (size_t)min(r0 + e, p.n_expert - 1) * k * es;
-        float w[EB], xv[JL_LOGITS_TOK], wn[EB], xn[JL_LOGITS_TOK];
+        float w[NS][EB], xv[NS][JL_LOGITS_TOK];
         const int trips = (k + 127) >> 7;
         auto load = [&](float (&a)[EB], float (&b)[JL_LOGITS_TOK], int trip) __attribute__((always_inline)) {
             const u32 i = (u32)min(128 * trip + tid, k - 1);
@@ -1622,32 +1625,32 @@ __device__ __forceinline__ void moe_logits_body(const MoeLogitsArgs& p, float* p
 #pragma unroll
             for (int t = 0; t < JL_LOGITS_TOK; t++) b[t] = *(const float*)((const char*)xp[t] + 4 * i);
         };
-        load(w, xv, 0);
-        for (int trip = 0; trip + 1 < trips; trip++) {
-            load(wn, xn, trip + 1);
-            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int e = 0; e < EB; e++) {
+        for (int u = 0; u + 1 < NS; u++) load(w[u], xv[u], u);
+        for (int trip = 0; trip < trips; trip += NS) {
 #pragma unroll
-                for (int t = 0; t < JL_LOGITS_TOK; t++) {
-                    const float prod = w[e] * xv[t];
-                    acc[e][t] = acc[e][t] + prod;
+            for (int u = 0; u < NS; u++) {
+                if (trip + u >= trips) break;   // uniform
+                load(w[(u + NS - 1) % NS], xv[(u + NS - 1) % NS], trip + u + NS - 1);
+                __builtin_amdgcn_sched_barrier(0);
+                if (128 * (trip + u) + 128 > k) {   // uniform: in the ragged last trip a lane past the row's end adds +0
+                    const bool in = 128 * (trip + u) + tid < k;
+#pragma unroll
+                    for (int e = 0; e < EB; e++) w[u][e] = in ? w[u][e] : 0.f;
+#pragma unroll
+                    for (int t = 0; t < JL_LOGITS_TOK; t++) xv[u][t] = in ? xv[u][t] : 0.f;
                 }
-                __builtin_amdgcn_sched_barrier(0);   // (products not formed far ahead of their sums, in registers of their own)
+#pragma unroll
+                for (int e = 0; e < EB; e++) {
+#pragma unroll
+                    for (int t = 0; t < JL_LOGITS_TOK; t++) {
+                        const float prod = w[u][e] * xv[u][t];
+                        acc[e][t] = acc[e][t] + prod;
+                    }
+                    __builtin_amdgcn_sched_barrier(0);   // (products not formed far ahead of their sums, in registers of their own)
+                }
             }
-#pragma unroll
-            for (int e = 0; e < EB; e++) w[e] = wn[e];
-#pragma unroll
-            for (int t = 0; t < JL_LOGITS_TOK; t++) xv[t] = xn[t];
         }
-        const bool in = 128 * (trips - 1) + tid < k;   // in the ragged last trip a lane past the row's end adds +0
-#pragma unroll
-        for (int e = 0; e < EB; e++)
-#pragma unroll
-            for (int t = 0; t < JL_LOGITS_TOK; t++) {
-                const float prod = w[e] * xv[t];
-                acc[e][t] = acc[e][t] + (in ? prod : 0.f);
-            }
     }
     // The tree, one token per 16 lanes: lane j of a token's row takes the partial sums the
     // tree would bring to thread j by s = 16 (levels 64, 32, 16: seven adds in tree order),

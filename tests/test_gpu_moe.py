@@ -512,6 +512,30 @@ def test_router_logits_bit_exact_then_route(dev, devbuf, case, form):
     dev.set_tuning(moe__logits=0)
 
 
+@pytest.mark.parametrize("form", [2, 4])
+@pytest.mark.parametrize("case", [(1, 1, 4, "f32"), (9, 5, 130, "f32"), (17, 7, 384, "f16"), (65, 66, 1000, "f32"), (8, 3, 255, "f16")],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_router_logits_by_two_and_four_rows(dev, devbuf, case, form):
+    """Two and four expert rows a workgroup: experts and tokens that fill no group, K below, off and of a number of trips both
+    even and odd; the oracle's bits, as of the other forms."""
+    ntok, n_expert, k, wdt = case
+    rng = np.random.default_rng(ntok * 7 + n_expert)
+    w = rng.standard_normal((n_expert, k)).astype(np.float32) * np.float32(0.05)
+    x = rng.standard_normal((ntok, k)).astype(np.float32)
+    w = w.astype(np.float16).view(np.uint16) if wdt == "f16" else w
+    want = oracle.router_logits(w, x, n_expert, k, ntok)
+    ld = devbuf(shape=(ntok * n_expert + 3,), dtype=np.float32, fill=np.float32(7e30))
+    dev.set_tuning(moe__logits=form)
+    try:
+        assert dev.moe_logits_dev(ld.ptr, 1 if wdt == "f16" else 0, devbuf(w).ptr, devbuf(x).ptr, n_expert, k, ntok)
+        dev.synchronize()
+    finally:
+        dev.set_tuning(moe__logits=0)
+    got = ld.get()
+    assert np.all(got[ntok * n_expert:] == np.float32(7e30))
+    assert np.array_equal(got[:ntok * n_expert].view(np.uint32), np.ascontiguousarray(want).reshape(-1).view(np.uint32))
+
+
 def _pack_bank(dev, devbuf, t, bank, n_expert, nrows, k, layout):
     """A GGUF bank -> packed planes on the device.  layout "sheets": every expert's sheet packed
     on its own, plane sets `page` bytes apart as a container's expert pages are
