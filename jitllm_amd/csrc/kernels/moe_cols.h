@@ -115,8 +115,27 @@ __device__ __forceinline__ void mc_store(const MoeColsArgs& p, const f32x16 (&ou
 
 // Q4_K rows.  G: groups of 32 columns (n columns exist).  The rows' bytes come to LDS as they lie, 144 contiguous bytes a
 // row (straight into registers, a lane a row, is sixteen bytes of 64 lines an instruction), and each wavefront reads its own.
+struct MoeColsQ4Rows { u32 woff[4], xoff; };   // a lane's places among the rows' bytes
+__device__ __forceinline__ void moe_cols_q4_rows(const MoeColsArgs& p, uint8_t* smem, const uint8_t* sheet, int last, MoeColsQ4Rows& w) {
+    constexpr int O_W = 2 * JL_MC_A;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const u32 lds0 = lds_address(smem);
+    // 18 instructions of 64 pieces, nine pieces a row; four a wavefront, the last two the first two wavefronts'
+    auto piece_at = [&](int i) {
+        const int idx = 64 * i + lane, row = idx / 9;
+        return (u32)min(row, last) * (u32)p.row_bytes + 16 * (u32)(idx - 9 * row);
+    };
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        w.woff[i] = piece_at(4 * wave + i);
+        load_lds16(sheet, w.woff[i], __builtin_amdgcn_readfirstlane(lds0 + O_W + 4096 * wave + 1024 * i));
+    }
+    w.xoff = piece_at(16 + (wave & 1));
+    if (wave < 2) load_lds16(sheet, w.xoff, __builtin_amdgcn_readfirstlane(lds0 + O_W + 1024 * (16 + wave)));
+}
+// w: the places, and the first super-block's rows already asked for
 template <int G>
-__device__ __forceinline__ void moe_cols_q4_tile(const MoeColsArgs& p, uint8_t* smem, int e, int mat, int r0, u32 c0, int n) {
+__device__ __forceinline__ void moe_cols_q4_tile(const MoeColsArgs& p, uint8_t* smem, const uint8_t* sheet, const MoeColsQ4Rows& w, int mat, int r0, u32 c0, int n) {
     constexpr int O_W = 2 * JL_MC_A, O_AUG = O_W + 2 * JL_MC_W, O_DA = O_AUG + 2 * 64 * 32;
     constexpr int NA = 2 * G;   // a wavefront's instructions for half a super-block of columns; NS: for its weights, sums, scales
     constexpr int NS = 5;
@@ -124,21 +143,14 @@ __device__ __forceinline__ void moe_cols_q4_tile(const MoeColsArgs& p, uint8_t* 
     const int l32 = lane & 31, kg = lane >> 5, nsb = p.k / 256;
     const u32 lds0 = lds_address(smem);
     const u32 crec = p.map ? p.map[c0 + min(lane, n - 1)] : c0 + min(lane, n - 1);
-    const uint8_t* sheet = p.bank[mat] + (size_t)e * p.sheet_bytes + (size_t)r0 * p.row_bytes;
-    const int last = p.nrows - 1 - r0;
-    // weights: 18 instructions of 64 pieces, nine pieces a row; four a wavefront, the last two the first two wavefronts'
-    auto piece_at = [&](int i) {
-        const int idx = 64 * i + lane, row = idx / 9;
-        return (u32)min(row, last) * (u32)p.row_bytes + 16 * (u32)(idx - 9 * row);
-    };
-    u32 woff[4], xoff;
+    u32 woff[4], xoff = w.xoff;
 #pragma unroll
-    for (int i = 0; i < 4; i++) woff[i] = piece_at(4 * wave + i);
+    for (int i = 0; i < 4; i++) woff[i] = w.woff[i];
     // the fifth: weights, or 32 columns' sums (wavefronts 2, 3); and wavefront 0 brings the scales
     const uint8_t* xbase = wave < 2 ? sheet : p.aug;
     const u32 xstep = wave < 2 ? 144 : 32, xto = wave < 2 ? O_W + 1024 * (16 + wave) : O_AUG + 1024 * (wave & 1), xpar = wave < 2 ? JL_MC_W : 64 * 32;
     const u32 srec = (u32)__shfl((int)crec, 32 * (wave & 1) + (lane >> 1), 64);
-    xoff = wave < 2 ? piece_at(16 + wave) : srec * (u32)(nsb * 32) + 16 * (lane & 1);
+    if (wave >= 2) xoff = srec * (u32)(nsb * 32) + 16 * (lane & 1);
     // columns: four an instruction, sixteen pieces each; piece P of column c lies at place P ^ c % 16, so that a fragment's
     // reads spread over the banks
     u32 aoff[NA];
@@ -154,16 +166,17 @@ __device__ __forceinline__ void moe_cols_q4_tile(const MoeColsArgs& p, uint8_t* 
 #pragma unroll
         for (int i = 0; i < NA; i++) load_lds16(base, aoff[i], __builtin_amdgcn_readfirstlane(to + 1024 * i));
     };
-    auto load_w = [&](int sb) __attribute__((always_inline)) {
+    auto load_w = [&](int sb, auto ROWS) __attribute__((always_inline)) {
         const uint8_t* base = sheet + (size_t)sb * 144;
         const u32 to = lds0 + O_W + (sb & 1) * JL_MC_W + 4096 * wave;
+        if constexpr (decltype(ROWS)::value != 0)
 #pragma unroll
-        for (int i = 0; i < 4; i++) load_lds16(base, woff[i], __builtin_amdgcn_readfirstlane(to + 1024 * i));
-        load_lds16(xbase + (size_t)sb * xstep, xoff, __builtin_amdgcn_readfirstlane(lds0 + xto + (sb & 1) * xpar));
+            for (int i = 0; i < 4; i++) load_lds16(base, woff[i], __builtin_amdgcn_readfirstlane(to + 1024 * i));
+        if (decltype(ROWS)::value != 0 || wave >= 2) load_lds16(xbase + (size_t)sb * xstep, xoff, __builtin_amdgcn_readfirstlane(lds0 + xto + (sb & 1) * xpar));
         if (wave == 0) load_lds4((const uint8_t*)p.da + (size_t)sb * 4, doff, __builtin_amdgcn_readfirstlane(lds0 + O_DA + (sb & 1) * 256));
     };
     load_a(0);
-    load_w(0);
+    load_w(0, GemmIntC<0>{});
     f32x16 out[G], acc[G];
     const f32x16 zero = {0.f};
 #pragma unroll
@@ -191,7 +204,7 @@ __device__ __forceinline__ void moe_cols_q4_tile(const MoeColsArgs& p, uint8_t* 
             else wait_loads<NS>();
             lds_barrier();
             if (hf == 0 || more) load_a(2 * sb + hf + 1);
-            if (hf == 0 && more) load_w(sb + 1);
+            if (hf == 0 && more) load_w(sb + 1, GemmIntC<1>{});
             const uint8_t* A = smem + hf * JL_MC_A;
             if (hf == 0) {
                 hd = *(const u32x4*)W;
@@ -572,18 +585,25 @@ __device__ __forceinline__ void moe_cols_body(const MoeColsArgs& p, uint8_t* sme
     const u32 per_xcd = gridDim.x >> 3, item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (item >= (u32)p.items) return;
     const u32 z = item % (u32)p.shares, i1 = item / (u32)p.shares, rb = i1 % (u32)p.rblocks, i2 = i1 / (u32)p.rblocks;
-    const int mat = (int)(i2 % (u32)p.nmat), e = (int)(i2 / (u32)p.nmat);
-    const u32 c_hi = p.start[e + 1];
-    for (u32 c0 = p.start[e] + 64 * z; c0 < c_hi; c0 += 64 * (u32)p.shares) {   // uniform
+    const int mat = __builtin_amdgcn_readfirstlane((int)(i2 % (u32)p.nmat)), e = __builtin_amdgcn_readfirstlane((int)(i2 / (u32)p.nmat));
+    const int r0 = __builtin_amdgcn_readfirstlane((int)rb * 128);
+    // Which columns are the expert's takes two trips to memory (start, then the records' numbers): the rows' bytes, which do not
+    // depend on it, are asked for first.
+    const uint8_t* sheet = p.bank[mat] + (size_t)e * p.sheet_bytes + (size_t)r0 * p.row_bytes;
+    MoeColsQ4Rows w4;
+    if constexpr (KO == 0) moe_cols_q4_rows(p, smem, sheet, p.nrows - 1 - r0, w4);
+    const u32 c_hi = p.start[e + 1], c_lo = p.start[e] + 64 * z;
+    for (u32 c0 = c_lo; c0 < c_hi; c0 += 64 * (u32)p.shares) {   // uniform
         const int n = (int)min(64u, c_hi - c0);
-        const int r0 = (int)rb * 128;
+        if (KO == 0 && c0 != c_lo) moe_cols_q4_rows(p, smem, sheet, p.nrows - 1 - r0, w4);
         auto tile = [&](auto G) __attribute__((always_inline)) {
             constexpr int g = decltype(G)::value;
-            if constexpr (KO == 0) moe_cols_q4_tile<g>(p, smem, e, mat, r0, c0, n);
+            if constexpr (KO == 0) moe_cols_q4_tile<g>(p, smem, sheet, w4, mat, r0, c0, n);
             else if constexpr (KO == 1) moe_cols_planes_tile<g>(p, smem, e, mat, r0, c0, n);
             else moe_cols_q6_tile<g>(p, smem, e, mat, r0, c0, n);
         };
         if (n > 32) tile(GemmIntC<2>{});
         else tile(GemmIntC<1>{});
     }
+    if constexpr (KO == 0) wait_loads<0>();   // (no columns: LDS is written until the rows have come)
 }
