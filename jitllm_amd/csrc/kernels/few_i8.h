@@ -235,10 +235,21 @@ template <int TYPE, bool W256> struct FewA {
 // (Scaled after each half, d P rounded first, and the wavefronts' sums added one after the other: NMSE against 64 bits at K = 4096
 // 8.8e-15 for Q4_K, so 6.5e-15, the tiles 7.5e-15; Q6_K 5.3e-15, so 3.9e-15, the tiles 4.8e-15.  And half as many scalings: Q4_K
 // 14336 x 4096, 48 tokens 24.4 -> 21.5 us, Q6_K 4096 x 4096, 96 tokens 17.6 -> 16.4.)
+// Q6_K, window 32: the half's four blocks are summed with the tokens' scales alone, and the sum meets the row's scale once: four
+// vector instructions a result and block where each product met both in five.  44 shapes of 2 to 400 tokens 0.967 times as long
+// (5649 x 13824 planes, 35 tokens 49.1 -> 45.2 us, 4663 x 3840 rows, 42 tokens 19.2 -> 18.6), NMSE against 64 bits 4.4e-15 -> 4.1e-15
+// at K = 1024, 6.2e-15 -> 5.2e-15 at 2560.  (Summed over the super-block: 4.9e-15 and 5.9e-15.)
 template <int TYPE, bool PL, int NT, int RT, bool W256, int H>
 __device__ __forceinline__ void few_blocks(const FewR<TYPE, PL>* R, const float* sc, const FewA<TYPE, W256>* X, u32 m0, int g,
                                            i32x4 (*P)[NT], i32x4 (*M)[NT], f32x4 (*acc)[NT]) {
     const i32x4 zero = {0, 0, 0, 0};
+    constexpr bool SUMS = TYPE == JL_Q6_K && !W256;
+    f32x4 sum[RT][NT];
+    if constexpr (SUMS)
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+            for (int t = 0; t < NT; t++) sum[rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     if constexpr (W256 && H == 0)
 #pragma unroll
         for (int rt = 0; rt < RT; rt++)
@@ -256,7 +267,6 @@ __device__ __forceinline__ void few_blocks(const FewR<TYPE, PL>* R, const float*
             if constexpr (TYPE == JL_Q6_K) {
                 const u32x2 b0 = u32x2{b.x & m0, b.y & m0}, b1 = u32x2{b.x & ~m0, b.y & ~m0};
                 const i32x4 s0 = ((const i32x4*)scr)[(2 * s) * 4 + g], s1 = ((const i32x4*)scr)[(2 * s + 1) * 4 + g];
-                const f32x4 d4 = ((const f32x4*)(scr + 128))[g];
 #pragma unroll
                 for (int t = 0; t < NT; t++) {
                     const u32x2 a = X[t].block(s);
@@ -265,7 +275,7 @@ __device__ __forceinline__ void few_blocks(const FewR<TYPE, PL>* R, const float*
                     for (int i = 0; i < 4; i++) {
                         const i32 v = __mul24(y0[i], s0[i]) + __mul24(y1[i], s1[i]);
                         if constexpr (W256) P[rt][t][i] += v;
-                        else acc[rt][t][i] = fmaf((float)v, d4[i] * X[t].da[s], acc[rt][t][i]);
+                        else sum[rt][t][i] = fmaf((float)v, X[t].da[s], sum[rt][t][i]);
                     }
                 }
             } else if constexpr (TYPE == JL_Q4_K && W256) {
@@ -297,12 +307,22 @@ __device__ __forceinline__ void few_blocks(const FewR<TYPE, PL>* R, const float*
 #pragma unroll
             for (int t = 0; t < NT; t++) {
                 if constexpr (W256) asm volatile("" : "+v"(P[rt][t]));
+                else if constexpr (SUMS) asm volatile("" : "+v"(sum[rt][t]));
                 else asm volatile("" : "+v"(acc[rt][t]));
                 if constexpr (W256 && TYPE == JL_Q4_K) asm volatile("" : "+v"(M[rt][t]));
             }
         }
     }
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (SUMS)
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) {
+            const f32x4 d4 = ((const f32x4*)(sc + rt * (JL_FEW_SC_BYTES / 4) + 128))[g];
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[rt][t][i] = fmaf(sum[rt][t][i], d4[i], acc[rt][t][i]);
+        }
     if constexpr (W256 && H == 1)
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
@@ -540,6 +560,43 @@ __device__ __forceinline__ void few_planes_half(int c, const FewPlaneW<TYPE>* W,
 }
 
 // grid = (ceil(nrows / (16 RT)), experts or token groups, matrices), block = 64 * p.nwaves, dynamic LDS: JL_FEW_LDS_BYTES.
+// Q6_K, window 32: result (row r, token tok of a slot) block by block.  A row's scale that is infinite meets the sum of four blocks
+// above; the decode matvec's infinities and NaN are those of its products with the blocks one by one.
+template <bool PL>
+__device__ __forceinline__ float few_q6_one(const FewI8Args& p, const FewMat& m, int e, int r, u32 slot, int tok) {
+    const uint8_t* row = PL ? nullptr : m.w + (size_t)r * p.row_bytes;
+    const size_t n = (size_t)p.pstride, at = (size_t)(p.prow0 + e * p.row_step + r);
+    float o = 0.f;
+#pragma unroll 1
+    for (int b = 0; b < p.k / 32; b++) {
+        const int sb = b >> 3, half = (b >> 2) & 1, s = b & 3;
+        const size_t x = (size_t)(b >> 2) * p.nslots + slot;
+        const u32* a = (const u32*)p.bq + x * 512 + (s >> 1) * 256 + tok * 4 + 2 * (s & 1);
+        const uint8_t* blk = PL ? nullptr : row + (size_t)sb * 210;
+        i32 P = 0;
+#pragma unroll 1
+        for (int l = 0; l < 32; l++) {
+            const int run = l >> 4, i = (l >> 2) & 3, j = l & 3;
+            u32 q;
+            i32 sc;
+            if constexpr (PL) {
+                const u32* w = m.qs + ((size_t)(sb * 16 + half * 8 + 2 * s + run) * 3) * n + at;
+                q = ((w[(i & 1) * n] >> (8 * j + 4 * (i >> 1))) & 15) | (((w[2 * n] >> (8 * j + 2 * i)) & 3) << 4);
+                sc = (i32)((m.sp[((size_t)sb * 4 + 2 * half + (s >> 1)) * n + at] >> (16 * (s & 1) + 8 * run)) & 255) - 128;
+            } else {
+                q = ((blk[64 * half + 32 * (s & 1) + l] >> (4 * (s >> 1))) & 15) | (((blk[128 + 32 * half + l] >> (2 * s)) & 3) << 4);
+                sc = (int8_t)blk[192 + 8 * half + 2 * s + run];
+            }
+            int g, h;
+            jl_few_order(PL ? 2 : 0, l >> 2, g, h);
+            P += sc * ((i32)q - 32) * (int8_t)(a[g * 64 + h] >> (8 * j));
+        }
+        const u32 d = PL ? m.dp[(size_t)sb * n + at] : (u32)ld2(blk + 208);
+        o = fmaf((float)P, half_bits_to_f32((uint16_t)d) * p.da[x * 64 + 4 * tok + s], o);
+    }
+    return o;
+}
+
 template <int TYPE, bool PL, int NT, int RT, bool W256>
 __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem) {
     FewI8Args p;   // the matrix's arguments, asked for at once
@@ -767,6 +824,8 @@ __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem
             for (; q + 4 <= nw; q += 4, at += 4 * W) v += (at[0] + at[W]) + (at[2 * W] + at[3 * W]);
             for (; q < nw; q++, at += W) v += at[0];
             if ((u32)tok < left && r0 + rr < p.nrows) {
+                if constexpr (TYPE == JL_Q6_K && !W256)
+                    if (!__builtin_isfinite(v)) v = few_q6_one<PL>(p, m, e, r0 + rr, slot0 + t0 + (tok >> 4), tok & 15);
                 const size_t o = (size_t)(col0 + t0 * 16 + tok) * p.nrows + r0 + rr;
                 if (p.out[0]) p.out[0][o] = v;
                 if (p.resid) p.resid[o] += v;

@@ -15,8 +15,10 @@
 // three, 53 vector instructions a matrix instruction with everything else, now 37.  Q8_0, 2048 tokens x 4096 -> 14336, tiles of
 // 256 tokens x 128 rows: the vector unit issues 76 % of the time and the matrix instructions take most of the rest, the two do
 // not overlap on a SIMD; L1 0.35 of 0.69 million cycles (0.70 of 0.67 under tiles of 128 tokens, whose weights' narrow loads bound
-// it then): 320 us, 363 before, 460 as f16 operands.  Q6_K, two operands and two matrix instructions a block, 41 vector instructions
-// each, 86 % and 16 %.  Window 256 (551 us as f16 operands, 14336 -> 4096, now 400): 12 vector instructions a matrix instruction, most of
+// it then): 320 us, 363 before, 460 as f16 operands.  Q6_K, two operands and two matrix instructions a block: four
+// vector instructions an output element and block, now three and an eighth (a super-block's sum meets the row's scale once): 14336 x 4096,
+// 2048 tokens 621 -> 568 us, 12957 x 1536, 1138 147 -> 136, NMSE against 64 bits 1.4e-14 -> 4.8e-15 (13183 x 1280, 102 tokens).
+// Window 256 (551 us as f16 operands, 14336 -> 4096, now 400): 12 vector instructions a matrix instruction, most of
 // them the making of Q6_K's two operands, which every workgroup of 128 tokens does anew; vector unit 43 %, matrix cores 27 %, L1
 // 0.66 of 0.85 million cycles.
 //
@@ -120,6 +122,19 @@ __device__ __forceinline__ float gemm_i8_one(const GemmArgs& p, const uint8_t* r
 #pragma unroll 1
     for (int b = 0; b < p.k / 32; b++) {
         const u32x4* f = a + ((size_t)(b >> 2) * (p.tok_pad >> 5) * 4 + (b & 3)) * 64;
+        if constexpr (TYPE == JL_Q6_K) {
+            const uint8_t* blk = row + (size_t)(b >> 3) * 210;
+            const int n = (b >> 2) & 1, g = b & 3;
+            i32 P = 0;
+#pragma unroll 1
+            for (int l = 0; l < 32; l++) {
+                const u32 lo = blk[64 * n + 32 * (g & 1) + l] >> (4 * (g >> 1)), hi = blk[128 + 32 * n + l] >> (2 * g);
+                const int8_t v = (int8_t)((const uint8_t*)(f + 32 * (l >> 4)))[l & 15];
+                P += (int8_t)blk[192 + 8 * n + 2 * g + (l >> 4)] * ((i32)((lo & 15) | ((hi & 3) << 4)) - 32) * v;
+            }
+            o = fmaf((float)P * p.da[(size_t)b * p.tok_pad + t], half_bits_to_f32(ld2(blk + 208)), o);
+            continue;
+        }
         const uint8_t* blk = TYPE == JL_Q4_K ? row + (size_t)(b >> 3) * 144 : row + (size_t)b * 34;
         const uint8_t* q = TYPE == JL_Q4_K ? blk + 16 + 32 * ((b & 7) >> 1) : blk + 2;
         i32 P = 0;
@@ -360,6 +375,86 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
             stage(GemmIntC<0>{}, step);
             stage(GemmIntC<1>{}, step + 1);
         }
+    } else if constexpr (Q6) {
+        // The row's scale holds for a super-block, the token's for a block: the blocks are summed with the token's scale alone, and
+        // the super-block's sum meets the row's once, three vector instructions an element and block (shift and add, conversion,
+        // multiply-add) where a product and a multiply-add with both scales made it four.  (A row with a scale that is infinite
+        // is summed again where it is stored, block by block.)
+        i32x16 acc[2][2];
+        f32x16 sum[RT];
+        f32x4 dav[4];
+        float d[RT];   // the row scales of the super-block that is summed
+#pragma unroll
+        for (int pl = 0; pl < 2; pl++) acc[1][pl] = zero;
+#pragma unroll
+        for (int j = 0; j < RT; j++) {
+            d[j] = 0.f;
+#pragma unroll
+            for (int e = 0; e < 16; e++) sum[j][e] = 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) dav[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // s = (begin: nothing) + y, scaled; move: the block ends, and the token scales of the next take each quarter's place
+        auto scale = [&](bool begin, bool move, const i32x16 (&y)[2], f32x16& s, const float* next) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+#pragma unroll
+                for (int e = 4 * i; e < 4 * i + 4; e++) {
+                    const float v = (float)((y[0][e] << 7) + y[1][e]);
+                    s[e] = begin ? v * dav[i][e & 3] : fmaf(v, dav[i][e & 3], s[e]);
+                }
+                if (move) dav[i] = *(const f32x4*)(next + 8 * i);
+            }
+        };
+        auto fold = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < RT; j++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) out[j][e] = fmaf(sum[j][e], d[j], out[j][e]);
+        };
+        auto stage = [&](auto HALF, int step) __attribute__((always_inline)) {
+            constexpr int half = decltype(HALF)::value;
+            uint8_t *cur = smem + half * BUF, *nxt = smem + (half ^ 1) * BUF;
+            const uint8_t* w0 = cur + (row0 + arow) * 128;
+            const int nstep = min(step + 1, nsteps - 1);
+            i32x4 wf[2][2];
+            auto read_w = [&](int n) __attribute__((always_inline)) {   // tile n = RT * block + row group
+#pragma unroll
+                for (int pl = 0; pl < 2; pl++)
+                    wf[n & 1][pl] = *(const i32x4*)(w0 + (pl * ROWS + 32 * (n % RT)) * 128 + piece[n / RT]);
+            };
+            const float* sDa = (const float*)(cur + O_DA) + 32 * tg + 4 * kg;
+            read_w(0);
+#pragma unroll
+            for (int n = 0; n < 4 * RT; n++) {
+                const int b = n / RT, j = n % RT;
+                if (n + 1 < 4 * RT) read_w(n + 1);
+#pragma unroll
+                for (int pl = 0; pl < 2; pl++)
+                    acc[n & 1][pl] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ring[b], wf[n & 1][pl], zero, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                // the tile before
+                if (j == 0) scale(half == 0 && b == 1, true, acc[1], sum[RT - 1], sDa + b * 32 * TW);
+                else scale(half == 0 && b == 0, false, acc[(n + 1) & 1], sum[j - 1], nullptr);
+                if (half == 0 && n == 0) {   // the super-block before is whole
+                    fold();
+#pragma unroll
+                    for (int i = 0; i < RT; i++) d[i] = ((const float*)(cur + O_D))[(row0 + 32 * i + arow) * 4];
+                }
+                if (j == RT - 1) {
+                    ring[b] = a_frag(nstep, b);
+                    part(nxt, step + 1, b);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            lds_barrier();
+        };
+        for (int step = 0; step < nsteps; step += 2) {
+            stage(GemmIntC<0>{}, step);
+            stage(GemmIntC<1>{}, step + 1);
+        }
+        scale(false, false, acc[1], sum[RT - 1], nullptr);
+        fold();
     } else {
         i32x16 first = {0};
         if constexpr (MAGIC) {
@@ -370,26 +465,24 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
         // Three wavefronts a SIMD (Q8_0, two row tiles): a tile's scaling right behind its own matrix instruction, whose latency the
         // other wavefronts fill; a second accumulator would be spilled.
         constexpr bool ONE = MAGIC && !Q4 && RT == 2 && TW == 4;
-        i32x16 acc[ONE ? 1 : 2][NPL];
+        i32x16 acc[ONE ? 1 : 2];
         f32x4 dav[4], dsv[4];
         float pd = 0.f, pm = 0.f, pc = 0.f;   // the row scales of the tile whose sums wait in the other accumulator; -M * pd
-#pragma unroll
-        for (int pl = 0; pl < NPL; pl++) acc[ONE ? 0 : 1][pl] = zero;
+        acc[ONE ? 0 : 1] = zero;
 #pragma unroll
         for (int i = 0; i < 4; i++) { dav[i] = f32x4{0.f, 0.f, 0.f, 0.f}; dsv[i] = f32x4{0.f, 0.f, 0.f, 0.f}; }
         // o += the sums y, scaled; next: where the token scales of the block behind lie, which take each quarter's
         // place when it has been used (MOVE: the block ends)
-        auto scale = [&](auto MOVE, const i32x16 (&y)[NPL], f32x16& o, const float* next, const float* next_s) __attribute__((always_inline)) {
+        auto scale = [&](auto MOVE, const i32x16& y, f32x16& o, const float* next, const float* next_s) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
 #pragma unroll
                 for (int e = 4 * i; e < 4 * i + 4; e++) {
                     if constexpr (MAGIC) {
-                        const i32 v = y[0][e];   // (a copy: bit_cast of a vector's element takes another element's bits)
+                        const i32 v = y[e];   // (a copy: bit_cast of a vector's element takes another element's bits)
                         o[e] = fmaf(fmaf(__builtin_bit_cast(float, v), pd, pc), dav[i][e & 3], o[e]);
                     } else {
-                        const i32 v = NPL == 2 ? (y[0][e] << 7) + y[NPL - 1][e] : y[0][e];
-                        o[e] = fmaf((float)v * dav[i][e & 3], pd, o[e]);
+                        o[e] = fmaf((float)y[e] * dav[i][e & 3], pd, o[e]);
                     }
                     if constexpr (Q4) o[e] = fmaf(dsv[i][e & 3], pm, o[e]);
                 }
@@ -403,11 +496,9 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
             uint8_t *cur = smem + (step & 1) * BUF, *nxt = smem + ((step + 1) & 1) * BUF;
             const uint8_t* w0 = cur + (row0 + arow) * 128;
             const int nstep = min(step + 1, nsteps - 1);
-            i32x4 wf[2][NPL];
+            i32x4 wf[2];
             auto read_w = [&](int n) __attribute__((always_inline)) {   // tile n = RT * block + row group
-#pragma unroll
-                for (int pl = 0; pl < NPL; pl++)
-                    wf[n & 1][pl] = *(const i32x4*)(w0 + (pl * ROWS + 32 * (n % RT)) * 128 + piece[n / RT]);
+                wf[n & 1] = *(const i32x4*)(w0 + 32 * (n % RT) * 128 + piece[n / RT]);
             };
             const float *sDa = (const float*)(cur + O_DA) + 32 * tg + 4 * kg, *sDs = (const float*)(cur + O_DS) + 32 * tg + 4 * kg;
             read_w(0);
@@ -430,7 +521,7 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
                             if constexpr (Q4) dsv[i] = *(const f32x4*)(sDs + b * 32 * TW + 8 * i);
                         }
                     }
-                    acc[0][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ring[b], wf[n & 1][0], first, 0, 0, 0);
+                    acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ring[b], wf[n & 1], first, 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
                     pd = dd[j][b];
                     pc = -12582912.f * pd;
@@ -444,9 +535,7 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
                     __builtin_amdgcn_sched_barrier(0);
                     continue;
                 }
-#pragma unroll
-                for (int pl = 0; pl < NPL; pl++)
-                    acc[n & 1][pl] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ring[b], wf[n & 1][pl], MAGIC ? first : zero, 0, 0, 0);
+                acc[n & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ring[b], wf[n & 1], MAGIC ? first : zero, 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 // the tile before
                 if (j == 0) scale(GemmIntC<1>{}, acc[1], out[RT - 1], sDa + b * 32 * TW, sDs + b * 32 * TW);
@@ -475,13 +564,13 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
             if (t < p.ntok) p.out[(size_t)t * p.out_stride + r] = out[j][e];
         }
     }
-    // MAGIC: an infinite scale makes a row's every sum NaN, whatever the token.  The decode matvec and the few-token kernel give
-    // the product's infinities there, and NaN where it has none.
-    if constexpr (MAGIC) {
+    // An infinite scale makes a row's every sum NaN (Q6_K: NaN or infinite), whatever the token.  The decode matvec and the few-token
+    // kernel give the product's infinities there, and NaN where it has none.
+    if constexpr (MAGIC || (Q6 && !W256)) {
 #pragma unroll
         for (int j = 0; j < RT; j++) {
             const int r = r0 + row0 + 32 * j + arow;
-            if (r >= p.nrows || !__builtin_isnan(out[j][0])) continue;
+            if (r >= p.nrows || !(MAGIC ? __builtin_isnan(out[j][0]) : !__builtin_isfinite(out[j][0]))) continue;
 #pragma unroll 1
             for (int e = 0; e < 16; e++) {
                 const int t = t0 + 32 * tg + 8 * (e >> 2) + 4 * kg + (e & 3);

@@ -6,6 +6,7 @@ import pytest
 import oracle
 from conftest import nmse
 from jitllm_amd import quant, synth
+from jitllm_amd.device import Packed
 
 pytestmark = pytest.mark.gpu
 FILL = np.float32(4e30)
@@ -176,4 +177,48 @@ def test_scales_that_are_no_numbers(dev, devbuf, t, ntok):
                 check(o, form)
     finally:
         dev.set_tuning(gemm__few=0, gemm__i8=0, gemm__split=0, moe__form=0)
+        dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("planes", [False, True], ids=["rows", "planes"])
+@pytest.mark.parametrize("ntok", [12, 40, 300])   # (fewer may be the matvec's, which sums four sub-scales first: row 77 is infinite there)
+def test_q6_scales_that_are_no_numbers(dev, devbuf, planes, ntok):
+    """Q6_K, window 32, where the row's scale meets sums of blocks: a row whose scale is infinite in a super-block has the infinities and NaN of its blocks' products one by one, in the few-token kernel, the tiles and K slices; the other rows as ever."""
+    nrows, k, window, t = 131, 1536, 32, quant.Q6_K
+    dev.SetActWindow(window)
+    w = synth.random_weights(t, nrows, k, seed=4)
+    x = np.abs(np.stack([synth.activations(k, seed=950 + i) for i in range(ntok)])) + np.float32(0.1)
+    b = w.reshape(nrows, -1, 210)
+    b[:, :, :128] |= 0x11                                   # every weight 33 .. 47 less 32, every sub-scale 1 .. 127: a block's products have one sign
+    b[:, :, 128:192] = 0xAA
+    b[:, :, 192:208] = b[:, :, 192:208] & 0x7F | 1
+    b[:, :, 209] &= 0x7F
+    inf, ninf, nan = (0x00, 0x7C), (0x00, 0xFC), (0x00, 0x7E)
+    b[5, 0, 208:], b[64, 5, 208:], b[127, 2, 208:], b[130, 1, 208:] = inf, ninf, nan, inf
+    b[100, 0, 208:], b[100, 4, 208:] = inf, ninf
+    b[77, 3, 208:] = inf
+    b[77, 3, 192:194] = 0xFF                                # (one block's products below zero, the sum of the super-block's above)
+    want = oracle.matmul_q8act_f64(t, w, x, nrows, k, ntok, window)
+    want[:, [5, 64, 77, 100, 127, 130]] = np.inf, -np.inf, np.nan, np.nan, np.nan, np.inf
+    wd, xd = devbuf(w), devbuf(x)
+    mat = wd.ptr
+    if planes:
+        bufs = [devbuf(shape=(n,), dtype=np.uint32) for n in quant.packed_words(t, nrows, k)]
+        assert dev.pack_weights_dev(t, wd.ptr, nrows, k, *[a.ptr for a in bufs])
+        mat = Packed(*[a.ptr for a in bufs], 0, nrows)
+    try:
+        for few, split in ((0, 0), (1, 0), (2, 0), (2, 2), (2, 3)):
+            dev.set_tuning(gemm__few=few, gemm__split=split)
+            o = devbuf(shape=(ntok * nrows + 8,), dtype=np.float32, fill=FILL)
+            assert (dev.matmul_packed_dev if planes else dev.matmul_dev)(o.ptr, t, mat, xd.ptr, nrows, k, ntok)
+            dev.synchronize()
+            got = o.get()
+            assert np.all(got[ntok * nrows:] == FILL)
+            got = got[:ntok * nrows].reshape(ntok, nrows)
+            assert np.array_equal(np.isnan(got), np.isnan(want)), (few, split)
+            assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want)), (few, split)
+            ok = np.isfinite(want)
+            assert nmse(got[ok], want[ok]) <= 1e-10, (few, split)
+    finally:
+        dev.set_tuning(gemm__few=0, gemm__split=0)
         dev.SetActWindow(32)
