@@ -105,7 +105,7 @@ int jl_synchronize(jl_ctx *ctx);
  * packed-plane matvec: 16, 32, 64), "packed.block" (its threads per workgroup), "moe.shares"
  * (row shares an expert's matrix is split into), "moe.form" (grouped matmul: 10 a decode matvec a column, 1 dot products,
  * 2 / 3 groups of 32 / 16 columns on the matrix cores, 4 the prefill tile per expert, 5 the int8
- * few-token kernel, 6 / 7 / 8 the int8 tiles of 128 columns x 64 rows, 64 x 128 and (Q8_0) 128 x 128,
+ * few-token kernel, 6 / 7 / 8 the int8 tiles of 128 columns x 64 rows, 64 x 128 (Q6_K, window 32) and (Q8_0) 128 x 128,
  * 9 columns against rows decoded in registers; a routed block: 11 a handful of pairs without grouping),
  * "moe.group16" (form 3: 1 a prep kernel quantizes the columns, 2 the matrix kernel does, 3 groups
  * of 32 columns),

@@ -1824,12 +1824,16 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     const size_t sheet = (size_t)nrows * row_bytes;
     // The int8 forms, by columns an expert on average (us of one matrix of 128 experts x 2048 x 768 / 32 x 2048 x 1024 /
     // 16 x 1024 x 2048, what they replace -> them; "moe.form" = 5 forces the few-token kernel, 6, 7, 8 the tiles of 128
-    // columns x 64 rows, 64 x 128 and, Q8_0, 128 x 128):
+    // columns x 64 rows, 64 x 128 (Q6_K, window 32: else as 6) and, Q8_0, 128 x 128):
     //   Q8_0 window 32    1: 39/16/13 -> 36/15/12   8: 90/29/25 -> 53/21/14   32: 235/71/69 -> 92/30/20   128: 853/238/236 -> 170/56/41
     //   Q6_K window 32    1: 32/16/15 -> 39/16/12   8: 98/40/31 -> 62/22/15   32: 308/110/89 -> 114/37/25   128: 1065/403/304 -> 254/86/60
     //   Q6_K window 256   2: 48/20/18 -> 47/19/14   8: 67/27/30 -> 59/21/15   48: 179/47/48 -> 111/38/28    128: 238/81/56 -> 183/61/43
     // The few-token kernel reads an expert's sheet once for 64 columns and the columns once for every row tile, so it
-    // gives way to the tiles where the columns are the more; a tile of 64 columns needs two workgroups a CU.  With a
+    // gives way to the tiles where the columns are the more; a tile of 64 columns needs two workgroups a CU.  From 40 columns on,
+    // window 32, Q8_0 takes tiles of 128 columns, Q6_K of 64, Q4_K from 56 on 128; blocks of 128 experts of 768 x 2048 and 60 of 1280 x 2048,
+    // 42 columns: Q8_0 on tiles of 64 311 and 249, of 128 303 and 242 (54 columns 348, 321), Q6_K down on tiles of 64 356 and 260, of 128 359 and
+    // 284, Q4_K on tiles of 64, whose registers spilled, 1704 and 1391, on the few-token kernel 405 and 324.  (Tiles of 128 columns would take
+    // Q4_K 380 and 283 there, and Q8_0 288 against 318 at 32 columns; their one chain of sums rounds more than what serves them.)  With a
     // column or two an expert Q6_K's dot-product kernel is as fast while rows are short.  Q4_K with the k-quant window
     // has the forms below, and the few-token kernel where moe_few_faster finds it faster.
     {
@@ -1864,7 +1868,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
             else if (q6 && c->act_window == 256 && avg > 8 && avg < 60) form = moe_few_faster(type, n_expert, ncols, nmat, nrows, k) ? 5 : 9;
             else if (q6 && avg < (c->act_window == 32 ? 3 : 2) && k < 2048) form = 0;
             else if (avg < (q6 && c->act_window == 256 ? 28 : 40)) form = 5;
-            else if (avg < (q6 && c->act_window == 32 ? 64 : 56)) form = tiles64 >= 2 * c->num_cu ? 7 : 5;
+            else if (avg < (q6 && c->act_window == 32 ? 64 : 56)) form = tiles64 < 2 * c->num_cu || type == JL_TYPE_Q4_K ? 5 : q6 && c->act_window == 32 ? 7 : 6;
             else form = type == JL_TYPE_Q8_0 && avg >= 64 && tiles64 >= 2 * c->num_cu ? 8 : 6;
         }
         // Planes (gate + up + down of 128 x 768 x 2048 and 32 x 1024 x 2048, the block's us, the forms below against columns):
@@ -1882,7 +1886,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
         }
         if (form >= 6 && !planes && gemm_i8_applies(c, type, nrows, k, ncols)) {
             rc = moe_gemm_i8_launch(c, out0, out1, type, bank0, bank1, x, x2, src, start, n_expert, ncols, nrows, k,
-                                    form == 7 ? I8Shape{2, 2} : form == 8 && type == JL_TYPE_Q8_0 ? I8Shape{4, 4} : I8Shape{2, 4}, st, lists);
+                                    form == 7 && q6 && c->act_window == 32 ? I8Shape{2, 2} : form == 8 && type == JL_TYPE_Q8_0 ? I8Shape{4, 4} : I8Shape{2, 4}, st, lists);
             if (rc != JL_DECLINED) return rc;
         }
         if (form == 5 && align && few_fits(c, type, planes, nrows, k, ncols, planes ? pb0->stride : 0)) {
@@ -2207,11 +2211,12 @@ int jl_ctx_create(jl_ctx** out, const jl_options* opts) {
     for (const char* tag : {"q4k", "q4k_planes", "q6k"})
         for (const char* form : {"jl_moe_cols_", "jl_moe_cols_prep_"}) names.push_back(std::string(form) + tag);
     for (const char* tag : {"q8_0", "q4k", "q6k", "q6kw"})
-        for (const char* form : {"jl_gemm_i8_%s_r2t4", "jl_moe_gemm_i8_%s_r2t4", "jl_moe_gemm_i8_%s_r2t2"}) {
+        for (const char* form : {"jl_gemm_i8_%s_r2t4", "jl_moe_gemm_i8_%s_r2t4"}) {
             char nm[64];
             snprintf(nm, sizeof nm, form, tag);
             names.push_back(nm);
         }
+    names.push_back("jl_moe_gemm_i8_q6k_r2t2");
     names.push_back("jl_gemm_i8_q8_0_r4t4");
     names.push_back("jl_gemm_i8_q8_0_r4t8");
     names.push_back("jl_moe_gemm_i8_q8_0_r4t4");

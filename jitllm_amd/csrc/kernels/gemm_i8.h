@@ -171,9 +171,9 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
     // One operand, window 32: the sums start at the bits of M = 1.5 * 2^23, so that what comes out of the matrix core IS the float
     // M + P (|P| <= 32 * 127 * 128 < 2^22), and P * d = fma(M + P, d, -M d) with -M d exact (d has 17 bits at most): no
     // conversion.  (A row with a scale that is infinite comes out as NaN so: it is summed again where it is stored.)
-    constexpr bool MAGIC = !W256 && NPL == 1 && !(Q4 && TW == 2);   // (that tile has no sixteen registers to spare)
+    constexpr bool MAGIC = !W256 && NPL == 1;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), tg = wave % TW, rg = wave / TW;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), tg = TW < 4 ? wave % TW : wave;
     const bool live = t0 + 32 * tg < p.ntok;                   // else no token of its 32 exists
     const int arow = lane & 31, kg = lane >> 5;
     const int nsteps = p.k / 128;
@@ -313,7 +313,7 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
     i32x4 ring[4];
 #pragma unroll
     for (int b = 0; b < 4; b++) ring[b] = a_frag(0, b);
-    const int row0 = 32 * RT * rg;   // the wavefront's first row of the tile
+    const int row0 = TW < 4 ? 32 * RT * (wave / TW) : 0;   // the wavefront's first row of the tile
     const i32x16 zero = {0};
     int piece[4];   // where the lane's piece of a block lies in its row
 #pragma unroll
@@ -379,9 +379,10 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
         // The row's scale holds for a super-block, the token's for a block: the blocks are summed with the token's scale alone, and
         // the super-block's sum meets the row's once, three vector instructions an element and block (shift and add, conversion,
         // multiply-add) where a product and a multiply-add with both scales made it four.  (A row with a scale that is infinite
-        // is summed again where it is stored, block by block.)
+        // is summed again where it is stored, block by block.)  The tile of 128 rows has no registers for the second set of sums.
+        constexpr bool SUMS = TW >= 4;
         i32x16 acc[2][2];
-        f32x16 sum[RT];
+        f32x16 sum[SUMS ? RT : 1];
         f32x4 dav[4];
         float d[RT];   // the row scales of the super-block that is summed
 #pragma unroll
@@ -390,27 +391,29 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
         for (int j = 0; j < RT; j++) {
             d[j] = 0.f;
 #pragma unroll
-            for (int e = 0; e < 16; e++) sum[j][e] = 0.f;
+            for (int e = 0; e < 16; e++) sum[SUMS ? j : 0][e] = 0.f;
         }
 #pragma unroll
         for (int i = 0; i < 4; i++) dav[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // s = (begin: nothing) + y, scaled; move: the block ends, and the token scales of the next take each quarter's place
-        auto scale = [&](bool begin, bool move, const i32x16 (&y)[2], f32x16& s, const float* next) __attribute__((always_inline)) {
+        // s, row tile j's sums = (begin: nothing) + y, scaled; move: the block ends, and the token scales of the next take each quarter's place
+        auto scale = [&](bool begin, bool move, const i32x16 (&y)[2], int j, const float* next) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
 #pragma unroll
                 for (int e = 4 * i; e < 4 * i + 4; e++) {
                     const float v = (float)((y[0][e] << 7) + y[1][e]);
-                    s[e] = begin ? v * dav[i][e & 3] : fmaf(v, dav[i][e & 3], s[e]);
+                    if constexpr (SUMS) sum[j][e] = begin ? v * dav[i][e & 3] : fmaf(v, dav[i][e & 3], sum[j][e]);
+                    else out[j][e] = fmaf(v * dav[i][e & 3], d[j], out[j][e]);
                 }
                 if (move) dav[i] = *(const f32x4*)(next + 8 * i);
             }
         };
         auto fold = [&]() __attribute__((always_inline)) {
+            if constexpr (!SUMS) return;
 #pragma unroll
             for (int j = 0; j < RT; j++)
 #pragma unroll
-                for (int e = 0; e < 16; e++) out[j][e] = fmaf(sum[j][e], d[j], out[j][e]);
+                for (int e = 0; e < 16; e++) out[j][e] = fmaf(sum[SUMS ? j : 0][e], d[j], out[j][e]);
         };
         auto stage = [&](auto HALF, int step) __attribute__((always_inline)) {
             constexpr int half = decltype(HALF)::value;
@@ -434,8 +437,8 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
                     acc[n & 1][pl] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ring[b], wf[n & 1][pl], zero, 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 // the tile before
-                if (j == 0) scale(half == 0 && b == 1, true, acc[1], sum[RT - 1], sDa + b * 32 * TW);
-                else scale(half == 0 && b == 0, false, acc[(n + 1) & 1], sum[j - 1], nullptr);
+                if (j == 0) scale(half == 0 && b == 1, true, acc[1], RT - 1, sDa + b * 32 * TW);
+                else scale(half == 0 && b == 0, false, acc[(n + 1) & 1], j - 1, nullptr);
                 if (half == 0 && n == 0) {   // the super-block before is whole
                     fold();
 #pragma unroll
@@ -453,7 +456,7 @@ __device__ __forceinline__ void gemm_i8_body(const GemmArgs& p, uint8_t* smem, i
             stage(GemmIntC<0>{}, step);
             stage(GemmIntC<1>{}, step + 1);
         }
-        scale(false, false, acc[1], sum[RT - 1], nullptr);
+        scale(false, false, acc[1], RT - 1, nullptr);
         fold();
     } else {
         i32x16 first = {0};

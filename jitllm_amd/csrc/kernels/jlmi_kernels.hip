@@ -248,7 +248,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void jl_gemm_q4k_r64(GemmArgs p)
 // The int8 form (kernels/gemm_i8.h): prep grid = (ceil(k/256), tok_pad/32), block = 1024; matrix kernel
 // jl_gemm_i8_<type>_<shape>: grid = (token tiles, row tiles, K splits), block = 256, dynamic LDS = JL_GEMM_I8_LDS_BYTES;
 // shape r4t4: 128 tokens x 128 rows (Q8_0: the others have no registers for it), r2t4: 128 x 64.  jl_moe_gemm_i8_...:
-// the same tile per expert, and r2t2: 64 columns x 128 rows.
+// the same tile per expert, and r2t2, Q6_K with the window of 32: 64 columns x 128 rows.
 extern "C" __global__ __launch_bounds__(1024) void jl_gemm_i8_prep(GemmPrepArgs p) {
     __shared__ u32 lds[JL_GEMM_I8_PREP_WORDS];
     gemm_i8_prep_body(p, lds);
@@ -292,9 +292,10 @@ __device__ __forceinline__ void moe_gemm_i8_tiles(const MoeGemmArgs& p) {
         moe_gemm_i8_tiles<TYPE, W256, RT, TW>(p);                                                                  \
     }
 #define JL_GEMM_I8_SHAPES(T, TYPE, W256, OCC)                                                                      \
-    JL_GEMM_I8_DENSE(T, TYPE, W256, 2, 4, OCC) JL_GEMM_I8_MOE(T, TYPE, W256, 2, 4, OCC) JL_GEMM_I8_MOE(T, TYPE, W256, 2, 2, OCC)
+    JL_GEMM_I8_DENSE(T, TYPE, W256, 2, 4, OCC) JL_GEMM_I8_MOE(T, TYPE, W256, 2, 4, OCC)
 JL_GEMM_I8_SHAPES(q8_0, JL_Q8_0, false, 3) JL_GEMM_I8_SHAPES(q4k, JL_Q4_K, false, 2) JL_GEMM_I8_SHAPES(q6k, JL_Q6_K, false, 2)
 JL_GEMM_I8_SHAPES(q6kw, JL_Q6_K, true, 2)
+JL_GEMM_I8_MOE(q6k, JL_Q6_K, false, 2, 2, 2)
 extern "C" __global__ __launch_bounds__(512) void jl_gemm_i8_q8_0_r4t8(GemmArgs p) {
     gemm_i8_split_slice<JL_Q8_0, false>(p);
     const int y = blockIdx.y;

@@ -222,3 +222,33 @@ def test_q6_scales_that_are_no_numbers(dev, devbuf, planes, ntok):
     finally:
         dev.set_tuning(gemm__few=0, gemm__split=0)
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("t,form", [(quant.Q8_0, 6), (quant.Q4_K, 5), (quant.Q6_K, 7)], ids=["q8_0", "q4_k", "q6_k"])
+@pytest.mark.parametrize("avg", [40, 55])
+def test_banks_at_forty_to_fifty_six_columns(dev, devbuf, t, form, avg):
+    """What a grouped matmul takes by itself between the few-token kernel and the large tiles, window 32: the forced form's values bit for bit, and the oracle's."""
+    n_expert, nrows, k = 128, 160, 256
+    ncols = n_expert * avg
+    dev.SetActWindow(32)
+    w = synth.random_weights(t, nrows, k, seed=21)
+    x = np.stack([synth.activations(k, seed=400 + i) for i in range(61)])
+    src = (np.arange(ncols) * 7 % 61).astype(np.uint32)
+    cuts = np.arange(n_expert + 1, dtype=np.int64) * avg
+    cuts[1:-1] += np.random.default_rng(5).integers(-avg // 2, avg // 2, n_expert - 1)   # (up to two averages an expert)
+    want = oracle.matmul_q8act_f64(t, w, x, nrows, k, 61, 32)[src]
+    bank, xd, sd, cd = devbuf(np.tile(w, n_expert)), devbuf(x), devbuf(src), devbuf(cuts.astype(np.uint32))
+    try:
+        got = []
+        for f in (0, form):
+            dev.set_tuning(moe__form=f)
+            o = [devbuf(shape=(ncols * nrows + 8,), dtype=np.float32, fill=FILL) for _ in range(2)]
+            assert dev.moe_matvec_dev(o[0].ptr, o[1].ptr, t, bank.ptr, bank.ptr, xd.ptr, None, sd.ptr, cd.ptr, n_expert, ncols, nrows, k)
+            dev.synchronize()
+            got.append([a.get() for a in o])
+        for a, b in zip(*got):
+            assert np.all(a[ncols * nrows:] == FILL) and np.array_equal(a, b)
+            assert nmse(a[:ncols * nrows].reshape(ncols, nrows), want) <= 1e-10
+    finally:
+        dev.set_tuning(moe__form=0)
+        dev.SetActWindow(32)
