@@ -1068,11 +1068,23 @@ FewShape few_shape(const jl_ctx* c, int type, bool w256, bool planes, int nrows,
     const int nsb = (k + 255) / 256, form = few_form(type, w256);
     const long avg = ((long)ncols + n_expert - 1) / n_expert, sheets = (long)n_expert * nmat, cus = c->num_cu;
     FewShape f = {1, 1, std::min(8, nsb)};
-    if (groups) f.nt = avg <= 16 ? 1 : avg <= 32 ? 2 : 4;
+    if (groups) {
+        f.nt = avg <= 16 ? 1 : avg <= 32 ? 2 : 4;
+        // Rows, more than 32 columns: three token tiles where a CU holds three workgroups of them for four of two, else, k-quants, two (four
+        // would take every group's activations and registers for columns that most experts do not have; Q8_0's are few enough).  us, two / three /
+        // four tiles, window 32, 36 columns: Q8_0 128 x 768 x 2048 twice 209 / 162 / 222, 60 x 1280 x 2048 162 / 124 / 172, Q6_K 128 x 2048 x 768
+        // 123 / 115 / 156, 60 x 2048 x 1280 131 / 150 / 155, 100 x 512 x 1024 42 / 40 / 47; 48 columns 238 / 221 / 230, 178 / 161 / 174, 139 / 147 /
+        // 161, 152 / 201 / 167, 47 / 52 / 49.
+        if (avg > 32 && !planes) {
+            const int w = (f.nw + 3) / 4, two = c->few_simd[form][0][1][0] / w, three = c->few_simd[form][0][2][0] / w;
+            if (avg <= (type == JL_TYPE_Q8_0 ? 48 : 44) && 4 * three >= 3 * two) f.nt = 3;
+            else if (type != JL_TYPE_Q8_0) f.nt = 2;
+        }
+    }
     else f.nt = (int)std::min<long>((avg + 15) / 16, 4);
     if (c->tune.few_nt) f.nt = c->tune.few_nt;
     if (groups) {
-        if (planes ? (nrows + 31) / 32 * sheets >= cus : f.nt != 2 && (type == JL_TYPE_Q4_K || f.nt == 4) && (nrows + 31) / 32 * sheets >= cus)
+        if (planes ? (nrows + 31) / 32 * sheets >= cus : (f.nt == 4 || (f.nt == 1 && type == JL_TYPE_Q4_K)) && (nrows + 31) / 32 * sheets >= cus)
             f.rt = 2;
         if (planes && f.nt <= 2 && (f.nt == 2 || type != JL_TYPE_Q6_K) && (nrows + 63) / 64 * sheets * 10 >= cus * 7) f.rt = 4;
     } else {
@@ -1829,11 +1841,12 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     //   Q6_K window 32    1: 32/16/15 -> 39/16/12   8: 98/40/31 -> 62/22/15   32: 308/110/89 -> 114/37/25   128: 1065/403/304 -> 254/86/60
     //   Q6_K window 256   2: 48/20/18 -> 47/19/14   8: 67/27/30 -> 59/21/15   48: 179/47/48 -> 111/38/28    128: 238/81/56 -> 183/61/43
     // The few-token kernel reads an expert's sheet once for 64 columns and the columns once for every row tile, so it
-    // gives way to the tiles where the columns are the more; a tile of 64 columns needs two workgroups a CU.  From 40 columns on,
-    // window 32, Q8_0 takes tiles of 128 columns, Q6_K of 64, Q4_K from 56 on 128; blocks of 128 experts of 768 x 2048 and 60 of 1280 x 2048,
-    // 42 columns: Q8_0 on tiles of 64 311 and 249, of 128 303 and 242 (54 columns 348, 321), Q6_K down on tiles of 64 356 and 260, of 128 359 and
-    // 284, Q4_K on tiles of 64, whose registers spilled, 1704 and 1391, on the few-token kernel 405 and 324.  (Tiles of 128 columns would take
-    // Q4_K 380 and 283 there, and Q8_0 288 against 318 at 32 columns; their one chain of sums rounds more than what serves them.)  With a
+    // gives way to the tiles where the columns are the more; a tile of 64 columns needs two workgroups a CU.  From 40 columns on
+    // (52 for Q6_K's rows of up to 1024), window 32, Q8_0 takes tiles of 128 columns, Q6_K of 64, Q4_K from 56 on 128.  us, few-token kernel / tiles: Q8_0 60 x 1280 x 2048 twice, 40 columns 127 / 140, 46
+    // 156 / 141, 60 x 2048 x 1280, 42 columns 101 / 82; Q6_K 128 x 2048 x 768, 46 columns 135 / 131, 100 x 512 x 1024 47 / 52, 60 x 2048 x 1280
+    // 150 / 102.  Tiles of 64 columns were Q8_0's and Q4_K's too: blocks of 128 experts of 768 x 2048, 54 columns 348 (321 on 128) and, spilling,
+    // 1912 (few-token kernel 410).  (Q8_0's and Q4_K's tiles of 128 would be faster earlier for long rows; their one chain of sums rounds more
+    // than the few-token kernel's.)  With a
     // column or two an expert Q6_K's dot-product kernel is as fast while rows are short.  Q4_K with the k-quant window
     // has the forms below, and the few-token kernel where moe_few_faster finds it faster.
     {
@@ -1867,7 +1880,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
             if (q4w) form = ncols <= 8L * n_expert ? 0 : moe_few_faster(type, n_expert, ncols, nmat, nrows, k) ? 5 : 9;
             else if (q6 && c->act_window == 256 && avg > 8 && avg < 60) form = moe_few_faster(type, n_expert, ncols, nmat, nrows, k) ? 5 : 9;
             else if (q6 && avg < (c->act_window == 32 ? 3 : 2) && k < 2048) form = 0;
-            else if (avg < (q6 && c->act_window == 256 ? 28 : 40)) form = 5;
+            else if (avg < (q6 ? c->act_window == 256 ? 28 : k <= 1024 ? 52 : 40 : 40)) form = 5;
             else if (avg < (q6 && c->act_window == 32 ? 64 : 56)) form = tiles64 < 2 * c->num_cu || type == JL_TYPE_Q4_K ? 5 : q6 && c->act_window == 32 ? 7 : 6;
             else form = type == JL_TYPE_Q8_0 && avg >= 64 && tiles64 >= 2 * c->num_cu ? 8 : 6;
         }

@@ -75,7 +75,7 @@ def test_tiles_per_expert(dev, devbuf, t, window, nrows, k):
                     # (the gated activation: an exponential of another machine in front of the quantizer)
                     assert nmse(got[:ncols * nrows].reshape(ncols, nrows), want[b]) <= (1e-6 if gated else 1e-10), (gated, form, b)
     finally:
-        dev.set_tuning(moe__form=0)
+        dev.set_tuning(moe__form=0, few__nt=0)
         dev.SetActWindow(32)
 
 
@@ -224,10 +224,9 @@ def test_q6_scales_that_are_no_numbers(dev, devbuf, planes, ntok):
         dev.SetActWindow(32)
 
 
-@pytest.mark.parametrize("t,form", [(quant.Q8_0, 6), (quant.Q4_K, 5), (quant.Q6_K, 7)], ids=["q8_0", "q4_k", "q6_k"])
-@pytest.mark.parametrize("avg", [40, 55])
-def test_banks_at_forty_to_fifty_six_columns(dev, devbuf, t, form, avg):
-    """What a grouped matmul takes by itself between the few-token kernel and the large tiles, window 32: the forced form's values bit for bit, and the oracle's."""
+@pytest.mark.parametrize("t,avg,form", [(quant.Q8_0, 36, 5), (quant.Q8_0, 46, 6), (quant.Q4_K, 40, 5), (quant.Q4_K, 55, 5), (quant.Q6_K, 36, 5), (quant.Q6_K, 55, 7)])
+def test_banks_at_forty_to_fifty_six_columns(dev, devbuf, t, avg, form):
+    """What a grouped matmul takes by itself between the few-token kernel and the large tiles, window 32: the forced form's values bit for bit, the few-token kernel's also with its columns in fours of tiles, and the oracle's."""
     n_expert, nrows, k = 128, 160, 256
     ncols = n_expert * avg
     dev.SetActWindow(32)
@@ -240,8 +239,8 @@ def test_banks_at_forty_to_fifty_six_columns(dev, devbuf, t, form, avg):
     bank, xd, sd, cd = devbuf(np.tile(w, n_expert)), devbuf(x), devbuf(src), devbuf(cuts.astype(np.uint32))
     try:
         got = []
-        for f in (0, form):
-            dev.set_tuning(moe__form=f)
+        for f, nt in ((0, 0), (form, 4 if form == 5 else 0)):
+            dev.set_tuning(moe__form=f, few__nt=nt)
             o = [devbuf(shape=(ncols * nrows + 8,), dtype=np.float32, fill=FILL) for _ in range(2)]
             assert dev.moe_matvec_dev(o[0].ptr, o[1].ptr, t, bank.ptr, bank.ptr, xd.ptr, None, sd.ptr, cd.ptr, n_expert, ncols, nrows, k)
             dev.synchronize()
@@ -250,5 +249,5 @@ def test_banks_at_forty_to_fifty_six_columns(dev, devbuf, t, form, avg):
             assert np.all(a[ncols * nrows:] == FILL) and np.array_equal(a, b)
             assert nmse(a[:ncols * nrows].reshape(ncols, nrows), want) <= 1e-10
     finally:
-        dev.set_tuning(moe__form=0)
+        dev.set_tuning(moe__form=0, few__nt=0)
         dev.SetActWindow(32)
