@@ -99,7 +99,8 @@ int jl_synchronize(jl_ctx *ctx);
  * token), "gemm.few" (1: form 4 for any number of tokens, 2: never,
  * 3: a decode matvec a token in one launch, up to sixteen), "few.nt" / "few.rt" /
  * "few.waves" (its token tiles, row tiles and wavefronts a workgroup), "gemm.i8" (the int8 tiles of
- * Q8_0: 1 / 2 / 3 for 128 x 128 / 128 tokens x 64 rows / 256 x 128), "matvec.lanes" (lanes a row of a decode matvec: 16, 32, 64), "gemm.rows" (64 or 128),
+ * Q8_0: 1 / 2 / 3 for 128 x 128 / 128 tokens x 64 rows / 256 x 128), "gemm.tall" (of the last: 1 no tiles of 64 rows behind
+ * the others, 2 + n: from row tile n on), "matvec.lanes" (lanes a row of a decode matvec: 16, 32, 64), "gemm.rows" (64 or 128),
  * "gemm.split" (K slices), "gemm.prep" (4: the four-wavefront activation prep), "gemm.planes"
  * (2: restore rows from planes before the GEMM), "packed.rw" (rows per wavefront of the
  * packed-plane matvec: 16, 32, 64), "packed.block" (its threads per workgroup), "moe.shares"
@@ -114,7 +115,8 @@ int jl_synchronize(jl_ctx *ctx);
  * block's other kernels),
  * "mxfp4.split" (K slices of the MXFP4 GEMM), "mxfp4.rows" (96 or 128 rows a tile; 1: the
  * general decode matvec also for one token), "mxfp4.few" / "mxfp4.few_min" (the MXFP4
- * few-token form up to / from this many tokens), "mxfp4.planes" (3 / 4: 64-token tiles of 64 / 96
+ * few-token form up to / from this many tokens), "mxfp4.one" (its single launch: 1 never, 11 / 12 with 16 / 32 rows
+ * a workgroup), "mxfp4.planes" (3 / 4: 64-token tiles of 64 / 96
  * rows over planes, rows turned into planes first; packed MXFP4: 2 restores rows first,
  * 64 / 32 / 16 rows a workgroup of the plane matvec); value 0 restores the built-in choice.  These change launch shapes and f32 summation
  * order only.  Two keys change values, both off unless set: "mxfp4.scaled" = 1 runs

@@ -3313,7 +3313,7 @@ MxRowsPlan mx_rows_plan(const jl_ctx* c, int nrows, int k, int ntok) {
 
 // Few tokens: 16-row workgroups whose wavefronts split K, in chunks of up to 64 tokens, one launch after a prep
 // that lays the activations out in the order the block decode produces.
-// From where: the kernels for a handful of tokens grow with the tokens, this one does not, but it is two launches, which a
+// (The same tiles in one launch come first, mx_one_rows.)  From where: the kernels for a handful of tokens grow with the tokens, this one does not, but it is two launches, which a
 // host that issues calls one after the other cannot do in less than 6.7 us.  From three tokens, so, where the one launch
 // is estimated to take more than that and more than this form: over rows a token costs what a round of their workgroups
 // does, four rows each, on all CUs, over planes what K and the matrix do (fitted to 17 shapes, 512 x 512 to 12288 x 2048,

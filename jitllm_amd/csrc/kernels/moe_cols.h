@@ -8,7 +8,8 @@
 // quantized once each (the prep), not once a column: a column's record is found through the routing's own list.
 //
 // 128 experts, 48 columns each, us (prep included): Q4_K, two banks of 768 x 2048 177 -> 98; 2048 x 768 98 -> 67; Q6_K
-// 2048 x 768 115 -> 87.  The block of 777 rows, top 8 (Q4_K, Q6_K down): 339 -> 234.
+// 2048 x 768 115 -> 87.  The block of 777 rows, top 8 (Q4_K, Q6_K down): 339 -> 234, 216 with all that came behind (router, lists, the first
+// rows asked for ahead of the routing).
 //
 // What bounds it (two banks of 768 x 2048, timestamps in the kernel): a super-block takes 1.0 us of work -- vector
 // instructions, eight a matrix instruction (decoding 4.5 at 64 columns, the epilogue 3), which a SIMD issues one after the
