@@ -559,7 +559,6 @@ __device__ __forceinline__ void few_planes_half(int c, const FewPlaneW<TYPE>* W,
     }
 }
 
-// grid = (ceil(nrows / (16 RT)), experts or token groups, matrices), block = 64 * p.nwaves, dynamic LDS: JL_FEW_LDS_BYTES.
 // Q6_K, window 32: result (row r, token tok of a slot) block by block.  A row's scale that is infinite meets the sum of four blocks
 // above; the decode matvec's infinities and NaN are those of its products with the blocks one by one.
 template <bool PL>
@@ -574,22 +573,29 @@ __device__ __forceinline__ float few_q6_one(const FewI8Args& p, const FewMat& m,
         const u32* a = (const u32*)p.bq + x * 512 + (s >> 1) * 256 + tok * 4 + 2 * (s & 1);
         const uint8_t* blk = PL ? nullptr : row + (size_t)sb * 210;
         i32 P = 0;
-#pragma unroll 1
-        for (int l = 0; l < 32; l++) {
-            const int run = l >> 4, i = (l >> 2) & 3, j = l & 3;
-            u32 q;
-            i32 sc;
+#pragma unroll
+        for (int run = 0; run < 2; run++) {
+            u32x4 lo, hi = {0u, 0u, 0u, 0u};   // the run's words
+            u32 hw = 0;
+            i32 sc, v = 0;
             if constexpr (PL) {
                 const u32* w = m.qs + ((size_t)(sb * 16 + half * 8 + 2 * s + run) * 3) * n + at;
-                q = ((w[(i & 1) * n] >> (8 * j + 4 * (i >> 1))) & 15) | (((w[2 * n] >> (8 * j + 2 * i)) & 3) << 4);
+                lo = u32x4{w[0], w[n], w[0] >> 4, w[n] >> 4};
+                hw = w[2 * n];
                 sc = (i32)((m.sp[((size_t)sb * 4 + 2 * half + (s >> 1)) * n + at] >> (16 * (s & 1) + 8 * run)) & 255) - 128;
             } else {
-                q = ((blk[64 * half + 32 * (s & 1) + l] >> (4 * (s >> 1))) & 15) | (((blk[128 + 32 * half + l] >> (2 * s)) & 3) << 4);
+                lo = ld16_a2(blk + 64 * half + 32 * (s & 1) + 16 * run);
+                hi = ld16_a2(blk + 128 + 32 * half + 16 * run);
                 sc = (int8_t)blk[192 + 8 * half + 2 * s + run];
             }
-            int g, h;
-            jl_few_order(PL ? 2 : 0, l >> 2, g, h);
-            P += sc * ((i32)q - 32) * (int8_t)(a[g * 64 + h] >> (8 * j));
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const u32 h2 = PL ? hw >> (2 * i) : hi[i] >> (2 * s), q = ((PL ? lo[i] : lo[i] >> (4 * (s >> 1))) & 0x0F0F0F0Fu) | ((h2 & 0x03030303u) << 4);
+                int g, h;
+                jl_few_order(PL ? 2 : 0, 4 * run + i, g, h);
+                v = dot4(0xE0E0E0E0u, a[g * 64 + h], dot4(q, a[g * 64 + h], v));   // q - 32
+            }
+            P += sc * v;
         }
         const u32 d = PL ? m.dp[(size_t)sb * n + at] : (u32)ld2(blk + 208);
         o = fmaf((float)P, half_bits_to_f32((uint16_t)d) * p.da[x * 64 + 4 * tok + s], o);
@@ -597,6 +603,7 @@ __device__ __forceinline__ float few_q6_one(const FewI8Args& p, const FewMat& m,
     return o;
 }
 
+// grid = (ceil(nrows / (16 RT)), experts or token groups, matrices), block = 64 * p.nwaves, dynamic LDS: JL_FEW_LDS_BYTES.
 template <int TYPE, bool PL, int NT, int RT, bool W256>
 __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem) {
     FewI8Args p;   // the matrix's arguments, asked for at once
@@ -823,9 +830,26 @@ __device__ __forceinline__ void few_i8_body(const FewI8Args& args, uint8_t* smem
             int q = 0;
             for (; q + 4 <= nw; q += 4, at += 4 * W) v += (at[0] + at[W]) + (at[2 * W] + at[3 * W]);
             for (; q < nw; q++, at += W) v += at[0];
+            if constexpr (TYPE == JL_Q6_K && !W256) {
+                // Again where a row's scale is infinite or four blocks' sum passes the largest f32, but not where the token has a scale that
+                // is no number: its blocks' integers are zero, its sums NaN in every row and form.  (4096 x 4096, 12 tokens, one of them with
+                // an infinite activation: 485 us without that second look, 22 as a call without.)  Sixteen lanes in a row hold one token.
+                const bool mine = (u32)tok < left && r0 + rr < p.nrows && !__builtin_isfinite(v);
+                if (__ballot(mine)) {
+                    u32 l = threadIdx.x & 63;
+                    few_pin(l);   // (nothing of this ahead of the wavefront's super-blocks, in registers of theirs)
+                    bool bad = false;
+                    if ((u32)tok < left)
+                        for (int x = l & 15; x < p.k / 128; x += 16) {
+                            const f32x4 d = *(const f32x4*)(p.da + ((size_t)x * p.nslots + slot0 + t0 + (tok >> 4)) * 64 + 4 * (tok & 15));
+#pragma unroll
+                            for (int b = 0; b < 4; b++) bad |= !__builtin_isfinite(d[b]);
+                        }
+                    const bool token = ((u32)(__ballot(bad) >> (l & 48)) & 0xFFFFu) == 0;
+                    if (mine && token) v = few_q6_one<PL>(p, m, e, r0 + rr, slot0 + t0 + (tok >> 4), tok & 15);
+                }
+            }
             if ((u32)tok < left && r0 + rr < p.nrows) {
-                if constexpr (TYPE == JL_Q6_K && !W256)
-                    if (!__builtin_isfinite(v)) v = few_q6_one<PL>(p, m, e, r0 + rr, slot0 + t0 + (tok >> 4), tok & 15);
                 const size_t o = (size_t)(col0 + t0 * 16 + tok) * p.nrows + r0 + rr;
                 if (p.out[0]) p.out[0][o] = v;
                 if (p.resid) p.resid[o] += v;

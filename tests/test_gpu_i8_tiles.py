@@ -1,5 +1,7 @@
 """The int8 tile kernels (kernels/gemm_i8.h), dense and per expert, at the edges of their tiles: rows and tokens one
 short of, at and one past a tile, K of an odd number of stages, K splits, every shape; against the oracle in f64."""
+import time
+
 import numpy as np
 import pytest
 
@@ -222,6 +224,58 @@ def test_q6_scales_that_are_no_numbers(dev, devbuf, planes, ntok):
     finally:
         dev.set_tuning(gemm__few=0, gemm__split=0)
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("ntok,few", [(12, 0), (200, 2)], ids=["few", "tiles"])
+@pytest.mark.parametrize("t", [quant.Q8_0, quant.Q4_K, quant.Q6_K], ids=["q8_0", "q4_k", "q6_k"])
+def test_an_activation_that_is_no_number(dev, devbuf, t, ntok, few):
+    """Window 32, one activation infinite or NaN, in the first and the last token: that token's sums are NaN, the others' bits are those
+    without it, and the call takes about as long (three times allowed; summed again row by row it was 6 to 130 times).  One that is
+    finite but large enough for sums without the row's scale to pass the largest f32: the oracle's values."""
+    nrows, k = 2048, 2048
+    dev.SetActWindow(32)
+    w = synth.quantized_weights(t, nrows, k, seed=31)
+    x = np.stack([synth.activations(k, seed=970 + i) for i in range(ntok)])
+    wd, o = devbuf(w), devbuf(shape=(ntok, nrows), dtype=np.float32)
+
+    def call(xd):
+        assert dev.matmul_dev(o.ptr, t, wd.ptr, xd.ptr, nrows, k, ntok)
+
+    def us(xd):
+        best = 1e30
+        for _ in range(5):
+            dev.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(20):
+                call(xd)
+            dev.synchronize()
+            best = min(best, (time.perf_counter() - t0) / 20 * 1e6)
+        return best
+
+    dev.set_tuning(gemm__few=few)
+    try:
+        clean = devbuf(x)
+        call(clean)
+        dev.synchronize()
+        ref, base = o.get(), us(clean)
+        for tok in (0, ntok - 1):
+            for v in (np.inf, np.nan, 3e36):
+                y = x.copy()
+                y[tok, 77] = v
+                yd = devbuf(y)
+                call(yd)
+                dev.synchronize()
+                got = o.get()
+                others = np.arange(ntok) != tok
+                assert np.array_equal(got[others].view(np.uint32), ref[others].view(np.uint32))
+                if np.isfinite(v):
+                    want = oracle.matmul_q8act_f64(t, w, y[tok:tok + 1], nrows, k, 1, 32)
+                    assert np.isfinite(got[tok]).all() and nmse(got[tok].astype(np.float64) * 1e-20, want[0] * 1e-20) <= 1e-10
+                else:
+                    assert np.isnan(got[tok]).all()
+                    assert us(yd) <= 3 * base, (tok, v)
+    finally:
+        dev.set_tuning(gemm__few=0)
 
 
 @pytest.mark.parametrize("t,avg,form", [(quant.Q8_0, 36, 5), (quant.Q8_0, 46, 6), (quant.Q4_K, 40, 5), (quant.Q4_K, 55, 5), (quant.Q6_K, 36, 5), (quant.Q6_K, 55, 7)])
