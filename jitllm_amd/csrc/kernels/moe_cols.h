@@ -9,7 +9,7 @@
 //
 // 128 experts, 48 columns each, us (prep included): Q4_K, two banks of 768 x 2048 177 -> 98; 2048 x 768 98 -> 67; Q6_K
 // 2048 x 768 115 -> 87.  The block of 777 rows, top 8 (Q4_K, Q6_K down): 339 -> 234, 216 with all that came behind (router, lists, the first
-// rows asked for ahead of the routing).
+// rows asked for ahead of the columns).
 //
 // What bounds it (two banks of 768 x 2048, timestamps in the kernel): a super-block takes 1.0 us of work -- vector
 // instructions, eight a matrix instruction (decoding 4.5 at 64 columns, the epilogue 3), which a SIMD issues one after the
@@ -114,9 +114,8 @@ __device__ __forceinline__ void mc_store(const MoeColsArgs& p, const f32x16 (&ou
         }
 }
 
-// Q4_K rows.  G: groups of 32 columns (n columns exist).  The rows' bytes come to LDS as they lie, 144 contiguous bytes a
-// row (straight into registers, a lane a row, is sixteen bytes of 64 lines an instruction), and each wavefront reads its own.
-struct MoeColsQ4Rows { u32 woff[4], xoff; };   // a lane's places among the rows' bytes
+// Asks for a super-block of a Q4_K tile's rows; w: a lane's places among the rows' bytes.
+struct MoeColsQ4Rows { u32 woff[4], xoff; };
 __device__ __forceinline__ void moe_cols_q4_rows(const MoeColsArgs& p, uint8_t* smem, const uint8_t* sheet, int last, MoeColsQ4Rows& w) {
     constexpr int O_W = 2 * JL_MC_A;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -134,7 +133,9 @@ __device__ __forceinline__ void moe_cols_q4_rows(const MoeColsArgs& p, uint8_t* 
     w.xoff = piece_at(16 + (wave & 1));
     if (wave < 2) load_lds16(sheet, w.xoff, __builtin_amdgcn_readfirstlane(lds0 + O_W + 1024 * (16 + wave)));
 }
-// w: the places, and the first super-block's rows already asked for
+// Q4_K rows.  G: groups of 32 columns (n columns exist).  The rows' bytes come to LDS as they lie, 144 contiguous bytes a
+// row (straight into registers, a lane a row, is sixteen bytes of 64 lines an instruction), and each wavefront reads its own.
+// w: the places, and the first super-block's rows already asked for.
 template <int G>
 __device__ __forceinline__ void moe_cols_q4_tile(const MoeColsArgs& p, uint8_t* smem, const uint8_t* sheet, const MoeColsQ4Rows& w, int mat, int r0, u32 c0, int n) {
     constexpr int O_W = 2 * JL_MC_A, O_AUG = O_W + 2 * JL_MC_W, O_DA = O_AUG + 2 * 64 * 32;
@@ -588,15 +589,15 @@ __device__ __forceinline__ void moe_cols_body(const MoeColsArgs& p, uint8_t* sme
     const u32 z = item % (u32)p.shares, i1 = item / (u32)p.shares, rb = i1 % (u32)p.rblocks, i2 = i1 / (u32)p.rblocks;
     const int mat = __builtin_amdgcn_readfirstlane((int)(i2 % (u32)p.nmat)), e = __builtin_amdgcn_readfirstlane((int)(i2 / (u32)p.nmat));
     const int r0 = __builtin_amdgcn_readfirstlane((int)rb * 128);
-    // Which columns are the expert's takes two trips to memory (start, then the records' numbers): the rows' bytes, which do not
-    // depend on it, are asked for first.
     const uint8_t* sheet = p.bank[mat] + (size_t)e * p.sheet_bytes + (size_t)r0 * p.row_bytes;
-    MoeColsQ4Rows w4;
-    if constexpr (KO == 0) moe_cols_q4_rows(p, smem, sheet, p.nrows - 1 - r0, w4);
-    const u32 c_hi = p.start[e + 1], c_lo = p.start[e] + 64 * z;
-    for (u32 c0 = c_lo; c0 < c_hi; c0 += 64 * (u32)p.shares) {   // uniform
+    const u32 c_hi = p.start[e + 1];
+    for (u32 c0 = p.start[e] + 64 * z; c0 < c_hi; c0 += 64 * (u32)p.shares) {   // uniform
         const int n = (int)min(64u, c_hi - c0);
-        if (KO == 0 && c0 != c_lo) moe_cols_q4_rows(p, smem, sheet, p.nrows - 1 - r0, w4);
+        // The rows' bytes are asked for ahead of the columns, which wait for the records' numbers.  Ahead of start as well they save even
+        // routing nothing (1.00, 55 banks and column counts), and a workgroup without columns, which brings 18 KB for nothing, costs uneven
+        // routing: 128 experts of 2048 x 768, eight of them with columns, 32 an expert on average 84 us, so 64; half of the experts 53 and 50.
+        MoeColsQ4Rows w4;
+        if constexpr (KO == 0) moe_cols_q4_rows(p, smem, sheet, p.nrows - 1 - r0, w4);
         auto tile = [&](auto G) __attribute__((always_inline)) {
             constexpr int g = decltype(G)::value;
             if constexpr (KO == 0) moe_cols_q4_tile<g>(p, smem, sheet, w4, mat, r0, c0, n);
@@ -606,5 +607,4 @@ __device__ __forceinline__ void moe_cols_body(const MoeColsArgs& p, uint8_t* sme
         if (n > 32) tile(GemmIntC<2>{});
         else tile(GemmIntC<1>{});
     }
-    if constexpr (KO == 0) wait_loads<0>();   // (no columns: LDS is written until the rows have come)
 }

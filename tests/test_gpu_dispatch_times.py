@@ -1,0 +1,62 @@
+"""What a rule takes by itself is about as fast as the best of the forms it could have taken, where a rule once was not: device time of
+calls queued behind a wait, the fastest of several windows of either in turn.  The limits are half of what the wrong pick cost, several
+times what two measurements of one launch differ."""
+import numpy as np
+import pytest
+
+from jitllm_amd import quant, synth
+from jitllm_amd.hipmem import Gate, timed_windows
+
+pytestmark = pytest.mark.gpu
+
+
+def us(dev, calls, steps=30):
+    """calls: name -> (tuning, call).  us a call of each, the fastest of fifteen windows, in turn."""
+    best = {n: 1e30 for n in calls}
+    for _ in range(3):
+        for n, (tuning, call) in calls.items():
+            dev.set_tuning(**tuning)
+            try:
+                for _ in range(3):
+                    assert call()
+                dev.synchronize()
+                _, per = timed_windows(lambda i: call(), steps, dev.stream, 5, Gate(dev))
+                best[n] = min(best[n], min(per) * 1e3)
+            finally:
+                dev.set_tuning(**{k: 0 for k in tuning})
+    return best
+
+
+def random_bank(devbuf, t, sheets, nrows, k):
+    """A bank of equal sheets (what the kernels read has no part in their time)."""
+    return devbuf(np.tile(synth.random_weights(t, nrows, k, seed=3), sheets))
+
+
+class Columns:
+    """A grouped matmul of `counts` columns an expert over n banks."""
+
+    def __init__(self, dev, devbuf, t, counts, nrows, k, nmat):
+        self.dev, self.n, ncols = dev, len(counts), int(np.sum(counts))
+        self.banks = [random_bank(devbuf, t, len(counts), nrows, k) for _ in range(nmat)]
+        self.x, self.src = devbuf(np.stack([synth.activations(k, seed=i) for i in range(64)])), devbuf((np.arange(ncols) % 64).astype(np.uint32))
+        self.start = devbuf(np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32))
+        self.out = [devbuf(shape=(ncols, nrows), dtype=np.float32) for _ in range(nmat)]
+        second = (self.out[1].ptr, self.banks[1].ptr) if nmat == 2 else (None, None)
+        self.args = (self.out[0].ptr, second[0], t, self.banks[0].ptr, second[1], self.x.ptr, None, self.src.ptr, self.start.ptr, len(counts), ncols, nrows, k)
+
+    def __call__(self):
+        return self.dev.moe_matvec_dev(*self.args)
+
+
+def test_experts_without_columns(dev, devbuf):
+    """Q4_K columns against decoded rows: eight of 128 experts with all of the columns against all with 32 each, 1.4 times; with every
+    other workgroup bringing rows for nothing it was 1.9."""
+    dev.SetActWindow(256)
+    try:
+        even, few = np.full(128, 32), np.zeros(128, int)
+        few[5::16] = 512
+        form = dict(moe__form=9)
+        t = us(dev, {n: (form, Columns(dev, devbuf, quant.Q4_K, c, 2048, 768, 1)) for n, c in (("even", even), ("few", few))})
+        assert t["few"] <= 1.65 * t["even"], t
+    finally:
+        dev.SetActWindow(32)
