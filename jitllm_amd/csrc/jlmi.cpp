@@ -1070,15 +1070,28 @@ FewShape few_shape(const jl_ctx* c, int type, bool w256, bool planes, int nrows,
     FewShape f = {1, 1, std::min(8, nsb)};
     if (groups) {
         f.nt = avg <= 16 ? 1 : avg <= 32 ? 2 : 4;
-        // Rows, more than 32 columns: three token tiles where a CU holds three workgroups of them for four of two, else, k-quants, two (four
-        // would take every group's activations and registers for columns that most experts do not have; Q8_0's are few enough).  us, two / three /
-        // four tiles, window 32, 36 columns: Q8_0 128 x 768 x 2048 twice 209 / 162 / 222, 60 x 1280 x 2048 162 / 124 / 172, Q6_K 128 x 2048 x 768
-        // 123 / 115 / 156, 60 x 2048 x 1280 131 / 150 / 155, 100 x 512 x 1024 42 / 40 / 47; 48 columns 238 / 221 / 230, 178 / 161 / 174, 139 / 147 /
-        // 161, 152 / 201 / 167, 47 / 52 / 49.
+        // Rows, more than 32 columns.  Many workgroups: three token tiles where a CU holds three workgroups of them for four of two, else, k-quants,
+        // two (four would take every group's activations and registers for columns that most experts do not have; Q8_0's are few enough, and from
+        // K = 4096 on a second pass costs more).  us, two / three / four tiles, window 32, 36 columns: Q8_0 128 x 768 x 2048 twice 209 / 162 / 222,
+        // 60 x 1280 x 2048 162 / 124 / 172, Q6_K 128 x 2048 x 768 123 / 115 / 156, 60 x 2048 x 1280 131 / 150 / 155, 100 x 512 x 1024 42 / 40 / 47;
+        // 48 columns 238 / 221 / 230, 178 / 161 / 174, 139 / 147 / 161, 152 / 201 / 167, 47 / 52 / 49, 8 x 4096 x 4096 85 / 92 / 76.
+        // Few workgroups, fewer than eight a CU of one row tile: they run at once, and the launch lasts as long as the passes of its fullest expert
+        // (columns taken as dealt at random).  Three tiles where its columns should fit them: 36 columns, Q8_0 8 x 512 x 1024 9.5 / 7.9 / 8.5.  Else
+        // four: 44 columns 9.7 / 10.7 / 8.7, Q6_K 2 x 1024 x 4096 twice 17 / 19 / 14, the same 8 with the k-quant window 10.2 / 11.1 / 8.9; two
+        // where four would come with two row tiles, whose pass is twice as long, and K is short: Q8_0 8 x 512 x 512 twice 10.0 / 11.2 / 11.4.
+        // 486 launches of 2 to 128 experts, 33 to 54 columns: 1.0 % behind the best of the three, always four 10 %.
         if (avg > 32 && !planes) {
             const int w = (f.nw + 3) / 4, two = c->few_simd[form][0][1][0] / w, three = c->few_simd[form][0][2][0] / w;
-            if (avg <= (type == JL_TYPE_Q8_0 ? 48 : 44) && 4 * three >= 3 * two) f.nt = 3;
-            else if (type != JL_TYPE_Q8_0) f.nt = 2;
+            const bool packs = 4 * three >= 3 * two, q8 = type == JL_TYPE_Q8_0;
+            const long wgs = (nrows + 15) / 16 * sheets;
+            const auto any_over = [&](int n) { return 1 - std::pow(1 - 0.5 * std::erfc((n + 0.5 - avg) / std::sqrt(2.0 * avg)), n_expert); };
+            if (avg <= 34 && !packs && wgs > 2 * cus) f.nt = 2;   // (Q6_K 8 x 4096 x 4096, 33 columns 57 / 71 / 73)
+            else if (wgs >= 8 * cus) {
+                if (avg <= (q8 && nsb < 16 ? 48 : 44) && packs) f.nt = 3;
+                else if (!q8 && nsb < 16) f.nt = 2;
+            } else if (any_over(48) < 0.3 && (packs || wgs <= 2 * cus)) f.nt = 3;
+            else if (nsb < 8 && (nrows + 31) / 32 * sheets >= cus) f.nt = 2;
+            else if (any_over(64) >= 0.5) f.nt = packs ? 3 : 2;
         }
     }
     else f.nt = (int)std::min<long>((avg + 15) / 16, 4);
@@ -1585,7 +1598,7 @@ int moe_g16_blocks(const jl_ctx* c, int nrows, int k, int n_expert, int ncols, i
 bool moe_few_faster(int type, int n_expert, int ncols, int nmat, int nrows, int k) {
     const double avg = (double)ncols / n_expert, nsb = k / 256, melem = 1e-6 * n_expert * nmat * (double)nrows * k;
     const auto over = [&](int n) { return 0.5 * std::erfc((n + 0.5 - avg) / std::sqrt(2 * avg)); };   // an expert's columns pass n
-    const int nt = avg <= 16 ? 1 : avg <= 32 ? 2 : 4;
+    const int nt = avg <= 16 ? 1 : avg <= 32 ? 2 : 4;   // (few_shape takes fewer where those are faster than four)
     const double passes = melem * (1 + over(16 * nt));
     if (type == JL_TYPE_Q4_K) {
         if (avg >= 32) return false;
@@ -1840,7 +1853,7 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     //   Q8_0 window 32    1: 39/16/13 -> 36/15/12   8: 90/29/25 -> 53/21/14   32: 235/71/69 -> 92/30/20   128: 853/238/236 -> 170/56/41
     //   Q6_K window 32    1: 32/16/15 -> 39/16/12   8: 98/40/31 -> 62/22/15   32: 308/110/89 -> 114/37/25   128: 1065/403/304 -> 254/86/60
     //   Q6_K window 256   2: 48/20/18 -> 47/19/14   8: 67/27/30 -> 59/21/15   48: 179/47/48 -> 111/38/28    128: 238/81/56 -> 183/61/43
-    // The few-token kernel reads an expert's sheet once for 64 columns and the columns once for every row tile, so it
+    // The few-token kernel reads an expert's sheet once for 16 to 64 columns (few_shape) and the columns once for every row tile, so it
     // gives way to the tiles where the columns are the more; a tile of 64 columns needs two workgroups a CU.  From 40 columns on
     // (52 for Q6_K's rows of up to 1024), window 32, Q8_0 takes tiles of 128 columns, Q6_K of 64, Q4_K from 56 on 128.  us, few-token kernel / tiles: Q8_0 60 x 1280 x 2048 twice, 40 columns 127 / 140, 46
     // 156 / 141, 60 x 2048 x 1280, 42 columns 101 / 82; Q6_K 128 x 2048 x 768, 46 columns 135 / 131, 100 x 512 x 1024 47 / 52, 60 x 2048 x 1280

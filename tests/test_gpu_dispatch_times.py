@@ -60,3 +60,21 @@ def test_experts_without_columns(dev, devbuf):
         assert t["few"] <= 1.65 * t["even"], t
     finally:
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("t,window,n_expert,nrows,k,nmat,avg", [
+    (quant.Q8_0, 32, 8, 512, 1024, 1, 44), (quant.Q4_K, 32, 4, 2048, 2048, 1, 44), (quant.Q6_K, 32, 2, 1024, 4096, 2, 44),
+    (quant.Q6_K, 256, 8, 512, 1024, 1, 44), (quant.Q8_0, 32, 128, 768, 2048, 2, 36)], ids=lambda v: str(v))
+def test_token_tiles_of_a_group(dev, devbuf, t, window, n_expert, nrows, k, nmat, avg):
+    """Banks of few experts and a large one at more than 32 columns an expert: the token tiles a workgroup of the few-token kernel takes."""
+    dev.SetActWindow(window)
+    try:
+        counts = np.full(n_expert, avg)
+        counts[::2] += 7
+        counts[1::2] -= 7
+        call = Columns(dev, devbuf, t, counts, nrows, k, nmat)
+        forms = {"auto": ({}, call)} | {nt: (dict(moe__form=5, few__nt=nt), call) for nt in (2, 3, 4)}
+        got = us(dev, forms)
+        assert got["auto"] <= 1.1 * min(got[nt] for nt in (2, 3, 4)), got
+    finally:
+        dev.SetActWindow(32)
