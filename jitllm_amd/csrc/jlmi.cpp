@@ -2762,19 +2762,25 @@ int jl_moe_logits_dev(jl_ctx* c, float* logits, int wtype, const void* w, const 
     // other's dependent adds.  us by 1 / 2 / 4 / 8 rows, x from memory: 128 experts x 2048, 64 tokens 5.3 / 6.0 / 6.7 / 9.4, 128 9.2 /
     // 6.4 / 7.2 / 9.6, 256 13.6 / 9.0 / 7.7 / 10.3, 512 22 / 14.6 / 11.7 / 11.6, 1024 47 / 31 / 23 / 18.9; 64 x 2048, 512 tokens 14.5 /
     // 10.1 / 7.7 / 10.3; 87 x 1024, 1024 tokens 29 / 12.3 / 9.5 / 10.0; 16 x 2816, 1024 tokens 18.6 / 10.8 / 11.5 / 14.1.  Tuning
-    // "moe.logits" = 1 / 2 / 4 / 8 forces a form.
-    int eb = c->tune.moe_logits;
+    // "moe.logits" = 1 / 2 / 4 / 8 forces a form, and 16 or 32 more the order of the grid below: token groups or rows of the router.
+    int eb = c->tune.moe_logits % 16;
     if (eb != 1 && eb != 2 && eb != 4 && eb != 8) {
         const auto a_cu = [&](int e) { return (double)((n_expert + e - 1) / e) * ((ntok + 7) / 8) / c->num_cu; };
         eb = a_cu(1) <= 4 ? 1 : a_cu(2) <= 5 ? 2 : a_cu(4) <= std::max(5.75, 11776.0 / k) ? 4 : 8;
     }
-    const unsigned gx = (unsigned)std::min(8, (ntok + 7) / 8);   // token groups side by side
-    if (eb > 1) {
-        Name name;
-        name << "jl_moe_logits_e" << eb << (a.f16 ? "_f16" : "");
-        return launch(c, name, gx, (unsigned)((n_expert + eb - 1) / eb), 128, 0, pick_stream(c, stream), params, (unsigned)((ntok + 63) / 64));
-    }
-    return launch(c, "jl_moe_logits", gx, (unsigned)n_expert, 128, 0, pick_stream(c, stream), params, (unsigned)((ntok + 63) / 64));   // JL_LOGITS_TOK
+    const unsigned groups = (unsigned)(ntok + 7) / 8, blocks = (unsigned)(n_expert + eb - 1) / eb;   // JL_LOGITS_TOK
+    // Workgroups go round the XCDs in the order of their numbers.  Token groups side by side bring each its rows of x to one L2, and every
+    // row of the router to all; rows of the router side by side bring each to one L2, and x to all.  The first where many tokens meet a router that an L2
+    // holds (4 MB), the second where it does not, and for a few tokens where the router is large.  us, token groups / rows: 384 x 7168 in f32,
+    // 2048 tokens 334 / 265, 256 x 7168 192 / 181, 128 x 7168 93 / 100; 256 x 7168 in f16, 16 tokens 21.7 / 13.7, 160 x 5120 in f16, 32 tokens
+    // 16.3 / 11.2, in f32 16 tokens 8.4 / 7.6; 128 x 2048 in f32, 128 tokens 6.4 / 7.3.  (275 shapes: 0.4 % behind the better order.)
+    const size_t elems = (size_t)n_expert * k;
+    a.by_expert = c->tune.moe_logits >= 16 ? c->tune.moe_logits >= 32 : (elems >= 800000 && ntok <= 64) || elems * (a.f16 ? 2 : 4) > ((size_t)4 << 20);
+    Name name;
+    name << "jl_moe_logits";
+    if (eb > 1) name << "_e" << eb << (a.f16 ? "_f16" : "");
+    if (a.by_expert) return launch(c, name, blocks, groups, 128, 0, pick_stream(c, stream), params);
+    return launch(c, name, std::min(8u, groups), blocks, 128, 0, pick_stream(c, stream), params, (groups + 7) / 8);
 }
 
 namespace {

@@ -358,6 +358,7 @@ struct MoeLogitsArgs {
     const float* x;         // [ntok][k]
     float* logits;          // [ntok][n_expert]
     int n_expert, k, ntok, f16;
+    int by_expert;          // the grid's order: 0 token groups side by side, 1 expert rows (moe_logits_body)
 };
 
 // Column activations of a mixture pass: column c reads x[src(c)] (or silu(x[src(c)]) *

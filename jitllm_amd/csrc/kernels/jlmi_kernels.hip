@@ -348,7 +348,8 @@ extern "C" __global__ __launch_bounds__(256, 2) void jl_gemm_q4k_w16(GemmW16Args
 extern "C" __global__ __launch_bounds__(64) void jl_moe_route(MoeRouteArgs p) { moe_route_body<16>(p); }
 extern "C" __global__ __launch_bounds__(64) void jl_moe_route_g2(MoeRouteArgs p) { moe_route_body<2>(p); }
 extern "C" __global__ __launch_bounds__(64) void jl_moe_route_g4(MoeRouteArgs p) { moe_route_body<4>(p); }
-// grid = (token groups, 8 at most, experts, ceil(token groups / 8)), block = 128; a group is JL_LOGITS_TOK tokens
+// grid = (token groups, 8 at most, experts, ceil(token groups / 8)), by_expert: (experts, token groups); block = 128; a group is
+// JL_LOGITS_TOK tokens
 extern "C" __global__ __launch_bounds__(128) void jl_moe_logits(MoeLogitsArgs p) {
     __shared__ float part[JL_LOGITS_TOK * 128];
     moe_logits_body<1>(p, part);

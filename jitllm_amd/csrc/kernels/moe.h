@@ -1564,13 +1564,15 @@ __device__ __forceinline__ void moe_gather_down_body(const MoeGatherDownArgs& ar
 // JL_LOGITS_TOK tokens: the row is read once for all of them.
 // With many tokens the launch is bound by re-reading x from L2 for every expert row (2048
 // tokens x 128 experts x k = 2048: 88 us), so there a workgroup takes EB = 8 expert rows
-// for its eight tokens and every x value loaded meets eight weights (grid.x = ceil(rows/EB)): 34 us, a
+// for its eight tokens and every x value loaded meets eight weights: 34 us, a
 // product and a sum an instruction each (12 us of issue), four wavefronts a SIMD.
 #define JL_LOGITS_TOK 8
 template <int EB, bool F16 = false>
 __device__ __forceinline__ void moe_logits_body(const MoeLogitsArgs& p, float* part) {
-    // (workgroups go round the eight XCDs in the order of their ids: a token group's rows of x are fetched into one L2)
-    const int r0 = blockIdx.y * EB, t0 = (blockIdx.x + 8 * blockIdx.z) * JL_LOGITS_TOK, tid = threadIdx.x;
+    // (workgroups go round the eight XCDs in the order of their ids: a token group's rows of x, or the rows of every eighth group
+    // of experts, are fetched into one L2)
+    const int r0 = (p.by_expert ? blockIdx.x : blockIdx.y) * EB, t0 = (p.by_expert ? blockIdx.y : blockIdx.x + 8 * blockIdx.z) * JL_LOGITS_TOK;
+    const int tid = threadIdx.x;
     if (t0 >= p.ntok) return;   // uniform
     const int nt = min(JL_LOGITS_TOK, p.ntok - t0), k = p.k;
     float acc[EB][JL_LOGITS_TOK];

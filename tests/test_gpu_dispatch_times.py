@@ -1,6 +1,8 @@
 """What a rule takes by itself is about as fast as the best of the forms it could have taken, where a rule once was not: device time of
 calls queued behind a wait, the fastest of several windows of either in turn.  The limits are half of what the wrong pick cost, several
 times what two measurements of one launch differ."""
+import itertools
+
 import numpy as np
 import pytest
 
@@ -78,3 +80,20 @@ def test_token_tiles_of_a_group(dev, devbuf, t, window, n_expert, nrows, k, nmat
         assert got["auto"] <= 1.1 * min(got[nt] for nt in (2, 3, 4)), got
     finally:
         dev.SetActWindow(32)
+
+
+@pytest.mark.parametrize("wdt,n_expert,k,ntok,rows", [("f16", 256, 7168, 16, 1), ("f32", 384, 7168, 2048, 8), ("f32", 128, 2048, 2048, 8)])
+def test_order_of_the_router_s_grid(dev, devbuf, wdt, n_expert, k, ntok, rows):
+    """Token groups or rows of the router side by side (tuning 16 / 32 + rows a workgroup): one where an L2 does not hold the router, a
+    large router with few tokens, and a small one with many."""
+    w = np.random.default_rng(1).standard_normal((n_expert, k)).astype(np.float16 if wdt == "f16" else np.float32)
+    x = np.random.default_rng(2).standard_normal((ntok, k)).astype(np.float32)
+    wd, xd, ld = [devbuf(w) for _ in range(3)], [devbuf(x) for _ in range(3)], devbuf(shape=(ntok, n_expert), dtype=np.float32)
+    turn = itertools.count()   # (copies in turn, past what an L2 still holds)
+
+    def call():
+        i = next(turn) % 3
+        return dev.moe_logits_dev(ld.ptr, 1 if wdt == "f16" else 0, wd[i].ptr, xd[i].ptr, n_expert, k, ntok)
+
+    got = us(dev, {"auto": ({}, call), "tokens": (dict(moe__logits=16 + rows), call), "rows": (dict(moe__logits=32 + rows), call)})
+    assert got["auto"] <= 1.08 * min(got["tokens"], got["rows"]), got

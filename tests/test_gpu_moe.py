@@ -536,6 +536,29 @@ def test_router_logits_by_two_and_four_rows(dev, devbuf, case, form):
     assert np.array_equal(got[:ntok * n_expert].view(np.uint32), np.ascontiguousarray(want).reshape(-1).view(np.uint32))
 
 
+@pytest.mark.parametrize("order", [16, 32], ids=["tokens", "rows"])
+@pytest.mark.parametrize("case", [(1, 1, 4, 1, "f32"), (65, 9, 255, 1, "f16"), (73, 13, 130, 2, "f32"), (64, 17, 384, 4, "f16"), (130, 66, 129, 8, "f32")],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_router_logits_in_either_order(dev, devbuf, case, order):
+    """Token groups or rows of the router side by side: counts of neither that fill a group; the oracle's bits."""
+    ntok, n_expert, k, rows, wdt = case
+    rng = np.random.default_rng(ntok + n_expert)
+    w = rng.standard_normal((n_expert, k)).astype(np.float32)
+    x = rng.standard_normal((ntok, k)).astype(np.float32)
+    w = w.astype(np.float16).view(np.uint16) if wdt == "f16" else w
+    want = oracle.router_logits(w, x, n_expert, k, ntok)
+    wd, xd, ld = devbuf(w), devbuf(x), devbuf(shape=(ntok * n_expert + 3,), dtype=np.float32, fill=np.float32(7e30))
+    dev.set_tuning(moe__logits=order + rows)
+    try:
+        assert dev.moe_logits_dev(ld.ptr, 1 if wdt == "f16" else 0, wd.ptr, xd.ptr, n_expert, k, ntok)
+        dev.synchronize()
+    finally:
+        dev.set_tuning(moe__logits=0)
+    got = ld.get()
+    assert np.all(got[ntok * n_expert:] == np.float32(7e30))
+    assert np.array_equal(got[:ntok * n_expert].view(np.uint32), np.ascontiguousarray(want).reshape(-1).view(np.uint32))
+
+
 def _pack_bank(dev, devbuf, t, bank, n_expert, nrows, k, layout):
     """A GGUF bank -> packed planes on the device.  layout "sheets": every expert's sheet packed
     on its own, plane sets `page` bytes apart as a container's expert pages are
