@@ -961,12 +961,17 @@ I8Plan gemm_i8_plan(const jl_ctx* c, int type, int nrows, int k, int ntok) {
             if (left) us += 0.15 + std::max(h.many * waves * ((left + c->num_cu - 1) / c->num_cu), h.alone) * block;
             if (s > 1) us += 0.25 + 1.16e-6 * (s + 1) * n;
             // 256 tokens x 128 rows: a last round of at most half of the CUs gives its rows to tiles of 64 instead, which take 0.59 of a
-            // tile's time and fill it (2048 tokens of 14336 x 4096, 3.5 rounds: 334 -> 322)
+            // tile's time and fill it (17 shapes whose tiles are these anyway, K 256 to 2688: 0.94 of the time on average, none more than 0.97;
+            // 2048 tokens of 14336 x 4096, 3.5 rounds, 334 -> 322).  With it these tiles take over from the others from K = 1536 on alone
+            // (23 shapes 0.93, none slower; below, 20 shapes, 0.86 to 1.14: a short chain's start, which the estimate leaves out, is longer here).
             int high = 1 << 24;
             if (h.tw == 8 && s == 1 && full && left && c->tune.gemm_tall != 1) {
                 const long ttiles = (ntok + 255) / 256, tall_n = full * c->num_cu / ttiles, low = ((nrows - 128 * tall_n + 63) / 64) * ttiles;
                 const double mixed = full * (0.15 + h.many * waves * block) + 0.15 + 0.59 * h.many * waves * block;
-                if (low <= c->num_cu && mixed < us) us = mixed, high = (int)tall_n;
+                if (low <= c->num_cu && mixed < us) {
+                    high = (int)tall_n;
+                    if (k >= 1536) us = mixed;
+                }
             }
             if (us < best) { best = us; f = {rt, h.tw}; nsplit = s; tall = high; }
         }

@@ -97,3 +97,26 @@ def test_order_of_the_router_s_grid(dev, devbuf, wdt, n_expert, k, ntok, rows):
 
     got = us(dev, {"auto": ({}, call), "tokens": (dict(moe__logits=16 + rows), call), "rows": (dict(moe__logits=32 + rows), call)})
     assert got["auto"] <= 1.08 * min(got["tokens"], got["rows"]), got
+
+
+@pytest.mark.parametrize("nrows,k,ntok,gains", [(11009, 512, 1535, False), (14336, 1024, 2048, True)])
+def test_tail_of_64_rows_by_itself(dev, devbuf, nrows, k, ntok, gains):
+    """Q8_0: where the rows of a last round go to tiles of 64 rows, which gives the bits of the tiles of 128 rows and is faster, and where
+    it must not take the call from another tile."""
+    dev.SetActWindow(32)
+    w, x = random_bank(devbuf, quant.Q8_0, 1, nrows, k), devbuf(np.random.default_rng(1).standard_normal((ntok, k)).astype(np.float32))
+    o = devbuf(shape=(ntok, nrows), dtype=np.float32)
+
+    def call():
+        return dev.matmul_dev(o.ptr, quant.Q8_0, w.ptr, x.ptr, nrows, k, ntok)
+
+    got = us(dev, {"auto": ({}, call), "flat": (dict(gemm__tall=1), call)}, 20)
+    assert got["auto"] <= (0.98 if gains else 1.05) * got["flat"], got
+    values = []
+    for tall in (0, 1):
+        dev.set_tuning(gemm__tall=tall)
+        assert call()
+        dev.synchronize()
+        dev.set_tuning(gemm__tall=0)
+        values.append(o.get())
+    assert np.array_equal(values[0].view(np.uint32), values[1].view(np.uint32))
