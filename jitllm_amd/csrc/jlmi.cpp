@@ -963,7 +963,7 @@ I8Plan gemm_i8_plan(const jl_ctx* c, int type, int nrows, int k, int ntok) {
             // 256 tokens x 128 rows: a last round of at most half of the CUs gives its rows to tiles of 64 instead, which take 0.59 of a
             // tile's time and fill it (17 shapes whose tiles are these anyway, K 256 to 2688: 0.94 of the time on average, none more than 0.97;
             // 2048 tokens of 14336 x 4096, 3.5 rounds, 334 -> 322).  With it these tiles take over from the others from K = 1536 on alone
-            // (23 shapes 0.93, none slower; below, 20 shapes, 0.86 to 1.14: a short chain's start, which the estimate leaves out, is longer here).
+            // (25 shapes 0.93, none slower; below, 18 shapes, 0.96 to 1.14: a short chain's start, which the estimate leaves out, is longer here).
             int high = 1 << 24;
             if (h.tw == 8 && s == 1 && full && left && c->tune.gemm_tall != 1) {
                 const long ttiles = (ntok + 255) / 256, tall_n = full * c->num_cu / ttiles, low = ((nrows - 128 * tall_n + 63) / 64) * ttiles;
@@ -3404,7 +3404,17 @@ int mx_one_rows(const jl_ctx* c, int nrows, int k, int ntok, bool planes) {
     const int rt = us1 <= us2 ? 1 : 2;
     double other;
     if (ntok <= 8 && !mx_few_applies(c, nrows, k, ntok, planes)) {
-        if (planes) return rt;
+        if (planes) {
+            // Two tokens over many rows: the plane matvec's rounds of 64 rows a workgroup (fitted to 16384 x 1024 to 201088 x 2880, 5 % where it
+            // decides), where LDS leaves this form one workgroup a CU.  us, matvec / so: 32768 x 2880 19.6 / 21.3, 65536 x 2880 36.5 / 40.2, 201088 x
+            // 2880 100 / 123; 28672 x 4096 26.4 / 25.7, 14336 x 4096 15.2 / 14.1, 8448 x 8192 30.4 / 19.0, 512 x 14336 13.3 / 9.7, and with two
+            // workgroups a CU 65536 x 2048 27.6 / 22.0.  From three tokens on this form is never behind (65536 x 2880 44.9 / 40.8).  No guard for long
+            // rows: it rounds less at every K (NMSE, 8 tokens, 1024 x 5760 2.7e-15, the matvec 4.6e-15, 4096 x 14336 4.4e-15, 6.5e-15).
+            const long r64 = (nrows + 63) / 64;
+            if (ntok > 2 || 2 * JL_MX_ONE_LDS(k, nt) <= 160 * 1024 || r64 * 10 < c->num_cu * 7) return rt;
+            const double full64 = (double)r64 / c->num_cu;
+            return us <= 2.5 + 3.0 * kk * (full64 < 2 ? std::ceil(full64) : 0.5 * (full64 + std::ceil(full64))) ? rt : 0;
+        }
         if (k > 4096) return 0;   // (the decode matvec rounds less there: 5760 x 5760, NMSE 2.35e-15 against 2.61)
         const long r4 = ((nrows + 3) / 4 + (long)c->num_cu - 1) / c->num_cu;
         other = (3.2 + ntok * (0.1 + 0.13e-3 * k * r4)) / 1.08;

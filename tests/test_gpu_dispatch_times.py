@@ -120,3 +120,26 @@ def test_tail_of_64_rows_by_itself(dev, devbuf, nrows, k, ntok, gains):
         dev.set_tuning(gemm__tall=0)
         values.append(o.get())
     assert np.array_equal(values[0].view(np.uint32), values[1].view(np.uint32))
+
+
+def mxfp4_planes(devbuf, nrows, k, ntok):
+    from jitllm_amd.device import Packed
+    rng = np.random.default_rng(1)
+    nq, nd, _ = quant.packed_words(quant.MXFP4, nrows, k)
+    qs = devbuf(rng.integers(0, 1 << 32, nq, dtype=np.uint32))
+    d = devbuf(np.full(nd, 0x78787878, np.uint32))
+    x = devbuf((rng.standard_normal((ntok, k)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16))
+    return qs, d, x, devbuf(shape=(ntok, nrows), dtype=np.float32), Packed(qs.ptr, d.ptr, None, 0, nrows)
+
+
+@pytest.mark.parametrize("nrows,k", [(201088, 2880), (8448, 8192), (1024, 5760)], ids=str)
+def test_mxfp4_planes_two_tokens(dev, devbuf, nrows, k):
+    """The plane matvec where its rounds are the shorter ones, else the one-launch form: a tall matrix, one whose matvec leaves half of
+    the CUs idle, a small one of long rows."""
+    qs, d, x, o, p = mxfp4_planes(devbuf, nrows, k, 2)
+
+    def call():
+        return dev.matmul_mxfp4_packed_bf16_dev(o.ptr, p, x.ptr, nrows, k, 2)
+
+    got = us(dev, {"auto": ({}, call), "matvec": (dict(mxfp4__one=1), call), "one": (dict(mxfp4__one=11), call), "one of 32 rows": (dict(mxfp4__one=12), call)}, 20)
+    assert got["auto"] <= 1.07 * min(got.values()), got
