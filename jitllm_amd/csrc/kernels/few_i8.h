@@ -255,13 +255,17 @@ __device__ __forceinline__ void few_blocks(const FewR<TYPE, PL>* R, const float*
         for (int rt = 0; rt < RT; rt++)
 #pragma unroll
             for (int t = 0; t < NT; t++) { P[rt][t] = zero; M[rt][t] = zero; }
+    // (planes, four token tiles: a row tile's four blocks one after the other, so that one tile's sums are held, 168 registers for 175
+    // and three wavefronts a SIMD for two)
+    constexpr int OUTER = SUMS && PL && NT == 4 ? RT : 1, INNER = RT / OUTER;
 #pragma unroll
-    for (int s = 0; s < 4; s++) {
+    for (int u = 0; u < 4 * OUTER; u++) {
+        const int s = u & 3;
         // (block by block: the compiler would gather the scale reads and decodes of all four, and sink
         // the sums' arithmetic behind the loop: registers)
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++) {
+        for (int rt = (u >> 2) * INNER; rt < ((u >> 2) + 1) * INNER; rt++) {
             const u32x2 b = few_decode<TYPE, PL>(R[rt], s, g);
             const float* scr = sc + rt * (JL_FEW_SC_BYTES / 4);
             if constexpr (TYPE == JL_Q6_K) {
@@ -277,6 +281,10 @@ __device__ __forceinline__ void few_blocks(const FewR<TYPE, PL>* R, const float*
                         if constexpr (W256) P[rt][t][i] += v;
                         else sum[rt][t][i] = fmaf((float)v, X[t].da[s], sum[rt][t][i]);
                     }
+                    // (the products of four tiles in flight made 129 registers, and 128 are two workgroups of eight wavefronts a CU: planes
+                    // 2401 x 1280, 151 tokens 14.6 us, so 12.1)
+                    if constexpr (SUMS && PL && NT == 4 && RT == 1)
+                        if (t == 1) __builtin_amdgcn_sched_barrier(0);
                 }
             } else if constexpr (TYPE == JL_Q4_K && W256) {
                 const i32x4 s4 = ((const i32x4*)scr)[s * 4 + g], m4 = ((const i32x4*)(scr + 64))[s * 4 + g];
@@ -312,9 +320,21 @@ __device__ __forceinline__ void few_blocks(const FewR<TYPE, PL>* R, const float*
                 if constexpr (W256 && TYPE == JL_Q4_K) asm volatile("" : "+v"(M[rt][t]));
             }
         }
+        if constexpr (OUTER > 1)
+            if (s == 3) {
+                const int rt = u >> 2;
+                __builtin_amdgcn_sched_barrier(0);
+                const f32x4 d4 = ((const f32x4*)(sc + rt * (JL_FEW_SC_BYTES / 4) + 128))[g];
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[rt][t][i] = fmaf(sum[rt][t][i], d4[i], acc[rt][t][i]);
+                    asm volatile("" : "+v"(acc[rt][t]));
+                }
+            }
     }
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (SUMS)
+    if constexpr (SUMS && OUTER == 1)
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
             const f32x4 d4 = ((const f32x4*)(sc + rt * (JL_FEW_SC_BYTES / 4) + 128))[g];

@@ -163,7 +163,8 @@ JL_MATVEC_TOKENS_LANES(q6kw, JL_Q6_KW, 32) JL_MATVEC_TOKENS_LANES(q6kw, JL_Q6_KW
 extern "C" __global__ __launch_bounds__(256) void jl_few_prep(FewI8PrepArgs p) { few_i8_prep_body(p); }
 // jl_few_<type>_<rows | planes>_t<token tiles>r<row tiles>: grid = (row tiles, experts, matrices)
 #define JL_FEW_KERNEL(T, TYPE, P, PL, NT, RT, W256)                                                             \
-    extern "C" __global__ __launch_bounds__(512) void jl_few_##T##_##P##_t##NT##r##RT(FewI8Args p) {            \
+    extern "C" __global__ __launch_bounds__(512, TYPE == JL_Q6_K && !W256 && PL && NT == 4 && RT == 2 ? 3 : 2)  \
+    void jl_few_##T##_##P##_t##NT##r##RT(FewI8Args p) {                                                         \
         few_i8_body<TYPE, PL, NT, RT, W256>(p, jl_smem);                                                        \
     }
 #define JL_FEW_SIZES(T, TYPE, P, PL, W256)                                                                      \

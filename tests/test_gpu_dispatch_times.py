@@ -143,3 +143,21 @@ def test_mxfp4_planes_two_tokens(dev, devbuf, nrows, k):
 
     got = us(dev, {"auto": ({}, call), "matvec": (dict(mxfp4__one=1), call), "one": (dict(mxfp4__one=11), call), "one of 32 rows": (dict(mxfp4__one=12), call)}, 20)
     assert got["auto"] <= 1.07 * min(got.values()), got
+
+
+@pytest.mark.parametrize("kernel,waves", [("jl_few_q6k_planes_t4r1", 4), ("jl_few_q6k_planes_t4r2", 3)])
+def test_wavefronts_a_simd_holds(dev, kernel, waves):
+    """Kernels a register or seven past a step of the register file: it holds 512 a lane, and a workgroup of eight wavefronts takes two on
+    each SIMD, so that one wavefront fewer can be half of a CU's workgroups."""
+    import ctypes as C
+
+    from jitllm_amd import _lib
+    from jitllm_amd.hipmem import check, hip
+    module, function, regs = C.c_void_p(), C.c_void_p(), C.c_int()
+    check(hip().hipModuleLoad(C.byref(module), _lib.CODE_OBJECT_PATH.encode()), "hipModuleLoad")
+    try:
+        check(hip().hipModuleGetFunction(C.byref(function), module, kernel.encode()), kernel)
+        check(hip().hipFuncGetAttribute(C.byref(regs), 4, function), kernel)   # HIP_FUNC_ATTRIBUTE_NUM_REGS
+    finally:
+        check(hip().hipModuleUnload(module), "hipModuleUnload")
+    assert 512 // (-(-regs.value // 8) * 8) >= waves, regs.value
