@@ -1860,11 +1860,13 @@ int moe_matvec_launch(jl_ctx* c, float* out0, float* out1, int type, const void*
     //   Q6_K window 256   2: 48/20/18 -> 47/19/14   8: 67/27/30 -> 59/21/15   48: 179/47/48 -> 111/38/28    128: 238/81/56 -> 183/61/43
     // The few-token kernel reads an expert's sheet once for 16 to 64 columns (few_shape) and the columns once for every row tile, so it
     // gives way to the tiles where the columns are the more; a tile of 64 columns needs two workgroups a CU.  From 40 columns on
-    // (52 for Q6_K's rows of up to 1024), window 32, Q8_0 takes tiles of 128 columns, Q6_K of 64, Q4_K from 56 on 128.  us, few-token kernel / tiles: Q8_0 60 x 1280 x 2048 twice, 40 columns 127 / 140, 46
-    // 156 / 141, 60 x 2048 x 1280, 42 columns 101 / 82; Q6_K 128 x 2048 x 768, 46 columns 135 / 131, 100 x 512 x 1024 47 / 52, 60 x 2048 x 1280
-    // 150 / 102.  Tiles of 64 columns were Q8_0's and Q4_K's too: blocks of 128 experts of 768 x 2048, 54 columns 348 (321 on 128) and, spilling,
-    // 1912 (few-token kernel 410).  (Q8_0's and Q4_K's tiles of 128 would be faster earlier for long rows; their one chain of sums rounds more
-    // than the few-token kernel's.)  With a
+    // (52 for Q6_K's rows of up to 1024), window 32, Q8_0 takes tiles of 128 columns, Q6_K of 64, Q4_K from 56 on 128.  us, few-token kernel /
+    // tiles: Q8_0 60 x 1280 x 2048 twice, 40 columns 127 / 140, 46 156 / 141, 60 x 2048 x 1280, 42 columns 101 / 82; Q6_K 60 x 2048 x 1280, 46 columns
+    // 150 / 102; K up to 1024, 48 / 53 columns: 128 x 2048 x 768 135 / 126, 140 / 133, 128 x 2880 x 768 193 / 182, 199 / 184, 60 x 1536 x 1024 twice
+    // 127 / 122, 129 / 131, 128 x 1024 x 1024 94 / 90, 99 / 104, 32 x 2048 x 768 38 / 37, 40 / 49, 128 x 2048 x 512 95 / 100, 100 / 104, 60 x 2048 x 512 46 /
+    // 50, 47 / 56.  Tiles of 64 columns were Q8_0's and Q4_K's too: blocks of 128 experts of 768 x 2048, 54 columns 348 (321 on 128) and, spilling,
+    // 1912 (few-token kernel 410).  (The tiles would be faster earlier in places, for long rows and in the largest Q6_K banks; their one chain of
+    // sums rounds more than the few-token kernel's.)  With a
     // column or two an expert Q6_K's dot-product kernel is as fast while rows are short.  Q4_K with the k-quant window
     // has the forms below, and the few-token kernel where moe_few_faster finds it faster.
     {
@@ -3337,10 +3339,11 @@ MxRowsPlan mx_rows_plan(const jl_ctx* c, int nrows, int k, int ntok) {
 
 // Few tokens: 16-row workgroups whose wavefronts split K, in chunks of up to 64 tokens, one launch after a prep
 // that lays the activations out in the order the block decode produces.
-// (The same tiles in one launch come first, mx_one_rows.)  From where: the kernels for a handful of tokens grow with the tokens, this one does not, but it is two launches, which a
-// host that issues calls one after the other cannot do in less than 6.7 us.  From three tokens, so, where the one launch
-// is estimated to take more than that and more than this form: over rows a token costs what a round of their workgroups
-// does, four rows each, on all CUs, over planes what K and the matrix do (fitted to 17 shapes, 512 x 512 to 12288 x 2048,
+// (The same tiles in one launch come first, mx_one_rows.)  From where: the kernels for a handful of tokens grow with the
+// tokens, this one does not, but it is two launches, which a host that issues calls one after the other cannot do in less
+// than 6.7 us.  From three tokens, so, where the one launch is estimated to take more than that and more than this form:
+// over rows a token costs what a round of their workgroups does, four rows each, on all CUs, over planes what K and the
+// matrix do (fitted to 17 shapes, 512 x 512 to 12288 x 2048,
 // 2 to 8 tokens, 6 % each).  Device us, these against this one: rows 2880 x 2880, 3 and 5 tokens 6.5 and 6.8, 8.9 and 6.9,
 // 5760 x 2880, 3 tokens 11.3 and 9.3; planes 5760 x 2880, 3 tokens 9.1 and 7.0, 3413 x 1536, 5 and 8 tokens 6.0 and 5.4,
 // 7.5 and 5.4.  (By device time alone it would begin earlier: planes 2124 x 1120, 5 tokens 5.5 and 4.7, but call by call

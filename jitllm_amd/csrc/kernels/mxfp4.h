@@ -1017,7 +1017,7 @@ __device__ __forceinline__ void mx_few_body(const MxGemmArgs& args, float* part)
 // row r = lane % 16, kq = lane / 16) supplies elements 8 c .. 8 c + 7 of block 4 G + kq, one piece of the activations and,
 // of the weights, the low (c < 2) or high nibbles of code words 2 (c % 2) and 2 (c % 2) + 1.
 //
-// What bounds it: the trips -- weights and the first groups' activations, asked for together, then NBUF groups a trip -- and
+// What bounds it: the trips -- weights and the first groups' activations, asked for together, then four token tiles of a group a trip -- and
 // the activations, of which every workgroup brings all to its CU (2880 x 2880, 64 tokens: 369 KB, 2.4 us of L1's 64 bytes a
 // cycle).
 //

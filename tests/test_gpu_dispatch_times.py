@@ -145,6 +145,17 @@ def test_mxfp4_planes_two_tokens(dev, devbuf, nrows, k):
     assert got["auto"] <= 1.07 * min(got.values()), got
 
 
+@pytest.mark.parametrize("packed,nrows,k,ntok", [(True, 2880, 2880, 64), (True, 5760, 5760, 16), (False, 2880, 2880, 16), (False, 2880, 2880, 128)])
+def test_mxfp4_one_launch_by_itself(dev, devbuf, packed, nrows, k, ntok):
+    """A few tokens take the form without a prep launch, whichever of its widths, unasked."""
+    qs, d, x, o, p = mxfp4_planes(devbuf, nrows, k, ntok)
+    w = None if packed else devbuf(synth.random_weights(quant.MXFP4, nrows, k, seed=1))
+    n0 = dev.launch_count()
+    assert dev.matmul_mxfp4_packed_bf16_dev(o.ptr, p, x.ptr, nrows, k, ntok) if packed else dev.matmul_mxfp4_bf16_dev(o.ptr, w.ptr, x.ptr, nrows, k, ntok)
+    dev.synchronize()
+    assert dev.launch_count() - n0 == 1
+
+
 @pytest.mark.parametrize("kernel,waves", [("jl_few_q6k_planes_t4r1", 4), ("jl_few_q6k_planes_t4r2", 3)])
 def test_wavefronts_a_simd_holds(dev, kernel, waves):
     """Kernels a register or seven past a step of the register file: it holds 512 a lane, and a workgroup of eight wavefronts takes two on

@@ -65,7 +65,8 @@ def test_tiles_per_expert(dev, devbuf, t, window, nrows, k):
                     cols = slice(start[e], start[e + 1])
                     if counts[e]:
                         want[b][cols] = oracle.matmul_q8act_f64(t, banks[b][e * sheet:(e + 1) * sheet], act[src[cols]], nrows, k, counts[e], window)
-            for form in (0, 5, 6, 7, 8) if t == quant.Q8_0 else (0, 5, 6, 7):
+            # (8: Q8_0's tiles of 128 x 128; 7: Q6_K's of 64 columns, window 32)
+            for form in (0, 5, 6) + ((8,) if t == quant.Q8_0 else (7,) if t == quant.Q6_K and window == 32 else ()):
                 dev.set_tuning(moe__form=form)
                 o = [devbuf(shape=(ncols * nrows + 8,), dtype=np.float32, fill=FILL) for _ in banks]
                 assert dev.moe_matvec_dev(o[0].ptr, o[1].ptr, t, bd[0].ptr, bd[1].ptr, xd.ptr, ud.ptr if gated else None, sd.ptr, dstart.ptr,
@@ -77,7 +78,7 @@ def test_tiles_per_expert(dev, devbuf, t, window, nrows, k):
                     # (the gated activation: an exponential of another machine in front of the quantizer)
                     assert nmse(got[:ncols * nrows].reshape(ncols, nrows), want[b]) <= (1e-6 if gated else 1e-10), (gated, form, b)
     finally:
-        dev.set_tuning(moe__form=0, few__nt=0)
+        dev.set_tuning(moe__form=0)
         dev.SetActWindow(32)
 
 
@@ -172,7 +173,7 @@ def test_scales_that_are_no_numbers(dev, devbuf, t, ntok):
                 o = devbuf(shape=(ntok * nrows + 8,), dtype=np.float32, fill=FILL)
                 assert dev.matmul_dev(o.ptr, t, wd.ptr, xd.ptr, nrows, k, ntok)
                 check(o, (few, shape, split))
-            for form in (0, 5, 6, 7, 8) if t == quant.Q8_0 else (0, 5, 6, 7):
+            for form in (0, 5, 6, 8) if t == quant.Q8_0 else (0, 5, 6):
                 dev.set_tuning(gemm__few=0, gemm__i8=0, gemm__split=0, moe__form=form)
                 o = devbuf(shape=(ntok * nrows + 8,), dtype=np.float32, fill=FILL)
                 assert dev.moe_matvec_dev(o.ptr, None, t, bank.ptr, None, xd.ptr, None, None, start.ptr, 2, ntok, nrows, k)
