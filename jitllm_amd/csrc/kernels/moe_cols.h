@@ -114,30 +114,33 @@ __device__ __forceinline__ void mc_store(const MoeColsArgs& p, const f32x16 (&ou
         }
 }
 
-// Asks for a super-block of a Q4_K tile's rows; w: a lane's places among the rows' bytes.
+// A lane's places among a Q4_K tile's rows: 18 instructions of 64 pieces, nine pieces a row; four a wavefront, the last two the first two
+// wavefronts'.
 struct MoeColsQ4Rows { u32 woff[4], xoff; };
-__device__ __forceinline__ void moe_cols_q4_rows(const MoeColsArgs& p, uint8_t* smem, const uint8_t* sheet, int last, MoeColsQ4Rows& w) {
-    constexpr int O_W = 2 * JL_MC_A;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const u32 lds0 = lds_address(smem);
-    // 18 instructions of 64 pieces, nine pieces a row; four a wavefront, the last two the first two wavefronts'
+__device__ __forceinline__ void moe_cols_q4_places(const MoeColsArgs& p, int last, MoeColsQ4Rows& w) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     auto piece_at = [&](int i) {
         const int idx = 64 * i + lane, row = idx / 9;
         return (u32)min(row, last) * (u32)p.row_bytes + 16 * (u32)(idx - 9 * row);
     };
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        w.woff[i] = piece_at(4 * wave + i);
-        load_lds16(sheet, w.woff[i], __builtin_amdgcn_readfirstlane(lds0 + O_W + 4096 * wave + 1024 * i));
-    }
+    for (int i = 0; i < 4; i++) w.woff[i] = piece_at(4 * wave + i);
     w.xoff = piece_at(16 + (wave & 1));
+}
+// Asks for the first super-block's rows.
+__device__ __forceinline__ void moe_cols_q4_rows(uint8_t* smem, const uint8_t* sheet, const MoeColsQ4Rows& w) {
+    constexpr int O_W = 2 * JL_MC_A;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const u32 lds0 = lds_address(smem);
+#pragma unroll
+    for (int i = 0; i < 4; i++) load_lds16(sheet, w.woff[i], __builtin_amdgcn_readfirstlane(lds0 + O_W + 4096 * wave + 1024 * i));
     if (wave < 2) load_lds16(sheet, w.xoff, __builtin_amdgcn_readfirstlane(lds0 + O_W + 1024 * (16 + wave)));
 }
 // Q4_K rows.  G: groups of 32 columns (n columns exist).  The rows' bytes come to LDS as they lie, 144 contiguous bytes a
 // row (straight into registers, a lane a row, is sixteen bytes of 64 lines an instruction), and each wavefront reads its own.
-// w: the places, and the first super-block's rows already asked for.
+// asked: the first super-block's rows are already on their way.
 template <int G>
-__device__ __forceinline__ void moe_cols_q4_tile(const MoeColsArgs& p, uint8_t* smem, const uint8_t* sheet, const MoeColsQ4Rows& w, int mat, int r0, u32 c0, int n) {
+__device__ __forceinline__ void moe_cols_q4_tile(const MoeColsArgs& p, uint8_t* smem, const uint8_t* sheet, const MoeColsQ4Rows& w, bool asked, int mat, int r0, u32 c0, int n) {
     constexpr int O_W = 2 * JL_MC_A, O_AUG = O_W + 2 * JL_MC_W, O_DA = O_AUG + 2 * 64 * 32;
     constexpr int NA = 2 * G;   // a wavefront's instructions for half a super-block of columns; NS: for its weights, sums, scales
     constexpr int NS = 5;
@@ -178,6 +181,7 @@ __device__ __forceinline__ void moe_cols_q4_tile(const MoeColsArgs& p, uint8_t* 
         if (wave == 0) load_lds4((const uint8_t*)p.da + (size_t)sb * 4, doff, __builtin_amdgcn_readfirstlane(lds0 + O_DA + (sb & 1) * 256));
     };
     load_a(0);
+    if (!asked) moe_cols_q4_rows(smem, sheet, w);   // uniform
     load_w(0, GemmIntC<0>{});
     f32x16 out[G], acc[G];
     const f32x16 zero = {0.f};
@@ -590,17 +594,19 @@ __device__ __forceinline__ void moe_cols_body(const MoeColsArgs& p, uint8_t* sme
     const int mat = __builtin_amdgcn_readfirstlane((int)(i2 % (u32)p.nmat)), e = __builtin_amdgcn_readfirstlane((int)(i2 / (u32)p.nmat));
     const int r0 = __builtin_amdgcn_readfirstlane((int)rb * 128);
     const uint8_t* sheet = p.bank[mat] + (size_t)e * p.sheet_bytes + (size_t)r0 * p.row_bytes;
-    const u32 c_hi = p.start[e + 1];
-    for (u32 c0 = p.start[e] + 64 * z; c0 < c_hi; c0 += 64 * (u32)p.shares) {   // uniform
+    MoeColsQ4Rows w4;
+    if constexpr (KO == 0) moe_cols_q4_places(p, p.nrows - 1 - r0, w4);
+    const u32 c_hi = p.start[e + 1], c_lo = p.start[e] + 64 * z;
+    for (u32 c0 = c_lo; c0 < c_hi; c0 += 64 * (u32)p.shares) {   // uniform
         const int n = (int)min(64u, c_hi - c0);
-        // The rows' bytes are asked for ahead of the columns, which wait for the records' numbers.  Ahead of start as well they save even
-        // routing nothing (1.00, 55 banks and column counts), and a workgroup without columns, which brings 18 KB for nothing, costs uneven
-        // routing: 128 experts of 2048 x 768, eight of them with columns, 32 an expert on average 84 us, so 64; half of the experts 53 and 50.
-        MoeColsQ4Rows w4;
-        if constexpr (KO == 0) moe_cols_q4_rows(p, smem, sheet, p.nrows - 1 - r0, w4);
+        // The rows' bytes, from memory the first time, are asked for ahead of the columns, which wait for the records' numbers.  Ahead of start as
+        // well they save even routing nothing (1.00, 55 banks and column counts), and a workgroup without columns, which brings 18 KB for
+        // nothing, costs uneven routing: 128 experts of 2048 x 768, eight of them with columns, 32 an expert on average 84 us, so 64; half of the
+        // experts 53 and 48.
+        if (KO == 0 && c0 == c_lo) moe_cols_q4_rows(smem, sheet, w4);
         auto tile = [&](auto G) __attribute__((always_inline)) {
             constexpr int g = decltype(G)::value;
-            if constexpr (KO == 0) moe_cols_q4_tile<g>(p, smem, sheet, w4, mat, r0, c0, n);
+            if constexpr (KO == 0) moe_cols_q4_tile<g>(p, smem, sheet, w4, c0 == c_lo, mat, r0, c0, n);
             else if constexpr (KO == 1) moe_cols_planes_tile<g>(p, smem, e, mat, r0, c0, n);
             else moe_cols_q6_tile<g>(p, smem, e, mat, r0, c0, n);
         };
