@@ -2777,12 +2777,15 @@ int jl_moe_logits_dev(jl_ctx* c, float* logits, int wtype, const void* w, const 
     }
     const unsigned groups = (unsigned)(ntok + 7) / 8, blocks = (unsigned)(n_expert + eb - 1) / eb;   // JL_LOGITS_TOK
     // Workgroups go round the XCDs in the order of their numbers.  Token groups side by side bring each its rows of x to one L2, and every
-    // row of the router to all; rows of the router side by side bring each to one L2, and x to all.  The first where many tokens meet a router that an L2
-    // holds (4 MB), the second where it does not, and for a few tokens where the router is large.  us, token groups / rows: 384 x 7168 in f32,
-    // 2048 tokens 334 / 265, 256 x 7168 192 / 181, 128 x 7168 93 / 100; 256 x 7168 in f16, 16 tokens 21.7 / 13.7, 160 x 5120 in f16, 32 tokens
-    // 16.3 / 11.2, in f32 16 tokens 8.4 / 7.6; 128 x 2048 in f32, 128 tokens 6.4 / 7.3.  (275 shapes: 0.4 % behind the better order.)
+    // row of the router to all; rows of the router side by side bring each to one L2, and x to all.  Many tokens: the first, unless the router is
+    // more than an L2 holds (4 MB).  Up to 64: the second where the router is large, in f32 with a row a workgroup only while the workgroups are few.
+    // us, token groups / rows: 384 x 7168 in f32, 2048 tokens 334 / 265, 256 x 7168 192 / 181, 128 x 7168 93 / 100; 256 x 7168 in f16, 16 tokens
+    // 21.7 / 13.7, 160 x 5120 in f16, 32 tokens 16.3 / 11.2, in f32 16 tokens 8.4 / 7.6; 128 x 7168 in f32, 64 tokens 13.9 / 15.0; 128 x 2048 in
+    // f32, 128 tokens 4.8 / 5.2.  (275 shapes: 0.3 % behind the better order.)
     const size_t elems = (size_t)n_expert * k;
-    a.by_expert = c->tune.moe_logits >= 16 ? c->tune.moe_logits >= 32 : (elems >= 800000 && ntok <= 64) || elems * (a.f16 ? 2 : 4) > ((size_t)4 << 20);
+    if (c->tune.moe_logits >= 16) a.by_expert = c->tune.moe_logits >= 32;
+    else if (ntok <= 64) a.by_expert = elems >= 800000 && (a.f16 || eb > 1 || (long)blocks * groups <= 3L * c->num_cu);
+    else a.by_expert = elems * (a.f16 ? 2 : 4) > ((size_t)4 << 20);
     Name name;
     name << "jl_moe_logits";
     if (eb > 1) name << "_e" << eb << (a.f16 ? "_f16" : "");
