@@ -111,8 +111,8 @@ int jl_synchronize(jl_ctx *ctx);
  * "moe.group16" (form 3: 1 a prep kernel quantizes the columns, 2 the matrix kernel does, 3 groups
  * of 32 columns),
  * "moe.chunk" (form 3: super-blocks a step, 1-3),
- * "moe.group" / "moe.logits" / "moe.waves" / "moe.lpr" (forms of the mixture
- * block's other kernels),
+ * "moe.group" / "moe.logits" / "moe.waves" / "moe.lpr" (forms of the mixture block's other kernels; "moe.logits": expert
+ * rows a workgroup, and 16 / 32 more for token groups / expert rows side by side),
  * "mxfp4.split" (K slices of the MXFP4 GEMM), "mxfp4.rows" (96 or 128 rows a tile; 1: the
  * general decode matvec also for one token), "mxfp4.few" / "mxfp4.few_min" (the MXFP4
  * few-token form up to / from this many tokens), "mxfp4.one" (its single launch: 1 never, 11 / 12 with 16 / 32 rows
